@@ -1,0 +1,90 @@
+"""The native eager path (csrc/torch_binding.cpp) against the Python autograd Functions, which call the same kernels: same
+bits in outputs and gradients, whichever inputs ask for a gradient, and the same errors for what the kernels do not take."""
+import pytest
+import torch
+
+from oracle import inputs
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _flat(d, n, dtype=torch.bfloat16):
+    B, T, H, C = d[n].shape
+    return d[n].reshape(B, T, H * C).to(DEV, dtype)
+
+
+def _run(fn, leaves, wanted, grads):
+    xs = [t.detach().clone().requires_grad_(i in wanted) for i, t in enumerate(leaves)]
+    outs = fn(*xs)
+    gs = torch.autograd.grad(outs, [x for i, x in enumerate(xs) if i in wanted], grads)
+    return [o.detach() for o in outs] + list(gs)
+
+
+def _same(native, function, leaves, grads, wanted_sets):
+    for wanted in wanted_sets:
+        for x, y in zip(_run(native, leaves, wanted, grads), _run(function, leaves, wanted, grads)):
+            assert x.dtype == y.dtype and torch.equal(x.reshape(-1), y.reshape(-1))
+
+
+@pytest.mark.parametrize('state_dtype', [torch.float32, torch.bfloat16, None])
+@pytest.mark.parametrize('B,T,H,C', [(1, 16, 1, 64), (2, 48, 3, 64), (2, 32, 3, 128), (1, 2048, 2, 64)])
+def test_attn_and_attn_ln_equal_the_python_functions(B, T, H, C, state_dtype):
+    from wind_rwkv.rwkv7 import attn, attn_ln
+    from wind_rwkv.rwkv7.wkv_attn import WindRWKV7, no_state
+    from wind_rwkv.rwkv7.wkv_attn_ln import WindRWKV7LN
+    d = inputs.attn_ln_inputs(B, T, H, C, 3, dtype=torch.bfloat16)
+    gen = torch.Generator().manual_seed(4)
+    seqs = [_flat(d, n) for n in 'qwkvab']
+    heads = lambda t: t.view(B, T, H, C)
+    state = [] if state_dtype is None else [torch.randn(B, H, C, C, generator=gen).to(DEV, state_dtype)]
+    s0_of = lambda st: st[0] if st else no_state(torch.bfloat16, DEV)
+    dy = _flat(d, 'dy')
+    dsT = torch.randn(B, H, C, C, generator=gen).to(DEV, state_dtype or torch.bfloat16)
+    every = set(range(6 + len(state)))
+    def function(r, w, k, v, a, b, *st):
+        y, sT, _ = WindRWKV7.apply(*map(heads, (w, r, k, v, a, b)), s0_of(st))
+        return y.view(B, T, H * C), sT
+    native = lambda *x: attn(*x[:6], C, s0=x[6] if x[6:] else None, return_state=True)
+    _same(native, function, seqs + state, [dy, dsT], [every, {1, 3}, {max(every)}])
+    def function_ln(r, w, k, v, a, b, g, p, *st):
+        y, sT, _ = WindRWKV7LN.apply(*map(heads, (w, r, k, v, a, b, g)), p, s0_of(st))
+        return y.view(B, T, H * C), sT
+    native_ln = lambda *x: attn_ln(*x[:8], C, s0=x[8] if x[8:] else None, return_state=True)
+    every = set(range(8 + len(state)))
+    _same(native_ln, function_ln, seqs + [_flat(d, 'g'), d['params'].to(DEV)] + state, [dy, dsT], [every, {6, 7}, {max(every)}])
+
+
+@pytest.mark.parametrize('param_dtype', [torch.float32, torch.bfloat16])
+def test_ddlerp_and_expand_loras_equal_the_python_functions(param_dtype):
+    from wind_rwkv.rwkv7 import ddlerp, expand_loras
+    from wind_rwkv.rwkv7.loras import ExpandLoras
+    from wind_rwkv.rwkv7.token_shift import DDLerp
+    B, T, C = 2, 48, 128
+    d = inputs.ddlerp_inputs(B, T, C, 32, 5, dtype=torch.bfloat16)
+    leaves = [d['x'].to(DEV)] + [d[n].to(DEV, param_dtype) for n in ('alpha', 'L', 'R', 'beta')]
+    _same(ddlerp, DDLerp.apply, leaves, [g.to(DEV) for g in d['dy']], [set(range(5)), {0}, {2}])
+    d = inputs.expand_loras_inputs(B, T, C, 16, 6, dtype=torch.bfloat16)
+    acts = [d[n].to(DEV) for n in ('w_in', 'k_in', 'z_in', 'a_in', 'ma_in', 'mk_in')]
+    params = [d[n].to(DEV, param_dtype) for n in ('Wz', 'Wa', 'Wma', 'Wmk', 'w_bias', 'a_bias', 'ma_bias', 'mk_bias')]
+    _same(lambda *x: expand_loras(*x, 64), lambda *x: ExpandLoras.apply(*x, 64), acts + params, [g.to(DEV) for g in d['dy']],
+          [set(range(14)), {2, 5}, {9, 13}])
+
+
+def test_what_the_native_path_leaves_to_python():
+    """Strided inputs and wrong types raise as before; a changed checkpoint interval is an error in backward."""
+    from wind_rwkv.rwkv7 import attn, checkpoint_interval, set_checkpoint_interval
+    d = inputs.wkv7_inputs(1, 32, 2, 64, 7, dtype=torch.bfloat16)
+    seqs = [_flat(d, n).requires_grad_() for n in 'qwkvab']
+    with pytest.raises(AssertionError):
+        attn(*[t.mT.contiguous().mT for t in seqs], 64)
+    with pytest.raises(AssertionError):
+        attn(seqs[0].half(), *seqs[1:], 64)
+    before = checkpoint_interval()
+    y = attn(*seqs, 64)
+    set_checkpoint_interval(48 - before)
+    try:
+        with pytest.raises(RuntimeError, match='checkpoint interval'):
+            y.sum().backward()
+    finally:
+        set_checkpoint_interval(before)

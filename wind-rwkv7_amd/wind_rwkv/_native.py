@@ -1,9 +1,11 @@
-"""ctypes binding of the C-ABI library (include/wind_rwkv7.h).
+"""Bindings of the C-ABI library (include/wind_rwkv7.h): ctypes, and the native eager path of the operators.
 
 The HIP library is the only implementation: if it is missing, importing the ops fails loudly
 instead of falling back to anything slower.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -106,6 +108,25 @@ def lib():
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+BINDING_PATH = os.path.join(_PKG_DIR, 'lib', 'torch_binding.so')
+_binding = None
+
+
+def binding():
+    """The native eager path of the operators (csrc/torch_binding.cpp) on the loaded library; like it, required."""
+    global _binding
+    if _binding is None:
+        lib()
+        if not os.path.exists(BINDING_PATH):
+            raise ImportError(f'{BINDING_PATH} is missing: build it with `make -C {os.path.dirname(_PKG_DIR)}`.')
+        loader = importlib.machinery.ExtensionFileLoader('torch_binding', BINDING_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('torch_binding', BINDING_PATH, loader=loader))
+        loader.exec_module(module)
+        module.load(LIB_PATH)
+        _binding = module
+    return _binding
 
 
 def check(code):

@@ -94,4 +94,11 @@ class ExpandLoras(torch.autograd.Function):
         return (*grads[:6], *_grads_like(flat, pgrads, ctx.param_dtype), None)
 
 
-expand_loras = ExpandLoras.apply
+def expand_loras(w_in, k_in, z_in, a_in, ma_in, mk_in, Wz, Wa, Wma, Wmk, w_bias, a_bias, ma_bias, mk_bias, HEAD_SIZE):
+    """(w, k, kk, b) from the first-half products and the second LoRA factors, rwkv7_expand_loras.py:214-241."""
+    ins = (w_in, k_in, z_in, a_in, ma_in, mk_in, Wz, Wa, Wma, Wmk, w_bias, a_bias, ma_bias, mk_bias)
+    if not torch.compiler.is_compiling():
+        outs = _native.binding().expand_loras(ins, HEAD_SIZE)   # (None: not the plain case)
+        if outs is not None:
+            return outs
+    return ExpandLoras.apply(*ins, HEAD_SIZE)

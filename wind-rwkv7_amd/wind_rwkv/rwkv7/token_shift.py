@@ -104,6 +104,10 @@ def ddlerp(x, alpha, L, R, beta):
     """ddlerp(x, alpha, L, R, beta) -> (y0, y1, y2, y3), rwkv7_ddlerp.py:306-336.  A LoRA rank above 64 runs as pieces of
     at most 64: the interpolation weight is a sum over the rank, c_k = sum_d bmid[k,d] R[k,:,d] + beta_k, so with the
     rank cut in n pieces (beta in the first one only) y_k = sum_i y_k^(i) - (n - 1) x.  The pieces are added in fp32."""
+    if not torch.compiler.is_compiling():
+        ys = _native.binding().ddlerp(x, alpha, L, R, beta)   # (None: not the plain case)
+        if ys is not None:
+            return ys
     D = R.shape[2]
     if D <= 64:
         return DDLerp.apply(x, alpha, L, R, beta)

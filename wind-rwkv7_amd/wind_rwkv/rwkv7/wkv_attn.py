@@ -452,7 +452,12 @@ def attn(r, w, k, v, a, b, HEAD_SIZE, s0=None, return_state=False):
     Head sizes: multiples of 16 up to 128 (the reference compiles its CUDA kernel per head size,
     rwkv7_attn.py:46-51, and has rwkv7_attn_triton_bighead.py for large ones).  bf16 sequences run matrix-core
     kernels at every one of them: the fused kernels at 64, the three-phase kernels of csrc/wkv7_wide.hip at the
-    others."""
+    others.  Eager calls on plain arguments run in the native binding; the rest of this function is what
+    torch.compile traces, and the path of every other case."""
+    if not torch.compiler.is_compiling():
+        out = _native.binding().attn(r, w, k, v, a, b, HEAD_SIZE, s0, return_state)
+        if out is not None:
+            return out
     B, T, HC = w.shape
     C = HEAD_SIZE
     H = HC // C

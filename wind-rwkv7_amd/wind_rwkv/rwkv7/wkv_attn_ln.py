@@ -246,11 +246,15 @@ def attn_ln(r, w, k, v, a, b, g, params, HEAD_SIZE, s0=None, return_state=False,
     epilogue in PyTorch in fp32, about seventeen times slower at head size 128; None / 'bf16' / 'tf32' the bf16
     kernels.  float32 tensors always take the fp32 route.  It has no effect at head size 64."""
     from .wkv_attn import attn, _attn_bf16_head, _bf16_head
+    if dot_prec not in (None, 'fp32', 'tf32', 'bf16'):
+        raise ValueError(f"dot_prec must be None, 'fp32', 'tf32' or 'bf16', got {dot_prec!r}")
+    if not torch.compiler.is_compiling() and (dot_prec != 'fp32' or HEAD_SIZE == 64):
+        out = _native.binding().attn_ln(r, w, k, v, a, b, g, params, HEAD_SIZE, s0, return_state)   # (None: not the plain case)
+        if out is not None:
+            return out
     B, T, HC = w.shape
     C = HEAD_SIZE
     H = HC // C
-    if dot_prec not in (None, 'fp32', 'tf32', 'bf16'):
-        raise ValueError(f"dot_prec must be None, 'fp32', 'tf32' or 'bf16', got {dot_prec!r}")
     if w.dtype == torch.float32 or not (_bf16_head(C) or (dot_prec != 'fp32' and _attn_bf16_head(C))):
         # the fp32 WKV7 kernels followed by the epilogue in PyTorch (fp32 arithmetic), as the reference composes its
         # own unfused path (time_mixer.py:158-163); accurate to fp32 rounding, the result cast to the sequences' dtype
