@@ -271,6 +271,10 @@ size_t wind_rwkv7_ddlerp_bwd_workspace_bytes(int B, int T, int C, int D);
 int wind_rwkv7_ddlerp_forward(int B, int T, int C, int D,
                               const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                               void* bmid, void* bder, void* y, void* stream);
+/* The forward of a piece of a longer sequence: x_prev [B,C] bf16 is the token before x[:, 0] (NULL: a zero row, as above). */
+int wind_rwkv7_ddlerp_forward_from(int B, int T, int C, int D, const void* x, const void* x_prev, const void* alpha,
+                                   const void* L, const void* R, const void* beta, void* bmid, void* bder, void* y,
+                                   void* stream);
 int wind_rwkv7_ddlerp_backward(int B, int T, int C, int D,
                                const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                                const void* bmid, const void* bder,
@@ -370,6 +374,10 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
                                   const void* const* x, const long long* ld_x,
                                   void* const* dW, int out_dtype,
                                   void* workspace, size_t workspace_bytes, void* stream);
+
+/* Tokens first .. T-1 of the recurrence's operands w, k, b [B,T,C] bf16 become ones that leave a state as it is: decay 1,
+ * k = b = 0.  A sequence of any length then runs padded to whole chunks and its final state is that of token first-1. */
+int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* stream);
 
 /* Column blocks of token-major bf16 matrices, moved in one launch: piece t is width[t] columns of M rows, read at
  * src[t] (row stride src_ld[t] elements, first column src_col0[t]; a null src reads as zeros) and written at

@@ -88,3 +88,69 @@ def test_what_the_native_path_leaves_to_python():
             y.sum().backward()
     finally:
         set_checkpoint_interval(before)
+
+
+class _Absent:
+    """A binding that takes no case: every call falls to the Python path."""
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+@pytest.mark.parametrize('C,H,x_dtype,param_dtype,frozen', [
+    (128, 2, torch.bfloat16, torch.float32, ()), (192, 6, torch.float32, torch.float32, ('Wr', 'gate_w2', 'ln_x.weight')),
+    (256, 2, torch.bfloat16, torch.bfloat16, ('Wo', 'time_maa_w1'))])
+def test_block_equals_the_python_path(monkeypatch, C, H, x_dtype, param_dtype, frozen):
+    """Forward, backward and the forward without autograd of the whole block, with some parameters frozen; same kernels and
+    library products in the same order, so the same bits."""
+    from collections import namedtuple
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import TimeMixer
+    gen = torch.Generator().manual_seed(C)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, C), 1)
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+            p.requires_grad_(n not in frozen)
+    model = model.to(DEV, param_dtype)
+    x = torch.randn(2, 48, C, generator=gen).to(DEV, x_dtype)
+    dy = torch.randn(2, 48, C, generator=gen).to(DEV, torch.bfloat16)
+    results = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(_native, 'binding', lambda: _Absent())
+        leaves = [x.clone().requires_grad_()] + [p for p in model.parameters() if p.requires_grad]
+        y = model(leaves[0])
+        with torch.no_grad():
+            z = model(x)
+        results.append([y.detach(), z] + list(torch.autograd.grad(y, leaves, dy)))
+    for i, (a, b) in enumerate(zip(*results)):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
+
+
+@pytest.mark.parametrize('T', [2, 15, 17, 100])
+@pytest.mark.parametrize('continued', [False, True])
+def test_prompt_of_any_length_equals_the_python_path(monkeypatch, T, continued):
+    """A prompt padded to whole chunks against whole chunks followed by single-token steps: other roundings, so at the
+    block's gate (1.27e-2 where `step` computed the tokens, see tests/test_gpu_time_mixer_state.py), state at 1e-2."""
+    from collections import namedtuple
+    from oracle import seq_ref
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import TimeMixer
+    gen = torch.Generator().manual_seed(T)
+    C, H, B = 256, 4, 3
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, C), 1)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+    model = model.to(DEV)
+    x = torch.randn(B, T, C, generator=gen).bfloat16().to(DEV)
+    state = (torch.randn(B, C, generator=gen).bfloat16().to(DEV), torch.randn(B, H, 64, 64, generator=gen).to(DEV)) if continued else None
+    with torch.no_grad():
+        y, (last, S) = model(x, state=state, return_state=True)
+        monkeypatch.setattr(_native, 'binding', lambda: _Absent())
+        y0, (last0, S0) = model(x, state=state, return_state=True)
+    assert y.shape == y0.shape and y.is_contiguous() and torch.equal(last, last0) and torch.equal(last, x[:, -1])
+    assert S.dtype == S0.dtype == torch.float32
+    first = 0 if continued else 1     # from a zero state the first token's GroupNorm is ill conditioned
+    assert seq_ref.rel_err(y[:, first:].float().cpu(), y0[:, first:].float().cpu()) <= 1.27e-2
+    assert seq_ref.rel_err(S.cpu(), S0.cpu()) <= 1e-2

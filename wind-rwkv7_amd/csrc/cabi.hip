@@ -541,10 +541,16 @@ size_t wind_rwkv7_ddlerp_bwd_workspace_bytes(int B, int T, int C, int D) {
 int wind_rwkv7_ddlerp_forward(int B, int T, int C, int D,
                               const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                               void* bmid, void* bder, void* y, void* stream) {
+    return wind_rwkv7_ddlerp_forward_from(B, T, C, D, x, nullptr, alpha, L, R, beta, bmid, bder, y, stream);
+}
+
+int wind_rwkv7_ddlerp_forward_from(int B, int T, int C, int D, const void* x, const void* x_prev, const void* alpha,
+                                   const void* L, const void* R, const void* beta, void* bmid, void* bder, void* y,
+                                   void* stream) {
     const int rc = check_ddlerp(B, T, C, D);
     if (rc) return rc;
     if (!x || !alpha || !L || !R || !beta || !bmid || !bder || !y) return WIND_RWKV7_ERR_NULL_POINTER;
-    wkv::launch_ddlerp_forward((long)B * T, T, C, D, x, alpha, L, R, beta, bmid, bder, y,
+    wkv::launch_ddlerp_forward((long)B * T, T, C, D, x, x_prev, alpha, L, R, beta, bmid, bder, y,
                                static_cast<hipStream_t>(stream));
     return launch_status();
 }
@@ -783,6 +789,14 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
     if (!wkv::launch_linear_wgrad_group(n, (long)tokens, O, I, dy, ldy, x, ldx, dW, out_dtype == WIND_RWKV7_F32, workspace,
                                         static_cast<hipStream_t>(stream)))
         return WIND_RWKV7_ERR_CHANNELS;
+    return launch_status();
+}
+
+int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* stream) {
+    if (B <= 0 || T <= 0 || C <= 0 || C % 8 != 0 || first < 0 || first > T || (long long)B * T * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if ((long long)B * (T - first) * (C / 8) > 0x7fffffffLL) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!w || !k || !b) return WIND_RWKV7_ERR_NULL_POINTER;
+    if (first < T) wkv::launch_neutral_rows(B, T, C, first, w, k, b, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

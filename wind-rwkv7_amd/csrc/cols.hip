@@ -58,7 +58,28 @@ __global__ __launch_bounds__(256) void copy_columns_kernel(ColsArgs g) {
     *reinterpret_cast<bf16x8*>(p.dst + m * p.dst_ld + p.dst_col0 + c) = x;
 }
 
+// w = -80 gives the decay exp(-exp(w)) = 1 in float32
+__global__ __launch_bounds__(256) void neutral_rows_kernel(int T, int C, int first, int vectors, __bf16* __restrict__ w,
+                                                           __bf16* __restrict__ k, __bf16* __restrict__ b) {
+    const int v = blockIdx.x * 256 + threadIdx.x;
+    if (v >= vectors) return;
+    const int per_row = C / 8, row = v / per_row, rows = T - first;
+    const long at = ((long)(row / rows) * T + first + row % rows) * C + (v % per_row) * 8;
+    bf16x8 none, zero = {};
+#pragma unroll
+    for (int e = 0; e < 8; e++) none[e] = (__bf16)-80.f;
+    *reinterpret_cast<bf16x8*>(w + at) = none;
+    *reinterpret_cast<bf16x8*>(k + at) = zero;
+    *reinterpret_cast<bf16x8*>(b + at) = zero;
+}
+
 }  // namespace
+
+void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, hipStream_t stream) {
+    const int vectors = B * (T - first) * (C / 8);
+    hipLaunchKernelGGL(neutral_rows_kernel, dim3((unsigned)((vectors + 255) / 256)), dim3(256), 0, stream, T, C, first, vectors,
+                       static_cast<__bf16*>(w), static_cast<__bf16*>(k), static_cast<__bf16*>(b));
+}
 
 void launch_copy_columns(long long M, int n, const ColumnPiece* pieces, hipStream_t stream) {
     for (int first = 0; first < n; first += COLS_MAX_PIECES) {

@@ -29,10 +29,22 @@ struct Dy4 {  // the four upstream gradients, each [M, C]
 struct XTile {
     TileF x, xx;
 };
-__device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, long m0, int T, int C, int c0, const Lane& L) {
+// the row before token m at the lane's channels: the token before it, at a sequence's start the carried token of x_prev,
+// or (has_prev false: to be read as zeros) the row itself
+struct PrevRow {
+    const __bf16* row;
+    bool has_prev;
+};
+__device__ __forceinline__ PrevRow prev_row(const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev, long m, int T, int C, int c) {
+    const bool inside = (m % T) != 0;
+    const __bf16* row = x + m * C + c;
+    return {inside ? row - C : x_prev ? x_prev + (m / T) * C + c : row, inside || x_prev};
+}
+__device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev, long m0, int T, int C,
+                                             int c0, const Lane& L) {
     XTile r;
     const long m = m0 + L.n;
-    const bool has_prev = (m % T) != 0;
+    const PrevRow before = prev_row(x, x_prev, m, T, C, c0 + 8 * L.g);
     // 16-byte accesses: blocks 2p and 2p+1 of the tile are the interleaved channels of chan16 (frag.hpp); every
     // per-channel operand of these kernels is indexed through the same map
     const __bf16* row = x + m * C + c0 + 8 * L.g;
@@ -40,7 +52,7 @@ __device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, long 
     for (int pr = 0; pr < NBLK / 2; pr++) {
         const bf16x8 cur = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
         bf16x8 prev = {};
-        if (has_prev) prev = *reinterpret_cast<const bf16x8*>(row - C + 32 * pr);
+        if (before.has_prev) prev = *reinterpret_cast<const bf16x8*>(before.row + 32 * pr);
 #pragma unroll
         for (int hlf = 0; hlf < 2; hlf++) {
             const f32x4 c = to_f32(hlf ? __builtin_shufflevector(cur, cur, 4, 5, 6, 7) : __builtin_shufflevector(cur, cur, 0, 1, 2, 3));
@@ -94,6 +106,7 @@ __device__ __forceinline__ void load_r_fragments(bf16x4 (&raw)[NB / 4][NBLK], co
 // forward 1: bmid = tanh((x + xx*alpha) L^T), bder = 1 - bmid^2
 template <int D, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int C, const __bf16* __restrict__ x,
+                                                             const __bf16* __restrict__ x_prev,
                                                              const __bf16* __restrict__ alpha,
                                                              const __bf16* __restrict__ Lw, __bf16* __restrict__ bmid,
                                                              __bf16* __restrict__ bder) {
@@ -126,12 +139,13 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
         bf16x8 xc[NBLK / 2], xp[NBLK / 2];
         bf16x4 al[NBLK];
     };
-    const bool has_prev = ((m0 + L.n) % T) != 0;
+    const PrevRow before = prev_row(x, x_prev, m0 + L.n, T, C, 8 * L.g);
+    const bool has_prev = before.has_prev;
     auto fetch = [&](Set& st, int cbk) {
         const int c0 = 64 * cbk;
         load_mid_weights<NB>(st.wr, Lw, C, c0, wave, L);
         const __bf16* row = x + (m0 + L.n) * C + c0 + 8 * L.g;
-        const __bf16* prow = has_prev ? row - C : row;
+        const __bf16* prow = before.row + c0;
 #pragma unroll
         for (int pr = 0; pr < NBLK / 2; pr++) {
             st.xc[pr] = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
@@ -353,8 +367,8 @@ __device__ __forceinline__ void load_mid_pairs(bf16x8 (&out)[NPAIR], const __bf1
 // forward 2: y_k = x + xx * (bmid_k R_k^T + beta_k).  Block = (64 channels, range of token tiles).
 template <int D>
 __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int C, int tiles_per_split,
-                                                              const __bf16* __restrict__ x, const __bf16* __restrict__ R,
-                                                              const __bf16* __restrict__ beta,
+                                                              const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev,
+                                                              const __bf16* __restrict__ R, const __bf16* __restrict__ beta,
                                                               const __bf16* __restrict__ bmid, __bf16* __restrict__ y) {
     constexpr int ND = D / 16;
     __shared__ LerpWeights<D> w;
@@ -368,7 +382,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int
     __syncthreads();
     for (long tile = tile_begin + wave; tile < tile_end; tile += 4) {
         const long m0 = tile * TOK;
-        const XTile xt = load_x_tile(x, m0, T, C, c0, L);
+        const XTile xt = load_x_tile(x, x_prev, m0, T, C, c0, L);
         bf16x8 bm[4 * ND / 2];
         load_mid_pairs(bm, bmid + (m0 + L.n) * (4 * D), L);
 #pragma unroll
@@ -708,20 +722,20 @@ size_t ddlerp_bwd_workspace_bytes(long M, int C, int D) {
 
 namespace {
 template <int D>
-void forward_rank(long M, int T, int C, const void* x, const void* alpha, const void* Lw, const void* R, const void* beta,
+void forward_rank(long M, int T, int C, const void* x, const void* x_prev, const void* alpha, const void* Lw, const void* R, const void* beta,
                   void* bmid, void* bder, void* y, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     // four tiles per block when that still gives every compute unit a block, else two
     const long ntiles = M / TOK;
     if (ntiles >= 4 * 256)
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 4>), dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, stream, M, T, C,
-                           c(x), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+                           c(x), c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     else
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 2>), dim3((unsigned)((ntiles + 1) / 2)), dim3(256), 0, stream, M, T, C,
-                           c(x), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+                           c(x), c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     const StreamSplit sp = stream_splits(M, C / 64, 4 * compute_units());   // two blocks per compute unit, two rounds
     hipLaunchKernelGGL(ddlerp_fwd_out2_kernel<D>, dim3(C / 64, sp.nsplit), dim3(256), 0, stream, M, T, C, sp.tiles_per_split,
-                       c(x), c(R), c(beta), c(bmid), static_cast<__bf16*>(y));
+                       c(x), c(x_prev), c(R), c(beta), c(bmid), static_cast<__bf16*>(y));
 }
 
 template <int D>
@@ -753,10 +767,10 @@ void backward_rank(long M, int T, int C, const void* x, const void* alpha, const
 }  // namespace
 
 // (the callers have checked ddlerp_rank_supported(D))
-void launch_ddlerp_forward(long M, int T, int C, int D, const void* x, const void* alpha, const void* Lw, const void* R,
-                           const void* beta, void* bmid, void* bder, void* y, hipStream_t stream) {
-    if (D == 64) forward_rank<64>(M, T, C, x, alpha, Lw, R, beta, bmid, bder, y, stream);
-    else forward_rank<32>(M, T, C, x, alpha, Lw, R, beta, bmid, bder, y, stream);
+void launch_ddlerp_forward(long M, int T, int C, int D, const void* x, const void* x_prev, const void* alpha, const void* Lw,
+                           const void* R, const void* beta, void* bmid, void* bder, void* y, hipStream_t stream) {
+    if (D == 64) forward_rank<64>(M, T, C, x, x_prev, alpha, Lw, R, beta, bmid, bder, y, stream);
+    else forward_rank<32>(M, T, C, x, x_prev, alpha, Lw, R, beta, bmid, bder, y, stream);
 }
 
 void launch_ddlerp_backward(long M, int T, int C, int D, const void* x, const void* alpha, const void* Lw, const void* R,

@@ -45,4 +45,7 @@ constexpr int CAST_MAX_TENSORS = 32;   // per launch; longer lists take several
 void launch_cast_to_bf16(int n, const void* const* src, const int* src_f32, const long long* numel,
                          const long long* dst_offset, void* dst, hipStream_t stream);
 
+// rows first .. T-1 of w, k, b [B, T, C] (bf16): decay 1, k = b = 0
+void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, hipStream_t stream);
+
 }  // namespace wkv

@@ -14,6 +14,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include "../../include/wind_rwkv7.h"
@@ -34,7 +35,9 @@ namespace py = pybind11;
     X(attn_ln_forward) X(attn_ln_prefill) X(attn_ln_backward)                                                        \
     X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward)                             \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
-    X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)
+    X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
+    X(ddlerp_forward_from) X(neutral_rows) X(copy_columns) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode)
 
 struct Lib {
 #define X(name) decltype(&wind_rwkv7_##name) name = nullptr;
@@ -491,6 +494,425 @@ py::object expand_loras(const variable_list& in, int64_t head_size) {
     return py::make_tuple(y[0], y[1], y[2], y[3]);
 }
 
+// ------------------------------------------------------------------------------------------------
+// TimeMixer: the whole block as one node (training), as one call (prompts) and one token at a time
+// ------------------------------------------------------------------------------------------------
+// The block's parameters: the weights in the order of wind_rwkv7_mixer_weights, then the GroupNorm's and the bonus.
+enum Param {
+    MAA_X, MAA, MAA_W1, MAA_W2, WR, WK, WV, WO, GATE_W1, DECAY_W1, KKK_W1, MK_W1, AAA_W1, MA_W1, GATE_W2, DECAY_W2, KKK_W2,
+    MK_W2, AAA_W2, MA_W2, DECAY, AAAAA, MISC_A, MISC_K, LN_W, LN_B, FAAAA, PARAMS
+};
+constexpr int WEIGHTS = LN_W;   // the ones whose bf16 copies the kernels take
+const char* const PARAM_NAMES[PARAMS] = {
+    "time_maa_x", "time_maa", "time_maa_w1", "time_maa_w2", "Wr", "Wk", "Wv", "Wo", "gate_w1", "time_decay_w1", "time_kkk_w1",
+    "mk_w1", "time_aaa_w1", "ma_w1", "gate_w2", "time_decay_w2", "time_kkk_w2", "mk_w2", "time_aaa_w2", "ma_w2", "time_decay",
+    "time_aaaaa", "time_misc_a", "time_misc_k", "weight", "bias", "time_faaaa"};
+constexpr int R_MIX = 32, R_DECAY = 64, R_GATE = 128, R_LORA = 16;   // LoRA ranks (time_mixer.py:69-94); R_LORA: aaa, kkk, ma, mk
+constexpr int W_KKMK = 2 * R_LORA, W_DECAY_AAA_MA = R_DECAY + 2 * R_LORA;
+
+std::vector<int64_t> param_shape(int i, int64_t C) {
+    switch (i) {
+        case MAA: return {4, 1, 1, C};
+        case MAA_W1: return {4 * R_MIX, C};
+        case MAA_W2: return {4, C, R_MIX};
+        case WR: case WK: case WV: case WO: return {C, C};
+        case GATE_W1: return {R_GATE, C};
+        case DECAY_W1: return {R_DECAY, C};
+        case KKK_W1: case MK_W1: case AAA_W1: case MA_W1: return {R_LORA, C};
+        case GATE_W2: return {C, R_GATE};
+        case DECAY_W2: return {C, R_DECAY};
+        case KKK_W2: case MK_W2: case AAA_W2: case MA_W2: return {C, R_LORA};
+        default: return {C};
+    }
+}
+// Where each parameter lies in a buffer of all of them, in elements.  Every piece is a multiple of 64 elements, so the two
+// concatenated first halves [kkk; mk] and [decay; aaa; ma] are one matrix each and the GroupNorm's weight, bias and the
+// bonus are the [3, C] tensor of attn_ln.
+struct ParamLayout {
+    int64_t at[PARAMS + 1];
+    explicit ParamLayout(int64_t C) {
+        static const int order[PARAMS] = {WR, WK, WV, WO, GATE_W1, KKK_W1, MK_W1, DECAY_W1, AAA_W1, MA_W1, GATE_W2, DECAY_W2, MAA_W1,
+                                          MAA_W2, KKK_W2, MK_W2, AAA_W2, MA_W2, MAA_X, MAA, DECAY, AAAAA, MISC_A, MISC_K, LN_W, LN_B, FAAAA};
+        int64_t o = 0;
+        for (int i : order) {
+            at[i] = o;
+            o += c10::multiply_integers(param_shape(i, C));
+        }
+        at[PARAMS] = o;
+    }
+};
+
+struct Block {   // the sizes of a call
+    int64_t B, T, C, H;
+    int64_t rows() const { return B * T; }
+    int64_t N() const { return C / H; }
+    int64_t plane() const { return rows() * C; }
+};
+using B16 = c10::BFloat16;
+B16* at_elem(const Tensor& t, int64_t o) { return static_cast<B16*>(t.data_ptr()) + o; }
+Tensor matrix(const Tensor& buf, int64_t offset, int64_t rows, int64_t cols) { return buf.as_strided({rows, cols}, {cols, 1}, offset); }
+
+// Activations of a block in one buffer; offsets in elements (all multiples of 256: rows() is a multiple of 16).
+struct Activations {
+    int64_t streams, r, k, v, g, w2, w, k2, kk, b, ya, mid, der, tg1, tw1, kk1, mk1, a1, ma1, kept, g1, kkmk, w1a1ma1, total;
+    explicit Activations(const Block& s) {
+        int64_t o = 0;
+        auto take = [&](int64_t n) { const int64_t r = o; o += n; return r; };
+        const int64_t M = s.rows(), P = s.plane();
+        streams = take(4 * P);
+        r = take(P), k = take(P), v = take(P), g = take(P), w2 = take(P), w = take(P), k2 = take(P), kk = take(P), b = take(P), ya = take(P);
+        mid = take(4 * R_MIX * M), der = take(4 * R_MIX * M);
+        tg1 = take(R_GATE * M), tw1 = take(R_DECAY * M);
+        kk1 = take(R_LORA * M), mk1 = take(R_LORA * M), a1 = take(R_LORA * M), ma1 = take(R_LORA * M);
+        kept = o;
+        g1 = take(R_GATE * M), kkmk = take(W_KKMK * M), w1a1ma1 = take(W_DECAY_AAA_MA * M);   // dead once they are split
+        total = o;
+    }
+};
+
+// column slices in one launch (wind_rwkv7_copy_columns)
+struct Columns {
+    std::vector<const void*> src, aux;
+    std::vector<void*> dst;
+    std::vector<long long> src_ld, dst_ld;
+    std::vector<int> src_col, dst_col, width, op;
+    void add(const void* s, int sld, int sc, void* d, int dld, int dc, int w, int o, const void* x = nullptr) {
+        src.push_back(s), src_ld.push_back(sld), src_col.push_back(sc), dst.push_back(d), dst_ld.push_back(dld), dst_col.push_back(dc);
+        width.push_back(w), op.push_back(o), aux.push_back(x);
+    }
+    void run(int64_t rows, void* stream) {
+        check(L.copy_columns(rows, (int)dst.size(), src.data(), src_ld.data(), src_col.data(), dst.data(), dst_ld.data(), dst_col.data(),
+                             width.data(), op.data(), aux.data(), stream));
+    }
+};
+
+// dW = dy^T x for several pairs on the same tokens: one grouped launch (a single pair goes through its own entry point)
+struct WeightGrads {
+    std::vector<int> O, I;
+    std::vector<const void*> dy, x;
+    std::vector<long long> ld_dy, ld_x;
+    std::vector<void*> dW;
+    void add(const void* d, int o, const void* a, int i, void* w) {
+        dy.push_back(d), O.push_back(o), ld_dy.push_back(o), x.push_back(a), I.push_back(i), ld_x.push_back(i), dW.push_back(w);
+    }
+    void run(int64_t tokens, const Tensor& like, void* stream) {
+        const int n = (int)O.size();
+        if (n == 0) return;
+        if (n == 1) {
+            const Tensor ws = scratch_bytes(L.linear_wgrad_workspace_bytes(tokens, O[0], I[0]), like);
+            check(L.linear_wgrad(tokens, O[0], I[0], dy[0], ld_dy[0], x[0], ld_x[0], dW[0], WIND_RWKV7_F32, ptr(ws), ws.numel(), stream));
+            return;
+        }
+        const Tensor ws = scratch_bytes(L.linear_wgrad_group_workspace_bytes(n, tokens, O.data(), I.data()), like);
+        check(L.linear_wgrad_group(n, tokens, O.data(), I.data(), dy.data(), ld_dy.data(), x.data(), ld_x.data(), dW.data(), WIND_RWKV7_F32,
+                                   ptr(ws), ws.numel(), stream));
+    }
+};
+
+struct BlockForward {   // what one forward pass leaves
+    Tensor xb, weights, lnp, acts, saved, y, sT;
+};
+
+// x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  `valid` < T: the tokens from
+// there on are padding and leave the state as it is.  x_prev [B,C] bf16 / s0: a carried state (undefined: zero).
+BlockForward block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const Tensor& x_prev,
+                           const Tensor& s0, at::ScalarType state_type) {
+    const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
+    const int64_t M = s.rows();
+    void* stream = stream_of(xb);
+    const ParamLayout at_(C);
+    BlockForward f;
+    f.xb = xb;
+    f.weights = at::empty({at_.at[LN_W]}, xb.options());
+    {
+        const void* src[WEIGHTS];
+        int dtype[WEIGHTS];
+        long long numel[WEIGHTS], offset[WEIGHTS];
+        for (int i = 0; i < WEIGHTS; i++) {
+            src[i] = p[i].data_ptr();
+            dtype[i] = p[i].scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
+            numel[i] = p[i].numel();
+            offset[i] = at_.at[i];
+        }
+        check(L.cast_to_bf16(WEIGHTS, src, dtype, numel, offset, f.weights.data_ptr(), stream));
+    }
+    f.lnp = at::stack({p[LN_W], p[LN_B], p[FAAAA]}).to(at::kFloat);
+    const Activations A(s);
+    f.acts = at::empty({save ? A.kept : A.total}, xb.options());
+    // (training keeps the activations: the concatenated first halves, which nothing needs later, go to a buffer of their own)
+    const Tensor firsts = save ? at::empty({A.total - A.kept}, xb.options()) : f.acts;
+    const int64_t shift = save ? A.kept : 0;
+    auto a = [&](int64_t o) -> void* { return at_elem(f.acts, o); };
+    auto w = [&](int i) -> void* { return at_elem(f.weights, at_.at[i]); };
+    auto weight = [&](int i, int64_t rows, int64_t cols) { return matrix(f.weights, at_.at[i], rows, cols); };
+    auto times = [&](const Tensor& out, int64_t in_off, int64_t in_cols, const Tensor& wt) {
+        Tensor o = out;
+        at::mm_out(o, matrix(f.acts, in_off, M, in_cols), wt.t());
+    };
+    check(L.ddlerp_forward_from(B, T, C, R_MIX, ptr(xb), ptr(x_prev), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), a(A.streams),
+                                stream));
+    const int64_t P = s.plane(), xrg = A.streams, xwa = A.streams + P, xk = A.streams + 2 * P, xv = A.streams + 3 * P;
+    const Tensor g1 = matrix(firsts, A.g1 - shift, M, R_GATE), kkmk = matrix(firsts, A.kkmk - shift, M, W_KKMK),
+                 w1a1ma1 = matrix(firsts, A.w1a1ma1 - shift, M, W_DECAY_AAA_MA);
+    times(matrix(f.acts, A.r, M, C), xrg, C, weight(WR, C, C));
+    times(g1, xrg, C, weight(GATE_W1, R_GATE, C));
+    times(matrix(f.acts, A.k, M, C), xk, C, weight(WK, C, C));
+    times(kkmk, xk, C, weight(KKK_W1, W_KKMK, C));
+    times(matrix(f.acts, A.v, M, C), xv, C, weight(WV, C, C));
+    times(w1a1ma1, xwa, C, weight(DECAY_W1, W_DECAY_AAA_MA, C));
+    Columns cols;
+    cols.add(ptr(kkmk), W_KKMK, 0, a(A.kk1), R_LORA, 0, R_LORA, 0);
+    cols.add(ptr(kkmk), W_KKMK, R_LORA, a(A.mk1), R_LORA, 0, R_LORA, 0);
+    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, 0, a(A.tw1), R_DECAY, 0, R_DECAY, 1);
+    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, R_DECAY, a(A.a1), R_LORA, 0, R_LORA, 0);
+    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, R_DECAY + R_LORA, a(A.ma1), R_LORA, 0, R_LORA, 0);
+    cols.add(ptr(g1), R_GATE, 0, a(A.tg1), R_GATE, 0, R_GATE, 1);
+    cols.run(M, stream);
+    times(matrix(f.acts, A.g, M, C), A.tg1, R_GATE, weight(GATE_W2, C, R_GATE));
+    times(matrix(f.acts, A.w2, M, C), A.tw1, R_DECAY, weight(DECAY_W2, C, R_DECAY));
+    check(L.expand_loras_forward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
+                                 w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b), stream));
+    if (valid < T) check(L.neutral_rows(B, T, C, (int)valid, a(A.w), a(A.k2), a(A.b), stream));
+    f.sT = at::empty({B, H, N, N}, xb.options().dtype(state_type));
+    const size_t ws = std::max<size_t>(L.attn_ln_fwd_workspace_bytes(B, T, H, N), 256);
+    const size_t keep_bytes = (L.attn_ln_saved_bytes(B, T, H, N) + 255) / 256 * 256;
+    f.saved = scratch_bytes(keep_bytes + ws, xb);
+    char* base = static_cast<char*>(f.saved.data_ptr());
+    check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
+        B, T, H, N, WIND_RWKV7_BF16, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b),
+        a(A.g), ptr(f.lnp), ptr(s0), a(A.ya), base, ptr(f.sT), base + keep_bytes, ws, stream));
+    f.y = at::empty({B, T, C}, xb.options());
+    times(f.y.view({M, C}), A.ya, C, weight(WO, C, C));
+    return f;
+}
+
+struct MixerBlock : torch::autograd::Function<MixerBlock> {
+    template <class... Ts>
+    static variable_list forward(AutogradContext* ctx, int64_t H, const Tensor& x, const Ts&... params) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Block s{x.size(0), x.size(1), x.size(2), H};
+        const variable_list p{params...};
+        BlockForward f = block_forward(s, x.to(at::kBFloat16).contiguous(), p, true, s.T, Tensor(), Tensor(), at::kBFloat16);
+        ctx->save_for_backward({f.xb, f.weights, f.lnp, f.acts, f.saved});
+        std::vector<int64_t> types{H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
+        for (const auto& t : p) types.push_back((int64_t)t.scalar_type());
+        ctx->saved_data["k"] = types;
+        return {f.y};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto t = ctx->get_saved_variables();
+        const auto types = ctx->saved_data["k"].toIntVector();
+        const Tensor &xb = t[0], &weights = t[1], &lnp = t[2], &acts = t[3], &saved = t[4];
+        const Block s{xb.size(0), xb.size(1), xb.size(2), types[0]};
+        same_interval({{}, (int)types[1], at::kBFloat16, false});
+        c10::DeviceGuard guard(xb.device());
+        at::AutoDispatchBelowADInplaceOrView below;
+        const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
+        const int64_t M = s.rows(), P = s.plane();
+        void* stream = stream_of(xb);
+        const ParamLayout at_(C);
+        const Activations A(s);
+        const Tensor dout = grads[0].contiguous();
+        const Tensor flat = at::empty({at_.at[PARAMS]}, xb.options().dtype(at::kFloat));   // every parameter gradient
+        // gradients of activations: nine planes, reused as they are consumed, and the LoRA columns
+        const int64_t lora = 9 * P;
+        const int64_t o_z = lora, o_a1 = o_z + R_LORA * M, o_ma1 = o_a1 + R_LORA * M, o_mk1 = o_ma1 + R_LORA * M, o_tg1 = o_mk1 + R_LORA * M,
+                      o_tw1 = o_tg1 + R_GATE * M, o_g1 = o_tw1 + R_DECAY * M, o_kkmk = o_g1 + R_GATE * M, o_w1 = o_kkmk + W_KKMK * M,
+                      total = o_w1 + W_DECAY_AAA_MA * M;
+        const Tensor buf = at::empty({total}, xb.options());
+        auto a = [&](int64_t o) -> void* { return at_elem(acts, o); };
+        auto d = [&](int64_t o) -> void* { return at_elem(buf, o); };
+        auto w = [&](int i) -> void* { return at_elem(weights, at_.at[i]); };
+        auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + at_.at[i]; };
+        auto weight = [&](int i, int64_t rows, int64_t cols) { return matrix(weights, at_.at[i], rows, cols); };
+        auto need = [&](int i) { return ctx->needs_input_grad(1 + i); };
+        auto times = [&](int64_t out, int64_t out_cols, int64_t in, int64_t in_cols, const Tensor& wt) {
+            Tensor o = matrix(buf, out, M, out_cols);
+            at::mm_out(o, matrix(buf, in, M, in_cols), wt);
+        };
+        auto plus = [&](int64_t out, int64_t in, int64_t in_cols, const Tensor& wt) {
+            Tensor o = matrix(buf, out, M, C);
+            at::addmm_out(o, o, matrix(buf, in, M, in_cols), wt);
+        };
+        size_t ws_bytes = L.attn_ln_bwd_workspace_bytes(B, T, H, N);
+        ws_bytes = std::max(ws_bytes, L.expand_loras_bwd_workspace_bytes(B, T, C, R_LORA));
+        ws_bytes = std::max(ws_bytes, L.ddlerp_bwd_workspace_bytes(B, T, C, R_MIX));
+        const Tensor ws = scratch_bytes(ws_bytes, xb);
+
+        // planes: 0 dya then dw2, 1 dr, 2 dw, 3 dk', 4 dv, 5 dkk, 6 db, 7 dg, 8 dk
+        {
+            Tensor dya = matrix(buf, 0, M, C);
+            at::mm_out(dya, dout.view({M, C}), weight(WO, C, C));
+            WeightGrads wg;
+            if (need(WO)) wg.add(ptr(dout), C, a(A.ya), C, g(WO));
+            wg.run(M, xb, stream);
+        }
+        check(L.attn_ln_backward(B, T, H, N, WIND_RWKV7_BF16, WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), ptr(lnp),
+                                 d(0), ptr(saved), nullptr, d(2 * P), d(P), d(3 * P), d(4 * P), d(5 * P), d(6 * P), d(7 * P), g(LN_W), nullptr,
+                                 ptr(ws), ws.numel(), stream));
+        check(L.expand_loras_backward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
+                                      w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), d(2 * P), d(3 * P), d(5 * P), d(6 * P), d(0), d(8 * P),
+                                      d(o_z), d(o_a1), d(o_ma1), d(o_mk1), g(KKK_W2), g(AAA_W2), g(MA_W2), g(MK_W2), g(DECAY), g(AAAAA),
+                                      g(MISC_A), g(MISC_K), ptr(ws), ws.numel(), stream));
+        times(o_tg1, R_GATE, 7 * P, C, weight(GATE_W2, C, R_GATE));
+        times(o_tw1, R_DECAY, 0, C, weight(DECAY_W2, C, R_DECAY));
+        {
+            WeightGrads wg;
+            if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
+            if (need(DECAY_W2)) wg.add(d(0), C, a(A.tw1), R_DECAY, g(DECAY_W2));
+            wg.run(M, xb, stream);
+        }
+        Columns cols;
+        cols.add(d(o_z), R_LORA, 0, d(o_kkmk), W_KKMK, 0, R_LORA, 0);
+        cols.add(d(o_mk1), R_LORA, 0, d(o_kkmk), W_KKMK, R_LORA, R_LORA, 0);
+        cols.add(d(o_tw1), R_DECAY, 0, d(o_w1), W_DECAY_AAA_MA, 0, R_DECAY, 2, a(A.tw1));
+        cols.add(d(o_a1), R_LORA, 0, d(o_w1), W_DECAY_AAA_MA, R_DECAY, R_LORA, 0);
+        cols.add(d(o_ma1), R_LORA, 0, d(o_w1), W_DECAY_AAA_MA, R_DECAY + R_LORA, R_LORA, 0);
+        cols.add(d(o_tg1), R_GATE, 0, d(o_g1), R_GATE, 0, R_GATE, 2, a(A.tg1));
+        cols.run(M, stream);
+        // the streams' gradients go to the planes that are free now: 2, 5, 3, 6
+        const int64_t dxrg = 2 * P, dxwa = 5 * P, dxk = 3 * P, dxv = 6 * P;
+        times(dxrg, C, P, C, weight(WR, C, C));
+        plus(dxrg, o_g1, R_GATE, weight(GATE_W1, R_GATE, C));
+        times(dxk, C, 8 * P, C, weight(WK, C, C));
+        plus(dxk, o_kkmk, W_KKMK, weight(KKK_W1, W_KKMK, C));
+        times(dxv, C, 4 * P, C, weight(WV, C, C));
+        times(dxwa, C, o_w1, W_DECAY_AAA_MA, weight(DECAY_W1, W_DECAY_AAA_MA, C));
+        {
+            WeightGrads wg;
+            if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
+            if (need(GATE_W1)) wg.add(d(o_g1), R_GATE, a(A.streams), C, g(GATE_W1));
+            if (need(WK)) wg.add(d(8 * P), C, a(A.streams + 2 * P), C, g(WK));
+            if (need(KKK_W1) || need(MK_W1)) wg.add(d(o_kkmk), W_KKMK, a(A.streams + 2 * P), C, g(KKK_W1));
+            if (need(WV)) wg.add(d(4 * P), C, a(A.streams + 3 * P), C, g(WV));
+            if (need(DECAY_W1) || need(AAA_W1) || need(MA_W1)) wg.add(d(o_w1), W_DECAY_AAA_MA, a(A.streams + P), C, g(DECAY_W1));
+            wg.run(M, xb, stream);
+        }
+        Tensor dx = at::empty_like(xb);
+        check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), d(dxrg), d(dxwa), d(dxk), d(dxv),
+                                ptr(dx), g(MAA_X), g(MAA_W1), g(MAA_W2), g(MAA), ptr(ws), ws.numel(), stream));
+        variable_list out{Tensor(), dx.to((at::ScalarType)types[2])};
+        for (int i = 0; i < PARAMS; i++) {
+            if (!need(i)) {
+                out.emplace_back();
+                continue;
+            }
+            const auto shape = param_shape(i, C);
+            std::vector<int64_t> stride(shape.size());
+            int64_t n = 1;
+            for (size_t k = stride.size(); k-- > 0; n *= shape[k]) stride[k] = n;
+            out.push_back(flat.as_strided(shape, stride, at_.at[i]).to((at::ScalarType)types[3 + i]));
+        }
+        return out;
+    }
+};
+
+template <size_t... I>
+Tensor mixer_node(int64_t H, const Tensor& x, const variable_list& p, std::index_sequence<I...>) {
+    return MixerBlock::apply(H, x, p[I]...)[0];
+}
+
+// The parameters by name out of the module's (and its GroupNorm's) `_parameters`; false where one is missing or not a
+// plain float32 / bf16 tensor of the expected shape on x's device.
+bool mixer_params(const py::dict& own, const py::dict& norm, const Tensor& x, variable_list& out) {
+    static PyObject* names[PARAMS] = {};
+    if (!names[0])
+        for (int i = 0; i < PARAMS; i++) names[i] = PyUnicode_InternFromString(PARAM_NAMES[i]);
+    const int64_t C = x.size(-1);
+    out.clear();
+    out.reserve(PARAMS);
+    for (int i = 0; i < PARAMS; i++) {
+        PyObject* o = PyDict_GetItem((i == LN_W || i == LN_B ? norm : own).ptr(), names[i]);   // (borrowed)
+        if (!o || !THPVariable_Check(o)) return false;
+        const Tensor& t = THPVariable_Unpack(o);
+        if (!plain_param(t, x) || t.sizes() != at::IntArrayRef(param_shape(i, C))) return false;
+        out.push_back(t);
+    }
+    return true;
+}
+bool floating(const Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kDouble;
+}
+
+py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int64_t H, const std::optional<Tensor>& x_prev_,
+                 const std::optional<Tensor>& s0_, bool return_state) {
+    if (!x.defined() || !x.is_cuda() || !floating(x) || x.layout() != at::kStrided || at::isTensorSubclassLike(x) || x.dim() != 3 || H <= 0 ||
+        x.size(2) % H || x.numel() == 0)
+        return py::none();
+    const bool stateful = return_state || x_prev_ || s0_;
+    const int64_t T = x.size(1);
+    const Block s{x.size(0), (T + 15) / 16 * 16, x.size(2), H};
+    if (T % 16 && !stateful) return py::none();
+    if (s.rows() > std::numeric_limits<int>::max() || s.C % 64 || !L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()) ||
+        !L.expand_loras_bwd_workspace_bytes(s.B, s.T, s.C, R_LORA) || !L.ddlerp_bwd_workspace_bytes(s.B, s.T, s.C, R_MIX))
+        return py::none();
+    variable_list p;
+    if (!mixer_params(own, norm, x, p)) return py::none();
+    bool grad = x.requires_grad();
+    for (const auto& t : p) grad = grad || t.requires_grad();
+    grad = grad && at::GradMode::is_enabled();
+    c10::DeviceGuard guard(x.device());
+    if (grad) return stateful ? py::object(py::none()) : py::cast(mixer_node(H, x, p, std::make_index_sequence<PARAMS>()));
+    Tensor x_prev, s0;
+    if (x_prev_) {
+        if (!x_prev_->is_cuda() || x_prev_->device() != x.device() || x_prev_->sizes() != at::IntArrayRef({s.B, s.C})) return py::none();
+        x_prev = x_prev_->to(at::kBFloat16).contiguous();
+    }
+    if (s0_) {
+        s0 = *s0_;
+        if (!(plain(s0, at::kFloat) || plain(s0, at::kBFloat16)) || s0.device() != x.device() ||
+            s0.sizes() != at::IntArrayRef({s.B, s.H, s.N(), s.N()}))
+            return py::none();
+    }
+    Tensor xb = x.to(at::kBFloat16);
+    xb = s.T == T ? xb.contiguous() : at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
+    BlockForward f = block_forward(s, xb, p, false, T, x_prev, s0, s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16);
+    const Tensor y = s.T == T ? f.y : f.y.narrow(1, 0, T).contiguous();
+    if (!return_state) return py::cast(y);
+    return py::make_tuple(y, py::make_tuple(x.select(1, T - 1).clone(), f.sT));
+}
+
+// One token per sequence.  `cache` = (key, 24 bf16 copies, [3,C] float32, workspaces by batch) as the module keeps it;
+// None where it is not there or a parameter has changed since (the caller then remakes it and calls again).
+py::object mixer_step(const Tensor& x, const Tensor& x_prev, const Tensor& S, const py::dict& own, const py::dict& norm, const py::object& cache,
+                      int64_t H) {
+    if (!x.defined() || x.dim() != 2 || !x.is_cuda() || !floating(x) || at::isTensorSubclassLike(x) || !floating(x_prev) ||
+        x_prev.device() != x.device() || x_prev.sizes() != x.sizes() || H <= 0)
+        return py::none();
+    const int64_t B = x.size(0), C = x.size(1);
+    if (!(plain(S, at::kFloat) || plain(S, at::kBFloat16)) || S.device() != x.device() || C != 64 * H ||
+        S.sizes() != at::IntArrayRef({B, H, 64, 64}) || !PyTuple_Check(cache.ptr()) || PyTuple_GET_SIZE(cache.ptr()) != 4)
+        return py::none();
+    variable_list p;
+    if (!mixer_params(own, norm, x, p)) return py::none();
+    PyObject *key = PyTuple_GET_ITEM(cache.ptr(), 0), *copies = PyTuple_GET_ITEM(cache.ptr(), 1);
+    if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != PARAMS || !PyList_Check(copies) || PyList_GET_SIZE(copies) != WEIGHTS) return py::none();
+    for (int i = 0; i < PARAMS; i++) {
+        PyObject* pair = PyTuple_GET_ITEM(key, i);
+        if (PyLong_AsVoidPtr(PyTuple_GET_ITEM(pair, 0)) != p[i].data_ptr() || PyLong_AsLongLong(PyTuple_GET_ITEM(pair, 1)) != (long long)p[i]._version())
+            return py::none();
+    }
+    const void* w[WEIGHTS + 1];
+    static_assert(sizeof(w) == sizeof(wind_rwkv7_mixer_weights), "the enumeration above is the header's order");
+    for (int i = 0; i < WEIGHTS; i++) {
+        PyObject* o = PyList_GET_ITEM(copies, i);
+        if (!THPVariable_Check(o) || THPVariable_Unpack(o).device() != x.device()) return py::none();
+        w[i] = THPVariable_Unpack(o).data_ptr();
+    }
+    w[WEIGHTS] = THPVariable_Unpack(PyTuple_GET_ITEM(cache.ptr(), 2)).data_ptr();
+    wind_rwkv7_mixer_weights weights;
+    memcpy(&weights, w, sizeof(w));
+    c10::DeviceGuard guard(x.device());
+    at::AutoDispatchBelowADInplaceOrView below;
+    // the workspace belongs to the call (the allocator hands the same memory out again on this stream): two threads or
+    // streams stepping one module do not share it
+    const Tensor ws = scratch_bytes(L.mixer_decode_workspace_bytes((int)B, (int)C), x);
+    const Tensor xb = x.to(at::kBFloat16).contiguous(), xp = x_prev.to(at::kBFloat16).contiguous();
+    const Tensor y = at::empty({B, C}, xb.options()), carry = at::empty({B, C}, xb.options());
+    check(L.mixer_decode((int)B, (int)C, (int)H, state_code(S), &weights, ptr(xb), ptr(xp), ptr(S), ptr(y), ptr(carry), ptr(ws), ws.numel(), stream_of(x)));
+    return py::make_tuple(y, py::make_tuple(carry, S));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -499,4 +921,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attn_ln", &attn_ln);
     m.def("ddlerp", &ddlerp);
     m.def("expand_loras", &expand_loras);
+    m.def("mixer", &mixer);
+    m.def("mixer_step", &mixer_step);
 }

@@ -223,8 +223,16 @@ class TimeMixer(nn.Module):
         `state` = (last token of the preceding segment [B,C], WKV7 state [B,H,N,N]) continues a sequence, and
         `return_state=True` returns (y, state) to continue from - a prompt is run in one or several such calls
         and then token by token with `step`.  Either needs attn_impl='cuda' and no autograd, and lifts the
-        reference's restriction of T to multiples of 16 (the tokens after the last full chunk go through `step`)."""
+        reference's restriction of T to multiples of 16.  With the default switches an eager call runs in the native
+        binding, forward and backward as one autograd node (a length that is no multiple of 16 padded with tokens that
+        leave the state alone); what follows here is what torch.compile traces, and every other case (there the tokens
+        after the last full chunk go through `step`)."""
         B, T, C = x.shape
+        if (x.is_cuda and not torch.compiler.is_compiling() and self.attn_impl == 'cuda' and self.use_triton_ddlerp
+                and self._loras_kernel and not (T == 1 and (state is not None or return_state))):   # (one token: `step`)
+            out = _native.binding().mixer(x, self._parameters, self.ln_x._parameters, self.n_head, *(state or (None, None)), return_state)
+            if out is not None:
+                return out
         H, N = self.n_head, self.head_size
         fused = self.use_triton_ddlerp or self.use_triton_loras or self.attn_impl != 'ref'
         dt = torch.bfloat16 if fused else x.dtype          # the all-PyTorch path keeps the caller's precision
@@ -327,7 +335,13 @@ class TimeMixer(nn.Module):
 
     def _step_fused(self, x, x_prev, S):
         """`step` in five launches (wind_rwkv7_mixer_decode): token shift, all first-half products, LoRA second halves
-        with the elementwise tail, the WKV7 step with its epilogue, output projection."""
+        with the elementwise tail, the WKV7 step with its epilogue, output projection.  The native binding makes the call
+        while the kept copies are those of the parameters; else they are remade here first."""
+        for _ in range(2):
+            out = _native.binding().mixer_step(x, x_prev, S, self._parameters, self.ln_x._parameters, self.__dict__.get('_decode_cache'), self.n_head)
+            if out is not None:
+                return out
+            self._decode_weights()
         B, C = x.shape
         _, copies, ln, workspaces = self._decode_weights()
         weights = _native.MixerWeights(*[c.data_ptr() for c in copies], ln.data_ptr())
