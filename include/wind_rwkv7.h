@@ -253,6 +253,14 @@ int wind_rwkv7_mixer_decode(int B, int C, int H, int state_dtype, const wind_rwk
                             const void* x, const void* x_prev, void* state, void* y, void* x_carry,
                             void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same for T tokens per sequence, one after the other on a state that stays in registers: for prompts of a few tokens,
+ * where the sequence kernels' launches are the cost.  x, y: [B,T,C]; x_prev: NULL (zeros) or [B,C]; s0: NULL (zeros) or the
+ * state before, sT: the state after (may be s0 itself); x_carry: NULL or [B,C], the last tokens.
+ * workspace: wind_rwkv7_mixer_decode_workspace_bytes(B*T, C) bytes. */
+int wind_rwkv7_mixer_prompt(int B, int T, int C, int H, int state_dtype, const wind_rwkv7_mixer_weights* weights,
+                            const void* x, const void* x_prev, const void* s0, void* sT, void* y, void* x_carry,
+                            void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- ddlerp: data-dependent token-shift interpolation ------------------------------------------------ */
 
 /* Replaces the Triton kernels behind DDLerp (rwkv7_ddlerp.py:306-336; launches :43-48, :76-83, :132-138,

@@ -1,0 +1,55 @@
+"""The single-token kernels of the block (csrc/mixer_decode.hip) where their dispatch changes: columns and tiles per block of
+the products, rows per block of the head kernel, wavefronts of the first product, and a few tokens per sequence.  Against
+the same step on the sequence kernels, at the gates of tests/test_gpu_time_mixer_state.py (both sides round to bf16 between
+stages; they differ in summation order)."""
+from collections import namedtuple
+
+import pytest
+import torch
+
+from oracle import seq_ref
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _model(H, seed):
+    from wind_rwkv.rwkv7 import TimeMixer
+    gen = torch.Generator().manual_seed(seed)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, 64 * H), 1)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+    return model.to(DEV), gen
+
+
+@pytest.mark.parametrize('B,H', [(2, 1), (17, 12), (47, 12), (80, 12), (200, 12), (3, 20), (300, 3)])
+@pytest.mark.parametrize('state_dtype', [torch.float32, torch.bfloat16])
+def test_step_over_the_dispatch_of_its_kernels(B, H, state_dtype):
+    model, gen = _model(H, seed=B)
+    C = 64 * H
+    x, prev = torch.randn(2, B, C, generator=gen).bfloat16().to(DEV)
+    S = torch.randn(B, H, 64, 64, generator=gen).to(DEV, state_dtype)
+    with torch.no_grad():
+        want, (_, Sw) = model._step_on_kernels(x, prev, S.clone())
+        got, (carry, Sg) = model.step(x, (prev, S.clone()))
+    assert torch.equal(carry, x)
+    assert seq_ref.rel_err(got.float().cpu(), want.float().cpu()) <= 5e-3
+    assert seq_ref.rel_err(Sg.float().cpu(), Sw.float().cpu()) <= (2e-3 if state_dtype == torch.float32 else 8e-3)
+
+
+@pytest.mark.parametrize('B,T,H', [(1, 3, 2), (5, 17, 3), (8, 63, 12)])
+def test_a_few_tokens_equal_as_many_steps(B, T, H):
+    """Within one rounding of the outputs: the same kernels' arithmetic, the state in registers between the tokens (fp32)."""
+    model, gen = _model(H, seed=T)
+    x = torch.randn(B, T, 64 * H, generator=gen).bfloat16().to(DEV)
+    state = (torch.randn(B, 64 * H, generator=gen).bfloat16().to(DEV), torch.randn(B, H, 64, 64, generator=gen).to(DEV))
+    with torch.no_grad():
+        y, (last, S) = model(x, state=state, return_state=True)
+        st, ys = (state[0], state[1].clone()), []
+        for t in range(T):
+            yt, st = model.step(x[:, t], st)
+            ys.append(yt)
+    assert torch.equal(last, x[:, -1])
+    assert seq_ref.rel_err(y.float().cpu(), torch.stack(ys, 1).float().cpu()) <= 2e-3
+    assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4

@@ -517,7 +517,29 @@ int wind_rwkv7_mixer_decode(int B, int C, int H, int state_dtype, const wind_rwk
     static_assert(sizeof(wkv::MixerWeights) == sizeof(wind_rwkv7_mixer_weights), "the two declarations list the same pointers");
     wkv::MixerWeights mw;
     memcpy(&mw, weights, sizeof(mw));
-    wkv::launch_mixer_decode(B, C, H, state_dtype == WIND_RWKV7_F32, mw, x, x_prev, state, y, x_carry, workspace,
+    wkv::launch_mixer_decode(B, 1, C, H, state_dtype == WIND_RWKV7_F32, mw, x, x_prev, state, state, y, x_carry, workspace,
+                             static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
+int wind_rwkv7_mixer_prompt(int B, int T, int C, int H, int state_dtype, const wind_rwkv7_mixer_weights* weights, const void* x,
+                            const void* x_prev, const void* s0, void* sT, void* y, void* x_carry, void* workspace,
+                            size_t workspace_bytes, void* stream) {
+    if (B <= 0 || T <= 0 || (long long)B * T > (1 << 24)) return WIND_RWKV7_ERR_BAD_SHAPE;
+    int rc = check_mixer_decode(B * T, C, H);
+    if (rc) return rc;
+    rc = check_dtypes(WIND_RWKV7_BF16, state_dtype);
+    if (rc) return rc;
+    if (!weights || !x || !sT || !y) return WIND_RWKV7_ERR_NULL_POINTER;   // (x_prev, s0, x_carry may be null)
+    if (x_carry && x_carry == x_prev) return WIND_RWKV7_ERR_BAD_SHAPE;
+    const void* const* wp = reinterpret_cast<const void* const*>(weights);
+    for (size_t i = 0; i < sizeof(*weights) / sizeof(void*); i++)
+        if (!wp[i]) return WIND_RWKV7_ERR_NULL_POINTER;
+    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_mixer_decode_workspace_bytes(B * T, C));
+    if (rc) return rc;
+    wkv::MixerWeights mw;
+    memcpy(&mw, weights, sizeof(mw));
+    wkv::launch_mixer_decode(B, T, C, H, state_dtype == WIND_RWKV7_F32, mw, x, x_prev, s0, sT, y, x_carry, workspace,
                              static_cast<hipStream_t>(stream));
     return launch_status();
 }

@@ -1,24 +1,29 @@
-// One token per sequence through the whole RWKV-7 time mixer (decoding), for gfx950: five launches.
+// One token per sequence, or a few, through the whole RWKV-7 time mixer (decoding, short prompts), for gfx950: four launches.
 //
 // The reference's block has no single-token form: its forward (time_mixer.py:96-167) is the specification, taken at
 // T = 1 with the previous token and the WKV7 state carried by the caller.  A step through the sequence kernels is some
 // twenty launches of kernels built for thousands of tokens, each waiting out its own launch and drain; here the B
-// tokens are the rows of 16-row tiles (rows past B are zero and never stored) and every stage is a kernel whose grid
-// is as wide as the stage's OUTPUT, so the weights (6 MB) stream once through many compute units:
-//   1. mix      the four token-shifted streams (rwkv7_ddlerp.py:20-84): one block per tile, a wavefront per 64
-//               channels, the contraction over the channels added in LDS
+// tokens are the rows of 16-row tiles (rows past B are zero or repeats and never stored) and every stage is a kernel
+// whose grid is as wide as the stage's OUTPUT, so the weights (6 MB) stream once through many compute units:
+//   1. mid      the token shift's first product with tanh (rwkv7_ddlerp.py:20-49), 16 of its 128 columns per block
 //   2. linear   all first-half products (time_mixer.py:120-131) - r, k, v and the six LoRA first halves, nine weight
-//               matrices - in one launch: a block per 16 output columns, its wavefronts splitting the contraction
-//   3. expand   the LoRA second halves with the elementwise tail (rwkv7_expand_loras.py:33-70) and the gate's and the
-//               decay's second halves, one wavefront per (tile, head)
-//   4. the single-token WKV7 recurrence with GroupNorm, bonus and gate (wkv7_decode.hip)
-//   5. linear   the output projection
+//               matrices - in one launch; a block computes the interpolated stream (rwkv7_ddlerp.py:53-84) it multiplies
+//               itself, 32 channels at a time, so the four streams never exist in memory
+//   3. head     per (tile, head): the LoRA second halves with the elementwise tail (rwkv7_expand_loras.py:33-70), the gate's
+//               and the decay's second halves, then the single-token WKV7 recurrence with GroupNorm, bonus and gate
+//   4. linear   the output projection
 // Rounding follows the sequence path: every tensor that path keeps in bf16 between its kernels is rounded to bf16
 // here at the same place.
+//
+// At B = 1 every stage is bound by its launch, one trip to memory and its drain, so what counts is how few stages there
+// are and that no stage leaves its loads to a few compute units.  (Five stages with the whole token shift in the ONE
+// block of the tile: 18.4 us for that block to fetch 400 KB, 39.8 us per step at 768 channels.)
 #include "mixer_decode_kernels.hpp"
 
+#include "device_info.hpp"
 #include "frag.hpp"
-#include "wkv7_kernels.hpp"
+#include "ln_epilogue.hpp"
+#include "wkv7_common.hpp"
 
 namespace wkv {
 
@@ -46,130 +51,125 @@ __device__ __forceinline__ bf16x8 cat8(bf16x4 a, bf16x4 b) { return __builtin_sh
 // load each): the order of the summed index is free as long as the operands agree.
 
 // ------------------------------------------------------------------------------------------------
-// 1. mix: y_k = x + xx (tanh((x + xx alpha) L^T)_k R_k^T + beta_k),  xx = x_prev - x
+// 1. mid = tanh((x + xx alpha) L^T),  xx = x_prev - x.  Block = 16 of the 128 columns x one 16-row tile; its NW wavefronts
+// take every NW-th 32-channel step of the contraction.
 // ------------------------------------------------------------------------------------------------
-constexpr int MIX_MAX_WAVES = 12;   // one wavefront per 64-channel block up to C = 768; 8 KiB of partial sums each
-__global__ __launch_bounds__(64 * MIX_MAX_WAVES) void decode_mix_kernel(int B, int Bp, int C, const __bf16* __restrict__ x,
-                                                         const __bf16* __restrict__ x_prev,
-                                                         const __bf16* __restrict__ alpha, const __bf16* __restrict__ beta,
-                                                         const __bf16* __restrict__ Lw, const __bf16* __restrict__ R,
-                                                         __bf16* __restrict__ streams, __bf16* __restrict__ x_carry) {
-    constexpr int NOB = 4 * R_MIX / 16;               // 8 blocks of 16 mid values
-    __shared__ f32x4 part[MIX_MAX_WAVES][NOB][WAVE];  // the wavefronts' partial sums of the first product
-    __shared__ __attribute__((aligned(16))) __bf16 s_bm[4][WAVE * 8];   // tanh(...)_k as the second product's operand
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    const Lane L;
-    const int row = blockIdx.x * TOK + L.n;
-    const bool valid = row < B;
-    const long xrow = (long)(valid ? row : B - 1) * C;
-    const int ncb = C / 64;
+constexpr int MID = 4 * R_MIX;
 
-    f32x4 acc[NOB];
+struct MixIn {   // the token shift's operands
+    const __bf16 *x, *x_prev;   // [B*T, C]; [B, C], the tokens before the sequences' first (null: zeros)
+    const __bf16 *R, *beta;     // [4, C, 32], [4, C]
+    __bf16* mid;                // [rows padded to 16, 128]
+    int rows, T;                // B*T, tokens per sequence
+};
+// A lane's row of x (a row past the last repeats it) and the row before it; at a sequence's start without x_prev the row
+// itself is loaded and `zero` says to take zeros.
+struct TokenRows {
+    long at, prev;         // element offsets: into x, and into x or x_prev
+    const __bf16* prev_of;
+    bool zero;
+};
+__device__ __forceinline__ TokenRows token_rows(const MixIn& in, int row, int C) {
+    const int m = row < in.rows ? row : in.rows - 1;
+    const int seq = m / in.T;
+    TokenRows r;
+    r.at = (long)m * C;
+    const bool start = m == seq * in.T;
+    r.zero = start && in.x_prev == nullptr;
+    r.prev_of = start && in.x_prev != nullptr ? in.x_prev : in.x;
+    r.prev = start ? (in.x_prev != nullptr ? (long)seq * C : r.at) : r.at - C;
+    return r;
+}
+__device__ __forceinline__ bf16x8 or_zero(bf16x8 v, bool zero) { return zero ? bf16x8{} : v; }
+
+template <int NW, int U>   // wavefronts, and steps of a wavefront in flight at a time
+__global__ __launch_bounds__(64 * NW) void decode_mid_kernel(const MixIn in, int C, const __bf16* __restrict__ alpha,
+                                                         const __bf16* __restrict__ Lw, __bf16* __restrict__ x_carry) {
+    __shared__ f32x4 part[NW][WAVE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const Lane L;
+    const int ob = blockIdx.x, row = blockIdx.y * TOK + L.n;
+    const TokenRows tr = token_rows(in, row, C);
+    const __bf16 *xrow = in.x + tr.at + 8 * L.g, *prow = tr.prev_of + tr.prev + 8 * L.g;
+    const __bf16* lrow = Lw + (long)(16 * ob + L.n) * C + 8 * L.g;   // lane = mid index
+    f32x4 acc0 = zero4(), acc1 = zero4();
+    const int nk = C / 32;
+    for (int s0 = wave; s0 < nk; s0 += NW * U) {   // U steps of this wavefront at a time, all loads before the products
+        bf16x8 xc[U], xp[U], al[U], lw[U];
 #pragma unroll
-    for (int ob = 0; ob < NOB; ob++) acc[ob] = zero4();
-    for (int cb = wave; cb < ncb; cb += nw) {
-        // every load of the channel block is issued before the first product (left to itself the compiler loads
-        // each weight fragment right before its use and waits for it: sixteen memory latencies in a row)
-        bf16x8 xc[2], xp[2], al[2], lw[2][NOB];
-#pragma unroll
-        for (int pr = 0; pr < 2; pr++) {
-            const int c = 64 * cb + 32 * pr + 8 * L.g;
-            xc[pr] = *reinterpret_cast<const bf16x8*>(x + xrow + c);
-            xp[pr] = *reinterpret_cast<const bf16x8*>(x_prev + xrow + c);
-            al[pr] = *reinterpret_cast<const bf16x8*>(alpha + c);
-#pragma unroll
-            for (int ob = 0; ob < NOB; ob++) lw[pr][ob] = *reinterpret_cast<const bf16x8*>(Lw + (long)(16 * ob + L.n) * C + c);   // lane = mid index
+        for (int u = 0; u < U; u++) {
+            const int c = 32 * (s0 + NW * u < nk ? s0 + NW * u : s0);   // (past the end: the first step again, not used)
+            xc[u] = *reinterpret_cast<const bf16x8*>(xrow + c);
+            xp[u] = *reinterpret_cast<const bf16x8*>(prow + c);
+            al[u] = *reinterpret_cast<const bf16x8*>(alpha + c + 8 * L.g);
+            lw[u] = *reinterpret_cast<const bf16x8*>(lrow + c);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int pr = 0; pr < 2; pr++) {
+        for (int u = 0; u < U; u++) {
+            if (s0 + NW * u >= nk) break;
             // the interpolated input as a bf16 pair (hi + lo), as the sequence kernel has it: it feeds tanh', which
             // is steep, and must not be rounded to 8 bits before the C-term sum
             bf16x4 h[2], l[2];
+            xp[u] = or_zero(xp[u], tr.zero);
 #pragma unroll
             for (int hf = 0; hf < 2; hf++) {
-                const f32x4 cv = to_f32(hf ? hi4(xc[pr]) : lo4(xc[pr]));
-                const f32x4 av = cv + (to_f32(hf ? hi4(xp[pr]) : lo4(xp[pr])) - cv) * to_f32(hf ? hi4(al[pr]) : lo4(al[pr]));
+                const f32x4 cv = to_f32(hf ? hi4(xc[u]) : lo4(xc[u]));
+                const f32x4 av = cv + (to_f32(hf ? hi4(xp[u]) : lo4(xp[u])) - cv) * to_f32(hf ? hi4(al[u]) : lo4(al[u]));
                 h[hf] = to_bf16(av);
                 l[hf] = to_bf16(av - to_f32(h[hf]));
             }
-            const bf16x8 a_hi = cat8(h[0], h[1]), a_lo = cat8(l[0], l[1]);
-#pragma unroll
-            for (int ob = 0; ob < NOB; ob++) {
-                acc[ob] = mma8(acc[ob], lw[pr][ob], a_hi);   // lane = token
-                acc[ob] = mma8(acc[ob], lw[pr][ob], a_lo);
-            }
+            acc0 = mma8(acc0, lw[u], cat8(h[0], h[1]));   // lane = token
+            acc1 = mma8(acc1, lw[u], cat8(l[0], l[1]));
         }
     }
-#pragma unroll
-    for (int ob = 0; ob < NOB; ob++) part[wave][ob][lane] = acc[ob];
-    __syncthreads();
-    // wavefront w < 8 adds block w in a fixed order, applies tanh and files the result where the second product's lane
-    // group 2(ob&1) + (g>>1) of interpolation k = ob/2 looks for mid indices 8g' .. 8g'+7
-    if (wave < NOB) {
-        const int ob = wave;
-        f32x4 s = part[0][ob][lane];
-        for (int w = 1; w < nw; w++) s += part[w][ob][lane];
-        f32x4 t;
-#pragma unroll
-        for (int r = 0; r < 4; r++) t[r] = tanhf_(s[r]);
-        const int k = ob >> 1, gq = 2 * (ob & 1) + (L.g >> 1);
-        *reinterpret_cast<bf16x4*>(&s_bm[k][(16 * gq + L.n) * 8 + 4 * (L.g & 1)]) = to_bf16(t);
+    part[wave][lane] = acc0 + acc1;
+    // the tokens to hand on, the last of each sequence: dealt over all blocks
+    if (x_carry) {
+        const int per_row = C / 8, nseq = in.rows / in.T;
+        const int step = gridDim.x * gridDim.y * 64 * NW;
+        for (int v = (blockIdx.y * gridDim.x + ob) * 64 * NW + threadIdx.x; v < nseq * per_row; v += step) {
+            const int seq = v / per_row, c = 8 * (v - seq * per_row);
+            *reinterpret_cast<bf16x8*>(x_carry + (long)seq * C + c) =
+                *reinterpret_cast<const bf16x8*>(in.x + ((long)seq * in.T + in.T - 1) * C + c);
+        }
     }
     __syncthreads();
-    bf16x8 bm[4];
+    if (wave != 0) return;
+    f32x4 t = part[0][lane];   // lane = token, reg = column 4g + r
 #pragma unroll
-    for (int k = 0; k < 4; k++) bm[k] = *reinterpret_cast<const bf16x8*>(&s_bm[k][lane * 8]);
-    for (int cb = wave; cb < ncb; cb += nw) {
-        bf16x8 rw[4][4];      // [s][k]: lane = channel
-        bf16x4 xq[4], xpq[4], bq[4][4];
+    for (int w = 1; w < NW; w++) t += part[w][lane];
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int c = 64 * cb + 16 * s;
-            xq[s] = *reinterpret_cast<const bf16x4*>(x + xrow + c + 4 * L.g);
-            xpq[s] = *reinterpret_cast<const bf16x4*>(x_prev + xrow + c + 4 * L.g);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                rw[s][k] = *reinterpret_cast<const bf16x8*>(R + ((long)k * C + c + L.n) * R_MIX + 8 * L.g);
-                bq[s][k] = *reinterpret_cast<const bf16x4*>(beta + (long)k * C + c + 4 * L.g);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int c = 64 * cb + 16 * s;
-            const f32x4 xv = to_f32(xq[s]);
-            const f32x4 xxv = to_f32(xpq[s]) - xv;
-            if (x_carry && valid) *reinterpret_cast<bf16x4*>(x_carry + (long)row * C + c + 4 * L.g) = xq[s];   // the next step's x_prev
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const f32x4 coef = mma8(to_f32(bq[s][k]), rw[s][k], bm[k]);   // lane = token
-                const bf16x4 y = valid ? to_bf16(xv + xxv * coef) : bf16x4{};
-                *reinterpret_cast<bf16x4*>(streams + ((long)k * Bp + row) * C + c + 4 * L.g) = y;
-            }
-        }
-    }
+    for (int r = 0; r < 4; r++) t[r] = tanhf_(t[r]);
+    *reinterpret_cast<bf16x4*>(in.mid + (long)row * MID + 16 * ob + 4 * L.g) = to_bf16(t);
 }
 
 // ------------------------------------------------------------------------------------------------
-// 2./5. linear: out_s = in_s W_s^T for up to nine (input, weight) pairs.  Block = 16 output columns of one pair
-// x one 16-row tile; its four wavefronts take every fourth 32-channel step of the contraction.
+// 2./4. linear: out_s = in_s W_s^T for up to nine (input, weight) pairs.  Block = CB x 16 output columns of one pair
+// x RT 16-row tiles; its four wavefronts take every fourth 32-channel step of the contraction.  LERP: the input is the
+// pair's token-shifted stream y_k = x + xx (mid_k R_k^T + beta_k), made 32 channels at a time where it is multiplied (one
+// row of R per lane, ordered so that the two 16-channel results are the lane's eight contiguous channels 8g .. 8g+7).
+// Every column block repeats that for its stream, so few columns per block where the launch is latency (a tile or two),
+// four and two tiles at a time where the work counts.
 // ------------------------------------------------------------------------------------------------
 struct LinSeg {
-    const __bf16* in;    // [Bp, C]
+    const __bf16* in;    // [Bp, C] (not LERP)
     const __bf16* W;     // [N, C]
     __bf16* out;         // [rows, N]
     int N;               // multiple of 16
     int tanh_out;        // the output is tanh of the (bf16-rounded) product
+    int stream;          // LERP: which interpolation
 };
 constexpr int MAX_SEGS = 9;
 struct LinArgs {
     LinSeg seg[MAX_SEGS];
-    int nseg, C, rows;   // rows: output rows that exist (stores beyond are dropped)
+    int nseg, C, rows, ntiles;   // rows: output rows that exist (stores beyond are dropped)
 };
 
-__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A) {
-    __shared__ f32x4 part[4][WAVE];
+template <bool LERP, int CB, int RT>
+__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, const MixIn mix) {
+    constexpr int NW = 4;
+    __shared__ f32x4 part[NW][RT][CB][WAVE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const Lane L;
     // which pair this block belongs to (the descriptor fields through scalar selects, not an indexed copy of the
@@ -178,12 +178,12 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A) {
     const __bf16* __restrict__ in = nullptr;
     const __bf16* __restrict__ W = nullptr;
     __bf16* __restrict__ out = nullptr;
-    int N = 0, act = 0;
+    int N = 0, act = 0, ks = 0;
     bool found = false;
 #pragma unroll
     for (int i = 0; i < MAX_SEGS; i++) {
         if (!found && i < A.nseg) {
-            const int nb = A.seg[i].N / 16;
+            const int nb = (A.seg[i].N + 16 * CB - 1) / (16 * CB);
             if (blk < nb) {
                 found = true;
                 in = A.seg[i].in;
@@ -191,6 +191,7 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A) {
                 out = A.seg[i].out;
                 N = A.seg[i].N;
                 act = A.seg[i].tanh_out;
+                ks = A.seg[i].stream;
             } else {
                 blk -= nb;
             }
@@ -198,149 +199,341 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A) {
     }
     if (!found) return;   // (whole block; the grid is exactly the sum of the pairs' blocks)
     const int C = A.C;
-    const int row = blockIdx.y * TOK + L.n;
-    const __bf16* wrow = W + (long)(16 * blk + L.n) * C + 8 * L.g;   // lane = output column
-    const __bf16* irow = in + (long)row * C + 8 * L.g;               // lane = token
-    f32x4 acc0 = zero4(), acc1 = zero4();
-    const int nk = C / 32;
-    for (int s0 = wave; s0 < nk; s0 += 32) {   // eight steps of this wavefront at a time, all loads before the products
-        bf16x8 wv[8], iv[8];
+    const int col0 = 16 * CB * blk;
+    int trow[RT];       // this lane's row of each tile (a tile past the last repeats it and is not stored)
+    const __bf16 *irow[RT], *prow[RT];
+    bf16x8 bm[RT];
+    bool zero[RT];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int s = s0 + 4 * u < nk ? s0 + 4 * u : s0;   // (past the end: the first step again, not used)
-            wv[u] = *reinterpret_cast<const bf16x8*>(wrow + 32 * s);
-            iv[u] = *reinterpret_cast<const bf16x8*>(irow + 32 * s);
+    for (int t = 0; t < RT; t++) {
+        const int tile = blockIdx.y * RT + t < (unsigned)A.ntiles ? blockIdx.y * RT + t : A.ntiles - 1;
+        trow[t] = tile * TOK + L.n;
+        if constexpr (LERP) {
+            const TokenRows tr = token_rows(mix, trow[t], C);
+            irow[t] = mix.x + tr.at + 8 * L.g;
+            prow[t] = tr.prev_of + tr.prev + 8 * L.g;
+            zero[t] = tr.zero;
+            bm[t] = *reinterpret_cast<const bf16x8*>(mix.mid + (long)trow[t] * MID + R_MIX * ks + 8 * L.g);
+        } else {
+            irow[t] = in + (long)trow[t] * C + 8 * L.g;
+        }
+    }
+    const __bf16* wrow[CB];   // lane = output column
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) wrow[cb] = W + (long)((col0 + 16 * cb < N ? col0 + 16 * cb : col0) + L.n) * C + 8 * L.g;
+    // row j of the step's two R fragments: channel 8(n/4) + 4j + n%4
+    const __bf16* rrow = LERP ? mix.R + ((long)ks * C + 8 * (L.n >> 2) + (L.n & 3)) * R_MIX + 8 * L.g : nullptr;
+    const __bf16* brow = LERP ? mix.beta + (long)ks * C + 8 * L.g : nullptr;
+    f32x4 acc[RT][CB];
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++) acc[t][cb] = zero4();
+    const int nk = C / 32;
+    constexpr int U = CB * RT == 1 ? 6 : CB * RT <= 4 ? 3 : 2;
+    for (int s0 = wave; s0 < nk; s0 += NW * U) {   // U steps of this wavefront at a time, all loads before the products
+        bf16x8 wv[U][CB], iv[U][RT], pv[U][RT], r0[U], r1[U], be[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int s = s0 + NW * u < nk ? s0 + NW * u : s0;   // (past the end: the first step again, not used)
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) wv[u][cb] = *reinterpret_cast<const bf16x8*>(wrow[cb] + 32 * s);
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+                iv[u][t] = *reinterpret_cast<const bf16x8*>(irow[t] + 32 * s);
+                if constexpr (LERP) pv[u][t] = *reinterpret_cast<const bf16x8*>(prow[t] + 32 * s);
+            }
+            if constexpr (LERP) {
+                r0[u] = *reinterpret_cast<const bf16x8*>(rrow + (long)32 * s * R_MIX);
+                r1[u] = *reinterpret_cast<const bf16x8*>(rrow + (long)(32 * s + 4) * R_MIX);
+                be[u] = *reinterpret_cast<const bf16x8*>(brow + 32 * s);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < 8; u += 2) {
-            if (s0 + 4 * u < nk) acc0 = mma8(acc0, wv[u], iv[u]);
-            if (s0 + 4 * (u + 1) < nk) acc1 = mma8(acc1, wv[u + 1], iv[u + 1]);
+        for (int u = 0; u < U; u++) {
+            if (s0 + NW * u >= nk) break;
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+                if constexpr (LERP) {
+                    const f32x4 c0 = mma8(to_f32(lo4(be[u])), r0[u], bm[t]);   // lane = token, channels 8g + r
+                    const f32x4 c1 = mma8(to_f32(hi4(be[u])), r1[u], bm[t]);   // channels 8g + 4 + r
+                    pv[u][t] = or_zero(pv[u][t], zero[t]);
+                    const f32x4 x0 = to_f32(lo4(iv[u][t])), x1 = to_f32(hi4(iv[u][t]));
+                    iv[u][t] = cat8(to_bf16(x0 + (to_f32(lo4(pv[u][t])) - x0) * c0), to_bf16(x1 + (to_f32(hi4(pv[u][t])) - x1) * c1));
+                }
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++) acc[t][cb] = mma8(acc[t][cb], wv[u][cb], iv[u][t]);
+            }
         }
     }
-    part[wave][lane] = acc0 + acc1;
-    __syncthreads();
-    if (wave != 0) return;
-    f32x4 r = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);   // lane = token, reg = column 4g + r
-    if (act) {
-        r = to_f32(to_bf16(r));
 #pragma unroll
-        for (int q = 0; q < 4; q++) r[q] = tanhf_(r[q]);
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++) part[wave][t][cb][lane] = acc[t][cb];
+    __syncthreads();
+    for (int o = wave; o < RT * CB; o += NW) {   // a wavefront finishes a 16 x 16 result
+        const int t = o / CB, cb = o % CB;
+        f32x4 r = part[0][t][cb][lane];   // lane = token, reg = column 4g + r
+#pragma unroll
+        for (int w = 1; w < NW; w++) r += part[w][t][cb][lane];
+        if (act) {
+            r = to_f32(to_bf16(r));
+#pragma unroll
+            for (int q = 0; q < 4; q++) r[q] = tanhf_(r[q]);
+        }
+        const int row = (blockIdx.y * RT + t) * TOK + L.n;
+        if (row < A.rows && col0 + 16 * cb < N) *reinterpret_cast<bf16x4*>(out + (long)row * N + col0 + 16 * cb + 4 * L.g) = to_bf16(r);
     }
-    if (row < A.rows) *reinterpret_cast<bf16x4*>(out + (long)row * N + 16 * blk + 4 * L.g) = to_bf16(r);
 }
 
 // ------------------------------------------------------------------------------------------------
-// 3. expand: one wavefront per (16-row tile, head of 64 channels)
+// 3. head: per head of 64 channels and 16 tokens, by four wavefronts (16 channels each)
 //     g  = tanh(g1) Wg2^T ;   w2 = tanh(w1) Ww2^T ;   w = -softplus(-(w_bias + w2)) - 0.5
 //     z  = tanh(kk1) Wz^T + k ;   kk = z / sqrt(max(sum_head z^2, 1e-12))
 //     a  = sigmoid(a1 Wa^T + a_bias) ;  ma, mk likewise ;   k' = k (ma + a - ma a) exp(w mk) ;   b = -kk a
+// with the results as bf16 in LDS (the decay exp(-exp(w)) of the rounded w in fp32); then per token, a wavefront per 16 value
+// rows of the state,
+//     sa = S kk ;   S <- S diag(exp(-exp(w))) + sa b^T + v k'^T ;   y = S r ;   out = g (groupnorm(y) + (sum r k' bonus) v)
 // ------------------------------------------------------------------------------------------------
-struct ExpandArgs {
-    int Bp, C;
-    const __bf16 *k, *tg1, *tw1, *kk1, *mk1, *a1, *ma1;                 // [Bp, C], [Bp, 128], [Bp, 64], 4 x [Bp, 16]
+struct HeadArgs {
+    int rows, T, C, H, state_f32;                                         // rows = B*T
+    const __bf16 *r, *k, *v;                                              // [rows padded to 16, C]
+    const __bf16 *tg1, *tw1, *kk1, *mk1, *a1, *ma1;                       // likewise x 128, 64, 4 times 16
     const __bf16 *gate_w2, *decay_w2, *kkk_w2, *aaa_w2, *ma_w2, *mk_w2;   // [C, rank]
     const __bf16 *time_decay, *time_aaaaa, *time_misc_a, *time_misc_k;   // [C]
-    __bf16 *w, *k2, *kk, *b, *g;                                          // [Bp, C]
+    const float* ln_params;                                               // [3, C]
+    const void* state_in;                                                 // [B, H, 64, 64], null: zeros
+    void* state;                                                          // may be state_in itself
+    __bf16* ya;                                                           // [rows padded to 16, C]
+};
+struct HeadTile {   // 16 tokens of a head
+    static constexpr int LD = HEAD + 8, LF = HEAD + 4;   // (row pitches: 16 bytes off a multiple of the bank width)
+    __attribute__((aligned(16))) __bf16 r[TOK][LD], v[TOK][LD], k[TOK][LD], kk[TOK][LD], b[TOK][LD], g[TOK][LD];
+    __attribute__((aligned(16))) float decay[TOK][LF];
+    float ss[NBLK][TOK], y[TOK][HEAD];
 };
 
-__global__ __launch_bounds__(64) void decode_expand_kernel(const ExpandArgs A) {
-    const Lane L;
-    const int h = blockIdx.x;
-    const int row = blockIdx.y * TOK + L.n;
-    const int C = A.C;
-    bf16x8 tg1[R_GATE / 32], tw1[R_DECAY / 32];
+// The tile's operands into LDS: token n of the tile is row first + n (past `last`: row `last` again).  The first 256 threads
+// load r and v, the first four wavefronts expand; every wavefront of the block takes part in the barriers.
+__device__ __forceinline__ void expand_tile(HeadTile& s, const HeadArgs& A, int h, int first, int last, int wave, const Lane& L) {
+    const int C = A.C, ib = wave & 3;
+    if (threadIdx.x < 256) {   // 16 bytes per thread
+        const int t = threadIdx.x & 127, n = t >> 3, c = 8 * (t & 7);
+        const __bf16* src = threadIdx.x < 128 ? A.r : A.v;
+        __bf16(*dst)[HeadTile::LD] = threadIdx.x < 128 ? s.r : s.v;
+        *reinterpret_cast<bf16x8*>(&dst[n][c]) =
+            *reinterpret_cast<const bf16x8*>(src + (long)(first + n < last ? first + n : last) * C + h * HEAD + c);
+    }
+    f32x4 z, av;
+    if (wave < 4) {
+        const int row = first + L.n < last ? first + L.n : last, c = h * HEAD + 16 * ib;   // lane n: token as an operand's row; channel c + n as a weight row
+        bf16x8 tg1[R_GATE / 32], tw1[R_DECAY / 32], gw[R_GATE / 32], dw[R_DECAY / 32];
+        // every load before the first product (else each weight fragment is loaded right before its use and waited for)
 #pragma unroll
-    for (int j = 0; j < R_GATE / 32; j++) tg1[j] = *reinterpret_cast<const bf16x8*>(A.tg1 + (long)row * R_GATE + 32 * j + 8 * L.g);
+        for (int j = 0; j < R_GATE / 32; j++) {
+            tg1[j] = *reinterpret_cast<const bf16x8*>(A.tg1 + (long)row * R_GATE + 32 * j + 8 * L.g);
+            gw[j] = *reinterpret_cast<const bf16x8*>(A.gate_w2 + (long)(c + L.n) * R_GATE + 32 * j + 8 * L.g);
+        }
 #pragma unroll
-    for (int j = 0; j < R_DECAY / 32; j++) tw1[j] = *reinterpret_cast<const bf16x8*>(A.tw1 + (long)row * R_DECAY + 32 * j + 8 * L.g);
-    auto act16 = [&](const __bf16* p) { return *reinterpret_cast<const bf16x4*>(p + (long)row * 16 + 4 * L.g); };
-    bf16x4 tz;
-    {
-        f32x4 t = to_f32(act16(A.kk1));
+        for (int j = 0; j < R_DECAY / 32; j++) {
+            tw1[j] = *reinterpret_cast<const bf16x8*>(A.tw1 + (long)row * R_DECAY + 32 * j + 8 * L.g);
+            dw[j] = *reinterpret_cast<const bf16x8*>(A.decay_w2 + (long)(c + L.n) * R_DECAY + 32 * j + 8 * L.g);
+        }
+        auto act16 = [&](const __bf16* p) { return *reinterpret_cast<const bf16x4*>(p + (long)row * 16 + 4 * L.g); };
+        auto w16 = [&](const __bf16* W) { return *reinterpret_cast<const bf16x4*>(W + (long)(c + L.n) * 16 + 4 * L.g); };
+        auto bias4 = [&](const __bf16* p) { return *reinterpret_cast<const bf16x4*>(p + c + 4 * L.g); };
+        const bf16x4 kk1 = act16(A.kk1), a1 = act16(A.a1), ma1 = act16(A.ma1), mk1 = act16(A.mk1);
+        const bf16x4 wz = w16(A.kkk_w2), wa = w16(A.aaa_w2), wma = w16(A.ma_w2), wmk = w16(A.mk_w2);
+        const bf16x4 bd = bias4(A.time_decay), ba = bias4(A.time_aaaaa), bma = bias4(A.time_misc_a), bmk = bias4(A.time_misc_k);
+        const bf16x4 kq = *reinterpret_cast<const bf16x4*>(A.k + (long)row * C + c + 4 * L.g);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 t = to_f32(kk1);
 #pragma unroll
         for (int q = 0; q < 4; q++) t[q] = tanhf_(t[q]);
-        tz = to_bf16(t);
-    }
-    const bf16x4 a1 = act16(A.a1), ma1 = act16(A.ma1), mk1 = act16(A.mk1);
-
-    // every weight fragment of the head is requested before the first product (else each is loaded right before its
-    // use and waited for)
-    bf16x8 gw[NBLK][R_GATE / 32], dw[NBLK][R_DECAY / 32];
-    bf16x4 wz[NBLK], wa[NBLK], wma[NBLK], wmk[NBLK], bias[NBLK][4], kq[NBLK];
-#pragma unroll
-    for (int cb = 0; cb < NBLK; cb++) {
-        const int c = h * HEAD + 16 * cb;            // lane n: channel c + n as a weight row; column 4g + r of the result
-#pragma unroll
-        for (int j = 0; j < R_GATE / 32; j++)
-            gw[cb][j] = *reinterpret_cast<const bf16x8*>(A.gate_w2 + (long)(c + L.n) * R_GATE + 32 * j + 8 * L.g);
-#pragma unroll
-        for (int j = 0; j < R_DECAY / 32; j++)
-            dw[cb][j] = *reinterpret_cast<const bf16x8*>(A.decay_w2 + (long)(c + L.n) * R_DECAY + 32 * j + 8 * L.g);
-        auto w16 = [&](const __bf16* W) { return *reinterpret_cast<const bf16x4*>(W + (long)(c + L.n) * 16 + 4 * L.g); };
-        wz[cb] = w16(A.kkk_w2);
-        wa[cb] = w16(A.aaa_w2);
-        wma[cb] = w16(A.ma_w2);
-        wmk[cb] = w16(A.mk_w2);
-        bias[cb][0] = *reinterpret_cast<const bf16x4*>(A.time_decay + c + 4 * L.g);
-        bias[cb][1] = *reinterpret_cast<const bf16x4*>(A.time_aaaaa + c + 4 * L.g);
-        bias[cb][2] = *reinterpret_cast<const bf16x4*>(A.time_misc_a + c + 4 * L.g);
-        bias[cb][3] = *reinterpret_cast<const bf16x4*>(A.time_misc_k + c + 4 * L.g);
-        kq[cb] = *reinterpret_cast<const bf16x4*>(A.k + (long)row * C + c + 4 * L.g);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    f32x4 z[NBLK], av[NBLK];
-    float ss = 0.f;
-#pragma unroll
-    for (int cb = 0; cb < NBLK; cb++) {
-        const long o = (long)row * C + h * HEAD + 16 * cb + 4 * L.g;
         f32x4 gacc = zero4(), w2 = zero4();
 #pragma unroll
-        for (int j = 0; j < R_GATE / 32; j++) gacc = mma8(gacc, gw[cb][j], tg1[j]);
+        for (int j = 0; j < R_GATE / 32; j++) gacc = mma8(gacc, gw[j], tg1[j]);
 #pragma unroll
-        for (int j = 0; j < R_DECAY / 32; j++) w2 = mma8(w2, dw[cb][j], tw1[j]);
-        *reinterpret_cast<bf16x4*>(A.g + o) = to_bf16(gacc);
-        const f32x4 kin = to_f32(kq[cb]);
-        z[cb] = mma(kin, wz[cb], tz);
-        const f32x4 pa = mma(to_f32(bias[cb][1]), wa[cb], a1);
-        const f32x4 pma = mma(to_f32(bias[cb][2]), wma[cb], ma1);
-        const f32x4 pmk = mma(to_f32(bias[cb][3]), wmk[cb], mk1);
-        const f32x4 u = to_f32(bias[cb][0]) + to_f32(to_bf16(w2));   // (w2 is a bf16 tensor in the sequence path)
+        for (int j = 0; j < R_DECAY / 32; j++) w2 = mma8(w2, dw[j], tw1[j]);
+        const f32x4 kin = to_f32(kq);
+        z = mma(kin, wz, to_bf16(t));
+        const f32x4 pa = mma(to_f32(ba), wa, a1), pma = mma(to_f32(bma), wma, ma1), pmk = mma(to_f32(bmk), wmk, mk1);
+        const f32x4 u = to_f32(bd) + to_f32(to_bf16(w2));   // (w2 is a bf16 tensor in the sequence path)
         f32x4 w, k;
+        float ss = 0.f;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const float a = sigmoidf_(pa[q]), ma = sigmoidf_(pma[q]), mk = sigmoidf_(pmk[q]);
             w[q] = -(fmaxf(-u[q], 0.f) + log1pexp_(u[q])) - 0.5f;
             k[q] = kin[q] * (ma + a - ma * a) * __expf(w[q] * mk);
-            av[cb][q] = a;
-            ss += z[cb][q] * z[cb][q];
+            av[q] = a;
+            ss += z[q] * z[q];
         }
-        *reinterpret_cast<bf16x4*>(A.w + o) = to_bf16(w);
-        *reinterpret_cast<bf16x4*>(A.k2 + o) = to_bf16(k);
-    }
-    const float inorm = rsqrtf(fmaxf(group_sum(ss), 1e-12f));
+        f32x4 d = to_f32(to_bf16(w));
 #pragma unroll
-    for (int cb = 0; cb < NBLK; cb++) {
-        const long o = (long)row * C + h * HEAD + 16 * cb + 4 * L.g;
-        const f32x4 kk = z[cb] * inorm;
-        *reinterpret_cast<bf16x4*>(A.kk + o) = to_bf16(kk);
-        *reinterpret_cast<bf16x4*>(A.b + o) = to_bf16(-kk * av[cb]);
+        for (int q = 0; q < 4; q++) d[q] = __expf(-__expf(d[q]));
+        const int at = 16 * ib + 4 * L.g;
+        *reinterpret_cast<bf16x4*>(&s.g[L.n][at]) = to_bf16(gacc);
+        *reinterpret_cast<f32x4*>(&s.decay[L.n][at]) = d;
+        *reinterpret_cast<bf16x4*>(&s.k[L.n][at]) = to_bf16(k);
+        ss = group_sum(ss);
+        if (L.g == 0) s.ss[ib][L.n] = ss;
     }
+    lds_barrier();
+    if (wave < 4) {
+        const float inorm = rsqrtf(fmaxf((s.ss[0][L.n] + s.ss[1][L.n]) + (s.ss[2][L.n] + s.ss[3][L.n]), 1e-12f));
+        const f32x4 kk = z * inorm;
+        const int at = 16 * ib + 4 * L.g;
+        *reinterpret_cast<bf16x4*>(&s.kk[L.n][at]) = to_bf16(kk);
+        *reinterpret_cast<bf16x4*>(&s.b[L.n][at]) = to_bf16(-kk * av);
+    }
+    lds_barrier();
+}
+
+// token n of the tile on value rows chan16(ib, .) of the state; y goes to LDS
+__device__ __forceinline__ void update_state(HeadTile& s, f32x4 (&S)[NBLK], int n, int ib, const Lane& L) {
+    auto vec = [&](const __bf16 (&a)[TOK][HeadTile::LD], int jb) { return to_f32(*reinterpret_cast<const bf16x4*>(&a[n][chan16(jb, 4 * L.g)])); };
+    float sa = 0.f;
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) {
+        const f32x4 a = vec(s.kk, jb);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sa += S[jb][q] * a[q];
+    }
+    sa = group_sum(sa);   // over the four lanes that share the state's row
+    const float vrow = (float)s.v[n][chan16(ib, L.n)];
+    float acc = 0.f;
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) {
+        const f32x4 d = *reinterpret_cast<const f32x4*>(&s.decay[n][chan16(jb, 4 * L.g)]);
+        const f32x4 b = vec(s.b, jb), k = vec(s.k, jb), r = vec(s.r, jb);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            S[jb][q] = S[jb][q] * d[q] + sa * b[q] + vrow * k[q];
+            acc += S[jb][q] * r[q];
+        }
+    }
+    acc = group_sum(acc);
+    if (L.g == 0) s.y[n][chan16(ib, L.n)] = acc;
+}
+
+// GroupNorm, bonus and gate of token n (row m of the output), lane = channel
+__device__ __forceinline__ void finish_token(const HeadTile& s, const HeadArgs& A, int h, int n, long m, int lane) {
+    auto head_sum = [](float x) {
+        x = row_sum(x);
+        return group_sum(x);
+    };
+    const float y = s.y[n][lane];
+    const float mean = head_sum(y) * (1.f / HEAD);
+    const float istd = rsqrtf(head_sum((y - mean) * (y - mean)) * (1.f / HEAD) + LN_EPS);
+    const float* lp = A.ln_params + h * HEAD + lane;
+    const float dot = head_sum((float)s.r[n][lane] * (float)s.k[n][lane] * lp[2 * (long)A.C]);
+    const float out = ((y - mean) * istd * lp[0] + lp[A.C] + dot * (float)s.v[n][lane]) * (float)s.g[n][lane];
+    A.ya[m * A.C + h * HEAD + lane] = (__bf16)out;
+}
+
+// One token per sequence: block = (some rows of a 16-row tile, head).  Every wavefront asks for the first state it updates
+// before the expansion starts, and for the next before it updates one.
+template <int GROUPS>   // row groups: a wavefront updates every GROUPS-th of the block's rows
+__global__ __launch_bounds__(256 * GROUPS) void decode_head_kernel(const HeadArgs A, int rows_per_block) {
+    __shared__ HeadTile s;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Lane L;
+    const int h = blockIdx.x;
+    const int first = blockIdx.y * rows_per_block;                      // the block's rows: first .. first + count - 1
+    const int row0 = first / TOK * TOK, r0 = first - row0;              // (inside the tile: r0 .. end - 1)
+    const int end = r0 + (A.rows - first < rows_per_block ? A.rows - first : rows_per_block);
+    const int ib = wave & 3, group = wave >> 2;
+    f32x4 S[NBLK], Sn[NBLK];
+    auto fetch = [&](f32x4 (&D)[NBLK], int r) {
+        const int bh = (row0 + (r < end ? r : end - 1)) * A.H + h;
+#pragma unroll
+        for (int jb = 0; jb < NBLK; jb++) D[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+    };
+    fetch(S, r0 + group);
+    expand_tile(s, A, h, row0, A.rows - 1, wave, L);
+    for (int r = r0 + group; r < end; r += GROUPS) {
+        fetch(Sn, r + GROUPS);   // (past the last row: that row again, unused)
+        update_state(s, S, r, ib, L);
+#pragma unroll
+        for (int jb = 0; jb < NBLK; jb++) {
+            store_state_frag(A.state, A.state_f32, (row0 + r) * A.H + h, ib, jb, L, S[jb]);
+            S[jb] = Sn[jb];
+        }
+    }
+    lds_barrier();
+    for (int r = r0 + wave; r < end; r += 4 * GROUPS) finish_token(s, A, h, r, row0 + r, lane);
+}
+
+// T tokens per sequence, one after the other on a state that stays in registers: block = (sequence, head).
+__global__ __launch_bounds__(256) void prompt_head_kernel(const HeadArgs A) {
+    __shared__ HeadTile s;
+    const int lane = threadIdx.x & 63, ib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Lane L;
+    const int h = blockIdx.x, seq = blockIdx.y, bh = seq * A.H + h;
+    f32x4 S[NBLK];
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+    for (int t0 = 0; t0 < A.T; t0 += TOK) {
+        const int first = seq * A.T + t0, n = A.T - t0 < TOK ? A.T - t0 : TOK;
+        expand_tile(s, A, h, first, first + n - 1, ib, L);
+        for (int t = 0; t < n; t++) update_state(s, S, t, ib, L);
+        lds_barrier();
+        for (int t = ib; t < n; t += 4) finish_token(s, A, h, t, first + t, lane);
+        lds_barrier();   // (the next tile overwrites what the epilogue reads)
+    }
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.state, A.state_f32, bh, ib, jb, L, S[jb]);
 }
 
 constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
 int padded_rows(int B) { return (B + TOK - 1) / TOK * TOK; }
+// How much of the output a block of a linear kernel takes: the least that keeps the launch under so many blocks.  Below
+// them (about three blocks for two compute units) narrower blocks spread the loads wider; above, they repeat the
+// interpolation and re-read the inputs without any more of the chip to use.  us per step at 768 channels, 33 and 48
+// sequences: 16 columns 28.8 and 32.3, 32 columns 25.0 and 28.0; 64 x 2048 channels: 64 columns x 16 rows 69.6, x 32 rows 58.8.
+constexpr int LIN_BLOCKS = 400, LIN_SINGLE_BLOCKS = 320;
 
 }  // namespace
 
+// B: tokens in all (sequences times tokens per sequence)
 size_t mixer_decode_workspace_bytes(int B, int C) {
     const size_t Bp = padded_rows(B);
     return 13 * A256(Bp * C * 2) + A256(Bp * R_GATE * 2) + A256(Bp * R_DECAY * 2) + 4 * A256(Bp * 16 * 2);
 }
 
-void launch_mixer_decode(int B, int C, int H, int state_f32, const MixerWeights& mw, const void* x, const void* x_prev,
-                         void* state, void* y, void* x_carry, void* workspace, hipStream_t stream) {
-    const int Bp = padded_rows(B);
+// A block repeats the expansion of its whole tile for the rows it updates, so it takes as many rows (up to 8) as leave about
+// one block per compute unit.  us per step at 768 channels: 16 sequences in blocks of 16 rows 34.8, of 1 row 22.7; 256
+// sequences in blocks of 4 rows 66, of 8 rows 54.
+namespace {
+int head_rows_per_block(int B, int H) {
+    int rpb = 1;
+    while (rpb < 8 && (long)H * ((B + rpb - 1) / rpb) > compute_units()) rpb *= 2;
+    return rpb;
+}
+template <bool LERP>
+void launch_linear(const LinArgs& a, const MixIn& mix, hipStream_t stream) {
+    auto blocks = [&](int columns) {
+        int n = 0;
+        for (int i = 0; i < a.nseg; i++) n += (a.seg[i].N + columns - 1) / columns;
+        return n;
+    };
+    const dim3 threads(256);
+    if (blocks(16) * a.ntiles <= LIN_BLOCKS)
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 1, 1>), dim3(blocks(16), a.ntiles), threads, 0, stream, a, mix);
+    else if (blocks(32) * a.ntiles <= LIN_BLOCKS)
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 2, 1>), dim3(blocks(32), a.ntiles), threads, 0, stream, a, mix);
+    else if (blocks(64) * a.ntiles <= LIN_SINGLE_BLOCKS)
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 1>), dim3(blocks(64), a.ntiles), threads, 0, stream, a, mix);
+    else
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 2>), dim3(blocks(64), (a.ntiles + 1) / 2), threads, 0, stream, a, mix);
+}
+}  // namespace
+
+void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerWeights& mw, const void* x, const void* x_prev,
+                         const void* state_in, void* state, void* y, void* x_carry, void* workspace, hipStream_t stream) {
+    const int rows = B * T, Bp = padded_rows(rows), ntiles = Bp / TOK;
     char* p = static_cast<char*>(workspace);
     auto take = [&](size_t elems) {
         __bf16* r = reinterpret_cast<__bf16*>(p);
@@ -348,50 +541,59 @@ void launch_mixer_decode(int B, int C, int H, int state_f32, const MixerWeights&
         return r;
     };
     const size_t BC = (size_t)Bp * C;
-    __bf16* streams = take(4 * BC);   // (4 x A256(BC*2) >= A256(4*BC*2): the budget above covers it)
-    __bf16 *r = take(BC), *k = take(BC), *v = take(BC);
-    __bf16 *w = take(BC), *k2 = take(BC), *kk = take(BC), *b = take(BC), *g = take(BC), *ya = take(BC);
+    __bf16 *mid = take((size_t)Bp * MID), *r = take(BC), *k = take(BC), *v = take(BC), *ya = take(BC);   // (well inside the workspace)
     __bf16 *tg1 = take((size_t)Bp * R_GATE), *tw1 = take((size_t)Bp * R_DECAY);
     __bf16 *kk1 = take((size_t)Bp * 16), *mk1 = take((size_t)Bp * 16), *a1 = take((size_t)Bp * 16), *ma1 = take((size_t)Bp * 16);
     auto c = [](const void* q) { return static_cast<const __bf16*>(q); };
-    const dim3 tiles(Bp / TOK);
+    const MixIn mix{c(x), c(x_prev), c(mw.time_maa_w2), c(mw.time_maa), mid, rows, T};
 
-    // at least eight wavefronts (the eight 16-wide blocks of the first product are added by one each)
-    const int mix_waves = C / 64 < 8 ? 8 : (C / 64 < MIX_MAX_WAVES ? C / 64 : MIX_MAX_WAVES);
-    hipLaunchKernelGGL(decode_mix_kernel, tiles, dim3(64 * mix_waves), 0, stream, B, Bp, C, c(x), c(x_prev), c(mw.time_maa_x),
-                       c(mw.time_maa), c(mw.time_maa_w1), c(mw.time_maa_w2), streams, static_cast<__bf16*>(x_carry));
-    const __bf16 *xrg = streams, *xwa = streams + BC, *xk = streams + 2 * BC, *xv = streams + 3 * BC;
+    // (one round of loads for four wavefronts up to 768 channels; beyond, sixteen: 2048 channels 9.3 -> 6.5 us)
+    if (C <= 768)
+        hipLaunchKernelGGL((decode_mid_kernel<4, 6>), dim3(MID / 16, ntiles), dim3(256), 0, stream, mix, C, c(mw.time_maa_x),
+                           c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
+    else
+        hipLaunchKernelGGL((decode_mid_kernel<16, 4>), dim3(MID / 16, ntiles), dim3(1024), 0, stream, mix, C, c(mw.time_maa_x),
+                           c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
     {
         LinArgs a{};
-        a.seg[0] = {xrg, c(mw.Wr), r, C, 0};
-        a.seg[1] = {xk, c(mw.Wk), k, C, 0};
-        a.seg[2] = {xv, c(mw.Wv), v, C, 0};
-        a.seg[3] = {xrg, c(mw.gate_w1), tg1, R_GATE, 1};
-        a.seg[4] = {xwa, c(mw.time_decay_w1), tw1, R_DECAY, 1};
-        a.seg[5] = {xk, c(mw.time_kkk_w1), kk1, R_KKK, 0};
-        a.seg[6] = {xk, c(mw.mk_w1), mk1, R_MK, 0};
-        a.seg[7] = {xwa, c(mw.time_aaa_w1), a1, R_AAA, 0};
-        a.seg[8] = {xwa, c(mw.ma_w1), ma1, R_MA, 0};
+        enum { XRG, XWA, XK, XV };
+        a.seg[0] = {nullptr, c(mw.Wr), r, C, 0, XRG};
+        a.seg[1] = {nullptr, c(mw.Wk), k, C, 0, XK};
+        a.seg[2] = {nullptr, c(mw.Wv), v, C, 0, XV};
+        a.seg[3] = {nullptr, c(mw.gate_w1), tg1, R_GATE, 1, XRG};
+        a.seg[4] = {nullptr, c(mw.time_decay_w1), tw1, R_DECAY, 1, XWA};
+        a.seg[5] = {nullptr, c(mw.time_kkk_w1), kk1, R_KKK, 0, XK};
+        a.seg[6] = {nullptr, c(mw.mk_w1), mk1, R_MK, 0, XK};
+        a.seg[7] = {nullptr, c(mw.time_aaa_w1), a1, R_AAA, 0, XWA};
+        a.seg[8] = {nullptr, c(mw.ma_w1), ma1, R_MA, 0, XWA};
         a.nseg = 9;
         a.C = C;
         a.rows = Bp;
-        const int nblk = (3 * C + R_GATE + R_DECAY + R_KKK + R_MK + R_AAA + R_MA) / 16;
-        hipLaunchKernelGGL(decode_linear_kernel, dim3(nblk, Bp / TOK), dim3(256), 0, stream, a);
+        a.ntiles = ntiles;
+        launch_linear<true>(a, mix, stream);
     }
     {
-        const ExpandArgs a{Bp, C, k, tg1, tw1, kk1, mk1, a1, ma1,
-                           c(mw.gate_w2), c(mw.time_decay_w2), c(mw.time_kkk_w2), c(mw.time_aaa_w2), c(mw.ma_w2), c(mw.mk_w2),
-                           c(mw.time_decay), c(mw.time_aaaaa), c(mw.time_misc_a), c(mw.time_misc_k), w, k2, kk, b, g};
-        hipLaunchKernelGGL(decode_expand_kernel, dim3(H, Bp / TOK), dim3(64), 0, stream, a);
+        const HeadArgs a{rows, T, C, H, state_f32, r, k, v, tg1, tw1, kk1, mk1, a1, ma1,
+                         c(mw.gate_w2), c(mw.time_decay_w2), c(mw.time_kkk_w2), c(mw.time_aaa_w2), c(mw.ma_w2), c(mw.mk_w2),
+                         c(mw.time_decay), c(mw.time_aaaaa), c(mw.time_misc_a), c(mw.time_misc_k),
+                         static_cast<const float*>(mw.ln_params), state_in, state, ya};
+        const int rpb = head_rows_per_block(B, H);
+        const dim3 grid(H, (B + rpb - 1) / rpb);
+        if (T > 1)
+            hipLaunchKernelGGL(prompt_head_kernel, dim3(H, B), dim3(256), 0, stream, a);
+        else if (rpb == 1)
+            hipLaunchKernelGGL(decode_head_kernel<1>, grid, dim3(256), 0, stream, a, rpb);
+        else
+            hipLaunchKernelGGL(decode_head_kernel<2>, grid, dim3(512), 0, stream, a, rpb);
     }
-    launch_decode(B, H, state_f32, w, r, k2, v, kk, b, state, ya, stream, g, mw.ln_params);
     {
         LinArgs a{};
-        a.seg[0] = {ya, c(mw.Wo), static_cast<__bf16*>(y), C, 0};
+        a.seg[0] = {ya, c(mw.Wo), static_cast<__bf16*>(y), C, 0, 0};
         a.nseg = 1;
         a.C = C;
-        a.rows = B;
-        hipLaunchKernelGGL(decode_linear_kernel, dim3(C / 16, Bp / TOK), dim3(256), 0, stream, a);
+        a.rows = rows;
+        a.ntiles = ntiles;
+        launch_linear<false>(a, mix, stream);
     }
 }
 

@@ -16,9 +16,10 @@ struct MixerWeights {
 };
 
 size_t mixer_decode_workspace_bytes(int B, int C);
-// x, x_prev [B,C] bf16; state [B,H,64,64] (bf16 or fp32), updated in place; y [B,C] bf16; x_carry: null or [B,C] bf16
-// that receives a copy of x (the next step's x_prev; must not alias x_prev)
-void launch_mixer_decode(int B, int C, int H, int state_f32, const MixerWeights& w, const void* x, const void* x_prev,
-                         void* state, void* y, void* x_carry, void* workspace, hipStream_t stream);
+// x [B,T,C] bf16; x_prev null or [B,C] bf16, the token before; state_in null or, and state, [B,H,64,64] (bf16 or fp32; may be
+// the same); y [B,T,C] bf16; x_carry: null or [B,C] bf16 that receives the last tokens (the next call's x_prev; must not
+// alias x_prev).  workspace: mixer_decode_workspace_bytes(B*T, C).
+void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerWeights& w, const void* x, const void* x_prev,
+                         const void* state_in, void* state, void* y, void* x_carry, void* workspace, hipStream_t stream);
 
 }  // namespace wkv

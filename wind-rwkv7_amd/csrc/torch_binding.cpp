@@ -37,7 +37,8 @@ namespace py = pybind11;
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
     X(ddlerp_forward_from) X(neutral_rows) X(copy_columns) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
-    X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode)
+    X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
+    X(mixer_prompt)
 
 struct Lib {
 #define X(name) decltype(&wind_rwkv7_##name) name = nullptr;
@@ -609,6 +610,27 @@ struct WeightGrads {
     }
 };
 
+// bf16 copies of the block's weights in one launch, and its [3,C] float32 parameters of attn_ln
+struct BlockWeights {
+    Tensor flat, ln;
+    ParamLayout at_;
+    BlockWeights(const variable_list& p, const Tensor& like) : at_(like.size(-1)) {
+        flat = at::empty({at_.at[LN_W]}, like.options().dtype(at::kBFloat16));
+        const void* src[WEIGHTS];
+        int dtype[WEIGHTS];
+        long long numel[WEIGHTS], offset[WEIGHTS];
+        for (int i = 0; i < WEIGHTS; i++) {
+            src[i] = p[i].data_ptr();
+            dtype[i] = p[i].scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
+            numel[i] = p[i].numel();
+            offset[i] = at_.at[i];
+        }
+        check(L.cast_to_bf16(WEIGHTS, src, dtype, numel, offset, flat.data_ptr(), stream_of(flat)));
+        ln = at::stack({p[LN_W], p[LN_B], p[FAAAA]}).to(at::kFloat);
+    }
+    void* w(int i) const { return at_elem(flat, at_.at[i]); }
+};
+
 struct BlockForward {   // what one forward pass leaves
     Tensor xb, weights, lnp, acts, saved, y, sT;
 };
@@ -623,20 +645,9 @@ BlockForward block_forward(const Block& s, const Tensor& xb, const variable_list
     const ParamLayout at_(C);
     BlockForward f;
     f.xb = xb;
-    f.weights = at::empty({at_.at[LN_W]}, xb.options());
-    {
-        const void* src[WEIGHTS];
-        int dtype[WEIGHTS];
-        long long numel[WEIGHTS], offset[WEIGHTS];
-        for (int i = 0; i < WEIGHTS; i++) {
-            src[i] = p[i].data_ptr();
-            dtype[i] = p[i].scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
-            numel[i] = p[i].numel();
-            offset[i] = at_.at[i];
-        }
-        check(L.cast_to_bf16(WEIGHTS, src, dtype, numel, offset, f.weights.data_ptr(), stream));
-    }
-    f.lnp = at::stack({p[LN_W], p[LN_B], p[FAAAA]}).to(at::kFloat);
+    const BlockWeights bw(p, xb);
+    f.weights = bw.flat;
+    f.lnp = bw.ln;
     const Activations A(s);
     f.acts = at::empty({save ? A.kept : A.total}, xb.options());
     // (training keeps the activations: the concatenated first halves, which nothing needs later, go to a buffer of their own)
@@ -834,6 +845,32 @@ bool floating(const Tensor& t) {
     return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kDouble;
 }
 
+// A prompt this short that would have to be padded runs token by token on a state in registers, in the four launches of a
+// step; the sequence kernels take some twenty launches whatever the length.  (Whole chunks stay with them: the same bits as the
+// same tokens inside a longer call.)
+constexpr int64_t SHORT_PROMPT = 64, SHORT_PROMPT_ROWS = 512;
+
+py::object short_prompt(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& x, const variable_list& p, const Tensor& x_prev,
+                        const Tensor& s0, at::ScalarType state_type, bool return_state) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor xb = x.to(at::kBFloat16).contiguous();
+    const BlockWeights bw(p, xb);
+    const void* w[WEIGHTS + 1];
+    for (int i = 0; i < WEIGHTS; i++) w[i] = bw.w(i);
+    w[WEIGHTS] = bw.ln.data_ptr();
+    wind_rwkv7_mixer_weights weights;
+    static_assert(sizeof(w) == sizeof(weights), "the enumeration above is the header's order");
+    memcpy(&weights, w, sizeof(w));
+    const Tensor y = at::empty({B, T, C}, xb.options()), sT = at::empty({B, H, 64, 64}, xb.options().dtype(state_type));
+    const bool carry_here = return_state && x.scalar_type() == at::kBFloat16;   // (the carried token keeps x's own type)
+    const Tensor carry = carry_here ? at::empty({B, C}, xb.options()) : return_state ? x.select(1, T - 1).clone() : Tensor();
+    const Tensor ws = scratch_bytes(L.mixer_decode_workspace_bytes((int)(B * T), (int)C), xb);
+    check(L.mixer_prompt((int)B, (int)T, (int)C, (int)H, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, &weights, ptr(xb), ptr(x_prev),
+                         ptr(s0), ptr(sT), ptr(y), carry_here ? ptr(carry) : nullptr, ptr(ws), ws.numel(), stream_of(xb)));
+    if (!return_state) return py::cast(y);
+    return py::make_tuple(y, py::make_tuple(carry, sT));
+}
+
 py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int64_t H, const std::optional<Tensor>& x_prev_,
                  const std::optional<Tensor>& s0_, bool return_state) {
     if (!x.defined() || !x.is_cuda() || !floating(x) || x.layout() != at::kStrided || at::isTensorSubclassLike(x) || x.dim() != 3 || H <= 0 ||
@@ -864,9 +901,11 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
             s0.sizes() != at::IntArrayRef({s.B, s.H, s.N(), s.N()}))
             return py::none();
     }
+    const at::ScalarType state_type = s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16;
+    if (T % 16 && s.N() == 64 && T <= SHORT_PROMPT && s.B * T <= SHORT_PROMPT_ROWS) return short_prompt(s.B, T, s.C, H, x, p, x_prev, s0, state_type, return_state);
     Tensor xb = x.to(at::kBFloat16);
     xb = s.T == T ? xb.contiguous() : at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
-    BlockForward f = block_forward(s, xb, p, false, T, x_prev, s0, s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16);
+    BlockForward f = block_forward(s, xb, p, false, T, x_prev, s0, state_type);
     const Tensor y = s.T == T ? f.y : f.y.narrow(1, 0, T).contiguous();
     if (!return_state) return py::cast(y);
     return py::make_tuple(y, py::make_tuple(x.select(1, T - 1).clone(), f.sT));

@@ -55,6 +55,7 @@ SIGNATURES = {
     'wind_rwkv7_attn_ln_decode': (_i, [_i] * 5 + [_vp] * 8 + [_vp, _vp, _vp]),
     'wind_rwkv7_mixer_decode_workspace_bytes': (_sz, [_i, _i]),
     'wind_rwkv7_mixer_decode': (_i, [_i] * 4 + [_vp] * 6 + [_vp, _sz, _vp]),
+    'wind_rwkv7_mixer_prompt': (_i, [_i] * 5 + [_vp] * 8 + [_sz, _vp]),
     'wind_rwkv7_ddlerp_rank_supported': (_i, [_i]),
     'wind_rwkv7_ddlerp_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_ddlerp_forward': (_i, [_i] * 4 + [_vp] * 5 + [_vp] * 3 + [_vp]),

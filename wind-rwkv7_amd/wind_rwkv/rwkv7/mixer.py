@@ -334,8 +334,8 @@ class TimeMixer(nn.Module):
         return state
 
     def _step_fused(self, x, x_prev, S):
-        """`step` in five launches (wind_rwkv7_mixer_decode): token shift, all first-half products, LoRA second halves
-        with the elementwise tail, the WKV7 step with its epilogue, output projection.  The native binding makes the call
+        """`step` in four launches (wind_rwkv7_mixer_decode): the token shift's first product, all first-half products, per
+        head the LoRA second halves with the WKV7 step and its epilogue, output projection.  The native binding makes the call
         while the kept copies are those of the parameters; else they are remade here first."""
         for _ in range(2):
             out = _native.binding().mixer_step(x, x_prev, S, self._parameters, self.ln_x._parameters, self.__dict__.get('_decode_cache'), self.n_head)
