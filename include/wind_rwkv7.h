@@ -321,6 +321,19 @@ int wind_rwkv7_expand_loras_backward(int B, int T, int C, int D, int head_size,
                                      void* dWz, void* dWa, void* dWma, void* dWmk,
                                      void* dw_bias, void* da_bias, void* dma_bias, void* dmk_bias,
                                      void* workspace, size_t workspace_bytes, void* stream);
+/* The same with row strides ld_din[0..3] (elements, multiples of 8) for dz_in, da_in, dma_in, dmk_in: they can be columns of
+ * wider matrices. */
+int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_size,
+                                     const void* w_in, const void* k_in,
+                                     const void* z_in, const void* a_in, const void* ma_in, const void* mk_in,
+                                     const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
+                                     const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
+                                     const void* dw_out, const void* dk_out, const void* dkk_out, const void* db_out,
+                                     void* dw_in, void* dk_in,
+                                     void* dz_in, void* da_in, void* dma_in, void* dmk_in, const long long* ld_din,
+                                     void* dWz, void* dWa, void* dWma, void* dWmk,
+                                     void* dw_bias, void* da_bias, void* dma_bias, void* dmk_bias,
+                                     void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- WKV7 in fp32 (accuracy mode, and head sizes other than 64) ------------------------------------- */
 
@@ -382,6 +395,39 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
                                   const void* const* x, const long long* ld_x,
                                   void* const* dW, int out_dtype,
                                   void* workspace, size_t workspace_bytes, void* stream);
+
+/* Working copies of up to WIND_RWKV7_PACK_MAX parameters in one launch: dst [rows, cols] in dst_dtype, and, where dstT is
+ * given (dst_dtype bf16, rows % 16 == 0), the transposed copy dstT[c * ldT + r] (ldT >= rows, a multiple of 8).  cols is a
+ * multiple of 16 (a vector is one row); bases are 16-byte aligned. */
+#define WIND_RWKV7_PACK_MAX 32
+typedef struct {
+    const void* src;
+    void *dst, *dstT;
+    int src_dtype, dst_dtype, rows, cols;
+    long long ldT;
+} wind_rwkv7_pack;
+int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream);
+
+/* Products of token-major bf16 matrices with weights, up to WIND_RWKV7_LINEAR_GROUP_MAX of them on the same M tokens in one
+ * launch; replaces the matmuls of TimeMixer.forward (time_mixer.py:120-131, :167) and of their input gradients.  A problem is
+ *   D[m][n] = sum_k A[0][m][k] W[0][n][k]  (+ sum_k A[1][m][k] W[1][n][k] where K[1] > 0),     fp32 accumulation,
+ * A[g]: [M, K[g]] bf16 (row stride lda[g] elements), W[g]: [N, K[g]] bf16 (ldw[g]).  D's columns are cut into npieces (1-4)
+ * blocks of width[t] columns, in order and covering N, each written in bf16 to out[t] (ld_out[t]) with op[t] = 0 as it
+ * is, 1 through tanh (of the bf16 value), 2 times 1 - aux^2 (aux[t]: contiguous [M, width[t]] bf16).  K, widths: multiples of
+ * 16; row strides: multiples of 8; bases 16-byte aligned. */
+#define WIND_RWKV7_LINEAR_GROUP_MAX 8
+typedef struct {
+    const void* A[2];
+    const void* W[2];
+    long long lda[2], ldw[2];
+    int K[2];
+    int N, npieces;
+    void* out[4];
+    const void* aux[4];
+    long long ld_out[4];
+    int width[4], op[4];
+} wind_rwkv7_linear;
+int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problems, void* stream);
 
 /* Tokens first .. T-1 of the recurrence's operands w, k, b [B,T,C] bf16 become ones that leave a state as it is: decay 1,
  * k = b = 0.  A sequence of any length then runs padded to whole chunks and its final state is that of token first-1. */

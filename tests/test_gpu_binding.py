@@ -100,9 +100,12 @@ class _Absent:
     (128, 2, torch.bfloat16, torch.float32, ()), (192, 6, torch.float32, torch.float32, ('Wr', 'gate_w2', 'ln_x.weight')),
     (256, 2, torch.bfloat16, torch.bfloat16, ('Wo', 'time_maa_w1'))])
 def test_block_equals_the_python_path(monkeypatch, C, H, x_dtype, param_dtype, frozen):
-    """Forward, backward and the forward without autograd of the whole block, with some parameters frozen; same kernels and
-    library products in the same order, so the same bits."""
+    """Forward, backward and the forward without autograd of the whole block, with some parameters frozen, against the
+    Python path, whose products are the BLAS library's: other summation orders inside them, so bf16 values differ by a
+    rounding here and there, and what follows from those: a gate of 5e-3 on the output and 1e-2 on gradients (what the block
+    is held to against its oracle is 1e-2 to 1.6e-2)."""
     from collections import namedtuple
+    from oracle import seq_ref
     from wind_rwkv import _native
     from wind_rwkv.rwkv7 import TimeMixer
     gen = torch.Generator().manual_seed(C)
@@ -124,7 +127,8 @@ def test_block_equals_the_python_path(monkeypatch, C, H, x_dtype, param_dtype, f
             z = model(x)
         results.append([y.detach(), z] + list(torch.autograd.grad(y, leaves, dy)))
     for i, (a, b) in enumerate(zip(*results)):
-        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
+        assert a.dtype == b.dtype and a.shape == b.shape
+        assert seq_ref.rel_err(a.float().cpu(), b.float().cpu()) <= (5e-3 if i < 2 else 1e-2), i
 
 
 @pytest.mark.parametrize('T', [2, 15, 17, 100])

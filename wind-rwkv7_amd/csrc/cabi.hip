@@ -643,6 +643,24 @@ int wind_rwkv7_expand_loras_backward(int B, int T, int C, int D, int head_size,
                                      void* dWz, void* dWa, void* dWma, void* dWmk,
                                      void* dw_bias, void* da_bias, void* dma_bias, void* dmk_bias,
                                      void* workspace, size_t workspace_bytes, void* stream) {
+    const long long ld[4] = {D, D, D, D};
+    return wind_rwkv7_expand_loras_backward_to(B, T, C, D, head_size, w_in, k_in, z_in, a_in, ma_in, mk_in, Wz, Wa, Wma, Wmk, w_bias, a_bias,
+                                               ma_bias, mk_bias, dw_out, dk_out, dkk_out, db_out, dw_in, dk_in, dz_in, da_in, dma_in,
+                                               dmk_in, ld, dWz, dWa, dWma, dWmk, dw_bias, da_bias, dma_bias, dmk_bias, workspace,
+                                               workspace_bytes, stream);
+}
+
+int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_size,
+                                     const void* w_in, const void* k_in,
+                                     const void* z_in, const void* a_in, const void* ma_in, const void* mk_in,
+                                     const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
+                                     const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
+                                     const void* dw_out, const void* dk_out, const void* dkk_out, const void* db_out,
+                                     void* dw_in, void* dk_in,
+                                     void* dz_in, void* da_in, void* dma_in, void* dmk_in, const long long* ld_din,
+                                     void* dWz, void* dWa, void* dWma, void* dWmk,
+                                     void* dw_bias, void* da_bias, void* dma_bias, void* dmk_bias,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
     int rc = check_loras(B, T, C, D, head_size);
     if (rc) return rc;
     const void* const acts[4] = {z_in, a_in, ma_in, mk_in};
@@ -658,7 +676,13 @@ int wind_rwkv7_expand_loras_backward(int B, int T, int C, int D, int head_size,
             return WIND_RWKV7_ERR_NULL_POINTER;
     rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_expand_loras_bwd_workspace_bytes(B, T, C, D));
     if (rc) return rc;
-    wkv::launch_expand_loras_backward((long)B * T, C, D, head_size, w_in, k_in, acts, Ws, biases, dys, dw_in, dk_in, dacts, dWs,
+    if (!ld_din) return WIND_RWKV7_ERR_NULL_POINTER;
+    long ld[4];
+    for (int i = 0; i < 4; i++) {
+        if (ld_din[i] < D || ld_din[i] % 8 != 0 || reinterpret_cast<uintptr_t>(dacts[i]) % 16 != 0) return WIND_RWKV7_ERR_BAD_SHAPE;
+        ld[i] = (long)ld_din[i];
+    }
+    wkv::launch_expand_loras_backward((long)B * T, C, D, head_size, w_in, k_in, acts, Ws, biases, dys, dw_in, dk_in, dacts, ld, dWs,
                                       dbiases, workspace, static_cast<hipStream_t>(stream));
     return launch_status();
 }
@@ -811,6 +835,71 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
     if (!wkv::launch_linear_wgrad_group(n, (long)tokens, O, I, dy, ldy, x, ldx, dW, out_dtype == WIND_RWKV7_F32, workspace,
                                         static_cast<hipStream_t>(stream)))
         return WIND_RWKV7_ERR_CHANNELS;
+    return launch_status();
+}
+
+int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream) {
+    if (n < 1 || n > WIND_RWKV7_PACK_MAX) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!tensors) return WIND_RWKV7_ERR_NULL_POINTER;
+    wkv::PackTensor P[WIND_RWKV7_PACK_MAX];
+    for (int t = 0; t < n; t++) {
+        const wind_rwkv7_pack& u = tensors[t];
+        if (u.rows <= 0 || u.cols <= 0 || u.cols % 16 != 0 || (long long)u.rows * u.cols > (1LL << 30)) return WIND_RWKV7_ERR_BAD_SHAPE;
+        if (!u.src || !u.dst) return WIND_RWKV7_ERR_NULL_POINTER;
+        for (int d : {u.src_dtype, u.dst_dtype})
+            if (d != WIND_RWKV7_BF16 && d != WIND_RWKV7_F32) return WIND_RWKV7_ERR_DTYPE;
+        if (u.dstT && (u.dst_dtype != WIND_RWKV7_BF16 || u.rows % 16 != 0 || u.ldT < u.rows || u.ldT % 8 != 0)) return WIND_RWKV7_ERR_BAD_SHAPE;
+        for (const void* q : {u.src, (const void*)u.dst, (const void*)u.dstT})
+            if (reinterpret_cast<uintptr_t>(q) % 16 != 0) return WIND_RWKV7_ERR_BAD_SHAPE;
+        P[t] = wkv::PackTensor{u.src, u.dst, u.dstT, u.rows, u.cols, (long)u.ldT, u.src_dtype == WIND_RWKV7_F32, u.dst_dtype == WIND_RWKV7_F32};
+    }
+    wkv::launch_pack_weights(n, P, static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
+int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problems, void* stream) {
+    if (n < 1 || n > WIND_RWKV7_LINEAR_GROUP_MAX || M <= 0 || M > (1LL << 30)) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!problems) return WIND_RWKV7_ERR_NULL_POINTER;
+    auto misaligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
+    wkv::LinearProblem P[WIND_RWKV7_LINEAR_GROUP_MAX] = {};
+    for (int j = 0; j < n; j++) {
+        const wind_rwkv7_linear& u = problems[j];
+        wkv::LinearProblem& p = P[j];
+        if (u.N <= 0 || u.N > (1 << 20) || u.K[0] <= 0 || u.K[1] < 0 || u.npieces < 1 || u.npieces > wkv::LinearProblem::PIECES)
+            return WIND_RWKV7_ERR_BAD_SHAPE;
+        for (int g = 0; g < 2; g++) {
+            if (u.K[g] == 0) continue;
+            if (u.K[g] % 16 != 0 || u.K[g] > (1 << 20)) return WIND_RWKV7_ERR_CHANNELS;
+            if (!u.A[g] || !u.W[g]) return WIND_RWKV7_ERR_NULL_POINTER;
+            // (a tile's rows are addressed with 32-bit byte offsets from its first)
+            if (u.lda[g] < u.K[g] || u.ldw[g] < u.K[g] || u.lda[g] % 8 != 0 || u.ldw[g] % 8 != 0 || u.lda[g] > (1 << 22) ||
+                u.ldw[g] > (1 << 22) || misaligned(u.A[g]) || misaligned(u.W[g]))
+                return WIND_RWKV7_ERR_BAD_SHAPE;
+            p.A[g] = static_cast<const __bf16*>(u.A[g]);
+            p.W[g] = static_cast<const __bf16*>(u.W[g]);
+            p.lda[g] = (long)u.lda[g];
+            p.ldw[g] = (long)u.ldw[g];
+            p.K[g] = u.K[g];
+        }
+        int start = 0;
+        for (int t = 0; t < u.npieces; t++) {
+            if (u.width[t] <= 0 || u.width[t] % 16 != 0) return WIND_RWKV7_ERR_CHANNELS;
+            if (u.op[t] < wkv::LINEAR_PLAIN || u.op[t] > wkv::LINEAR_TANH_GRAD) return WIND_RWKV7_ERR_BAD_SHAPE;
+            if (!u.out[t] || (u.op[t] == wkv::LINEAR_TANH_GRAD && !u.aux[t])) return WIND_RWKV7_ERR_NULL_POINTER;
+            if (u.ld_out[t] < u.width[t] || u.ld_out[t] % 8 != 0 || misaligned(u.out[t]) || misaligned(u.aux[t])) return WIND_RWKV7_ERR_BAD_SHAPE;
+            p.out[t] = static_cast<__bf16*>(u.out[t]);
+            p.aux[t] = static_cast<const __bf16*>(u.aux[t]);
+            p.ld_out[t] = (long)u.ld_out[t];
+            p.start[t] = start;
+            p.width[t] = u.width[t];
+            p.op[t] = u.op[t];
+            start += u.width[t];
+        }
+        if (start != u.N) return WIND_RWKV7_ERR_BAD_SHAPE;
+        p.N = u.N;
+        p.npieces = u.npieces;
+    }
+    wkv::launch_linear_group(n, (long)M, P, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

@@ -54,7 +54,70 @@ __global__ __launch_bounds__(256) void cast_to_bf16_kernel(CastArgs g, __bf16* _
     }
 }
 
+// pack: a block takes 64 rows x 64 columns of one tensor, 16 contiguous elements of a row per thread; where a transposed
+// copy is wanted the tile turns in LDS and leaves as rows of the transposed matrix.
+constexpr int PT = 64;
+struct PackArgs {
+    PackTensor t[PACK_MAX_TENSORS];
+    int first[PACK_MAX_TENSORS + 1];   // first block of tensor t
+    int n;
+};
+__global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs g) {
+    __shared__ __bf16 s[PT][PT + 2];   // (pitch 33 words: columns are read across the banks)
+    int t = 0;
+    while (t + 1 < g.n && (int)blockIdx.x >= g.first[t + 1]) t++;   // the same for every thread of the block
+    const PackTensor& p = g.t[t];
+    const int tile = blockIdx.x - g.first[t], ntc = (p.cols + PT - 1) / PT;
+    const int r0 = tile / ntc * PT, c0 = tile % ntc * PT;
+    const int r = r0 + (threadIdx.x >> 2), c = c0 + 16 * (threadIdx.x & 3);
+    if (r < p.rows && c < p.cols) {
+        const long at = (long)r * p.cols + c;
+        f32x4 v[4];
+        if (p.src_f32) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.src) + at + 4 * i);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = to_f32(*reinterpret_cast<const bf16x4*>(static_cast<const __bf16*>(p.src) + at + 4 * i));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (p.dst_f32) {
+                *reinterpret_cast<f32x4*>(static_cast<float*>(p.dst) + at + 4 * i) = v[i];
+            } else {
+                const bf16x4 b = to_bf16(v[i]);
+                *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(p.dst) + at + 4 * i) = b;
+                if (p.dstT)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s[r - r0][c - c0 + 4 * i + e] = b[e];
+            }
+        }
+    }
+    if (!p.dstT) return;
+    __syncthreads();
+    // row c of the transposed copy: 16 source rows per thread
+    const int tc = c0 + (threadIdx.x >> 2), tr = r0 + 16 * (threadIdx.x & 3);
+    if (tc >= p.cols || tr >= p.rows) return;
+    bf16x8 o[2];
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[e / 8][e % 8] = s[tr - r0 + e][tc - c0];
+    __bf16* out = static_cast<__bf16*>(p.dstT) + (long)tc * p.ldT + tr;
+    *reinterpret_cast<bf16x8*>(out) = o[0];
+    *reinterpret_cast<bf16x8*>(out + 8) = o[1];
+}
+
 }  // namespace
+
+void launch_pack_weights(int n, const PackTensor* tensors, hipStream_t stream) {
+    PackArgs g;
+    g.n = n;
+    g.first[0] = 0;
+    for (int t = 0; t < n; t++) {
+        g.t[t] = tensors[t];
+        g.first[t + 1] = g.first[t] + ((tensors[t].rows + PT - 1) / PT) * ((tensors[t].cols + PT - 1) / PT);
+    }
+    hipLaunchKernelGGL(pack_weights_kernel, dim3(g.first[n]), dim3(256), 0, stream, g);
+}
 
 void launch_cast_to_bf16(int n, const void* const* src, const int* src_f32, const long long* numel,
                          const long long* dst_offset, void* dst, hipStream_t stream) {

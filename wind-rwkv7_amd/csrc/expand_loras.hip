@@ -924,44 +924,54 @@ __global__ __launch_bounds__(256) void expand_loras_bwd16_kernel(long M, int C, 
         *reinterpret_cast<f32x4*>(out + 4 * i) = *reinterpret_cast<const f32x4*>(comb + 4 * i);
 }
 
-// d_in[i][m][d] = sum over heads of the per-head partials (bf16 in, fp32 sum, bf16 out); one thread per
-// 8 consecutive rank channels
-__global__ __launch_bounds__(256) void expand_loras_din_reduce_kernel(long M, int H, int D, LoraDIn part, LoraDIn out) {
-    const long n8 = M * D / 8;
-    const long e = blockIdx.x * 256L + threadIdx.x;
-    if (e >= 4 * n8) return;
-    const int i = (int)(e / n8);
-    const long r = (e % n8) * 8;          // element offset in [M][D]
-    const long m = r / D;
-    const int d = (int)(r % D);
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const __bf16* src = part.p[i] + m * H * D + d;
-    for (int h = 0; h < H; h++) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(src + (long)h * D);
-#pragma unroll
-        for (int q = 0; q < 8; q++) acc[q] += (float)v[q];
-    }
-    bf16x8 o;
-#pragma unroll
-    for (int q = 0; q < 8; q++) o[q] = (__bf16)acc[q];
-    *reinterpret_cast<bf16x8*>(out.p[i] + r) = o;
-}
-
-// dW_i [C][D] and dbias_i [C]: sum of the block records over the token splits, in order; one thread per element
-struct LoraParamOut {
+// What the backward kernel's blocks leave is summed in one launch: blocks below `din_blocks` the input gradients
+// d_in[i][m][d] over the heads (bf16 in, fp32 sum, bf16 out; one thread per 8 consecutive rank channels, row stride ld[i]), the
+// others dW_i [C][D] and dbias_i [C] over the token splits (one thread per element).  The order of the sums is fixed.
+struct LoraReduceOut {
+    __bf16* din[4];
+    long ld[4];
     float* dW[4];
     float* db[4];
 };
-__global__ __launch_bounds__(256) void expand_loras_param_reduce_kernel(int C, int D, int nsplit,
-                                                                        const float* __restrict__ partial,
-                                                                        LoraParamOut out) {
+__global__ __launch_bounds__(256) void expand_loras_reduce_kernel(long M, int C, int D, int nsplit, int din_blocks, int param_blocks,
+                                                                  LoraDIn part, const float* __restrict__ partial, LoraReduceOut out) {
     const int H = C / HEAD;
-    const int h = blockIdx.y;
+    if (blockIdx.x < (unsigned)din_blocks) {
+        const long n8 = M * D / 8;
+        const long e = blockIdx.x * 256L + threadIdx.x;
+        if (e >= 4 * n8) return;
+        const int i = (int)(e / n8);
+        const long r = (e % n8) * 8;          // element offset in [M][D]
+        const long m = r / D;
+        const int d = (int)(r % D);
+        float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        const __bf16* src = part.p[i] + m * H * D + d;
+        for (int h = 0; h < H; h++) {
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(src + (long)h * D);
+#pragma unroll
+            for (int q = 0; q < 8; q++) acc[q] += (float)v[q];
+        }
+        bf16x8 o;
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = (__bf16)acc[q];
+        *reinterpret_cast<bf16x8*>(out.din[i] + m * out.ld[i] + d) = o;
+        return;
+    }
+    const int b = blockIdx.x - din_blocks;
+    const int h = b / param_blocks;
     const int REC = 4 * HEAD * D + 4 * HEAD;
-    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int e = (b - h * param_blocks) * 256 + threadIdx.x;
     if (e >= REC) return;
-    float s = 0.f;
-    for (int sp = 0; sp < nsplit; sp++) s += partial[((long)sp * H + h) * REC + e];
+    // four running sums, so that four loads are in flight at a time
+    float s4[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* src = partial + (long)h * REC + e;
+    const long pitch = (long)H * REC;
+    int sp = 0;
+    for (; sp + 4 <= nsplit; sp += 4)
+#pragma unroll
+        for (int u = 0; u < 4; u++) s4[u] += src[(sp + u) * pitch];
+    for (; sp < nsplit; sp++) s4[0] += src[sp * pitch];
+    const float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     if (e < 4 * HEAD * D) {
         const int i = e / (HEAD * D), r = e % (HEAD * D);
         out.dW[i][(long)h * HEAD * D + r] = s;
@@ -1068,7 +1078,7 @@ void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in,
 
 void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                   const void* const Ws[4], const void* const biases[4], const void* const dys[4],
-                                  void* dw_in, void* dk_in, void* const dacts[4], void* const dWs[4],
+                                  void* dw_in, void* dk_in, void* const dacts[4], const long ld_dacts[4], void* const dWs[4],
                                   void* const dbiases[4], void* workspace, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     auto m = [](void* p) { return static_cast<__bf16*>(p); };
@@ -1087,7 +1097,6 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
     const int nsplit = loras_splits(M, H);
     p += A256((size_t)nsplit * H * (4 * HEAD * D + 4 * HEAD) * 4);
     HeadStat* stats = reinterpret_cast<HeadStat*>(p);
-    const LoraDIn dout{{m(dacts[0]), m(dacts[1]), m(dacts[2]), m(dacts[3])}};
     const int tiles_per_split = (int)((M / TOK + nsplit - 1) / nsplit);
     const dim3 grid(H, nsplit), block(256);
 #define WKV_LAUNCH_BWD(ND, STATS)                                                                                       \
@@ -1118,13 +1127,14 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
     else WKV_LAUNCH_BWD(4, false);
 #undef WKV_LAUNCH_BWD
 #undef WKV_LAUNCH_BWD16
-    hipLaunchKernelGGL(expand_loras_din_reduce_kernel, dim3((unsigned)((4 * M * D / 8 + 255) / 256)), dim3(256), 0, stream,
-                       M, H, D, part, dout);
-    const LoraParamOut pout{{f(dWs[0]), f(dWs[1]), f(dWs[2]), f(dWs[3])},
+    const LoraReduceOut out{{m(dacts[0]), m(dacts[1]), m(dacts[2]), m(dacts[3])},
+                            {ld_dacts[0], ld_dacts[1], ld_dacts[2], ld_dacts[3]},
+                            {f(dWs[0]), f(dWs[1]), f(dWs[2]), f(dWs[3])},
                             {f(dbiases[0]), f(dbiases[1]), f(dbiases[2]), f(dbiases[3])}};
-    const int rec = 4 * HEAD * D + 4 * HEAD;
-    hipLaunchKernelGGL(expand_loras_param_reduce_kernel, dim3((rec + 255) / 256, H), dim3(256), 0, stream, C, D, nsplit,
-                       partial, pout);
+    const int rec = 4 * HEAD * D + 4 * HEAD, param_blocks = (rec + 255) / 256;
+    const int din_blocks = (int)((4 * M * D / 8 + 255) / 256);
+    hipLaunchKernelGGL(expand_loras_reduce_kernel, dim3(din_blocks + param_blocks * H), dim3(256), 0, stream, M, C, D, nsplit,
+                       din_blocks, param_blocks, part, partial, out);
 }
 
 }  // namespace wkv

@@ -15,10 +15,10 @@ size_t expand_loras_bwd_workspace_bytes(long M, int C, int D);
 void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                  const void* const Ws[4], const void* const biases[4], void* const outs[4],
                                  hipStream_t stream);
-// dys: dw_out, dk_out, dkk_out, db_out [M, C]; dacts: [M, D] bf16; dWs [C, D] and dbiases [C]: fp32
+// dys: dw_out, dk_out, dkk_out, db_out [M, C]; dacts: [M, D] bf16 with row strides ld_dacts; dWs [C, D] and dbiases [C]: fp32
 void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                   const void* const Ws[4], const void* const biases[4], const void* const dys[4],
-                                  void* dw_in, void* dk_in, void* const dacts[4], void* const dWs[4],
+                                  void* dw_in, void* dk_in, void* const dacts[4], const long ld_dacts[4], void* const dWs[4],
                                   void* const dbiases[4], void* workspace, hipStream_t stream);
 
 }  // namespace wkv

@@ -1,0 +1,305 @@
+// Projections y = x W^T (and input gradients dx = dy W, on the transposed weight) of a block, several in one launch.
+//
+// The reference leaves every product of the block to the BLAS library (time_mixer.py:120-131, :167).  The block has six
+// first-half products on four inputs, two second-half ones, the output projection, and as many input gradients: most are
+// too small to fill the chip on their own, each library call costs 10-15 us of host time, and the library knows neither
+// that two products add up to one input gradient nor that a concatenated output is cut into columns (some through tanh)
+// right after.  Here a launch takes up to eight problems on the same M tokens.  A problem is
+//     D[m][n] = sum over up to two segments of  sum_k A[m][k] W[n][k]
+// with D's columns going to up to four tensors, each as it is, through tanh, or times 1 - aux^2 (the derivative).
+//
+// Both operands lie with the contraction index fastest, so a tile goes from memory to LDS without passing registers
+// (buffer_load ... lds) and from LDS into v_mfma_f32_32x32x16_bf16 as it lies: eight consecutive k of one row per lane and
+// 16-byte read.  The pieces of 16 bytes of a row are permuted by the row number on the way into LDS (by choosing which
+// piece a lane fetches), which makes those reads free of bank conflicts.  A block of four wavefronts (2 x 2) computes
+// 64 TMB tokens x 64 TNB columns; what bounds it is the LDS read rate against the matrix rate: 32 x 32 blocks TMB x TNB
+// per wavefront need TMB + TNB reads of 1 KB for TMB TNB instructions of 32 cycles.  Two blocks share a compute unit, so
+// one's matrix work covers the other's barriers and last loads.
+//
+// Measured (us; in brackets the library's kernels for the same, replayed without host time): six first-half products of a
+// 768-channel block at 2006 / 8192 / 32768 tokens 21 (48) / 51 (70) / 169 (204); three input gradients with one second
+// segment at 8192 43 (66); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.6 (6.8) / 17.9 (16.9) / 92 (69).  Stages of
+// 32 (half lines): 14 % slower at 65536 tokens; 256 x 192 tiles, one block per compute unit, a whole stage's operands in
+// registers: 13 % slower (768 contraction indices are twelve stages, too few to amortise its start and end alone);
+// walking the contraction from different places per tile: 5-15 % slower.
+#include "linear_kernels.hpp"
+#include "device_info.hpp"
+
+#include "frag.hpp"
+
+namespace wkv {
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+using Rsrc = __amdgpu_buffer_rsrc_t;
+
+constexpr int BK = 64;           // contraction indices per stage: whole 128-byte lines of a row
+constexpr int MAX_PROBLEMS = 8;
+
+template <int TMB, int TNB>
+struct Tile {
+    static constexpr int BM = 64 * TMB, BN = 64 * TNB;
+    static constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
+};
+
+struct GroupArgs {
+    LinearProblem p[MAX_PROBLEMS];
+    int first_tile[MAX_PROBLEMS + 1];   // problem j owns tiles first_tile[j] .. first_tile[j+1]-1
+    int shape[MAX_PROBLEMS];            // TNB
+    int M, n;
+};
+
+// STAGES in LDS: two where blocks share a compute unit; four in launches that have less than a block per compute unit, where
+// nothing but a block's own loads in flight covers their latency (512 x 768 x 768: 10.5 -> 8.9 us).
+template <int TMB, int TNB, int STAGES>
+__device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProblem& p, const int M, const int m0, const int n0) {
+    using S = Tile<TMB, TNB>;
+    constexpr int CPR = BK / 8;                      // 16-byte pieces per row
+    constexpr int RPP = 256 / CPR;                   // rows per pass of the block
+    constexpr int QA = S::BM / RPP, QB = S::BN / RPP, LOADS = QA + QB;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int lrow = tid / CPR;                      // this thread's row in a pass
+    auto swizzle = [](int row) { return row & 7; };
+    static_assert(CPR == 8, "a row of a stage is one 128-byte line");
+    const int piece = (tid % CPR) ^ swizzle(lrow);   // the piece of the row it fetches (RPP is a multiple of 8: the same in every pass)
+
+    f32x16 acc[TMB][TNB];
+#pragma unroll
+    for (int mb = 0; mb < TMB; mb++)
+#pragma unroll
+        for (int nb = 0; nb < TNB; nb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[mb][nb][r] = 0.f;
+
+    // stages of both segments in a row
+    const int nk0 = (p.K[0] + BK - 1) / BK, nk = nk0 + (p.K[1] + BK - 1) / BK;
+    Rsrc ra, rb;
+    unsigned aoff[QA], boff[QB];
+    int kseg = 0;
+    auto enter_segment = [&](int g) {   // descriptors at the tile's first rows; rows past the ends repeat the last
+        ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.A[g] + (long)m0 * p.lda[g]), 0, 0x7fffffff, 0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.W[g] + (long)n0 * p.ldw[g]), 0, 0x7fffffff, 0x00020000);
+#pragma unroll
+        for (int q = 0; q < QA; q++) aoff[q] = (unsigned)min(lrow + RPP * q, M - 1 - m0) * (unsigned)p.lda[g] * 2;
+#pragma unroll
+        for (int q = 0; q < QB; q++) boff[q] = (unsigned)min(lrow + RPP * q, p.N - 1 - n0) * (unsigned)p.ldw[g] * 2;
+        kseg = p.K[g];
+    };
+    auto k_of = [&](int kt) { return BK * (kt >= nk0 ? kt - nk0 : kt); };
+    auto issue = [&](int kt) {
+        if (kt == nk0) enter_segment(1);
+        const int k0 = k_of(kt);
+        const int c = k0 + 8 * piece < kseg ? k0 + 8 * piece : k0;   // (past the segment's end: a piece that is not used)
+        unsigned char* dst = lds + (kt % STAGES) * S::STAGE_BYTES + wave * 1024;
+#pragma unroll
+        for (int q = 0; q < QA; q++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst + q * 4096, 16, aoff[q] + 2 * c, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < QB; q++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, dst + S::BM * BK * 2 + q * 4096, 16, boff[q] + 2 * c, 0, 0, 0);
+    };
+    // operand reads: lane = row (lane % 32) of a 32-row block, k = 16 ks + 8 (lane / 32) ..
+    const int r32 = lane & 31, half = lane >> 5;
+    int rd[BK / 16];
+#pragma unroll
+    for (int ks = 0; ks < BK / 16; ks++) rd[ks] = r32 * (BK * 2) + (((2 * ks + half) ^ swizzle(r32)) << 4);
+    const int a_base = wm * TMB * 32 * BK * 2, b_base = S::BM * BK * 2 + wn * TNB * 32 * BK * 2;
+
+    // a stage of every wavefront has arrived when at most `after` stages behind it are on their way, and nobody reads the one
+    // before it any more (own LDS reads are waited for: their consumers could be scheduled behind the barrier)
+    auto arrived = [&](int after) {
+        if (STAGES > 3 && after >= 3)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(3 * LOADS) : "memory");
+        else if (STAGES > 2 && after == 2)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LOADS) : "memory");
+        else if (after == 1)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    enter_segment(0);
+    // Operands of a 16-wide step are read from LDS while the step before multiplies, across stages too: the barrier for
+    // stage kt + 1 stands before the last step of stage kt, whose operands are in registers by then, so that stage's place
+    // is free for stage kt + STAGES right there.
+    constexpr int KS = BK / 16;
+    bf16x8 a[2][TMB], b[2][TNB];
+    auto read = [&](int set, int kt, int ks) {
+        const unsigned char* st = lds + (kt % STAGES) * S::STAGE_BYTES;
+#pragma unroll
+        for (int mb = 0; mb < TMB; mb++) a[set][mb] = *reinterpret_cast<const bf16x8*>(st + a_base + mb * 32 * BK * 2 + rd[ks]);
+#pragma unroll
+        for (int nb = 0; nb < TNB; nb++) b[set][nb] = *reinterpret_cast<const bf16x8*>(st + b_base + nb * 32 * BK * 2 + rd[ks]);
+        if (ks > 0 && 16 * ks >= p.K[kt >= nk0 ? 1 : 0] - k_of(kt)) {   // past a segment's end: zeros
+#pragma unroll
+            for (int mb = 0; mb < TMB; mb++) a[set][mb] = bf16x8{};
+#pragma unroll
+            for (int nb = 0; nb < TNB; nb++) b[set][nb] = bf16x8{};
+        }
+    };
+#pragma unroll
+    for (int st = 0; st < STAGES; st++)
+        if (st < nk) issue(st);
+    arrived(min(nk - 1, STAGES - 1));
+    read(0, 0, 0);
+    for (int kt = 0; kt < nk; kt++) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks < KS - 1) {
+                read((ks + 1) & 1, kt, ks + 1);
+            } else if (kt + 1 < nk) {
+                arrived(min(nk - 2 - kt, STAGES - 2));
+                if (kt + STAGES < nk) issue(kt + STAGES);
+                read((ks + 1) & 1, kt + 1, 0);
+            }
+#pragma unroll
+            for (int mb = 0; mb < TMB; mb++)
+#pragma unroll
+                for (int nb = 0; nb < TNB; nb++)
+                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[ks & 1][nb], a[ks & 1][mb], acc[mb][nb], 0, 0, 0);
+        }
+    }
+    // Register r of lane l of block (mb, nb): token 32 mb + l % 32, column 32 nb + 8 (r / 4) + 4 (l / 32) + r % 4.  Two lanes
+    // swap their halves so that a lane has eight consecutive columns of a token; the wavefront's tile then goes through LDS
+    // and leaves in rows (as it lies in registers every store would touch 32 rows for 32 bytes each: 8192 x 768 x 64, which
+    // is all output, 13 us instead of 9).
+    constexpr int CH = 4 * TNB, PITCH = 32 * TNB * 2 + 16;   // 16-byte pieces per row of the wavefront; its LDS row, bank-shifted
+    static_assert(4 * 32 * TMB * PITCH <= STAGES * (64 * TMB + 64 * TNB) * BK * 2, "the output tile fits where the stages were");
+    arrived(0);
+    unsigned char* const mine = lds + wave * (32 * TMB * PITCH);
+#pragma unroll
+    for (int mb = 0; mb < TMB; mb++)
+#pragma unroll
+        for (int nb = 0; nb < TNB; nb++)
+#pragma unroll
+            for (int pr = 0; pr < 2; pr++) {
+                const f32x16& x = acc[mb][nb];
+                const u32x2 lo = __builtin_bit_cast(u32x2, pack_bf16(x[8 * pr], x[8 * pr + 1], x[8 * pr + 2], x[8 * pr + 3]));
+                const u32x2 hi = __builtin_bit_cast(u32x2, pack_bf16(x[8 * pr + 4], x[8 * pr + 5], x[8 * pr + 6], x[8 * pr + 7]));
+                // lanes below 32 take columns 0 .. 7 of the sixteen, the others 8 .. 15
+                const auto s0 = __builtin_amdgcn_permlane32_swap(lo[0], hi[0], false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(lo[1], hi[1], false, false);
+                typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+                *reinterpret_cast<u32x4*>(mine + (32 * mb + r32) * PITCH + (4 * nb + 2 * pr + half) * 16) = (u32x4){s0[0], s1[0], s0[1], s1[1]};
+            }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wavefront reads what it wrote itself)
+    auto rows_of = [&](int i, int& m, int& col) -> const bf16x8* {
+        const int id = lane + 64 * i, row = id / CH, ch = id % CH;
+        m = m0 + 32 * TMB * wm + row, col = n0 + 32 * TNB * wn + 8 * ch;
+        return reinterpret_cast<const bf16x8*>(mine + row * PITCH + ch * 16);
+    };
+    if (p.npieces == 1 && p.op[0] == LINEAR_PLAIN) {
+#pragma unroll
+        for (int i = 0; i < 2 * TMB * TNB; i++) {
+            int m, col;
+            const bf16x8* v = rows_of(i, m, col);
+            if (m < M && col < p.N) *reinterpret_cast<bf16x8*>(p.out[0] + (long)m * p.ld_out[0] + col) = *v;
+        }
+        return;
+    }
+#pragma unroll 1
+    for (int i = 0; i < 2 * TMB * TNB; i++) {
+        int m, col;
+        const bf16x8* src = rows_of(i, m, col);
+        if (m >= M || col >= p.N) continue;
+        int t = 0;   // the output tensor these columns belong to (eight columns lie in one)
+#pragma unroll
+        for (int k = 1; k < LinearProblem::PIECES; k++) t += k < p.npieces && col >= p.start[k] ? 1 : 0;
+        auto of = [&](auto f) {
+            auto r = f(0);
+#pragma unroll
+            for (int k = 1; k < LinearProblem::PIECES; k++) r = t == k ? f(k) : r;
+            return r;
+        };
+        const int c = col - of([&](int k) { return p.start[k]; }), op = of([&](int k) { return p.op[k]; });
+        bf16x8 v = *src;
+        if (op != LINEAR_PLAIN) {
+            bf16x8 y = {};
+            if (op == LINEAR_TANH_GRAD)
+                y = *reinterpret_cast<const bf16x8*>(of([&](int k) { return p.aux[k]; }) + (long)m * of([&](int k) { return p.width[k]; }) + c);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float f = (float)v[e], g = (float)y[e];
+                v[e] = (__bf16)(op == LINEAR_TANH ? tanhf(f) : f * (1.f - g * g));
+            }
+        }
+        *reinterpret_cast<bf16x8*>(of([&](int k) { return p.out[k]; }) + (long)m * of([&](int k) { return p.ld_out[k]; }) + c) = v;
+    }
+}
+
+template <int TMB, int STAGES>
+__global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void linear_group_kernel(const GroupArgs G) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[STAGES * Tile<TMB, 3>::STAGE_BYTES];
+    // Blocks go to the eight XCDs in turn (block b to XCD b % 8), and each XCD has an L2 of its own.  An XCD takes a run of
+    // consecutive tiles, i.e. some row blocks of a problem with all their column blocks: it reads each of its rows of the
+    // input once and keeps the weight.
+    const int nt = G.first_tile[G.n];
+    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
+    int t = -1;
+    {   // problem by problem: tiles of XCD x are [T x / 8, T (x+1) / 8) of each problem's T
+        int rest = i;
+#pragma unroll 1
+        for (int j = 0; j < G.n && t < 0; j++) {
+            const int T = G.first_tile[j + 1] - G.first_tile[j];
+            const int lo = T * x / 8, hi = T * (x + 1) / 8;
+            if (rest < hi - lo) t = G.first_tile[j] + lo + rest;
+            else rest -= hi - lo;
+        }
+    }
+    if (t < 0 || t >= nt) return;   // (whole block)
+    int j = 0;
+#pragma unroll
+    for (int k = 1; k < MAX_PROBLEMS; k++) j += (k < G.n && t >= G.first_tile[k]) ? 1 : 0;
+    const LinearProblem& p = G.p[j];
+    const int bn = 64 * G.shape[j], ncol = (p.N + bn - 1) / bn;
+    const int tile = t - G.first_tile[j];
+    const int m0 = tile / ncol * (64 * TMB), n0 = tile % ncol * bn;
+    switch (G.shape[j]) {
+        case 1: gemm_tile<TMB, 1, STAGES>(lds, p, G.M, m0, n0); break;
+        case 2: gemm_tile<TMB, 2, STAGES>(lds, p, G.M, m0, n0); break;
+        default: gemm_tile<TMB, 3, STAGES>(lds, p, G.M, m0, n0); break;
+    }
+}
+
+}  // namespace
+
+void launch_linear_group(int n, long M, const LinearProblem* problems, hipStream_t stream) {
+    GroupArgs G{};
+    G.n = n;
+    G.M = (int)M;
+    // Columns per block (64 times this): as many of a problem's as the shape allows, since wide tiles read least per product.
+    auto plan = [&](int rows, int widest) {
+        G.first_tile[0] = 0;
+        for (int j = 0; j < n; j++) {
+            const int N = problems[j].N, blocks = (N + 63) / 64;
+            G.shape[j] = blocks < widest ? blocks : widest == 3 && N % 192 != 0 && N <= 256 ? 2 : widest;
+            const int bn = 64 * G.shape[j];
+            G.first_tile[j + 1] = G.first_tile[j] + (int)((M + rows - 1) / rows) * ((N + bn - 1) / bn);
+        }
+        return G.first_tile[n];
+    };
+    for (int j = 0; j < n; j++) G.p[j] = problems[j];
+    // 128 tokens x 192 columns where that gives every compute unit a block; else 64 tokens, and narrower until most have one
+    const int enough = compute_units() * 3 / 4;
+    const bool small = plan(128, 3) < compute_units();
+    if (small && plan(64, 3) < enough && plan(64, 2) < enough) plan(64, 1);
+    // the largest share of an XCD, times eight
+    int most = 0;
+    for (int x = 0; x < 8; x++) {
+        int c = 0;
+        for (int j = 0; j < n; j++) {
+            const int T = G.first_tile[j + 1] - G.first_tile[j];
+            c += T * (x + 1) / 8 - T * x / 8;
+        }
+        most = c > most ? c : most;
+    }
+    const dim3 grid(8 * most), block(256);
+    if (!small) hipLaunchKernelGGL((linear_group_kernel<2, 2>), grid, block, 0, stream, G);
+    else if (G.first_tile[n] > compute_units()) hipLaunchKernelGGL((linear_group_kernel<1, 2>), grid, block, 0, stream, G);
+    else hipLaunchKernelGGL((linear_group_kernel<1, 4>), grid, block, 0, stream, G);
+}
+
+}  // namespace wkv

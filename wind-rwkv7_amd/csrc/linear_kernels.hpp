@@ -48,4 +48,32 @@ void launch_cast_to_bf16(int n, const void* const* src, const int* src_f32, cons
 // rows first .. T-1 of w, k, b [B, T, C] (bf16): decay 1, k = b = 0
 void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, hipStream_t stream);
 
+// dst [rows, cols] (bf16, or f32 where dst_f32) from src (f32 or bf16); dstT: null or the transposed bf16 copy, row stride ldT
+struct PackTensor {
+    const void* src;
+    void *dst, *dstT;
+    int rows, cols;
+    long ldT;
+    int src_f32, dst_f32;
+};
+constexpr int PACK_MAX_TENSORS = 32;
+void launch_pack_weights(int n, const PackTensor* tensors, hipStream_t stream);
+
+// D[m][n] = sum_k A0[m][k] W0[n][k] (+ sum_k A1[m][k] W1[n][k]); see linear_group.hip.  K[1] = 0: one segment.  The columns
+// start[t] .. start[t] + width[t] - 1 go to out[t] (row stride ld_out[t]); aux[t]: [M, width[t]].
+enum { LINEAR_PLAIN = 0, LINEAR_TANH = 1, LINEAR_TANH_GRAD = 2 };
+struct LinearProblem {
+    static constexpr int PIECES = 4;
+    const __bf16* A[2];
+    const __bf16* W[2];
+    long lda[2], ldw[2];
+    int K[2];
+    int N, npieces;
+    __bf16* out[PIECES];
+    const __bf16* aux[PIECES];
+    long ld_out[PIECES];
+    int start[PIECES], width[PIECES], op[PIECES];
+};
+void launch_linear_group(int n, long M, const LinearProblem* problems, hipStream_t stream);
+
 }  // namespace wkv

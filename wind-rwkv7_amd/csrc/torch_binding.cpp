@@ -36,9 +36,9 @@ namespace py = pybind11;
     X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward)                             \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
-    X(ddlerp_forward_from) X(neutral_rows) X(copy_columns) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(ddlerp_forward_from) X(neutral_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
-    X(mixer_prompt)
+    X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
 struct Lib {
 #define X(name) decltype(&wind_rwkv7_##name) name = nullptr;
@@ -543,19 +543,59 @@ struct ParamLayout {
     }
 };
 
+// The weights as the kernels take them, in one buffer (bf16 elements): copies of all of them in ParamLayout's places, the
+// [3, C] float32 parameters of attn_ln, and for a backward pass the transposed copies of the projections' weights.
+struct WeightLayout {
+    ParamLayout at_;
+    int64_t C, ln, Tr, Tk, Tv, To, Tg1, Tkkmk, Tw1, Tg2, Tw2, total[2];   // total[whether the transposed copies are there]
+    explicit WeightLayout(int64_t C_) : at_(C_), C(C_) {
+        int64_t o = at_.at[LN_W];
+        auto take = [&](int64_t n) { const int64_t r = o; o += n; return r; };
+        ln = take(2 * 3 * C);
+        total[0] = o;
+        Tr = take(C * C), Tk = take(C * C), Tv = take(C * C), To = take(C * C);
+        Tg1 = take(C * R_GATE), Tkkmk = take(C * W_KKMK), Tw1 = take(C * W_DECAY_AAA_MA), Tg2 = take(C * R_GATE), Tw2 = take(C * R_DECAY);
+        total[1] = o;
+    }
+};
+using B16 = c10::BFloat16;
+B16* at_elem(const Tensor& t, int64_t o) { return static_cast<B16*>(t.data_ptr()) + o; }
+
+void pack_weights(const WeightLayout& L_, const variable_list& p, const Tensor& buf, bool transposed) {
+    wind_rwkv7_pack t[PARAMS];
+    for (int i = 0; i < PARAMS; i++) {
+        const auto shape = param_shape(i, L_.C);
+        const bool norm = i >= WEIGHTS;
+        t[i].src = p[i].data_ptr();
+        t[i].src_dtype = p[i].scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
+        t[i].dst_dtype = norm ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
+        t[i].dst = at_elem(buf, norm ? L_.ln + 2 * (L_.at_.at[i] - L_.at_.at[LN_W]) : L_.at_.at[i]);
+        t[i].cols = (int)shape.back();
+        t[i].rows = (int)(p[i].numel() / shape.back());
+        t[i].dstT = nullptr;
+        t[i].ldT = 0;
+    }
+    if (transposed) {
+        auto turn = [&](int i, int64_t at, int64_t ld) { t[i].dstT = at_elem(buf, at), t[i].ldT = ld; };
+        turn(WR, L_.Tr, L_.C), turn(WK, L_.Tk, L_.C), turn(WV, L_.Tv, L_.C), turn(WO, L_.To, L_.C);
+        turn(GATE_W1, L_.Tg1, R_GATE), turn(GATE_W2, L_.Tg2, L_.C), turn(DECAY_W2, L_.Tw2, L_.C);
+        turn(KKK_W1, L_.Tkkmk, W_KKMK), turn(MK_W1, L_.Tkkmk + R_LORA, W_KKMK);
+        turn(DECAY_W1, L_.Tw1, W_DECAY_AAA_MA), turn(AAA_W1, L_.Tw1 + R_DECAY, W_DECAY_AAA_MA);
+        turn(MA_W1, L_.Tw1 + R_DECAY + R_LORA, W_DECAY_AAA_MA);
+    }
+    check(L.pack_weights(PARAMS, t, stream_of(buf)));
+}
+
 struct Block {   // the sizes of a call
     int64_t B, T, C, H;
     int64_t rows() const { return B * T; }
     int64_t N() const { return C / H; }
     int64_t plane() const { return rows() * C; }
 };
-using B16 = c10::BFloat16;
-B16* at_elem(const Tensor& t, int64_t o) { return static_cast<B16*>(t.data_ptr()) + o; }
-Tensor matrix(const Tensor& buf, int64_t offset, int64_t rows, int64_t cols) { return buf.as_strided({rows, cols}, {cols, 1}, offset); }
 
 // Activations of a block in one buffer; offsets in elements (all multiples of 256: rows() is a multiple of 16).
 struct Activations {
-    int64_t streams, r, k, v, g, w2, w, k2, kk, b, ya, mid, der, tg1, tw1, kk1, mk1, a1, ma1, kept, g1, kkmk, w1a1ma1, total;
+    int64_t streams, r, k, v, g, w2, w, k2, kk, b, ya, mid, der, tg1, tw1, kk1, mk1, a1, ma1, total;
     explicit Activations(const Block& s) {
         int64_t o = 0;
         auto take = [&](int64_t n) { const int64_t r = o; o += n; return r; };
@@ -565,25 +605,44 @@ struct Activations {
         mid = take(4 * R_MIX * M), der = take(4 * R_MIX * M);
         tg1 = take(R_GATE * M), tw1 = take(R_DECAY * M);
         kk1 = take(R_LORA * M), mk1 = take(R_LORA * M), a1 = take(R_LORA * M), ma1 = take(R_LORA * M);
-        kept = o;
-        g1 = take(R_GATE * M), kkmk = take(W_KKMK * M), w1a1ma1 = take(W_DECAY_AAA_MA * M);   // dead once they are split
         total = o;
     }
 };
 
-// column slices in one launch (wind_rwkv7_copy_columns)
-struct Columns {
-    std::vector<const void*> src, aux;
-    std::vector<void*> dst;
-    std::vector<long long> src_ld, dst_ld;
-    std::vector<int> src_col, dst_col, width, op;
-    void add(const void* s, int sld, int sc, void* d, int dld, int dc, int w, int o, const void* x = nullptr) {
-        src.push_back(s), src_ld.push_back(sld), src_col.push_back(sc), dst.push_back(d), dst_ld.push_back(dld), dst_col.push_back(dc);
-        width.push_back(w), op.push_back(o), aux.push_back(x);
+// Products out = in W^T on the same rows in one launch (wind_rwkv7_linear_group).  The library's kernel for a single large
+// product is the better one by a quarter where each fills the chip several times over (65536 x 768 x 768: 70 us against 92;
+// 32768 rows as a group of six: 204 against 169), so there a large product goes to it.
+struct Products {
+    static constexpr double LIBRARY_FROM = 2.5e10;   // rows x columns x contraction length
+    std::vector<wind_rwkv7_linear> ps;
+    void add(const void* in, const void* W, int64_t K, int64_t N) {
+        wind_rwkv7_linear p{};
+        p.A[0] = in, p.W[0] = W, p.lda[0] = p.ldw[0] = K, p.K[0] = (int)K;
+        p.N = (int)N;
+        ps.push_back(p);
     }
-    void run(int64_t rows, void* stream) {
-        check(L.copy_columns(rows, (int)dst.size(), src.data(), src_ld.data(), src_col.data(), dst.data(), dst_ld.data(), dst_col.data(),
-                             width.data(), op.data(), aux.data(), stream));
+    void plus(const void* in, const void* W, int64_t K) {
+        auto& p = ps.back();
+        p.A[1] = in, p.W[1] = W, p.lda[1] = p.ldw[1] = K, p.K[1] = (int)K;
+    }
+    void to(void* out, int64_t width, int op = 0, const void* aux = nullptr, int64_t ld = 0) {
+        auto& p = ps.back();
+        const int t = p.npieces++;
+        p.out[t] = out, p.width[t] = (int)width, p.ld_out[t] = ld ? ld : width, p.op[t] = op, p.aux[t] = aux;
+    }
+    void run(int64_t rows, const Tensor& like) {
+        std::vector<wind_rwkv7_linear> group;
+        for (const auto& p : ps) {
+            if ((double)rows * p.N * p.K[0] < LIBRARY_FROM || p.npieces > 1 || p.op[0]) {
+                group.push_back(p);
+                continue;
+            }
+            auto view = [&](const void* q, int64_t r, int64_t c) { return at::from_blob(const_cast<void*>(q), {r, c}, like.options()); };
+            Tensor out = view(p.out[0], rows, p.N);
+            at::mm_out(out, view(p.A[0], rows, p.K[0]), view(p.W[0], p.N, p.K[0]).t());
+            if (p.K[1]) at::addmm_out(out, out, view(p.A[1], rows, p.K[1]), view(p.W[1], p.N, p.K[1]).t());
+        }
+        if (!group.empty()) check(L.linear_group((int)group.size(), rows, group.data(), stream_of(like)));
     }
 };
 
@@ -610,91 +669,133 @@ struct WeightGrads {
     }
 };
 
-// bf16 copies of the block's weights in one launch, and its [3,C] float32 parameters of attn_ln
-struct BlockWeights {
-    Tensor flat, ln;
-    ParamLayout at_;
-    BlockWeights(const variable_list& p, const Tensor& like) : at_(like.size(-1)) {
-        flat = at::empty({at_.at[LN_W]}, like.options().dtype(at::kBFloat16));
-        const void* src[WEIGHTS];
-        int dtype[WEIGHTS];
-        long long numel[WEIGHTS], offset[WEIGHTS];
-        for (int i = 0; i < WEIGHTS; i++) {
-            src[i] = p[i].data_ptr();
-            dtype[i] = p[i].scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16;
-            numel[i] = p[i].numel();
-            offset[i] = at_.at[i];
-        }
-        check(L.cast_to_bf16(WEIGHTS, src, dtype, numel, offset, flat.data_ptr(), stream_of(flat)));
-        ln = at::stack({p[LN_W], p[LN_B], p[FAAAA]}).to(at::kFloat);
+// What a forward pass leaves: the caller's results and what a backward pass needs.
+struct BlockBuffers {
+    Tensor weights, acts, saved, y, sT;
+    static int64_t saved_bytes(const Block& s) { return L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()); }
+    BlockBuffers(const Block& s, const Tensor& xb, bool save, at::ScalarType state_type) {
+        weights = at::empty({WeightLayout(s.C).total[save]}, xb.options());
+        acts = at::empty({Activations(s).total}, xb.options());
+        saved = scratch_bytes(saved_bytes(s), xb);
+        y = at::empty({s.B, s.T, s.C}, xb.options());
+        sT = at::empty({s.B, s.H, s.N(), s.N()}, xb.options().dtype(state_type));
     }
-    void* w(int i) const { return at_elem(flat, at_.at[i]); }
-};
-
-struct BlockForward {   // what one forward pass leaves
-    Tensor xb, weights, lnp, acts, saved, y, sT;
+    BlockBuffers(Tensor w, Tensor a, Tensor s, Tensor y_, Tensor st)
+        : weights(std::move(w)), acts(std::move(a)), saved(std::move(s)), y(std::move(y_)), sT(std::move(st)) {}
 };
 
 // x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  `valid` < T: the tokens from
 // there on are padding and leave the state as it is.  x_prev [B,C] bf16 / s0: a carried state (undefined: zero).
-BlockForward block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const Tensor& x_prev,
-                           const Tensor& s0, at::ScalarType state_type) {
+void block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const Tensor& x_prev,
+                   const Tensor& s0, const BlockBuffers& f) {
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
-    const int64_t M = s.rows();
+    const int64_t M = s.rows(), P = s.plane();
     void* stream = stream_of(xb);
-    const ParamLayout at_(C);
-    BlockForward f;
-    f.xb = xb;
-    const BlockWeights bw(p, xb);
-    f.weights = bw.flat;
-    f.lnp = bw.ln;
+    const WeightLayout W(C);
     const Activations A(s);
-    f.acts = at::empty({save ? A.kept : A.total}, xb.options());
-    // (training keeps the activations: the concatenated first halves, which nothing needs later, go to a buffer of their own)
-    const Tensor firsts = save ? at::empty({A.total - A.kept}, xb.options()) : f.acts;
-    const int64_t shift = save ? A.kept : 0;
+    pack_weights(W, p, f.weights, save);
     auto a = [&](int64_t o) -> void* { return at_elem(f.acts, o); };
-    auto w = [&](int i) -> void* { return at_elem(f.weights, at_.at[i]); };
-    auto weight = [&](int i, int64_t rows, int64_t cols) { return matrix(f.weights, at_.at[i], rows, cols); };
-    auto times = [&](const Tensor& out, int64_t in_off, int64_t in_cols, const Tensor& wt) {
-        Tensor o = out;
-        at::mm_out(o, matrix(f.acts, in_off, M, in_cols), wt.t());
-    };
+    auto w = [&](int i) -> void* { return at_elem(f.weights, W.at_.at[i]); };
     check(L.ddlerp_forward_from(B, T, C, R_MIX, ptr(xb), ptr(x_prev), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), a(A.streams),
                                 stream));
-    const int64_t P = s.plane(), xrg = A.streams, xwa = A.streams + P, xk = A.streams + 2 * P, xv = A.streams + 3 * P;
-    const Tensor g1 = matrix(firsts, A.g1 - shift, M, R_GATE), kkmk = matrix(firsts, A.kkmk - shift, M, W_KKMK),
-                 w1a1ma1 = matrix(firsts, A.w1a1ma1 - shift, M, W_DECAY_AAA_MA);
-    times(matrix(f.acts, A.r, M, C), xrg, C, weight(WR, C, C));
-    times(g1, xrg, C, weight(GATE_W1, R_GATE, C));
-    times(matrix(f.acts, A.k, M, C), xk, C, weight(WK, C, C));
-    times(kkmk, xk, C, weight(KKK_W1, W_KKMK, C));
-    times(matrix(f.acts, A.v, M, C), xv, C, weight(WV, C, C));
-    times(w1a1ma1, xwa, C, weight(DECAY_W1, W_DECAY_AAA_MA, C));
-    Columns cols;
-    cols.add(ptr(kkmk), W_KKMK, 0, a(A.kk1), R_LORA, 0, R_LORA, 0);
-    cols.add(ptr(kkmk), W_KKMK, R_LORA, a(A.mk1), R_LORA, 0, R_LORA, 0);
-    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, 0, a(A.tw1), R_DECAY, 0, R_DECAY, 1);
-    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, R_DECAY, a(A.a1), R_LORA, 0, R_LORA, 0);
-    cols.add(ptr(w1a1ma1), W_DECAY_AAA_MA, R_DECAY + R_LORA, a(A.ma1), R_LORA, 0, R_LORA, 0);
-    cols.add(ptr(g1), R_GATE, 0, a(A.tg1), R_GATE, 0, R_GATE, 1);
-    cols.run(M, stream);
-    times(matrix(f.acts, A.g, M, C), A.tg1, R_GATE, weight(GATE_W2, C, R_GATE));
-    times(matrix(f.acts, A.w2, M, C), A.tw1, R_DECAY, weight(DECAY_W2, C, R_DECAY));
+    const void *xrg = a(A.streams), *xwa = a(A.streams + P), *xk = a(A.streams + 2 * P), *xv = a(A.streams + 3 * P);
+    {
+        Products first;
+        first.add(xrg, w(WR), C, C), first.to(a(A.r), C);
+        first.add(xk, w(WK), C, C), first.to(a(A.k), C);
+        first.add(xv, w(WV), C, C), first.to(a(A.v), C);
+        first.add(xrg, w(GATE_W1), C, R_GATE), first.to(a(A.tg1), R_GATE, 1);
+        first.add(xwa, w(DECAY_W1), C, W_DECAY_AAA_MA);
+        first.to(a(A.tw1), R_DECAY, 1), first.to(a(A.a1), R_LORA), first.to(a(A.ma1), R_LORA);
+        first.add(xk, w(KKK_W1), C, W_KKMK), first.to(a(A.kk1), R_LORA), first.to(a(A.mk1), R_LORA);
+        first.run(M, xb);
+        Products second;
+        second.add(a(A.tg1), w(GATE_W2), R_GATE, C), second.to(a(A.g), C);
+        second.add(a(A.tw1), w(DECAY_W2), R_DECAY, C), second.to(a(A.w2), C);
+        second.run(M, xb);
+    }
     check(L.expand_loras_forward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
                                  w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b), stream));
     if (valid < T) check(L.neutral_rows(B, T, C, (int)valid, a(A.w), a(A.k2), a(A.b), stream));
-    f.sT = at::empty({B, H, N, N}, xb.options().dtype(state_type));
-    const size_t ws = std::max<size_t>(L.attn_ln_fwd_workspace_bytes(B, T, H, N), 256);
-    const size_t keep_bytes = (L.attn_ln_saved_bytes(B, T, H, N) + 255) / 256 * 256;
-    f.saved = scratch_bytes(keep_bytes + ws, xb);
-    char* base = static_cast<char*>(f.saved.data_ptr());
+    const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
     check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
-        B, T, H, N, WIND_RWKV7_BF16, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b),
-        a(A.g), ptr(f.lnp), ptr(s0), a(A.ya), base, ptr(f.sT), base + keep_bytes, ws, stream));
-    f.y = at::empty({B, T, C}, xb.options());
-    times(f.y.view({M, C}), A.ya, C, weight(WO, C, C));
-    return f;
+        B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln), ptr(s0),
+        a(A.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
+    Products out;
+    out.add(a(A.ya), w(WO), C, C), out.to(ptr(f.y), C);
+    out.run(M, xb);
+}
+
+// dx and the gradient of every parameter (ParamLayout's places in `flat`, float32); need(i): whether parameter i's is wanted.
+template <class Need>
+void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout,
+                    const Tensor& dx, const Tensor& flat, const Need& need) {
+    const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
+    const int64_t M = s.rows(), P = s.plane();
+    void* stream = stream_of(xb);
+    const WeightLayout W(C);
+    const Activations A(s);
+    // gradients of activations: nine planes, reused as they are consumed, and the gradients of the three first halves
+    const int64_t o_g1 = 9 * P, o_kkmk = o_g1 + R_GATE * M, o_w1 = o_kkmk + W_KKMK * M, total = o_w1 + W_DECAY_AAA_MA * M;
+    const Tensor buf = at::empty({total}, xb.options());
+    auto a = [&](int64_t o) -> void* { return at_elem(acts, o); };
+    auto d = [&](int64_t o) -> void* { return at_elem(buf, o); };
+    auto w = [&](int i) -> void* { return at_elem(weights, W.at_.at[i]); };
+    auto t = [&](int64_t o) -> void* { return at_elem(weights, o); };
+    auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + W.at_.at[i]; };
+    size_t ws_bytes = L.attn_ln_bwd_workspace_bytes(B, T, H, N);
+    ws_bytes = std::max(ws_bytes, L.expand_loras_bwd_workspace_bytes(B, T, C, R_LORA));
+    ws_bytes = std::max(ws_bytes, L.ddlerp_bwd_workspace_bytes(B, T, C, R_MIX));
+    const Tensor ws = scratch_bytes(ws_bytes, xb);
+
+    // planes: 0 dya then dw2, 1 dr, 2 dw, 3 dk', 4 dv, 5 dkk, 6 db, 7 dg, 8 dk
+    {
+        Products p;
+        p.add(ptr(dout), t(W.To), C, C), p.to(d(0), C);
+        p.run(M, xb);
+        WeightGrads wg;
+        if (need(WO)) wg.add(ptr(dout), C, a(A.ya), C, g(WO));
+        wg.run(M, xb, stream);
+    }
+    check(L.attn_ln_backward(B, T, H, N, WIND_RWKV7_BF16, WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), t(W.ln), d(0),
+                             ptr(saved), nullptr, d(2 * P), d(P), d(3 * P), d(4 * P), d(5 * P), d(6 * P), d(7 * P), g(LN_W), nullptr, ptr(ws),
+                             ws.numel(), stream));
+    B16 *dkkmk = at_elem(buf, o_kkmk), *dw1 = at_elem(buf, o_w1);
+    const long long ld_din[4] = {W_KKMK, W_DECAY_AAA_MA, W_DECAY_AAA_MA, W_KKMK};
+    check(L.expand_loras_backward_to(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
+                                     w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), d(2 * P), d(3 * P), d(5 * P), d(6 * P), d(0), d(8 * P),
+                                     dkkmk, dw1 + R_DECAY, dw1 + R_DECAY + R_LORA, dkkmk + R_LORA, ld_din, g(KKK_W2), g(AAA_W2), g(MA_W2),
+                                     g(MK_W2), g(DECAY), g(AAAAA), g(MISC_A), g(MISC_K), ptr(ws), ws.numel(), stream));
+    {
+        Products p;   // through the derivative of the tanh between the halves
+        p.add(d(7 * P), t(W.Tg2), C, R_GATE), p.to(d(o_g1), R_GATE, 2, a(A.tg1));
+        p.add(d(0), t(W.Tw2), C, R_DECAY), p.to(dw1, R_DECAY, 2, a(A.tw1), W_DECAY_AAA_MA);
+        p.run(M, xb);
+        WeightGrads wg;
+        if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
+        if (need(DECAY_W2)) wg.add(d(0), C, a(A.tw1), R_DECAY, g(DECAY_W2));
+        wg.run(M, xb, stream);
+    }
+    // the streams' gradients go to the planes that are free now: 2, 5, 3, 6
+    void *dxrg = d(2 * P), *dxwa = d(5 * P), *dxk = d(3 * P), *dxv = d(6 * P);
+    {
+        Products p;
+        p.add(d(P), t(W.Tr), C, C), p.plus(d(o_g1), t(W.Tg1), R_GATE), p.to(dxrg, C);
+        p.add(d(8 * P), t(W.Tk), C, C), p.plus(dkkmk, t(W.Tkkmk), W_KKMK), p.to(dxk, C);
+        p.add(d(4 * P), t(W.Tv), C, C), p.to(dxv, C);
+        p.add(dw1, t(W.Tw1), W_DECAY_AAA_MA, C), p.to(dxwa, C);
+        p.run(M, xb);
+        WeightGrads wg;
+        if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
+        if (need(GATE_W1)) wg.add(d(o_g1), R_GATE, a(A.streams), C, g(GATE_W1));
+        if (need(WK)) wg.add(d(8 * P), C, a(A.streams + 2 * P), C, g(WK));
+        if (need(KKK_W1) || need(MK_W1)) wg.add(dkkmk, W_KKMK, a(A.streams + 2 * P), C, g(KKK_W1));
+        if (need(WV)) wg.add(d(4 * P), C, a(A.streams + 3 * P), C, g(WV));
+        if (need(DECAY_W1) || need(AAA_W1) || need(MA_W1)) wg.add(dw1, W_DECAY_AAA_MA, a(A.streams + P), C, g(DECAY_W1));
+        wg.run(M, xb, stream);
+    }
+    check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), dxrg, dxwa, dxk, dxv, ptr(dx),
+                            g(MAA_X), g(MAA_W1), g(MAA_W2), g(MAA), ptr(ws), ws.numel(), stream));
 }
 
 struct MixerBlock : torch::autograd::Function<MixerBlock> {
@@ -703,8 +804,10 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         at::AutoDispatchBelowADInplaceOrView below;
         const Block s{x.size(0), x.size(1), x.size(2), H};
         const variable_list p{params...};
-        BlockForward f = block_forward(s, x.to(at::kBFloat16).contiguous(), p, true, s.T, Tensor(), Tensor(), at::kBFloat16);
-        ctx->save_for_backward({f.xb, f.weights, f.lnp, f.acts, f.saved});
+        const Tensor xb = x.to(at::kBFloat16).contiguous();
+        const BlockBuffers f(s, xb, true, at::kBFloat16);
+        block_forward(s, xb, p, true, s.T, Tensor(), Tensor(), f);
+        ctx->save_for_backward({xb, f.weights, f.acts, f.saved});
         std::vector<int64_t> types{H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
         for (const auto& t : p) types.push_back((int64_t)t.scalar_type());
         ctx->saved_data["k"] = types;
@@ -713,102 +816,22 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const auto t = ctx->get_saved_variables();
         const auto types = ctx->saved_data["k"].toIntVector();
-        const Tensor &xb = t[0], &weights = t[1], &lnp = t[2], &acts = t[3], &saved = t[4];
+        const Tensor& xb = t[0];
         const Block s{xb.size(0), xb.size(1), xb.size(2), types[0]};
         same_interval({{}, (int)types[1], at::kBFloat16, false});
         c10::DeviceGuard guard(xb.device());
         at::AutoDispatchBelowADInplaceOrView below;
-        const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
-        const int64_t M = s.rows(), P = s.plane();
-        void* stream = stream_of(xb);
-        const ParamLayout at_(C);
-        const Activations A(s);
-        const Tensor dout = grads[0].contiguous();
-        const Tensor flat = at::empty({at_.at[PARAMS]}, xb.options().dtype(at::kFloat));   // every parameter gradient
-        // gradients of activations: nine planes, reused as they are consumed, and the LoRA columns
-        const int64_t lora = 9 * P;
-        const int64_t o_z = lora, o_a1 = o_z + R_LORA * M, o_ma1 = o_a1 + R_LORA * M, o_mk1 = o_ma1 + R_LORA * M, o_tg1 = o_mk1 + R_LORA * M,
-                      o_tw1 = o_tg1 + R_GATE * M, o_g1 = o_tw1 + R_DECAY * M, o_kkmk = o_g1 + R_GATE * M, o_w1 = o_kkmk + W_KKMK * M,
-                      total = o_w1 + W_DECAY_AAA_MA * M;
-        const Tensor buf = at::empty({total}, xb.options());
-        auto a = [&](int64_t o) -> void* { return at_elem(acts, o); };
-        auto d = [&](int64_t o) -> void* { return at_elem(buf, o); };
-        auto w = [&](int i) -> void* { return at_elem(weights, at_.at[i]); };
-        auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + at_.at[i]; };
-        auto weight = [&](int i, int64_t rows, int64_t cols) { return matrix(weights, at_.at[i], rows, cols); };
         auto need = [&](int i) { return ctx->needs_input_grad(1 + i); };
-        auto times = [&](int64_t out, int64_t out_cols, int64_t in, int64_t in_cols, const Tensor& wt) {
-            Tensor o = matrix(buf, out, M, out_cols);
-            at::mm_out(o, matrix(buf, in, M, in_cols), wt);
-        };
-        auto plus = [&](int64_t out, int64_t in, int64_t in_cols, const Tensor& wt) {
-            Tensor o = matrix(buf, out, M, C);
-            at::addmm_out(o, o, matrix(buf, in, M, in_cols), wt);
-        };
-        size_t ws_bytes = L.attn_ln_bwd_workspace_bytes(B, T, H, N);
-        ws_bytes = std::max(ws_bytes, L.expand_loras_bwd_workspace_bytes(B, T, C, R_LORA));
-        ws_bytes = std::max(ws_bytes, L.ddlerp_bwd_workspace_bytes(B, T, C, R_MIX));
-        const Tensor ws = scratch_bytes(ws_bytes, xb);
-
-        // planes: 0 dya then dw2, 1 dr, 2 dw, 3 dk', 4 dv, 5 dkk, 6 db, 7 dg, 8 dk
-        {
-            Tensor dya = matrix(buf, 0, M, C);
-            at::mm_out(dya, dout.view({M, C}), weight(WO, C, C));
-            WeightGrads wg;
-            if (need(WO)) wg.add(ptr(dout), C, a(A.ya), C, g(WO));
-            wg.run(M, xb, stream);
-        }
-        check(L.attn_ln_backward(B, T, H, N, WIND_RWKV7_BF16, WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), ptr(lnp),
-                                 d(0), ptr(saved), nullptr, d(2 * P), d(P), d(3 * P), d(4 * P), d(5 * P), d(6 * P), d(7 * P), g(LN_W), nullptr,
-                                 ptr(ws), ws.numel(), stream));
-        check(L.expand_loras_backward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
-                                      w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), d(2 * P), d(3 * P), d(5 * P), d(6 * P), d(0), d(8 * P),
-                                      d(o_z), d(o_a1), d(o_ma1), d(o_mk1), g(KKK_W2), g(AAA_W2), g(MA_W2), g(MK_W2), g(DECAY), g(AAAAA),
-                                      g(MISC_A), g(MISC_K), ptr(ws), ws.numel(), stream));
-        times(o_tg1, R_GATE, 7 * P, C, weight(GATE_W2, C, R_GATE));
-        times(o_tw1, R_DECAY, 0, C, weight(DECAY_W2, C, R_DECAY));
-        {
-            WeightGrads wg;
-            if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
-            if (need(DECAY_W2)) wg.add(d(0), C, a(A.tw1), R_DECAY, g(DECAY_W2));
-            wg.run(M, xb, stream);
-        }
-        Columns cols;
-        cols.add(d(o_z), R_LORA, 0, d(o_kkmk), W_KKMK, 0, R_LORA, 0);
-        cols.add(d(o_mk1), R_LORA, 0, d(o_kkmk), W_KKMK, R_LORA, R_LORA, 0);
-        cols.add(d(o_tw1), R_DECAY, 0, d(o_w1), W_DECAY_AAA_MA, 0, R_DECAY, 2, a(A.tw1));
-        cols.add(d(o_a1), R_LORA, 0, d(o_w1), W_DECAY_AAA_MA, R_DECAY, R_LORA, 0);
-        cols.add(d(o_ma1), R_LORA, 0, d(o_w1), W_DECAY_AAA_MA, R_DECAY + R_LORA, R_LORA, 0);
-        cols.add(d(o_tg1), R_GATE, 0, d(o_g1), R_GATE, 0, R_GATE, 2, a(A.tg1));
-        cols.run(M, stream);
-        // the streams' gradients go to the planes that are free now: 2, 5, 3, 6
-        const int64_t dxrg = 2 * P, dxwa = 5 * P, dxk = 3 * P, dxv = 6 * P;
-        times(dxrg, C, P, C, weight(WR, C, C));
-        plus(dxrg, o_g1, R_GATE, weight(GATE_W1, R_GATE, C));
-        times(dxk, C, 8 * P, C, weight(WK, C, C));
-        plus(dxk, o_kkmk, W_KKMK, weight(KKK_W1, W_KKMK, C));
-        times(dxv, C, 4 * P, C, weight(WV, C, C));
-        times(dxwa, C, o_w1, W_DECAY_AAA_MA, weight(DECAY_W1, W_DECAY_AAA_MA, C));
-        {
-            WeightGrads wg;
-            if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
-            if (need(GATE_W1)) wg.add(d(o_g1), R_GATE, a(A.streams), C, g(GATE_W1));
-            if (need(WK)) wg.add(d(8 * P), C, a(A.streams + 2 * P), C, g(WK));
-            if (need(KKK_W1) || need(MK_W1)) wg.add(d(o_kkmk), W_KKMK, a(A.streams + 2 * P), C, g(KKK_W1));
-            if (need(WV)) wg.add(d(4 * P), C, a(A.streams + 3 * P), C, g(WV));
-            if (need(DECAY_W1) || need(AAA_W1) || need(MA_W1)) wg.add(d(o_w1), W_DECAY_AAA_MA, a(A.streams + P), C, g(DECAY_W1));
-            wg.run(M, xb, stream);
-        }
-        Tensor dx = at::empty_like(xb);
-        check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), d(dxrg), d(dxwa), d(dxk), d(dxv),
-                                ptr(dx), g(MAA_X), g(MAA_W1), g(MAA_W2), g(MAA), ptr(ws), ws.numel(), stream));
+        const ParamLayout at_(s.C);
+        const Tensor dx = at::empty_like(xb), flat = at::empty({at_.at[PARAMS]}, xb.options().dtype(at::kFloat));
+        block_backward(s, xb, t[1], t[2], t[3], grads[0].contiguous(), dx, flat, need);
         variable_list out{Tensor(), dx.to((at::ScalarType)types[2])};
         for (int i = 0; i < PARAMS; i++) {
             if (!need(i)) {
                 out.emplace_back();
                 continue;
             }
-            const auto shape = param_shape(i, C);
+            const auto shape = param_shape(i, s.C);
             std::vector<int64_t> stride(shape.size());
             int64_t n = 1;
             for (size_t k = stride.size(); k-- > 0; n *= shape[k]) stride[k] = n;
@@ -817,6 +840,29 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         return out;
     }
 };
+
+// The same two passes as the registered operators that torch.compile records: every buffer comes from the caller, sized by
+// block_sizes (bf16 elements of `weights` with and without the transposed copies, of `acts` per token, of `flat`, and each
+// parameter's place in `flat`); an empty tensor stands for one that is not there.
+std::vector<int64_t> block_sizes(int64_t C) {
+    const WeightLayout W(C);
+    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16};
+    r.insert(r.end(), W.at_.at, W.at_.at + PARAMS + 1);
+    return r;
+}
+void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, const Tensor& x_prev, const Tensor& s0, const Tensor& weights,
+                          const Tensor& acts, const Tensor& saved, const Tensor& y, const Tensor& sT, bool save) {
+    c10::DeviceGuard guard(xb.device());
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Block s{xb.size(0), xb.size(1), xb.size(2), H};
+    block_forward(s, xb, p, save, s.T, x_prev.numel() ? x_prev : Tensor(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
+}
+void traced_block_backward(const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout, int64_t H,
+                           const Tensor& dx, const Tensor& flat) {
+    c10::DeviceGuard guard(xb.device());
+    at::AutoDispatchBelowADInplaceOrView below;
+    block_backward({xb.size(0), xb.size(1), xb.size(2), H}, xb, weights, acts, saved, dout, dx, flat, [](int) { return true; });
+}
 
 template <size_t... I>
 Tensor mixer_node(int64_t H, const Tensor& x, const variable_list& p, std::index_sequence<I...>) {
@@ -854,10 +900,12 @@ py::object short_prompt(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor
                         const Tensor& s0, at::ScalarType state_type, bool return_state) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor xb = x.to(at::kBFloat16).contiguous();
-    const BlockWeights bw(p, xb);
+    const WeightLayout W(C);
+    const Tensor packed = at::empty({W.total[0]}, xb.options());
+    pack_weights(W, p, packed, false);
     const void* w[WEIGHTS + 1];
-    for (int i = 0; i < WEIGHTS; i++) w[i] = bw.w(i);
-    w[WEIGHTS] = bw.ln.data_ptr();
+    for (int i = 0; i < WEIGHTS; i++) w[i] = at_elem(packed, W.at_.at[i]);
+    w[WEIGHTS] = at_elem(packed, W.ln);
     wind_rwkv7_mixer_weights weights;
     static_assert(sizeof(w) == sizeof(weights), "the enumeration above is the header's order");
     memcpy(&weights, w, sizeof(w));
@@ -905,7 +953,8 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     if (T % 16 && s.N() == 64 && T <= SHORT_PROMPT && s.B * T <= SHORT_PROMPT_ROWS) return short_prompt(s.B, T, s.C, H, x, p, x_prev, s0, state_type, return_state);
     Tensor xb = x.to(at::kBFloat16);
     xb = s.T == T ? xb.contiguous() : at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
-    BlockForward f = block_forward(s, xb, p, false, T, x_prev, s0, state_type);
+    const BlockBuffers f(s, xb, false, state_type);
+    block_forward(s, xb, p, false, T, x_prev, s0, f);
     const Tensor y = s.T == T ? f.y : f.y.narrow(1, 0, T).contiguous();
     if (!return_state) return py::cast(y);
     return py::make_tuple(y, py::make_tuple(x.select(1, T - 1).clone(), f.sT));
@@ -962,4 +1011,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("expand_loras", &expand_loras);
     m.def("mixer", &mixer);
     m.def("mixer_step", &mixer_step);
+    m.def("block_sizes", &block_sizes);
+    m.def("block_forward", &traced_block_forward);
+    m.def("block_backward", &traced_block_backward);
 }

@@ -69,10 +69,13 @@ SIGNATURES = {
     'wind_rwkv7_expand_loras_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_expand_loras_forward': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp]),
     'wind_rwkv7_expand_loras_backward': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp] * 14 + [_vp, _sz, _vp]),
+    'wind_rwkv7_expand_loras_backward_to': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp] * 7 + [_vp] * 8 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_f32_saved_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_f32_forward': (_i, [_i] * 4 + [_vp] * 7 + [_vp] * 3 + [_vp]),
     'wind_rwkv7_attn_f32_prefill': (_i, [_i] * 4 + [_vp] * 7 + [_vp] * 2 + [_vp]),
     'wind_rwkv7_attn_f32_backward': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp] * 7 + [_vp]),
+    'wind_rwkv7_pack_weights': (_i, [_i, _vp, _vp]),
+    'wind_rwkv7_linear_group': (_i, [_i, _ll, _vp, _vp]),
     'wind_rwkv7_linear_wgrad_workspace_bytes': (_sz, [_ll, _i, _i]),
     'wind_rwkv7_linear_wgrad': (_i, [_ll, _i, _i, _vp, _ll, _vp, _ll, _vp, _i, _vp, _sz, _vp]),
     'wind_rwkv7_linear_wgrad_group_workspace_bytes': (_sz, [_i, _ll, _vp, _vp]),
@@ -91,6 +94,15 @@ MIXER_WEIGHT_NAMES = ('time_maa_x', 'time_maa', 'time_maa_w1', 'time_maa_w2', 'W
 
 class MixerWeights(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in MIXER_WEIGHT_NAMES]
+
+
+class Linear(ctypes.Structure):   # wind_rwkv7_linear
+    _fields_ = [('A', _vp * 2), ('W', _vp * 2), ('lda', _ll * 2), ('ldw', _ll * 2), ('K', _i * 2), ('N', _i), ('npieces', _i),
+                ('out', _vp * 4), ('aux', _vp * 4), ('ld_out', _ll * 4), ('width', _i * 4), ('op', _i * 4)]
+
+
+class Pack(ctypes.Structure):   # wind_rwkv7_pack
+    _fields_ = [('src', _vp), ('dst', _vp), ('dstT', _vp), ('src_dtype', _i), ('dst_dtype', _i), ('rows', _i), ('cols', _i), ('ldT', _ll)]
 
 
 _lib = None

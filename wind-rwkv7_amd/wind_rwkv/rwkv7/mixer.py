@@ -2,9 +2,9 @@
 
 Mirrors the reference's ``TimeMixer`` (time_mixer.py:18-167): same constructor signature, same parameter
 names and shapes (so a state dict moves over unchanged), same forward contract
-(``x [B,T,C]`` of any float dtype -> ``[B,T,C]`` bf16).  The projections (:120-131, :167) are bf16 matmuls: the
-product and its input gradient go to the BLAS library as in the reference, the weight gradient to this
-package's kernel (linear.py); everything else runs in this package's kernels:
+(``x [B,T,C]`` of any float dtype -> ``[B,T,C]`` bf16).  The projections (:120-131, :167) are bf16
+products with fp32 accumulation, all of them in this package's kernels, grouped into few launches (linear_group.hip,
+linear_wgrad.hip; single very large ones go to the BLAS library):
 
     ddlerp -> r, k, v, gate and LoRA first halves (matmuls) -> expand_loras -> attn_ln -> output matmul
 
@@ -27,10 +27,65 @@ from .. import _native
 from .linear import bf16_copies, projection, projection_sets, split_columns
 from .loras import expand_loras
 from .token_shift import ddlerp
-from .wkv_attn import _attn_bf16_head, _bf16_head, attn_triton, load_attn
-from .wkv_attn_ln import attn_ln, attn_ln_step, group_norm_heads, load_attn_ln
+from .wkv_attn import _OPS, _attn_bf16_head, _bf16_head, _differentiating, _no_cpu, attn_triton, load_attn, no_state
+from .wkv_attn_ln import _saved_unit, attn_ln, attn_ln_step, group_norm_heads, load_attn_ln
 
 LORA_RANKS = dict(mix=32, decay=64, aaa=16, kkk=16, gate=128, ma=16, mk=16)  # time_mixer.py:69-94
+
+
+# ---- the block as registered operators: what torch.compile records of the native path (csrc/torch_binding.cpp) ----
+_OPS.define('block_forward(Tensor x, Tensor[] params, int H, Tensor x_prev, Tensor s0, Tensor(a!) weights, Tensor(b!) acts, '
+            'Tensor(c!) saved, Tensor(d!) y, Tensor(e!) sT, bool save) -> ()')
+_OPS.define('block_backward(Tensor x, Tensor weights, Tensor acts, Tensor saved, Tensor dy, int H, Tensor(a!) dx, '
+            'Tensor(b!) flat) -> ()')
+for _name, _impl in (('block_forward', lambda *a: _native.binding().block_forward(*a)),
+                     ('block_backward', lambda *a: _native.binding().block_backward(*a))):
+    _OPS.impl(_name, _impl, 'CUDA')
+    _OPS.impl(_name, _no_cpu, 'CPU')
+    _OPS.impl(_name, lambda *a: None, 'Meta')
+
+
+@torch.compiler.assume_constant_result
+def _block_sizes(C):
+    return _native.binding().block_sizes(C)
+
+
+def _block_forward(x, params, H, x_prev, s0, state_dtype, save):
+    """(y, sT, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev and s0 may be the empty stand-in."""
+    B, T, C = x.shape
+    N = C // H
+    sizes = _block_sizes(C)
+    new = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=x.device)
+    weights, acts = new(sizes[1 if save else 0]), new(sizes[2] * B * T)
+    saved, y = new(B, H, T // 16, _saved_unit(N)), new(B, T, C)
+    sT = torch.empty(B, H, N, N, dtype=state_dtype, device=x.device)
+    torch.ops.wind_rwkv7.block_forward(x, params, H, x_prev, s0, weights, acts, saved, y, sT, save)
+    return y, sT, weights, acts, saved
+
+
+class Block(torch.autograd.Function):
+    """y = the block on bf16 x with the parameters in the binding's order, as torch.compile records it."""
+
+    @staticmethod
+    def forward(ctx, x, H, *params):
+        none = no_state(torch.bfloat16, x.device)
+        y, _, weights, acts, saved = _block_forward(x, [p.detach() for p in params], H, none, none, torch.bfloat16, True)
+        ctx.save_for_backward(x, weights, acts, saved)
+        ctx.H = H
+        ctx.params = [(tuple(p.shape), p.dtype) for p in params]
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weights, acts, saved = ctx.saved_tensors
+        sizes = _block_sizes(x.shape[2])
+        dx = torch.empty_like(x)
+        flat = torch.empty(sizes[-1], dtype=torch.float32, device=x.device)
+        torch.ops.wind_rwkv7.block_backward(x, weights, acts, saved, dy.contiguous(), ctx.H, dx, flat)
+        grads = []
+        for (shape, dtype), at in zip(ctx.params, sizes[3:]):
+            grads.append(flat[at:at + math.prod(shape)].view(shape).to(dtype))
+        return (dx, None, *grads)
 
 
 def ref_attn(q, w, k, v, a, b, HEAD_SIZE):
@@ -228,8 +283,12 @@ class TimeMixer(nn.Module):
         leave the state alone); what follows here is what torch.compile traces, and every other case (there the tokens
         after the last full chunk go through `step`)."""
         B, T, C = x.shape
-        if (x.is_cuda and not torch.compiler.is_compiling() and self.attn_impl == 'cuda' and self.use_triton_ddlerp
-                and self._loras_kernel and not (T == 1 and (state is not None or return_state))):   # (one token: `step`)
+        native = (x.is_cuda and self.attn_impl == 'cuda' and self.use_triton_ddlerp and self._loras_kernel
+                  and _attn_bf16_head(self.head_size))
+        if native and torch.compiler.is_compiling():
+            if T % 16 == 0:
+                return self._traced_block(x, state, return_state)
+        elif native and not (T == 1 and (state is not None or return_state)):   # (one token: `step`)
             out = _native.binding().mixer(x, self._parameters, self.ln_x._parameters, self.n_head, *(state or (None, None)), return_state)
             if out is not None:
                 return out
@@ -271,6 +330,24 @@ class TimeMixer(nn.Module):
         if return_state:
             return mm_o(y), (x[:, -1].clone(), wkv_state)
         return mm_o(y)
+
+    def _block_params(self):
+        """The parameters in the native binding's order."""
+        return [getattr(self, n) for n in _native.MIXER_WEIGHT_NAMES[:-1]] + [self.ln_x.weight, self.ln_x.bias, self.time_faaaa]
+
+    def _traced_block(self, x, state, return_state):
+        """`forward` as torch.compile records it: one registered operator each way, the native path's own passes."""
+        params = [p if p.dtype in (torch.float32, torch.bfloat16) else p.float() for p in self._block_params()]
+        xb = x.bfloat16().contiguous()
+        if state is None and not return_state and _differentiating(x, *params):
+            return Block.apply(xb, self.n_head, *params)
+        assert not _differentiating(x, *params), 'a carried state is for inference: run under torch.no_grad()'
+        x_prev, s0 = state if state is not None else (None, None)
+        none = no_state(torch.bfloat16, x.device)
+        state_dtype = s0.dtype if s0 is not None else torch.float32 if state is not None or return_state else torch.bfloat16
+        y, sT, _, _, _ = _block_forward(xb, [p.detach() for p in params], self.n_head, none if x_prev is None else x_prev.bfloat16().contiguous(),
+                                        none if s0 is None else s0.contiguous(), state_dtype, False)
+        return (y, (x[:, -1].clone(), sT)) if return_state else y
 
     def _forward_any_length(self, x, state, return_state):
         """Inference on a length that is no multiple of 16 (the sequence kernels' chunk): the longest such prefix as
@@ -315,7 +392,7 @@ class TimeMixer(nn.Module):
         (`p.data.copy_(...)`, as manual weight loading or an EMA update may do) does not change what the cache is keyed
         on (storage address and version counter): call `invalidate_decode_cache()` after such a write."""
         names = _native.MIXER_WEIGHT_NAMES[:-1]
-        ps = [getattr(self, n) for n in names] + [self.ln_x.weight, self.ln_x.bias, self.time_faaaa]
+        ps = self._block_params()
         key = tuple((p.data_ptr(), p._version) for p in ps)
         cache = self.__dict__.get('_decode_cache')
         if cache is None or cache[0] != key:
