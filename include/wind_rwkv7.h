@@ -344,7 +344,9 @@ int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_siz
  * than 64, its large-head variant (rwkv7_attn_triton_bighead.py:31-322; `assert C%16 == 0`, :335).
  * All tensors are float32: w,q,k,v,a,b,y,dy and the six gradients [B,T,H,C]; s0,sT,dsT,ds0 [B,H,C,C];
  * s = wind_rwkv7_attn_f32_saved_bytes bytes (the state every 16 tokens and a [B,T,H,C] tensor of row sums).
- * No workspace.  The backward zeroes dq, dk, da, db, dw itself and adds two parts per element onto them (atomics; the result does not depend on their order).  C a multiple of 16 from 16 to 128 (wind_rwkv7_f32_head_size_supported), T % 16 == 0. */
+ * wind_rwkv7_attn_f32_backward takes no workspace: it zeroes dq, dk, da, db, dw itself and adds two parts per element
+ * onto them (atomics; the result does not depend on their order).  wind_rwkv7_attn_f32_backward_split computes the same
+ * gradients faster, with wind_rwkv7_attn_f32_bwd_workspace_bytes bytes of workspace (256-byte aligned).  C a multiple of 16 from 16 to 128 (wind_rwkv7_f32_head_size_supported), T % 16 == 0. */
 int wind_rwkv7_f32_head_size_supported(int C);
 size_t wind_rwkv7_attn_f32_saved_bytes(int B, int T, int H, int C);
 int wind_rwkv7_attn_f32_forward(int B, int T, int H, int C,
@@ -363,6 +365,13 @@ int wind_rwkv7_attn_f32_backward(int B, int T, int H, int C,
                                  const void* dy, const void* s, const void* dsT,
                                  void* dw, void* dq, void* dk, void* dv, void* da, void* db, void* ds0,
                                  void* stream);
+size_t wind_rwkv7_attn_f32_bwd_workspace_bytes(int B, int T, int H, int C);
+int wind_rwkv7_attn_f32_backward_split(int B, int T, int H, int C,
+                                       const void* w, const void* q, const void* k, const void* v,
+                                       const void* a, const void* b,
+                                       const void* dy, const void* s, const void* dsT,
+                                       void* dw, void* dq, void* dk, void* dv, void* da, void* db, void* ds0,
+                                       void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- projection weight gradient ------------------------------------------------------------------ */
 

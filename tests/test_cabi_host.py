@@ -229,6 +229,13 @@ def test_f32_entry_points_validate_on_host():
         bad = list(ok)
         bad[idx] = val
         assert lib.wind_rwkv7_attn_f32_backward(*bad) == code, (idx, val)
+    need = lib.wind_rwkv7_attn_f32_bwd_workspace_bytes(2, 32, 3, 64)   # a state every 16 tokens and a float per token and channel
+    assert need == lib.wind_rwkv7_attn_f32_saved_bytes(2, 32, 3, 64) and lib.wind_rwkv7_attn_f32_bwd_workspace_bytes(2, 8, 3, 64) == 0
+    ok = [2, 32, 3, 64] + [0x1000] * 16 + [0x2000, need, None]
+    for idx, val, code in [(2, -1, 2), (1, 8, 4), (3, 136, 3), (12, None, 1), (19, None, 1), (20, None, 6), (20, 0x2010, 6), (21, need - 1, 6)]:
+        bad = list(ok)
+        bad[idx] = val
+        assert lib.wind_rwkv7_attn_f32_backward_split(*bad) == code, (idx, val)
 
 
 def test_linear_wgrad_sizes_and_validation_on_host():

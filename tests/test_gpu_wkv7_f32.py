@@ -94,6 +94,29 @@ def test_f32_large_head_long_sequence(c_oracle):
         assert seq_ref.rel_err(g.cpu(), ref['d' + n]) <= TOL, n
 
 
+@pytest.mark.parametrize('B,T,H,C', [(2, 48, 3, 64), (1, 16, 2, 16), (1, 48, 2, 80), (2, 32, 2, 128)])
+def test_f32_backward_entry_points_agree(B, T, H, C):
+    """The backward without a workspace and the one that uses it.  Both are within a few units of the last place of sums of
+    at most C terms (2^-24 sqrt(C) each) over windows of the same recurrence: 1e-5 leaves a factor of ten."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    d = inputs.wkv7_inputs(B, T, H, C, seed=300 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
+    xs = [d[n].float().to(DEV) for n in NAMES]
+    s0, dy, dsT = [d[n].float().to(DEV) for n in ('s0', 'dy', 'dsT')]
+    p = lambda ts: [t.data_ptr() for t in ts]
+    stream = torch.cuda.current_stream().cuda_stream
+    y, sT, s = torch.empty_like(dy), torch.empty_like(s0), torch.empty(lib.wind_rwkv7_attn_f32_saved_bytes(B, T, H, C) // 4, device=DEV)
+    _native.check(lib.wind_rwkv7_attn_f32_forward(B, T, H, C, *p(xs + [s0, y, s, sT]), stream))
+    need = lib.wind_rwkv7_attn_f32_bwd_workspace_bytes(B, T, H, C)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    fresh = lambda: [torch.full_like(x, float('nan')) for x in xs + [s0]]
+    alone, split = fresh(), fresh()
+    _native.check(lib.wind_rwkv7_attn_f32_backward(B, T, H, C, *p(xs + [dy, s, dsT] + alone), stream))
+    _native.check(lib.wind_rwkv7_attn_f32_backward_split(B, T, H, C, *p(xs + [dy, s, dsT] + split), ws.data_ptr(), need, stream))
+    for n, g, h in zip(list('wqkvab') + ['s0'], alone, split):
+        assert seq_ref.rel_err(h.cpu(), g.cpu()) <= 1e-5, n
+
+
 def test_other_head_sizes_through_the_public_names():
     """attn, attn_triton and attn_triton_bighead on bf16 tensors with head sizes other than 64: attn and
     dot_prec='bf16' run the bf16 matrix-core kernels for those head sizes (1e-2 gate), the default dot_prec='fp32'
@@ -139,8 +162,7 @@ def test_f32_public_wrapper_and_dot_prec():
 
 @pytest.mark.parametrize('B,T,H,C', [(8, 256, 12, 64), (2, 128, 3, 128), (2, 64, 5, 48)])
 def test_f32_backward_is_reproducible(B, T, H, C):
-    """dq, dk, da, db, dw are sums of two blocks' parts added by atomics onto zeros: two addends, so the order in
-    which they arrive does not show in the result."""
+    """dq, dk, da, db, dw are sums over the wavefronts of a block in a fixed order: the same bits every time."""
     d = inputs.wkv7_inputs(B, T, H, C, seed=77, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
     first = _run(d, B, T, H, C, True)
     for _ in range(3):

@@ -778,6 +778,29 @@ int wind_rwkv7_attn_f32_backward(int B, int T, int H, int C,
     return launch_status();
 }
 
+// (the workspace holds of the backward scan what `s` holds of the forward: a state per chunk and a row sum per token)
+size_t wind_rwkv7_attn_f32_bwd_workspace_bytes(int B, int T, int H, int C) {
+    if (check_shape_f32(B, T, H, C)) return 0;
+    return align_up(wkv::wkv7_f32_saved_bytes(B, T, H, C));
+}
+
+int wind_rwkv7_attn_f32_backward_split(int B, int T, int H, int C,
+                                       const void* w, const void* q, const void* k, const void* v, const void* a, const void* b,
+                                       const void* dy, const void* s, const void* dsT,
+                                       void* dw, void* dq, void* dk, void* dv, void* da, void* db, void* ds0,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+    int rc = check_shape_f32(B, T, H, C);
+    if (rc) return rc;
+    if (!w || !q || !k || !v || !a || !b || !dy || !s || !dsT || !dw || !dq || !dk || !dv || !da || !db || !ds0)
+        return WIND_RWKV7_ERR_NULL_POINTER;
+    if ((rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_f32_bwd_workspace_bytes(B, T, H, C)))) return rc;
+    auto f = [](const void* p) { return static_cast<const float*>(p); };
+    auto g = [](void* p) { return static_cast<float*>(p); };
+    wkv::launch_wkv7_f32_backward_split(B, T, H, C, f(w), f(q), f(k), f(v), f(a), f(b), f(dy), f(s), f(dsT), g(workspace), g(dw),
+                                        g(dq), g(dk), g(dv), g(da), g(db), g(ds0), static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
 static int check_linear(long long tokens, int O, int I) {
     if (tokens <= 0 || O <= 0 || I <= 0 || tokens > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (O % 16 != 0 || I % 16 != 0) return WIND_RWKV7_ERR_CHANNELS;

@@ -33,7 +33,8 @@ namespace py = pybind11;
     X(attn_forward) X(attn_prefill) X(attn_backward)                                                                 \
     X(attn_ln_saved_bytes) X(attn_ln_fwd_workspace_bytes) X(attn_ln_bwd_workspace_bytes)                             \
     X(attn_ln_forward) X(attn_ln_prefill) X(attn_ln_backward)                                                        \
-    X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward)                             \
+    X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward_split)                       \
+    X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
     X(ddlerp_forward_from) X(neutral_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
@@ -202,8 +203,10 @@ struct Wkv7F32 : torch::autograd::Function<Wkv7F32> {
         variable_list d(6);
         for (auto& g : d) g = at::empty_like(t[3]);
         Tensor ds0 = at::empty_like(dsT);
-        check(L.attn_f32_backward(s.B, s.T, s.H, s.C, ptr(t[0]), ptr(t[1]), ptr(t[2]), ptr(t[3]), ptr(t[4]), ptr(t[5]), ptr(dy), ptr(t[6]),
-                                  ptr(dsT), ptr(d[0]), ptr(d[1]), ptr(d[2]), ptr(d[3]), ptr(d[4]), ptr(d[5]), ptr(ds0), stream_of(dy)));
+        const Tensor mem = scratch_bytes(L.attn_f32_bwd_workspace_bytes(s.B, s.T, s.H, s.C), t[3]);
+        check(L.attn_f32_backward_split(s.B, s.T, s.H, s.C, ptr(t[0]), ptr(t[1]), ptr(t[2]), ptr(t[3]), ptr(t[4]), ptr(t[5]), ptr(dy), ptr(t[6]),
+                                  ptr(dsT), ptr(d[0]), ptr(d[1]), ptr(d[2]), ptr(d[3]), ptr(d[4]), ptr(d[5]), ptr(ds0), ptr(mem), mem.numel(),
+                                        stream_of(dy)));
         return {Tensor(), d[0], d[1], d[2], d[3], d[4], d[5], ds0};
     }
 };

@@ -14,16 +14,21 @@
 // of a token are read as one 16-byte LDS access each, one token ahead of their use.
 // The value rows of a state never mix, so a head can be cut over blocks by rows.  Forward: eight wavefronts per block
 // (two per SIMD cover each other's waits), four or two blocks per head (a quarter or half of the rows each) while every
-// block still gets a compute unit of its own, else one block with all rows.  Backward: always two blocks of four wavefronts per head (all
-// rows in one block need more registers than a wavefront has); the gradients that sum over value rows (dq, dk, da, db,
-// dw) are the sum of the two blocks' parts, added with floating-point atomics onto zeroed tensors - with exactly two
-// addends per element the result does not depend on their order, so results are reproducible.
-// The forward keeps the state every CHUNK tokens and S a of every token; the backward walks the chunks in reverse,
-// recomputes a window of states of a chunk into registers (three multiply-adds per element, no row sums to wait for)
-// and runs the adjoint recurrence through them.
+// block still gets a compute unit of its own, else one block with all rows.
+// The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
+// direction (it keeps the state gradient arriving at every chunk's end and dsa of every token, and leaves dv and ds0)
+// and then a kernel in which every chunk is on its own: it recomputes states and state gradients without a row sum to
+// wait for, and makes the other five gradients.
+// A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
+// windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
+// with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
+//   1 x 256 tokens x 4 heads of 64   274 -> 122        8 x 1024 x 6 heads of 128   2420 -> 1365
+//   8 x 1024 x 12 heads of 64        844 -> 702        32 x 1024 x 12 heads of 64  2395 -> 1954
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 namespace wkv {
 namespace {
@@ -128,7 +133,12 @@ __device__ __forceinline__ float wave_sum(float x) {
 // then S a of every token ([B,T,H,C]; the backward's recomputation of the states inside a chunk then needs no row sums).
 __host__ __device__ inline long saved_states(long BH, int T, int C) { return BH * (T / CH64) * C * C; }
 
-template <int C, int R, int NW, bool FULL>
+// ADJ: the same recurrence backwards in time.  With E the state gradient that arrives from the tokens after t,
+//     dsa = E b + dy (q . b);   dv = E k + dy (q . k);   E <- E diag(decay) + dsa a^T + dy (decay * q)^T
+// is the forward's step with (a, decay q, b, k, v) in the places of (b, k, a, decay q, dy): two row sums on the state
+// before its update, a rank-one term with the first of them and one with the row vector.  v, s0, y, ckpt, sT are then
+// dy, dsT, dv, the workspace of the gradient kernel below (E arriving at every chunk's end, dsa of every token) and ds0.
+template <int C, int R, int NW, bool FULL, bool ADJ>
 __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H, int CR, const float* __restrict__ w,
                                                              const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ v, const float* __restrict__ a,
@@ -176,8 +186,9 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
             }
         }
     };
-    fetch(0);
-    for (int c0 = 0; c0 < T; c0 += CH) {
+    fetch(ADJ ? T - CH : 0);
+    for (int n0 = 0; n0 < T; n0 += CH) {
+        const int c0 = ADJ ? T - CH - n0 : n0;
         // stage the chunk: the decay instead of w, decay * q instead of q.  With them
         //   y_t = S_t q = S_{t-1} (decay * q) + (S_{t-1} a) (b . q) + v (k . q),
         // so that both row sums of a token work on the state BEFORE its update and neither waits for the other.
@@ -202,38 +213,40 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
             }
         }
         __syncthreads();
-        fetch(c0 + CH < T ? c0 + CH : c0);   // (after the last chunk: the same one again, not used)
+        fetch(n0 + CH >= T ? c0 : ADJ ? c0 - CH : c0 + CH);   // (after the last chunk: the same one again, not used)
         // a token's operands are requested from LDS one token ahead (the stores of the results in between keep the
         // compiler from moving the reads up by itself)
         struct Ops {
-            f4 dec, av, bv, kv, dqv;
+            f4 dec, x1, x2, u1, u2;   // operands of the two row sums, column vectors of the two rank-one terms
             RowVals<R> vr;
             f2 sc;
         };
         auto read_ops = [&](int t) {
             Ops o;
-            o.dec = *reinterpret_cast<const f4*>(&in[V_DEC][t][col0]), o.av = *reinterpret_cast<const f4*>(&in[V_A][t][col0]);
-            o.bv = *reinterpret_cast<const f4*>(&in[V_B][t][col0]), o.kv = *reinterpret_cast<const f4*>(&in[V_K][t][col0]);
-            o.dqv = *reinterpret_cast<const f4*>(&in[V_Q][t][col0]);
+            o.dec = *reinterpret_cast<const f4*>(&in[V_DEC][t][col0]);
+            o.x1 = *reinterpret_cast<const f4*>(&in[ADJ ? V_B : V_A][t][col0]);
+            o.u1 = *reinterpret_cast<const f4*>(&in[ADJ ? V_A : V_B][t][col0]);
+            o.u2 = *reinterpret_cast<const f4*>(&in[ADJ ? V_Q : V_K][t][col0]);
+            o.x2 = *reinterpret_cast<const f4*>(&in[ADJ ? V_K : V_Q][t][col0]);
             o.vr = lds_rows<R>(&in[V_V][t][row0]);
             o.sc = bkq[t][0];
             if constexpr (NH == 2) o.sc += bkq[t][1];
             return o;
         };
-        Ops ahead = read_ops(0);
+        Ops ahead = read_ops(ADJ ? CH - 1 : 0);
 #pragma unroll
-        for (int t = 0; t < CH; t++) {
+        for (int i = 0; i < CH; i++) {
+            const int t = ADJ ? CH - 1 - i : i;
             const Ops o = ahead;
-            if (t + 1 < CH) ahead = read_ops(t + 1);
-            const f4 dec = o.dec, av = o.av, bv = o.bv, kv = o.kv, dqv = o.dqv;
-            const RowVals<R> vr = o.vr;
-            const f2 sc = o.sc;
+            if (i + 1 < CH) ahead = read_ops(ADJ ? t - 1 : t + 1);
             RowVals<R> yr, sar;
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                sar.x[r] = row_sum<LPR>(dot4(S[r], av));
-                yr.x[r] = row_sum<LPR>(dot4(S[r], dqv)) + sar.x[r] * sc[0] + vr.x[r] * sc[1];
-                S[r] = S[r] * dec + sar.x[r] * bv + vr.x[r] * kv;
+                sar.x[r] = row_sum<LPR>(dot4(S[r], o.x1));
+                if constexpr (ADJ) sar.x[r] += o.vr.x[r] * o.sc[0];
+                yr.x[r] = row_sum<LPR>(dot4(S[r], o.x2)) + o.vr.x[r] * o.sc[1];
+                if constexpr (!ADJ) yr.x[r] += sar.x[r] * o.sc[0];
+                S[r] = S[r] * o.dec + sar.x[r] * o.u1 + o.vr.x[r] * o.u2;
             }
             if (jb == 0) {
 #pragma unroll
@@ -462,6 +475,141 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
     }
 }
 
+// The gradients of one chunk (16 tokens) of one head and 64 of its columns, from the state entering the chunk, the state
+// gradient arriving at its end, and S a and dsa of every token: nothing is left to wait for, every chunk is its own block.
+// A lane holds ONE column of GR rows (CR / GR wavefronts), so every column sum is a chain of multiply-adds inside the lane
+// and one sum over the wavefronts through LDS; what belongs to a row (v, S a, dy, dsa) is read from LDS as a broadcast.
+// The states of GWIN tokens are recomputed into registers; the second half of a chunk first runs through the first.
+// Bound: vector issue, 13 instructions per state element and token: 236 us at 8 x 1024 tokens x 12 heads of 64, of which
+// 176 us are issue alone.  Through scalar loads and registers the row operands cost more (390 us: every token waits for
+// them, and the scalar cache holds a quarter of what the blocks of a compute unit read).
+constexpr int GR = 8, GWIN = 8, GRED = 4;   // rows per wavefront, tokens of kept states, tokens between sums over wavefronts
+
+template <int NWMAX>
+__global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, int H, int CR, const float* __restrict__ w,
+                                                                       const float* __restrict__ q, const float* __restrict__ k,
+                                                                       const float* __restrict__ v, const float* __restrict__ a,
+                                                                       const float* __restrict__ b, const float* __restrict__ dy,
+                                                                       const float* __restrict__ ckpt,
+                                                                       const float* __restrict__ work, float* __restrict__ dw,
+                                                                       float* __restrict__ dq, float* __restrict__ dk,
+                                                                       float* __restrict__ da, float* __restrict__ db) {
+    constexpr int CH = CH64, COLS = 64;
+    static_assert(CH == 2 * GWIN && GWIN % GRED == 0 && GR == 8, "two windows per chunk; two sums of four rows");
+    enum { G_DEC = 0, G_Q, G_K, G_A, G_B, G_DDEC, G_VECS };
+    enum { Q_V = 0, Q_SA, Q_DY, Q_DSA, Q_VECS };
+    __shared__ float in[G_VECS][CH][COLS];
+    __shared__ __attribute__((aligned(16))) float rows[Q_VECS][CH][GR * NWMAX];
+    __shared__ float red[NWMAX][RED_VECS][GRED][COLS];
+    const int NC = T / CH, NW = CR / GR, bh = blockIdx.x / NC, chunk = blockIdx.x - bh * NC, h = bh % H;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row0 = wv * GR;
+    const int col = COLS * blockIdx.y + lane;
+    const bool col_ok = col < CR;
+    const int colc = col_ok ? col : 0;   // (lanes past the head size read column 0 and write nothing)
+    const long base = seq_index((long)(bh / H) * T + (long)chunk * CH, H, h, 0, CR);
+    const unsigned ld = (unsigned)H * CR;
+    const long nstate = saved_states(gridDim.x / NC, T, CR), st = (long)blockIdx.x * CR * CR + (long)row0 * CR;
+    const float* const row_src[Q_VECS] = {v, ckpt + nstate, dy, work + nstate};
+
+    float Sx[GR], dS[GR];
+#pragma unroll
+    for (int r = 0; r < GR; r++) {
+        Sx[r] = (ckpt + st)[(unsigned)(r * CR + colc)];
+        dS[r] = (work + st)[(unsigned)(r * CR + colc)];
+    }
+    for (int e = threadIdx.x; e < CH * CR; e += 64 * NW) {
+        const int t = e / CR, r = e - t * CR;
+#pragma unroll
+        for (int x = 0; x < Q_VECS; x++) rows[x][t][r] = (row_src[x] + base)[(unsigned)t * ld + r];
+    }
+    for (int t = wv; t < CH; t += NW) {
+        const unsigned at = (unsigned)t * ld + colc;
+        const float ew = expf((w + base)[at]), d = expf(-ew);
+        in[G_DEC][t][lane] = d, in[G_DDEC][t][lane] = -ew * d;
+        in[G_Q][t][lane] = (q + base)[at], in[G_K][t][lane] = (k + base)[at];
+        in[G_A][t][lane] = (a + base)[at], in[G_B][t][lane] = (b + base)[at];
+    }
+    __syncthreads();
+    auto row_vals = [&](int x, int t) { return lds_rows<GR>(&rows[x][t][row0]); };
+    struct AdvOps {
+        RowVals<GR> vr, sar;
+        float dec, bv, kv;
+    };
+    auto read_adv = [&](int t) { return AdvOps{row_vals(Q_V, t), row_vals(Q_SA, t), in[G_DEC][t][lane], in[G_B][t][lane], in[G_K][t][lane]}; };
+    auto advance = [&](const float (&from)[GR], float (&to)[GR], const AdvOps& o) {
+#pragma unroll
+        for (int r = 0; r < GR; r++) to[r] = from[r] * o.dec + o.sar.x[r] * o.bv + o.vr.x[r] * o.kv;
+    };
+    float* const dst[RED_VECS] = {dq, dk, db, da, dw};
+#pragma unroll 1
+    for (int t0 = CH - GWIN; t0 >= 0; t0 -= GWIN) {
+        float S[GWIN + 1][GR];   // S[t] enters token t0 + t
+#pragma unroll
+        for (int r = 0; r < GR; r++) S[0][r] = Sx[r];
+        AdvOps adv = read_adv(0);
+#pragma unroll 2
+        for (int t = 0; t < t0; t++) {
+            const AdvOps o = adv;
+            adv = read_adv(t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            advance(S[0], S[0], o);
+        }
+#pragma unroll
+        for (int t = 0; t < GWIN; t++) {
+            const AdvOps o = adv;
+            if (t + 1 < GWIN) adv = read_adv(t0 + t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            advance(S[t], S[t + 1], o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tw = GWIN - 1; tw >= 0; tw--) {
+            const int t = t0 + tw;
+            const float qv = in[G_Q][t][lane], av = in[G_A][t][lane], dec = in[G_DEC][t][lane];
+            // dq = S_t^T dy;  dS_t += dy q^T;  dk = dS^T v;  db = dS^T sa;  da = S_{t-1}^T dsa;  ddecay: rows of dS * S_{t-1}
+            // (two chains of four rows each: half the rounding of one, and half the operands at a time)
+            float s[2][RED_VECS];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                const RowVals<4> dyr = lds_rows<4>(&rows[Q_DY][t][row0 + 4 * half]), vr = lds_rows<4>(&rows[Q_V][t][row0 + 4 * half]);
+                const RowVals<4> sar = lds_rows<4>(&rows[Q_SA][t][row0 + 4 * half]), dsar = lds_rows<4>(&rows[Q_DSA][t][row0 + 4 * half]);
+                float(&u)[RED_VECS] = s[half];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = 4 * half + i;
+                    dS[r] += dyr.x[i] * qv;
+                    u[R_DQ] = i ? u[R_DQ] + S[tw + 1][r] * dyr.x[i] : S[tw + 1][r] * dyr.x[i];
+                    u[R_DK] = i ? u[R_DK] + dS[r] * vr.x[i] : dS[r] * vr.x[i];
+                    u[R_DB] = i ? u[R_DB] + dS[r] * sar.x[i] : dS[r] * sar.x[i];
+                    u[R_DA] = i ? u[R_DA] + S[tw][r] * dsar.x[i] : S[tw][r] * dsar.x[i];
+                    u[R_DW] = i ? u[R_DW] + S[tw][r] * dS[r] : S[tw][r] * dS[r];
+                    dS[r] = dS[r] * dec + dsar.x[i] * av;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int x = 0; x < RED_VECS; x++) red[wv][x][tw % GRED][lane] = s[0][x] + s[1][x];
+            __builtin_amdgcn_sched_barrier(0);
+            if (tw % GRED == 0) {
+                __syncthreads();
+                // the wavefronts' sums of GRED tokens, in a fixed order, and out
+                for (int e = wv; e < RED_VECS * GRED; e += NW) {
+                    const int x = e / GRED, j = e % GRED;
+                    float even = 0.f, odd = 0.f;   // (sums of pairs in two chains; NW is even)
+                    for (int g = 0; g < NW; g += 4) {
+                        even += red[g][x][j][lane] + red[g + 1][x][j][lane];
+                        if (g + 2 < NW) odd += red[g + 2][x][j][lane] + red[g + 3][x][j][lane];
+                    }
+                    float sum = even + odd;
+                    if (x == R_DW) sum *= in[G_DDEC][t + j][lane];
+                    if (col_ok) (dst[x] + base)[(unsigned)(t + j) * ld + colc] = sum;
+                }
+                __syncthreads();
+            }
+        }
+    }
+}
+
 // five tensors of n floats each to zero (what the two-blocks-per-head backward adds its parts onto)
 __global__ __launch_bounds__(256) void zero5_kernel(long n4, f4* __restrict__ p0, f4* __restrict__ p1, f4* __restrict__ p2,
                                                     f4* __restrict__ p3, f4* __restrict__ p4) {
@@ -491,9 +639,9 @@ size_t wkv7_f32_saved_bytes(int B, int T, int H, int C) {
 }
 
 // (head sizes up to 64 run at a width of 64 channels, larger ones at 128; FULL: the head fills the width)
-void launch_wkv7_f32_forward(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,
-                             const float* a, const float* b, const float* s0, float* y, float* ckpt, float* sT,
-                             hipStream_t stream) {
+template <bool ADJ>
+static void launch_scan(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v, const float* a,
+                        const float* b, const float* s0, float* y, float* ckpt, float* sT, hipStream_t stream) {
     const int split = forward_split(B * H);
     auto go = [&](auto k4, auto k2, auto k1, int threads4) {
         auto launch = [&](auto kernel, int threads) {
@@ -504,10 +652,37 @@ void launch_wkv7_f32_forward(int B, int T, int H, int C, const float* w, const f
         else launch(k1, 512);
     };
     // (width, rows per thread, wavefronts): rows per block = wavefronts x row groups per wavefront x rows per thread
-    if (C == 64) go(wkv7_f32_fwd_thin_kernel<64, 1, 4, true>, wkv7_f32_fwd_thin_kernel<64, 1, 8, true>, wkv7_f32_fwd_thin_kernel<64, 2, 8, true>, 256);
-    else if (C < 64) go(wkv7_f32_fwd_thin_kernel<64, 1, 4, false>, wkv7_f32_fwd_thin_kernel<64, 1, 8, false>, wkv7_f32_fwd_thin_kernel<64, 2, 8, false>, 256);
-    else if (C == 128) go(wkv7_f32_fwd_thin_kernel<128, 2, 8, true>, wkv7_f32_fwd_thin_kernel<128, 4, 8, true>, wkv7_f32_fwd_thin_kernel<128, 8, 8, true>, 512);
-    else go(wkv7_f32_fwd_thin_kernel<128, 2, 8, false>, wkv7_f32_fwd_thin_kernel<128, 4, 8, false>, wkv7_f32_fwd_thin_kernel<128, 8, 8, false>, 512);
+    auto width64 = [&](auto full) {
+        constexpr bool F = decltype(full)::value;
+        go(wkv7_f32_fwd_thin_kernel<64, 1, 4, F, ADJ>, wkv7_f32_fwd_thin_kernel<64, 1, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<64, 2, 8, F, ADJ>, 256);
+    };
+    auto width128 = [&](auto full) {
+        constexpr bool F = decltype(full)::value;
+        go(wkv7_f32_fwd_thin_kernel<128, 2, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<128, 4, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<128, 8, 8, F, ADJ>, 512);
+    };
+    if (C == 64) width64(std::true_type());
+    else if (C < 64) width64(std::false_type());
+    else if (C == 128) width128(std::true_type());
+    else width128(std::false_type());
+}
+
+void launch_wkv7_f32_forward(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,
+                             const float* a, const float* b, const float* s0, float* y, float* ckpt, float* sT,
+                             hipStream_t stream) {
+    launch_scan<false>(B, T, H, C, w, q, k, v, a, b, s0, y, ckpt, sT, stream);
+}
+
+void launch_wkv7_f32_backward_split(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,
+                                    const float* a, const float* b, const float* dy, const float* ckpt, const float* dsT,
+                                    float* work, float* dw, float* dq, float* dk, float* dv, float* da, float* db, float* ds0,
+                                    hipStream_t stream) {
+    launch_scan<true>(B, T, H, C, w, q, k, dy, a, b, dsT, dv, work, ds0, stream);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(B * H * (T / CH64), (C + 63) / 64), dim3(64 * (C / GR)), 0, stream, T, H, C, w, q, k, v, a, b, dy,
+                           ckpt, work, dw, dq, dk, da, db);
+    };
+    if (C <= 64) go(wkv7_f32_grads_kernel<8>);
+    else go(wkv7_f32_grads_kernel<16>);
 }
 
 void launch_wkv7_f32_backward(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,

@@ -19,5 +19,10 @@ void launch_wkv7_f32_backward(int B, int T, int H, int C, const float* w, const 
                               const float* a, const float* b, const float* dy, const float* ckpt, const float* dsT,
                               float* dw, float* dq, float* dk, float* dv, float* da, float* db, float* ds0,
                               hipStream_t stream);
+// The same gradients from a scan and a kernel that takes every chunk on its own; work: wkv7_f32_saved_bytes.
+void launch_wkv7_f32_backward_split(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,
+                                    const float* a, const float* b, const float* dy, const float* ckpt, const float* dsT,
+                                    float* work, float* dw, float* dq, float* dk, float* dv, float* da, float* db, float* ds0,
+                                    hipStream_t stream);
 
 }  // namespace wkv

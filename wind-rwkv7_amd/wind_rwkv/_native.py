@@ -74,6 +74,8 @@ SIGNATURES = {
     'wind_rwkv7_attn_f32_forward': (_i, [_i] * 4 + [_vp] * 7 + [_vp] * 3 + [_vp]),
     'wind_rwkv7_attn_f32_prefill': (_i, [_i] * 4 + [_vp] * 7 + [_vp] * 2 + [_vp]),
     'wind_rwkv7_attn_f32_backward': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp] * 7 + [_vp]),
+    'wind_rwkv7_attn_f32_bwd_workspace_bytes': (_sz, [_i] * 4),
+    'wind_rwkv7_attn_f32_backward_split': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp] * 7 + [_vp, _sz] + [_vp]),
     'wind_rwkv7_pack_weights': (_i, [_i, _vp, _vp]),
     'wind_rwkv7_linear_group': (_i, [_i, _ll, _vp, _vp]),
     'wind_rwkv7_linear_wgrad_workspace_bytes': (_sz, [_ll, _i, _i]),

@@ -319,11 +319,13 @@ def _attn_f32_prefill_impl(w, q, k, v, a, b, s0, y, sT):
 
 def _attn_f32_backward_impl(w, q, k, v, a, b, dy, s, dsT, dw, dq, dk, dv, da, db, ds0):
     B, T, H, C = w.shape
+    need = _native.lib().wind_rwkv7_attn_f32_bwd_workspace_bytes(B, T, H, C)
     with torch.cuda.device(w.device):
-        _native.check(_native.lib().wind_rwkv7_attn_f32_backward(
+        ws = torch.empty(need, dtype=torch.uint8, device=w.device)
+        _native.check(_native.lib().wind_rwkv7_attn_f32_backward_split(
             B, T, H, C, w.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), a.data_ptr(), b.data_ptr(),
             dy.data_ptr(), s.data_ptr(), dsT.data_ptr(), dw.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            da.data_ptr(), db.data_ptr(), ds0.data_ptr(), _stream(w)))
+            da.data_ptr(), db.data_ptr(), ds0.data_ptr(), ws.data_ptr(), need, _stream(w)))
 
 
 _OPS.impl('attn_f32_forward', _attn_f32_forward_impl, 'CUDA')
