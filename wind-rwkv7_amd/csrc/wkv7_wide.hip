@@ -23,6 +23,7 @@
 // At the end of the file: the single-token step (decoding) for the same head sizes.
 #include "wkv7_wide_kernels.hpp"
 
+#include "device_info.hpp"
 #include "frag.hpp"
 
 namespace wkv {
@@ -270,7 +271,7 @@ struct ScanOps {
 };
 
 template <int NB, bool FWD, bool KEEP>
-__global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
+__global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, int rows, const __bf16* __restrict__ rec,
                                                    const void* __restrict__ s_in, void* __restrict__ s_out,
                                                    __bf16* __restrict__ y_, __bf16* __restrict__ kept,
                                                    float* __restrict__ centers) {
@@ -281,7 +282,8 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
     constexpr int UPW = (NU + 3) / 4;                     // units per wavefront in a full block (more in a partial one)
     constexpr int SLOT = NU * 1024, SLOTS = 3, DG = 3;    // ring; chunks a fetch runs ahead of its hand-over
     __shared__ __attribute__((aligned(16))) unsigned char ring[SLOTS * SLOT];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ib = 4 * blockIdx.y + wave;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ib = wave < rows ? rows * blockIdx.y + wave : NB;   // (rows: value blocks, one per wavefront, of this block)
     const int bh = blockIdx.x, NC = T / CHUNK;
     const Lane L;
 
@@ -711,15 +713,24 @@ constexpr size_t kept_bytes() { return (size_t)Kept<NB>::ELEMS * sizeof(__bf16);
 inline const __bf16* c(const void* p) { return static_cast<const __bf16*>(p); }
 inline __bf16* m(void* p) { return static_cast<__bf16*>(p); }
 
+// Value blocks per block of the scan: the fewest of 1, 2, 4 that still leave every block a compute unit of its own.
+inline int scan_rows(int BH, int NB) {
+    for (int rows = 1; rows < 4; rows *= 2) {
+        if ((long)BH * ((NB + rows - 1) / rows) <= compute_units()) return rows;
+    }
+    return 4;
+}
+
 template <int NB>
 void forward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v, const void* a,
              const void* b, const void* s_in, void* s_out, void* y, void* rec, void* kept, float* centers, hipStream_t stream) {
     const int nchunks = B * H * (T / CHUNK);
     hipLaunchKernelGGL(fwd_prepare_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q),
                        c(k), c(v), c(a), c(b), m(rec));
-    const dim3 grid(B * H, (NB + 3) / 4), block(256);
-    if (kept) hipLaunchKernelGGL((scan_kernel<NB, true, true>), grid, block, 0, stream, T, H, state_f32, c(rec), s_in, s_out, m(y), m(kept), centers);
-    else hipLaunchKernelGGL((scan_kernel<NB, true, false>), grid, block, 0, stream, T, H, state_f32, c(rec), s_in, s_out, m(y), m(kept), centers);
+    const int rows = scan_rows(B * H, NB);
+    const dim3 grid(B * H, (NB + rows - 1) / rows), block(256);
+    if (kept) hipLaunchKernelGGL((scan_kernel<NB, true, true>), grid, block, 0, stream, T, H, state_f32, rows, c(rec), s_in, s_out, m(y), m(kept), centers);
+    else hipLaunchKernelGGL((scan_kernel<NB, true, false>), grid, block, 0, stream, T, H, state_f32, rows, c(rec), s_in, s_out, m(y), m(kept), centers);
 }
 template <int NB>
 void backward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v, const void* a,
@@ -728,8 +739,9 @@ void backward(int B, int T, int H, int state_f32, const void* w, const void* q, 
     const int nchunks = B * H * (T / CHUNK);
     hipLaunchKernelGGL(bwd_prepare_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q),
                        c(a), c(b), c(dy), m(rec));
-    hipLaunchKernelGGL((scan_kernel<NB, false, true>), dim3(B * H, (NB + 3) / 4), dim3(256), 0, stream, T, H,
-                       state_f32, c(rec), ds_in, ds_out, static_cast<__bf16*>(nullptr), m(kept_b), static_cast<float*>(nullptr));
+    const int rows = scan_rows(B * H, NB);
+    hipLaunchKernelGGL((scan_kernel<NB, false, true>), dim3(B * H, (NB + rows - 1) / rows), dim3(256), 0, stream, T, H,
+                       state_f32, rows, c(rec), ds_in, ds_out, static_cast<__bf16*>(nullptr), m(kept_b), static_cast<float*>(nullptr));
     hipLaunchKernelGGL(grads_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k),
                        c(v), c(a), c(b), c(dy), c(kept_f), c(kept_b), m(dw), m(dq), m(dk), m(dv), m(da), m(db));
 }
