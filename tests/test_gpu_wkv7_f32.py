@@ -69,7 +69,18 @@ def test_f32_head_sizes(c_oracle, C):
 @pytest.mark.parametrize('C', [64, 128])
 def test_f32_many_heads(c_oracle, C):
     """More (batch, head) pairs than half the compute units: the forward runs one block per head with all its rows."""
-    B, T, H = 34, 32, 4
+    _many_heads(c_oracle, 34, 4, C)
+
+
+# blocks per head: 64 channels 2 (70 heads), 2 (260); 128 channels 2 (70), 8 (16); 96 channels 4 (50)
+@pytest.mark.parametrize('B,H,C', [(14, 5, 64), (65, 4, 64), (14, 5, 128), (4, 4, 128), (10, 5, 96), (65, 4, 32)])
+def test_f32_blocks_per_head(c_oracle, B, H, C):
+    """The scan cuts a head over more or fewer blocks by the number of (batch, head) pairs."""
+    _many_heads(c_oracle, B, H, C)
+
+
+def _many_heads(c_oracle, B, H, C):
+    T = 32
     d = inputs.wkv7_inputs(B, T, H, C, seed=260 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
     args = [d[n] for n in 'qwkvab']
     y_ref, sT_ref = c_oracle.forward(*args, d['s0'])

@@ -12,9 +12,12 @@
 // DPP adds (and one lane swap); a wavefront holds 4 or 2 such row groups, and a column sum over them (S^T dy, dS^T v,
 // ...) is three (one) of gfx950's lane swaps (col_sum4, store_col_sums), then LDS across the wavefronts.  The vectors
 // of a token are read as one 16-byte LDS access each, one token ahead of their use.
-// The value rows of a state never mix, so a head can be cut over blocks by rows.  Forward: eight wavefronts per block
-// (two per SIMD cover each other's waits), four or two blocks per head (a quarter or half of the rows each) while every
-// block still gets a compute unit of its own, else one block with all rows.
+// The value rows of a state never mix, so a head is cut over blocks by rows (scan_split).  In the scan, four or eight
+// wavefronts of a block carry the recurrence and touch LDS only; four more fetch the next chunk, turn it into operands in
+// the other half of a double buffer and carry the results of the chunk before to memory, with one barrier per chunk.
+// (Staging by the recurrence's own wavefronts, between barriers, was a third of its time: 227 -> 170 us at 8 x 1024 tokens
+// x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  What bounds it now is LDS: a wavefront reads five vectors of
+// 64 channels per token, 360 of the 400 cycles that a token takes with eight wavefronts on a compute unit.
 // The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
 // direction (it keeps the state gradient arriving at every chunk's end and dsa of every token, and leaves dv and ds0)
 // and then a kernel in which every chunk is on its own: it recomputes states and state gradients without a row sum to
@@ -22,16 +25,25 @@
 // A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
-//   1 x 256 tokens x 4 heads of 64   274 -> 122        8 x 1024 x 6 heads of 128   2420 -> 1365
-//   8 x 1024 x 12 heads of 64        844 -> 702        32 x 1024 x 12 heads of 64  2395 -> 1954
+//   1 x 256 tokens x 4 heads of 64   274 -> 121        8 x 1024 x 6 heads of 128   2420 -> 1250
+//   8 x 1024 x 12 heads of 64        844 -> 629        32 x 1024 x 12 heads of 64  2395 -> 1954
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
 
+#include "device_info.hpp"
+
 namespace wkv {
 namespace {
+
+// a barrier that orders LDS only: loads and stores to memory stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -138,23 +150,23 @@ __host__ __device__ inline long saved_states(long BH, int T, int C) { return BH 
 // is the forward's step with (a, decay q, b, k, v) in the places of (b, k, a, decay q, dy): two row sums on the state
 // before its update, a rank-one term with the first of them and one with the row vector.  v, s0, y, ckpt, sT are then
 // dy, dsT, dv, the workspace of the gradient kernel below (E arriving at every chunk's end, dsa of every token) and ds0.
-template <int C, int R, int NW, bool FULL, bool ADJ>
-__global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H, int CR, const float* __restrict__ w,
+template <int C, int R, int NW, int NP, bool FULL, bool ADJ>
+__global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, int H, int CR, const float* __restrict__ w,
                                                              const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ v, const float* __restrict__ a,
                                                              const float* __restrict__ b, const float* __restrict__ s0,
                                                              float* __restrict__ y, float* __restrict__ ckpt,
                                                              float* __restrict__ sT) {
     typedef float f2 __attribute__((ext_vector_type(2)));
-    constexpr int CH = CH64, LPR = C / 4, GPW = 64 / LPR, THREADS = 64 * NW, ROWS = NW * GPW * R, NSPLIT = C / ROWS;
-    constexpr int PER = CH * C / THREADS, TPJ = THREADS / C, NH = C / 64;
-    static_assert(C % ROWS == 0 && (CH * C) % THREADS == 0 && (CH * ROWS) % THREADS == 0, "whole tokens and rows per thread");
-    __shared__ __attribute__((aligned(16))) float in[FWD_VECS][CH][C];    // the slot of q holds decay * q
-    __shared__ f2 bkq[CH][NH];                                            // (b . q, k . q) of every token, per 64 channels
-    __shared__ __attribute__((aligned(16))) float yout[CH][ROWS], saout[CH][ROWS];
+    constexpr int CH = CH64, LPR = C / 4, GPW = 64 / LPR, ROWS = NW * GPW * R, NSPLIT = C / ROWS, NH = C / 64;
+    constexpr int PT = 64 * NP, PER = CH * C / PT, TPJ = PT / C;
+    static_assert(C % ROWS == 0 && (CH * C) % PT == 0 && PT % C == 0 && (CH * ROWS) % PT == 0, "whole tokens and rows per thread");
+    __shared__ __attribute__((aligned(16))) float in[2][FWD_VECS][CH][C];   // the slot of q holds decay * q
+    __shared__ f2 bkq[2][CH][NH];                                           // (b . q, k . q) of every token, per 64 channels
+    __shared__ __attribute__((aligned(16))) float yout[2][CH][ROWS + 1], saout[2][CH][ROWS + 1];
     const int bh = blockIdx.x / NSPLIT, part = blockIdx.x % NSPLIT, h = bh % H;
     const long bt0 = (long)(bh / H) * T;
-    const int tid = threadIdx.x, lane = tid & 63, jb = lane % LPR, rl = ((tid >> 6) * GPW + lane / LPR) * R;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, jb = lane % LPR, rl = (wv * GPW + lane / LPR) * R;
     const int row0 = part * ROWS + rl, col0 = 4 * jb;
     const float* const src[FWD_VECS] = {w, q, k, v, a, b};
     float* const sav = ckpt == nullptr ? nullptr : ckpt + saved_states(gridDim.x / NSPLIT, T, CR);
@@ -163,20 +175,17 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
     // CR: the head size itself; C: the width the block works at (channels and rows past CR read as zero, are never
     // written, and stay zero in the state).  FULL: CR == C, no access needs a bound.
     const unsigned ld = (unsigned)H * CR;                                    // floats between consecutive tokens
-    const bool col_ok = FULL || col0 < CR, stage_ok = FULL || (int)(tid % C) < CR;
-    const unsigned state_off = (unsigned)(row0 * CR + (col_ok ? col0 : 0));  // this thread's first row in a CR x CR state
-    const unsigned tok_off = (unsigned)(tid / C) * ld + (stage_ok ? tid % C : 0);   // (token, channel) this thread stages
-    auto chunk_base = [&](int c0) { return seq_index(bt0 + c0, H, h, 0, CR); };
-    auto row_ok = [&](int r) { return FULL || (col_ok && row0 + r < CR); };
-    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int NC = T / CH;
+    auto chunk_start = [&](int n) { return CH * (ADJ ? NC - 1 - n : n); };   // first token of the n-th chunk in the order of the walk
+    auto chunk_base = [&](int n) { return seq_index(bt0 + chunk_start(n), H, h, 0, CR); };
 
-    f4 S[R];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        S[r] = row_ok(r) ? *reinterpret_cast<const f4*>(s0 + (long)bh * CR * CR + (state_off + r * CR)) : zero;
+    // ---- moving data: thread ptid of PT ----
+    const int ptid = threadIdx.x - 64 * NW, pch = ptid % C;
+    const bool stage_ok = FULL || pch < CR;
+    const unsigned tok_off = (unsigned)(ptid / C) * ld + (stage_ok ? pch : 0);   // (token, channel) this thread stages
     float pre[FWD_VECS][PER];
-    auto fetch = [&](int c0) {
-        const long base = chunk_base(c0);
+    auto fetch = [&](int n) {
+        const long base = chunk_base(n < NC ? n : NC - 1);   // (past the last chunk: the same one again, not used)
 #pragma unroll
         for (int vec = 0; vec < FWD_VECS; vec++) {
 #pragma unroll
@@ -186,36 +195,70 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
             }
         }
     };
-    fetch(ADJ ? T - CH : 0);
-    for (int n0 = 0; n0 < T; n0 += CH) {
-        const int c0 = ADJ ? T - CH - n0 : n0;
-        // stage the chunk: the decay instead of w, decay * q instead of q.  With them
-        //   y_t = S_t q = S_{t-1} (decay * q) + (S_{t-1} a) (b . q) + v (k . q),
-        // so that both row sums of a token work on the state BEFORE its update and neither waits for the other.
+    // the fetched chunk into a buffer: the decay instead of w, decay * q instead of q.  With them
+    //   y_t = S_t q = S_{t-1} (decay * q) + (S_{t-1} a) (b . q) + v (k . q),
+    // so that both row sums of a token work on the state BEFORE its update and neither waits for the other.
+    auto stage = [&](int buf) {
 #pragma unroll
         for (int j = 0; j < PER; j++) {
-            const int tok = TPJ * j + tid / C, ch = tid % C;
+            const int tok = TPJ * j + ptid / C;
             const float d = expf(-expf(pre[V_DEC][j]));
-            in[V_DEC][tok][ch] = d;
-            in[V_Q][tok][ch] = d * pre[V_Q][j];
-            in[V_K][tok][ch] = pre[V_K][j];
-            in[V_V][tok][ch] = pre[V_V][j];
-            in[V_A][tok][ch] = pre[V_A][j];
-            in[V_B][tok][ch] = pre[V_B][j];
+            in[buf][V_DEC][tok][pch] = d;
+            in[buf][V_Q][tok][pch] = d * pre[V_Q][j];
+            in[buf][V_K][tok][pch] = pre[V_K][j];
+            in[buf][V_V][tok][pch] = pre[V_V][j];
+            in[buf][V_A][tok][pch] = pre[V_A][j];
+            in[buf][V_B][tok][pch] = pre[V_B][j];
             const float bq = wave_sum(pre[V_B][j] * pre[V_Q][j]), kq = wave_sum(pre[V_K][j] * pre[V_Q][j]);
-            if (lane == 0) bkq[tok][ch >> 6] = f2{bq, kq};
+            if (lane == 0) bkq[buf][tok][pch >> 6] = f2{bq, kq};
         }
+    };
+    auto copy_out = [&](int n, int buf) {
+        const long base = chunk_base(n);
+#pragma unroll
+        for (int m = 0; m < CH * ROWS / PT; m++) {
+            const int e = ptid + PT * m;
+            const int tok = e / ROWS, ch = e % ROWS;
+            const unsigned at = (unsigned)tok * ld + (unsigned)(part * ROWS + ch);
+            if (FULL || part * ROWS + ch < CR) {
+                (y + base)[at] = yout[buf][tok][ch];
+                if (sav != nullptr) (sav + base)[at] = saout[buf][tok][ch];
+            }
+        }
+    };
+    if (wv >= NW) {   // (the same number of barriers as below)
+        fetch(0);
+        stage(0);
+        fetch(1);
+        lds_barrier();
+        for (int n = 0; n < NC; n++) {
+            if (n + 1 < NC) stage((n + 1) & 1);
+            fetch(n + 2);
+            if (n > 0) copy_out(n - 1, (n - 1) & 1);
+            lds_barrier();
+        }
+        copy_out(NC - 1, (NC - 1) & 1);
+        return;
+    }
+
+    // ---- the recurrence ----
+    const bool col_ok = FULL || col0 < CR;
+    const unsigned state_off = (unsigned)(row0 * CR + (col_ok ? col0 : 0));  // this thread's first row in a CR x CR state
+    auto row_ok = [&](int r) { return FULL || (col_ok && row0 + r < CR); };
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    f4 S[R];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        S[r] = row_ok(r) ? *reinterpret_cast<const f4*>(s0 + (long)bh * CR * CR + (state_off + r * CR)) : zero;
+    auto walk = [&](int n, int buf) {
         if (ckpt != nullptr) {
-            float* const to = ckpt + ((long)bh * (T / CH) + c0 / CH) * CR * CR;
+            float* const to = ckpt + ((long)bh * NC + chunk_start(n) / CH) * CR * CR;
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 if (row_ok(r)) *reinterpret_cast<f4*>(to + (state_off + r * CR)) = S[r];
             }
         }
-        __syncthreads();
-        fetch(n0 + CH >= T ? c0 : ADJ ? c0 - CH : c0 + CH);   // (after the last chunk: the same one again, not used)
-        // a token's operands are requested from LDS one token ahead (the stores of the results in between keep the
-        // compiler from moving the reads up by itself)
+        // a token's operands are requested from LDS one token ahead
         struct Ops {
             f4 dec, x1, x2, u1, u2;   // operands of the two row sums, column vectors of the two rank-one terms
             RowVals<R> vr;
@@ -223,22 +266,24 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
         };
         auto read_ops = [&](int t) {
             Ops o;
-            o.dec = *reinterpret_cast<const f4*>(&in[V_DEC][t][col0]);
-            o.x1 = *reinterpret_cast<const f4*>(&in[ADJ ? V_B : V_A][t][col0]);
-            o.u1 = *reinterpret_cast<const f4*>(&in[ADJ ? V_A : V_B][t][col0]);
-            o.u2 = *reinterpret_cast<const f4*>(&in[ADJ ? V_Q : V_K][t][col0]);
-            o.x2 = *reinterpret_cast<const f4*>(&in[ADJ ? V_K : V_Q][t][col0]);
-            o.vr = lds_rows<R>(&in[V_V][t][row0]);
-            o.sc = bkq[t][0];
-            if constexpr (NH == 2) o.sc += bkq[t][1];
+            o.dec = *reinterpret_cast<const f4*>(&in[buf][V_DEC][t][col0]);
+            o.x1 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_B : V_A][t][col0]);
+            o.u1 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_A : V_B][t][col0]);
+            o.u2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_Q : V_K][t][col0]);
+            o.x2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_K : V_Q][t][col0]);
+            o.vr = lds_rows<R>(&in[buf][V_V][t][row0]);
+            o.sc = bkq[buf][t][0];
+            if constexpr (NH == 2) o.sc += bkq[buf][t][1];
             return o;
         };
         Ops ahead = read_ops(ADJ ? CH - 1 : 0);
+        RowVals<R> ykeep = {}, sakeep = {};
 #pragma unroll
         for (int i = 0; i < CH; i++) {
             const int t = ADJ ? CH - 1 - i : i;
             const Ops o = ahead;
             if (i + 1 < CH) ahead = read_ops(ADJ ? t - 1 : t + 1);
+            asm volatile("" ::: "memory");   // (else all sixteen tokens' operands are requested at once)
             RowVals<R> yr, sar;
 #pragma unroll
             for (int r = 0; r < R; r++) {
@@ -248,25 +293,25 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_fwd_thin_kernel(int T, int H
                 if constexpr (!ADJ) yr.x[r] += sar.x[r] * o.sc[0];
                 S[r] = S[r] * o.dec + sar.x[r] * o.u1 + o.vr.x[r] * o.u2;
             }
-            if (jb == 0) {
+            // lane t of a row's lanes keeps token t's results (a store per token by one lane would be a branch per token,
+            // which nothing is scheduled across); 32 lanes per row: both of its DPP rows hold and store the same
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    yout[t][rl + r] = yr.x[r];
-                    saout[t][rl + r] = sar.x[r];
-                }
+            for (int r = 0; r < R; r++) {
+                ykeep.x[r] = jb % CH == t ? yr.x[r] : ykeep.x[r];
+                sakeep.x[r] = jb % CH == t ? sar.x[r] : sakeep.x[r];
+                asm volatile("" : "+v"(ykeep.x[r]));   // (here and now: put off, it keeps every token's operands alive)
             }
         }
-        __syncthreads();
 #pragma unroll
-        for (int m = 0; m < CH * ROWS / THREADS; m++) {
-            const int e = tid + THREADS * m;
-            const int tok = e / ROWS, ch = e % ROWS;
-            const unsigned at = (unsigned)tok * ld + (unsigned)(part * ROWS + ch);
-            if (FULL || part * ROWS + ch < CR) {
-                (y + chunk_base(c0))[at] = yout[tok][ch];
-                if (sav != nullptr) (sav + chunk_base(c0))[at] = saout[tok][ch];
-            }
+        for (int r = 0; r < R; r++) {
+            yout[buf][jb % CH][rl + r] = ykeep.x[r];
+            saout[buf][jb % CH][rl + r] = sakeep.x[r];
         }
+    };
+    lds_barrier();
+    for (int n = 0; n < NC; n++) {
+        walk(n, n & 1);
+        lds_barrier();
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -622,14 +667,18 @@ __global__ __launch_bounds__(256) void zero5_kernel(long n4, f4* __restrict__ p0
 }
 
 
-// blocks per head in the forward kernel: as many of 4, 2, 1 as still leave every block a compute unit of its own
-int forward_split(int BH) {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
-        return n;
-    }();
-    return 4 * BH <= cus ? 4 : 2 * BH <= cus ? 2 : 1;
+// Blocks per head in the scan.  Up to 64 channels: as many of 4, 2, 1 as still leave every block a compute unit of its own
+// (us per 1024 tokens: 98, 160, 250; 96 heads in 4 blocks each 184, in 2 165; 256 heads in 2 blocks each 340, in 1 290),
+// and 2 again past one head per compute unit, where several blocks share one and smaller ones fill it more evenly (384
+// heads x 512 tokens in 1 block each 264 us, in 2 245 us).  Above 64 channels a block has a compute unit to itself (LDS),
+// so the blocks run in rounds: the fewest rounds x time of a round (ns per token: 215, 350, 600 in 8, 4, 2 blocks; 192
+// heads x 256 tokens: 350, 275, 311 us).
+int scan_split(int BH, int C) {
+    const long cus = compute_units(), n = BH;
+    if (C <= 64) return 4 * n <= cus ? 4 : 2 * n <= cus || n > cus ? 2 : 1;
+    auto cost = [&](int split, int ns) { return (split * n + cus - 1) / cus * ns; };
+    const long c8 = cost(8, 215), c4 = cost(4, 350), c2 = cost(2, 600);
+    return c8 <= c4 && c8 <= c2 ? 8 : c4 <= c2 ? 4 : 2;
 }
 
 }  // namespace
@@ -642,23 +691,24 @@ size_t wkv7_f32_saved_bytes(int B, int T, int H, int C) {
 template <bool ADJ>
 static void launch_scan(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v, const float* a,
                         const float* b, const float* s0, float* y, float* ckpt, float* sT, hipStream_t stream) {
-    const int split = forward_split(B * H);
-    auto go = [&](auto k4, auto k2, auto k1, int threads4) {
-        auto launch = [&](auto kernel, int threads) {
-            hipLaunchKernelGGL(kernel, dim3(split * B * H), dim3(threads), 0, stream, T, H, C, w, q, k, v, a, b, s0, y, ckpt, sT);
-        };
-        if (split == 4) launch(k4, threads4);
-        else if (split == 2) launch(k2, 512);
-        else launch(k1, 512);
+    const int split = scan_split(B * H, C);
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(split * B * H), dim3(threads), 0, stream, T, H, C, w, q, k, v, a, b, s0, y, ckpt, sT);
     };
-    // (width, rows per thread, wavefronts): rows per block = wavefronts x row groups per wavefront x rows per thread
+    // (width, rows per thread, wavefronts of the recurrence, of the moves): rows per block = wavefronts x row groups per
+    // wavefront x rows per thread
     auto width64 = [&](auto full) {
         constexpr bool F = decltype(full)::value;
-        go(wkv7_f32_fwd_thin_kernel<64, 1, 4, F, ADJ>, wkv7_f32_fwd_thin_kernel<64, 1, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<64, 2, 8, F, ADJ>, 256);
+        if (split == 4) launch(wkv7_f32_scan_kernel<64, 1, 4, 4, F, ADJ>, 512);
+        else if (split == 2 && B * H > compute_units()) launch(wkv7_f32_scan_kernel<64, 2, 4, 4, F, ADJ>, 512);
+        else if (split == 2) launch(wkv7_f32_scan_kernel<64, 1, 8, 4, F, ADJ>, 768);
+        else launch(wkv7_f32_scan_kernel<64, 2, 8, 4, F, ADJ>, 768);
     };
     auto width128 = [&](auto full) {
         constexpr bool F = decltype(full)::value;
-        go(wkv7_f32_fwd_thin_kernel<128, 2, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<128, 4, 8, F, ADJ>, wkv7_f32_fwd_thin_kernel<128, 8, 8, F, ADJ>, 512);
+        if (split == 8) launch(wkv7_f32_scan_kernel<128, 2, 4, 4, F, ADJ>, 512);
+        else if (split == 4) launch(wkv7_f32_scan_kernel<128, 2, 8, 4, F, ADJ>, 768);
+        else launch(wkv7_f32_scan_kernel<128, 4, 8, 4, F, ADJ>, 768);
     };
     if (C == 64) width64(std::true_type());
     else if (C < 64) width64(std::false_type());
