@@ -25,8 +25,8 @@
 // A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
-//   1 x 256 tokens x 4 heads of 64   274 -> 121        8 x 1024 x 6 heads of 128   2420 -> 1250
-//   8 x 1024 x 12 heads of 64        844 -> 629        32 x 1024 x 12 heads of 64  2395 -> 1954
+//   1 x 256 tokens x 4 heads of 64   274 -> 102        8 x 1024 x 6 heads of 128   2420 -> 1214
+//   8 x 1024 x 12 heads of 64        844 -> 595        32 x 1024 x 12 heads of 64  2395 -> 1778
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -525,13 +525,14 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
 // A lane holds ONE column of GR rows (CR / GR wavefronts), so every column sum is a chain of multiply-adds inside the lane
 // and one sum over the wavefronts through LDS; what belongs to a row (v, S a, dy, dsa) is read from LDS as a broadcast.
 // The states of GWIN tokens are recomputed into registers; the second half of a chunk first runs through the first.
-// Bound: vector issue, 13 instructions per state element and token: 236 us at 8 x 1024 tokens x 12 heads of 64, of which
-// 176 us are issue alone.  Through scalar loads and registers the row operands cost more (390 us: every token waits for
-// them, and the scalar cache holds a quarter of what the blocks of a compute unit read).
+// Bound: vector issue, 13 instructions per state element and token: 217 us at 8 x 1024 tokens x 12 heads of 64, of which
+// 176 us are issue alone.  Tried instead: the row operands through scalar loads into scalar registers, 390 us (every token
+// waits for them, and the scalar cache holds a quarter of what the blocks of a compute unit read); two columns and eight
+// rows per lane (half the reads of row operands per multiply-add, but two wavefronts per SIMD instead of four), 307 us.
 constexpr int GR = 8, GWIN = 8, GRED = 4;   // rows per wavefront, tokens of kept states, tokens between sums over wavefronts
 
-template <int NWMAX>
-__global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, int H, int CR, const float* __restrict__ w,
+template <int CR>   // head size
+__global__ __launch_bounds__(64 * (CR / GR), 4) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w,
                                                                        const float* __restrict__ q, const float* __restrict__ k,
                                                                        const float* __restrict__ v, const float* __restrict__ a,
                                                                        const float* __restrict__ b, const float* __restrict__ dy,
@@ -539,17 +540,18 @@ __global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, in
                                                                        const float* __restrict__ work, float* __restrict__ dw,
                                                                        float* __restrict__ dq, float* __restrict__ dk,
                                                                        float* __restrict__ da, float* __restrict__ db) {
-    constexpr int CH = CH64, COLS = 64;
+    constexpr int CH = CH64, COLS = 64, NW = CR / GR, THREADS = 64 * NW;
+    constexpr int RPT = (CH * CR + THREADS - 1) / THREADS, TPW = (CH + NW - 1) / NW;   // row values and tokens a thread stages
     static_assert(CH == 2 * GWIN && GWIN % GRED == 0 && GR == 8, "two windows per chunk; two sums of four rows");
     enum { G_DEC = 0, G_Q, G_K, G_A, G_B, G_DDEC, G_VECS };
     enum { Q_V = 0, Q_SA, Q_DY, Q_DSA, Q_VECS };
     __shared__ float in[G_VECS][CH][COLS];
-    __shared__ __attribute__((aligned(16))) float rows[Q_VECS][CH][GR * NWMAX];
-    __shared__ float red[NWMAX][RED_VECS][GRED][COLS];
-    const int NC = T / CH, NW = CR / GR, bh = blockIdx.x / NC, chunk = blockIdx.x - bh * NC, h = bh % H;
+    __shared__ __attribute__((aligned(16))) float rows[Q_VECS][CH][CR];
+    __shared__ float red[NW][RED_VECS][GRED][COLS];
+    const int NC = T / CH, bh = blockIdx.x / NC, chunk = blockIdx.x - bh * NC, h = bh % H;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row0 = wv * GR;
     const int col = COLS * blockIdx.y + lane;
-    const bool col_ok = col < CR;
+    const bool col_ok = CR % COLS == 0 || col < CR;
     const int colc = col_ok ? col : 0;   // (lanes past the head size read column 0 and write nothing)
     const long base = seq_index((long)(bh / H) * T + (long)chunk * CH, H, h, 0, CR);
     const unsigned ld = (unsigned)H * CR;
@@ -562,17 +564,35 @@ __global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, in
         Sx[r] = (ckpt + st)[(unsigned)(r * CR + colc)];
         dS[r] = (work + st)[(unsigned)(r * CR + colc)];
     }
-    for (int e = threadIdx.x; e < CH * CR; e += 64 * NW) {
-        const int t = e / CR, r = e - t * CR;
+    // everything is requested before anything is waited for (with trip counts known only at run time 236 instead of 217 us)
+    float row_pre[RPT][Q_VECS], col_pre[TPW][5];
+    const float* const col_src[5] = {w, q, k, a, b};
 #pragma unroll
-        for (int x = 0; x < Q_VECS; x++) rows[x][t][r] = (row_src[x] + base)[(unsigned)t * ld + r];
+    for (int i = 0; i < RPT; i++) {
+        const int e = min((int)threadIdx.x + THREADS * i, CH * CR - 1), t = e / CR, r = e - t * CR;
+#pragma unroll
+        for (int x = 0; x < Q_VECS; x++) row_pre[i][x] = (row_src[x] + base)[(unsigned)t * ld + r];
     }
-    for (int t = wv; t < CH; t += NW) {
-        const unsigned at = (unsigned)t * ld + colc;
-        const float ew = expf((w + base)[at]), d = expf(-ew);
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const unsigned at = (unsigned)min(wv + NW * i, CH - 1) * ld + colc;
+#pragma unroll
+        for (int x = 0; x < 5; x++) col_pre[i][x] = (col_src[x] + base)[at];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < RPT; i++) {   // (indices past the end repeat the last: the same value to the same place)
+        const int e = min((int)threadIdx.x + THREADS * i, CH * CR - 1), t = e / CR, r = e - t * CR;
+#pragma unroll
+        for (int x = 0; x < Q_VECS; x++) rows[x][t][r] = row_pre[i][x];
+    }
+#pragma unroll
+    for (int i = 0; i < TPW; i++) {
+        const int t = min(wv + NW * i, CH - 1);
+        const float ew = expf(col_pre[i][0]), d = expf(-ew);
         in[G_DEC][t][lane] = d, in[G_DDEC][t][lane] = -ew * d;
-        in[G_Q][t][lane] = (q + base)[at], in[G_K][t][lane] = (k + base)[at];
-        in[G_A][t][lane] = (a + base)[at], in[G_B][t][lane] = (b + base)[at];
+        in[G_Q][t][lane] = col_pre[i][1], in[G_K][t][lane] = col_pre[i][2];
+        in[G_A][t][lane] = col_pre[i][3], in[G_B][t][lane] = col_pre[i][4];
     }
     __syncthreads();
     auto row_vals = [&](int x, int t) { return lds_rows<GR>(&rows[x][t][row0]); };
@@ -585,26 +605,17 @@ __global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, in
 #pragma unroll
         for (int r = 0; r < GR; r++) to[r] = from[r] * o.dec + o.sar.x[r] * o.bv + o.vr.x[r] * o.kv;
     };
-    float* const dst[RED_VECS] = {dq, dk, db, da, dw};
 #pragma unroll 1
     for (int t0 = CH - GWIN; t0 >= 0; t0 -= GWIN) {
         float S[GWIN + 1][GR];   // S[t] enters token t0 + t
 #pragma unroll
         for (int r = 0; r < GR; r++) S[0][r] = Sx[r];
-        AdvOps adv = read_adv(0);
 #pragma unroll 2
-        for (int t = 0; t < t0; t++) {
-            const AdvOps o = adv;
-            adv = read_adv(t + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            advance(S[0], S[0], o);
-        }
+        for (int t = 0; t < t0; t++) advance(S[0], S[0], read_adv(t));
 #pragma unroll
         for (int t = 0; t < GWIN; t++) {
-            const AdvOps o = adv;
-            if (t + 1 < GWIN) adv = read_adv(t0 + t + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            advance(S[t], S[t + 1], o);
+            advance(S[t], S[t + 1], read_adv(t0 + t));
+            if (t > GWIN / 2) __builtin_amdgcn_sched_barrier(0);   // (reading further ahead would spill by then)
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -638,16 +649,21 @@ __global__ __launch_bounds__(64 * NWMAX, 4) void wkv7_f32_grads_kernel(int T, in
             if (tw % GRED == 0) {
                 __syncthreads();
                 // the wavefronts' sums of GRED tokens, in a fixed order, and out
-                for (int e = wv; e < RED_VECS * GRED; e += NW) {
-                    const int x = e / GRED, j = e % GRED;
-                    float even = 0.f, odd = 0.f;   // (sums of pairs in two chains; NW is even)
-                    for (int g = 0; g < NW; g += 4) {
-                        even += red[g][x][j][lane] + red[g + 1][x][j][lane];
-                        if (g + 2 < NW) odd += red[g + 2][x][j][lane] + red[g + 3][x][j][lane];
+#pragma unroll 1
+                for (int i = 0; i < (RED_VECS * GRED + NW - 1) / NW; i++) {
+                    const int e = wv + NW * i, x = e / GRED, j = e % GRED;
+                    if (e < RED_VECS * GRED) {
+                        float even = 0.f, odd = 0.f;   // (sums of pairs in two chains)
+#pragma unroll 2
+                        for (int g = 0; g < NW; g += 4) {
+                            even += red[g][x][j][lane] + red[g + 1][x][j][lane];
+                            if (g + 2 < NW) odd += red[g + 2][x][j][lane] + red[g + 3][x][j][lane];
+                        }
+                        float sum = even + odd;
+                        if (x == R_DW) sum *= in[G_DDEC][t + j][lane];
+                        float* const to = x == R_DQ ? dq : x == R_DK ? dk : x == R_DB ? db : x == R_DA ? da : dw;
+                        if (col_ok) (to + base)[(unsigned)(t + j) * ld + colc] = sum;
                     }
-                    float sum = even + odd;
-                    if (x == R_DW) sum *= in[G_DDEC][t + j][lane];
-                    if (col_ok) (dst[x] + base)[(unsigned)(t + j) * ld + colc] = sum;
                 }
                 __syncthreads();
             }
@@ -728,11 +744,19 @@ void launch_wkv7_f32_backward_split(int B, int T, int H, int C, const float* w, 
                                     hipStream_t stream) {
     launch_scan<true>(B, T, H, C, w, q, k, dy, a, b, dsT, dv, work, ds0, stream);
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(B * H * (T / CH64), (C + 63) / 64), dim3(64 * (C / GR)), 0, stream, T, H, C, w, q, k, v, a, b, dy,
-                           ckpt, work, dw, dq, dk, da, db);
+        hipLaunchKernelGGL(kernel, dim3(B * H * (T / CH64), (C + 63) / 64), dim3(64 * (C / GR)), 0, stream, T, H, w, q, k, v, a, b, dy, ckpt,
+                           work, dw, dq, dk, da, db);
     };
-    if (C <= 64) go(wkv7_f32_grads_kernel<8>);
-    else go(wkv7_f32_grads_kernel<16>);
+    switch (C) {
+        case 16: go(wkv7_f32_grads_kernel<16>); break;
+        case 32: go(wkv7_f32_grads_kernel<32>); break;
+        case 48: go(wkv7_f32_grads_kernel<48>); break;
+        case 64: go(wkv7_f32_grads_kernel<64>); break;
+        case 80: go(wkv7_f32_grads_kernel<80>); break;
+        case 96: go(wkv7_f32_grads_kernel<96>); break;
+        case 112: go(wkv7_f32_grads_kernel<112>); break;
+        default: go(wkv7_f32_grads_kernel<128>);
+    }
 }
 
 void launch_wkv7_f32_backward(int B, int T, int H, int C, const float* w, const float* q, const float* k, const float* v,
