@@ -23,6 +23,8 @@
 // At the end of the file: the single-token step (decoding) for the same head sizes.
 #include "wkv7_wide_kernels.hpp"
 
+#include <type_traits>
+
 #include "device_info.hpp"
 #include "frag.hpp"
 
@@ -254,14 +256,15 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(int T, int H, int nchu
 }
 
 // ------------------------------------------------------------------------------------------------
-// scan: wavefront ib owns value rows 16 ib .. 16 ib + 15 of the state (NB fp32 fragments); a block is up to four of
-// them (one per SIMD, each with the whole register file), a (batch, head) takes ceil(NB / 4) blocks.  Rows of the
-// state evolve independently, so the wavefronts never exchange results.  What they share is the chunk's operands
-// (all but the (U0, V) pair of their own value block): the block's wavefronts each fetch a quarter of that run of the
-// record, three chunks ahead, and hand it on through a ring of three LDS slots two chunks ahead of its use; one
-// LDS-only barrier per chunk.  (Each wavefront fetching everything for itself needs three sets of 104 registers at
-// C = 128 for the same distance; beyond 256 registers the allocator parks freshly loaded values in accumulator
-// registers, which waits for the load: 1.4 us per chunk instead of 0.5.)
+// scan: a working wavefront owns value rows 16 ib .. 16 ib + 15 of the state (NB fp32 fragments); a block has W of them,
+// a (batch, head) takes ceil(NB / W) blocks.  Rows of the state evolve independently, so the wavefronts never exchange
+// results.  Working wavefronts touch LDS only: loading wavefronts fetch the chunk's operands three chunks ahead into
+// registers and hand them on through a ring of three LDS slots two chunks ahead of their use, storing ones carry what the
+// workers left in a double buffer one chunk ago to memory, 16 bytes per lane; one LDS-only barrier per chunk.
+// Forward + backward, us, against workers that fetch and store for themselves: 1 x 512 tokens x 4 heads of 128 106 -> 92,
+// 8 x 1024 x 6 heads of 128 319 -> 312, 16 x 1024 x 6 heads of 128 571 -> 554, 4 x 1024 x 5 heads of 112 161 -> 142.  Bound:
+// the kept states' 113 MB per direction at 8 x 1024 x 6 heads of 128 (without the stores the two scans together take 76 us
+// instead of 129, without the loads 98).
 // ------------------------------------------------------------------------------------------------
 template <int NB, bool FWD>
 struct ScanOps {
@@ -270,20 +273,24 @@ struct ScanOps {
     f32x4 fw[NB];
 };
 
-template <int NB, bool FWD, bool KEEP>
-__global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, int rows, const __bf16* __restrict__ rec,
-                                                   const void* __restrict__ s_in, void* __restrict__ s_out,
-                                                   __bf16* __restrict__ y_, __bf16* __restrict__ kept,
-                                                   float* __restrict__ centers) {
+constexpr int scan_helpers(int W) { return W == 4 ? 4 : 2; }
+
+template <int NB, bool FWD, bool KEEP, int W>
+__global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
+                                                                          const void* __restrict__ s_in, void* __restrict__ s_out,
+                                                                          __bf16* __restrict__ y_, __bf16* __restrict__ kept,
+                                                                          float* __restrict__ centers) {
     using R = Rec<NB, FWD>;
     using K = Kept<NB>;
-    constexpr int C = 16 * NB, NP = (NB + 1) / 2;   // key blocks are contracted two at a time (one 16x16x32 instruction)
-    constexpr int NU = (R::SHARED_BYTES + 1023) / 1024;   // units of 1 KiB (16 bytes per lane) of the shared run
-    constexpr int UPW = (NU + 3) / 4;                     // units per wavefront in a full block (more in a partial one)
-    constexpr int SLOT = NU * 1024, SLOTS = 3, DG = 3;    // ring; chunks a fetch runs ahead of its hand-over
+    constexpr int C = 16 * NB, NP = (NB + 1) / 2, LW = scan_helpers(W) / 2;   // LW wavefronts load, as many store; key blocks are contracted two at a time (one 16x16x32 instruction)
+    constexpr int NU = (R::SHARED_BYTES + 1023) / 1024;   // units of 1 KiB (16 bytes per lane) of the shared run; then one per working wavefront
+    constexpr int UPW = (NU + W + LW - 1) / LW;           // units per loading wavefront
+    constexpr int SLOT = (NU + W) * 1024, SLOTS = 3, DG = 3;    // ring; chunks a fetch runs ahead of its hand-over
+    // results of a chunk: the NB state fragments and U^T of every working wavefront in the order of Kept, y by tokens, centres
+    constexpr int KEPT_BYTES = KEEP ? (NB + 1) * W * 512 : 0, Y_BYTES = FWD ? W * 512 : 0, OUT = KEPT_BYTES + Y_BYTES + (FWD ? 64 * W : 0);
     __shared__ __attribute__((aligned(16))) unsigned char ring[SLOTS * SLOT];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ib = wave < rows ? rows * blockIdx.y + wave : NB;   // (rows: value blocks, one per wavefront, of this block)
+    __shared__ __attribute__((aligned(16))) unsigned char results[2 * OUT];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ib0 = W * blockIdx.y, ib = ib0 + wave;
     const int bh = blockIdx.x, NC = T / CHUNK;
     const Lane L;
 
@@ -292,25 +299,72 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
         const int j = i < NC ? i : NC - 1;
         return (long)bh * NC + (FWD ? j : NC - 1 - j);
     };
-    // this wavefront's units of the shared run: wave, wave + 4, ... (indices past the end repeat the last unit: the
-    // same bytes to the same place).  Every block has four wavefronts for this; those without a value block of
-    // their own (NB no multiple of four) only keep the ring filled.
-    struct Stage {
-        f32x4 u[UPW];
-    };
-    auto unit = [&](int k) { const int u = wave + 4 * k; return u < NU ? u : NU - 1; };
-    auto issue = [&](Stage& st, int step) {
-        const char* base = reinterpret_cast<const char*>(rec + chunk_of(step) * R::ELEMS);
+    if (wave >= W) {
+        const int hw = wave - W, ht = threadIdx.x - 64 * (W + LW);
+        // a loading wavefront's units: hw, hw + LW, ... (indices past the end repeat the last unit: the same bytes to the same place)
+        struct Stage {
+            f32x4 u[UPW];
+        };
+        auto unit = [&](int k) { const int u = hw + LW * k; return u < NU + W ? u : NU + W - 1; };
+        auto issue = [&](Stage& st, int step) {
+            const long cid = chunk_of(step);
+            const char* const shared = reinterpret_cast<const char*>(rec + cid * R::ELEMS);
 #pragma unroll
-        for (int k = 0; k < UPW; k++) st.u[k] = *reinterpret_cast<const f32x4*>(base + unit(k) * 1024 + lane * 16);
-    };
-    auto to_ring = [&](int step, const Stage& st) {
-        unsigned char* slot = ring + (step % SLOTS) * SLOT;
+            for (int k = 0; k < UPW; k++) {
+                const int u = unit(k), own = ib0 + u - NU;   // (a value block past the last: the last one's, not used)
+                const char* const from = u < NU ? shared + u * 1024 : reinterpret_cast<const char*>(rec + R::i(cid, own < NB ? own : NB - 1));
+                st.u[k] = *reinterpret_cast<const f32x4*>(from + lane * 16);
+            }
+        };
+        auto to_ring = [&](int step, const Stage& st) {
+            unsigned char* slot = ring + (step % SLOTS) * SLOT;
 #pragma unroll
-        for (int k = 0; k < UPW; k++) *reinterpret_cast<f32x4*>(slot + unit(k) * 1024 + lane * 16) = st.u[k];
-    };
-    Stage st[DG];
-    if (ib >= NB) {   // ring duty only: the same hand-overs and barriers as the working wavefronts below
+            for (int k = 0; k < UPW; k++) *reinterpret_cast<f32x4*>(slot + unit(k) * 1024 + lane * 16) = st.u[k];
+        };
+        auto copy_out = [&](int step) {
+            const unsigned char* const from = results + (step & 1) * OUT;
+            const long cid = chunk_of(step);
+            const int blocks = NB - ib0 < W ? NB - ib0 : W;   // value blocks of this block
+            if constexpr (KEEP) {
+                constexpr int PIECES = (NB + 1) * W * 32;     // of 16 bytes
+#pragma unroll
+                for (int m = 0; m < (PIECES + 64 * LW - 1) / (64 * LW); m++) {
+                    const int e = ht + 64 * LW * m, jb = e / (W * 32), in = e % (W * 32);
+                    __bf16* const to = kept + (jb < NB ? K::ck(cid, jb, ib0) : K::ut(cid, ib0)) + in * 8;
+                    if (e < PIECES && in / 32 < blocks) *reinterpret_cast<f32x4*>(to) = *reinterpret_cast<const f32x4*>(from + e * 16);
+                }
+            }
+            if constexpr (FWD) {
+                const Addr<NB> ca((int)cid, T, H);
+#pragma unroll
+                for (int e = ht; e < 32 * W; e += 64 * LW) {
+                    const int token = e / (2 * W), piece = e % (2 * W);
+                    if (piece / 2 < blocks)
+                        *reinterpret_cast<f32x4*>(y_ + ca.row0 + (long)token * ca.ld + 16 * ib0 + 8 * piece) =
+                            *reinterpret_cast<const f32x4*>(from + KEPT_BYTES + e * 16);
+                }
+                if (centers != nullptr && ht < 16 * W) {
+                    const int token = ht / W, blk = ht % W;
+                    const int bb = ca.bh / H, hh = ca.bh - bb * H;
+                    if (blk < blocks)
+                        centers[(((long)bb * T + (long)ca.c * CHUNK + token) * H + hh) * NB + ib0 + blk] =
+                            *reinterpret_cast<const float*>(from + KEPT_BYTES + Y_BYTES + ht * 4);
+                }
+            }
+        };
+        if (hw >= LW) {   // round i: chunk i - 1's results out
+            lds_barrier();
+            for (int i = 0; i < NC; i++) {
+                if (i > 0) copy_out(i - 1);
+                lds_barrier();
+            }
+            copy_out(NC - 1);
+            return;
+        }
+        // chunks 0 and 1 into the ring, chunks 2 .. 4 in flight; then round i: chunk i + 2 into the ring (fetched three rounds
+        // ago) and chunk i + 5 requested.  The set of registers of a round is a constant (the rounds go by threes): an index
+        // known only at run time would put them in memory.
+        Stage st[DG];
 #pragma unroll
         for (int d = 0; d < DG; d++) issue(st[d], d);
         to_ring(0, st[0]);
@@ -318,22 +372,20 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
         issue(st[0], DG);
         issue(st[1], DG + 1);
         lds_barrier();
-        int i = 0;
-        for (; i + DG <= NC; i += DG) {
+        for (int i = 0; i < NC; i += DG) {
 #pragma unroll
             for (int d = 0; d < DG; d++) {
-                to_ring(i + d + 2, st[(d + 2) % DG]);
-                issue(st[(d + 2) % DG], i + d + 2 + DG);
-                lds_barrier();
+                if (i + d < NC) {
+                    to_ring(i + d + 2, st[(d + 2) % DG]);
+                    issue(st[(d + 2) % DG], i + d + 2 + DG);
+                    lds_barrier();
+                }
             }
         }
-#pragma unroll
-        for (int d = 0; d < DG - 1; d++) {
-            if (i + d < NC) {
-                to_ring(i + d + 2, st[(d + 2) % DG]);
-                lds_barrier();
-            }
-        }
+        return;
+    }
+    if (ib >= NB) {   // no value block of its own: only the barriers
+        for (int i = 0; i <= NC; i++) lds_barrier();
         return;
     }
 
@@ -359,17 +411,17 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
         }
         if constexpr (FWD) o.q = *reinterpret_cast<const bf16x8*>(slot + R::Q * 2 + lane * 16);
     };
-    auto load_private = [&](int step) { return load_pair(rec + R::i(chunk_of(step), ib), lane); };
     auto lo = [](bf16x8 p) { return __builtin_shufflevector(p, p, 0, 1, 2, 3); };
     auto hi = [](bf16x8 p) { return __builtin_shufflevector(p, p, 4, 5, 6, 7); };
 
     auto step = [&](const ScanOps<NB, FWD>& o, bf16x8 iv, int i) {
-        const long cid = chunk_of(i);
+        unsigned char* const out = results + (i & 1) * OUT;
+        auto keep = [&](int row, bf16x4 x) { *reinterpret_cast<bf16x4*>(out + (row * W + wave) * 512 + lane * 8) = x; };
         bf16x4 Sb[2 * NP];
 #pragma unroll
         for (int jb = 0; jb < NB; jb++) {
             Sb[jb] = to_bf16(S[jb]);
-            if constexpr (KEEP) store_frag(kept + K::ck(cid, jb, ib), lane, Sb[jb]);
+            if constexpr (KEEP) keep(jb, Sb[jb]);
         }
         if constexpr (NB & 1) Sb[NB] = zero_bf16();
         // F(U_ib^T) = F(U0_ib^T + S_ib Wm^T), two partial sums (the products are one dependent chain otherwise)
@@ -388,7 +440,7 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
             else UT = mma8(UT, join(m0, m1), join(Sb[2 * p], Sb[2 * p + 1]));
         }
         const bf16x4 UTb = to_bf16(UT + UT1);
-        if constexpr (KEEP) store_frag(kept + K::ut(cid, ib), lane, UTb);
+        if constexpr (KEEP) keep(NB, UTb);
         const bf16x8 VU = join(hi(iv), UTb);      // (V^T, U^T) forward, (dY^T, D^T) backward
         if constexpr (FWD) {
             f32x4 Y = mma8(zero4(), VU, o.q);     // F(QK V_ib + QB U_ib): lane = token, reg = value ch
@@ -397,60 +449,27 @@ __global__ __launch_bounds__(256) void scan_kernel(int T, int H, int state_f32, 
                 const bf16x4 w1 = 2 * p + 1 < NB ? hi(o.mw[2 * p + 1 < NB ? 2 * p + 1 : 0]) : zero_bf16();
                 Y = mma8(Y, join(Sb[2 * p], Sb[2 * p + 1]), join(hi(o.mw[2 * p]), w1));
             }
-            const Addr<NB> ca((int)cid, T, H);
             // centers != nullptr (the output is attn_ln's kept one): written centred per token and block of 16 channels,
             // the centres [token][head][block] beside it, so that its bf16 rounding is relative to the spread GroupNorm
             // divides by and not to the mean
             if (centers != nullptr) {
                 const float cen = row_sum16_bf16(Y) * (1.f / 16);
                 Y = Y - cen;
-                const int bb = ca.bh / H, hh = ca.bh - bb * H;
-                centers[(((long)bb * T + (long)ca.c * CHUNK + L.n) * H + hh) * NB + ib] = cen;   // (the four lanes of a token write the same value)
+                *reinterpret_cast<float*>(out + KEPT_BYTES + Y_BYTES + (L.n * W + wave) * 4) = cen;   // (the four lanes of a token write the same value)
             }
-            store_frag_rows(y_ + ca.row0, ca.ld, ib, L, to_bf16(Y));
+            *reinterpret_cast<bf16x4*>(out + KEPT_BYTES + (L.n * W + wave) * 32 + L.g * 8) = to_bf16(Y);
         }
 #pragma unroll
         for (int jb = 0; jb < NB; jb++) S[jb] = mma8(S[jb] * o.fw[jb], o.xz[jb], VU);
     };
 
-    // prologue: chunks 0 and 1 into the ring, chunks 2 .. 4 in flight; this wavefront's own pairs three chunks ahead
-    bf16x8 pv[DG];
-#pragma unroll
-    for (int d = 0; d < DG; d++) {
-        issue(st[d], d);
-        pv[d] = load_private(d);
-    }
-    to_ring(0, st[0]);
-    to_ring(1, st[1]);
-    issue(st[0], DG);
-    issue(st[1], DG + 1);
     lds_barrier();
-    // round i: chunk i's operands out of the ring, chunk i + 2 into it (fetched three rounds ago), chunk i + 5
-    // requested; then the chunk's arithmetic.  The loop body is one basic block (loads are otherwise sunk into
-    // the block of their use); the last NC % 3 rounds find everything they need in flight already.
-    ScanOps<NB, FWD> o;
-    int i = 0;
-    for (; i + DG <= NC; i += DG) {
-#pragma unroll
-        for (int d = 0; d < DG; d++) {
-            read_ring(o, i + d);
-            to_ring(i + d + 2, st[(d + 2) % DG]);
-            issue(st[(d + 2) % DG], i + d + 2 + DG);
-            const bf16x8 iv = pv[d];
-            pv[d] = load_private(i + d + DG);
-            __builtin_amdgcn_sched_barrier(0);
-            step(o, iv, i + d);
-            lds_barrier();
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < DG - 1; d++) {
-        if (i + d < NC) {
-            read_ring(o, i + d);
-            to_ring(i + d + 2, st[(d + 2) % DG]);
-            step(o, pv[d], i + d);
-            lds_barrier();
-        }
+    for (int i = 0; i < NC; i++) {
+        ScanOps<NB, FWD> o;
+        read_ring(o, i);
+        const bf16x8 iv = *reinterpret_cast<const bf16x8*>(ring + (i % SLOTS) * SLOT + (NU + wave) * 1024 + lane * 16);
+        step(o, iv, i);
+        lds_barrier();
     }
     if (s_out != nullptr) {
 #pragma unroll
@@ -721,16 +740,29 @@ inline int scan_rows(int BH, int NB) {
     return 4;
 }
 
+template <int NB, bool FWD, bool KEEP>
+void scan(int B, int T, int H, int state_f32, const __bf16* rec, const void* s_in, void* s_out, __bf16* y, __bf16* kept, float* centers,
+          hipStream_t stream) {
+    auto launch = [&](auto width) {
+        constexpr int W = decltype(width)::value;
+        hipLaunchKernelGGL((scan_kernel<NB, FWD, KEEP, W>), dim3(B * H, (NB + W - 1) / W), dim3(64 * (W + scan_helpers(W))), 0, stream, T, H,
+                           state_f32, rec, s_in, s_out, y, kept, centers);
+    };
+    switch (scan_rows(B * H, NB)) {
+        case 1: launch(std::integral_constant<int, 1>()); break;
+        case 2: launch(std::integral_constant<int, 2>()); break;
+        default: launch(std::integral_constant<int, 4>());
+    }
+}
+
 template <int NB>
 void forward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v, const void* a,
              const void* b, const void* s_in, void* s_out, void* y, void* rec, void* kept, float* centers, hipStream_t stream) {
     const int nchunks = B * H * (T / CHUNK);
     hipLaunchKernelGGL(fwd_prepare_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q),
                        c(k), c(v), c(a), c(b), m(rec));
-    const int rows = scan_rows(B * H, NB);
-    const dim3 grid(B * H, (NB + rows - 1) / rows), block(256);
-    if (kept) hipLaunchKernelGGL((scan_kernel<NB, true, true>), grid, block, 0, stream, T, H, state_f32, rows, c(rec), s_in, s_out, m(y), m(kept), centers);
-    else hipLaunchKernelGGL((scan_kernel<NB, true, false>), grid, block, 0, stream, T, H, state_f32, rows, c(rec), s_in, s_out, m(y), m(kept), centers);
+    if (kept) scan<NB, true, true>(B, T, H, state_f32, c(rec), s_in, s_out, m(y), m(kept), centers, stream);
+    else scan<NB, true, false>(B, T, H, state_f32, c(rec), s_in, s_out, m(y), m(kept), centers, stream);
 }
 template <int NB>
 void backward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v, const void* a,
@@ -739,9 +771,7 @@ void backward(int B, int T, int H, int state_f32, const void* w, const void* q, 
     const int nchunks = B * H * (T / CHUNK);
     hipLaunchKernelGGL(bwd_prepare_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q),
                        c(a), c(b), c(dy), m(rec));
-    const int rows = scan_rows(B * H, NB);
-    hipLaunchKernelGGL((scan_kernel<NB, false, true>), dim3(B * H, (NB + rows - 1) / rows), dim3(256), 0, stream, T, H,
-                       state_f32, rows, c(rec), ds_in, ds_out, static_cast<__bf16*>(nullptr), m(kept_b), static_cast<float*>(nullptr));
+    scan<NB, false, true>(B, T, H, state_f32, c(rec), ds_in, ds_out, nullptr, m(kept_b), nullptr, stream);
     hipLaunchKernelGGL(grads_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k),
                        c(v), c(a), c(b), c(dy), c(kept_f), c(kept_b), m(dw), m(dq), m(dk), m(dv), m(da), m(db));
 }
