@@ -59,12 +59,44 @@ __device__ __forceinline__ bf16x4 load_frag_rows(const __bf16* __restrict__ p, l
 __device__ __forceinline__ void store_frag_rows(__bf16* __restrict__ p, long ld, int jb, const Lane& L, bf16x4 x) {
     *reinterpret_cast<bf16x4*>(p + (long)L.n * ld + 16 * jb + 4 * L.g) = x;
 }
+// Tiles come from memory 16 bytes per lane, two fragments at a time: a lane of group g holds eight channels of block
+// 2p + g % 2 (its lower half for g < 2), 64 bytes of a token's row per access instead of 32; swapping neighbouring groups
+// makes fragments 2p and 2p + 1 of it.  (An odd last fragment is read as it lies.)  Reading and swapping are apart so that a
+// kernel can request everything before it waits for anything.
 template <int NB>
-__device__ __forceinline__ TB<NB> load_tile(const __bf16* __restrict__ p, long ld, const Lane& L) {
-    TB<NB> t;
+struct RawTile {
+    bf16x8 pair[NB / 2 > 0 ? NB / 2 : 1];
+    bf16x4 last;
+};
+template <int NB>
+__device__ __forceinline__ RawTile<NB> load_tile(const __bf16* __restrict__ p, long ld, const Lane& L) {
+    RawTile<NB> t;
 #pragma unroll
-    for (int i = 0; i < NB; i++) t.f[i] = load_frag_rows(p, ld, i, L);
+    for (int i = 0; i < NB / 2; i++)
+        t.pair[i] = *reinterpret_cast<const bf16x8*>(p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1));
+    if constexpr (NB & 1) t.last = load_frag_rows(p, ld, NB - 1, L);
     return t;
+}
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void swap_groups(u32x4 x, bf16x4& even, bf16x4& odd) {
+    const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], x[2], false, false), s1 = __builtin_amdgcn_permlane16_swap(x[1], x[3], false, false);
+    even = __builtin_bit_cast(bf16x4, u32x2{s0[0], s1[0]});
+    odd = __builtin_bit_cast(bf16x4, u32x2{s0[1], s1[1]});
+}
+template <int NB>
+__device__ __forceinline__ TB<NB> fragments(const RawTile<NB>& t) {
+    TB<NB> r;
+#pragma unroll
+    for (int i = 0; i < NB / 2; i++) swap_groups(__builtin_bit_cast(u32x4, t.pair[i]), r.f[2 * i], r.f[2 * i + 1]);
+    if constexpr (NB & 1) r.f[NB - 1] = t.last;
+    return r;
+}
+
+// fragments 2i and 2i + 1 to memory, 16 bytes per lane: the same swap is its own inverse
+__device__ __forceinline__ void store_pair_rows(__bf16* __restrict__ p, long ld, int i, const Lane& L, bf16x4 even, bf16x4 odd) {
+    const u32x2 x = __builtin_bit_cast(u32x2, even), y = __builtin_bit_cast(u32x2, odd);
+    const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false), s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+    *reinterpret_cast<u32x4*>(p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1)) = u32x4{s0[0], s1[0], s0[1], s1[1]};
 }
 
 // F(X Y^T), contraction over the C channels
@@ -170,10 +202,11 @@ __global__ __launch_bounds__(256) void fwd_prepare_kernel(int T, int H, int nchu
 
     // all of the chunk's rows are requested before any is used (the compiler would place each load next to its
     // use and wait for it there)
-    const TB<NB> w = load_tile<NB>(w_ + ca.row0, ca.ld, L), q = load_tile<NB>(q_ + ca.row0, ca.ld, L);
-    const TB<NB> k = load_tile<NB>(k_ + ca.row0, ca.ld, L), a = load_tile<NB>(a_ + ca.row0, ca.ld, L);
-    const TB<NB> b = load_tile<NB>(b_ + ca.row0, ca.ld, L), v = load_tile<NB>(v_ + ca.row0, ca.ld, L);
+    const RawTile<NB> w_raw = load_tile<NB>(w_ + ca.row0, ca.ld, L), q_raw = load_tile<NB>(q_ + ca.row0, ca.ld, L);
+    const RawTile<NB> k_raw = load_tile<NB>(k_ + ca.row0, ca.ld, L), a_raw = load_tile<NB>(a_ + ca.row0, ca.ld, L);
+    const RawTile<NB> b_raw = load_tile<NB>(b_ + ca.row0, ca.ld, L), v_raw = load_tile<NB>(v_ + ca.row0, ca.ld, L);
     __builtin_amdgcn_sched_barrier(0);
+    const TB<NB> w = fragments(w_raw), q = fragments(q_raw), k = fragments(k_raw), a = fragments(a_raw), b = fragments(b_raw), v = fragments(v_raw);
     TB<NB> wq, wa, kwi, bwi;
 #pragma unroll
     for (int jb = 0; jb < NB; jb++) {
@@ -222,10 +255,11 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(int T, int H, int nchu
     const Addr<NB> ca(cid, T, H);
     const bf16x4 eye = identity_bf16(L);
 
-    const TB<NB> w = load_tile<NB>(w_ + ca.row0, ca.ld, L), q = load_tile<NB>(q_ + ca.row0, ca.ld, L);
-    const TB<NB> a = load_tile<NB>(a_ + ca.row0, ca.ld, L), b = load_tile<NB>(b_ + ca.row0, ca.ld, L);
-    const TB<NB> dy = load_tile<NB>(dy_ + ca.row0, ca.ld, L);
+    const RawTile<NB> w_raw = load_tile<NB>(w_ + ca.row0, ca.ld, L), q_raw = load_tile<NB>(q_ + ca.row0, ca.ld, L);
+    const RawTile<NB> a_raw = load_tile<NB>(a_ + ca.row0, ca.ld, L), b_raw = load_tile<NB>(b_ + ca.row0, ca.ld, L);
+    const RawTile<NB> dy_raw = load_tile<NB>(dy_ + ca.row0, ca.ld, L);
     __builtin_amdgcn_sched_barrier(0);
+    const TB<NB> w = fragments(w_raw), q = fragments(q_raw), a = fragments(a_raw), b = fragments(b_raw), dy = fragments(dy_raw);
     TB<NB> wq, wa, bwi, bf;
 #pragma unroll
     for (int jb = 0; jb < NB; jb++) {
@@ -483,9 +517,14 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
 // ------------------------------------------------------------------------------------------------
 // gradients: one wavefront per chunk (the algebra of bwd_grads_kernel in wkv7_bwd.hip, with the state fragments
 // streamed one key block at a time instead of held: at C = 128 both states of a chunk are 128 fragments).
+// Two wavefronts per SIMD, so that one loads while the other multiplies: what every key block reads again (v, dY, U, D) lies
+// in LDS, decay factors are made twice, and the next key block's states are loaded into the registers just used; that is 248
+// of 256 registers at C = 128 (all of it held: 484 and one wavefront).  With 16-byte accesses to the sequences' rows (the
+// outputs of an even key block wait in LDS for the odd one's): 110 -> 90 us at 8 x 1024 tokens x 6 heads of 128, where its 390
+// MB take 73 us at a copy's rate.
 // ------------------------------------------------------------------------------------------------
 template <int NB>
-__global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, const __bf16* __restrict__ w_,
+__global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks, const __bf16* __restrict__ w_,
                                                     const __bf16* __restrict__ q_, const __bf16* __restrict__ k_,
                                                     const __bf16* __restrict__ v_, const __bf16* __restrict__ a_,
                                                     const __bf16* __restrict__ b_, const __bf16* __restrict__ dy_,
@@ -500,17 +539,22 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
     const Lane L;
     const Addr<NB> ca(cid, T, H);
     const bf16x4 eye = identity_bf16(L);
+    // value-side fragments that every key block reads again: each lane's own 8 bytes, so no barrier
+    enum { VS_V = 0, VS_DY, VS_U, VS_D, VS_TILES };
+    __shared__ bf16x4 vals[4][VS_TILES][NB][WAVE];
+    __shared__ bf16x4 waiting[4][5][WAVE];
+    bf16x4(&mine)[VS_TILES][NB][WAVE] = vals[threadIdx.x >> 6];
 
     // Everything the chunk needs up front is requested before any of it is used (left to itself the compiler
     // places each load next to its use and waits for it there: one memory latency per fragment).
-    const TB<NB> w = load_tile<NB>(w_ + ca.row0, ca.ld, L);
-    const TB<NB> q = load_tile<NB>(q_ + ca.row0, ca.ld, L);
-    const TB<NB> k = load_tile<NB>(k_ + ca.row0, ca.ld, L);
-    const TB<NB> a = load_tile<NB>(a_ + ca.row0, ca.ld, L);
-    const TB<NB> b = load_tile<NB>(b_ + ca.row0, ca.ld, L);
-    const TB<NB> v = load_tile<NB>(v_ + ca.row0, ca.ld, L);
-    const TB<NB> dy = load_tile<NB>(dy_ + ca.row0, ca.ld, L);
-    TB<NB> UT, DT, Ur, Dr, dYT;
+    const RawTile<NB> w_raw = load_tile<NB>(w_ + ca.row0, ca.ld, L);
+    const RawTile<NB> q_raw = load_tile<NB>(q_ + ca.row0, ca.ld, L);
+    const RawTile<NB> k_raw = load_tile<NB>(k_ + ca.row0, ca.ld, L);
+    const RawTile<NB> a_raw = load_tile<NB>(a_ + ca.row0, ca.ld, L);
+    const RawTile<NB> b_raw = load_tile<NB>(b_ + ca.row0, ca.ld, L);
+    const RawTile<NB> v_raw = load_tile<NB>(v_ + ca.row0, ca.ld, L);
+    const RawTile<NB> dy_raw = load_tile<NB>(dy_ + ca.row0, ca.ld, L);
+    TB<NB> UT, DT;
 #pragma unroll
     for (int ib = 0; ib < NB; ib++) {
         UT.f[ib] = load_frag(kept_f + K::ut(cid, ib), lane);   // F(U_ib^T)   lane = value ch
@@ -524,6 +568,7 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
         dsn[ib] = load_frag(kept_b + K::ck(cid, 0, ib), lane);
     }
     __builtin_amdgcn_sched_barrier(0);
+    const TB<NB> w = fragments(w_raw), q = fragments(q_raw), k = fragments(k_raw), a = fragments(a_raw), b = fragments(b_raw), v = fragments(v_raw), dy = fragments(dy_raw);
 
     // key side: the decayed operands of all key blocks (needed whole for the 16x16 products)
     TB<NB> wq, wa, kwi, bwi, kf;
@@ -537,22 +582,26 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
         bwi.f[jb] = to_bf16(to_f32(b.f[jb]) * d.Pi);
         kf.f[jb] = to_bf16(kwi_f * d.fw);
     }
-    // value side
+    // value side: the 16x16 products over the value channels, each in both orientations
+    f32x4 p_ab = zero4(), p_abT = zero4(), p_ak = zero4(), p_akT = zero4(), p_qb = zero4(), p_qbT = zero4(), p_qk = zero4(), p_qkT = zero4();
 #pragma unroll
     for (int ib = 0; ib < NB; ib++) {
-        Ur.f[ib] = transpose(UT.f[ib], eye);                   // F(U_ib)     lane = token
-        Dr.f[ib] = transpose(DT.f[ib], eye);
-        dYT.f[ib] = transpose(dy.f[ib], eye);
+        const bf16x4 Ur = transpose(UT.f[ib], eye), Dr = transpose(DT.f[ib], eye);   // F(U_ib), F(D_ib): lane = token
+        p_ab = mma(p_ab, Ur, Dr), p_abT = mma(p_abT, Dr, Ur);
+        p_ak = mma(p_ak, v.f[ib], Dr), p_akT = mma(p_akT, Dr, v.f[ib]);
+        p_qb = mma(p_qb, Ur, dy.f[ib]), p_qbT = mma(p_qbT, dy.f[ib], Ur);
+        p_qk = mma(p_qk, v.f[ib], dy.f[ib]), p_qkT = mma(p_qkT, dy.f[ib], v.f[ib]);
+        mine[VS_V][ib][lane] = v.f[ib], mine[VS_DY][ib][lane] = dy.f[ib];
+        mine[VS_U][ib][lane] = Ur, mine[VS_D][ib][lane] = Dr;
     }
-    // 16x16 products over the value channels, each in both orientations
-    const bf16x4 dab = to_bf16(mask_lower_strict(xyT(Dr, Ur), L));   // [t][s] = D_t . U_s,  s < t
-    const bf16x4 dabT = to_bf16(mask_upper_strict(xyT(Ur, Dr), L));
-    const bf16x4 dak = to_bf16(mask_lower_strict(xyT(Dr, v), L));    // [t][s] = D_t . v_s
-    const bf16x4 dakT = to_bf16(mask_upper_strict(xyT(v, Dr), L));
-    const bf16x4 dqb = to_bf16(mask_lower_incl(xyT(dy, Ur), L));     // [t][s] = dY_t . U_s,  s <= t
-    const bf16x4 dqbT = to_bf16(mask_upper_incl(xyT(Ur, dy), L));
-    const bf16x4 dqk = to_bf16(mask_lower_incl(xyT(dy, v), L));      // [t][s] = dY_t . v_s
-    const bf16x4 dqkT = to_bf16(mask_upper_incl(xyT(v, dy), L));
+    const bf16x4 dab = to_bf16(mask_lower_strict(p_ab, L));      // [t][s] = D_t . U_s,  s < t
+    const bf16x4 dabT = to_bf16(mask_upper_strict(p_abT, L));
+    const bf16x4 dak = to_bf16(mask_lower_strict(p_ak, L));      // [t][s] = D_t . v_s
+    const bf16x4 dakT = to_bf16(mask_upper_strict(p_akT, L));
+    const bf16x4 dqb = to_bf16(mask_lower_incl(p_qb, L));        // [t][s] = dY_t . U_s,  s <= t
+    const bf16x4 dqbT = to_bf16(mask_upper_incl(p_qbT, L));
+    const bf16x4 dqk = to_bf16(mask_lower_incl(p_qk, L));        // [t][s] = dY_t . v_s
+    const bf16x4 dqkT = to_bf16(mask_upper_incl(p_qkT, L));
     // over the key channels (rows = the token being written)
     const bf16x4 QKT = to_bf16(mask_upper_incl(xyT(kwi, wq), L));    // [t][s] = kwi_t . wq_s, s >= t
     const bf16x4 AKT = to_bf16(mask_upper_strict(xyT(kwi, wa), L));  // [t][s] = kwi_t . wa_s, s >  t
@@ -560,23 +609,13 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
     // dv = QK^T dY + AK^T D + kf dS^T: the last term is gathered key block by key block below
     f32x4 dv[NB];
 #pragma unroll
-    for (int ib = 0; ib < NB; ib++) dv[ib] = mma(mma(zero4(), dYT.f[ib], QKT), DT.f[ib], AKT);
+    for (int ib = 0; ib < NB; ib++) dv[ib] = mma(mma(zero4(), transpose(dy.f[ib], eye), QKT), DT.f[ib], AKT);
 
 #pragma unroll
     for (int jb = 0; jb < NB; jb++) {
-        bf16x4 s0c[NB], dsc[NB];   // F(S0[16 ib.., 16 jb..]), F(dS[16 ib.., 16 jb..]): lane = value row
-#pragma unroll
-        for (int ib = 0; ib < NB; ib++) {
-            s0c[ib] = s0n[ib];
-            dsc[ib] = dsn[ib];
-        }
-        if (jb + 1 < NB) {
-#pragma unroll
-            for (int ib = 0; ib < NB; ib++) {
-                s0n[ib] = load_frag(kept_f + K::ck(cid, jb + 1, ib), lane);
-                dsn[ib] = load_frag(kept_b + K::ck(cid, jb + 1, ib), lane);
-            }
-        }
+        asm volatile("" ::: "memory");   // (else the compiler keeps the value-side fragments in registers across key blocks)
+        // (read again: kept from above, the compiler keeps the 20 factors per key block computed there too)
+        const bf16x4 w_again = load_frag_rows(w_ + ca.row0, ca.ld, jb, L);
         __builtin_amdgcn_sched_barrier(0);
         f32x4 sds = zero4();                       // sum over the value rows of S0 * dS, this key block
         f32x4 Bq = mma(mma(zero4(), transpose(bwi.f[jb], eye), dqb), transpose(kwi.f[jb], eye), dqk);
@@ -586,16 +625,21 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
         f32x4 UdS = zero4(), VdS = zero4();
 #pragma unroll
         for (int ib = 0; ib < NB; ib++) {
-            const bf16x4 s0 = s0c[ib], ds = dsc[ib];
+            const bf16x4 s0 = s0n[ib], ds = dsn[ib];   // F(S0[16 ib.., 16 jb..]), F(dS[16 ib.., 16 jb..]): lane = value row
             sds += to_f32(s0) * to_f32(ds);
             const bf16x4 s0T = transpose(s0, eye), dsT = transpose(ds, eye);  // lane = key column, reg = value row
             dv[ib] = mma(dv[ib], ds, kf.f[jb]);
-            Bq = mma(Bq, s0T, dy.f[ib]);          // + dY S0
-            Ba = mma(Ba, s0T, Dr.f[ib]);          // + D S0
-            UdS = mma(UdS, dsT, Ur.f[ib]);        // U dS
-            VdS = mma(VdS, dsT, v.f[ib]);         // V dS
+            Bq = mma(Bq, s0T, mine[VS_DY][ib][lane]);    // + dY S0
+            Ba = mma(Ba, s0T, mine[VS_D][ib][lane]);     // + D S0
+            UdS = mma(UdS, dsT, mine[VS_U][ib][lane]);   // U dS
+            VdS = mma(VdS, dsT, mine[VS_V][ib][lane]);   // V dS
+            if (jb + 1 < NB) {   // into the same registers: the next key block's, a whole key block ahead of their use
+                s0n[ib] = load_frag(kept_f + K::ck(cid, jb + 1, ib), lane);
+                dsn[ib] = load_frag(kept_b + K::ck(cid, jb + 1, ib), lane);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        const DecayF d = decay_frag(w.f[jb]);
+        const DecayF d = decay_frag(w_again);
         const f32x4 wqf = to_f32(wq.f[jb]), waf = to_f32(wa.f[jb]), kwif = to_f32(kwi.f[jb]), bwif = to_f32(bwi.f[jb]);
         f32x4 dq, da, dk, db, dw;
 #pragma unroll
@@ -614,14 +658,19 @@ __global__ __launch_bounds__(256) void grads_kernel(int T, int H, int nchunks, c
             const float dlogw = row_suffix_sum(g_incl + g_strict) - g_strict + tail;
             dw[r] = dlogw * d.lw[r];
         }
-        store_frag_rows(dq_ + ca.row0, ca.ld, jb, L, to_bf16(dq));
-        store_frag_rows(da_ + ca.row0, ca.ld, jb, L, to_bf16(da));
-        store_frag_rows(dk_ + ca.row0, ca.ld, jb, L, to_bf16(dk));
-        store_frag_rows(db_ + ca.row0, ca.ld, jb, L, to_bf16(db));
-        store_frag_rows(dw_ + ca.row0, ca.ld, jb, L, to_bf16(dw));
+        // an even block's gradients wait in LDS for the odd one's
+        const bf16x4 grads[5] = {to_bf16(dq), to_bf16(da), to_bf16(dk), to_bf16(db), to_bf16(dw)};
+        __bf16* const dst[5] = {dq_, da_, dk_, db_, dw_};
+#pragma unroll
+        for (int x = 0; x < 5; x++) {
+            if (jb & 1) store_pair_rows(dst[x] + ca.row0, ca.ld, jb / 2, L, waiting[threadIdx.x >> 6][x][lane], grads[x]);
+            else if (jb + 1 < NB) waiting[threadIdx.x >> 6][x][lane] = grads[x];
+            else store_frag_rows(dst[x] + ca.row0, ca.ld, jb, L, grads[x]);
+        }
     }
 #pragma unroll
-    for (int ib = 0; ib < NB; ib++) store_frag_rows(dv_ + ca.row0, ca.ld, ib, L, to_bf16(dv[ib]));
+    for (int i = 0; i < NB / 2; i++) store_pair_rows(dv_ + ca.row0, ca.ld, i, L, to_bf16(dv[2 * i]), to_bf16(dv[2 * i + 1]));
+    if constexpr (NB & 1) store_frag_rows(dv_ + ca.row0, ca.ld, NB - 1, L, to_bf16(dv[NB - 1]));
 }
 
 // ------------------------------------------------------------------------------------------------
