@@ -163,10 +163,6 @@ struct Rec {
 __device__ __forceinline__ void store_pair(__bf16* __restrict__ p, int lane, bf16x4 u, bf16x4 v) {
     *reinterpret_cast<bf16x8*>(p + 8 * lane) = __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-// one half of a pair: which = 0 first fragment, 1 second
-__device__ __forceinline__ void store_half(__bf16* __restrict__ p, int lane, int which, bf16x4 u) {
-    *reinterpret_cast<bf16x4*>(p + 8 * lane + 4 * which) = u;
-}
 __device__ __forceinline__ bf16x8 load_pair(const __bf16* __restrict__ p, int lane) {
     return *reinterpret_cast<const bf16x8*>(p + 8 * lane);
 }
@@ -218,7 +214,6 @@ __global__ __launch_bounds__(256) void fwd_prepare_kernel(int T, int H, int nchu
         kwi.f[jb] = to_bf16(kwi_f);
         bwi.f[jb] = to_bf16(bwi_f);
         store_pair(rec + R::xz(cid, jb), lane, transpose(to_bf16(kwi_f * d.fw), eye), transpose(to_bf16(bwi_f * d.fw), eye));
-        store_half(rec + R::mw(cid, jb), lane, 1, wq.f[jb]);
         if (L.n == 0) *reinterpret_cast<f32x4*>(R::fw(rec, cid) + 16 * jb + 4 * L.g) = d.fw;
     }
     const f32x4 AB = mask_lower_strict(xyT(wa, bwi), L);     // [t][s] = wa_t . bwi_s, s < t
@@ -235,8 +230,8 @@ __global__ __launch_bounds__(256) void fwd_prepare_kernel(int T, int H, int nchu
         store_pair(rec + R::i(cid, ib), lane, to_bf16(mma(zero4(), Tinv_b, to_bf16(RT))), VT);
     }
 #pragma unroll
-    for (int jb = 0; jb < NB; jb++)   // F(Tinv wa_jb): lane = token, reg = key ch
-        store_half(rec + R::mw(cid, jb), lane, 0, to_bf16(mma(zero4(), transpose(wa.f[jb], eye), Tinv_b)));
+    for (int jb = 0; jb < NB; jb++)   // (F(Tinv wa_jb), wq): lane = token, reg = key ch
+        store_pair(rec + R::mw(cid, jb), lane, to_bf16(mma(zero4(), transpose(wa.f[jb], eye), Tinv_b)), wq.f[jb]);
 }
 
 // ------------------------------------------------------------------------------------------------
