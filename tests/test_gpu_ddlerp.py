@@ -51,6 +51,14 @@ def test_ddlerp_parity(B, T, C):
     check(*run_both(B, T, C, 32, seed=300 + T + C))
 
 
+# the kernel for few tokens up to 256 tiles of 16 (two per block, the last count odd) and the one after it; 5, 12 and 13
+# channel blocks over its four wavefronts
+@pytest.mark.parametrize('D', [32, 64])
+@pytest.mark.parametrize('B,T,C', [(1, 4096, 320), (1, 4112, 768), (5, 816, 832)])
+def test_ddlerp_around_the_few_token_limit(B, T, C, D):
+    check(*run_both(B, T, C, D, seed=500 + T + D))
+
+
 # rank 64 (two 32-wide contractions per interpolation; the second backward pass keeps its weight fragments in
 # registers): a single tile, a ragged count of tiles, the two- and four-tiles-per-block kernels, 64 channel blocks
 @pytest.mark.parametrize('B,T,C', [(1, 16, 64), (2, 48, 128), (3, 64, 768), (8, 1024, 768), (17, 976, 256), (2, 4112, 128),

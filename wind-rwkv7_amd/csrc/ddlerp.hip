@@ -103,6 +103,134 @@ __device__ __forceinline__ void load_r_fragments(bf16x4 (&raw)[NB / 4][NBLK], co
     }
 }
 
+// a = x + xx*alpha as a bf16 pair (hi + lo): the pre-activation feeds tanh', which is steep, so the interpolated input must
+// not be rounded to 8 bits before the 768-term sum (L itself is bf16)
+__device__ __forceinline__ void interpolate(const bf16x8 cur, const bf16x8 prev, const bf16x4 al0, const bf16x4 al1, bf16x8& hi, bf16x8& lo) {
+    f32x4 av[2];
+#pragma unroll
+    for (int hlf = 0; hlf < 2; hlf++) {
+        const f32x4 c = to_f32(hlf ? __builtin_shufflevector(cur, cur, 4, 5, 6, 7) : __builtin_shufflevector(cur, cur, 0, 1, 2, 3));
+        const f32x4 q = to_f32(hlf ? __builtin_shufflevector(prev, prev, 4, 5, 6, 7) : __builtin_shufflevector(prev, prev, 0, 1, 2, 3));
+        av[hlf] = c + (q - c) * to_f32(hlf ? al1 : al0);
+    }
+    const bf16x4 h0 = to_bf16(av[0]), h1 = to_bf16(av[1]);
+    hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+    lo = __builtin_shufflevector(to_bf16(av[0] - to_f32(h0)), to_bf16(av[1] - to_f32(h1)), 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// tanh and its derivative 1 - tanh^2 = 4e/(e+1)^2, e = exp(2s).  The derivative is stored on its own:
+// recovering it from a bf16-rounded tanh loses all precision where the unit saturates.
+__device__ __forceinline__ void store_activation(f32x4 s, __bf16* __restrict__ bmid, __bf16* __restrict__ bder, long off) {
+    f32x4 t, dt;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float e = __expf(2.f * fminf(s[r], 40.f));
+        const float inv = __builtin_amdgcn_rcpf(e + 1.f);   // 1 ulp; an IEEE division is ten instructions
+        t[r] = 1.f - 2.f * inv;
+        dt[r] = 4.f * e * inv * inv;
+    }
+    *reinterpret_cast<bf16x4*>(bmid + off) = to_bf16(t);
+    *reinterpret_cast<bf16x4*>(bder + off) = to_bf16(dt);
+}
+
+// forward 1 for few tokens: a block takes TPB tiles and one of SPLIT parts of the outputs, its four wavefronts a quarter of
+// the channel blocks each, every operand straight from memory; one sum over the wavefronts at the end.  What bounds a
+// launch of this size is what ONE compute unit can fetch (some 25 bytes per ns: 8 us for the whole of the weights), so the
+// weights are spread over the blocks.  The kernel below fetches all of them per block, a barrier per channel block.
+template <int D, int SPLIT, int TPB>
+__global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, int C, const __bf16* __restrict__ x,
+                                                                 const __bf16* __restrict__ x_prev,
+                                                                 const __bf16* __restrict__ alpha,
+                                                                 const __bf16* __restrict__ Lw, __bf16* __restrict__ bmid,
+                                                                 __bf16* __restrict__ bder) {
+    constexpr int NB = 4 * D / 16 / SPLIT, NA = NB * TPB;   // output blocks of 16; with the tiles: accumulators
+    __shared__ f32x4 part[4][NA][WAVE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const Lane L;
+    const long ntiles = M / TOK;
+    const int ncb = C / 64, db0 = NB * blockIdx.y;
+    long m0[TPB];
+    PrevRow before[TPB];
+#pragma unroll
+    for (int p = 0; p < TPB; p++) {
+        const long tile = (long)blockIdx.x * TPB + p;
+        m0[p] = (tile < ntiles ? tile : ntiles - 1) * TOK;   // (a spare tile is the last one again and stores nothing)
+        before[p] = prev_row(x, x_prev, m0[p] + L.n, T, C, 8 * L.g);
+    }
+    f32x4 acc[TPB][NB];
+#pragma unroll
+    for (int p = 0; p < TPB; p++)
+#pragma unroll
+        for (int i = 0; i < NB; i++) acc[p][i] = zero4();
+    struct Set {
+        bf16x8 wr[NB][2], xc[TPB][NBLK / 2], xp[TPB][NBLK / 2];
+        bf16x4 al[NBLK];
+    };
+    auto fetch = [&](Set& st, int cb) {
+        const int c0 = 64 * (cb < ncb ? cb : ncb - 1);   // (past the last block: it again, not used)
+#pragma unroll
+        for (int p = 0; p < TPB; p++) {
+            const __bf16 *row = x + (m0[p] + L.n) * C + c0 + 8 * L.g, *prow = before[p].row + c0;
+#pragma unroll
+            for (int pr = 0; pr < NBLK / 2; pr++) {
+                st.xc[p][pr] = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
+                st.xp[p][pr] = *reinterpret_cast<const bf16x8*>(prow + 32 * pr);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NBLK; i++) st.al[i] = *reinterpret_cast<const bf16x4*>(alpha + c0 + chan16(i, 4 * L.g));
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            const TileB t = load_rows16(Lw + (long)(16 * (db0 + i)) * C + c0, C, L);
+            st.wr[i][0] = __builtin_shufflevector(t.f[0], t.f[1], 0, 1, 2, 3, 4, 5, 6, 7);
+            st.wr[i][1] = __builtin_shufflevector(t.f[2], t.f[3], 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    auto use = [&](const Set& st) {
+        bf16x8 a[TPB][4];   // hi, hi, lo, lo
+#pragma unroll
+        for (int p = 0; p < TPB; p++)
+#pragma unroll
+            for (int pr = 0; pr < NBLK / 2; pr++) {
+                const bf16x8 zero = {};
+                interpolate(st.xc[p][pr], before[p].has_prev ? st.xp[p][pr] : zero, st.al[2 * pr], st.al[2 * pr + 1], a[p][pr], a[p][2 + pr]);
+            }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int p = 0; p < TPB; p++)
+#pragma unroll
+                for (int i = 0; i < NB; i++) acc[p][i] = mma8(acc[p][i], st.wr[i][k & 1], a[p][k]);
+    };
+    constexpr int SETS = 3;   // channel blocks in flight
+    Set st[SETS];
+#pragma unroll
+    for (int d = 0; d < SETS; d++) fetch(st[d], wave + 4 * d);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int cb = wave; cb < ncb; cb += 4 * SETS) {
+#pragma unroll
+        for (int d = 0; d < SETS; d++) {
+            if (cb + 4 * d < ncb) {
+                use(st[d]);
+                if (cb + 4 * (d + SETS) < ncb) fetch(st[d], cb + 4 * (d + SETS));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    // the sums over the wavefronts, each by one wavefront and in their order
+#pragma unroll
+    for (int p = 0; p < TPB; p++)
+#pragma unroll
+        for (int i = 0; i < NB; i++) part[wave][p * NB + i][lane] = acc[p][i];
+    __syncthreads();
+    for (int e = wave; e < NA; e += 4) {
+        const int p = e / NB, i = e % NB;
+        const long tile = (long)blockIdx.x * TPB + p;
+        if (tile >= ntiles) break;
+        const f32x4 s = (part[0][e][lane] + part[1][e][lane]) + (part[2][e][lane] + part[3][e][lane]);
+        store_activation(s, bmid, bder, (tile * TOK + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g);
+    }
+}
+
 // forward 1: bmid = tanh((x + xx*alpha) L^T), bder = 1 - bmid^2
 template <int D, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int C, const __bf16* __restrict__ x,
@@ -167,24 +295,11 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
             w.f[buf][wave * (NB / 4) + i][1][lane] = st.wr[i][1];
         }
         __syncthreads();
-        // a = x + xx*alpha as a bf16 pair (hi + lo): the pre-activation feeds tanh', which is steep, so the
-        // interpolated input must not be rounded to 8 bits before the 768-term sum (L itself is bf16)
         bf16x8 a[2], alo[2];
 #pragma unroll
         for (int pr = 0; pr < NBLK / 2; pr++) {
             const bf16x8 zero = {};
-            const bf16x8 prev = has_prev ? st.xp[pr] : zero;
-            f32x4 av[2];
-#pragma unroll
-            for (int hlf = 0; hlf < 2; hlf++) {
-                const f32x4 c = to_f32(hlf ? __builtin_shufflevector(st.xc[pr], st.xc[pr], 4, 5, 6, 7)
-                                           : __builtin_shufflevector(st.xc[pr], st.xc[pr], 0, 1, 2, 3));
-                const f32x4 q = to_f32(hlf ? __builtin_shufflevector(prev, prev, 4, 5, 6, 7) : __builtin_shufflevector(prev, prev, 0, 1, 2, 3));
-                av[hlf] = c + (q - c) * to_f32(st.al[2 * pr + hlf]);
-            }
-            const bf16x4 h0 = to_bf16(av[0]), h1 = to_bf16(av[1]);
-            a[pr] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-            alo[pr] = __builtin_shufflevector(to_bf16(av[0] - to_f32(h0)), to_bf16(av[1] - to_f32(h1)), 0, 1, 2, 3, 4, 5, 6, 7);
+            interpolate(st.xc[pr], has_prev ? st.xp[pr] : zero, st.al[2 * pr], st.al[2 * pr + 1], a[pr], alo[pr]);
         }
         fetch(st, next_cb);   // (the last two rounds fetch blocks that are not used)
         next_cb = advance(next_cb);
@@ -205,21 +320,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
     if (it < ncb) round(sa, 0);
     if (!live) return;
 #pragma unroll
-    for (int i = 0; i < NBW; i++) {
-        // tanh and its derivative 1 - tanh^2 = 4e/(e+1)^2, e = exp(2s).  The derivative is stored on its own:
-        // recovering it from a bf16-rounded tanh loses all precision where the unit saturates.
-        f32x4 t, dt;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float e = __expf(2.f * fminf(acc[i][r], 40.f));
-            const float inv = __builtin_amdgcn_rcpf(e + 1.f);   // 1 ulp; an IEEE division is ten instructions
-            t[r] = 1.f - 2.f * inv;
-            dt[r] = 4.f * e * inv * inv;
-        }
-        const long off = (m0 + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g;
-        *reinterpret_cast<bf16x4*>(bmid + off) = to_bf16(t);
-        *reinterpret_cast<bf16x4*>(bder + off) = to_bf16(dt);
-    }
+    for (int i = 0; i < NBW; i++) store_activation(acc[i], bmid, bder, (m0 + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -721,13 +822,19 @@ size_t ddlerp_bwd_workspace_bytes(long M, int C, int D) {
 }
 
 namespace {
+// up to two blocks per compute unit of the kernel for few tokens; us, that one / the other: 768 channels, 16 tokens 8.7 / 14.1,
+// 2016 9.5 / 15.7, 4096 14.1 / 16.2, 8192 22 / 17; 2048 channels, 2016 16 / 33, 4096 28 / 33, 8192 51 / 34
+bool few_tokens(long ntiles) { return (ntiles + 1) / 2 * 4 <= 2 * compute_units(); }
 template <int D>
 void forward_rank(long M, int T, int C, const void* x, const void* x_prev, const void* alpha, const void* Lw, const void* R, const void* beta,
                   void* bmid, void* bder, void* y, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     // four tiles per block when that still gives every compute unit a block, else two
     const long ntiles = M / TOK;
-    if (ntiles >= 4 * 256)
+    if (few_tokens(ntiles))
+        hipLaunchKernelGGL((ddlerp_fwd_mid_few_kernel<D, 4, 2>), dim3((unsigned)((ntiles + 1) / 2), 4), dim3(256), 0, stream, M, T, C, c(x),
+                           c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+    else if (ntiles >= 4 * 256)
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 4>), dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, stream, M, T, C,
                            c(x), c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     else
