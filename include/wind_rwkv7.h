@@ -346,7 +346,8 @@ int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_siz
  * s = wind_rwkv7_attn_f32_saved_bytes bytes (the state every 16 tokens and a [B,T,H,C] tensor of row sums).
  * wind_rwkv7_attn_f32_backward takes no workspace: it zeroes dq, dk, da, db, dw itself and adds two parts per element
  * onto them (atomics; the result does not depend on their order).  wind_rwkv7_attn_f32_backward_split computes the same
- * gradients faster, with wind_rwkv7_attn_f32_bwd_workspace_bytes bytes of workspace (256-byte aligned).  C a multiple of 16 from 16 to 128 (wind_rwkv7_f32_head_size_supported), T % 16 == 0. */
+ * gradients faster, with wind_rwkv7_attn_f32_bwd_workspace_bytes bytes of workspace (256-byte aligned).
+ * C a multiple of 16 from 16 to 128 (wind_rwkv7_f32_head_size_supported), T % 16 == 0. */
 int wind_rwkv7_f32_head_size_supported(int C);
 size_t wind_rwkv7_attn_f32_saved_bytes(int B, int T, int H, int C);
 int wind_rwkv7_attn_f32_forward(int B, int T, int H, int C,
