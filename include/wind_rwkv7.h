@@ -443,6 +443,10 @@ int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problem
  * k = b = 0.  A sequence of any length then runs padded to whole chunks and its final state is that of token first-1. */
 int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* stream);
 
+/* x [B,T,C] bf16 to out [B,T_out,C]: its first min(T, T_out) tokens, zeros behind them.  last (may be NULL, needs
+ * T_out >= T) [B,C] receives token T-1.  C % 8 == 0. */
+int wind_rwkv7_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, void* stream);
+
 /* Column blocks of token-major bf16 matrices, moved in one launch: piece t is width[t] columns of M rows, read at
  * src[t] (row stride src_ld[t] elements, first column src_col0[t]; a null src reads as zeros) and written at
  * dst[t] (dst_ld[t], dst_col0[t]), with op[t] = 0 copy, 1 tanh, 2 multiplication by 1 - aux^2 (aux[t]: the

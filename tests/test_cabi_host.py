@@ -350,3 +350,13 @@ def test_operators_fail_loudly_without_the_library(monkeypatch, tmp_path):
         attn(x, x, x, x, x, x, 64)
     with pytest.raises((ImportError, RuntimeError)):
         ddlerp(x, torch.zeros(64), torch.zeros(128, 64), torch.zeros(4, 64, 32), torch.zeros(4, 1, 1, 64))
+
+
+def test_pad_rows_validates_on_host():
+    lib = _native.lib()
+    ok = [2, 19, 32, 64, 0x1000, 0x2000, None, None]
+    for idx, val, code in [(0, 0, 2), (1, 0, 2), (2, -1, 2), (3, 60, 2), (4, None, 1), (5, None, 1)]:
+        bad = list(ok)
+        bad[idx] = val
+        assert lib.wind_rwkv7_pad_rows(*bad) == code, (idx, val)
+    assert lib.wind_rwkv7_pad_rows(2, 32, 19, 64, 0x1000, 0x2000, 0x3000, None) == 2   # token T-1 is not among the output's

@@ -53,3 +53,16 @@ def test_a_few_tokens_equal_as_many_steps(B, T, H):
     assert torch.equal(last, x[:, -1])
     assert seq_ref.rel_err(y.float().cpu(), torch.stack(ys, 1).float().cpu()) <= 2e-3
     assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4
+
+
+@pytest.mark.parametrize('B,T,T_out,C', [(1, 1, 16, 64), (2, 1003, 1008, 768), (3, 32, 19, 72), (1, 5, 5, 8)])
+def test_pad_rows(B, T, T_out, C):
+    """Whole numbers through a copy: exact."""
+    from wind_rwkv import _native
+    x = torch.randn(B, T, C, device='cuda').bfloat16()
+    out, last = torch.full((B, T_out, C), 7., device='cuda').bfloat16(), torch.empty(B, C, device='cuda').bfloat16()
+    _native.check(_native.lib().wind_rwkv7_pad_rows(B, T, T_out, C, x.data_ptr(), out.data_ptr(), last.data_ptr() if T_out >= T else None,
+                                                    torch.cuda.current_stream().cuda_stream))
+    n = min(T, T_out)
+    assert torch.equal(out[:, :n], x[:, :n]) and not out[:, n:].any()
+    assert T_out < T or torch.equal(last, x[:, -1])

@@ -934,6 +934,15 @@ int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, vo
     return launch_status();
 }
 
+int wind_rwkv7_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, void* stream) {
+    if (B <= 0 || T <= 0 || T_out <= 0 || C <= 0 || C % 8 != 0 || (long long)B * T * C > (1LL << 38) || (long long)B * T_out * C > (1LL << 38))
+        return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (last && T_out < T) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!x || !out) return WIND_RWKV7_ERR_NULL_POINTER;
+    wkv::launch_pad_rows(B, T, T_out, C, x, out, last, static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
 int wind_rwkv7_copy_columns(long long M, int n, const void* const* src, const long long* src_ld, const int* src_col0,
                             void* const* dst, const long long* dst_ld, const int* dst_col0, const int* width,
                             const int* op, const void* const* aux, void* stream) {

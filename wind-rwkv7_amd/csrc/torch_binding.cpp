@@ -37,7 +37,7 @@ namespace py = pybind11;
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
-    X(ddlerp_forward_from) X(neutral_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(ddlerp_forward_from) X(neutral_rows) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
     X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
@@ -954,13 +954,25 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     }
     const at::ScalarType state_type = s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16;
     if (T % 16 && s.N() == 64 && T <= SHORT_PROMPT && s.B * T <= SHORT_PROMPT_ROWS) return short_prompt(s.B, T, s.C, H, x, p, x_prev, s0, state_type, return_state);
-    Tensor xb = x.to(at::kBFloat16);
-    xb = s.T == T ? xb.contiguous() : at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
+    Tensor xb = x.to(at::kBFloat16).contiguous(), carry;
+    const bool pad = s.T != T, pad_here = pad && reinterpret_cast<uintptr_t>(xb.data_ptr()) % 16 == 0;
+    if (pad_here) {
+        const Tensor whole = at::empty({s.B, s.T, s.C}, xb.options());
+        if (return_state && x.scalar_type() == at::kBFloat16) carry = at::empty({s.B, s.C}, xb.options());   // (the carried token keeps x's own type)
+        check(L.pad_rows((int)s.B, (int)T, (int)s.T, (int)s.C, ptr(xb), ptr(whole), ptr(carry), stream_of(xb)));
+        xb = whole;
+    } else if (pad) {
+        xb = at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
+    }
     const BlockBuffers f(s, xb, false, state_type);
     block_forward(s, xb, p, false, T, x_prev, s0, f);
-    const Tensor y = s.T == T ? f.y : f.y.narrow(1, 0, T).contiguous();
+    Tensor y = f.y;
+    if (pad) {
+        y = at::empty({s.B, T, s.C}, f.y.options());
+        check(L.pad_rows((int)s.B, (int)s.T, (int)T, (int)s.C, ptr(f.y), ptr(y), nullptr, stream_of(xb)));
+    }
     if (!return_state) return py::cast(y);
-    return py::make_tuple(y, py::make_tuple(x.select(1, T - 1).clone(), f.sT));
+    return py::make_tuple(y, py::make_tuple(carry.defined() ? carry : x.select(1, T - 1).clone(), f.sT));
 }
 
 // One token per sequence.  `cache` = (key, 24 bf16 copies, [3,C] float32, workspaces by batch) as the module keeps it;
