@@ -261,6 +261,15 @@ int wind_rwkv7_mixer_prompt(int B, int T, int C, int H, int state_dtype, const w
                             const void* x, const void* x_prev, const void* s0, void* sT, void* y, void* x_carry,
                             void* workspace, size_t workspace_bytes, void* stream);
 
+/* WKV7 with the attn_ln epilogue for n tokens per sequence, one after the other on a state in fp32 registers (head size 64): the
+ * end of a sequence that is no whole number of chunks.  q, v, a, g, y: [B,T,H*64] bf16, the tokens first .. first+n-1 are read and
+ * written; w, k, b: [B,wkb_T,H*64], the tokens wkb_first .. wkb_first+n-1 (as the others': wkb_T = T, wkb_first = first); params
+ * as for wind_rwkv7_attn_ln_forward; s0: NULL (zeros) or the state before, sT: the state after (may be s0 itself).
+ * B <= 65535; bases 16-byte aligned. */
+int wind_rwkv7_attn_ln_tokens(int B, int T, int H, int C, int first, int n, int state_dtype, const void* w, const void* q,
+                              const void* k, const void* v, const void* a, const void* b, const void* g, const void* params,
+                              int wkb_T, int wkb_first, const void* s0, void* y, void* sT, void* stream);
+
 /* ---- ddlerp: data-dependent token-shift interpolation ------------------------------------------------ */
 
 /* Replaces the Triton kernels behind DDLerp (rwkv7_ddlerp.py:306-336; launches :43-48, :76-83, :132-138,
@@ -440,8 +449,10 @@ typedef struct {
 int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problems, void* stream);
 
 /* Tokens first .. T-1 of the recurrence's operands w, k, b [B,T,C] bf16 become ones that leave a state as it is: decay 1,
- * k = b = 0.  A sequence of any length then runs padded to whole chunks and its final state is that of token first-1. */
+ * k = b = 0.  A sequence of any length then runs padded to whole chunks and its final state is that of token first-1.
+ * kept (may be NULL) [3,B,T-first,C] bf16: what the tokens' w, k and b were, for wind_rwkv7_attn_ln_tokens to go on with. */
 int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* stream);
+int wind_rwkv7_neutral_rows_keep(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, void* stream);
 
 /* x [B,T,C] bf16 to out [B,T_out,C]: its first min(T, T_out) tokens, zeros behind them.  last (may be NULL, needs
  * T_out >= T) [B,C] receives token T-1.  C % 8 == 0. */

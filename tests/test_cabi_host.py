@@ -360,3 +360,15 @@ def test_pad_rows_validates_on_host():
         bad[idx] = val
         assert lib.wind_rwkv7_pad_rows(*bad) == code, (idx, val)
     assert lib.wind_rwkv7_pad_rows(2, 32, 19, 64, 0x1000, 0x2000, 0x3000, None) == 2   # token T-1 is not among the output's
+
+
+def test_attn_ln_tokens_validates_on_host():
+    lib = _native.lib()
+    ok = [2, 32, 3, 64, 16, 5, _native.F32] + [0x1000] * 8 + [16, 0, None, 0x2000, 0x3000, None]
+    for idx, val, code in [(0, 0, 2), (0, 70000, 2), (1, 20, 2), (2, 0, 2), (3, 128, 3), (4, -1, 2), (4, 28, 2), (5, 0, 2), (6, 7, 5), (7, None, 1),
+                           (14, None, 1), (15, 4, 2), (16, 12, 2), (18, None, 1), (19, None, 1)]:
+        bad = list(ok)
+        bad[idx] = val
+        assert lib.wind_rwkv7_attn_ln_tokens(*bad) == code, (idx, val)
+    assert lib.wind_rwkv7_neutral_rows_keep(2, 32, 60, 16, 0x1000, 0x1000, 0x1000, 0x2000, None) == 2
+    assert lib.wind_rwkv7_neutral_rows_keep(2, 32, 64, 16, 0x1000, None, 0x1000, 0x2000, None) == 1

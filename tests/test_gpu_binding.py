@@ -134,7 +134,7 @@ def test_block_equals_the_python_path(monkeypatch, C, H, x_dtype, param_dtype, f
 @pytest.mark.parametrize('T', [2, 15, 17, 100])
 @pytest.mark.parametrize('continued', [False, True])
 def test_prompt_of_any_length_equals_the_python_path(monkeypatch, T, continued):
-    """A prompt padded to whole chunks against whole chunks followed by single-token steps: other roundings, so at the
+    """The native prompt against the Python path of whole chunks and single-token steps: other summation orders, so at the
     block's gate (1.27e-2 where `step` computed the tokens, see tests/test_gpu_time_mixer_state.py), state at 1e-2."""
     from collections import namedtuple
     from oracle import seq_ref

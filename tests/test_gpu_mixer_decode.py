@@ -55,6 +55,56 @@ def test_a_few_tokens_equal_as_many_steps(B, T, H):
     assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4
 
 
+@pytest.mark.parametrize('B,T,H', [(1, 1003, 3), (3, 100, 4), (2, 79, 12), (9, 65, 2), (40, 15, 2), (300, 2, 1)])
+@pytest.mark.parametrize('continued', [False, True])
+def test_a_ragged_prompt_is_whole_chunks_and_then_steps(B, T, H, continued):
+    """The tokens after the last whole chunk keep the state in fp32 from token to token, as steps do: the same sums in
+    registers, so the state is theirs to 1e-4 (operands of a chunk's products in bf16 would leave 2^-9 of every token's
+    share) and the outputs to a rounding here and there.  More than eight sequences, one token left and no whole chunk
+    take other launches."""
+    model, gen = _model(H, seed=B + T)
+    C, T0 = 64 * H, T - T % 16
+    x = torch.randn(B, T, C, generator=gen).bfloat16().to(DEV)
+    state = (torch.randn(B, C, generator=gen).bfloat16().to(DEV), torch.randn(B, H, 64, 64, generator=gen).to(DEV))
+    given = (state[0], state[1].clone()) if continued else None
+    with torch.no_grad():
+        y, (last, S) = model(x, state=given, return_state=True)
+        st = (state[0], state[1].clone()) if continued else (torch.zeros_like(state[0]), torch.zeros_like(state[1]))
+        ys = []
+        if T0:
+            y0, st = model(x[:, :T0].contiguous(), state=given, return_state=True)
+            ys.append(y0)
+        for t in range(T0, T):
+            yt, st = model.step(x[:, t], st)
+            ys.append(yt[:, None])
+    assert not continued or torch.equal(given[1], state[1])   # (the caller's is not written)
+    assert y.is_contiguous() and torch.equal(last, x[:, -1])
+    want = torch.cat(ys, 1)
+    start = 0 if continued else 1     # from a zero state the first token's GroupNorm is ill conditioned
+    for first in {start, max(start, T0)}:
+        assert seq_ref.rel_err(y[:, first:].float().cpu(), want[:, first:].float().cpu()) <= 2e-3
+    assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4
+
+
+def test_a_ragged_prompt_at_another_head_size_is_whole_chunks_and_then_steps():
+    from wind_rwkv.rwkv7 import TimeMixer
+    gen = torch.Generator().manual_seed(8)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, 2, 256), 1)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+    model = model.to(DEV)
+    x = torch.randn(2, 37, 256, generator=gen).bfloat16().to(DEV)
+    with torch.no_grad():
+        y, (_, S) = model(x, return_state=True)
+        y0, st = model(x[:, :32].contiguous(), return_state=True)
+        ys = [y0]
+        for t in range(32, 37):
+            yt, st = model.step(x[:, t], st)
+            ys.append(yt[:, None])
+    assert torch.equal(y, torch.cat(ys, 1)) and torch.equal(S, st[1])
+
+
 @pytest.mark.parametrize('B,T,T_out,C', [(1, 1, 16, 64), (2, 1003, 1008, 768), (3, 32, 19, 72), (1, 5, 5, 8)])
 def test_pad_rows(B, T, T_out, C):
     """Whole numbers through a copy: exact."""

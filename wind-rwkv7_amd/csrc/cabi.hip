@@ -544,6 +544,20 @@ int wind_rwkv7_mixer_prompt(int B, int T, int C, int H, int state_dtype, const w
     return launch_status();
 }
 
+int wind_rwkv7_attn_ln_tokens(int B, int T, int H, int C, int first, int n, int state_dtype, const void* w, const void* q, const void* k,
+                              const void* v, const void* a, const void* b, const void* g, const void* params, int wkb_T, int wkb_first,
+                              const void* s0, void* y, void* sT, void* stream) {
+    if (B <= 0 || T <= 0 || H <= 0 || first < 0 || n <= 0 || first > T - n || wkb_first < 0 || wkb_first > wkb_T - n) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (C != wkv::HEAD) return WIND_RWKV7_ERR_HEAD_SIZE;
+    if (B > 65535 || (long long)B * H > (1LL << 30) || (long long)B * (T > wkb_T ? T : wkb_T) * H * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
+    const int rc = check_dtypes(WIND_RWKV7_BF16, state_dtype);
+    if (rc) return rc;
+    if (!w || !q || !k || !v || !a || !b || !g || !params || !y || !sT) return WIND_RWKV7_ERR_NULL_POINTER;   // (s0 may be null)
+    wkv::launch_tokens(B, T, H, first, n, wkb_T, wkb_first, state_dtype == WIND_RWKV7_F32, w, q, k, v, a, b, g, params, s0, sT, y,
+                       static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
 static int check_ddlerp(int B, int T, int C, int D) {
     if (B <= 0 || T <= 0 || C <= 0 || D <= 0) return WIND_RWKV7_ERR_BAD_SHAPE;
     if ((long long)B * T * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
@@ -927,10 +941,14 @@ int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problem
 }
 
 int wind_rwkv7_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* stream) {
+    return wind_rwkv7_neutral_rows_keep(B, T, C, first, w, k, b, nullptr, stream);
+}
+
+int wind_rwkv7_neutral_rows_keep(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, void* stream) {
     if (B <= 0 || T <= 0 || C <= 0 || C % 8 != 0 || first < 0 || first > T || (long long)B * T * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
     if ((long long)B * (T - first) * (C / 8) > 0x7fffffffLL) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (!w || !k || !b) return WIND_RWKV7_ERR_NULL_POINTER;
-    if (first < T) wkv::launch_neutral_rows(B, T, C, first, w, k, b, static_cast<hipStream_t>(stream));
+    if (first < T) wkv::launch_neutral_rows(B, T, C, first, w, k, b, kept, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

@@ -60,11 +60,16 @@ __global__ __launch_bounds__(256) void copy_columns_kernel(ColsArgs g) {
 
 // w = -80 gives the decay exp(-exp(w)) = 1 in float32
 __global__ __launch_bounds__(256) void neutral_rows_kernel(int T, int C, int first, int vectors, __bf16* __restrict__ w,
-                                                           __bf16* __restrict__ k, __bf16* __restrict__ b) {
+                                                           __bf16* __restrict__ k, __bf16* __restrict__ b, __bf16* __restrict__ kept) {
     const int v = blockIdx.x * 256 + threadIdx.x;
     if (v >= vectors) return;
     const int per_row = C / 8, row = v / per_row, rows = T - first;
     const long at = ((long)(row / rows) * T + first + row % rows) * C + (v % per_row) * 8;
+    if (kept != nullptr) {   // (kept's rows lie as the vectors are counted)
+        const __bf16* const src[3] = {w + at, k + at, b + at};
+#pragma unroll
+        for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8*>(kept + 8 * ((long)i * vectors + v)) = *reinterpret_cast<const bf16x8*>(src[i]);
+    }
     bf16x8 none, zero = {};
 #pragma unroll
     for (int e = 0; e < 8; e++) none[e] = (__bf16)-80.f;
@@ -95,10 +100,10 @@ void launch_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, v
                        static_cast<const __bf16*>(x), static_cast<__bf16*>(out), static_cast<__bf16*>(last));
 }
 
-void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, hipStream_t stream) {
+void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, hipStream_t stream) {
     const int vectors = B * (T - first) * (C / 8);
     hipLaunchKernelGGL(neutral_rows_kernel, dim3((unsigned)((vectors + 255) / 256)), dim3(256), 0, stream, T, C, first, vectors,
-                       static_cast<__bf16*>(w), static_cast<__bf16*>(k), static_cast<__bf16*>(b));
+                       static_cast<__bf16*>(w), static_cast<__bf16*>(k), static_cast<__bf16*>(b), static_cast<__bf16*>(kept));
 }
 
 void launch_copy_columns(long long M, int n, const ColumnPiece* pieces, hipStream_t stream) {

@@ -45,10 +45,10 @@ constexpr int CAST_MAX_TENSORS = 32;   // per launch; longer lists take several
 void launch_cast_to_bf16(int n, const void* const* src, const int* src_f32, const long long* numel,
                          const long long* dst_offset, void* dst, hipStream_t stream);
 
-// rows first .. T-1 of w, k, b [B, T, C] (bf16): decay 1, k = b = 0
 // x [B,T,C] to out [B,T_out,C]: the first T tokens, zeros behind them; last (may be null) [B,C]: token T - 1, if out has it
 void launch_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, hipStream_t stream);
-void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, hipStream_t stream);
+// rows first .. T-1 of w, k, b [B, T, C] (bf16): decay 1, k = b = 0; kept (may be null) [3, B, T-first, C]: what they were
+void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, hipStream_t stream);
 
 // dst [rows, cols] (bf16, or f32 where dst_f32) from src (f32 or bf16); dstT: null or the transposed bf16 copy, row stride ldT
 struct PackTensor {

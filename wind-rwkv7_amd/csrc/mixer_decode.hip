@@ -418,8 +418,8 @@ __device__ __forceinline__ void update_state(HeadTile& s, f32x4 (&S)[NBLK], int 
     if (L.g == 0) s.y[n][chan16(ib, L.n)] = acc;
 }
 
-// GroupNorm, bonus and gate of token n (row m of the output), lane = channel
-__device__ __forceinline__ void finish_token(const HeadTile& s, const HeadArgs& A, int h, int n, long m, int lane) {
+// GroupNorm, bonus and gate of token n, lane = channel; out: its row
+__device__ __forceinline__ void finish_token(const HeadTile& s, const float* ln_params, int C, int h, int n, __bf16* out_row, int lane) {
     auto head_sum = [](float x) {
         x = row_sum(x);
         return group_sum(x);
@@ -427,10 +427,10 @@ __device__ __forceinline__ void finish_token(const HeadTile& s, const HeadArgs& 
     const float y = s.y[n][lane];
     const float mean = head_sum(y) * (1.f / HEAD);
     const float istd = rsqrtf(head_sum((y - mean) * (y - mean)) * (1.f / HEAD) + LN_EPS);
-    const float* lp = A.ln_params + h * HEAD + lane;
-    const float dot = head_sum((float)s.r[n][lane] * (float)s.k[n][lane] * lp[2 * (long)A.C]);
-    const float out = ((y - mean) * istd * lp[0] + lp[A.C] + dot * (float)s.v[n][lane]) * (float)s.g[n][lane];
-    A.ya[m * A.C + h * HEAD + lane] = (__bf16)out;
+    const float* lp = ln_params + h * HEAD + lane;
+    const float dot = head_sum((float)s.r[n][lane] * (float)s.k[n][lane] * lp[2 * (long)C]);
+    const float out = ((y - mean) * istd * lp[0] + lp[C] + dot * (float)s.v[n][lane]) * (float)s.g[n][lane];
+    out_row[h * HEAD + lane] = (__bf16)out;
 }
 
 // One token per sequence: block = (some rows of a 16-row tile, head).  Every wavefront asks for the first state it updates
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(256 * GROUPS) void decode_head_kernel(const HeadArg
         }
     }
     lds_barrier();
-    for (int r = r0 + wave; r < end; r += 4 * GROUPS) finish_token(s, A, h, r, row0 + r, lane);
+    for (int r = r0 + wave; r < end; r += 4 * GROUPS) finish_token(s, A.ln_params, A.C, h, r, A.ya + (long)(row0 + r) * A.C, lane);
 }
 
 // T tokens per sequence, one after the other on a state that stays in registers: block = (sequence, head).
@@ -480,8 +480,55 @@ __global__ __launch_bounds__(256) void prompt_head_kernel(const HeadArgs A) {
         expand_tile(s, A, h, first, first + n - 1, ib, L);
         for (int t = 0; t < n; t++) update_state(s, S, t, ib, L);
         lds_barrier();
-        for (int t = ib; t < n; t += 4) finish_token(s, A, h, t, first + t, lane);
+        for (int t = ib; t < n; t += 4) finish_token(s, A.ln_params, A.C, h, t, A.ya + (long)(first + t) * A.C, lane);
         lds_barrier();   // (the next tile overwrites what the epilogue reads)
+    }
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.state, A.state_f32, bh, ib, jb, L, S[jb]);
+}
+
+// The recurrence alone, token by token, with its operands in memory: the tokens of a prompt after its last whole chunk, whose
+// state the sequence kernels would multiply in bf16.  Block = (sequence, head).
+struct TokensArgs {
+    const __bf16 *w, *k, *b, *r, *v, *kk, *g;   // at the sequences' first token
+    __bf16* y;
+    long wkb_seq, seq;                          // elements from one sequence to the next: of w, k, b; of the others and y
+    int n, H, C, state_f32;                     // n tokens of each
+    const float* ln_params;
+    const void* state_in;                       // null: zeros
+    void* state;                                // may be state_in itself
+};
+__global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
+    __shared__ HeadTile s;
+    const int lane = threadIdx.x & 63, ib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Lane L;
+    const int h = blockIdx.x, seq = blockIdx.y, bh = seq * A.H + h;
+    f32x4 S[NBLK];
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+    // 16 bytes per thread and load: eight channels of one of the sixteen tokens, two tensors at a time (wavefronts 0, 1 and 2, 3)
+    const int row = (threadIdx.x & 127) >> 3, c = 8 * (threadIdx.x & 7);
+    const bool second = threadIdx.x >= 128;
+    for (int t0 = 0; t0 < A.n; t0 += TOK) {
+        const int n = A.n - t0 < TOK ? A.n - t0 : TOK;
+        const long t = t0 + (row < n ? row : n - 1);   // (a row past the last repeats it and is not used)
+        const long at = (long)seq * A.seq + t * A.C + h * HEAD + c, at_wkb = (long)seq * A.wkb_seq + t * A.C + h * HEAD + c;
+        auto load = [](const __bf16* p) { return *reinterpret_cast<const bf16x8*>(p); };
+        const bf16x8 x0 = load((second ? A.b : A.k) + at_wkb), x1 = load((second ? A.v : A.r) + at), x2 = load((second ? A.g : A.kk) + at);
+        const bf16x4 wv = *reinterpret_cast<const bf16x4*>(A.w + at_wkb + (second ? 4 : 0));
+        *reinterpret_cast<bf16x8*>(second ? &s.b[row][c] : &s.k[row][c]) = x0;
+        *reinterpret_cast<bf16x8*>(second ? &s.v[row][c] : &s.r[row][c]) = x1;
+        *reinterpret_cast<bf16x8*>(second ? &s.g[row][c] : &s.kk[row][c]) = x2;
+        f32x4 d = to_f32(wv);
+#pragma unroll
+        for (int q = 0; q < 4; q++) d[q] = __expf(-__expf(d[q]));
+        *reinterpret_cast<f32x4*>(&s.decay[row][c + (second ? 4 : 0)]) = d;
+        lds_barrier();
+        for (int i = 0; i < n; i++) update_state(s, S, i, ib, L);
+        lds_barrier();
+        for (int i = ib; i < n; i += 4)
+            finish_token(s, A.ln_params, A.C, h, i, A.y + (long)seq * A.seq + (long)(t0 + i) * A.C, lane);
+        lds_barrier();   // (the next sixteen overwrite what the epilogue reads)
     }
 #pragma unroll
     for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.state, A.state_f32, bh, ib, jb, L, S[jb]);
@@ -595,6 +642,17 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         a.ntiles = ntiles;
         launch_linear<false>(a, mix, stream);
     }
+}
+
+void launch_tokens(int B, int T, int H, int first, int n, int wkb_T, int wkb_first, int state_f32, const void* w, const void* q, const void* k,
+                   const void* v, const void* a, const void* b, const void* g, const void* params, const void* state_in, void* state,
+                   void* y, hipStream_t stream) {
+    const int C = H * HEAD;
+    auto at = [&](const void* p, int token) { return static_cast<const __bf16*>(p) + (long)token * C; };
+    const TokensArgs A{at(w, wkb_first), at(k, wkb_first), at(b, wkb_first), at(q, first), at(v, first), at(a, first), at(g, first),
+                       static_cast<__bf16*>(y) + (long)first * C, (long)wkb_T * C, (long)T * C, n, H, C, state_f32,
+                       static_cast<const float*>(params), state_in, state};
+    hipLaunchKernelGGL(tokens_kernel, dim3(H, B), dim3(256), 0, stream, A);
 }
 
 }  // namespace wkv

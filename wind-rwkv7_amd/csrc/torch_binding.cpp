@@ -37,7 +37,7 @@ namespace py = pybind11;
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
-    X(ddlerp_forward_from) X(neutral_rows) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(ddlerp_forward_from) X(neutral_rows_keep) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
     X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
@@ -676,19 +676,21 @@ struct WeightGrads {
 struct BlockBuffers {
     Tensor weights, acts, saved, y, sT;
     static int64_t saved_bytes(const Block& s) { return L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()); }
-    BlockBuffers(const Block& s, const Tensor& xb, bool save, at::ScalarType state_type) {
+    BlockBuffers(const Block& s, const Tensor& xb, bool save, int64_t valid, at::ScalarType state_type) {
         weights = at::empty({WeightLayout(s.C).total[save]}, xb.options());
         acts = at::empty({Activations(s).total}, xb.options());
         saved = scratch_bytes(saved_bytes(s), xb);
-        y = at::empty({s.B, s.T, s.C}, xb.options());
+        y = at::empty({s.B, valid, s.C}, xb.options());
         sT = at::empty({s.B, s.H, s.N(), s.N()}, xb.options().dtype(state_type));
     }
     BlockBuffers(Tensor w, Tensor a, Tensor s, Tensor y_, Tensor st)
         : weights(std::move(w)), acts(std::move(a)), saved(std::move(s)), y(std::move(y_)), sT(std::move(st)) {}
 };
 
-// x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  `valid` < T: the tokens from
-// there on are padding and leave the state as it is.  x_prev [B,C] bf16 / s0: a carried state (undefined: zero).
+// x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  x_prev [B,C] bf16 / s0: a carried
+// state (undefined: zero).  `valid` < T (head size 64, not with `save`): the tokens from there on are padding, y has none of
+// them.  The sequence kernels then take the whole chunks and leave the tokens after them to attn_ln_tokens, which keeps the
+// state in fp32 from token to token (a chunk's products would round those tokens' share of it to bf16 operands).
 void block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const Tensor& x_prev,
                    const Tensor& s0, const BlockBuffers& f) {
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
@@ -719,14 +721,36 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
     }
     check(L.expand_loras_forward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
                                  w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b), stream));
-    if (valid < T) check(L.neutral_rows(B, T, C, (int)valid, a(A.w), a(A.k2), a(A.b), stream));
-    const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
-    check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
-        B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln), ptr(s0),
-        a(A.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
+    const int whole = (int)(valid / 16 * 16), rest = (int)(valid - whole);
+    Tensor kept;
+    if (rest && whole) {
+        kept = at::empty({3, B, T - whole, C}, xb.options());
+        check(L.neutral_rows_keep(B, T, C, whole, a(A.w), a(A.k2), a(A.b), ptr(kept), stream));
+    }
+    if (whole) {
+        const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
+        check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
+            B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln),
+            ptr(s0), a(A.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
+    }
+    if (rest) {
+        const int64_t part = kept.defined() ? kept.stride(0) : 0;
+        check(L.attn_ln_tokens(B, T, H, N, whole, rest, state_code(f.sT), whole ? at_elem(kept, 0) : a(A.w), a(A.r),
+                               whole ? at_elem(kept, part) : a(A.k2), a(A.v), a(A.kk), whole ? at_elem(kept, 2 * part) : a(A.b), a(A.g),
+                               at_elem(f.weights, W.ln), whole ? T - whole : T, 0, whole ? ptr(f.sT) : ptr(s0), a(A.ya), ptr(f.sT), stream));
+    }
     Products out;
-    out.add(a(A.ya), w(WO), C, C), out.to(ptr(f.y), C);
-    out.run(M, xb);
+    if (!rest) {
+        out.add(a(A.ya), w(WO), C, C), out.to(ptr(f.y), C);
+        out.run(M, xb);
+    } else if (B <= WIND_RWKV7_LINEAR_GROUP_MAX) {   // a product per sequence: one launch, each straight to its place
+        for (int64_t b = 0; b < B; b++) out.add(a(A.ya + b * T * C), w(WO), C, C), out.to(at_elem(f.y, b * valid * C), C);
+        out.run(valid, xb);
+    } else {
+        out.add(a(A.ya), w(WO), C, C), out.to(a(A.streams), C);
+        out.run(M, xb);
+        check(L.pad_rows(B, T, (int)valid, C, a(A.streams), ptr(f.y), nullptr, stream));
+    }
 }
 
 // dx and the gradient of every parameter (ParamLayout's places in `flat`, float32); need(i): whether parameter i's is wanted.
@@ -808,7 +832,7 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         const Block s{x.size(0), x.size(1), x.size(2), H};
         const variable_list p{params...};
         const Tensor xb = x.to(at::kBFloat16).contiguous();
-        const BlockBuffers f(s, xb, true, at::kBFloat16);
+        const BlockBuffers f(s, xb, true, s.T, at::kBFloat16);
         block_forward(s, xb, p, true, s.T, Tensor(), Tensor(), f);
         ctx->save_for_backward({xb, f.weights, f.acts, f.saved});
         std::vector<int64_t> types{H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
@@ -894,8 +918,7 @@ bool floating(const Tensor& t) {
     return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat || t.scalar_type() == at::kHalf || t.scalar_type() == at::kDouble;
 }
 
-// A prompt this short that would have to be padded runs token by token on a state in registers, in the four launches of a
-// step; the sequence kernels take some twenty launches whatever the length.  (Whole chunks stay with them: the same bits as the
+// A ragged prompt this short runs token by token on a state in registers, in the four launches of a step; the sequence kernels take some twenty launches whatever the length.  (Whole chunks stay with them: the same bits as the
 // same tokens inside a longer call.)
 constexpr int64_t SHORT_PROMPT = 64, SHORT_PROMPT_ROWS = 512;
 
@@ -930,7 +953,7 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     const bool stateful = return_state || x_prev_ || s0_;
     const int64_t T = x.size(1);
     const Block s{x.size(0), (T + 15) / 16 * 16, x.size(2), H};
-    if (T % 16 && !stateful) return py::none();
+    if (T % 16 && (!stateful || s.N() != 64 || s.B > 65535)) return py::none();
     if (s.rows() > std::numeric_limits<int>::max() || s.C % 64 || !L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()) ||
         !L.expand_loras_bwd_workspace_bytes(s.B, s.T, s.C, R_LORA) || !L.ddlerp_bwd_workspace_bytes(s.B, s.T, s.C, R_MIX))
         return py::none();
@@ -964,15 +987,10 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     } else if (pad) {
         xb = at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
     }
-    const BlockBuffers f(s, xb, false, state_type);
+    const BlockBuffers f(s, xb, false, T, state_type);
     block_forward(s, xb, p, false, T, x_prev, s0, f);
-    Tensor y = f.y;
-    if (pad) {
-        y = at::empty({s.B, T, s.C}, f.y.options());
-        check(L.pad_rows((int)s.B, (int)s.T, (int)T, (int)s.C, ptr(f.y), ptr(y), nullptr, stream_of(xb)));
-    }
-    if (!return_state) return py::cast(y);
-    return py::make_tuple(y, py::make_tuple(carry.defined() ? carry : x.select(1, T - 1).clone(), f.sT));
+    if (!return_state) return py::cast(f.y);
+    return py::make_tuple(f.y, py::make_tuple(carry.defined() ? carry : x.select(1, T - 1).clone(), f.sT));
 }
 
 // One token per sequence.  `cache` = (key, 24 bf16 copies, [3,C] float32, workspaces by batch) as the module keeps it;

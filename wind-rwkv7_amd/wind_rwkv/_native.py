@@ -62,6 +62,8 @@ SIGNATURES = {
     'wind_rwkv7_ddlerp_forward_from': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp]),
     'wind_rwkv7_pad_rows': (_i, [_i] * 4 + [_vp] * 4),
     'wind_rwkv7_neutral_rows': (_i, [_i] * 4 + [_vp] * 4),
+    'wind_rwkv7_neutral_rows_keep': (_i, [_i] * 4 + [_vp] * 5),
+    'wind_rwkv7_attn_ln_tokens': (_i, [_i] * 7 + [_vp] * 8 + [_i] * 2 + [_vp] * 4),
     'wind_rwkv7_ddlerp_backward': (_i, [_i] * 4 + [_vp] * 7 + [_vp] * 4 + [_vp] * 5 + [_vp, _sz, _vp]),
     'wind_rwkv7_ln_epilogue_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_ln_epilogue_forward': (_i, [_i] * 4 + [_vp] * 8),

@@ -279,9 +279,9 @@ class TimeMixer(nn.Module):
         `return_state=True` returns (y, state) to continue from - a prompt is run in one or several such calls
         and then token by token with `step`.  Either needs attn_impl='cuda' and no autograd, and lifts the
         reference's restriction of T to multiples of 16.  With the default switches an eager call runs in the native
-        binding, forward and backward as one autograd node (a length that is no multiple of 16 padded with tokens that
-        leave the state alone); what follows here is what torch.compile traces, and every other case (there the tokens
-        after the last full chunk go through `step`)."""
+        binding, forward and backward as one autograd node; what follows here is what torch.compile traces, and every
+        other case.  The tokens after the last full chunk advance the state one by one, in fp32 as `step` does (here: by
+        calls of `step`)."""
         B, T, C = x.shape
         native = (x.is_cuda and self.attn_impl == 'cuda' and self.use_triton_ddlerp and self._loras_kernel
                   and _attn_bf16_head(self.head_size))
