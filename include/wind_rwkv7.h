@@ -288,10 +288,19 @@ size_t wind_rwkv7_ddlerp_bwd_workspace_bytes(int B, int T, int C, int D);
 int wind_rwkv7_ddlerp_forward(int B, int T, int C, int D,
                               const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                               void* bmid, void* bder, void* y, void* stream);
-/* The forward of a piece of a longer sequence: x_prev [B,C] bf16 is the token before x[:, 0] (NULL: a zero row, as above). */
-int wind_rwkv7_ddlerp_forward_from(int B, int T, int C, int D, const void* x, const void* x_prev, const void* alpha,
-                                   const void* L, const void* R, const void* beta, void* bmid, void* bder, void* y,
-                                   void* stream);
+/* The four streams of one token per sequence that follows a carried token (a continued sequence's first): as above with the
+ * token before it in place of the zero row, but in float32 throughout and on the parameters as they are.  x + b x_seq and
+ * x_prev + b C: the tokens, C elements of x_dtype; alpha, L, R, beta: of param_dtype, any alignment.
+ * y + k y_stream + b y_seq: C bf16 values (the streams' rows of a forward's y, to replace them).  B <= 65535.
+ * workspace: wind_rwkv7_ddlerp_first_workspace_bytes(B, D) bytes, 256-byte aligned. */
+typedef struct {
+    const void *x, *x_prev, *alpha, *L, *R, *beta;
+    long long x_seq, y_stream, y_seq;
+    int x_dtype, param_dtype;
+} wind_rwkv7_first_tokens;
+size_t wind_rwkv7_ddlerp_first_workspace_bytes(int B, int D);
+int wind_rwkv7_ddlerp_first(int B, int C, int D, const wind_rwkv7_first_tokens* t, void* y, void* workspace, size_t workspace_bytes,
+                            void* stream);
 int wind_rwkv7_ddlerp_backward(int B, int T, int C, int D,
                                const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                                const void* bmid, const void* bder,

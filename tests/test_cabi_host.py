@@ -372,3 +372,19 @@ def test_attn_ln_tokens_validates_on_host():
         assert lib.wind_rwkv7_attn_ln_tokens(*bad) == code, (idx, val)
     assert lib.wind_rwkv7_neutral_rows_keep(2, 32, 60, 16, 0x1000, 0x1000, 0x1000, 0x2000, None) == 2
     assert lib.wind_rwkv7_neutral_rows_keep(2, 32, 64, 16, 0x1000, None, 0x1000, 0x2000, None) == 1
+
+
+def test_ddlerp_first_validates_on_host():
+    import ctypes
+    lib = _native.lib()
+    assert lib.wind_rwkv7_ddlerp_first_workspace_bytes(3, 32) >= 3 * 4 * 32 * 4 and lib.wind_rwkv7_ddlerp_first_workspace_bytes(3, 48) == 0
+    fields = dict(x=0x1000, x_prev=0x1000, alpha=0x1000, L=0x1000, R=0x1000, beta=0x1000, x_seq=64, y_stream=64, y_seq=64,
+                  x_dtype=_native.F32, param_dtype=_native.BF16)
+    def call(B=2, C=64, D=32, y=0x2000, ws=0x3000, ws_bytes=1 << 20, t=True, **change):
+        args = _native.FirstTokens(**{**fields, **change})
+        return lib.wind_rwkv7_ddlerp_first(B, C, D, ctypes.byref(args) if t else None, y, ws, ws_bytes, None)
+    assert call(B=0) == 2 and call(B=70000) == 2 and call(C=72) == 9 and call(D=48) != 0
+    assert call(t=False) == 1 and call(y=None) == 1 and call(beta=None) == 1
+    assert call(x_dtype=7) == 5 and call(param_dtype=-1) == 5
+    assert call(x_seq=-1) == 2 and call(y_seq=-1) == 2
+    assert call(ws=None) == 6 and call(ws_bytes=256) == 6 and call(ws=0x3010) == 6

@@ -118,3 +118,35 @@ def test_ddlerp_rejects_unsupported_shapes():
     assert lib.wind_rwkv7_ddlerp_forward(1, 10, 64, 32, *([0x1000] * 8), None) == 4
     for rank in (8, 16, 48, 96, 128):
         assert lib.wind_rwkv7_ddlerp_forward(1, 16, 64, rank, *([0x1000] * 8), None) == 8
+
+
+@pytest.mark.parametrize('B,C,D,x_dtype,p_dtype', [(1, 64, 32, torch.bfloat16, torch.float32), (3, 768, 32, torch.float32, torch.float32),
+                                                   (2, 2112, 64, torch.bfloat16, torch.bfloat16), (5, 320, 64, torch.float32, torch.bfloat16)])
+def test_first_tokens_after_a_carried_one(B, C, D, x_dtype, p_dtype):
+    """The streams of one token per sequence in fp32 on the parameters as they are, against fp64: the rounding of an output with
+    seven stored bits, 2^-8 of a value, and 1e-5 for the sums.  The tokens and every parameter start one element off an allocation."""
+    from wind_rwkv import _native
+    gen = torch.Generator().manual_seed(C)
+    def off(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        flat[1:] = t.to(DEV).reshape(-1)
+        return flat[1:].view(t.shape)
+    T = 3
+    x, prev = off(torch.randn(B, T, C, generator=gen).to(x_dtype)), off(torch.randn(B, C, generator=gen).to(x_dtype))
+    alpha, L, R, beta = (off((torch.randn(shape, generator=gen) * scale).to(p_dtype))
+                         for shape, scale in [((C,), 0.5), ((4 * D, C), 0.1), ((4, C, D), 0.1), ((4, 1, 1, C), 0.5)])
+    lib = _native.lib()
+    y = torch.full((4, B, T, C), 7., device=DEV).bfloat16()
+    ws = torch.empty(lib.wind_rwkv7_ddlerp_first_workspace_bytes(B, D), dtype=torch.uint8, device=DEV)
+    dt = lambda t: _native.F32 if t.dtype == torch.float32 else _native.BF16
+    args = _native.FirstTokens(x.data_ptr(), prev.data_ptr(), alpha.data_ptr(), L.data_ptr(), R.data_ptr(), beta.data_ptr(),
+                               T * C, B * T * C, T * C, dt(x), dt(alpha))
+    import ctypes
+    _native.check(lib.wind_rwkv7_ddlerp_first(B, C, D, ctypes.byref(args), y.data_ptr(), ws.data_ptr(), ws.numel(),
+                                              torch.cuda.current_stream().cuda_stream))
+    xf, pf, al, l, r, be = (t.double().cpu() for t in (x[:, 0], prev, alpha, L, R, beta))
+    mid = torch.tanh((xf + (pf - xf) * al) @ l.mT).view(B, 4, D)
+    want = torch.stack([xf + (pf - xf) * (mid[:, k] @ r[k].mT + be[k, 0, 0]) for k in range(4)])
+    got = y.double().cpu()
+    assert ((got[:, :, 0] - want).abs() <= 2 ** -8 * want.abs() + 1e-5 * want.abs().max()).all()
+    assert (got[:, :, 1:] == 7).all()   # the other tokens are not written

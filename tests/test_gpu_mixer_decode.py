@@ -81,9 +81,13 @@ def test_a_ragged_prompt_is_whole_chunks_and_then_steps(B, T, H, continued):
     assert y.is_contiguous() and torch.equal(last, x[:, -1])
     want = torch.cat(ys, 1)
     start = 0 if continued else 1     # from a zero state the first token's GroupNorm is ill conditioned
+    # The sequence kernels mix a continued prompt's first token in fp32 where `step` rounds its weights to bf16.  Where a step
+    # is that token's reference (no whole chunk) its operands differ by up to a rounding each, 2^-8 of k, v, a and b and half of
+    # that in the mean: 2^-7 of its share of the state, and the block's gate on the outputs.
+    y_gate, S_gate = (1.27e-2, 2 ** -7) if continued and T0 == 0 else (2e-3, 1e-4)
     for first in {start, max(start, T0)}:
-        assert seq_ref.rel_err(y[:, first:].float().cpu(), want[:, first:].float().cpu()) <= 2e-3
-    assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4
+        assert seq_ref.rel_err(y[:, first:].float().cpu(), want[:, first:].float().cpu()) <= y_gate
+    assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= S_gate
 
 
 def test_a_ragged_prompt_at_another_head_size_is_whole_chunks_and_then_steps():

@@ -127,3 +127,31 @@ def test_any_prompt_length_with_a_carried_state(T):
     assert got.shape == whole.shape and state[1].dtype == torch.float32
     assert seq_ref.rel_err(got.float().cpu(), whole.float().cpu()) <= 1e-2
     assert torch.equal(state[0], x[:, -1])
+
+
+@pytest.mark.parametrize('T,B,x_dtype,compiled', [(16, 2, torch.bfloat16, False), (32, 3, torch.float32, False), (48, 2, torch.bfloat16, True),
+                                                  (100, 2, torch.bfloat16, False), (80, 9, torch.float32, True)])
+def test_the_first_token_of_a_continued_prompt_is_mixed_in_fp32(monkeypatch, T, B, x_dtype, compiled):
+    """Mix weights of 1 - 2^-10 after a carried token of zero leave 2^-10 of the first token in every stream; rounded to bf16
+    the weights are 1 and nothing is left.  Against the Python path, which mixes that token in fp32 and differs by bf16
+    roundings and summation orders from there on (the block's gate)."""
+    from wind_rwkv import _native
+    model, gen = _model(256, 4, seed=21)
+    with torch.no_grad():
+        model.time_maa.fill_(1 - 2 ** -10)
+        model.time_maa_w1.zero_()
+        model.ln_x.bias.zero_()
+    x = torch.randn(B, T, 256, generator=gen).to(DEV, x_dtype)
+    state = (torch.zeros(B, 256, dtype=x_dtype, device=DEV), torch.randn(B, 4, 64, 64, generator=gen).to(DEV))
+    fn = torch.compile(lambda t, st: model(t, state=st, return_state=True), fullgraph=True) if compiled else \
+        lambda t, st: model(t, state=st, return_state=True)
+    with torch.no_grad():
+        y, (_, S) = fn(x, state)
+
+        class Absent:
+            def __getattr__(self, name):
+                return lambda *args: None
+        monkeypatch.setattr(_native, 'binding', lambda: Absent())
+        y0, (_, S0) = model(x, state=state, return_state=True)
+    assert seq_ref.rel_err(y[:, 0].float().cpu(), y0[:, 0].float().cpu()) <= 1e-2
+    assert seq_ref.rel_err(S.cpu(), S0.cpu()) <= 1e-2

@@ -577,17 +577,32 @@ size_t wind_rwkv7_ddlerp_bwd_workspace_bytes(int B, int T, int C, int D) {
 int wind_rwkv7_ddlerp_forward(int B, int T, int C, int D,
                               const void* x, const void* alpha, const void* L, const void* R, const void* beta,
                               void* bmid, void* bder, void* y, void* stream) {
-    return wind_rwkv7_ddlerp_forward_from(B, T, C, D, x, nullptr, alpha, L, R, beta, bmid, bder, y, stream);
-}
-
-int wind_rwkv7_ddlerp_forward_from(int B, int T, int C, int D, const void* x, const void* x_prev, const void* alpha,
-                                   const void* L, const void* R, const void* beta, void* bmid, void* bder, void* y,
-                                   void* stream) {
     const int rc = check_ddlerp(B, T, C, D);
     if (rc) return rc;
     if (!x || !alpha || !L || !R || !beta || !bmid || !bder || !y) return WIND_RWKV7_ERR_NULL_POINTER;
-    wkv::launch_ddlerp_forward((long)B * T, T, C, D, x, x_prev, alpha, L, R, beta, bmid, bder, y,
-                               static_cast<hipStream_t>(stream));
+    wkv::launch_ddlerp_forward((long)B * T, T, C, D, x, alpha, L, R, beta, bmid, bder, y, static_cast<hipStream_t>(stream));
+    return launch_status();
+}
+
+size_t wind_rwkv7_ddlerp_first_workspace_bytes(int B, int D) {
+    if (B <= 0 || !wkv::ddlerp_rank_supported(D)) return 0;
+    return align_up((size_t)B * 4 * D * sizeof(float));
+}
+
+int wind_rwkv7_ddlerp_first(int B, int C, int D, const wind_rwkv7_first_tokens* t, void* y, void* workspace, size_t workspace_bytes,
+                            void* stream) {
+    int rc = check_ddlerp(B, 16, C, D);
+    if (rc) return rc;
+    if (B > 65535) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!t || !t->x || !t->x_prev || !t->alpha || !t->L || !t->R || !t->beta || !y) return WIND_RWKV7_ERR_NULL_POINTER;
+    for (int d : {t->x_dtype, t->param_dtype})
+        if (d != WIND_RWKV7_BF16 && d != WIND_RWKV7_F32) return WIND_RWKV7_ERR_DTYPE;
+    constexpr long long most = 1LL << 40;
+    if (t->x_seq < 0 || t->x_seq > most || t->y_stream < 0 || t->y_stream > most || t->y_seq < 0 || t->y_seq > most) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if ((rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_ddlerp_first_workspace_bytes(B, D)))) return rc;
+    const wkv::FirstTokens f{t->x, t->x_prev, t->alpha, t->L, t->R, t->beta, (long)t->x_seq, (long)t->y_stream, (long)t->y_seq,
+                             t->x_dtype == WIND_RWKV7_F32, t->param_dtype == WIND_RWKV7_F32};
+    wkv::launch_ddlerp_first(B, C, D, f, y, workspace, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

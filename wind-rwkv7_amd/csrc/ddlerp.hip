@@ -29,22 +29,21 @@ struct Dy4 {  // the four upstream gradients, each [M, C]
 struct XTile {
     TileF x, xx;
 };
-// the row before token m at the lane's channels: the token before it, at a sequence's start the carried token of x_prev,
-// or (has_prev false: to be read as zeros) the row itself
+// the row before token m at the lane's channels: the token before it, at a sequence's start (has_prev false: to be read as
+// zeros) the row itself
 struct PrevRow {
     const __bf16* row;
     bool has_prev;
 };
-__device__ __forceinline__ PrevRow prev_row(const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev, long m, int T, int C, int c) {
+__device__ __forceinline__ PrevRow prev_row(const __bf16* __restrict__ x, long m, int T, int C, int c) {
     const bool inside = (m % T) != 0;
     const __bf16* row = x + m * C + c;
-    return {inside ? row - C : x_prev ? x_prev + (m / T) * C + c : row, inside || x_prev};
+    return {inside ? row - C : row, inside};
 }
-__device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev, long m0, int T, int C,
-                                             int c0, const Lane& L) {
+__device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, long m0, int T, int C, int c0, const Lane& L) {
     XTile r;
     const long m = m0 + L.n;
-    const PrevRow before = prev_row(x, x_prev, m, T, C, c0 + 8 * L.g);
+    const PrevRow before = prev_row(x, m, T, C, c0 + 8 * L.g);
     // 16-byte accesses: blocks 2p and 2p+1 of the tile are the interleaved channels of chan16 (frag.hpp); every
     // per-channel operand of these kernels is indexed through the same map
     const __bf16* row = x + m * C + c0 + 8 * L.g;
@@ -138,7 +137,6 @@ __device__ __forceinline__ void store_activation(f32x4 s, __bf16* __restrict__ b
 // weights are spread over the blocks.  The kernel below fetches all of them per block, a barrier per channel block.
 template <int D, int SPLIT, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, int C, const __bf16* __restrict__ x,
-                                                                 const __bf16* __restrict__ x_prev,
                                                                  const __bf16* __restrict__ alpha,
                                                                  const __bf16* __restrict__ Lw, __bf16* __restrict__ bmid,
                                                                  __bf16* __restrict__ bder) {
@@ -154,7 +152,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, 
     for (int p = 0; p < TPB; p++) {
         const long tile = (long)blockIdx.x * TPB + p;
         m0[p] = (tile < ntiles ? tile : ntiles - 1) * TOK;   // (a spare tile is the last one again and stores nothing)
-        before[p] = prev_row(x, x_prev, m0[p] + L.n, T, C, 8 * L.g);
+        before[p] = prev_row(x, m0[p] + L.n, T, C, 8 * L.g);
     }
     f32x4 acc[TPB][NB];
 #pragma unroll
@@ -234,7 +232,6 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, 
 // forward 1: bmid = tanh((x + xx*alpha) L^T), bder = 1 - bmid^2
 template <int D, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int C, const __bf16* __restrict__ x,
-                                                             const __bf16* __restrict__ x_prev,
                                                              const __bf16* __restrict__ alpha,
                                                              const __bf16* __restrict__ Lw, __bf16* __restrict__ bmid,
                                                              __bf16* __restrict__ bder) {
@@ -267,7 +264,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
         bf16x8 xc[NBLK / 2], xp[NBLK / 2];
         bf16x4 al[NBLK];
     };
-    const PrevRow before = prev_row(x, x_prev, m0 + L.n, T, C, 8 * L.g);
+    const PrevRow before = prev_row(x, m0 + L.n, T, C, 8 * L.g);
     const bool has_prev = before.has_prev;
     auto fetch = [&](Set& st, int cbk) {
         const int c0 = 64 * cbk;
@@ -468,7 +465,7 @@ __device__ __forceinline__ void load_mid_pairs(bf16x8 (&out)[NPAIR], const __bf1
 // forward 2: y_k = x + xx * (bmid_k R_k^T + beta_k).  Block = (64 channels, range of token tiles).
 template <int D>
 __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int C, int tiles_per_split,
-                                                              const __bf16* __restrict__ x, const __bf16* __restrict__ x_prev,
+                                                              const __bf16* __restrict__ x,
                                                               const __bf16* __restrict__ R, const __bf16* __restrict__ beta,
                                                               const __bf16* __restrict__ bmid, __bf16* __restrict__ y) {
     constexpr int ND = D / 16;
@@ -483,7 +480,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int
     __syncthreads();
     for (long tile = tile_begin + wave; tile < tile_end; tile += 4) {
         const long m0 = tile * TOK;
-        const XTile xt = load_x_tile(x, x_prev, m0, T, C, c0, L);
+        const XTile xt = load_x_tile(x, m0, T, C, c0, L);
         bf16x8 bm[4 * ND / 2];
         load_mid_pairs(bm, bmid + (m0 + L.n) * (4 * D), L);
 #pragma unroll
@@ -782,6 +779,44 @@ __global__ __launch_bounds__(256) void ddlerp_param_reduce_kernel(int C, int nsp
 }
 
 // ------------------------------------------------------------------------------------------------
+// The four streams of ONE token per sequence whose predecessor is carried from an earlier call, in fp32 on the parameters
+// as they are (the kernels above round them, and the hidden activation, to bf16; a piece's first token decides what every
+// later token of a continued sequence meets, and is not rounded twice).  Bound by the launches: 128 x 768 + 4 x 768 x 32
+// weights spread over 32 and 12 blocks per sequence, 64 lanes on one row of L, then a channel per lane and a stream per
+// wavefront.  Elements one by one: parameters of any alignment.
+// ------------------------------------------------------------------------------------------------
+template <class X, class P>   // element types of the tokens and of the parameters
+__global__ __launch_bounds__(256) void first_mid_kernel(int C, int D4, const X* __restrict__ x, long x_seq, const X* __restrict__ x_prev,
+                                                        const P* __restrict__ alpha, const P* __restrict__ Lw, float* __restrict__ mid) {
+    const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;   // a wavefront per hidden unit
+    const X *xr = x + (long)b * x_seq, *pr = x_prev + (long)b * C;
+    const P* lr = Lw + (long)m * C;
+    float acc = 0.f;
+#pragma unroll 6
+    for (int c = lane; c < C; c += 64) {
+        const float cur = (float)xr[c];
+        acc += (cur + ((float)pr[c] - cur) * (float)alpha[c]) * (float)lr[c];
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) acc += __shfl_xor(acc, d);
+    if (lane == 0) mid[(long)b * D4 + m] = tanhf(acc);
+}
+template <class X, class P, int D>
+__global__ __launch_bounds__(256) void first_streams_kernel(int C, const X* __restrict__ x, long x_seq, const X* __restrict__ x_prev,
+                                                            const P* __restrict__ R, const P* __restrict__ beta, const float* __restrict__ mid,
+                                                            __bf16* __restrict__ y, long y_stream, long y_seq) {
+    const int c = blockIdx.x * 64 + (threadIdx.x & 63), b = blockIdx.y;
+    const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const P* r = R + ((long)k * C + c) * D;
+    const float* h = mid + ((long)b * 4 + k) * D;   // (the same for all lanes)
+    const float cur = (float)x[(long)b * x_seq + c], prev = (float)x_prev[(long)b * C + c];
+    float coeff = (float)beta[(long)k * C + c];
+#pragma unroll
+    for (int j = 0; j < D; j++) coeff += h[j] * (float)r[j];
+    y[k * y_stream + (long)b * y_seq + c] = (__bf16)(cur + (prev - cur) * coeff);
+}
+
+// ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
 namespace {
@@ -826,23 +861,23 @@ namespace {
 // 2016 9.5 / 15.7, 4096 14.1 / 16.2, 8192 22 / 17; 2048 channels, 2016 16 / 33, 4096 28 / 33, 8192 51 / 34
 bool few_tokens(long ntiles) { return (ntiles + 1) / 2 * 4 <= 2 * compute_units(); }
 template <int D>
-void forward_rank(long M, int T, int C, const void* x, const void* x_prev, const void* alpha, const void* Lw, const void* R, const void* beta,
+void forward_rank(long M, int T, int C, const void* x, const void* alpha, const void* Lw, const void* R, const void* beta,
                   void* bmid, void* bder, void* y, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     // four tiles per block when that still gives every compute unit a block, else two
     const long ntiles = M / TOK;
     if (few_tokens(ntiles))
         hipLaunchKernelGGL((ddlerp_fwd_mid_few_kernel<D, 4, 2>), dim3((unsigned)((ntiles + 1) / 2), 4), dim3(256), 0, stream, M, T, C, c(x),
-                           c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+                           c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     else if (ntiles >= 4 * 256)
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 4>), dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, stream, M, T, C,
-                           c(x), c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+                           c(x), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     else
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 2>), dim3((unsigned)((ntiles + 1) / 2)), dim3(256), 0, stream, M, T, C,
-                           c(x), c(x_prev), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
+                           c(x), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
     const StreamSplit sp = stream_splits(M, C / 64, 4 * compute_units());   // two blocks per compute unit, two rounds
     hipLaunchKernelGGL(ddlerp_fwd_out2_kernel<D>, dim3(C / 64, sp.nsplit), dim3(256), 0, stream, M, T, C, sp.tiles_per_split,
-                       c(x), c(x_prev), c(R), c(beta), c(bmid), static_cast<__bf16*>(y));
+                       c(x), c(R), c(beta), c(bmid), static_cast<__bf16*>(y));
 }
 
 template <int D>
@@ -873,11 +908,33 @@ void backward_rank(long M, int T, int C, const void* x, const void* alpha, const
 }
 }  // namespace
 
+namespace {
+template <class X, class P, int D>
+void first_tokens(int B, int C, const FirstTokens& t, void* y, float* mid, hipStream_t stream) {
+    auto x = [](const void* p) { return static_cast<const X*>(p); };
+    auto w = [](const void* p) { return static_cast<const P*>(p); };
+    hipLaunchKernelGGL((first_mid_kernel<X, P>), dim3(D, B), dim3(256), 0, stream, C, 4 * D, x(t.x), t.x_seq, x(t.x_prev), w(t.alpha), w(t.Lw), mid);
+    hipLaunchKernelGGL((first_streams_kernel<X, P, D>), dim3(C / 64, B), dim3(256), 0, stream, C, x(t.x), t.x_seq, x(t.x_prev), w(t.R), w(t.beta),
+                       mid, static_cast<__bf16*>(y), t.y_stream, t.y_seq);
+}
+template <int D>
+void first_tokens_rank(int B, int C, const FirstTokens& t, void* y, float* mid, hipStream_t stream) {
+    if (t.x_f32 && t.param_f32) first_tokens<float, float, D>(B, C, t, y, mid, stream);
+    else if (t.x_f32) first_tokens<float, __bf16, D>(B, C, t, y, mid, stream);
+    else if (t.param_f32) first_tokens<__bf16, float, D>(B, C, t, y, mid, stream);
+    else first_tokens<__bf16, __bf16, D>(B, C, t, y, mid, stream);
+}
+}  // namespace
+
 // (the callers have checked ddlerp_rank_supported(D))
-void launch_ddlerp_forward(long M, int T, int C, int D, const void* x, const void* x_prev, const void* alpha, const void* Lw,
-                           const void* R, const void* beta, void* bmid, void* bder, void* y, hipStream_t stream) {
-    if (D == 64) forward_rank<64>(M, T, C, x, x_prev, alpha, Lw, R, beta, bmid, bder, y, stream);
-    else forward_rank<32>(M, T, C, x, x_prev, alpha, Lw, R, beta, bmid, bder, y, stream);
+void launch_ddlerp_first(int B, int C, int D, const FirstTokens& t, void* y, void* workspace, hipStream_t stream) {
+    if (D == 64) first_tokens_rank<64>(B, C, t, y, static_cast<float*>(workspace), stream);
+    else first_tokens_rank<32>(B, C, t, y, static_cast<float*>(workspace), stream);
+}
+
+void launch_ddlerp_forward(long M, int T, int C, int D, const void* x, const void* alpha, const void* Lw, const void* R, const void* beta, void* bmid, void* bder, void* y, hipStream_t stream) {
+    if (D == 64) forward_rank<64>(M, T, C, x, alpha, Lw, R, beta, bmid, bder, y, stream);
+    else forward_rank<32>(M, T, C, x, alpha, Lw, R, beta, bmid, bder, y, stream);
 }
 
 void launch_ddlerp_backward(long M, int T, int C, int D, const void* x, const void* alpha, const void* Lw, const void* R,

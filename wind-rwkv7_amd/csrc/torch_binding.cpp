@@ -37,7 +37,7 @@ namespace py = pybind11;
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
-    X(ddlerp_forward_from) X(neutral_rows_keep) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(ddlerp_first_workspace_bytes) X(ddlerp_first) X(neutral_rows_keep) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
     X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
@@ -687,11 +687,36 @@ struct BlockBuffers {
         : weights(std::move(w)), acts(std::move(a)), saved(std::move(s)), y(std::move(y_)), sT(std::move(st)) {}
 };
 
-// x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  x_prev [B,C] bf16 / s0: a carried
-// state (undefined: zero).  `valid` < T (head size 64, not with `save`): the tokens from there on are padding, y has none of
+// A continued sequence's first token and the carried one before it, both float32 or both bf16 (no defined tensors: there is
+// none).  Its streams are made in fp32 on the parameters themselves.
+struct First {
+    Tensor x, prev;   // [B,C], x's rows anywhere
+    First() = default;
+    First(const Tensor& x_first, const Tensor& x_prev) : x(x_first), prev(x_prev) {
+        if (x.scalar_type() != at::kBFloat16 || prev.scalar_type() != at::kBFloat16) x = x.to(at::kFloat), prev = prev.to(at::kFloat);
+        if (x.stride(1) != 1) x = x.contiguous();
+        prev = prev.contiguous();
+    }
+    // y[k * y_stream + b * y_seq ..]: stream k of sequence b
+    void streams(const variable_list& p, void* y, int64_t y_stream, int64_t y_seq) const {
+        const int B = x.size(0), C = x.size(1);
+        Tensor w[4] = {p[MAA_X], p[MAA_W1], p[MAA_W2], p[MAA]};
+        bool f32 = false;
+        for (const auto& t : w) f32 = f32 || t.scalar_type() == at::kFloat;
+        if (f32)
+            for (auto& t : w) t = t.to(at::kFloat);
+        const wind_rwkv7_first_tokens t{ptr(x),      ptr(prev), ptr(w[0]), ptr(w[1]),       ptr(w[2]), ptr(w[3]),
+                                        x.stride(0), y_stream,  y_seq,     state_code(x), state_code(w[0])};
+        const Tensor ws = scratch_bytes(L.ddlerp_first_workspace_bytes(B, R_MIX), x);
+        check(L.ddlerp_first(B, C, R_MIX, &t, y, ptr(ws), ws.numel(), stream_of(x)));
+    }
+};
+
+// x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  `first` / s0: a carried state
+// (undefined: zero).  `valid` < T (head size 64, not with `save`): the tokens from there on are padding, y has none of
 // them.  The sequence kernels then take the whole chunks and leave the tokens after them to attn_ln_tokens, which keeps the
 // state in fp32 from token to token (a chunk's products would round those tokens' share of it to bf16 operands).
-void block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const Tensor& x_prev,
+void block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const First& first,
                    const Tensor& s0, const BlockBuffers& f) {
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
     const int64_t M = s.rows(), P = s.plane();
@@ -701,19 +726,19 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
     pack_weights(W, p, f.weights, save);
     auto a = [&](int64_t o) -> void* { return at_elem(f.acts, o); };
     auto w = [&](int i) -> void* { return at_elem(f.weights, W.at_.at[i]); };
-    check(L.ddlerp_forward_from(B, T, C, R_MIX, ptr(xb), ptr(x_prev), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), a(A.streams),
-                                stream));
+    check(L.ddlerp_forward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), a(A.streams), stream));
+    if (first.x.defined()) first.streams(p, a(A.streams), P, (int64_t)T * C);
     const void *xrg = a(A.streams), *xwa = a(A.streams + P), *xk = a(A.streams + 2 * P), *xv = a(A.streams + 3 * P);
     {
-        Products first;
-        first.add(xrg, w(WR), C, C), first.to(a(A.r), C);
-        first.add(xk, w(WK), C, C), first.to(a(A.k), C);
-        first.add(xv, w(WV), C, C), first.to(a(A.v), C);
-        first.add(xrg, w(GATE_W1), C, R_GATE), first.to(a(A.tg1), R_GATE, 1);
-        first.add(xwa, w(DECAY_W1), C, W_DECAY_AAA_MA);
-        first.to(a(A.tw1), R_DECAY, 1), first.to(a(A.a1), R_LORA), first.to(a(A.ma1), R_LORA);
-        first.add(xk, w(KKK_W1), C, W_KKMK), first.to(a(A.kk1), R_LORA), first.to(a(A.mk1), R_LORA);
-        first.run(M, xb);
+        Products halves;
+        halves.add(xrg, w(WR), C, C), halves.to(a(A.r), C);
+        halves.add(xk, w(WK), C, C), halves.to(a(A.k), C);
+        halves.add(xv, w(WV), C, C), halves.to(a(A.v), C);
+        halves.add(xrg, w(GATE_W1), C, R_GATE), halves.to(a(A.tg1), R_GATE, 1);
+        halves.add(xwa, w(DECAY_W1), C, W_DECAY_AAA_MA);
+        halves.to(a(A.tw1), R_DECAY, 1), halves.to(a(A.a1), R_LORA), halves.to(a(A.ma1), R_LORA);
+        halves.add(xk, w(KKK_W1), C, W_KKMK), halves.to(a(A.kk1), R_LORA), halves.to(a(A.mk1), R_LORA);
+        halves.run(M, xb);
         Products second;
         second.add(a(A.tg1), w(GATE_W2), R_GATE, C), second.to(a(A.g), C);
         second.add(a(A.tw1), w(DECAY_W2), R_DECAY, C), second.to(a(A.w2), C);
@@ -833,7 +858,7 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         const variable_list p{params...};
         const Tensor xb = x.to(at::kBFloat16).contiguous();
         const BlockBuffers f(s, xb, true, s.T, at::kBFloat16);
-        block_forward(s, xb, p, true, s.T, Tensor(), Tensor(), f);
+        block_forward(s, xb, p, true, s.T, First(), Tensor(), f);
         ctx->save_for_backward({xb, f.weights, f.acts, f.saved});
         std::vector<int64_t> types{H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
         for (const auto& t : p) types.push_back((int64_t)t.scalar_type());
@@ -877,12 +902,12 @@ std::vector<int64_t> block_sizes(int64_t C) {
     r.insert(r.end(), W.at_.at, W.at_.at + PARAMS + 1);
     return r;
 }
-void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, const Tensor& x_prev, const Tensor& s0, const Tensor& weights,
+void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, const Tensor& x_first, const Tensor& x_prev, const Tensor& s0, const Tensor& weights,
                           const Tensor& acts, const Tensor& saved, const Tensor& y, const Tensor& sT, bool save) {
     c10::DeviceGuard guard(xb.device());
     at::AutoDispatchBelowADInplaceOrView below;
     const Block s{xb.size(0), xb.size(1), xb.size(2), H};
-    block_forward(s, xb, p, save, s.T, x_prev.numel() ? x_prev : Tensor(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
+    block_forward(s, xb, p, save, s.T, x_prev.numel() ? First(x_first, x_prev) : First(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
 }
 void traced_block_backward(const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout, int64_t H,
                            const Tensor& dx, const Tensor& flat) {
@@ -939,7 +964,8 @@ py::object short_prompt(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor
     const bool carry_here = return_state && x.scalar_type() == at::kBFloat16;   // (the carried token keeps x's own type)
     const Tensor carry = carry_here ? at::empty({B, C}, xb.options()) : return_state ? x.select(1, T - 1).clone() : Tensor();
     const Tensor ws = scratch_bytes(L.mixer_decode_workspace_bytes((int)(B * T), (int)C), xb);
-    check(L.mixer_prompt((int)B, (int)T, (int)C, (int)H, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, &weights, ptr(xb), ptr(x_prev),
+    const Tensor prev = x_prev.defined() ? x_prev.to(at::kBFloat16).contiguous() : Tensor();   // (as `step` takes it)
+    check(L.mixer_prompt((int)B, (int)T, (int)C, (int)H, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, &weights, ptr(xb), ptr(prev),
                          ptr(s0), ptr(sT), ptr(y), carry_here ? ptr(carry) : nullptr, ptr(ws), ws.numel(), stream_of(xb)));
     if (!return_state) return py::cast(y);
     return py::make_tuple(y, py::make_tuple(carry, sT));
@@ -966,8 +992,8 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     if (grad) return stateful ? py::object(py::none()) : py::cast(mixer_node(H, x, p, std::make_index_sequence<PARAMS>()));
     Tensor x_prev, s0;
     if (x_prev_) {
-        if (!x_prev_->is_cuda() || x_prev_->device() != x.device() || x_prev_->sizes() != at::IntArrayRef({s.B, s.C})) return py::none();
-        x_prev = x_prev_->to(at::kBFloat16).contiguous();
+        if (!x_prev_->is_cuda() || !floating(*x_prev_) || s.B > 65535 || x_prev_->device() != x.device() || x_prev_->sizes() != at::IntArrayRef({s.B, s.C})) return py::none();
+        x_prev = *x_prev_;
     }
     if (s0_) {
         s0 = *s0_;
@@ -988,7 +1014,7 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
         xb = at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
     }
     const BlockBuffers f(s, xb, false, T, state_type);
-    block_forward(s, xb, p, false, T, x_prev, s0, f);
+    block_forward(s, xb, p, false, T, x_prev.defined() ? First(x.select(1, 0), x_prev) : First(), s0, f);
     if (!return_state) return py::cast(f.y);
     return py::make_tuple(f.y, py::make_tuple(carry.defined() ? carry : x.select(1, T - 1).clone(), f.sT));
 }

@@ -59,7 +59,8 @@ SIGNATURES = {
     'wind_rwkv7_ddlerp_rank_supported': (_i, [_i]),
     'wind_rwkv7_ddlerp_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_ddlerp_forward': (_i, [_i] * 4 + [_vp] * 5 + [_vp] * 3 + [_vp]),
-    'wind_rwkv7_ddlerp_forward_from': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp]),
+    'wind_rwkv7_ddlerp_first_workspace_bytes': (_sz, [_i] * 2),
+    'wind_rwkv7_ddlerp_first': (_i, [_i] * 3 + [_vp] * 3 + [_sz, _vp]),
     'wind_rwkv7_pad_rows': (_i, [_i] * 4 + [_vp] * 4),
     'wind_rwkv7_neutral_rows': (_i, [_i] * 4 + [_vp] * 4),
     'wind_rwkv7_neutral_rows_keep': (_i, [_i] * 4 + [_vp] * 5),
@@ -104,6 +105,11 @@ class MixerWeights(ctypes.Structure):
 class Linear(ctypes.Structure):   # wind_rwkv7_linear
     _fields_ = [('A', _vp * 2), ('W', _vp * 2), ('lda', _ll * 2), ('ldw', _ll * 2), ('K', _i * 2), ('N', _i), ('npieces', _i),
                 ('out', _vp * 4), ('aux', _vp * 4), ('ld_out', _ll * 4), ('width', _i * 4), ('op', _i * 4)]
+
+
+class FirstTokens(ctypes.Structure):   # wind_rwkv7_first_tokens
+    _fields_ = [(n, _vp) for n in ('x', 'x_prev', 'alpha', 'L', 'R', 'beta')] + [(n, _ll) for n in ('x_seq', 'y_stream', 'y_seq')] + \
+               [('x_dtype', _i), ('param_dtype', _i)]
 
 
 class Pack(ctypes.Structure):   # wind_rwkv7_pack

@@ -34,7 +34,7 @@ LORA_RANKS = dict(mix=32, decay=64, aaa=16, kkk=16, gate=128, ma=16, mk=16)  # t
 
 
 # ---- the block as registered operators: what torch.compile records of the native path (csrc/torch_binding.cpp) ----
-_OPS.define('block_forward(Tensor x, Tensor[] params, int H, Tensor x_prev, Tensor s0, Tensor(a!) weights, Tensor(b!) acts, '
+_OPS.define('block_forward(Tensor x, Tensor[] params, int H, Tensor x_first, Tensor x_prev, Tensor s0, Tensor(a!) weights, Tensor(b!) acts, '
             'Tensor(c!) saved, Tensor(d!) y, Tensor(e!) sT, bool save) -> ()')
 _OPS.define('block_backward(Tensor x, Tensor weights, Tensor acts, Tensor saved, Tensor dy, int H, Tensor(a!) dx, '
             'Tensor(b!) flat) -> ()')
@@ -50,8 +50,9 @@ def _block_sizes(C):
     return _native.binding().block_sizes(C)
 
 
-def _block_forward(x, params, H, x_prev, s0, state_dtype, save):
-    """(y, sT, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev and s0 may be the empty stand-in."""
+def _block_forward(x, params, H, x_first, x_prev, s0, state_dtype, save):
+    """(y, sT, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev (with x_first, the first token in its own
+    type) and s0 may be the empty stand-in."""
     B, T, C = x.shape
     N = C // H
     sizes = _block_sizes(C)
@@ -59,7 +60,7 @@ def _block_forward(x, params, H, x_prev, s0, state_dtype, save):
     weights, acts = new(sizes[1 if save else 0]), new(sizes[2] * B * T)
     saved, y = new(B, H, T // 16, _saved_unit(N)), new(B, T, C)
     sT = torch.empty(B, H, N, N, dtype=state_dtype, device=x.device)
-    torch.ops.wind_rwkv7.block_forward(x, params, H, x_prev, s0, weights, acts, saved, y, sT, save)
+    torch.ops.wind_rwkv7.block_forward(x, params, H, x_first, x_prev, s0, weights, acts, saved, y, sT, save)
     return y, sT, weights, acts, saved
 
 
@@ -69,7 +70,7 @@ class Block(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, H, *params):
         none = no_state(torch.bfloat16, x.device)
-        y, _, weights, acts, saved = _block_forward(x, [p.detach() for p in params], H, none, none, torch.bfloat16, True)
+        y, _, weights, acts, saved = _block_forward(x, [p.detach() for p in params], H, none, none, none, torch.bfloat16, True)
         ctx.save_for_backward(x, weights, acts, saved)
         ctx.H = H
         ctx.params = [(tuple(p.shape), p.dtype) for p in params]
@@ -345,8 +346,8 @@ class TimeMixer(nn.Module):
         x_prev, s0 = state if state is not None else (None, None)
         none = no_state(torch.bfloat16, x.device)
         state_dtype = s0.dtype if s0 is not None else torch.float32 if state is not None or return_state else torch.bfloat16
-        y, sT, _, _, _ = _block_forward(xb, [p.detach() for p in params], self.n_head, none if x_prev is None else x_prev.bfloat16().contiguous(),
-                                        none if s0 is None else s0.contiguous(), state_dtype, False)
+        first = (none, none) if x_prev is None else (x[:, 0].contiguous(), x_prev.contiguous())
+        y, sT, _, _, _ = _block_forward(xb, [p.detach() for p in params], self.n_head, *first, none if s0 is None else s0.contiguous(), state_dtype, False)
         return (y, (x[:, -1].clone(), sT)) if return_state else y
 
     def _forward_any_length(self, x, state, return_state):
