@@ -33,7 +33,8 @@ enum {
     WIND_RWKV7_ERR_NULL_POINTER = 1,   /* a required pointer is NULL */
     WIND_RWKV7_ERR_BAD_SHAPE = 2,      /* B, T, H or C not positive, or sizes overflow: more than 2^30 chunks of 16
                                         * tokens x heads, or at head size 64 a batch element's rows of one tensor
-                                        * (T*H*64 bf16) of 2 GiB or more */
+                                        * (T*H*64 bf16) of 2 GiB or more; or a stride or an address that is not aligned
+                                        * as the entry point asks */
     WIND_RWKV7_ERR_HEAD_SIZE = 3,      /* C is not a head size these kernels were built for */
     WIND_RWKV7_ERR_SEQ_MULTIPLE = 4,   /* T is not a multiple of the chunk length (16; rwkv7_attn.py:22) */
     WIND_RWKV7_ERR_DTYPE = 5,          /* unsupported io_dtype / state_dtype */
@@ -426,7 +427,7 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
 
 /* Working copies of up to WIND_RWKV7_PACK_MAX parameters in one launch: dst [rows, cols] in dst_dtype, and, where dstT is
  * given (dst_dtype bf16, rows % 16 == 0), the transposed copy dstT[c * ldT + r] (ldT >= rows, a multiple of 8).  cols is a
- * multiple of 16 (a vector is one row); bases are 16-byte aligned. */
+ * multiple of 16 (a vector is one row); dst and dstT are 16-byte aligned, src to its element. */
 #define WIND_RWKV7_PACK_MAX 32
 typedef struct {
     const void* src;

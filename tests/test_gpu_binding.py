@@ -158,3 +158,47 @@ def test_prompt_of_any_length_equals_the_python_path(monkeypatch, T, continued):
     first = 0 if continued else 1     # from a zero state the first token's GroupNorm is ill conditioned
     assert seq_ref.rel_err(y[:, first:].float().cpu(), y0[:, first:].float().cpu()) <= 1.27e-2
     assert seq_ref.rel_err(S.cpu(), S0.cpu()) <= 1e-2
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+def test_parameters_and_gradients_that_start_anywhere(dtype):
+    """Parameters as views into one flat buffer (flat optimizers), the input and its gradient one element off a 16-byte
+    boundary: the bits of the same values in tensors of their own, for the block, prompts, steps and the two stages."""
+    from collections import namedtuple
+    from wind_rwkv.rwkv7 import TimeMixer, ddlerp, expand_loras
+    C, H, B, T = 128, 2, 2, 48
+    gen = torch.Generator().manual_seed(5)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, C), 1)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+    model = model.to(DEV, dtype)
+    off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    x, dy = (torch.randn(B, T, C, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    state = (torch.randn(B, C, generator=gen).bfloat16().to(DEV), torch.randn(B, H, 64, 64, generator=gen).to(DEV))
+    def passes(move):
+        leaf = move(x).requires_grad_()
+        y = model(leaf)
+        out = [y] + list(torch.autograd.grad(y, [leaf] + list(model.parameters()), move(dy)))
+        with torch.no_grad():
+            for n in (T, 7, 35):
+                y, st = model(move(x[:, :n].contiguous()), state=(move(state[0]), state[1].clone()), return_state=True)
+                y2, st = model.step(move(x[:, n - 1].contiguous()), (move(st[0]), st[1]))
+                out += [y, y2, *st]
+            compiled = torch.compile(model, fullgraph=True)
+            out.append(compiled(move(x)))
+        m = model
+        out += ddlerp(x, m.time_maa_x, m.time_maa_w1, m.time_maa_w2, m.time_maa)
+        a16 = x[..., :16].contiguous()
+        out += expand_loras(x, dy, a16, a16, a16, a16, m.time_kkk_w2, m.time_aaa_w2, m.ma_w2, m.mk_w2, m.time_decay, m.time_aaaaa, m.time_misc_a, m.time_misc_k, 64)
+        return [t.detach().clone() for t in out]
+    want = passes(lambda t: t.clone())
+    flat = torch.cat([torch.zeros(1, dtype=dtype, device=DEV)] + [p.detach().reshape(-1) for p in model.parameters()])
+    at = 1
+    for p in model.parameters():
+        p.data = flat[at:at + p.numel()].view(p.shape)
+        at += p.numel()
+    assert all(p.data_ptr() % 16 for p in model.parameters())
+    model.invalidate_decode_cache()
+    for i, (a, b) in enumerate(zip(passes(off), want)):
+        assert torch.equal(a, b), i

@@ -70,10 +70,13 @@ def test_group_with_two_segments_and_cut_columns(M):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
-def test_packed_weights(dtype):
+@pytest.mark.parametrize('off', [0, 1])
+def test_packed_weights(dtype, off):
+    """`off`: elements that the sources start off a 16-byte boundary."""
     from wind_rwkv import _native
     gen = torch.Generator().manual_seed(3)
-    a, b, v = (torch.randn(*s, generator=gen).to(DEV, dtype) for s in ((16, 192), (80, 192), (1, 208)))
+    a, b, v = (torch.cat([torch.zeros(off), torch.randn(s[0] * s[1], generator=gen)]).to(DEV, dtype)[off:].view(s) for s in ((16, 192), (80, 192), (1, 208)))
+    assert all((t.data_ptr() % 16 == 0) == (off == 0) for t in (a, b, v))
     dst = [torch.zeros(t.shape, device=DEV, dtype=torch.bfloat16) for t in (a, b)] + [torch.zeros(v.shape, device=DEV)]
     both = torch.zeros(192, 96, device=DEV, dtype=torch.bfloat16)             # the transposed concatenation [a; b]
     arr = (_native.Pack * 3)()

@@ -144,7 +144,7 @@ const char* wind_rwkv7_strerror(int code) {
     switch (code) {
         case WIND_RWKV7_OK: return "success";
         case WIND_RWKV7_ERR_NULL_POINTER: return "a required pointer is NULL";
-        case WIND_RWKV7_ERR_BAD_SHAPE: return "B, T, H and C must be positive and the problem must fit the index range";
+        case WIND_RWKV7_ERR_BAD_SHAPE: return "sizes must be positive and fit the index range; strides and addresses must be aligned as the entry point asks";
         case WIND_RWKV7_ERR_HEAD_SIZE: return "unsupported head size (64; the plain WKV7 entry points: multiples of 16 up to 128)";
         case WIND_RWKV7_ERR_SEQ_MULTIPLE: return "T must be a multiple of the chunk length (16)";
         case WIND_RWKV7_ERR_DTYPE: return "unsupported element type";
@@ -901,9 +901,12 @@ int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream)
         for (int d : {u.src_dtype, u.dst_dtype})
             if (d != WIND_RWKV7_BF16 && d != WIND_RWKV7_F32) return WIND_RWKV7_ERR_DTYPE;
         if (u.dstT && (u.dst_dtype != WIND_RWKV7_BF16 || u.rows % 16 != 0 || u.ldT < u.rows || u.ldT % 8 != 0)) return WIND_RWKV7_ERR_BAD_SHAPE;
-        for (const void* q : {u.src, (const void*)u.dst, (const void*)u.dstT})
+        for (const void* q : {u.dst, u.dstT})
             if (reinterpret_cast<uintptr_t>(q) % 16 != 0) return WIND_RWKV7_ERR_BAD_SHAPE;
-        P[t] = wkv::PackTensor{u.src, u.dst, u.dstT, u.rows, u.cols, (long)u.ldT, u.src_dtype == WIND_RWKV7_F32, u.dst_dtype == WIND_RWKV7_F32};
+        const uintptr_t src = reinterpret_cast<uintptr_t>(u.src);
+        if (src % (u.src_dtype == WIND_RWKV7_F32 ? 4 : 2) != 0) return WIND_RWKV7_ERR_BAD_SHAPE;
+        P[t] = wkv::PackTensor{u.src, u.dst, u.dstT, u.rows, u.cols, (long)u.ldT, u.src_dtype == WIND_RWKV7_F32, u.dst_dtype == WIND_RWKV7_F32,
+                               src % 16 == 0};
     }
     wkv::launch_pack_weights(n, P, static_cast<hipStream_t>(stream));
     return launch_status();

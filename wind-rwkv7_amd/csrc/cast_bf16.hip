@@ -73,7 +73,11 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(PackArgs g) {
     if (r < p.rows && c < p.cols) {
         const long at = (long)r * p.cols + c;
         f32x4 v[4];
-        if (p.src_f32) {
+        if (!p.src_aligned) {   // (a parameter that is a view into a larger buffer) element by element
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                v[i / 4][i % 4] = p.src_f32 ? static_cast<const float*>(p.src)[at + i] : (float)static_cast<const __bf16*>(p.src)[at + i];
+        } else if (p.src_f32) {
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.src) + at + 4 * i);
         } else {

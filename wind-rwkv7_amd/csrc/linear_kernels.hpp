@@ -56,7 +56,7 @@ struct PackTensor {
     void *dst, *dstT;
     int rows, cols;
     long ldT;
-    int src_f32, dst_f32;
+    int src_f32, dst_f32, src_aligned;   // src_aligned: to 16 bytes
 };
 constexpr int PACK_MAX_TENSORS = 32;
 void launch_pack_weights(int n, const PackTensor* tensors, hipStream_t stream);

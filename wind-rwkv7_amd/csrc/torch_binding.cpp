@@ -73,6 +73,13 @@ bool plain_param(const Tensor& t, const Tensor& like) {   // a float32 or bf16 p
     return t.defined() && (plain(t, at::kFloat) || plain(t, at::kBFloat16)) && t.device() == like.device();
 }
 
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+// x in bf16, dense and where 16-byte accesses may go (a view may start anywhere)
+Tensor dense_bf16(const Tensor& x) {
+    const Tensor t = x.to(at::kBFloat16).contiguous();
+    return aligned(t) ? t : t.clone();
+}
+
 bool differentiating(std::initializer_list<const Tensor*> ts) {
     if (!at::GradMode::is_enabled()) return false;
     for (const Tensor* t : ts)
@@ -315,12 +322,12 @@ py::object attn_ln(const Tensor& r, const Tensor& w, const Tensor& k, const Tens
 constexpr int64_t ALIGN_ELEMS_BF16 = 128, ALIGN_ELEMS_F32 = 64;   // 256 bytes
 int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
-// bf16 device pointers of the parameters: their own where they are bf16, otherwise into `flat`, which one launch fills
+// bf16 device pointers of the parameters: their own where they are bf16 and aligned, otherwise into `flat`, which one launch fills
 // (in `flat` each starts on a 256-byte boundary).  `flat` given: it was filled by the forward, only the pointers are wanted.
 std::vector<void*> bf16_pointers(const std::vector<Tensor>& params, Tensor& flat) {
     std::vector<void*> out;
     bool all_bf16 = true;
-    for (const auto& p : params) all_bf16 = all_bf16 && p.scalar_type() == at::kBFloat16;
+    for (const auto& p : params) all_bf16 = all_bf16 && p.scalar_type() == at::kBFloat16 && aligned(p);
     if (all_bf16) {
         for (const auto& p : params) out.push_back(p.data_ptr());
         return out;
@@ -856,7 +863,7 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         at::AutoDispatchBelowADInplaceOrView below;
         const Block s{x.size(0), x.size(1), x.size(2), H};
         const variable_list p{params...};
-        const Tensor xb = x.to(at::kBFloat16).contiguous();
+        const Tensor xb = dense_bf16(x);
         const BlockBuffers f(s, xb, true, s.T, at::kBFloat16);
         block_forward(s, xb, p, true, s.T, First(), Tensor(), f);
         ctx->save_for_backward({xb, f.weights, f.acts, f.saved});
@@ -876,7 +883,7 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         auto need = [&](int i) { return ctx->needs_input_grad(1 + i); };
         const ParamLayout at_(s.C);
         const Tensor dx = at::empty_like(xb), flat = at::empty({at_.at[PARAMS]}, xb.options().dtype(at::kFloat));
-        block_backward(s, xb, t[1], t[2], t[3], grads[0].contiguous(), dx, flat, need);
+        block_backward(s, xb, t[1], t[2], t[3], dense_bf16(grads[0]), dx, flat, need);
         variable_list out{Tensor(), dx.to((at::ScalarType)types[2])};
         for (int i = 0; i < PARAMS; i++) {
             if (!need(i)) {
@@ -907,13 +914,13 @@ void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, c
     c10::DeviceGuard guard(xb.device());
     at::AutoDispatchBelowADInplaceOrView below;
     const Block s{xb.size(0), xb.size(1), xb.size(2), H};
-    block_forward(s, xb, p, save, s.T, x_prev.numel() ? First(x_first, x_prev) : First(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
+    block_forward(s, dense_bf16(xb), p, save, s.T, x_prev.numel() ? First(x_first, x_prev) : First(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
 }
 void traced_block_backward(const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout, int64_t H,
                            const Tensor& dx, const Tensor& flat) {
     c10::DeviceGuard guard(xb.device());
     at::AutoDispatchBelowADInplaceOrView below;
-    block_backward({xb.size(0), xb.size(1), xb.size(2), H}, xb, weights, acts, saved, dout, dx, flat, [](int) { return true; });
+    block_backward({xb.size(0), xb.size(1), xb.size(2), H}, dense_bf16(xb), weights, acts, saved, dense_bf16(dout), dx, flat, [](int) { return true; });
 }
 
 template <size_t... I>
@@ -950,7 +957,7 @@ constexpr int64_t SHORT_PROMPT = 64, SHORT_PROMPT_ROWS = 512;
 py::object short_prompt(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& x, const variable_list& p, const Tensor& x_prev,
                         const Tensor& s0, at::ScalarType state_type, bool return_state) {
     at::AutoDispatchBelowADInplaceOrView below;
-    const Tensor xb = x.to(at::kBFloat16).contiguous();
+    const Tensor xb = dense_bf16(x);
     const WeightLayout W(C);
     const Tensor packed = at::empty({W.total[0]}, xb.options());
     pack_weights(W, p, packed, false);
@@ -964,7 +971,7 @@ py::object short_prompt(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor
     const bool carry_here = return_state && x.scalar_type() == at::kBFloat16;   // (the carried token keeps x's own type)
     const Tensor carry = carry_here ? at::empty({B, C}, xb.options()) : return_state ? x.select(1, T - 1).clone() : Tensor();
     const Tensor ws = scratch_bytes(L.mixer_decode_workspace_bytes((int)(B * T), (int)C), xb);
-    const Tensor prev = x_prev.defined() ? x_prev.to(at::kBFloat16).contiguous() : Tensor();   // (as `step` takes it)
+    const Tensor prev = x_prev.defined() ? dense_bf16(x_prev) : Tensor();   // (as `step` takes it)
     check(L.mixer_prompt((int)B, (int)T, (int)C, (int)H, state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16, &weights, ptr(xb), ptr(prev),
                          ptr(s0), ptr(sT), ptr(y), carry_here ? ptr(carry) : nullptr, ptr(ws), ws.numel(), stream_of(xb)));
     if (!return_state) return py::cast(y);
@@ -1003,15 +1010,12 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     }
     const at::ScalarType state_type = s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16;
     if (T % 16 && s.N() == 64 && T <= SHORT_PROMPT && s.B * T <= SHORT_PROMPT_ROWS) return short_prompt(s.B, T, s.C, H, x, p, x_prev, s0, state_type, return_state);
-    Tensor xb = x.to(at::kBFloat16).contiguous(), carry;
-    const bool pad = s.T != T, pad_here = pad && reinterpret_cast<uintptr_t>(xb.data_ptr()) % 16 == 0;
-    if (pad_here) {
+    Tensor xb = dense_bf16(x), carry;
+    if (s.T != T) {
         const Tensor whole = at::empty({s.B, s.T, s.C}, xb.options());
         if (return_state && x.scalar_type() == at::kBFloat16) carry = at::empty({s.B, s.C}, xb.options());   // (the carried token keeps x's own type)
         check(L.pad_rows((int)s.B, (int)T, (int)s.T, (int)s.C, ptr(xb), ptr(whole), ptr(carry), stream_of(xb)));
         xb = whole;
-    } else if (pad) {
-        xb = at::constant_pad_nd(xb, {0, 0, 0, s.T - T});
     }
     const BlockBuffers f(s, xb, false, T, state_type);
     block_forward(s, xb, p, false, T, x_prev.defined() ? First(x.select(1, 0), x_prev) : First(), s0, f);
@@ -1054,7 +1058,7 @@ py::object mixer_step(const Tensor& x, const Tensor& x_prev, const Tensor& S, co
     // the workspace belongs to the call (the allocator hands the same memory out again on this stream): two threads or
     // streams stepping one module do not share it
     const Tensor ws = scratch_bytes(L.mixer_decode_workspace_bytes((int)B, (int)C), x);
-    const Tensor xb = x.to(at::kBFloat16).contiguous(), xp = x_prev.to(at::kBFloat16).contiguous();
+    const Tensor xb = dense_bf16(x), xp = dense_bf16(x_prev);
     const Tensor y = at::empty({B, C}, xb.options()), carry = at::empty({B, C}, xb.options());
     check(L.mixer_decode((int)B, (int)C, (int)H, state_code(S), &weights, ptr(xb), ptr(xp), ptr(S), ptr(y), ptr(carry), ptr(ws), ws.numel(), stream_of(x)));
     return py::make_tuple(y, py::make_tuple(carry, S));

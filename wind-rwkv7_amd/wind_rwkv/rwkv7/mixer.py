@@ -398,6 +398,7 @@ class TimeMixer(nn.Module):
         cache = self.__dict__.get('_decode_cache')
         if cache is None or cache[0] != key:
             copies = [getattr(self, n).detach().to(torch.bfloat16).contiguous() for n in names]
+            copies = [c if c.data_ptr() % 16 == 0 else c.clone() for c in copies]   # (bf16 views into a larger buffer)
             ln = torch.stack([self.ln_x.weight, self.ln_x.bias, self.time_faaaa]).detach().float().contiguous()
             cache = self.__dict__['_decode_cache'] = (key, copies, ln, {})
         return cache
