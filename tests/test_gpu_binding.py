@@ -3,7 +3,7 @@ bits in outputs and gradients, whichever inputs ask for a gradient, and the same
 import pytest
 import torch
 
-from oracle import inputs
+from oracle import inputs, seq_ref
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda'
@@ -202,3 +202,55 @@ def test_parameters_and_gradients_that_start_anywhere(dtype):
     model.invalidate_decode_cache()
     for i, (a, b) in enumerate(zip(passes(off), want)):
         assert torch.equal(a, b), i
+
+
+def _small_model(C, H, dtype, seed=5):
+    from collections import namedtuple
+    from wind_rwkv.rwkv7 import TimeMixer
+    gen = torch.Generator().manual_seed(seed)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, C), 1)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+    return model.to(DEV, dtype), gen
+
+
+EXPANSION = ('time_kkk_w2', 'time_aaa_w2', 'ma_w2', 'mk_w2', 'time_decay', 'time_aaaaa', 'time_misc_a', 'time_misc_k')
+
+
+@pytest.mark.parametrize('compiled', [False, True])
+@pytest.mark.parametrize('wanted', [('Wo',), ('ln_x.weight',), ('Wo', 'Wv'), ('gate_w1',), ('gate_w2', 'Wr'), ('mk_w1',), ('time_aaa_w1',),
+                                    ('time_decay_w2', 'Wk'), EXPANSION[1:2], EXPANSION, ('time_maa_w2',), ('x',), ('x', 'Wo', 'ma_w1')])
+def test_a_backward_pass_stops_behind_what_is_wanted(wanted, compiled):
+    """Any choice of wanted gradients: the values are those of the whole backward (the same products; a weight gradient alone or in
+    a smaller group is cut into other token ranges, fp32 sums: 1e-5).  With the output projection alone nothing of the
+    recurrence runs or is kept."""
+    from wind_rwkv import _native
+    B, T, C, H = 2, 64, 128, 2
+    model, gen = _small_model(C, H, torch.float32)
+    x, dy = (torch.randn(B, T, C, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    params = dict(model.named_parameters())
+    leaf = x.clone().requires_grad_()
+    every = dict(zip(['x'] + list(params), torch.autograd.grad(model(leaf), [leaf] + list(params.values()), dy)))
+    for n, p in params.items():
+        p.requires_grad_(n in wanted)
+    leaf = x.clone().requires_grad_('x' in wanted)
+    torch._dynamo.reset()   # (every case is another graph of the same code)
+    fn = torch.compile(model, fullgraph=True) if compiled else model
+    fn(leaf)   # (compiled, warmed up)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    y = fn(leaf)
+    kept = torch.cuda.memory_allocated() - before
+    _native.lib().wind_rwkv7_profile_enable(1)
+    try:
+        got = dict(zip(wanted, torch.autograd.grad(y, [leaf if n == 'x' else params[n] for n in wanted], dy)))
+        import ctypes
+        ran = _native.lib().wind_rwkv7_profile_read(1, (ctypes.c_float * 16)(), 16)
+    finally:
+        _native.lib().wind_rwkv7_profile_enable(0)
+    assert (ran > 0) == (wanted != ('Wo',))   # kernels of the recurrence's backward
+    for n in wanted:
+        assert seq_ref.rel_err(got[n].float().cpu(), every[n].float().cpu()) <= 1e-5, n
+    if wanted == ('Wo',):
+        assert kept <= 2 * x.numel() * 2 + 4096         # the output and what the projection multiplied

@@ -605,13 +605,13 @@ struct Block {   // the sizes of a call
 
 // Activations of a block in one buffer; offsets in elements (all multiples of 256: rows() is a multiple of 16).
 struct Activations {
-    int64_t streams, r, k, v, g, w2, w, k2, kk, b, ya, mid, der, tg1, tw1, kk1, mk1, a1, ma1, total;
+    int64_t streams, r, k, v, g, w2, w, k2, kk, b, mid, der, tg1, tw1, kk1, mk1, a1, ma1, total;
     explicit Activations(const Block& s) {
         int64_t o = 0;
         auto take = [&](int64_t n) { const int64_t r = o; o += n; return r; };
         const int64_t M = s.rows(), P = s.plane();
         streams = take(4 * P);
-        r = take(P), k = take(P), v = take(P), g = take(P), w2 = take(P), w = take(P), k2 = take(P), kk = take(P), b = take(P), ya = take(P);
+        r = take(P), k = take(P), v = take(P), g = take(P), w2 = take(P), w = take(P), k2 = take(P), kk = take(P), b = take(P);
         mid = take(4 * R_MIX * M), der = take(4 * R_MIX * M);
         tg1 = take(R_GATE * M), tw1 = take(R_DECAY * M);
         kk1 = take(R_LORA * M), mk1 = take(R_LORA * M), a1 = take(R_LORA * M), ma1 = take(R_LORA * M);
@@ -681,17 +681,18 @@ struct WeightGrads {
 
 // What a forward pass leaves: the caller's results and what a backward pass needs.
 struct BlockBuffers {
-    Tensor weights, acts, saved, y, sT;
+    Tensor weights, acts, saved, ya, y, sT;   // ya: what the output projection multiplies
     static int64_t saved_bytes(const Block& s) { return L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()); }
     BlockBuffers(const Block& s, const Tensor& xb, bool save, int64_t valid, at::ScalarType state_type) {
         weights = at::empty({WeightLayout(s.C).total[save]}, xb.options());
         acts = at::empty({Activations(s).total}, xb.options());
         saved = scratch_bytes(saved_bytes(s), xb);
+        ya = at::empty({s.plane()}, xb.options());
         y = at::empty({s.B, valid, s.C}, xb.options());
         sT = at::empty({s.B, s.H, s.N(), s.N()}, xb.options().dtype(state_type));
     }
-    BlockBuffers(Tensor w, Tensor a, Tensor s, Tensor y_, Tensor st)
-        : weights(std::move(w)), acts(std::move(a)), saved(std::move(s)), y(std::move(y_)), sT(std::move(st)) {}
+    BlockBuffers(Tensor w, Tensor a, Tensor s, Tensor ya_, Tensor y_, Tensor st)
+        : weights(std::move(w)), acts(std::move(a)), saved(std::move(s)), ya(std::move(ya_)), y(std::move(y_)), sT(std::move(st)) {}
 };
 
 // A continued sequence's first token and the carried one before it, both float32 or both bf16 (no defined tensors: there is
@@ -763,35 +764,62 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
         const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
         check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
             B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln),
-            ptr(s0), a(A.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
+            ptr(s0), ptr(f.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
     }
     if (rest) {
         const int64_t part = kept.defined() ? kept.stride(0) : 0;
         check(L.attn_ln_tokens(B, T, H, N, whole, rest, state_code(f.sT), whole ? at_elem(kept, 0) : a(A.w), a(A.r),
                                whole ? at_elem(kept, part) : a(A.k2), a(A.v), a(A.kk), whole ? at_elem(kept, 2 * part) : a(A.b), a(A.g),
-                               at_elem(f.weights, W.ln), whole ? T - whole : T, 0, whole ? ptr(f.sT) : ptr(s0), a(A.ya), ptr(f.sT), stream));
+                               at_elem(f.weights, W.ln), whole ? T - whole : T, 0, whole ? ptr(f.sT) : ptr(s0), ptr(f.ya), ptr(f.sT), stream));
     }
     Products out;
     if (!rest) {
-        out.add(a(A.ya), w(WO), C, C), out.to(ptr(f.y), C);
+        out.add(ptr(f.ya), w(WO), C, C), out.to(ptr(f.y), C);
         out.run(M, xb);
     } else if (B <= WIND_RWKV7_LINEAR_GROUP_MAX) {   // a product per sequence: one launch, each straight to its place
-        for (int64_t b = 0; b < B; b++) out.add(a(A.ya + b * T * C), w(WO), C, C), out.to(at_elem(f.y, b * valid * C), C);
+        for (int64_t b = 0; b < B; b++) out.add(at_elem(f.ya, b * T * C), w(WO), C, C), out.to(at_elem(f.y, b * valid * C), C);
         out.run(valid, xb);
     } else {
-        out.add(a(A.ya), w(WO), C, C), out.to(a(A.streams), C);
+        out.add(ptr(f.ya), w(WO), C, C), out.to(a(A.streams), C);
         out.run(M, xb);
         check(L.pad_rows(B, T, (int)valid, C, a(A.streams), ptr(f.y), nullptr, stream));
     }
 }
 
-// dx and the gradient of every parameter (ParamLayout's places in `flat`, float32); need(i): whether parameter i's is wanted.
+// The stages of a backward pass that the wanted gradients ask for; need(i): parameter i's is wanted, x: the input's.
+struct Stages {
+    bool streams, gate, decay, expand, attn;   // down to: the four streams, the first halves of gate and decay, the LoRA expansion, WKV7
+    template <class Need>
+    Stages(bool x, const Need& need) {
+        auto any = [&](std::initializer_list<int> is) {
+            for (int i : is)
+                if (need(i)) return true;
+            return false;
+        };
+        streams = x || any({MAA_X, MAA, MAA_W1, MAA_W2});
+        gate = streams || need(GATE_W1);
+        decay = streams || any({DECAY_W1, AAA_W1, MA_W1});
+        expand = decay || any({WK, KKK_W1, MK_W1, DECAY_W2, KKK_W2, AAA_W2, MA_W2, MK_W2, DECAY, AAAAA, MISC_A, MISC_K});
+        attn = gate || expand || any({WR, WV, GATE_W2, LN_W, LN_B, FAAAA});
+    }
+};
+
+// dx and the wanted gradients of the parameters (ParamLayout's places in `flat`, float32); need(i): whether parameter i's
+// is wanted.  A stage that nothing wanted lies behind does not run; without Stages::attn only ya is there to go back through.
 template <class Need>
-void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout,
-                    const Tensor& dx, const Tensor& flat, const Need& need) {
+void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& ya,
+                    const Tensor& dout, const Stages& st, const Tensor& dx, const Tensor& flat, const Need& need) {
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
     const int64_t M = s.rows(), P = s.plane();
-    void* stream = stream_of(xb);
+    void* stream = stream_of(dout);
+    const ParamLayout G(C);
+    auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + G.at[i]; };
+    {
+        WeightGrads wg;
+        if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
+        wg.run(M, dout, stream);
+    }
+    if (!st.attn) return;
     const WeightLayout W(C);
     const Activations A(s);
     // gradients of activations: nine planes, reused as they are consumed, and the gradients of the three first halves
@@ -801,10 +829,9 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
     auto d = [&](int64_t o) -> void* { return at_elem(buf, o); };
     auto w = [&](int i) -> void* { return at_elem(weights, W.at_.at[i]); };
     auto t = [&](int64_t o) -> void* { return at_elem(weights, o); };
-    auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + W.at_.at[i]; };
     size_t ws_bytes = L.attn_ln_bwd_workspace_bytes(B, T, H, N);
-    ws_bytes = std::max(ws_bytes, L.expand_loras_bwd_workspace_bytes(B, T, C, R_LORA));
-    ws_bytes = std::max(ws_bytes, L.ddlerp_bwd_workspace_bytes(B, T, C, R_MIX));
+    if (st.expand) ws_bytes = std::max(ws_bytes, L.expand_loras_bwd_workspace_bytes(B, T, C, R_LORA));
+    if (st.streams) ws_bytes = std::max(ws_bytes, L.ddlerp_bwd_workspace_bytes(B, T, C, R_MIX));
     const Tensor ws = scratch_bytes(ws_bytes, xb);
 
     // planes: 0 dya then dw2, 1 dr, 2 dw, 3 dk', 4 dv, 5 dkk, 6 db, 7 dg, 8 dk
@@ -812,23 +839,21 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         Products p;
         p.add(ptr(dout), t(W.To), C, C), p.to(d(0), C);
         p.run(M, xb);
-        WeightGrads wg;
-        if (need(WO)) wg.add(ptr(dout), C, a(A.ya), C, g(WO));
-        wg.run(M, xb, stream);
     }
     check(L.attn_ln_backward(B, T, H, N, WIND_RWKV7_BF16, WIND_RWKV7_BF16, a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), t(W.ln), d(0),
                              ptr(saved), nullptr, d(2 * P), d(P), d(3 * P), d(4 * P), d(5 * P), d(6 * P), d(7 * P), g(LN_W), nullptr, ptr(ws),
                              ws.numel(), stream));
     B16 *dkkmk = at_elem(buf, o_kkmk), *dw1 = at_elem(buf, o_w1);
     const long long ld_din[4] = {W_KKMK, W_DECAY_AAA_MA, W_DECAY_AAA_MA, W_KKMK};
-    check(L.expand_loras_backward_to(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
-                                     w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), d(2 * P), d(3 * P), d(5 * P), d(6 * P), d(0), d(8 * P),
-                                     dkkmk, dw1 + R_DECAY, dw1 + R_DECAY + R_LORA, dkkmk + R_LORA, ld_din, g(KKK_W2), g(AAA_W2), g(MA_W2),
-                                     g(MK_W2), g(DECAY), g(AAAAA), g(MISC_A), g(MISC_K), ptr(ws), ws.numel(), stream));
+    if (st.expand)
+        check(L.expand_loras_backward_to(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
+                                         w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), d(2 * P), d(3 * P), d(5 * P), d(6 * P), d(0),
+                                         d(8 * P), dkkmk, dw1 + R_DECAY, dw1 + R_DECAY + R_LORA, dkkmk + R_LORA, ld_din, g(KKK_W2), g(AAA_W2),
+                                         g(MA_W2), g(MK_W2), g(DECAY), g(AAAAA), g(MISC_A), g(MISC_K), ptr(ws), ws.numel(), stream));
     {
         Products p;   // through the derivative of the tanh between the halves
-        p.add(d(7 * P), t(W.Tg2), C, R_GATE), p.to(d(o_g1), R_GATE, 2, a(A.tg1));
-        p.add(d(0), t(W.Tw2), C, R_DECAY), p.to(dw1, R_DECAY, 2, a(A.tw1), W_DECAY_AAA_MA);
+        if (st.gate) p.add(d(7 * P), t(W.Tg2), C, R_GATE), p.to(d(o_g1), R_GATE, 2, a(A.tg1));
+        if (st.decay) p.add(d(0), t(W.Tw2), C, R_DECAY), p.to(dw1, R_DECAY, 2, a(A.tw1), W_DECAY_AAA_MA);
         p.run(M, xb);
         WeightGrads wg;
         if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
@@ -839,10 +864,12 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
     void *dxrg = d(2 * P), *dxwa = d(5 * P), *dxk = d(3 * P), *dxv = d(6 * P);
     {
         Products p;
-        p.add(d(P), t(W.Tr), C, C), p.plus(d(o_g1), t(W.Tg1), R_GATE), p.to(dxrg, C);
-        p.add(d(8 * P), t(W.Tk), C, C), p.plus(dkkmk, t(W.Tkkmk), W_KKMK), p.to(dxk, C);
-        p.add(d(4 * P), t(W.Tv), C, C), p.to(dxv, C);
-        p.add(dw1, t(W.Tw1), W_DECAY_AAA_MA, C), p.to(dxwa, C);
+        if (st.streams) {
+            p.add(d(P), t(W.Tr), C, C), p.plus(d(o_g1), t(W.Tg1), R_GATE), p.to(dxrg, C);
+            p.add(d(8 * P), t(W.Tk), C, C), p.plus(dkkmk, t(W.Tkkmk), W_KKMK), p.to(dxk, C);
+            p.add(d(4 * P), t(W.Tv), C, C), p.to(dxv, C);
+            p.add(dw1, t(W.Tw1), W_DECAY_AAA_MA, C), p.to(dxwa, C);
+        }
         p.run(M, xb);
         WeightGrads wg;
         if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
@@ -853,8 +880,9 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         if (need(DECAY_W1) || need(AAA_W1) || need(MA_W1)) wg.add(dw1, W_DECAY_AAA_MA, a(A.streams + P), C, g(DECAY_W1));
         wg.run(M, xb, stream);
     }
-    check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), dxrg, dxwa, dxk, dxv, ptr(dx),
-                            g(MAA_X), g(MAA_W1), g(MAA_W2), g(MAA), ptr(ws), ws.numel(), stream));
+    if (st.streams)
+        check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), dxrg, dxwa, dxk, dxv, ptr(dx),
+                                g(MAA_X), g(MAA_W1), g(MAA_W2), g(MAA), ptr(ws), ws.numel(), stream));
 }
 
 struct MixerBlock : torch::autograd::Function<MixerBlock> {
@@ -864,27 +892,32 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         const Block s{x.size(0), x.size(1), x.size(2), H};
         const variable_list p{params...};
         const Tensor xb = dense_bf16(x);
-        const BlockBuffers f(s, xb, true, s.T, at::kBFloat16);
-        block_forward(s, xb, p, true, s.T, First(), Tensor(), f);
-        ctx->save_for_backward({xb, f.weights, f.acts, f.saved});
-        std::vector<int64_t> types{H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
-        for (const auto& t : p) types.push_back((int64_t)t.scalar_type());
-        ctx->saved_data["k"] = types;
+        const bool attn = Stages(x.requires_grad(), [&](int i) { return p[i].requires_grad(); }).attn;
+        const BlockBuffers f(s, xb, attn, s.T, at::kBFloat16);
+        block_forward(s, xb, p, attn, s.T, First(), Tensor(), f);
+        if (attn) ctx->save_for_backward({f.ya, xb, f.weights, f.acts, f.saved});
+        else ctx->save_for_backward({f.ya});
+        std::vector<int64_t> kept{s.B, s.T, s.C, H, L.checkpoint_interval(), (int64_t)x.scalar_type()};
+        for (const auto& t : p) kept.push_back((int64_t)t.scalar_type());
+        ctx->saved_data["k"] = kept;
         return {f.y};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-        const auto t = ctx->get_saved_variables();
-        const auto types = ctx->saved_data["k"].toIntVector();
-        const Tensor& xb = t[0];
-        const Block s{xb.size(0), xb.size(1), xb.size(2), types[0]};
-        same_interval({{}, (int)types[1], at::kBFloat16, false});
-        c10::DeviceGuard guard(xb.device());
+        auto t = ctx->get_saved_variables();
+        t.resize(5);
+        const auto kept = ctx->saved_data["k"].toIntVector();
+        const int64_t* types = kept.data() + 6;
+        const Block s{kept[0], kept[1], kept[2], kept[3]};
+        same_interval({{}, (int)kept[4], at::kBFloat16, false});
+        c10::DeviceGuard guard(t[0].device());
         at::AutoDispatchBelowADInplaceOrView below;
         auto need = [&](int i) { return ctx->needs_input_grad(1 + i); };
-        const ParamLayout at_(s.C);
-        const Tensor dx = at::empty_like(xb), flat = at::empty({at_.at[PARAMS]}, xb.options().dtype(at::kFloat));
-        block_backward(s, xb, t[1], t[2], t[3], dense_bf16(grads[0]), dx, flat, need);
-        variable_list out{Tensor(), dx.to((at::ScalarType)types[2])};
+        const bool need_x = ctx->needs_input_grad(0);
+        const Stages st(need_x, need);
+        const ParamLayout G(s.C);
+        const Tensor dx = st.streams ? at::empty_like(t[1]) : Tensor(), flat = at::empty({G.at[PARAMS]}, t[0].options().dtype(at::kFloat));
+        block_backward(s, t[1], t[2], t[3], t[4], t[0], dense_bf16(grads[0]), st, dx, flat, need);
+        variable_list out{Tensor(), need_x ? dx.to((at::ScalarType)kept[5]) : Tensor()};
         for (int i = 0; i < PARAMS; i++) {
             if (!need(i)) {
                 out.emplace_back();
@@ -894,33 +927,42 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
             std::vector<int64_t> stride(shape.size());
             int64_t n = 1;
             for (size_t k = stride.size(); k-- > 0; n *= shape[k]) stride[k] = n;
-            out.push_back(flat.as_strided(shape, stride, at_.at[i]).to((at::ScalarType)types[3 + i]));
+            out.push_back(flat.as_strided(shape, stride, G.at[i]).to((at::ScalarType)types[i]));
         }
         return out;
     }
 };
 
-// The same two passes as the registered operators that torch.compile records: every buffer comes from the caller, sized by
-// block_sizes (bf16 elements of `weights` with and without the transposed copies, of `acts` per token, of `flat`, and each
-// parameter's place in `flat`); an empty tensor stands for one that is not there.
-std::vector<int64_t> block_sizes(int64_t C) {
+// The same two passes as the registered operators that torch.compile records: every buffer comes from the caller, an empty
+// tensor stands for one that is not there.  need[0]: x's gradient is wanted, need[1 + i]: parameter i's.  block_sizes: the
+// elements of `weights` with and without the transposed copies and of `acts` per token; whether the backward goes further than
+// the output projection; the elements of `flat`, and each wanted gradient's place in it.
+std::vector<int64_t> block_sizes(int64_t C, const std::vector<bool>& need) {
+    TORCH_CHECK(need.size() == PARAMS + 1, "one flag for x and one per parameter");
+    auto of = [&](int i) { return (bool)need[1 + i]; };
     const WeightLayout W(C);
-    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16};
-    r.insert(r.end(), W.at_.at, W.at_.at + PARAMS + 1);
+    const ParamLayout G(C);
+    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16, Stages(need[0], of).attn, G.at[PARAMS]};
+    for (int i = 0; i < PARAMS; i++) r.push_back(of(i) ? G.at[i] : -1);
     return r;
 }
-void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, const Tensor& x_first, const Tensor& x_prev, const Tensor& s0, const Tensor& weights,
-                          const Tensor& acts, const Tensor& saved, const Tensor& y, const Tensor& sT, bool save) {
+void traced_block_forward(const Tensor& xb, const variable_list& p, int64_t H, const Tensor& x_first, const Tensor& x_prev, const Tensor& s0,
+                          const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& ya, const Tensor& y, const Tensor& sT,
+                          bool save) {
     c10::DeviceGuard guard(xb.device());
     at::AutoDispatchBelowADInplaceOrView below;
     const Block s{xb.size(0), xb.size(1), xb.size(2), H};
-    block_forward(s, dense_bf16(xb), p, save, s.T, x_prev.numel() ? First(x_first, x_prev) : First(), s0.numel() ? s0 : Tensor(), BlockBuffers(weights, acts, saved, y, sT));
+    block_forward(s, dense_bf16(xb), p, save, s.T, x_prev.numel() ? First(x_first, x_prev) : First(), s0.numel() ? s0 : Tensor(),
+                  BlockBuffers(weights, acts, saved, ya, y, sT));
 }
-void traced_block_backward(const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& dout, int64_t H,
-                           const Tensor& dx, const Tensor& flat) {
+void traced_block_backward(const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& ya, const Tensor& dout,
+                           int64_t H, const std::vector<bool>& need, const Tensor& dx, const Tensor& flat) {
+    TORCH_CHECK(need.size() == PARAMS + 1, "one flag for x and one per parameter");
     c10::DeviceGuard guard(xb.device());
     at::AutoDispatchBelowADInplaceOrView below;
-    block_backward({xb.size(0), xb.size(1), xb.size(2), H}, dense_bf16(xb), weights, acts, saved, dense_bf16(dout), dx, flat, [](int) { return true; });
+    auto of = [&](int i) { return (bool)need[1 + i]; };
+    block_backward({xb.size(0), xb.size(1), xb.size(2), H}, dense_bf16(xb), weights, acts, saved, ya, dense_bf16(dout), Stages(need[0], of), dx,
+                   flat, of);
 }
 
 template <size_t... I>

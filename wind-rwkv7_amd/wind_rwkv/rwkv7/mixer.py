@@ -35,9 +35,9 @@ LORA_RANKS = dict(mix=32, decay=64, aaa=16, kkk=16, gate=128, ma=16, mk=16)  # t
 
 # ---- the block as registered operators: what torch.compile records of the native path (csrc/torch_binding.cpp) ----
 _OPS.define('block_forward(Tensor x, Tensor[] params, int H, Tensor x_first, Tensor x_prev, Tensor s0, Tensor(a!) weights, Tensor(b!) acts, '
-            'Tensor(c!) saved, Tensor(d!) y, Tensor(e!) sT, bool save) -> ()')
-_OPS.define('block_backward(Tensor x, Tensor weights, Tensor acts, Tensor saved, Tensor dy, int H, Tensor(a!) dx, '
-            'Tensor(b!) flat) -> ()')
+            'Tensor(c!) saved, Tensor(d!) ya, Tensor(e!) y, Tensor(f!) sT, bool save) -> ()')
+_OPS.define('block_backward(Tensor x, Tensor weights, Tensor acts, Tensor saved, Tensor ya, Tensor dy, int H, bool[] need, '
+            'Tensor(a!) dx, Tensor(b!) flat) -> ()')
 for _name, _impl in (('block_forward', lambda *a: _native.binding().block_forward(*a)),
                      ('block_backward', lambda *a: _native.binding().block_backward(*a))):
     _OPS.impl(_name, _impl, 'CUDA')
@@ -46,47 +46,51 @@ for _name, _impl in (('block_forward', lambda *a: _native.binding().block_forwar
 
 
 @torch.compiler.assume_constant_result
-def _block_sizes(C):
-    return _native.binding().block_sizes(C)
+def _block_sizes(C, need=(False,) * 28):
+    """need: whether x's gradient and each parameter's is wanted (see block_sizes in csrc/torch_binding.cpp)."""
+    return _native.binding().block_sizes(C, need)
 
 
 def _block_forward(x, params, H, x_first, x_prev, s0, state_dtype, save):
-    """(y, sT, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev (with x_first, the first token in its own
+    """(y, sT, ya, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev (with x_first, the first token in its own
     type) and s0 may be the empty stand-in."""
     B, T, C = x.shape
     N = C // H
     sizes = _block_sizes(C)
     new = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=x.device)
     weights, acts = new(sizes[1 if save else 0]), new(sizes[2] * B * T)
-    saved, y = new(B, H, T // 16, _saved_unit(N)), new(B, T, C)
+    saved, ya, y = new(B, H, T // 16, _saved_unit(N)), new(B, T, C), new(B, T, C)
     sT = torch.empty(B, H, N, N, dtype=state_dtype, device=x.device)
-    torch.ops.wind_rwkv7.block_forward(x, params, H, x_first, x_prev, s0, weights, acts, saved, y, sT, save)
-    return y, sT, weights, acts, saved
+    torch.ops.wind_rwkv7.block_forward(x, params, H, x_first, x_prev, s0, weights, acts, saved, ya, y, sT, save)
+    return y, sT, ya, weights, acts, saved
 
 
 class Block(torch.autograd.Function):
-    """y = the block on bf16 x with the parameters in the binding's order, as torch.compile records it."""
+    """y = the block on bf16 x with the parameters in the binding's order, as torch.compile records it; need: whether x's
+    gradient and each parameter's is wanted."""
 
     @staticmethod
-    def forward(ctx, x, H, *params):
+    def forward(ctx, x, H, need, *params):
         none = no_state(torch.bfloat16, x.device)
-        y, _, weights, acts, saved = _block_forward(x, [p.detach() for p in params], H, none, none, none, torch.bfloat16, True)
-        ctx.save_for_backward(x, weights, acts, saved)
-        ctx.H = H
+        attn = bool(_block_sizes(x.shape[2], need)[3])
+        y, _, ya, *kept = _block_forward(x, [p.detach() for p in params], H, none, none, none, torch.bfloat16, attn)
+        ctx.save_for_backward(x, ya, *(kept if attn else ()))
+        ctx.H, ctx.need = H, need
         ctx.params = [(tuple(p.shape), p.dtype) for p in params]
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, weights, acts, saved = ctx.saved_tensors
-        sizes = _block_sizes(x.shape[2])
+        x, ya, *kept = ctx.saved_tensors
+        sizes = _block_sizes(x.shape[2], ctx.need)
+        none = no_state(torch.bfloat16, x.device)
         dx = torch.empty_like(x)
-        flat = torch.empty(sizes[-1], dtype=torch.float32, device=x.device)
-        torch.ops.wind_rwkv7.block_backward(x, weights, acts, saved, dy.contiguous(), ctx.H, dx, flat)
+        flat = torch.empty(sizes[4], dtype=torch.float32, device=x.device)
+        torch.ops.wind_rwkv7.block_backward(x, *(kept or [none] * 3), ya, dy.contiguous(), ctx.H, ctx.need, dx, flat)
         grads = []
-        for (shape, dtype), at in zip(ctx.params, sizes[3:]):
-            grads.append(flat[at:at + math.prod(shape)].view(shape).to(dtype))
-        return (dx, None, *grads)
+        for (shape, dtype), at in zip(ctx.params, sizes[5:]):
+            grads.append(flat[at:at + math.prod(shape)].view(shape).to(dtype) if at >= 0 else None)
+        return (dx if ctx.need[0] else None, None, None, *grads)
 
 
 def ref_attn(q, w, k, v, a, b, HEAD_SIZE):
@@ -341,13 +345,14 @@ class TimeMixer(nn.Module):
         params = [p if p.dtype in (torch.float32, torch.bfloat16) else p.float() for p in self._block_params()]
         xb = x.bfloat16().contiguous()
         if state is None and not return_state and _differentiating(x, *params):
-            return Block.apply(xb, self.n_head, *params)
+            need = tuple(t.requires_grad for t in (x, *params))
+            return Block.apply(xb, self.n_head, need, *params)
         assert not _differentiating(x, *params), 'a carried state is for inference: run under torch.no_grad()'
         x_prev, s0 = state if state is not None else (None, None)
         none = no_state(torch.bfloat16, x.device)
         state_dtype = s0.dtype if s0 is not None else torch.float32 if state is not None or return_state else torch.bfloat16
         first = (none, none) if x_prev is None else (x[:, 0].contiguous(), x_prev.contiguous())
-        y, sT, _, _, _ = _block_forward(xb, [p.detach() for p in params], self.n_head, *first, none if s0 is None else s0.contiguous(), state_dtype, False)
+        y, sT, *_ = _block_forward(xb, [p.detach() for p in params], self.n_head, *first, none if s0 is None else s0.contiguous(), state_dtype, False)
         return (y, (x[:, -1].clone(), sT)) if return_state else y
 
     def _forward_any_length(self, x, state, return_state):
