@@ -224,7 +224,7 @@ EXPANSION = ('time_kkk_w2', 'time_aaa_w2', 'ma_w2', 'mk_w2', 'time_decay', 'time
 def test_a_backward_pass_stops_behind_what_is_wanted(wanted, compiled):
     """Any choice of wanted gradients: the values are those of the whole backward (the same products; a weight gradient alone or in
     a smaller group is cut into other token ranges, fp32 sums: 1e-5).  With the output projection alone nothing of the
-    recurrence runs or is kept."""
+    recurrence runs or is kept, and the buffer handed out holds the wanted gradients only."""
     from wind_rwkv import _native
     B, T, C, H = 2, 64, 128, 2
     model, gen = _small_model(C, H, torch.float32)
@@ -254,3 +254,21 @@ def test_a_backward_pass_stops_behind_what_is_wanted(wanted, compiled):
         assert seq_ref.rel_err(got[n].float().cpu(), every[n].float().cpu()) <= 1e-5, n
     if wanted == ('Wo',):
         assert kept <= 2 * x.numel() * 2 + 4096         # the output and what the projection multiplied
+        if not compiled:
+            assert got['Wo'].untyped_storage().nbytes() == 4 * C * C
+
+
+@pytest.mark.parametrize('mixed', [False, True])
+def test_gradients_of_bf16_parameters_are_converted_once(mixed):
+    model, gen = _small_model(128, 2, torch.bfloat16)
+    if mixed:
+        model.ln_x.float()
+    x, dy = (torch.randn(2, 32, 128, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    params = list(model.parameters())
+    grads = torch.autograd.grad(model(x), params, dy)
+    assert all(g.dtype == p.dtype and g.shape == p.shape and g.is_contiguous() for g, p in zip(grads, params))
+    assert len({g.untyped_storage().data_ptr() for g in grads}) == (2 if mixed else 1)
+    for p in params:
+        p.data = p.data.float()
+    for a, b in zip(grads, torch.autograd.grad(model(x), params, dy)):
+        assert torch.equal(a, b.to(a.dtype))

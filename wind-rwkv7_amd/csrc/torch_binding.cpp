@@ -804,7 +804,41 @@ struct Stages {
     }
 };
 
-// dx and the wanted gradients of the parameters (ParamLayout's places in `flat`, float32); need(i): whether parameter i's
+// Where the gradients lie, float32: the wanted ones in one buffer, in `at` from its start (the matrices that one product
+// computes together are neighbours, wanted or not); the others that a stage writes all the same behind them, in a scratch
+// buffer (offsets from `kept` on).
+struct GradLayout {
+    int64_t at[PARAMS], kept = 0, total = 0;
+    template <class Need>
+    GradLayout(int64_t C, const Need& need) {
+        static const std::vector<int> groups[] = {{WR}, {WK}, {WV}, {WO}, {GATE_W1}, {KKK_W1, MK_W1}, {DECAY_W1, AAA_W1, MA_W1}, {GATE_W2}, {DECAY_W2},
+                                                  {MAA_W1}, {MAA_W2}, {KKK_W2}, {MK_W2}, {AAA_W2}, {MA_W2}, {MAA_X}, {MAA}, {DECAY}, {AAAAA}, {MISC_A},
+                                                  {MISC_K}, {LN_W, LN_B, FAAAA}};
+        for (bool wanted : {true, false}) {
+            for (const auto& g : groups) {
+                bool any = false;
+                for (int i : g) any = any || need(i);
+                if (any != wanted) continue;
+                // (a weight gradient of the products that nobody wants is not computed)
+                if (!wanted && (g[0] == WR || g[0] == WK || g[0] == WV || g[0] == WO || g[0] == GATE_W1 || g[0] == KKK_W1 || g[0] == DECAY_W1 ||
+                                g[0] == GATE_W2 || g[0] == DECAY_W2))
+                    continue;
+                for (int i : g) at[i] = total, total += c10::multiply_integers(param_shape(i, C));
+            }
+            if (wanted) kept = total;
+        }
+    }
+    // the gradient of parameter i as its caller takes it: a view of the buffer of the wanted ones in that type
+    static Tensor view(const Tensor& flat, int i, int64_t C, int64_t offset) {
+        const auto shape = param_shape(i, C);
+        std::vector<int64_t> stride(shape.size());
+        int64_t n = 1;
+        for (size_t k = stride.size(); k-- > 0; n *= shape[k]) stride[k] = n;
+        return flat.as_strided(shape, stride, offset);
+    }
+};
+
+// dx and the wanted gradients of the parameters (in `flat`, GradLayout's first `kept` floats); need(i): whether parameter i's
 // is wanted.  A stage that nothing wanted lies behind does not run; without Stages::attn only ya is there to go back through.
 template <class Need>
 void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, const Tensor& acts, const Tensor& saved, const Tensor& ya,
@@ -812,14 +846,19 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
     const int64_t M = s.rows(), P = s.plane();
     void* stream = stream_of(dout);
-    const ParamLayout G(C);
-    auto g = [&](int i) -> void* { return static_cast<float*>(flat.data_ptr()) + G.at[i]; };
+    const GradLayout G(C, need);
+    Tensor unwanted;
+    auto g = [&](int i) -> void* {
+        const bool kept = G.at[i] < G.kept;
+        return static_cast<float*>((kept ? flat : unwanted).data_ptr()) + G.at[i] - (kept ? 0 : G.kept);
+    };
     {
         WeightGrads wg;
         if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
         wg.run(M, dout, stream);
     }
     if (!st.attn) return;
+    if (G.total > G.kept) unwanted = at::empty({G.total - G.kept}, flat.options());
     const WeightLayout W(C);
     const Activations A(s);
     // gradients of activations: nine planes, reused as they are consumed, and the gradients of the three first halves
@@ -914,20 +953,19 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
         auto need = [&](int i) { return ctx->needs_input_grad(1 + i); };
         const bool need_x = ctx->needs_input_grad(0);
         const Stages st(need_x, need);
-        const ParamLayout G(s.C);
-        const Tensor dx = st.streams ? at::empty_like(t[1]) : Tensor(), flat = at::empty({G.at[PARAMS]}, t[0].options().dtype(at::kFloat));
+        const GradLayout G(s.C, need);
+        const Tensor dx = st.streams ? at::empty_like(t[1]) : Tensor(), flat = at::empty({G.kept}, t[0].options().dtype(at::kFloat));
         block_backward(s, t[1], t[2], t[3], t[4], t[0], dense_bf16(grads[0]), st, dx, flat, need);
         variable_list out{Tensor(), need_x ? dx.to((at::ScalarType)kept[5]) : Tensor()};
+        Tensor flat16;   // bf16 parameters: one conversion of the whole buffer
         for (int i = 0; i < PARAMS; i++) {
             if (!need(i)) {
                 out.emplace_back();
                 continue;
             }
-            const auto shape = param_shape(i, s.C);
-            std::vector<int64_t> stride(shape.size());
-            int64_t n = 1;
-            for (size_t k = stride.size(); k-- > 0; n *= shape[k]) stride[k] = n;
-            out.push_back(flat.as_strided(shape, stride, G.at[i]).to((at::ScalarType)types[i]));
+            const bool f32 = types[i] == (int64_t)at::kFloat;
+            if (!f32 && !flat16.defined()) flat16 = flat.to(at::kBFloat16);
+            out.push_back(GradLayout::view(f32 ? flat : flat16, i, s.C, G.at[i]));
         }
         return out;
     }
@@ -941,8 +979,8 @@ std::vector<int64_t> block_sizes(int64_t C, const std::vector<bool>& need) {
     TORCH_CHECK(need.size() == PARAMS + 1, "one flag for x and one per parameter");
     auto of = [&](int i) { return (bool)need[1 + i]; };
     const WeightLayout W(C);
-    const ParamLayout G(C);
-    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16, Stages(need[0], of).attn, G.at[PARAMS]};
+    const GradLayout G(C, of);
+    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16, Stages(need[0], of).attn, G.kept};
     for (int i = 0; i < PARAMS; i++) r.push_back(of(i) ? G.at[i] : -1);
     return r;
 }
