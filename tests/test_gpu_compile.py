@@ -140,3 +140,26 @@ def test_compiled_operators_follow_a_changing_shape():
                 res.append([o.detach() for o in outs] + [x.grad for x in leaves])
             for i, (x, y) in enumerate(zip(*res)):
                 assert torch.equal(x, y), f'B={B} T={T}: compiled result {i} differs'
+
+
+@pytest.mark.parametrize('grad', [False, True])
+def test_blocks_of_several_widths_compile_in_one_process(grad):
+    """The second width makes the tracer take the number of channels as symbolic: it compiles all the same, whole, and equals
+    the eager block."""
+    from collections import namedtuple
+    from wind_rwkv.rwkv7 import TimeMixer
+    torch._dynamo.reset()
+    gen = torch.Generator().manual_seed(2)
+    for C, H in ((128, 2), (256, 4), (192, 3)):
+        model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, H, C), 1)
+        with torch.no_grad():
+            for p in model.parameters():
+                p.copy_(torch.randn(p.shape, generator=gen) * 0.1)
+        model = model.to(DEV)
+        x = torch.randn(2, 32, C, generator=gen).bfloat16().to(DEV).requires_grad_(grad)
+        with torch.set_grad_enabled(grad):
+            want, got = model(x), torch.compile(model, fullgraph=True)(x)
+        assert torch.equal(got, want)
+        if grad:
+            for a, b in zip(torch.autograd.grad(want.sum(), [x, *model.parameters()]), torch.autograd.grad(got.sum(), [x, *model.parameters()])):
+                assert torch.equal(a, b)

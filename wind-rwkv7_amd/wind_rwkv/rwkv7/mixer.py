@@ -51,10 +51,10 @@ def _block_sizes(C, need=(False,) * 28):
     return _native.binding().block_sizes(C, need)
 
 
-def _block_forward(x, params, H, x_first, x_prev, s0, state_dtype, save):
+def _block_forward(x, params, C, H, x_first, x_prev, s0, state_dtype, save):
     """(y, sT, ya, weights, acts, saved) of one block on bf16 x [B,T,C]; x_prev (with x_first, the first token in its own
-    type) and s0 may be the empty stand-in."""
-    B, T, C = x.shape
+    type) and s0 may be the empty stand-in.  (C is the module's own number: x's may be symbolic to the tracer.)"""
+    B, T, _ = x.shape
     N = C // H
     sizes = _block_sizes(C)
     new = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=x.device)
@@ -70,19 +70,19 @@ class Block(torch.autograd.Function):
     gradient and each parameter's is wanted."""
 
     @staticmethod
-    def forward(ctx, x, H, need, *params):
+    def forward(ctx, x, C, H, need, *params):
         none = no_state(torch.bfloat16, x.device)
-        attn = bool(_block_sizes(x.shape[2], need)[3])
-        y, _, ya, *kept = _block_forward(x, [p.detach() for p in params], H, none, none, none, torch.bfloat16, attn)
+        attn = bool(_block_sizes(C, need)[3])
+        y, _, ya, *kept = _block_forward(x, [p.detach() for p in params], C, H, none, none, none, torch.bfloat16, attn)
         ctx.save_for_backward(x, ya, *(kept if attn else ()))
-        ctx.H, ctx.need = H, need
+        ctx.C, ctx.H, ctx.need = C, H, need
         ctx.params = [(tuple(p.shape), p.dtype) for p in params]
         return y
 
     @staticmethod
     def backward(ctx, dy):
         x, ya, *kept = ctx.saved_tensors
-        sizes = _block_sizes(x.shape[2], ctx.need)
+        sizes = _block_sizes(ctx.C, ctx.need)
         none = no_state(torch.bfloat16, x.device)
         dx = torch.empty_like(x)
         flat = torch.empty(sizes[4], dtype=torch.float32, device=x.device)
@@ -90,7 +90,7 @@ class Block(torch.autograd.Function):
         grads = []
         for (shape, dtype), at in zip(ctx.params, sizes[5:]):
             grads.append(flat[at:at + math.prod(shape)].view(shape).to(dtype) if at >= 0 else None)
-        return (dx if ctx.need[0] else None, None, None, *grads)
+        return (dx if ctx.need[0] else None, None, None, None, *grads)
 
 
 def ref_attn(q, w, k, v, a, b, HEAD_SIZE):
@@ -346,13 +346,13 @@ class TimeMixer(nn.Module):
         xb = x.bfloat16().contiguous()
         if state is None and not return_state and _differentiating(x, *params):
             need = tuple(t.requires_grad for t in (x, *params))
-            return Block.apply(xb, self.n_head, need, *params)
+            return Block.apply(xb, self.n_embd, self.n_head, need, *params)
         assert not _differentiating(x, *params), 'a carried state is for inference: run under torch.no_grad()'
         x_prev, s0 = state if state is not None else (None, None)
         none = no_state(torch.bfloat16, x.device)
         state_dtype = s0.dtype if s0 is not None else torch.float32 if state is not None or return_state else torch.bfloat16
         first = (none, none) if x_prev is None else (x[:, 0].contiguous(), x_prev.contiguous())
-        y, sT, *_ = _block_forward(xb, [p.detach() for p in params], self.n_head, *first, none if s0 is None else s0.contiguous(), state_dtype, False)
+        y, sT, *_ = _block_forward(xb, [p.detach() for p in params], self.n_embd, self.n_head, *first, none if s0 is None else s0.contiguous(), state_dtype, False)
         return (y, (x[:, -1].clone(), sT)) if return_state else y
 
     def _forward_any_length(self, x, state, return_state):
