@@ -272,3 +272,27 @@ def test_gradients_of_bf16_parameters_are_converted_once(mixed):
         p.data = p.data.float()
     for a, b in zip(grads, torch.autograd.grad(model(x), params, dy)):
         assert torch.equal(a, b.to(a.dtype))
+
+
+@pytest.mark.parametrize('T', [1024, 1003])
+def test_memory_of_a_pass_without_gradients(T):
+    """Nine planes of activations, what the output projection multiplies, the output, the LoRA activations, the recurrence's
+    scratch and the weights' copies; a ragged prompt also its padded input and the sequences it does not cut in place.  (All
+    planes held to the end: 3.5 planes more.)"""
+    from wind_rwkv import _native
+    B, C, H = 2, 768, 12
+    model, gen = _small_model(C, H, torch.float32)
+    x = torch.randn(B, T, C, generator=gen).bfloat16().to(DEV)
+    Tp = -(-T // 16) * 16
+    plane = 2 * B * Tp * C
+    saved = _native.lib().wind_rwkv7_attn_ln_saved_bytes(B, Tp, H, 64) + _native.lib().wind_rwkv7_attn_ln_fwd_workspace_bytes(B, Tp, H, 64)
+    weights = 2 * sum(p.numel() for p in model.parameters()) + 12 * C
+    loras = 2 * B * Tp * (8 * 32 + 128 + 64 + 64)
+    with torch.no_grad():
+        model(x, return_state=True)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        model(x, return_state=True)
+        peak = torch.cuda.max_memory_allocated() - base
+    assert peak <= (11 + (T != Tp)) * plane + saved + weights + loras + 4 * B * H * 4096 + 3 * 32 * B * C + (2 << 20)

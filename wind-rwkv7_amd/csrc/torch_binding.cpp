@@ -603,15 +603,18 @@ struct Block {   // the sizes of a call
     int64_t plane() const { return rows() * C; }
 };
 
-// Activations of a block in one buffer; offsets in elements (all multiples of 256: rows() is a multiple of 16).
+// Activations of a block in one buffer; offsets in elements (all multiples of 256: rows() is a multiple of 16).  Where no
+// backward pass asks for them, what is made after the streams are multiplied takes their place: nine planes for thirteen.
 struct Activations {
     int64_t streams, r, k, v, g, w2, w, k2, kk, b, mid, der, tg1, tw1, kk1, mk1, a1, ma1, total;
-    explicit Activations(const Block& s) {
+    Activations(const Block& s, bool save) {
         int64_t o = 0;
         auto take = [&](int64_t n) { const int64_t r = o; o += n; return r; };
         const int64_t M = s.rows(), P = s.plane();
         streams = take(4 * P);
-        r = take(P), k = take(P), v = take(P), g = take(P), w2 = take(P), w = take(P), k2 = take(P), kk = take(P), b = take(P);
+        r = take(P), k = take(P), v = take(P), kk = take(P), b = take(P);
+        g = save ? take(P) : streams, w2 = save ? take(P) : streams + P, w = save ? take(P) : streams + 2 * P;
+        k2 = save ? take(P) : streams + 3 * P;
         mid = take(4 * R_MIX * M), der = take(4 * R_MIX * M);
         tg1 = take(R_GATE * M), tw1 = take(R_DECAY * M);
         kk1 = take(R_LORA * M), mk1 = take(R_LORA * M), a1 = take(R_LORA * M), ma1 = take(R_LORA * M);
@@ -685,7 +688,7 @@ struct BlockBuffers {
     static int64_t saved_bytes(const Block& s) { return L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()); }
     BlockBuffers(const Block& s, const Tensor& xb, bool save, int64_t valid, at::ScalarType state_type) {
         weights = at::empty({WeightLayout(s.C).total[save]}, xb.options());
-        acts = at::empty({Activations(s).total}, xb.options());
+        acts = at::empty({Activations(s, save).total}, xb.options());
         saved = scratch_bytes(saved_bytes(s), xb);
         ya = at::empty({s.plane()}, xb.options());
         y = at::empty({s.B, valid, s.C}, xb.options());
@@ -730,7 +733,7 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
     const int64_t M = s.rows(), P = s.plane();
     void* stream = stream_of(xb);
     const WeightLayout W(C);
-    const Activations A(s);
+    const Activations A(s, save);
     pack_weights(W, p, f.weights, save);
     auto a = [&](int64_t o) -> void* { return at_elem(f.acts, o); };
     auto w = [&](int i) -> void* { return at_elem(f.weights, W.at_.at[i]); };
@@ -780,9 +783,9 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
         for (int64_t b = 0; b < B; b++) out.add(at_elem(f.ya, b * T * C), w(WO), C, C), out.to(at_elem(f.y, b * valid * C), C);
         out.run(valid, xb);
     } else {
-        out.add(ptr(f.ya), w(WO), C, C), out.to(a(A.streams), C);
+        out.add(ptr(f.ya), w(WO), C, C), out.to(a(A.w), C);   // (w is done with)
         out.run(M, xb);
-        check(L.pad_rows(B, T, (int)valid, C, a(A.streams), ptr(f.y), nullptr, stream));
+        check(L.pad_rows(B, T, (int)valid, C, a(A.w), ptr(f.y), nullptr, stream));
     }
 }
 
@@ -860,7 +863,7 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
     if (!st.attn) return;
     if (G.total > G.kept) unwanted = at::empty({G.total - G.kept}, flat.options());
     const WeightLayout W(C);
-    const Activations A(s);
+    const Activations A(s, true);
     // gradients of activations: nine planes, reused as they are consumed, and the gradients of the three first halves
     const int64_t o_g1 = 9 * P, o_kkmk = o_g1 + R_GATE * M, o_w1 = o_kkmk + W_KKMK * M, total = o_w1 + W_DECAY_AAA_MA * M;
     const Tensor buf = at::empty({total}, xb.options());
@@ -973,14 +976,14 @@ struct MixerBlock : torch::autograd::Function<MixerBlock> {
 
 // The same two passes as the registered operators that torch.compile records: every buffer comes from the caller, an empty
 // tensor stands for one that is not there.  need[0]: x's gradient is wanted, need[1 + i]: parameter i's.  block_sizes: the
-// elements of `weights` with and without the transposed copies and of `acts` per token; whether the backward goes further than
+// elements of `weights` without and with the transposed copies and of `acts` per token without and with a backward; whether the backward goes further than
 // the output projection; the elements of `flat`, and each wanted gradient's place in it.
 std::vector<int64_t> block_sizes(int64_t C, const std::vector<bool>& need) {
     TORCH_CHECK(need.size() == PARAMS + 1, "one flag for x and one per parameter");
     auto of = [&](int i) { return (bool)need[1 + i]; };
     const WeightLayout W(C);
     const GradLayout G(C, of);
-    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}).total / 16, Stages(need[0], of).attn, G.kept};
+    std::vector<int64_t> r{W.total[0], W.total[1], Activations({1, 16, C, 1}, false).total / 16, Activations({1, 16, C, 1}, true).total / 16, Stages(need[0], of).attn, G.kept};
     for (int i = 0; i < PARAMS; i++) r.push_back(of(i) ? G.at[i] : -1);
     return r;
 }

@@ -58,7 +58,7 @@ def _block_forward(x, params, C, H, x_first, x_prev, s0, state_dtype, save):
     N = C // H
     sizes = _block_sizes(C)
     new = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device=x.device)
-    weights, acts = new(sizes[1 if save else 0]), new(sizes[2] * B * T)
+    weights, acts = new(sizes[1 if save else 0]), new(sizes[3 if save else 2] * B * T)
     saved, ya, y = new(B, H, T // 16, _saved_unit(N)), new(B, T, C), new(B, T, C)
     sT = torch.empty(B, H, N, N, dtype=state_dtype, device=x.device)
     torch.ops.wind_rwkv7.block_forward(x, params, H, x_first, x_prev, s0, weights, acts, saved, ya, y, sT, save)
@@ -72,7 +72,7 @@ class Block(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, C, H, need, *params):
         none = no_state(torch.bfloat16, x.device)
-        attn = bool(_block_sizes(C, need)[3])
+        attn = bool(_block_sizes(C, need)[4])
         y, _, ya, *kept = _block_forward(x, [p.detach() for p in params], C, H, none, none, none, torch.bfloat16, attn)
         ctx.save_for_backward(x, ya, *(kept if attn else ()))
         ctx.C, ctx.H, ctx.need = C, H, need
@@ -85,10 +85,10 @@ class Block(torch.autograd.Function):
         sizes = _block_sizes(ctx.C, ctx.need)
         none = no_state(torch.bfloat16, x.device)
         dx = torch.empty_like(x)
-        flat = torch.empty(sizes[4], dtype=torch.float32, device=x.device)
+        flat = torch.empty(sizes[5], dtype=torch.float32, device=x.device)
         torch.ops.wind_rwkv7.block_backward(x, *(kept or [none] * 3), ya, dy.contiguous(), ctx.H, ctx.need, dx, flat)
         grads = []
-        for (shape, dtype), at in zip(ctx.params, sizes[5:]):
+        for (shape, dtype), at in zip(ctx.params, sizes[6:]):
             grads.append(flat[at:at + math.prod(shape)].view(shape).to(dtype) if at >= 0 else None)
         return (dx if ctx.need[0] else None, None, None, None, *grads)
 
