@@ -296,3 +296,28 @@ def test_memory_of_a_pass_without_gradients(T):
         model(x, return_state=True)
         peak = torch.cuda.max_memory_allocated() - base
     assert peak <= (11 + (T != Tp)) * plane + saved + weights + loras + 4 * B * H * 4096 + 3 * 32 * B * C + (2 << 20)
+
+
+@pytest.mark.parametrize('stage', ['ddlerp', 'expand_loras', 'block'])
+def test_float32_parameters_may_be_written_to_before_the_backward_pass(stage):
+    """What a backward pass multiplies with is the bf16 copies that the forward made, as in the Python Functions: an optimizer
+    step or a swap of weights in between changes nothing and is no error."""
+    from wind_rwkv.rwkv7 import ddlerp, expand_loras
+    model, gen = _small_model(128, 2, torch.float32)
+    x = torch.randn(2, 32, 128, generator=gen).bfloat16().to(DEV)
+    a16 = torch.randn(2, 32, 16, generator=gen).bfloat16().to(DEV)
+    names = {'ddlerp': ('time_maa_x', 'time_maa_w1', 'time_maa_w2', 'time_maa'), 'expand_loras': EXPANSION,
+             'block': [n for n, _ in model.named_parameters()]}[stage]
+    params = [dict(model.named_parameters())[n] for n in names]
+    leaf = x.clone().requires_grad_()
+    grads = []
+    for write in (False, True):
+        y = {'ddlerp': lambda: ddlerp(leaf, *params), 'expand_loras': lambda: expand_loras(leaf, x, a16, a16, a16, a16, *params, 64),
+             'block': lambda: (model(leaf),)}[stage]()
+        if write:
+            with torch.no_grad():
+                for p in params:
+                    p.mul_(2)
+        grads.append(torch.autograd.grad(y, [leaf] + params, [x] * len(y)))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)

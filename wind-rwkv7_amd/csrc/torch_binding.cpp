@@ -322,34 +322,51 @@ py::object attn_ln(const Tensor& r, const Tensor& w, const Tensor& k, const Tens
 constexpr int64_t ALIGN_ELEMS_BF16 = 128, ALIGN_ELEMS_F32 = 64;   // 256 bytes
 int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
-// bf16 device pointers of the parameters: their own where they are bf16 and aligned, otherwise into `flat`, which one launch fills
-// (in `flat` each starts on a 256-byte boundary).  `flat` given: it was filled by the forward, only the pointers are wanted.
-std::vector<void*> bf16_pointers(const std::vector<Tensor>& params, Tensor& flat) {
-    std::vector<void*> out;
-    bool all_bf16 = true;
-    for (const auto& p : params) all_bf16 = all_bf16 && p.scalar_type() == at::kBFloat16 && aligned(p);
-    if (all_bf16) {
-        for (const auto& p : params) out.push_back(p.data_ptr());
-        return out;
-    }
-    std::vector<long long> offset, numel;
-    std::vector<const void*> src;
-    std::vector<int> dtype;
-    long long total = 0;
-    for (const auto& p : params) {
-        offset.push_back(total);
-        numel.push_back(p.numel());
-        src.push_back(p.data_ptr());
-        dtype.push_back(p.scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16);
-        total += round_up(p.numel(), ALIGN_ELEMS_BF16);
-    }
-    if (!flat.defined()) {
+// The parameters as bf16: the tensors themselves where all of them are, and aligned, otherwise copies in one buffer that one
+// launch fills (each on a 256-byte boundary).  A node saves what it multiplied - `saved` - and not a parameter it has a copy
+// of, which may be written to before the backward pass.
+struct Bf16Params {
+    variable_list own;   // the parameters, or none
+    Tensor flat;         // the copies, or undefined
+    explicit Bf16Params(const variable_list& params) {
+        bool direct = true;
+        for (const auto& p : params) direct = direct && p.scalar_type() == at::kBFloat16 && aligned(p);
+        if (direct) {
+            own = params;
+            return;
+        }
+        std::vector<long long> offset, numel;
+        std::vector<const void*> src;
+        std::vector<int> dtype;
+        long long total = 0;
+        for (const auto& p : params) {
+            offset.push_back(total);
+            numel.push_back(p.numel());
+            src.push_back(p.data_ptr());
+            dtype.push_back(p.scalar_type() == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16);
+            total += round_up(p.numel(), ALIGN_ELEMS_BF16);
+        }
         flat = at::empty({total}, params[0].options().dtype(at::kBFloat16));
         check(L.cast_to_bf16((int)params.size(), src.data(), dtype.data(), numel.data(), offset.data(), flat.data_ptr(), stream_of(flat)));
     }
-    for (long long o : offset) out.push_back(static_cast<char*>(flat.data_ptr()) + 2 * o);
-    return out;
-}
+    // from the tail of a node's saved variables: one flat buffer, or the parameters
+    Bf16Params(variable_list::const_iterator first, variable_list::const_iterator last) {
+        if (last - first == 1) flat = *first;
+        else own.assign(first, last);
+    }
+    variable_list saved() const { return flat.defined() ? variable_list{flat} : own; }
+    std::vector<void*> pointers(std::initializer_list<int64_t> numel) const {
+        std::vector<void*> out;
+        if (!flat.defined())
+            for (const auto& p : own) out.push_back(p.data_ptr());
+        int64_t o = 0;
+        for (int64_t n : numel) {
+            if (flat.defined()) out.push_back(static_cast<char*>(flat.data_ptr()) + 2 * o);
+            o += round_up(n, ALIGN_ELEMS_BF16);
+        }
+        return out;
+    }
+};
 
 // float32 gradients of tensors of the given shapes in one buffer, and the tensors to hand back: views of it, or of one
 // bf16 copy of it where the parameters are bf16.
@@ -387,30 +404,33 @@ struct DDLerp : torch::autograd::Function<DDLerp> {
                                  const Tensor& beta) {
         at::AutoDispatchBelowADInplaceOrView below;   // (the four outputs are slices of one buffer, not views to autograd)
         const int B = x.size(0), T = x.size(1), C = x.size(2), D = R.size(2);
-        Tensor flat;
-        const auto p = bf16_pointers({alpha, Lw, R, beta}, flat);
+        const Bf16Params params({alpha, Lw, R, beta});
+        const auto p = params.pointers({C, 4 * D * C, 4 * D * C, 4 * C});
         Tensor y = at::empty({4, B, T, C}, x.options()), mid = at::empty({2, B, T, 4 * D}, x.options());
         void* bder = static_cast<char*>(mid.data_ptr()) + mid.numel();   // the second half (2 bytes an element)
         check(L.ddlerp_forward(B, T, C, D, ptr(x), p[0], p[1], p[2], p[3], ptr(mid), bder, ptr(y), stream_of(x)));
-        ctx->save_for_backward({x, alpha, Lw, R, beta, flat, mid});
+        variable_list save{x, mid};
+        for (const auto& t : params.saved()) save.push_back(t);
+        ctx->save_for_backward(save);
+        ctx->saved_data["type"] = alpha.scalar_type();
         return {y.select(0, 0), y.select(0, 1), y.select(0, 2), y.select(0, 3)};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const auto t = ctx->get_saved_variables();
         const Tensor& x = t[0];
-        const int B = x.size(0), T = x.size(1), C = x.size(2), D = t[3].size(2);
+        const Tensor& mid = t[1];
+        const int B = x.size(0), T = x.size(1), C = x.size(2), D = mid.size(3) / 4;
         c10::DeviceGuard guard(x.device());
-        Tensor flat = t[5], dy[4];
-        const auto p = bf16_pointers({t[1], t[2], t[3], t[4]}, flat);
+        Tensor dy[4];
+        const auto p = Bf16Params(t.begin() + 2, t.end()).pointers({C, 4 * D * C, 4 * D * C, 4 * C});
         for (int i = 0; i < 4; i++) dy[i] = contiguous_or_zeros(grads[i], x);
         Tensor dx = at::empty_like(x);
         const FlatGrads g({{C}, {4 * D, C}, {4, C, D}, {4, 1, 1, C}}, x);
         const Tensor ws = scratch_bytes(L.ddlerp_bwd_workspace_bytes(B, T, C, D), x);
-        const Tensor& mid = t[6];
         check(L.ddlerp_backward(B, T, C, D, ptr(x), p[0], p[1], p[2], p[3], ptr(mid), static_cast<char*>(mid.data_ptr()) + mid.numel(),
                                 ptr(dy[0]), ptr(dy[1]), ptr(dy[2]), ptr(dy[3]), ptr(dx), g.p(0), g.p(1), g.p(2), g.p(3), ptr(ws),
                                 ws.numel(), stream_of(x)));
-        variable_list out = g.tensors(t[1].scalar_type());
+        variable_list out = g.tensors(ctx->saved_data["type"].toScalarType());
         out.insert(out.begin(), dx);
         return out;
     }
@@ -440,26 +460,27 @@ struct ExpandLoras : torch::autograd::Function<ExpandLoras> {
         at::AutoDispatchBelowADInplaceOrView below;
         const variable_list in{tensors...};
         const int B = in[0].size(0), T = in[0].size(1), C = in[0].size(2), D = in[2].size(2);
-        variable_list save(in);
+        variable_list save(in.begin(), in.begin() + 6);
         for (int i = 2; i < 6; i++) save[i] = in[i].contiguous();
-        Tensor flat;
-        const auto p = bf16_pointers(std::vector<Tensor>(in.begin() + 6, in.end()), flat);
+        const Bf16Params params(variable_list(in.begin() + 6, in.end()));
+        const auto p = params.pointers({C * D, C * D, C * D, C * D, C, C, C, C});
         variable_list out(4);
         for (auto& o : out) o = at::empty_like(in[0]);
         check(L.expand_loras_forward(B, T, C, D, (int)head_size, ptr(in[0]), ptr(in[1]), ptr(save[2]), ptr(save[3]), ptr(save[4]),
                                      ptr(save[5]), p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], ptr(out[0]), ptr(out[1]), ptr(out[2]),
                                      ptr(out[3]), stream_of(in[0])));
-        save.push_back(flat);
+        for (const auto& t : params.saved()) save.push_back(t);
         ctx->save_for_backward(save);
         ctx->saved_data["head_size"] = head_size;
+        ctx->saved_data["type"] = in[6].scalar_type();
         return out;
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const auto in = ctx->get_saved_variables();
         const int B = in[0].size(0), T = in[0].size(1), C = in[0].size(2), D = in[2].size(2);
         c10::DeviceGuard guard(in[0].device());
-        Tensor flat = in[14], dy[4];
-        const auto p = bf16_pointers(std::vector<Tensor>(in.begin() + 6, in.begin() + 14), flat);
+        Tensor dy[4];
+        const auto p = Bf16Params(in.begin() + 6, in.end()).pointers({C * D, C * D, C * D, C * D, C, C, C, C});
         for (int i = 0; i < 4; i++) dy[i] = contiguous_or_zeros(grads[i], in[0]);
         variable_list d(6);
         for (int i = 0; i < 6; i++) d[i] = at::empty_like(in[i]);
@@ -472,7 +493,7 @@ struct ExpandLoras : torch::autograd::Function<ExpandLoras> {
             stream_of(in[0])));
         variable_list out{Tensor()};
         out.insert(out.end(), d.begin(), d.end());
-        for (auto& t : g.tensors(in[6].scalar_type())) out.push_back(t);
+        for (auto& t : g.tensors(ctx->saved_data["type"].toScalarType())) out.push_back(t);
         return out;
     }
 };
