@@ -544,7 +544,9 @@ constexpr int LIN_BLOCKS = 400, LIN_SINGLE_BLOCKS = 320;
 
 }  // namespace
 
-// B: tokens in all (sequences times tokens per sequence)
+// B: tokens in all (sequences times tokens per sequence).  (Four planes and the hidden activation are used and thirteen planes asked for: callers size the
+// workspace with this, some with the number of an earlier release, and nothing is gained by less: 768 channels, 256
+// sequences 5 MB.)
 size_t mixer_decode_workspace_bytes(int B, int C) {
     const size_t Bp = padded_rows(B);
     return 13 * A256(Bp * C * 2) + A256(Bp * R_GATE * 2) + A256(Bp * R_DECAY * 2) + 4 * A256(Bp * 16 * 2);
@@ -588,7 +590,7 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         return r;
     };
     const size_t BC = (size_t)Bp * C;
-    __bf16 *mid = take((size_t)Bp * MID), *r = take(BC), *k = take(BC), *v = take(BC), *ya = take(BC);   // (well inside the workspace)
+    __bf16 *mid = take((size_t)Bp * MID), *r = take(BC), *k = take(BC), *v = take(BC), *ya = take(BC);   // (inside the workspace, see above)
     __bf16 *tg1 = take((size_t)Bp * R_GATE), *tw1 = take((size_t)Bp * R_DECAY);
     __bf16 *kk1 = take((size_t)Bp * 16), *mk1 = take((size_t)Bp * 16), *a1 = take((size_t)Bp * 16), *ma1 = take((size_t)Bp * 16);
     auto c = [](const void* q) { return static_cast<const __bf16*>(q); };
