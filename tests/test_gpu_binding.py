@@ -321,3 +321,32 @@ def test_float32_parameters_may_be_written_to_before_the_backward_pass(stage):
         grads.append(torch.autograd.grad(y, [leaf] + params, [x] * len(y)))
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+def test_errors_of_the_library_keep_their_class_and_code(tmp_path):
+    """With a library in the kernels' place that does nothing but return codes: the forward's error out of the call, the
+    backward's out of autograd."""
+    import ctypes
+    import subprocess
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import attn
+    codes = {'wind_rwkv7_attn_prefill': 5, 'wind_rwkv7_attn_backward': 7}
+    source = ['#include <stddef.h>']
+    for name, (res, _) in _native.SIGNATURES.items():
+        kind, value = {ctypes.c_char_p: ('const char*', '"nothing here"'), ctypes.c_size_t: ('size_t', 256)}.get(res, ('int', codes.get(name, 0)))
+        source.append(f'{kind} {name}() {{ return {value}; }}')
+    (tmp_path / 'stub.c').write_text('\n'.join(source))
+    subprocess.run(['cc', '-shared', '-fPIC', '-w', '-o', str(tmp_path / 'stub.so'), str(tmp_path / 'stub.c')], check=True)
+    x = torch.zeros(1, 16, 64, dtype=torch.bfloat16, device=DEV)
+    _native.binding().load(str(tmp_path / 'stub.so'), _native.WindRwkv7Error)
+    try:
+        for _ in range(2):   # (nothing is left over from an error)
+            with torch.no_grad(), pytest.raises(_native.WindRwkv7Error, match='nothing here') as info:
+                attn(x, x, x, x, x, x, 64)
+            assert info.value.code == 5
+            y = attn(x.clone().requires_grad_(), x, x, x, x, x, 64)
+            with pytest.raises(_native.WindRwkv7Error, match='nothing here') as info:
+                y.sum().backward()
+            assert info.value.code == 7
+    finally:
+        _native.binding().load(_native.LIB_PATH, _native.WindRwkv7Error)

@@ -13,6 +13,7 @@
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -47,7 +48,9 @@ struct Lib {
 #undef X
 } L;
 
-void load(const std::string& path) {
+PyObject* error_class = nullptr;   // WindRwkv7Error(code, message); kept for good
+
+void load(const std::string& path, const py::object& error) {
     void* handle = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
     TORCH_CHECK(handle, "cannot load ", path, ": ", dlerror());
 #define X(name)                                                                                       \
@@ -55,9 +58,20 @@ void load(const std::string& path) {
     TORCH_CHECK(L.name, path, " has no wind_rwkv7_" #name);
     WIND_SYMBOLS(X)
 #undef X
+    error_class = py::object(error).release().ptr();
 }
 
-void check(int code) { TORCH_CHECK(code == 0, "wind_rwkv7 error ", code, ": ", L.strerror(code)); }
+// An entry point's error as the Python class, out of a call as out of a backward pass (autograd's engine takes a python_error
+// to the thread that waits for it).
+void check(int code) {
+    if (code == 0) return;
+    py::gil_scoped_acquire gil;
+    const py::object error = py::reinterpret_borrow<py::object>(error_class)(code, L.strerror(code));
+    PyErr_SetObject(error_class, error.ptr());
+    python_error e;
+    e.persist();
+    throw e;
+}
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
@@ -1171,6 +1185,13 @@ py::object mixer_step(const Tensor& x, const Tensor& x_prev, const Tensor& S, co
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    py::register_local_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (python_error& e) {
+            e.restore();
+        }
+    });
     m.def("load", &load);
     m.def("attn", &attn);
     m.def("attn_ln", &attn_ln);

@@ -150,7 +150,7 @@ def binding():
         loader = importlib.machinery.ExtensionFileLoader('torch_binding', BINDING_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('torch_binding', BINDING_PATH, loader=loader))
         loader.exec_module(module)
-        module.load(LIB_PATH)
+        module.load(LIB_PATH, WindRwkv7Error)
         _binding = module
     return _binding
 
