@@ -388,3 +388,25 @@ def test_ddlerp_first_validates_on_host():
     assert call(x_dtype=7) == 5 and call(param_dtype=-1) == 5
     assert call(x_seq=-1) == 2 and call(y_seq=-1) == 2
     assert call(ws=None) == 6 and call(ws_bytes=256) == 6 and call(ws=0x3010) == 6
+
+
+def test_the_binding_belongs_to_its_torch(monkeypatch, tmp_path):
+    """Built against another torch, or not loadable into this one, it says so and how to build it; the Makefile rebuilds it when
+    torch's version changes."""
+    import subprocess
+    import torch
+    assert _native.binding().torch_version == torch.__version__.split('+')[0]
+    monkeypatch.setattr(_native, '_binding', None)
+    with monkeypatch.context() as m:
+        m.setattr(torch, '__version__', '1.2.3+other')
+        with pytest.raises(ImportError, match='built against torch .*1.2.3.* is running: build it again'):
+            _native.binding()
+    broken = tmp_path / 'torch_binding.so'
+    broken.write_bytes(b'not a library')
+    with monkeypatch.context() as m:
+        m.setattr(_native, 'BINDING_PATH', str(broken))
+        with pytest.raises(ImportError, match='does not load .*build it again'):
+            _native.binding()
+    target, package = 'wind_rwkv/lib/torch_binding.so', os.path.join(os.path.dirname(__file__), '..', 'wind-rwkv7_amd')
+    plan = lambda *a: subprocess.run(['make', '-n', '-C', package, *a, target], check=True, capture_output=True, text=True).stdout
+    assert '-o ' + target in plan('-W', 'build/torch_version')

@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/version.h>
 
 #include "../../include/wind_rwkv7.h"
 
@@ -1192,6 +1193,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             e.restore();
         }
     });
+    m.attr("torch_version") = TORCH_VERSION;   // (without the build's suffix)
     m.def("load", &load);
     m.def("attn", &attn);
     m.def("attn_ln", &attn_ln);

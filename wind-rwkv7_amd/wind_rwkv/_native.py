@@ -141,15 +141,24 @@ _binding = None
 
 
 def binding():
-    """The native eager path of the operators (csrc/torch_binding.cpp) on the loaded library; like it, required."""
+    """The native eager path of the operators (csrc/torch_binding.cpp) on the loaded library; like it, required, and built
+    against the torch that is running."""
     global _binding
     if _binding is None:
         lib()
         if not os.path.exists(BINDING_PATH):
             raise ImportError(f'{BINDING_PATH} is missing: build it with `make -C {os.path.dirname(_PKG_DIR)}`.')
         loader = importlib.machinery.ExtensionFileLoader('torch_binding', BINDING_PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('torch_binding', BINDING_PATH, loader=loader))
-        loader.exec_module(module)
+        import torch
+        again = (f'it belongs to the torch it was built against, and torch {torch.__version__} is running: build it again with '
+                 f'`make -C {os.path.dirname(_PKG_DIR)}`.')
+        try:
+            module = importlib.util.module_from_spec(importlib.util.spec_from_file_location('torch_binding', BINDING_PATH, loader=loader))
+            loader.exec_module(module)
+        except ImportError as e:
+            raise ImportError(f'{BINDING_PATH} does not load ({e}); {again}') from e
+        if module.torch_version != torch.__version__.split('+')[0]:
+            raise ImportError(f'{BINDING_PATH} was built against torch {module.torch_version}; {again}')
         module.load(LIB_PATH, WindRwkv7Error)
         _binding = module
     return _binding
