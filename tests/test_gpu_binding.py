@@ -131,6 +131,30 @@ def test_block_equals_the_python_path(monkeypatch, C, H, x_dtype, param_dtype, f
         assert seq_ref.rel_err(a.float().cpu(), b.float().cpu()) <= (5e-3 if i < 2 else 1e-2), i
 
 
+@pytest.mark.parametrize('C,H,B', [(2048, 32, 6), (768, 12, 42)])
+def test_a_block_of_large_products_equals_the_python_path(monkeypatch, C, H, B):
+    """Products of 2.5e10 and more, which go to the BLAS library: all of them at 2048 channels, those of one segment at 768.  At
+    the gates of the test above, the output's first token apart (its GroupNorm after a zero state is ill conditioned)."""
+    from wind_rwkv import _native
+    assert B * 1024 * C * C >= 2.5e10
+    model, gen = _small_model(C, H, torch.float32)
+    with torch.no_grad():
+        for p in model.parameters():
+            if p.dim() == 2:
+                p.mul_(10 * C ** -0.5)   # (unit gain: 0.1 N(0,1) as above is for small blocks)
+    x, dy = (torch.randn(B, 1024, C, generator=gen).bfloat16().to(DEV) for _ in range(2))
+    dy[:, 0] = 0
+    results = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(_native, 'binding', lambda: _Absent())
+        leaves = [x.clone().requires_grad_()] + list(model.parameters())
+        y = model(leaves[0])
+        results.append([y.detach()[:, 1:]] + list(torch.autograd.grad(y, leaves, dy)))
+    for i, (a, b) in enumerate(zip(*results)):
+        assert seq_ref.rel_err(a.float(), b.float()) <= (5e-3 if i < 1 else 1e-2), i
+
+
 @pytest.mark.parametrize('T', [2, 15, 17, 100])
 @pytest.mark.parametrize('continued', [False, True])
 def test_prompt_of_any_length_equals_the_python_path(monkeypatch, T, continued):

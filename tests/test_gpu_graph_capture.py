@@ -152,6 +152,28 @@ def test_time_mixer_block_capture():
     _capture_and_replay(make, run)
 
 
+def test_a_large_block_capture():
+    """The same where the products are large enough for the BLAS library, whose calls may record more than kernels."""
+    from collections import namedtuple
+    from wind_rwkv.rwkv7 import TimeMixer
+    B, T, C = 6, 1024, 2048
+    torch.manual_seed(3)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(12, 32, C), 6).to(DEV)
+    with torch.no_grad():
+        model.Wo.normal_(std=C ** -0.5)
+    params = list(model.parameters())
+
+    def make(seed):
+        g = torch.Generator(DEV).manual_seed(seed)
+        return [torch.randn(B, T, C, generator=g, device=DEV).requires_grad_()], [torch.randn(B, T, C, generator=g, device=DEV).bfloat16()]
+
+    def run(leaves, grads):
+        y = model(leaves[0])
+        return [y] + list(torch.autograd.grad([y], leaves + params, grads))
+
+    _capture_and_replay(make, run)
+
+
 @pytest.mark.skip(reason='torch.cuda.make_graphed_callables on the block ends in a host-side segmentation fault inside '
                          'the framework (capture_end of its separate backward graph, torch/cuda/graphs.py) on this '
                          'image; cause not established, so the case stays off the GPU.  Capturing the whole '

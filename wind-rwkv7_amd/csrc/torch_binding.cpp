@@ -659,10 +659,15 @@ struct Activations {
 };
 
 // Products out = in W^T on the same rows in one launch (wind_rwkv7_linear_group).  The library's kernel for a single large
-// product is the better one by a quarter where each fills the chip several times over (65536 x 768 x 768: 70 us against 92;
-// 32768 rows as a group of six: 204 against 169), so there a large product goes to it.
+// product is the better one by a quarter where each fills the chip several times over, so there a large product goes to it.
+// Measured, us for three C x C products as one group / as three library calls, at 1.2e10, 2.5e10 and 1e11 rows x columns x
+// contraction length each: C = 512 114/166, 237/204; 768 84/78, 189/143, 720/589; 1536 79/82, 156/124, 637/480; 2048 80/98,
+// 175/133, 627/497; 4096 96/95, 178/146, 649/470.  A second segment is a second library call that reads the result back and
+// adds to it in bf16; here it is more of the same sum (one product, 128 indices in the second segment, own / library): C =
+// 768 71/83, 1024 76/88, 1536 64/63, 2048 78/58, 4096 88/62 at 2.5e10, so with one it takes a contraction of 2048 as well.
 struct Products {
     static constexpr double LIBRARY_FROM = 2.5e10;   // rows x columns x contraction length
+    static constexpr int LIBRARY_FROM_K = 2048;      // with a second segment
     std::vector<wind_rwkv7_linear> ps;
     void add(const void* in, const void* W, int64_t K, int64_t N) {
         wind_rwkv7_linear p{};
@@ -682,7 +687,7 @@ struct Products {
     void run(int64_t rows, const Tensor& like) {
         std::vector<wind_rwkv7_linear> group;
         for (const auto& p : ps) {
-            if ((double)rows * p.N * p.K[0] < LIBRARY_FROM || p.npieces > 1 || p.op[0]) {
+            if ((double)rows * p.N * p.K[0] < LIBRARY_FROM || (p.K[1] && p.K[0] < LIBRARY_FROM_K) || p.npieces > 1 || p.op[0]) {
                 group.push_back(p);
                 continue;
             }
