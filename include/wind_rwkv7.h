@@ -231,7 +231,7 @@ int wind_rwkv7_ln_epilogue_backward(int B, int T, int H, int C,
                                     void* workspace, size_t workspace_bytes, void* stream);
 
 /* One token per sequence through the WHOLE time mixer (TimeMixer of time_mixer.py:18-167 taken at T = 1): token
- * shift, projections, LoRAs, the WKV7 step with GroupNorm / bonus / gate, output projection - five kernel launches.
+ * shift, projections, LoRAs, the WKV7 step with GroupNorm / bonus / gate, output projection - four kernel launches.
  * The reference's block has no single-token form; its forward (time_mixer.py:96-167) is the specification, with the
  * previous token x_prev and the WKV7 state carried by the caller.  Head size 64, C = 64 H, the block's LoRA ranks
  * (mix 32, decay 64, gate 128, the others 16).  Every parameter is a bf16 device array laid out as the module's

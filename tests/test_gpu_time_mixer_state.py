@@ -83,7 +83,7 @@ def test_stateful_calls_compile():
         want_t, _ = model.step(xt, a)
         got_t, _ = torch.compile(model.step, fullgraph=True)(xt, b)
     torch.cuda.synchronize()
-    # eager `step` is the five-launch single-token path, the traced one goes through the registered sequence operators:
+    # eager `step` is the four-launch single-token path, the traced one goes through the registered sequence operators:
     # the same roundings between stages, other summation orders inside them
     assert seq_ref.rel_err(got_t.float().cpu(), want_t.float().cpu()) <= 5e-3
     assert seq_ref.rel_err(b[1].float().cpu(), a[1].float().cpu()) <= 5e-3
@@ -91,7 +91,7 @@ def test_stateful_calls_compile():
 
 @pytest.mark.parametrize('C,H,B', [(768, 12, 1), (768, 12, 5), (256, 4, 16), (256, 4, 35), (192, 3, 2)])
 def test_single_token_path_against_the_sequence_kernels(C, H, B):
-    """`step` in five launches (wind_rwkv7_mixer_decode) against the same step on the sequence kernels (rows padded
+    """`step` in four launches (wind_rwkv7_mixer_decode) against the same step on the sequence kernels (rows padded
     to a tile), two tokens in a row: output, carried token and WKV7 state (fp32 and bf16)."""
     model, gen = _model(C, H, seed=15)
     x = torch.randn(B, 16, C, generator=gen).bfloat16().to(DEV)

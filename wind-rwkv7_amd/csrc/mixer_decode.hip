@@ -488,7 +488,9 @@ __global__ __launch_bounds__(256) void prompt_head_kernel(const HeadArgs A) {
 }
 
 // The recurrence alone, token by token, with its operands in memory: the tokens of a prompt after its last whole chunk, whose
-// state the sequence kernels would multiply in bf16.  Block = (sequence, head).
+// state the sequence kernels would multiply in bf16.  Block = (sequence, head).  Bound by latency: 11 tokens x 2 x 12 heads take
+// 10.4 us, of a token's two row sums one after the other, a barrier and the epilogue (operands of the next token asked for
+// one token ahead: 11.0).  The same tokens through the four kernels of a step instead: 26 us more for the prompt.
 struct TokensArgs {
     const __bf16 *w, *k, *b, *r, *v, *kk, *g;   // at the sequences' first token
     __bf16* y;

@@ -15,7 +15,7 @@
 // The value rows of a state never mix, so a head is cut over blocks by rows (scan_split).  In the scan, four or eight
 // wavefronts of a block carry the recurrence and touch LDS only; four more fetch the next chunk, turn it into operands in
 // the other half of a double buffer and carry the results of the chunk before to memory, with one barrier per chunk.
-// (Staging by the recurrence's own wavefronts, between barriers, was a third of its time: 227 -> 170 us at 8 x 1024 tokens
+// (Staging by the recurrence's own wavefronts, between barriers, was a fifth of its time: 227 -> 183 us at 8 x 1024 tokens
 // x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  What bounds it now is LDS: a wavefront reads five vectors of
 // 64 channels per token, 360 of the 400 cycles that a token takes with eight wavefronts on a compute unit.
 // The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
@@ -26,7 +26,8 @@
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
 //   1 x 256 tokens x 4 heads of 64   274 -> 102        8 x 1024 x 6 heads of 128   2420 -> 1214
-//   8 x 1024 x 12 heads of 64        844 -> 595        32 x 1024 x 12 heads of 64  2395 -> 1778
+//   8 x 1024 x 12 heads of 64        831 -> 541        32 x 1024 x 12 heads of 64  2395 -> 1778
+// (on different machines 511 to 548 for the third)
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>

@@ -3,8 +3,8 @@
 Mirrors the reference's ``TimeMixer`` (time_mixer.py:18-167): same constructor signature, same parameter
 names and shapes (so a state dict moves over unchanged), same forward contract
 (``x [B,T,C]`` of any float dtype -> ``[B,T,C]`` bf16).  The projections (:120-131, :167) are bf16
-products with fp32 accumulation, all of them in this package's kernels, grouped into few launches (linear_group.hip,
-linear_wgrad.hip; single very large ones go to the BLAS library):
+products with fp32 accumulation in this package's kernels, several per launch (linear_group.hip, linear_wgrad.hip), except
+that a product of 2.5e10 multiplications and more goes to the BLAS library:
 
     ddlerp -> r, k, v, gate and LoRA first halves (matmuls) -> expand_loras -> attn_ln -> output matmul
 
