@@ -236,3 +236,27 @@ def test_no_grad_forward_and_step_capture():
         return [y, y_t, state[1]]
 
     _capture_and_replay(make, run)
+
+
+@pytest.mark.parametrize('B,T', [(2, 100), (9, 65), (40, 7)])
+def test_continued_ragged_prompt_capture(B, T):
+    """A prompt of whole chunks and a few tokens after a carried state (up to eight sequences, more, and no whole chunk)."""
+    from collections import namedtuple
+    from wind_rwkv.rwkv7 import TimeMixer
+    torch.manual_seed(4)
+    model = TimeMixer(namedtuple('Config', ['n_layer', 'n_head', 'n_embd'])(4, 2, 128), 1).to(DEV)
+    with torch.no_grad():
+        for p in model.parameters():
+            p.normal_(std=0.1)
+
+    def make(seed):
+        g = torch.Generator(DEV).manual_seed(seed)
+        rn = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+        return [rn(B, T, 128).bfloat16(), rn(B, 128).bfloat16(), rn(B, 2, 64, 64)], []
+
+    def run(leaves, grads):
+        with torch.no_grad():
+            y, (last, S) = model(leaves[0], state=(leaves[1], leaves[2]), return_state=True)
+        return [y, last, S]
+
+    _capture_and_replay(make, run)
