@@ -266,7 +266,7 @@ int wind_rwkv7_mixer_prompt(int B, int T, int C, int H, int state_dtype, const w
  * end of a sequence that is no whole number of chunks.  q, v, a, g, y: [B,T,H*64] bf16, the tokens first .. first+n-1 are read and
  * written; w, k, b: [B,wkb_T,H*64], the tokens wkb_first .. wkb_first+n-1 (as the others': wkb_T = T, wkb_first = first); params
  * as for wind_rwkv7_attn_ln_forward; s0: NULL (zeros) or the state before, sT: the state after (may be s0 itself).
- * B <= 65535; bases 16-byte aligned. */
+ * Bases 16-byte aligned. */
 int wind_rwkv7_attn_ln_tokens(int B, int T, int H, int C, int first, int n, int state_dtype, const void* w, const void* q,
                               const void* k, const void* v, const void* a, const void* b, const void* g, const void* params,
                               int wkb_T, int wkb_first, const void* s0, void* y, void* sT, void* stream);
@@ -292,7 +292,7 @@ int wind_rwkv7_ddlerp_forward(int B, int T, int C, int D,
 /* The four streams of one token per sequence that follows a carried token (a continued sequence's first): as above with the
  * token before it in place of the zero row, but in float32 throughout and on the parameters as they are.  x + b x_seq and
  * x_prev + b C: the tokens, C elements of x_dtype; alpha, L, R, beta: of param_dtype, any alignment.
- * y + k y_stream + b y_seq: C bf16 values (the streams' rows of a forward's y, to replace them).  B <= 65535.
+ * y + k y_stream + b y_seq: C bf16 values (the streams' rows of a forward's y, to replace them).
  * workspace: wind_rwkv7_ddlerp_first_workspace_bytes(B, D) bytes, 256-byte aligned. */
 typedef struct {
     const void *x, *x_prev, *alpha, *L, *R, *beta;

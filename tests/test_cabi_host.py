@@ -365,7 +365,7 @@ def test_pad_rows_validates_on_host():
 def test_attn_ln_tokens_validates_on_host():
     lib = _native.lib()
     ok = [2, 32, 3, 64, 16, 5, _native.F32] + [0x1000] * 8 + [16, 0, None, 0x2000, 0x3000, None]
-    for idx, val, code in [(0, 0, 2), (0, 70000, 2), (1, 20, 2), (2, 0, 2), (3, 128, 3), (4, -1, 2), (4, 28, 2), (5, 0, 2), (6, 7, 5), (7, None, 1),
+    for idx, val, code in [(0, 0, 2), (0, 1 << 29, 2), (1, 20, 2), (2, 0, 2), (3, 128, 3), (4, -1, 2), (4, 28, 2), (5, 0, 2), (6, 7, 5), (7, None, 1),
                            (14, None, 1), (15, 4, 2), (16, 12, 2), (18, None, 1), (19, None, 1)]:
         bad = list(ok)
         bad[idx] = val
@@ -383,7 +383,7 @@ def test_ddlerp_first_validates_on_host():
     def call(B=2, C=64, D=32, y=0x2000, ws=0x3000, ws_bytes=1 << 20, t=True, **change):
         args = _native.FirstTokens(**{**fields, **change})
         return lib.wind_rwkv7_ddlerp_first(B, C, D, ctypes.byref(args) if t else None, y, ws, ws_bytes, None)
-    assert call(B=0) == 2 and call(B=70000) == 2 and call(C=72) == 9 and call(D=48) != 0
+    assert call(B=0) == 2 and call(C=72) == 9 and call(D=48) != 0
     assert call(t=False) == 1 and call(y=None) == 1 and call(beta=None) == 1
     assert call(x_dtype=7) == 5 and call(param_dtype=-1) == 5
     assert call(x_seq=-1) == 2 and call(y_seq=-1) == 2

@@ -121,7 +121,8 @@ def test_ddlerp_rejects_unsupported_shapes():
 
 
 @pytest.mark.parametrize('B,C,D,x_dtype,p_dtype', [(1, 64, 32, torch.bfloat16, torch.float32), (3, 768, 32, torch.float32, torch.float32),
-                                                   (2, 2112, 64, torch.bfloat16, torch.bfloat16), (5, 320, 64, torch.float32, torch.bfloat16)])
+                                                   (2, 2112, 64, torch.bfloat16, torch.bfloat16), (5, 320, 64, torch.float32, torch.bfloat16),
+                                                   (70001, 64, 32, torch.bfloat16, torch.float32)])
 def test_first_tokens_after_a_carried_one(B, C, D, x_dtype, p_dtype):
     """The streams of one token per sequence in fp32 on the parameters as they are, against fp64: the rounding of an output with
     seven stored bits, 2^-8 of a value, and 1e-5 for the sums.  The tokens and every parameter start one element off an allocation."""

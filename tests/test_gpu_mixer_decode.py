@@ -55,7 +55,7 @@ def test_a_few_tokens_equal_as_many_steps(B, T, H):
     assert seq_ref.rel_err(S.cpu(), st[1].cpu()) <= 1e-4
 
 
-@pytest.mark.parametrize('B,T,H', [(1, 1003, 3), (3, 100, 4), (2, 79, 12), (9, 65, 2), (40, 15, 2), (300, 2, 1)])
+@pytest.mark.parametrize('B,T,H', [(1, 1003, 3), (3, 100, 4), (2, 79, 12), (9, 65, 2), (40, 15, 2), (300, 2, 1), (66000, 2, 1)])
 @pytest.mark.parametrize('continued', [False, True])
 def test_a_ragged_prompt_is_whole_chunks_and_then_steps(B, T, H, continued):
     """The tokens after the last whole chunk keep the state in fp32 from token to token, as steps do: the same sums in

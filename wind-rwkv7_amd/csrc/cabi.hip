@@ -549,7 +549,7 @@ int wind_rwkv7_attn_ln_tokens(int B, int T, int H, int C, int first, int n, int 
                               const void* s0, void* y, void* sT, void* stream) {
     if (B <= 0 || T <= 0 || H <= 0 || first < 0 || n <= 0 || first > T - n || wkb_first < 0 || wkb_first > wkb_T - n) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (C != wkv::HEAD) return WIND_RWKV7_ERR_HEAD_SIZE;
-    if (B > 65535 || (long long)B * H > (1LL << 30) || (long long)B * (T > wkb_T ? T : wkb_T) * H * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if ((long long)B * H > (1LL << 30) || (long long)B * (T > wkb_T ? T : wkb_T) * H * C > (1LL << 40)) return WIND_RWKV7_ERR_BAD_SHAPE;
     const int rc = check_dtypes(WIND_RWKV7_BF16, state_dtype);
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !g || !params || !y || !sT) return WIND_RWKV7_ERR_NULL_POINTER;   // (s0 may be null)
@@ -593,7 +593,7 @@ int wind_rwkv7_ddlerp_first(int B, int C, int D, const wind_rwkv7_first_tokens* 
                             void* stream) {
     int rc = check_ddlerp(B, 16, C, D);
     if (rc) return rc;
-    if (B > 65535) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (C / 64 > 65535) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (!t || !t->x || !t->x_prev || !t->alpha || !t->L || !t->R || !t->beta || !y) return WIND_RWKV7_ERR_NULL_POINTER;
     for (int d : {t->x_dtype, t->param_dtype})
         if (d != WIND_RWKV7_BF16 && d != WIND_RWKV7_F32) return WIND_RWKV7_ERR_DTYPE;

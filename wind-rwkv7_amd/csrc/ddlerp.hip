@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void ddlerp_param_reduce_kernel(int C, int nsp
 template <class X, class P>   // element types of the tokens and of the parameters
 __global__ __launch_bounds__(256) void first_mid_kernel(int C, int D4, const X* __restrict__ x, long x_seq, const X* __restrict__ x_prev,
                                                         const P* __restrict__ alpha, const P* __restrict__ Lw, float* __restrict__ mid) {
-    const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6), b = blockIdx.y;   // a wavefront per hidden unit
+    const int lane = threadIdx.x & 63, m = blockIdx.y * 4 + (threadIdx.x >> 6), b = blockIdx.x;   // a wavefront per hidden unit
     const X *xr = x + (long)b * x_seq, *pr = x_prev + (long)b * C;
     const P* lr = Lw + (long)m * C;
     float acc = 0.f;
@@ -805,7 +805,7 @@ template <class X, class P, int D>
 __global__ __launch_bounds__(256) void first_streams_kernel(int C, const X* __restrict__ x, long x_seq, const X* __restrict__ x_prev,
                                                             const P* __restrict__ R, const P* __restrict__ beta, const float* __restrict__ mid,
                                                             __bf16* __restrict__ y, long y_stream, long y_seq) {
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63), b = blockIdx.y;
+    const int c = blockIdx.y * 64 + (threadIdx.x & 63), b = blockIdx.x;
     const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const P* r = R + ((long)k * C + c) * D;
     const float* h = mid + ((long)b * 4 + k) * D;   // (the same for all lanes)
@@ -913,8 +913,8 @@ template <class X, class P, int D>
 void first_tokens(int B, int C, const FirstTokens& t, void* y, float* mid, hipStream_t stream) {
     auto x = [](const void* p) { return static_cast<const X*>(p); };
     auto w = [](const void* p) { return static_cast<const P*>(p); };
-    hipLaunchKernelGGL((first_mid_kernel<X, P>), dim3(D, B), dim3(256), 0, stream, C, 4 * D, x(t.x), t.x_seq, x(t.x_prev), w(t.alpha), w(t.Lw), mid);
-    hipLaunchKernelGGL((first_streams_kernel<X, P, D>), dim3(C / 64, B), dim3(256), 0, stream, C, x(t.x), t.x_seq, x(t.x_prev), w(t.R), w(t.beta),
+    hipLaunchKernelGGL((first_mid_kernel<X, P>), dim3(B, D), dim3(256), 0, stream, C, 4 * D, x(t.x), t.x_seq, x(t.x_prev), w(t.alpha), w(t.Lw), mid);
+    hipLaunchKernelGGL((first_streams_kernel<X, P, D>), dim3(B, C / 64), dim3(256), 0, stream, C, x(t.x), t.x_seq, x(t.x_prev), w(t.R), w(t.beta),
                        mid, static_cast<__bf16*>(y), t.y_stream, t.y_seq);
 }
 template <int D>

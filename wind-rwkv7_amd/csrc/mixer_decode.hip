@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
     __shared__ HeadTile s;
     const int lane = threadIdx.x & 63, ib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Lane L;
-    const int h = blockIdx.x, seq = blockIdx.y, bh = seq * A.H + h;
+    const int bh = blockIdx.x, seq = bh / A.H, h = bh - seq * A.H;
     f32x4 S[NBLK];
 #pragma unroll
     for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
@@ -656,7 +656,7 @@ void launch_tokens(int B, int T, int H, int first, int n, int wkb_T, int wkb_fir
     const TokensArgs A{at(w, wkb_first), at(k, wkb_first), at(b, wkb_first), at(q, first), at(v, first), at(a, first), at(g, first),
                        static_cast<__bf16*>(y) + (long)first * C, (long)wkb_T * C, (long)T * C, n, H, C, state_f32,
                        static_cast<const float*>(params), state_in, state};
-    hipLaunchKernelGGL(tokens_kernel, dim3(H, B), dim3(256), 0, stream, A);
+    hipLaunchKernelGGL(tokens_kernel, dim3((unsigned)(B * H)), dim3(256), 0, stream, A);
 }
 
 }  // namespace wkv

@@ -1110,7 +1110,7 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     const bool stateful = return_state || x_prev_ || s0_;
     const int64_t T = x.size(1);
     const Block s{x.size(0), (T + 15) / 16 * 16, x.size(2), H};
-    if (T % 16 && (!stateful || s.N() != 64 || s.B > 65535)) return py::none();
+    if (T % 16 && (!stateful || s.N() != 64)) return py::none();
     if (s.rows() > std::numeric_limits<int>::max() || s.C % 64 || !L.attn_ln_saved_bytes(s.B, s.T, s.H, s.N()) ||
         !L.expand_loras_bwd_workspace_bytes(s.B, s.T, s.C, R_LORA) || !L.ddlerp_bwd_workspace_bytes(s.B, s.T, s.C, R_MIX))
         return py::none();
@@ -1123,7 +1123,7 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     if (grad) return stateful ? py::object(py::none()) : py::cast(mixer_node(H, x, p, std::make_index_sequence<PARAMS>()));
     Tensor x_prev, s0;
     if (x_prev_) {
-        if (!x_prev_->is_cuda() || !floating(*x_prev_) || s.B > 65535 || x_prev_->device() != x.device() || x_prev_->sizes() != at::IntArrayRef({s.B, s.C})) return py::none();
+        if (!x_prev_->is_cuda() || !floating(*x_prev_) || x_prev_->device() != x.device() || x_prev_->sizes() != at::IntArrayRef({s.B, s.C})) return py::none();
         x_prev = *x_prev_;
     }
     if (s0_) {
