@@ -128,6 +128,33 @@ def test_f32_backward_entry_points_agree(B, T, H, C):
         assert seq_ref.rel_err(h.cpu(), g.cpu()) <= 1e-5, n
 
 
+@pytest.mark.parametrize('C', [16, 64, 80])
+@pytest.mark.parametrize('w', [2.0, 4.5, 30.0])
+def test_f32_strong_decays(c_oracle, C, w):
+    """Decays that all but end a state within a token (exp(-exp(w)) 6e-4, 1e-39, 0) on some channels and tokens: the products
+    of decays underflow, the gradient of w is what little is left, and nothing larger may be left of the terms it is a difference of."""
+    B, T, H = 1, 48, 2
+    d = inputs.wkv7_inputs(B, T, H, C, seed=400 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
+    d['w'] = d['w'].clone()
+    d['w'][:, :, :, ::3] = w
+    d['w'][:, 5::7] = w
+    args = [d[n] for n in 'qwkvab']
+    y_ref, sT_ref = c_oracle.forward(*args, d['s0'])
+    ref = dict(zip(['dq', 'dw', 'dk', 'dv', 'da', 'db', 'ds0'], c_oracle.backward(*args, d['s0'], d['dy'], d['dsT'])))
+    y, sT, grads, ds0 = _run(d, B, T, H, C, True)
+    assert seq_ref.rel_err(y.detach().cpu(), y_ref) <= TOL and seq_ref.rel_err(sT.detach().cpu(), sT_ref) <= TOL
+    for n, g in zip(NAMES, grads):
+        assert seq_ref.rel_err(g.cpu(), ref['d' + n]) <= TOL, n
+    # the strongly decayed elements by themselves: to fp32 accuracy at w = 2.  At 4.5 what is left is a difference of some 64
+    # terms in fp64, none above max |dw|, times exp(w) = 90: 90 * 64 * 2^-53 = 6e-13 of max |dw|.  At 30 the decay is zero.
+    strong = d['w'] == w
+    got, want = grads[0].cpu()[strong], ref['dw'][strong]
+    if w == 2.0:
+        assert seq_ref.rel_err(got, want) <= TOL
+    else:
+        assert float((got.double() - want.double()).abs().max()) <= (1e-12 if w < 30 else 0.) * float(ref['dw'].abs().max())
+
+
 def test_other_head_sizes_through_the_public_names():
     """attn, attn_triton and attn_triton_bighead on bf16 tensors with head sizes other than 64: attn and
     dot_prec='bf16' run the bf16 matrix-core kernels for those head sizes (1e-2 gate), the default dot_prec='fp32'

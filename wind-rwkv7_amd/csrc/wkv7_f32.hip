@@ -20,14 +20,12 @@
 // 64 channels per token, 360 of the 400 cycles that a token takes with eight wavefronts on a compute unit.
 // The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
 // direction (it keeps the state gradient arriving at every chunk's end and dsa of every token, and leaves dv and ds0)
-// and then a kernel in which every chunk is on its own: it recomputes states and state gradients without a row sum to
-// wait for, and makes the other five gradients.
+// and then a kernel in which every chunk is on its own and makes the other five gradients.
 // A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
-//   1 x 256 tokens x 4 heads of 64   274 -> 102        8 x 1024 x 6 heads of 128   2420 -> 1214
-//   8 x 1024 x 12 heads of 64        831 -> 541        32 x 1024 x 12 heads of 64  2395 -> 1778
-// (on different machines 511 to 548 for the third)
+//   1 x 256 tokens x 4 heads of 64   274 -> 102        8 x 1024 x 6 heads of 128   2420 -> 980
+//   8 x 1024 x 12 heads of 64        831 -> 440        32 x 1024 x 12 heads of 64  2395 -> 1545
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -112,6 +110,16 @@ __device__ __forceinline__ RowVals<R> lds_rows(const float* p) {
         r.x[0] = *p;
     }
     return r;
+}
+
+// element at a 32-bit byte offset from a base that is the same in every lane (scalar base, one register per lane)
+template <class V>
+__device__ __forceinline__ const V& at_bytes(const float* p, unsigned o) {
+    return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + o);
+}
+template <class V>
+__device__ __forceinline__ V& at_bytes(float* p, unsigned o) {
+    return *reinterpret_cast<V*>(reinterpret_cast<char*>(p) + o);
 }
 
 // sum over the LPR lanes that share a state row (16: a DPP row; 32: two neighbouring DPP rows), result in all of them
@@ -521,153 +529,189 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
     }
 }
 
-// The gradients of one chunk (16 tokens) of one head and 64 of its columns, from the state entering the chunk, the state
-// gradient arriving at its end, and S a and dsa of every token: nothing is left to wait for, every chunk is its own block.
-// A lane holds ONE column of GR rows (CR / GR wavefronts), so every column sum is a chain of multiply-adds inside the lane
-// and one sum over the wavefronts through LDS; what belongs to a row (v, S a, dy, dsa) is read from LDS as a broadcast.
-// The states of GWIN tokens are recomputed into registers; the second half of a chunk first runs through the first.
-// Bound: vector issue, 13 instructions per state element and token: 217 us at 8 x 1024 tokens x 12 heads of 64, of which
-// 176 us are issue alone.  Tried instead: the row operands through scalar loads into scalar registers, 390 us (every token
-// waits for them, and the scalar cache holds a quarter of what the blocks of a compute unit read); two columns and eight
-// rows per lane (half the reads of row operands per multiply-add, but two wavefronts per SIMD instead of four), 307 us.
-constexpr int GR = 8, GWIN = 8, GRED = 4;   // rows per wavefront, tokens of kept states, tokens between sums over wavefronts
-
-template <int CR>   // head size
-__global__ __launch_bounds__(64 * (CR / GR), 4) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w,
-                                                                       const float* __restrict__ q, const float* __restrict__ k,
-                                                                       const float* __restrict__ v, const float* __restrict__ a,
-                                                                       const float* __restrict__ b, const float* __restrict__ dy,
-                                                                       const float* __restrict__ ckpt,
-                                                                       const float* __restrict__ work, float* __restrict__ dw,
-                                                                       float* __restrict__ dq, float* __restrict__ dk,
-                                                                       float* __restrict__ da, float* __restrict__ db) {
-    constexpr int CH = CH64, COLS = 64, NW = CR / GR, THREADS = 64 * NW;
-    constexpr int RPT = (CH * CR + THREADS - 1) / THREADS, TPW = (CH + NW - 1) / NW;   // row values and tokens a thread stages
-    static_assert(CH == 2 * GWIN && GWIN % GRED == 0 && GR == 8, "two windows per chunk; two sums of four rows");
-    enum { G_DEC = 0, G_Q, G_K, G_A, G_B, G_DDEC, G_VECS };
+// The gradients of one chunk (16 tokens) of one head and 64 of its columns, from the state S entering the chunk, the state
+// gradient E arriving at its end, and S a (sa) and dsa of every token: nothing is left to wait for, every chunk and column
+// block is one wavefront on its own.  Inside a chunk the state is S under the decays plus rank-one terms, S_t = S D(0..t) +
+// sum_{i<=t} (sa_i b_i^T + v_i k_i^T) D(i+1..t) with D(i..t) the product of the decays of tokens i .. t (never above one and
+// never divided by: the range of w stays the recurrence's), and likewise backwards, so
+//     dq_j = D(0..j) S^T dy_j + sum_{i<=j} D(i+1..j) ((sa_i.dy_j) b_i + (v_i.dy_j) k_i)       da_j: dsa_j, decays up to j - 1
+//     dk_i = D(i+1..15) E^T v_i + sum_{j>=i} D(i+1..j) (v_i.dy_j) q_j + sum_{j>i} D(i+1..j-1) (v_i.dsa_j) a_j       db_i: sa_i
+// each of them a Horner scheme in the decays: twelve multiply-adds per column and pair i <= j instead of thirteen per column,
+// token and ROW of the state.  With W_t the sum of all terms, times their own q, a, b or k, whose decays contain token t,
+//     dw_t = -exp(w_t) W_t,   W_t = M_t - a_t da_t,   M_{t+1} = W_t + b_t db_t + k_t dk_t - q_t dq_t.
+// What needs the rows of the states - S^T [dy dsa], E^T [v sa], the sums of S * E for M_0 and the four 16 x 16 products of row
+// vectors - is one pass of matrix instructions over them.  All of it in fp64, whose multiply-add is as fast as fp32's here and
+// whose matrix instruction takes twice as long: a sum over rows averages the roundings of its terms, a sum of the terms'
+// sums does not, and in fp32 the errors would be 1.7e-7 where recomputing the states row by row left 0.9e-7.
+// Bound: memory, 90 KB per chunk and 64 columns: 8 x 1024 tokens x 12 heads of 64 142 us for 553 MB (without the matrix
+// instructions 123, without the pairs of tokens 132, without either 118), where recomputing the states took 221; 32 x 1024 x 12
+// 848 -> 529, 8 x 1024 x 6 heads of 128 473 -> 211, 8 x 1024 x 16 heads of 32 157 -> 92.
+template <int CR, int COLS>   // head size, columns of a block
+__global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w, const float* __restrict__ q,
+                                                               const float* __restrict__ k, const float* __restrict__ v,
+                                                               const float* __restrict__ a, const float* __restrict__ b,
+                                                               const float* __restrict__ dy, const float* __restrict__ ckpt,
+                                                               const float* __restrict__ work, float* __restrict__ dw,
+                                                               float* __restrict__ dq, float* __restrict__ dk,
+                                                               float* __restrict__ da, float* __restrict__ db) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    constexpr int CH = CH64, HALF = 32, HALVES = COLS / HALF;
+    static_assert(CH == 16 && (HALVES == 1 || HALVES == 2), "a chunk is one tile of the matrix instruction; a lane per column");
     enum { Q_V = 0, Q_SA, Q_DY, Q_DSA, Q_VECS };
-    __shared__ float in[G_VECS][CH][COLS];
-    __shared__ __attribute__((aligned(16))) float rows[Q_VECS][CH][CR];
-    __shared__ float red[NW][RED_VECS][GRED][COLS];
+    enum { G_SY = 0, G_VY, G_SD, G_VD };
+    __shared__ __attribute__((aligned(16))) float xs[2][CH][HALF], ys[2][CH][2 * HALF];   // S^T dy and dsa of 32 columns; E^T v and sa
+    float(*const es)[2 * HALF] = reinterpret_cast<float(*)[2 * HALF]>(xs);                  // then exp(w) of all tokens and columns
+    __shared__ double zs[4][HALF];
+    __shared__ d4 gram[CH * (CH + 1) / 2];                                // sa.dy, v.dy, sa.dsa, v.dsa of tokens i <= j
+    auto pair = [](int i, int j) { return i * CH - i * (i - 1) / 2 + j - i; };
     const int NC = T / CH, bh = blockIdx.x / NC, chunk = blockIdx.x - bh * NC, h = bh % H;
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row0 = wv * GR;
-    const int col = COLS * blockIdx.y + lane;
-    const bool col_ok = CR % COLS == 0 || col < CR;
-    const int colc = col_ok ? col : 0;   // (lanes past the head size read column 0 and write nothing)
+    const int lane = threadIdx.x, g = lane >> 4, n = lane & 15;
+    const int col0 = COLS * blockIdx.y, col = col0 + lane;
+    const bool col_ok = (HALVES == 2 || lane < COLS) && (CR % COLS == 0 || col < CR);
+    const int colc = col_ok ? col : 0;                                    // (lanes past the columns: column 0, nothing written)
     const long base = seq_index((long)(bh / H) * T + (long)chunk * CH, H, h, 0, CR);
     const unsigned ld = (unsigned)H * CR;
-    const long nstate = saved_states(gridDim.x / NC, T, CR), st = (long)blockIdx.x * CR * CR + (long)row0 * CR;
+    const long nstate = saved_states(gridDim.x / NC, T, CR), st = (long)blockIdx.x * CR * CR;
     const float* const row_src[Q_VECS] = {v, ckpt + nstate, dy, work + nstate};
 
-    float Sx[GR], dS[GR];
-#pragma unroll
-    for (int r = 0; r < GR; r++) {
-        Sx[r] = (ckpt + st)[(unsigned)(r * CR + colc)];
-        dS[r] = (work + st)[(unsigned)(r * CR + colc)];
-    }
-    // everything is requested before anything is waited for (with trip counts known only at run time 236 instead of 217 us)
-    float row_pre[RPT][Q_VECS], col_pre[TPW][5];
-    const float* const col_src[5] = {w, q, k, a, b};
-#pragma unroll
-    for (int i = 0; i < RPT; i++) {
-        const int e = min((int)threadIdx.x + THREADS * i, CH * CR - 1), t = e / CR, r = e - t * CR;
-#pragma unroll
-        for (int x = 0; x < Q_VECS; x++) row_pre[i][x] = (row_src[x] + base)[(unsigned)t * ld + r];
-    }
-#pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const unsigned at = (unsigned)min(wv + NW * i, CH - 1) * ld + colc;
-#pragma unroll
-        for (int x = 0; x < 5; x++) col_pre[i][x] = (col_src[x] + base)[at];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < RPT; i++) {   // (indices past the end repeat the last: the same value to the same place)
-        const int e = min((int)threadIdx.x + THREADS * i, CH * CR - 1), t = e / CR, r = e - t * CR;
-#pragma unroll
-        for (int x = 0; x < Q_VECS; x++) rows[x][t][r] = row_pre[i][x];
-    }
-#pragma unroll
-    for (int i = 0; i < TPW; i++) {
-        const int t = min(wv + NW * i, CH - 1);
-        const float ew = expf(col_pre[i][0]), d = expf(-ew);
-        in[G_DEC][t][lane] = d, in[G_DDEC][t][lane] = -ew * d;
-        in[G_Q][t][lane] = col_pre[i][1], in[G_K][t][lane] = col_pre[i][2];
-        in[G_A][t][lane] = col_pre[i][3], in[G_B][t][lane] = col_pre[i][4];
-    }
-    __syncthreads();
-    auto row_vals = [&](int x, int t) { return lds_rows<GR>(&rows[x][t][row0]); };
-    struct AdvOps {
-        RowVals<GR> vr, sar;
-        float dec, bv, kv;
+    // Matrix instructions of 16 x 16 x 4: lane (g, n) gives element (n, k = g) of the left operand and (k = g, n) of the right
+    // one and gets elements (4 i + g, n) of the product.  Row r = 16 u + 4 g + s of a state is index g of step (u, s); column
+    // 32 half + 2 n + t is column n of tile t, so that a lane reads two columns of a row and four rows of a token at a time.
+    auto mma = [](double x, double y, d4 acc) { return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc, 0, 0, 0); };
+    float xqv[CH], xav[CH];
+    double z = 0.;
+    d4 gr[4] = {};
+    constexpr int STEPS = CR / 16;
+    struct Rows {   // 16 rows of the states and of the tokens' row vectors
+        f4 row[Q_VECS];
+        f2 S[4], E[4];
     };
-    auto read_adv = [&](int t) { return AdvOps{row_vals(Q_V, t), row_vals(Q_SA, t), in[G_DEC][t][lane], in[G_B][t][lane], in[G_K][t][lane]}; };
-    auto advance = [&](const float (&from)[GR], float (&to)[GR], const AdvOps& o) {
+    auto fetch = [&](int x) {   // those of step x of both halves (past the end: the last ones again)
+        Rows to;
+        const int y = min(x, HALVES * STEPS - 1), half = y >= STEPS, u = y - half * STEPS, c = col0 + HALF * half + 2 * n;
+        const unsigned lane_at = 4 * (4 * g * CR + (CR % COLS == 0 || c < CR ? c : 0));
 #pragma unroll
-        for (int r = 0; r < GR; r++) to[r] = from[r] * o.dec + o.sar.x[r] * o.bv + o.vr.x[r] * o.kv;
-    };
-#pragma unroll 1
-    for (int t0 = CH - GWIN; t0 >= 0; t0 -= GWIN) {
-        float S[GWIN + 1][GR];   // S[t] enters token t0 + t
+        for (int v = 0; v < Q_VECS; v++) to.row[v] = at_bytes<f4>(row_src[v] + (base + 16 * u), 4 * ((unsigned)n * ld + 4 * g));
 #pragma unroll
-        for (int r = 0; r < GR; r++) S[0][r] = Sx[r];
-#pragma unroll 2
-        for (int t = 0; t < t0; t++) advance(S[0], S[0], read_adv(t));
-#pragma unroll
-        for (int t = 0; t < GWIN; t++) {
-            advance(S[t], S[t + 1], read_adv(t0 + t));
-            if (t > GWIN / 2) __builtin_amdgcn_sched_barrier(0);   // (reading further ahead would spill by then)
+        for (int s = 0; s < 4; s++) {
+            const long at = st + (16 * u + s) * CR;
+            to.S[s] = at_bytes<f2>(ckpt + at, lane_at), to.E[s] = at_bytes<f2>(work + at, lane_at);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        return to;
+    };
+    Rows next0 = fetch(0), next1;
+    if (HALVES * STEPS > 1) next1 = fetch(1);
+    float cw[CH], cq[CH], ck[CH], ca[CH], cb[CH];   // the columns of the tokens' vectors
+    const unsigned lane_col = 4 * colc;
 #pragma unroll
-        for (int tw = GWIN - 1; tw >= 0; tw--) {
-            const int t = t0 + tw;
-            const float qv = in[G_Q][t][lane], av = in[G_A][t][lane], dec = in[G_DEC][t][lane];
-            // dq = S_t^T dy;  dS_t += dy q^T;  dk = dS^T v;  db = dS^T sa;  da = S_{t-1}^T dsa;  ddecay: rows of dS * S_{t-1}
-            // (two chains of four rows each: half the rounding of one, and half the operands at a time)
-            float s[2][RED_VECS];
+    for (int half = 0; half < HALVES; half++) {
+        d4 xq[2] = {}, xa[2] = {}, yk[2] = {}, yb[2] = {};
+        double zz[2] = {};
+        auto multiply = [&](const Rows& at) {
 #pragma unroll
-            for (int half = 0; half < 2; half++) {
-                const RowVals<4> dyr = lds_rows<4>(&rows[Q_DY][t][row0 + 4 * half]), vr = lds_rows<4>(&rows[Q_V][t][row0 + 4 * half]);
-                const RowVals<4> sar = lds_rows<4>(&rows[Q_SA][t][row0 + 4 * half]), dsar = lds_rows<4>(&rows[Q_DSA][t][row0 + 4 * half]);
-                float(&u)[RED_VECS] = s[half];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int r = 4 * half + i;
-                    dS[r] += dyr.x[i] * qv;
-                    u[R_DQ] = i ? u[R_DQ] + S[tw + 1][r] * dyr.x[i] : S[tw + 1][r] * dyr.x[i];
-                    u[R_DK] = i ? u[R_DK] + dS[r] * vr.x[i] : dS[r] * vr.x[i];
-                    u[R_DB] = i ? u[R_DB] + dS[r] * sar.x[i] : dS[r] * sar.x[i];
-                    u[R_DA] = i ? u[R_DA] + S[tw][r] * dsar.x[i] : S[tw][r] * dsar.x[i];
-                    u[R_DW] = i ? u[R_DW] + S[tw][r] * dS[r] : S[tw][r] * dS[r];
-                    dS[r] = dS[r] * dec + dsar.x[i] * av;
+            for (int s = 0; s < 4; s++) {
+                const double vr = at.row[Q_V][s], sar = at.row[Q_SA][s], dyr = at.row[Q_DY][s], dsar = at.row[Q_DSA][s];
+                if (half == 0) {
+                    gr[G_SY] = mma(sar, dyr, gr[G_SY]), gr[G_VY] = mma(vr, dyr, gr[G_VY]);
+                    gr[G_SD] = mma(sar, dsar, gr[G_SD]), gr[G_VD] = mma(vr, dsar, gr[G_VD]);
                 }
-                __builtin_amdgcn_sched_barrier(0);
-            }
 #pragma unroll
-            for (int x = 0; x < RED_VECS; x++) red[wv][x][tw % GRED][lane] = s[0][x] + s[1][x];
+                for (int t = 0; t < 2; t++) {
+                    const double Sd = at.S[s][t], Ed = at.E[s][t];
+                    xq[t] = mma(dyr, Sd, xq[t]), xa[t] = mma(dsar, Sd, xa[t]);
+                    yk[t] = mma(vr, Ed, yk[t]), yb[t] = mma(sar, Ed, yb[t]);
+                    zz[t] += Sd * Ed;
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
-            if (tw % GRED == 0) {
-                __syncthreads();
-                // the wavefronts' sums of GRED tokens, in a fixed order, and out
+        };
+        const bool some = CR % COLS == 0 || col0 + HALF * half < CR;   // (a column of this half)
+        int steps = some ? STEPS - (half == HALVES - 1) : 0;
+        asm volatile("" : "+s"(steps));   // (a loop also where it has one step: what follows must not move up into it)
 #pragma unroll 1
-                for (int i = 0; i < (RED_VECS * GRED + NW - 1) / NW; i++) {
-                    const int e = wv + NW * i, x = e / GRED, j = e % GRED;
-                    if (e < RED_VECS * GRED) {
-                        float even = 0.f, odd = 0.f;   // (sums of pairs in two chains)
-#pragma unroll 2
-                        for (int g = 0; g < NW; g += 4) {
-                            even += red[g][x][j][lane] + red[g + 1][x][j][lane];
-                            if (g + 2 < NW) odd += red[g + 2][x][j][lane] + red[g + 3][x][j][lane];
-                        }
-                        float sum = even + odd;
-                        if (x == R_DW) sum *= in[G_DDEC][t + j][lane];
-                        float* const to = x == R_DQ ? dq : x == R_DK ? dk : x == R_DB ? db : x == R_DA ? da : dw;
-                        if (col_ok) (to + base)[(unsigned)(t + j) * ld + colc] = sum;
-                    }
-                }
-                __syncthreads();
+        for (int u = 0; u < steps; u++) {
+            const Rows at = next0;
+            next0 = next1;
+            if (half < HALVES - 1 || u + 2 < STEPS) next1 = fetch(STEPS * half + u + 2);
+            multiply(at);
+        }
+        if (half == HALVES - 1) {
+#pragma unroll
+            for (int t = 0; t < CH; t++) {
+                const long at = base + (long)t * ld;
+                cw[t] = at_bytes<float>(w + at, lane_col), cq[t] = at_bytes<float>(q + at, lane_col);
+                ck[t] = at_bytes<float>(k + at, lane_col), ca[t] = at_bytes<float>(a + at, lane_col), cb[t] = at_bytes<float>(b + at, lane_col);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            if (some) multiply(next0);
+        }
+        // from tokens 4 i + g and columns 2 n + t to a column per lane
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (half == 0 && 4 * i + g <= n) gram[pair(4 * i + g, n)] = d4{gr[G_SY][i], gr[G_VY][i], gr[G_SD][i], gr[G_VD][i]};
+            *reinterpret_cast<f2*>(&xs[0][4 * i + g][2 * n]) = f2{(float)xq[0][i], (float)xq[1][i]};
+            *reinterpret_cast<f2*>(&xs[1][4 * i + g][2 * n]) = f2{(float)xa[0][i], (float)xa[1][i]};
+            *reinterpret_cast<f2*>(&ys[0][4 * i + g][HALF * half + 2 * n]) = f2{(float)yk[0][i], (float)yk[1][i]};
+            *reinterpret_cast<f2*>(&ys[1][4 * i + g][HALF * half + 2 * n]) = f2{(float)yb[0][i], (float)yb[1][i]};
+        }
+        zs[g][2 * n] = zz[0], zs[g][2 * n + 1] = zz[1];
+        __syncthreads();
+        if (HALVES == 1 || lane / HALF == half) {
+#pragma unroll
+            for (int t = 0; t < CH; t++) xqv[t] = xs[0][t][lane % HALF], xav[t] = xs[1][t][lane % HALF];
+            z = (zs[0][lane % HALF] + zs[1][lane % HALF]) + (zs[2][lane % HALF] + zs[3][lane % HALF]);
+        }
+        __syncthreads();
+    }
+    double dec[CH], qv[CH], av[CH], dqv[CH], dav[CH];
+    double P = 1., M = 0.;
+#pragma unroll
+    for (int t = 0; t < CH; t++) {
+        const float ew = expf(cw[t]);
+        es[t][lane] = ew, dec[t] = expf(-ew);
+        qv[t] = cq[t], av[t] = ca[t];
+        dqv[t] = xqv[t], dav[t] = xav[t];
+        M += av[t] * (P * dav[t]);
+        P *= dec[t];
+        M += qv[t] * (P * dqv[t]);
+    }
+    M += P * z;
+    // the pairs i <= j, i upwards and j downwards; the products of row vectors are read AHEAD pairs early
+    constexpr int AHEAD = 1;
+    d4 ahead[AHEAD];
+    int ni = 0, nj = CH - 1, slot = 0;   // (all known at compile time once the loops are unrolled)
+    auto read_next = [&](d4& m) {
+        if (ni < CH) m = gram[pair(ni, nj)];
+        if (nj > ni) nj--;
+        else ni++, nj = CH - 1;
+    };
+#pragma unroll
+    for (int x = 0; x < AHEAD; x++) read_next(ahead[x]);
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+        const double bi = cb[i], ki = ck[i];
+        double dki = ys[0][i][lane], dbi = ys[1][i][lane];
+#pragma unroll
+        for (int j = CH - 1; j >= i; j--) {
+            const d4 m = ahead[slot];
+            read_next(ahead[slot]);
+            slot = (slot + 1) % AHEAD;
+            dqv[j] = dqv[j] * dec[i] + (m[G_SY] * bi + m[G_VY] * ki);
+            dki += m[G_VY] * qv[j], dbi += m[G_SY] * qv[j];
+            if (j > i) {
+                dav[j] = dav[j] * dec[i] + (m[G_SD] * bi + m[G_VD] * ki);
+                dki = dki * dec[j] + m[G_VD] * av[j], dbi = dbi * dec[j] + m[G_SD] * av[j];
+            }
+            asm volatile("" : "+v"(dqv[j]), "+v"(dav[j]), "+v"(dki), "+v"(dbi) : : "memory");   // (else every pair's operands are in registers at once)
+        }
+        const double W = M - av[i] * dav[i];
+        M = W + (bi * dbi + ki * dki) - qv[i] * dqv[i];
+        if (col_ok) {
+            const long at = base + (long)i * ld;
+            at_bytes<float>(dq + at, lane_col) = (float)dqv[i], at_bytes<float>(da + at, lane_col) = (float)dav[i];
+            at_bytes<float>(dk + at, lane_col) = (float)dki, at_bytes<float>(db + at, lane_col) = (float)dbi;
+            at_bytes<float>(dw + at, lane_col) = -es[i][lane] * (dec[i] > 0. ? (float)W : 0.f);   // (W is a difference: not left to cancel)
         }
     }
 }
@@ -744,19 +788,24 @@ void launch_wkv7_f32_backward_split(int B, int T, int H, int C, const float* w, 
                                     float* work, float* dw, float* dq, float* dk, float* dv, float* da, float* db, float* ds0,
                                     hipStream_t stream) {
     launch_scan<true>(B, T, H, C, w, q, k, dy, a, b, dsT, dv, work, ds0, stream);
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(B * H * (T / CH64), (C + 63) / 64), dim3(64 * (C / GR)), 0, stream, T, H, w, q, k, v, a, b, dy, ckpt,
-                           work, dw, dq, dk, da, db);
+    // 64 columns a wavefront; 32 where a head has no more, and while the wavefronts are few enough for the wait for the matrix
+    // instructions of half as many columns to count for more than half the lanes idling: up to one wavefront per SIMD (us in
+    // 64 / 32 columns, 64 channels: 64 chunks 20.3/16.5, 256 24.1/22.2, 512 28.7/29.1; 128 channels, 8 chunks 30.7/23.7)
+    const bool narrow = C <= 32 || (long)B * H * (T / CH64) * ((C + 31) / 32) <= 4 * compute_units();
+    auto go = [&](auto kernel, auto narrow_kernel) {
+        const int cols = narrow ? 32 : 64;
+        hipLaunchKernelGGL(narrow ? narrow_kernel : kernel, dim3(B * H * (T / CH64), (C + cols - 1) / cols), dim3(64), 0, stream, T, H, w, q, k,
+                           v, a, b, dy, ckpt, work, dw, dq, dk, da, db);
     };
     switch (C) {
-        case 16: go(wkv7_f32_grads_kernel<16>); break;
-        case 32: go(wkv7_f32_grads_kernel<32>); break;
-        case 48: go(wkv7_f32_grads_kernel<48>); break;
-        case 64: go(wkv7_f32_grads_kernel<64>); break;
-        case 80: go(wkv7_f32_grads_kernel<80>); break;
-        case 96: go(wkv7_f32_grads_kernel<96>); break;
-        case 112: go(wkv7_f32_grads_kernel<112>); break;
-        default: go(wkv7_f32_grads_kernel<128>);
+        case 16: go(wkv7_f32_grads_kernel<16, 32>, wkv7_f32_grads_kernel<16, 32>); break;
+        case 32: go(wkv7_f32_grads_kernel<32, 32>, wkv7_f32_grads_kernel<32, 32>); break;
+        case 48: go(wkv7_f32_grads_kernel<48, 64>, wkv7_f32_grads_kernel<48, 32>); break;
+        case 64: go(wkv7_f32_grads_kernel<64, 64>, wkv7_f32_grads_kernel<64, 32>); break;
+        case 80: go(wkv7_f32_grads_kernel<80, 64>, wkv7_f32_grads_kernel<80, 32>); break;
+        case 96: go(wkv7_f32_grads_kernel<96, 64>, wkv7_f32_grads_kernel<96, 32>); break;
+        case 112: go(wkv7_f32_grads_kernel<112, 64>, wkv7_f32_grads_kernel<112, 32>); break;
+        default: go(wkv7_f32_grads_kernel<128, 64>, wkv7_f32_grads_kernel<128, 32>);
     }
 }
 
