@@ -38,6 +38,12 @@ def test_step_over_the_dispatch_of_its_kernels(B, H, state_dtype):
     assert seq_ref.rel_err(Sg.float().cpu(), Sw.float().cpu()) <= (2e-3 if state_dtype == torch.float32 else 8e-3)
 
 
+# rows no multiple of 16 or 64 and one past a multiple, heads past 256 and 2048 channels; the last also with the output grouped
+@pytest.mark.parametrize('B,H', [(161, 13), (33, 35), (257, 12), (400, 29)])
+def test_step_with_the_streams_in_memory(B, H):
+    test_step_over_the_dispatch_of_its_kernels(B, H, torch.float32)
+
+
 @pytest.mark.parametrize('B,T,H', [(1, 3, 2), (5, 17, 3), (8, 63, 12)])
 def test_a_few_tokens_equal_as_many_steps(B, T, H):
     """Within one rounding of the outputs: the same kernels' arithmetic, the state in registers between the tokens (fp32)."""

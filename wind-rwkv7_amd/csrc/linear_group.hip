@@ -34,7 +34,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 using Rsrc = __amdgpu_buffer_rsrc_t;
 
 constexpr int BK = 64;           // contraction indices per stage: whole 128-byte lines of a row
-constexpr int MAX_PROBLEMS = 8;
+constexpr int MAX_PROBLEMS = LINEAR_GROUP_MAX;
 
 template <int TMB, int TNB>
 struct Tile {

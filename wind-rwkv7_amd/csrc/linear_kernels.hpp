@@ -76,6 +76,7 @@ struct LinearProblem {
     long ld_out[PIECES];
     int start[PIECES], width[PIECES], op[PIECES];
 };
+constexpr int LINEAR_GROUP_MAX = 9;   // problems of a launch
 void launch_linear_group(int n, long M, const LinearProblem* problems, hipStream_t stream);
 
 }  // namespace wkv

@@ -8,7 +8,8 @@
 //   1. mid      the token shift's first product with tanh (rwkv7_ddlerp.py:20-49), 16 of its 128 columns per block
 //   2. linear   all first-half products (time_mixer.py:120-131) - r, k, v and the six LoRA first halves, nine weight
 //               matrices - in one launch; a block computes the interpolated stream (rwkv7_ddlerp.py:53-84) it multiplies
-//               itself, 32 channels at a time, so the four streams never exist in memory
+//               itself, 32 channels at a time, so the four streams never exist in memory (for many rows they do, a launch
+//               more: `streams_in_memory`)
 //   3. head     per (tile, head): the LoRA second halves with the elementwise tail (rwkv7_expand_loras.py:33-70), the gate's
 //               and the decay's second halves, then the single-token WKV7 recurrence with GroupNorm, bonus and gate
 //   4. linear   the output projection
@@ -21,6 +22,7 @@
 #include "mixer_decode_kernels.hpp"
 
 #include "device_info.hpp"
+#include "linear_kernels.hpp"
 #include "frag.hpp"
 #include "ln_epilogue.hpp"
 #include "wkv7_common.hpp"
@@ -142,6 +144,27 @@ __global__ __launch_bounds__(64 * NW) void decode_mid_kernel(const MixIn in, int
 #pragma unroll
     for (int r = 0; r < 4; r++) t[r] = tanhf_(t[r]);
     *reinterpret_cast<bf16x4*>(in.mid + (long)row * MID + 16 * ob + 4 * L.g) = to_bf16(t);
+}
+
+// The four interpolated streams y_k = x + xx (mid_k R_k^T + beta_k) in memory, for the products of many rows: block = 32
+// channels x one 16-row tile, a wavefront per stream.
+__global__ __launch_bounds__(256) void decode_lerp_kernel(const MixIn in, int C, __bf16* __restrict__ y, long stream_stride) {
+    const int ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Lane L;
+    const int row = blockIdx.y * TOK + L.n, c = 32 * blockIdx.x + 8 * L.g;
+    const TokenRows tr = token_rows(in, row, C);
+    const bf16x8 bm = *reinterpret_cast<const bf16x8*>(in.mid + (long)row * MID + R_MIX * ks + 8 * L.g);
+    // row j of the two R fragments: channel 8(n/4) + 4j + n%4, so that the products are the lane's eight channels 8g .. 8g+7
+    const __bf16* rrow = in.R + ((long)ks * C + 32 * blockIdx.x + 8 * (L.n >> 2) + (L.n & 3)) * R_MIX + 8 * L.g;
+    const bf16x8 r0 = *reinterpret_cast<const bf16x8*>(rrow), r1 = *reinterpret_cast<const bf16x8*>(rrow + 4 * R_MIX);
+    const bf16x8 be = *reinterpret_cast<const bf16x8*>(in.beta + (long)ks * C + c);
+    const bf16x8 xv = *reinterpret_cast<const bf16x8*>(in.x + tr.at + c);
+    const bf16x8 pv = or_zero(*reinterpret_cast<const bf16x8*>(tr.prev_of + tr.prev + c), tr.zero);
+    const f32x4 c0 = mma8(to_f32(lo4(be)), r0, bm), c1 = mma8(to_f32(hi4(be)), r1, bm);   // lane = token
+    const f32x4 x0 = to_f32(lo4(xv)), x1 = to_f32(hi4(xv));
+    if (row < in.rows)
+        *reinterpret_cast<bf16x8*>(y + ks * stream_stride + (long)row * C + c) =
+            cat8(to_bf16(x0 + (to_f32(lo4(pv)) - x0) * c0), to_bf16(x1 + (to_f32(hi4(pv)) - x1) * c1));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -546,8 +569,8 @@ constexpr int LIN_BLOCKS = 400, LIN_SINGLE_BLOCKS = 320;
 
 }  // namespace
 
-// B: tokens in all (sequences times tokens per sequence).  (Four planes and the hidden activation are used and thirteen planes asked for: callers size the
-// workspace with this, some with the number of an earlier release, and nothing is gained by less: 768 channels, 256
+// B: tokens in all (sequences times tokens per sequence).  (Four planes, eight with the streams in memory, and the hidden
+// activations are used and thirteen planes asked for: callers size the workspace with this, some with the number of an earlier release, and nothing is gained by less: 768 channels, 256
 // sequences 5 MB.)
 size_t mixer_decode_workspace_bytes(int B, int C) {
     const size_t Bp = padded_rows(B);
@@ -563,6 +586,16 @@ int head_rows_per_block(int B, int H) {
     while (rpb < 8 && (long)H * ((B + rpb - 1) / rpb) > compute_units()) rpb *= 2;
     return rpb;
 }
+// The first-half products of many rows: every column block of the linear kernel makes its stream again, so from some rows on
+// the streams are written once (decode_lerp_kernel, a launch more) and multiplied by the grouped kernel of the sequence path,
+// whose tiles share both operands through LDS.  us, linear / lerp + grouped: 768 channels 128 rows 13.3/13.2, 192 17.0/13.3,
+// 256 18.1/13.8, 512 25.0/17.3; 1024 channels 128 rows 14.8/14.4; 1280 channels 96 rows 17.0/15.9; 2048 channels 32 rows
+// 19.6/20.8, 48 33.3/21.2, 128 38.9/22.2, 256 73.5/27, 512 133/57 (and the launch costs about one).
+bool streams_in_memory(long rows, long C) { return rows * C * C >= (rows >= 160 ? 110000000 : 160000000) && rows > 32; }
+// The output projection alone makes nothing again, and the grouped kernel's tiles are few for it (2048 channels, 256 rows
+// 14.2/17.8 us, 512 rows 27.8/18.4; 1536 channels, 512 rows 19.8/15).
+bool output_grouped(long rows, long C) { return rows * C * C >= 1200000000; }
+
 template <bool LERP>
 void launch_linear(const LinArgs& a, const MixIn& mix, hipStream_t stream) {
     auto blocks = [&](int columns) {
@@ -621,7 +654,23 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         a.C = C;
         a.rows = Bp;
         a.ntiles = ntiles;
-        launch_linear<true>(a, mix, stream);
+        if (streams_in_memory(rows, C)) {
+            const long plane = (long)Bp * C;
+            __bf16* const streams = take(4 * BC);
+            hipLaunchKernelGGL(decode_lerp_kernel, dim3(C / 32, ntiles), dim3(256), 0, stream, mix, C, streams, plane);
+            LinearProblem p[MAX_SEGS]{};
+            for (int i = 0; i < a.nseg; i++) {
+                const LinSeg& s = a.seg[i];
+                p[i].A[0] = streams + s.stream * plane, p[i].W[0] = s.W;
+                p[i].lda[0] = p[i].ldw[0] = p[i].K[0] = C;
+                p[i].N = s.N, p[i].npieces = 1;
+                p[i].out[0] = s.out, p[i].ld_out[0] = p[i].width[0] = s.N;
+                p[i].op[0] = s.tanh_out ? LINEAR_TANH : LINEAR_PLAIN;
+            }
+            launch_linear_group(a.nseg, rows, p, stream);
+        } else {
+            launch_linear<true>(a, mix, stream);
+        }
     }
     {
         const HeadArgs a{rows, T, C, H, state_f32, r, k, v, tg1, tw1, kk1, mk1, a1, ma1,
@@ -644,7 +693,15 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         a.C = C;
         a.rows = rows;
         a.ntiles = ntiles;
-        launch_linear<false>(a, mix, stream);
+        if (output_grouped(rows, C)) {
+            LinearProblem p{};
+            p.A[0] = ya, p.W[0] = c(mw.Wo);
+            p.lda[0] = p.ldw[0] = p.K[0] = p.N = C;
+            p.npieces = 1, p.out[0] = static_cast<__bf16*>(y), p.ld_out[0] = p.width[0] = C;
+            launch_linear_group(1, rows, &p, stream);
+        } else {
+            launch_linear<false>(a, mix, stream);
+        }
     }
 }
 
