@@ -279,6 +279,18 @@ def test_split_columns_more_pieces_than_one_launch():
     assert torch.equal(a.grad, torch.cat(gs, dim=-1))
 
 
+# (768 x 768: 16 token ranges, 32 x 256: 256) the tokens of a range: below, at and past the first rounds of whole steps
+@pytest.mark.parametrize('O,I,ranges', [(768, 768, 16), (32, 256, 256)])
+@pytest.mark.parametrize('steps,extra', [(9, 0), (10, 0), (10, 5), (11, 31), (13, 0), (14, 1), (21, 17)])
+def test_linear_wgrad_rounds_of_whole_steps(O, I, ranges, steps, extra):
+    """Small whole numbers: every sum is exact in fp32, whatever its order, so not one token may be missed or counted twice."""
+    from wind_rwkv.rwkv7 import linear_wgrad
+    tokens = 32 * ranges * steps + extra
+    g = torch.Generator(DEV).manual_seed(tokens)
+    dy, x = [torch.randint(-2, 3, (tokens, n), generator=g, device=DEV).bfloat16() for n in (O, I)]
+    assert torch.equal(linear_wgrad(dy, x, torch.float32), (dy.double().T @ x.double()).float())
+
+
 @pytest.mark.parametrize('tokens,shapes', [
     (4096, [(768, 768), (768, 768), (768, 768)]),          # the time mixer's r, k, v projections
     (1000, [(896, 768), (160, 1024), (768, 144), (208, 400)]),   # both orientations, ragged sizes and token count

@@ -23,6 +23,8 @@
 #include "linear_kernels.hpp"
 #include "device_info.hpp"
 
+#include <type_traits>
+
 #include "frag.hpp"
 
 namespace wkv {
@@ -146,6 +148,21 @@ __device__ __forceinline__ void wgrad_block(WgradLds<S>& lds, const WgradArgs& g
         else
             *reinterpret_cast<bf16x8*>(b_dst[piece - QA] + buf * (STEP * S::PB)) = keep ? rb[set][piece - QA] : zero8;
     };
+    // The same where every step concerned is a whole one: no masks, and the loads as (scalar base of the step) + (32-bit byte
+    // offset), which a row stride of up to 2^25 elements allows.
+    unsigned a_bytes[QA], b_bytes[QB];
+#pragma unroll
+    for (int q = 0; q < QA; q++) a_bytes[q] = 2 * a_off[q];
+#pragma unroll
+    for (int q = 0; q < QB; q++) b_bytes[q] = 2 * b_off[q];
+    auto fetch_whole = [&](int set, const __bf16* a_step, const __bf16* b_step, int piece) {
+        if (piece < QA) ra[set][piece] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(a_step) + a_bytes[piece]);
+        else rb[set][piece - QA] = *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(b_step) + b_bytes[piece - QA]);
+    };
+    auto stage_whole = [&](int set, int buf, int piece) {
+        if (piece < QA) *reinterpret_cast<bf16x8*>(a_dst[piece] + buf * (STEP * S::PA)) = ra[set][piece];
+        else *reinterpret_cast<bf16x8*>(b_dst[piece - QA] + buf * (STEP * S::PB)) = rb[set][piece - QA];
+    };
     auto fetch = [&](int set, int step) {
 #pragma unroll
         for (int q = 0; q < PIECES; q++) fetch_one(set, step, q);
@@ -204,26 +221,47 @@ __device__ __forceinline__ void wgrad_block(WgradLds<S>& lds, const WgradArgs& g
         __syncthreads();
 #pragma unroll
         for (int n = 0; n < READS; n++) read_one(0, 0, n);
-        for (int base = 0; base < nsteps; base += DEPTH) {
+        auto step = [&](auto whole, int base, int k, const __bf16* a_step, const __bf16* b_step) {
+            __syncthreads();
+            // Issue order, pinned: before matrix instruction i its share of the step's transposed reads (for
+            // step s + 1), of the 16-byte LDS writes (step s + 2) and of the global loads (step s + 2 + DEPTH).
+            // An even spread measured best; bunching the LDS traffic early in the step costs 9 %.
 #pragma unroll
-            for (int k = 0; k < DEPTH; k++) {
-                __syncthreads();
-                // Issue order, pinned: before matrix instruction i its share of the step's transposed reads (for
-                // step s + 1), of the 16-byte LDS writes (step s + 2) and of the global loads (step s + 2 + DEPTH).
-                // An even spread measured best; bunching the LDS traffic early in the step costs 9 %.
+            for (int i = 0; i < MFMAS; i++) {
 #pragma unroll
-                for (int i = 0; i < MFMAS; i++) {
+                for (int n = READS * i / MFMAS; n < READS * (i + 1) / MFMAS; n++) read_one((k + 1) & 1, (k + 1) & 1, n);
 #pragma unroll
-                    for (int n = READS * i / MFMAS; n < READS * (i + 1) / MFMAS; n++) read_one((k + 1) & 1, (k + 1) & 1, n);
-#pragma unroll
-                    for (int q = PIECES * i / MFMAS; q < PIECES * (i + 1) / MFMAS; q++) {
+                for (int q = PIECES * i / MFMAS; q < PIECES * (i + 1) / MFMAS; q++) {
+                    if constexpr (decltype(whole)::value) {
+                        stage_whole((k + 2) % DEPTH, k & 1, q);
+                        fetch_whole((k + 2) % DEPTH, a_step, b_step, q);
+                    } else {
                         stage_one((k + 2) % DEPTH, k & 1, base + k + 2, q);
                         fetch_one((k + 2) % DEPTH, base + k + 2 + DEPTH, q);
                     }
-                    multiply_one(k & 1, i);
-                    __builtin_amdgcn_sched_barrier(0);
+                }
+                multiply_one(k & 1, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int base = 0;
+        if (g.lda <= 1 << 25 && g.ldb <= 1 << 25) {
+            // Rounds in which everything staged and fetched is a whole step.  The masks, selects and pointer choices of the other
+            // rounds are half of their 143 instructions a step, and with one wavefront per SIMD nothing hides them: the
+            // gradients of a 768-channel block's nine products, 8192 tokens, 77.6 -> 69.6 us (18 matrix instructions of 32 cycles
+            // a step of 1440; 4 row pitches of other bank offsets, 32 bytes or 64, 69.4).
+            const __bf16 *a_step = a_first + (long)(2 + DEPTH) * STEP * g.lda, *b_step = b_first + (long)(2 + DEPTH) * STEP * g.ldb;
+            for (; base + 2 * DEPTH + 1 < nfull; base += DEPTH) {
+#pragma unroll
+                for (int k = 0; k < DEPTH; k++) {
+                    step(std::true_type(), base, k, a_step, b_step);
+                    a_step += STEP * g.lda, b_step += STEP * g.ldb;
                 }
             }
+        }
+        for (; base < nsteps; base += DEPTH) {
+#pragma unroll
+            for (int k = 0; k < DEPTH; k++) step(std::false_type(), base, k, nullptr, nullptr);
         }
     }
 
