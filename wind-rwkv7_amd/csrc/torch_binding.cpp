@@ -700,7 +700,7 @@ struct Products {
     }
 };
 
-// dW = dy^T x for several pairs on the same tokens, in one grouped launch or in two (a single pair goes through its own entry point)
+// dW = dy^T x for several pairs on the same tokens: one grouped launch (a single pair goes through its own entry point)
 struct WeightGrads {
     std::vector<int> O, I;
     std::vector<const void*> dy, x;
@@ -710,21 +710,15 @@ struct WeightGrads {
         dy.push_back(d), O.push_back(o), ld_dy.push_back(o), x.push_back(a), I.push_back(i), ld_x.push_back(i), dW.push_back(w);
     }
     void run(int64_t tokens, const Tensor& like, void* stream) {
-        const int n = (int)O.size(), first = n > WIND_RWKV7_WGRAD_GROUP_MAX ? n / 2 : n;
-        run(0, first, tokens, like, stream);
-        run(first, n, tokens, like, stream);
-    }
-    void run(int from, int to, int64_t tokens, const Tensor& like, void* stream) {
-        const int n = to - from;
+        const int n = (int)O.size();
         if (n == 0) return;
         if (n == 1) {
-            const Tensor ws = scratch_bytes(L.linear_wgrad_workspace_bytes(tokens, O[from], I[from]), like);
-            check(L.linear_wgrad(tokens, O[from], I[from], dy[from], ld_dy[from], x[from], ld_x[from], dW[from], WIND_RWKV7_F32, ptr(ws), ws.numel(),
-                                 stream));
+            const Tensor ws = scratch_bytes(L.linear_wgrad_workspace_bytes(tokens, O[0], I[0]), like);
+            check(L.linear_wgrad(tokens, O[0], I[0], dy[0], ld_dy[0], x[0], ld_x[0], dW[0], WIND_RWKV7_F32, ptr(ws), ws.numel(), stream));
             return;
         }
-        const Tensor ws = scratch_bytes(L.linear_wgrad_group_workspace_bytes(n, tokens, &O[from], &I[from]), like);
-        check(L.linear_wgrad_group(n, tokens, &O[from], &I[from], &dy[from], &ld_dy[from], &x[from], &ld_x[from], &dW[from], WIND_RWKV7_F32,
+        const Tensor ws = scratch_bytes(L.linear_wgrad_group_workspace_bytes(n, tokens, O.data(), I.data()), like);
+        check(L.linear_wgrad_group(n, tokens, O.data(), I.data(), dy.data(), ld_dy.data(), x.data(), ld_x.data(), dW.data(), WIND_RWKV7_F32,
                                    ptr(ws), ws.numel(), stream));
     }
 };
@@ -902,9 +896,12 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         const bool kept = G.at[i] < G.kept;
         return static_cast<float*>((kept ? flat : unwanted).data_ptr()) + G.at[i] - (kept ? 0 : G.kept);
     };
-    WeightGrads wg;   // (together at the end: everything that they multiply is kept until then)
-    if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
-    if (!st.attn) return wg.run(M, dout, stream);
+    {
+        WeightGrads wg;
+        if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
+        wg.run(M, dout, stream);
+    }
+    if (!st.attn) return;
     if (G.total > G.kept) unwanted = at::empty({G.total - G.kept}, flat.options());
     const WeightLayout W(C);
     const Activations A(s, true);
@@ -954,14 +951,15 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         }
         p.run(M, xb);
     }
-    if (need(WV)) wg.add(d(4 * P), C, a(A.streams + 3 * P), C, g(WV));
-    if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
-    if (need(DECAY_W2)) wg.add(d(0), C, a(A.tw1), R_DECAY, g(DECAY_W2));
+    WeightGrads wg;   // (all at the end: everything that they multiply is kept until then)
     if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
     if (need(GATE_W1)) wg.add(d(o_g1), R_GATE, a(A.streams), C, g(GATE_W1));
     if (need(WK)) wg.add(d(8 * P), C, a(A.streams + 2 * P), C, g(WK));
     if (need(KKK_W1) || need(MK_W1)) wg.add(dkkmk, W_KKMK, a(A.streams + 2 * P), C, g(KKK_W1));
+    if (need(WV)) wg.add(d(4 * P), C, a(A.streams + 3 * P), C, g(WV));
     if (need(DECAY_W1) || need(AAA_W1) || need(MA_W1)) wg.add(dw1, W_DECAY_AAA_MA, a(A.streams + P), C, g(DECAY_W1));
+    if (need(GATE_W2)) wg.add(d(7 * P), C, a(A.tg1), R_GATE, g(GATE_W2));
+    if (need(DECAY_W2)) wg.add(d(0), C, a(A.tw1), R_DECAY, g(DECAY_W2));
     wg.run(M, xb, stream);
     if (st.streams)
         check(L.ddlerp_backward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), dxrg, dxwa, dxk, dxv, ptr(dx),
