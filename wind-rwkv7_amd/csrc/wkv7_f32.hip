@@ -16,8 +16,10 @@
 // wavefronts of a block carry the recurrence and touch LDS only; four more fetch the next chunk, turn it into operands in
 // the other half of a double buffer and carry the results of the chunk before to memory, with one barrier per chunk.
 // (Staging by the recurrence's own wavefronts, between barriers, was a fifth of its time: 227 -> 183 us at 8 x 1024 tokens
-// x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  What bounds it now is LDS: a wavefront reads five vectors of
-// 64 channels per token, 360 of the 400 cycles that a token takes with eight wavefronts on a compute unit.
+// x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  Bound: vector issue, 89 % of the cycles with eight wavefronts of
+// the recurrence on a compute unit, so what can wait is done for many tokens at once: the row sums of S (decay q) for four
+// (quad_sums), what the row vectors add to y once per chunk by the lane that keeps a token (518 -> 463 instructions per
+// chunk; forward / backward scan 183 / 187 -> 166 / 181 us, 6 heads of 128 384 / 375 -> 325 / 336).
 // The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
 // direction (it keeps the state gradient arriving at every chunk's end and dsa of every token, and leaves dv and ds0)
 // and then a kernel in which every chunk is on its own and makes the other five gradients.
@@ -142,12 +144,29 @@ __device__ __forceinline__ void store_col_sums(float* to, f4 p, int col0, int ib
     }
 }
 
-// sum over the 64 lanes of a wavefront, result in all of them
-__device__ __forceinline__ float wave_sum(float x) {
-    x = row_sum16(x);
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    return x;
+// Several values at once summed over lanes, each lane ending up with ONE of the sums: a halving of the values is a select of
+// what a lane keeps, one of what it gives away and an add.  pair_sums: over the 64 lanes, lane l gets the sum of x z (l even)
+// or y z (l odd); a multiply-add takes the kept product, which is not rounded by itself.  quad_sums: over the LPR lanes of a
+// state row, lane l gets that of x[l % 4], in eleven instructions (and a swap) for four sums that would be sixteen one by
+// one, four swaps and four selects.
+__device__ __forceinline__ float pair_sums(float x, float y, float z, int lane) {
+    const bool odd = lane & 1;
+    float s = fmaf(odd ? y : x, z, dpp<0xB1>((odd ? x : y) * z));   // quad_perm [1,0,3,2]
+    s += dpp<0x4E>(s);                                              // quad_perm [2,3,0,1]
+    s += dpp<0x124>(s);                                             // row_ror 4
+    s += dpp<0x128>(s);                                             // row_ror 8
+    s = swap_add16(s, s);
+    return swap_add32(s, s);
+}
+template <int LPR>
+__device__ __forceinline__ float quad_sums(const float (&x)[4], int lane) {
+    const bool odd = lane & 1, upper = lane & 2;
+    const float lo = (odd ? x[1] : x[0]) + dpp<0xB1>(odd ? x[0] : x[1]), hi = (odd ? x[3] : x[2]) + dpp<0xB1>(odd ? x[2] : x[3]);
+    float s = (upper ? hi : lo) + dpp<0x4E>(upper ? lo : hi);
+    s += dpp<0x124>(s);
+    s += dpp<0x128>(s);
+    if constexpr (LPR == 32) s = swap_add16(s, s);
+    return s;
 }
 
 // What the forward keeps for the backward, in one buffer: the state entering every CH64 tokens ([B,H,T/CH64,C,C]) and
@@ -191,7 +210,7 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
     // ---- moving data: thread ptid of PT ----
     const int ptid = threadIdx.x - 64 * NW, pch = ptid % C;
     const bool stage_ok = FULL || pch < CR;
-    const unsigned tok_off = (unsigned)(ptid / C) * ld + (stage_ok ? pch : 0);   // (token, channel) this thread stages
+    const unsigned tok_off = 4 * ((unsigned)(ptid / C) * ld + (stage_ok ? pch : 0));   // (token, channel) this thread stages, in bytes
     float pre[FWD_VECS][PER];
     auto fetch = [&](int n) {
         const long base = chunk_base(n < NC ? n : NC - 1);   // (past the last chunk: the same one again, not used)
@@ -199,7 +218,7 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
         for (int vec = 0; vec < FWD_VECS; vec++) {
 #pragma unroll
             for (int j = 0; j < PER; j++) {
-                const float x = (src[vec] + base)[tok_off + (unsigned)(TPJ * j) * ld];
+                const float x = at_bytes<float>(src[vec] + (base + (long)(TPJ * j) * ld), tok_off);
                 pre[vec][j] = stage_ok ? x : 0.f;
             }
         }
@@ -218,8 +237,8 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
             in[buf][V_V][tok][pch] = pre[V_V][j];
             in[buf][V_A][tok][pch] = pre[V_A][j];
             in[buf][V_B][tok][pch] = pre[V_B][j];
-            const float bq = wave_sum(pre[V_B][j] * pre[V_Q][j]), kq = wave_sum(pre[V_K][j] * pre[V_Q][j]);
-            if (lane == 0) bkq[buf][tok][pch >> 6] = f2{bq, kq};
+            const float bkq_lane = pair_sums(pre[V_B][j], pre[V_K][j], pre[V_Q][j], lane);   // lane 0: b . q, lane 1: k . q
+            if (lane < 2) reinterpret_cast<float*>(&bkq[buf][tok][pch >> 6])[lane] = bkq_lane;
         }
     };
     auto copy_out = [&](int n, int buf) {
@@ -271,7 +290,7 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
         struct Ops {
             f4 dec, x1, x2, u1, u2;   // operands of the two row sums, column vectors of the two rank-one terms
             RowVals<R> vr;
-            f2 sc;
+            float bq;
         };
         auto read_ops = [&](int t) {
             Ops o;
@@ -281,39 +300,50 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
             o.u2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_Q : V_K][t][col0]);
             o.x2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_K : V_Q][t][col0]);
             o.vr = lds_rows<R>(&in[buf][V_V][t][row0]);
-            o.sc = bkq[buf][t][0];
-            if constexpr (NH == 2) o.sc += bkq[buf][t][1];
+            if constexpr (ADJ) {
+                o.bq = bkq[buf][t][0][0];
+                if constexpr (NH == 2) o.bq += bkq[buf][t][1][0];
+            }
             return o;
         };
         Ops ahead = read_ops(ADJ ? CH - 1 : 0);
         RowVals<R> ykeep = {}, sakeep = {};
+        float ypart[R][4];   // four tokens' terms of S (decay * q)
 #pragma unroll
         for (int i = 0; i < CH; i++) {
             const int t = ADJ ? CH - 1 - i : i;
             const Ops o = ahead;
             if (i + 1 < CH) ahead = read_ops(ADJ ? t - 1 : t + 1);
             asm volatile("" ::: "memory");   // (else all sixteen tokens' operands are requested at once)
-            RowVals<R> yr, sar;
+            RowVals<R> sar;
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 sar.x[r] = row_sum<LPR>(dot4(S[r], o.x1));
-                if constexpr (ADJ) sar.x[r] += o.vr.x[r] * o.sc[0];
-                yr.x[r] = row_sum<LPR>(dot4(S[r], o.x2)) + o.vr.x[r] * o.sc[1];
-                if constexpr (!ADJ) yr.x[r] += sar.x[r] * o.sc[0];
+                if constexpr (ADJ) sar.x[r] += o.vr.x[r] * o.bq;
+                ypart[r][t % 4] = dot4(S[r], o.x2);
                 S[r] = S[r] * o.dec + sar.x[r] * o.u1 + o.vr.x[r] * o.u2;
             }
             // lane t of a row's lanes keeps token t's results (a store per token by one lane would be a branch per token,
             // which nothing is scheduled across); 32 lanes per row: both of its DPP rows hold and store the same
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                ykeep.x[r] = jb % CH == t ? yr.x[r] : ykeep.x[r];
                 sakeep.x[r] = jb % CH == t ? sar.x[r] : sakeep.x[r];
-                asm volatile("" : "+v"(ykeep.x[r]));   // (here and now: put off, it keeps every token's operands alive)
+                if (i % 4 == 3) {
+                    const float y4 = quad_sums<LPR>(ypart[r], lane);
+                    ykeep.x[r] = jb % CH / 4 == t / 4 ? y4 : ykeep.x[r];
+                }
+                asm volatile("" : "+v"(sakeep.x[r]));   // (here and now: put off, it keeps every token's operands alive)
             }
         }
+        // what the row vectors add to y, once for the token that a lane keeps
+        f2 sc = bkq[buf][jb % CH][0];
+        if constexpr (NH == 2) sc += bkq[buf][jb % CH][1];
+        const RowVals<R> vr = lds_rows<R>(&in[buf][V_V][jb % CH][row0]);
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            yout[buf][jb % CH][rl + r] = ykeep.x[r];
+            float yr = ykeep.x[r] + vr.x[r] * sc[1];
+            if constexpr (!ADJ) yr += sakeep.x[r] * sc[0];
+            yout[buf][jb % CH][rl + r] = yr;
             saout[buf][jb % CH][rl + r] = sakeep.x[r];
         }
     };
