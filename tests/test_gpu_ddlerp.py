@@ -59,6 +59,13 @@ def test_ddlerp_around_the_few_token_limit(B, T, C, D):
     check(*run_both(B, T, C, D, seed=500 + T + D))
 
 
+# an odd count of tiles beyond the few-token limit, and an odd count of channel blocks for the two images: one and three
+@pytest.mark.parametrize('D', [32, 64])
+@pytest.mark.parametrize('B,T,C', [(1, 4112, 64), (257, 16, 192)])
+def test_ddlerp_odd_channel_blocks(B, T, C, D):
+    check(*run_both(B, T, C, D, seed=600 + T + D))
+
+
 # rank 64 (two 32-wide contractions per interpolation; the second backward pass keeps its weight fragments in
 # registers): a single tile, a ragged count of tiles, the two- and four-tiles-per-block kernels, 64 channel blocks
 @pytest.mark.parametrize('B,T,C', [(1, 16, 64), (2, 48, 128), (3, 64, 768), (8, 1024, 768), (17, 976, 256), (2, 4112, 128),

@@ -65,42 +65,58 @@ __device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, long 
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
-// The two contractions over all C channels (forward 1 and backward 1) give a block TPB token tiles (16 tokens
-// each) and walk the channel blocks: the weight fragments of a channel block (16 KiB) are loaded once per block,
-// passed through a double-buffered LDS image in matrix-instruction order (one barrier per channel block), and
-// each tile is finished by 4 / TPB wavefronts, which split the output blocks.  A tile per block with the channel
-// contraction split over its wavefronts, as a first version had it, fetched the whole 196 KiB of weights from
-// L2 for every 16 tokens (1.6x the streamed bytes at C = 768) and needed a cross-wavefront reduction.
+// The two contractions over all C channels (forward 1 and backward 1) give a block TPB token tiles (16 tokens each) and
+// walk the channel blocks of 64: eight lanes fetch the 128 bytes of one row of a channel block, of the weights as of the
+// streams, a thread does the elementwise part for its eight channels of a token once, and everything passes through a
+// double-buffered LDS image from which the matrix instructions take their fragments (one barrier per channel block); each
+// tile is finished by 4 / TPB wavefronts, which split the output blocks.
+// What bounds these kernels is the number of lookups of a compute unit's vector cache: four lanes on four rows, the order
+// of a fragment, are four lookups, and a wavefront's 16-byte load takes 28 ns of the compute unit, against 9 for eight lanes
+// on each whole line (measured with everything in L2; stores 28 and 20).  Fragments straight from memory took 16.8 (forward 1)
+// and 22.2 us (backward 1) at 8192 tokens x 768 channels, no less with twice the wavefronts; this way 11.2 and 14.4, and 17.5
+// and 34.5 at 16384 tokens instead of 24.5 and 38.5.  What is left is a round of load, LDS and barrier per channel block,
+// which neither two blocks of channels at a time nor four sets of operands in flight made shorter; backward 1 moves 63 MB at
+// 8192 tokens, 12.4 us at the rate of a copy.
 // ------------------------------------------------------------------------------------------------
-template <int NB>
-struct MidWeights {   // LDS image of the weights of one 64-channel block: [output block][channel pair][lane]
-    bf16x8 f[2][NB][2][WAVE];
+// 16-byte pieces of rows of 64 channels.  A fragment read takes piece 4pr + g of 16 rows: eight pieces of two rows lie in
+// different banks, so the pieces of a pair of rows are permuted by the pair's number.
+__device__ __forceinline__ int piece_slot(int row, int piece) { return 8 * row + (piece ^ ((row >> 1) & 7)); }
+// the bytes at a 32-bit offset from a wavefront-uniform address: no 64-bit address per load
+__device__ __forceinline__ bf16x8 piece_at(const __bf16* base, unsigned bytes) {
+    return *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(base) + bytes);
+}
+// LDS instructions of one wavefront run in their order: what its lanes have written, the others of them may read
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bf16x4 half_of(const bf16x8 v, int hlf) {
+    return hlf ? __builtin_shufflevector(v, v, 4, 5, 6, 7) : __builtin_shufflevector(v, v, 0, 1, 2, 3);
+}
+__device__ __forceinline__ bf16x8 join(const bf16x4 lo, const bf16x4 hi) { return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7); }
+// a token's 8 channels and those of the token before it, as they lie in memory
+struct Shifted {
+    bf16x8 cur, prev;
 };
-// wavefront w loads output blocks 2w, 2w+1 of W[16 db .., c0 ..] (row stride C) as fragment pairs
-template <int NB>
-__device__ __forceinline__ void load_mid_weights(bf16x8 (&r)[NB / 4][2], const __bf16* __restrict__ W, int C, int c0,
-                                                 int wave, const Lane& L) {
+template <int TPB>
+struct TokenRows {   // this thread's tokens of a block's tiles: token t8 + 32 i, channels 8 piece of every channel block
+    static constexpr int N = TPB / 2;
+    const __bf16* row[N];
+    bool has_prev[N];
+    long m[N];
+    __device__ __forceinline__ TokenRows(const __bf16* __restrict__ x, long M, int T, int C, int t8, int piece) {
 #pragma unroll
-    for (int i = 0; i < NB / 4; i++) {
-        const TileB t = load_rows16(W + (long)(16 * (wave * (NB / 4) + i)) * C + c0, C, L);
-        r[i][0] = __builtin_shufflevector(t.f[0], t.f[1], 0, 1, 2, 3, 4, 5, 6, 7);
-        r[i][1] = __builtin_shufflevector(t.f[2], t.f[3], 0, 1, 2, 3, 4, 5, 6, 7);
+        for (int i = 0; i < N; i++) {
+            const long want = (long)blockIdx.x * (TPB * TOK) + t8 + 32 * i;
+            m[i] = want < M ? want : M - 1;   // (rows of a spare tile: the last one again, never stored)
+            has_prev[i] = m[i] % T != 0;
+            row[i] = x + m[i] * C + 8 * piece;
+        }
     }
-}
-
-// The same fragments of R^T ([4D, C], row kD+d) taken from R ([4, C, D]) itself: F(R_k[c.., 16j..]) is loaded with the
-// channels on the lanes (8 contiguous bytes each, raw registers) and transposed on the matrix cores when it is used.
-template <int NB, int D>
-__device__ __forceinline__ void load_r_fragments(bf16x4 (&raw)[NB / 4][NBLK], const __bf16* __restrict__ R, int C, int c0,
-                                                 int wave, const Lane& L) {
-#pragma unroll
-    for (int i = 0; i < NB / 4; i++) {
-        const int ob = wave * (NB / 4) + i, k = ob / (D / 16), j = ob % (D / 16);
-#pragma unroll
-        for (int cb = 0; cb < NBLK; cb++)
-            raw[i][cb] = *reinterpret_cast<const bf16x4*>(R + ((long)k * C + c0 + chan16(cb, L.n)) * D + 16 * j + 4 * L.g);
+    __device__ __forceinline__ Shifted load(int i, int C, int c0) const {
+        return {*reinterpret_cast<const bf16x8*>(row[i] + c0), *reinterpret_cast<const bf16x8*>(row[i] + c0 - (has_prev[i] ? C : 0))};
     }
-}
+};
 
 // a = x + xx*alpha as a bf16 pair (hi + lo): the pre-activation feeds tanh', which is steep, so the interpolated input must
 // not be rounded to 8 bits before the 768-term sum (L itself is bf16)
@@ -132,27 +148,35 @@ __device__ __forceinline__ void store_activation(f32x4 s, __bf16* __restrict__ b
 }
 
 // forward 1 for few tokens: a block takes TPB tiles and one of SPLIT parts of the outputs, its four wavefronts a quarter of
-// the channel blocks each, every operand straight from memory; one sum over the wavefronts at the end.  What bounds a
-// launch of this size is what ONE compute unit can fetch (some 25 bytes per ns: 8 us for the whole of the weights), so the
-// weights are spread over the blocks.  The kernel below fetches all of them per block, a barrier per channel block.
+// the channel blocks each, every one through its own part of LDS; one sum over the wavefronts at the end.  What bounds a
+// launch of this size is what ONE compute unit can fetch, so the weights are spread over the blocks.  The kernel below
+// fetches all of them per block, a barrier per channel block.  Whole lines as above,
+// 768 channels and 1024, 4096 tokens, 2048 channels and 4096 tokens: 9.3, 13.7, 28.5 -> 7.5, 10.9, 18.7 us.
 template <int D, int SPLIT, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, int C, const __bf16* __restrict__ x,
                                                                  const __bf16* __restrict__ alpha,
                                                                  const __bf16* __restrict__ Lw, __bf16* __restrict__ bmid,
                                                                  __bf16* __restrict__ bder) {
     constexpr int NB = 4 * D / 16 / SPLIT, NA = NB * TPB;   // output blocks of 16; with the tiles: accumulators
-    __shared__ f32x4 part[4][NA][WAVE];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NW = 2 * NB, NR = 2 * TPB;                // rows of the weights and tokens per lane
+    struct Image {   // of one wavefront and channel block
+        bf16x8 w[16 * NB * 8], a[2][16 * TPB * 8];
+    };
+    __shared__ union {
+        Image img[4];
+        f32x4 part[4][NA][WAVE];
+    } lds;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l8 = lane >> 3, piece = lane & 7;
     const Lane L;
     const long ntiles = M / TOK;
     const int ncb = C / 64, db0 = NB * blockIdx.y;
-    long m0[TPB];
-    PrevRow before[TPB];
+    const __bf16* row[NR];
+    bool has_prev[NR];
 #pragma unroll
-    for (int p = 0; p < TPB; p++) {
-        const long tile = (long)blockIdx.x * TPB + p;
-        m0[p] = (tile < ntiles ? tile : ntiles - 1) * TOK;   // (a spare tile is the last one again and stores nothing)
-        before[p] = prev_row(x, m0[p] + L.n, T, C, 8 * L.g);
+    for (int i = 0; i < NR; i++) {
+        const long want = (long)blockIdx.x * (TPB * TOK) + l8 + 8 * i, m = want < M ? want : M - 1;   // (a spare tile stores nothing)
+        has_prev[i] = m % T != 0;
+        row[i] = x + m * C + 8 * piece;
     }
     f32x4 acc[TPB][NB];
 #pragma unroll
@@ -160,44 +184,49 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, 
 #pragma unroll
         for (int i = 0; i < NB; i++) acc[p][i] = zero4();
     struct Set {
-        bf16x8 wr[NB][2], xc[TPB][NBLK / 2], xp[TPB][NBLK / 2];
-        bf16x4 al[NBLK];
+        bf16x8 w[NW];
+        Shifted x[NR];
+        bf16x4 al[2];
     };
     auto fetch = [&](Set& st, int cb) {
         const int c0 = 64 * (cb < ncb ? cb : ncb - 1);   // (past the last block: it again, not used)
 #pragma unroll
-        for (int p = 0; p < TPB; p++) {
-            const __bf16 *row = x + (m0[p] + L.n) * C + c0 + 8 * L.g, *prow = before[p].row + c0;
+        for (int i = 0; i < NW; i++) st.w[i] = piece_at(Lw + ((long)(16 * db0 + 8 * i) * C + c0), 2 * ((unsigned)l8 * C + 8 * piece));
 #pragma unroll
-            for (int pr = 0; pr < NBLK / 2; pr++) {
-                st.xc[p][pr] = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
-                st.xp[p][pr] = *reinterpret_cast<const bf16x8*>(prow + 32 * pr);
-            }
-        }
+        for (int i = 0; i < NR; i++)
+            st.x[i] = {*reinterpret_cast<const bf16x8*>(row[i] + c0), *reinterpret_cast<const bf16x8*>(row[i] + c0 - (has_prev[i] ? C : 0))};
 #pragma unroll
-        for (int i = 0; i < NBLK; i++) st.al[i] = *reinterpret_cast<const bf16x4*>(alpha + c0 + chan16(i, 4 * L.g));
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const TileB t = load_rows16(Lw + (long)(16 * (db0 + i)) * C + c0, C, L);
-            st.wr[i][0] = __builtin_shufflevector(t.f[0], t.f[1], 0, 1, 2, 3, 4, 5, 6, 7);
-            st.wr[i][1] = __builtin_shufflevector(t.f[2], t.f[3], 0, 1, 2, 3, 4, 5, 6, 7);
-        }
+        for (int h = 0; h < 2; h++) st.al[h] = *reinterpret_cast<const bf16x4*>(alpha + c0 + 8 * piece + 4 * h);
     };
+    Image& img = lds.img[wave];
     auto use = [&](const Set& st) {
-        bf16x8 a[TPB][4];   // hi, hi, lo, lo
+#pragma unroll
+        for (int i = 0; i < NW; i++) img.w[piece_slot(l8 + 8 * i, piece)] = st.w[i];
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const bf16x8 zero = {};
+            bf16x8 hi, lo;
+            interpolate(st.x[i].cur, has_prev[i] ? st.x[i].prev : zero, st.al[0], st.al[1], hi, lo);
+            img.a[0][piece_slot(l8 + 8 * i, piece)] = hi;
+            img.a[1][piece_slot(l8 + 8 * i, piece)] = lo;
+        }
+        wave_lds_order();
+        bf16x8 l[NB][2];
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int pr = 0; pr < 2; pr++) l[i][pr] = img.w[piece_slot(16 * i + L.n, 4 * pr + L.g)];
 #pragma unroll
         for (int p = 0; p < TPB; p++)
 #pragma unroll
-            for (int pr = 0; pr < NBLK / 2; pr++) {
-                const bf16x8 zero = {};
-                interpolate(st.xc[p][pr], before[p].has_prev ? st.xp[p][pr] : zero, st.al[2 * pr], st.al[2 * pr + 1], a[p][pr], a[p][2 + pr]);
-            }
+            for (int hl = 0; hl < 2; hl++)
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+                for (int pr = 0; pr < 2; pr++) {
+                    const bf16x8 a = img.a[hl][piece_slot(16 * p + L.n, 4 * pr + L.g)];
 #pragma unroll
-            for (int p = 0; p < TPB; p++)
-#pragma unroll
-                for (int i = 0; i < NB; i++) acc[p][i] = mma8(acc[p][i], st.wr[i][k & 1], a[p][k]);
+                    for (int i = 0; i < NB; i++) acc[p][i] = mma8(acc[p][i], l[i][pr], a);
+                }
+        wave_lds_order();
     };
     constexpr int SETS = 3;   // channel blocks in flight
     Set st[SETS];
@@ -215,16 +244,17 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, 
         }
     }
     // the sums over the wavefronts, each by one wavefront and in their order
+    __syncthreads();
 #pragma unroll
     for (int p = 0; p < TPB; p++)
 #pragma unroll
-        for (int i = 0; i < NB; i++) part[wave][p * NB + i][lane] = acc[p][i];
+        for (int i = 0; i < NB; i++) lds.part[wave][p * NB + i][lane] = acc[p][i];
     __syncthreads();
     for (int e = wave; e < NA; e += 4) {
         const int p = e / NB, i = e % NB;
         const long tile = (long)blockIdx.x * TPB + p;
         if (tile >= ntiles) break;
-        const f32x4 s = (part[0][e][lane] + part[1][e][lane]) + (part[2][e][lane] + part[3][e][lane]);
+        const f32x4 s = (lds.part[0][e][lane] + lds.part[1][e][lane]) + (lds.part[2][e][lane] + lds.part[3][e][lane]);
         store_activation(s, bmid, bder, (tile * TOK + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g);
     }
 }
@@ -238,14 +268,13 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
     constexpr int NB = 4 * D / 16;       // output blocks of 16
     constexpr int WPT = 4 / TPB;         // wavefronts per tile
     constexpr int NBW = NB / WPT;        // output blocks per wavefront
-    __shared__ MidWeights<NB> w;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NW = 4 * D / 32, NR = TokenRows<TPB>::N;   // rows of the weights and tokens per thread
+    __shared__ bf16x8 s_w[2][4 * D * 8], s_a[2][2][TPB * TOK * 8];   // a: hi, lo
+    const int wave = threadIdx.x >> 6, t8 = threadIdx.x >> 3, piece = threadIdx.x & 7;
     const Lane L;
-    const long ntiles = M / TOK;
-    const long tile_raw = (long)blockIdx.x * TPB + wave / WPT;
-    const bool live = tile_raw < ntiles;
-    const long m0 = (live ? tile_raw : ntiles - 1) * TOK;   // a spare wavefront repeats the last tile and stores nothing
-    const int db0 = (wave % WPT) * NBW;
+    const long tile = (long)blockIdx.x * TPB + wave / WPT;
+    const int db0 = (wave % WPT) * NBW, row0 = TOK * (wave / WPT);
+    const TokenRows<TPB> tokens(x, M, T, C, t8, piece);
 
     f32x4 acc[NBW];
 #pragma unroll
@@ -254,30 +283,22 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
     // moment queue on the few L2 channels that hold it.
     const int ncb = C / 64;
     auto advance = [&](int c) { return c + 1 < ncb ? c + 1 : 0; };
-    // Two sets of streamed operands (weights, x rows, alpha), each refilled right after the round that used it, so
-    // a load has two rounds to arrive.  The operands stay raw registers until the round that uses them: a
-    // conversion at the point of the load, or a load under a condition, makes the compiler wait for the data
-    // right there (8192 tokens: 24 -> 18 us with raw operands one round ahead, 17 us two rounds ahead; with every
-    // operand cache-resident the same instructions take 13.5 us, so what is left is the rounds themselves).
+    // Two sets of streamed operands, each refilled right after the round that used it, so a load has two rounds to arrive.
+    // The operands stay raw registers until the round that uses them: a conversion at the point of the load, or a load
+    // under a condition, makes the compiler wait for the data right there.
     struct Set {
-        bf16x8 wr[NB / 4][2];
-        bf16x8 xc[NBLK / 2], xp[NBLK / 2];
-        bf16x4 al[NBLK];
+        bf16x8 w[NW];
+        Shifted x[NR];
+        bf16x4 al[2];
     };
-    const PrevRow before = prev_row(x, m0 + L.n, T, C, 8 * L.g);
-    const bool has_prev = before.has_prev;
     auto fetch = [&](Set& st, int cbk) {
         const int c0 = 64 * cbk;
-        load_mid_weights<NB>(st.wr, Lw, C, c0, wave, L);
-        const __bf16* row = x + (m0 + L.n) * C + c0 + 8 * L.g;
-        const __bf16* prow = before.row + c0;
 #pragma unroll
-        for (int pr = 0; pr < NBLK / 2; pr++) {
-            st.xc[pr] = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
-            st.xp[pr] = *reinterpret_cast<const bf16x8*>(prow + 32 * pr);
-        }
+        for (int i = 0; i < NW; i++) st.w[i] = piece_at(Lw + ((long)32 * i * C + c0), 2 * ((unsigned)t8 * C + 8 * piece));
 #pragma unroll
-        for (int i = 0; i < NBLK; i++) st.al[i] = *reinterpret_cast<const bf16x4*>(alpha + c0 + chan16(i, 4 * L.g));
+        for (int i = 0; i < NR; i++) st.x[i] = tokens.load(i, C, c0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) st.al[h] = *reinterpret_cast<const bf16x4*>(alpha + c0 + 8 * piece + 4 * h);
     };
     int next_cb = blockIdx.x % ncb;
     Set sa, sb;
@@ -287,26 +308,32 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
     next_cb = advance(next_cb);
     auto round = [&](Set& st, int buf) {
 #pragma unroll
-        for (int i = 0; i < NB / 4; i++) {
-            w.f[buf][wave * (NB / 4) + i][0][lane] = st.wr[i][0];
-            w.f[buf][wave * (NB / 4) + i][1][lane] = st.wr[i][1];
+        for (int i = 0; i < NW; i++) s_w[buf][piece_slot(t8 + 32 * i, piece)] = st.w[i];
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            const bf16x8 zero = {};
+            bf16x8 hi, lo;
+            interpolate(st.x[i].cur, tokens.has_prev[i] ? st.x[i].prev : zero, st.al[0], st.al[1], hi, lo);
+            s_a[buf][0][piece_slot(t8 + 32 * i, piece)] = hi;
+            s_a[buf][1][piece_slot(t8 + 32 * i, piece)] = lo;
         }
         __syncthreads();
-        bf16x8 a[2], alo[2];
-#pragma unroll
-        for (int pr = 0; pr < NBLK / 2; pr++) {
-            const bf16x8 zero = {};
-            interpolate(st.xc[pr], has_prev ? st.xp[pr] : zero, st.al[2 * pr], st.al[2 * pr + 1], a[pr], alo[pr]);
-        }
         fetch(st, next_cb);   // (the last two rounds fetch blocks that are not used)
         next_cb = advance(next_cb);
+        bf16x8 a[2][2];
+#pragma unroll
+        for (int hl = 0; hl < 2; hl++)
+#pragma unroll
+            for (int pr = 0; pr < 2; pr++) a[hl][pr] = s_a[buf][hl][piece_slot(row0 + L.n, 4 * pr + L.g)];
 #pragma unroll
         for (int i = 0; i < NBW; i++) {
-            const bf16x8 l0 = w.f[buf][db0 + i][0][lane], l1 = w.f[buf][db0 + i][1][lane];   // F(L[16db.., c0..]) lane = output
-            acc[i] = mma8(acc[i], l0, a[0]);                                                     // + F(a L^T) lane = token
-            acc[i] = mma8(acc[i], l1, a[1]);
-            acc[i] = mma8(acc[i], l0, alo[0]);
-            acc[i] = mma8(acc[i], l1, alo[1]);
+            bf16x8 l[2];   // F(L[16db.., c0..]) lane = output
+#pragma unroll
+            for (int pr = 0; pr < 2; pr++) l[pr] = s_w[buf][piece_slot(16 * (db0 + i) + L.n, 4 * pr + L.g)];
+#pragma unroll
+            for (int hl = 0; hl < 2; hl++)
+#pragma unroll
+                for (int pr = 0; pr < 2; pr++) acc[i] = mma8(acc[i], l[pr], a[hl][pr]);   // + F(a L^T) lane = token
         }
     };
     int it = 0;
@@ -315,16 +342,26 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_kernel(long M, int T, int 
         round(sb, 1);
     }
     if (it < ncb) round(sa, 0);
-    if (!live) return;
+    if (tile * TOK >= M) return;
 #pragma unroll
-    for (int i = 0; i < NBW; i++) store_activation(acc[i], bmid, bder, (m0 + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g);
+    for (int i = 0; i < NBW; i++) store_activation(acc[i], bmid, bder, (tile * TOK + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g);
 }
 
 // ------------------------------------------------------------------------------------------------
 // backward 1: dpre = ((dy_k * xx) R_k) * (1 - bmid^2)        [M, 4D]   (the factor 1 - bmid^2 was saved by forward)
-// Same structure as forward 1; the weights are R^T ([4D, C], output block k*D/16 + j), transposed from R on the way
-// into LDS.
+// Same structure as forward 1; the weights are R [4, C, D], 64 rows of D elements per channel block and interpolation,
+// kept in LDS as they lie in memory and read back transposed (ds_read_b64_tr_b16, the lanes' addresses as in the WKV7
+// backward kernels: lane p of a group of 16 points at the 8 bytes of row p/4, columns 4(p%4).. of its four rows).
 // ------------------------------------------------------------------------------------------------
+// A transposing read takes 32 bytes of each of rows 8g' .. 8g'+3 for two groups at a time: four rows of 64 bytes (D = 32) are
+// the banks once over, two of 128 (D = 64) as well, so pieces move by pairs for odd g' and, at D = 64, rows 2 and 3.
+template <int D>
+__device__ __forceinline__ int r_slot(int channel, int piece) {
+    return (D / 8) * channel + (D == 32 ? piece ^ (channel >> 2 & 2) : piece ^ (channel & 2) ^ (channel >> 1 & 4));
+}
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef s16x4 __attribute__((address_space(3))) lds_s16x4;
+typedef unsigned char __attribute__((address_space(3))) lds_u8;
 template <int D, int TPB>
 __global__ __launch_bounds__(256) void ddlerp_bwd_mid_kernel(long M, int T, int C, const __bf16* __restrict__ x,
                                                              Dy4 dy,
@@ -334,90 +371,84 @@ __global__ __launch_bounds__(256) void ddlerp_bwd_mid_kernel(long M, int T, int 
     constexpr int ND = D / 16, NB = 4 * ND;
     constexpr int WPT = 4 / TPB, NBW = NB / WPT;
     static_assert(NBW % ND == 0, "a wavefront owns whole interpolations k");
-    __shared__ MidWeights<NB> w;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NW = 4 * D / 32, NR = TokenRows<TPB>::N;
+    __shared__ bf16x8 s_r[2][4][64 * D / 8], s_dc[2][4][TPB * TOK * 8];
+    const int wave = threadIdx.x >> 6, t8 = threadIdx.x >> 3, piece = threadIdx.x & 7;
     const Lane L;
-    const long ntiles = M / TOK;
-    const long tile_raw = (long)blockIdx.x * TPB + wave / WPT;
-    const bool live = tile_raw < ntiles;
-    const long m0 = (live ? tile_raw : ntiles - 1) * TOK;
-    const int db0 = (wave % WPT) * NBW, k0 = db0 / ND;
+    const long tile = (long)blockIdx.x * TPB + wave / WPT;
+    const int db0 = (wave % WPT) * NBW, k0 = db0 / ND, row0 = TOK * (wave / WPT);
+    const TokenRows<TPB> tokens(x, M, T, C, t8, piece);
 
     f32x4 acc[NBW];
 #pragma unroll
     for (int i = 0; i < NBW; i++) acc[i] = zero4();
-    struct Loads {
-        bf16x8 xc[NBLK / 2], xp[NBLK / 2], dy[NBW / ND][NBLK / 2];
+    struct Set {
+        bf16x8 r[NW], dy[4][NR];
+        Shifted x[NR];
     };
-    auto issue = [&](int c0) {
-        Loads ld;
-        const long m = m0 + L.n;
-        const __bf16* row = x + m * C + c0 + 8 * L.g;
-        const __bf16* prow = (m % T) != 0 ? row - C : row;
+    auto fetch = [&](Set& st, int c0) {
 #pragma unroll
-        for (int pr = 0; pr < NBLK / 2; pr++) {
-            ld.xc[pr] = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
-            ld.xp[pr] = *reinterpret_cast<const bf16x8*>(prow + 32 * pr);
+        for (int i = 0; i < NW; i++)   // R_k from channel c0 on: NW / 4 contiguous runs of 4 KiB
+            st.r[i] = piece_at(R + ((long)(i / (NW / 4)) * C + c0) * D + 2048 * (i % (NW / 4)), 16 * threadIdx.x);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            st.x[i] = tokens.load(i, C, c0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) st.dy[k][i] = *reinterpret_cast<const bf16x8*>(dy.p[k] + tokens.m[i] * C + c0 + 8 * piece);
+        }
+    };
+    auto round = [&](Set& st, int buf, int next) {
+#pragma unroll
+        for (int i = 0; i < NW; i++) {
+            const int p = threadIdx.x + 256 * (i % (NW / 4));
+            s_r[buf][i / (NW / 4)][r_slot<D>(p / (D / 8), p % (D / 8))] = st.r[i];
         }
 #pragma unroll
-        for (int k = 0; k < NBW / ND; k++)
+        for (int i = 0; i < NR; i++) {
+            const bf16x8 zero = {}, prev = tokens.has_prev[i] ? st.x[i].prev : zero;
+            f32x4 xx[2];
 #pragma unroll
-            for (int pr = 0; pr < NBLK / 2; pr++)
-                ld.dy[k][pr] = *reinterpret_cast<const bf16x8*>(dy.p[k0 + k] + m * C + c0 + 8 * L.g + 32 * pr);
-        return ld;
-    };
-    const bool has_prev = ((m0 + L.n) % T) != 0;
-    const bf16x4 eye = identity_bf16(L);
-    bf16x4 wr[NB / 4][NBLK];
-    load_r_fragments<NB, D>(wr, R, C, 0, wave, L);
-    Loads cur = issue(0);
-    for (int c0 = 0, it = 0; c0 < C; c0 += 64, it++) {
-        const int buf = it & 1;
+            for (int h = 0; h < 2; h++) xx[h] = to_f32(half_of(prev, h)) - to_f32(half_of(st.x[i].cur, h));
 #pragma unroll
-        for (int i = 0; i < NB / 4; i++) {
-            bf16x4 t[NBLK];
-#pragma unroll
-            for (int cb = 0; cb < NBLK; cb++) t[cb] = transpose(wr[i][cb], eye);
-            w.f[buf][wave * (NB / 4) + i][0][lane] = __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3, 4, 5, 6, 7);
-            w.f[buf][wave * (NB / 4) + i][1][lane] = __builtin_shufflevector(t[2], t[3], 0, 1, 2, 3, 4, 5, 6, 7);
+            for (int k = 0; k < 4; k++)
+                s_dc[buf][k][piece_slot(t8 + 32 * i, piece)] =
+                    join(to_bf16(to_f32(half_of(st.dy[k][i], 0)) * xx[0]), to_bf16(to_f32(half_of(st.dy[k][i], 1)) * xx[1]));
         }
-        const int cn = c0 + 64 < C ? c0 + 64 : c0;
-        load_r_fragments<NB, D>(wr, R, C, cn, wave, L);
-        const Loads nxt = issue(cn);
         __syncthreads();
-        f32x4 xx[NBLK];
-#pragma unroll
-        for (int pr = 0; pr < NBLK / 2; pr++) {
-            const bf16x8 zero = {};
-            const bf16x8 prev = has_prev ? cur.xp[pr] : zero;
-            xx[2 * pr] = to_f32(__builtin_shufflevector(prev, prev, 0, 1, 2, 3)) -
-                         to_f32(__builtin_shufflevector(cur.xc[pr], cur.xc[pr], 0, 1, 2, 3));
-            xx[2 * pr + 1] = to_f32(__builtin_shufflevector(prev, prev, 4, 5, 6, 7)) -
-                             to_f32(__builtin_shufflevector(cur.xc[pr], cur.xc[pr], 4, 5, 6, 7));
-        }
+        fetch(st, next);   // (the last rounds fetch blocks that are not used)
 #pragma unroll
         for (int k = 0; k < NBW / ND; k++) {
-            bf16x8 dc[2];
 #pragma unroll
             for (int pr = 0; pr < 2; pr++) {
-                const bf16x8 d = cur.dy[k][pr];
-                dc[pr] = __builtin_shufflevector(to_bf16(to_f32(__builtin_shufflevector(d, d, 0, 1, 2, 3)) * xx[2 * pr]),
-                                                 to_bf16(to_f32(__builtin_shufflevector(d, d, 4, 5, 6, 7)) * xx[2 * pr + 1]),
-                                                 0, 1, 2, 3, 4, 5, 6, 7);
-            }
+                const bf16x8 dc = s_dc[buf][k0 + k][piece_slot(row0 + L.n, 4 * pr + L.g)];
 #pragma unroll
-            for (int j = 0; j < ND; j++) {
-                const int i = k * ND + j;
-                acc[i] = mma8(acc[i], w.f[buf][db0 + i][0][lane], dc[0]);   // + F(dc R_k) lane = token
-                acc[i] = mma8(acc[i], w.f[buf][db0 + i][1][lane], dc[1]);
+                for (int j = 0; j < ND; j++) {
+                    bf16x4 rt[2];   // F(R_k^T) lane = mid index 16j + n, channels 32pr + 8g + 4h ..
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const int ch = 32 * pr + 8 * L.g + 4 * h + (L.n >> 2), col = 16 * j + 4 * (L.n & 3);
+                        rt[h] = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (lds_s16x4*)((lds_u8*)&s_r[buf][k0 + k][r_slot<D>(ch, col / 8)] + 2 * (col & 7))));
+                    }
+                    acc[k * ND + j] = mma8(acc[k * ND + j], join(rt[0], rt[1]), dc);   // + F(dc R_k) lane = token
+                }
             }
         }
-        cur = nxt;
+    };
+    auto block = [&](int cb) { return cb < C ? cb : C - 64; };
+    Set sa, sb;
+    fetch(sa, 0);
+    fetch(sb, block(64));
+    int c0 = 0;
+    for (; c0 + 128 <= C; c0 += 128) {
+        round(sa, 0, block(c0 + 128));
+        round(sb, 1, block(c0 + 192));
     }
-    if (!live) return;
+    if (c0 < C) round(sa, 0, C - 64);
+    if (tile * TOK >= M) return;
 #pragma unroll
     for (int i = 0; i < NBW; i++) {
-        const long off = (m0 + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g;
+        const long off = (tile * TOK + L.n) * (4 * D) + 16 * (db0 + i) + 4 * L.g;
         *reinterpret_cast<bf16x4*>(dpre + off) = to_bf16(acc[i] * to_f32(*reinterpret_cast<const bf16x4*>(bder + off)));
     }
 }
@@ -857,14 +888,15 @@ size_t ddlerp_bwd_workspace_bytes(long M, int C, int D) {
 }
 
 namespace {
-// up to two blocks per compute unit of the kernel for few tokens; us, that one / the other: 768 channels, 16 tokens 8.7 / 14.1,
-// 2016 9.5 / 15.7, 4096 14.1 / 16.2, 8192 22 / 17; 2048 channels, 2016 16 / 33, 4096 28 / 33, 8192 51 / 34
+// up to two blocks per compute unit of the kernel for few tokens; us, that one / the other: 768 channels, 256 tokens 7.3 / 10.3,
+// 1024 7.5 / 10.4, 4096 10.9 / 10.7; 2048 channels, 4096 18.7 / 21.5
 bool few_tokens(long ntiles) { return (ntiles + 1) / 2 * 4 <= 2 * compute_units(); }
 template <int D>
 void forward_rank(long M, int T, int C, const void* x, const void* alpha, const void* Lw, const void* R, const void* beta,
                   void* bmid, void* bder, void* y, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
-    // four tiles per block when that still gives every compute unit a block, else two
+    // four tiles per block when that still gives every compute unit a block, else two; us at 768 channels, four / two: 16384
+    // tokens 17.5 / 17.0, 32768 28.5 / 31.8.  (Backward 1 takes two at any size: 35.4 / 34.5 and 81 / 77, 65536 x 64 21.5 / 18.7.)
     const long ntiles = M / TOK;
     if (few_tokens(ntiles))
         hipLaunchKernelGGL((ddlerp_fwd_mid_few_kernel<D, 4, 2>), dim3((unsigned)((ntiles + 1) / 2), 4), dim3(256), 0, stream, M, T, C, c(x),
@@ -893,12 +925,8 @@ void backward_rank(long M, int T, int C, const void* x, const void* alpha, const
     const int tiles_per_split = (int)((M / TOK + param_splits(M, ncb) - 1) / param_splits(M, ncb));
     const int nsplit = (int)((M / TOK + tiles_per_split - 1) / tiles_per_split);   // no empty range: every block writes a record
 
-    if (M / TOK >= 4 * 256)
-        hipLaunchKernelGGL((ddlerp_bwd_mid_kernel<D, 4>), dim3((unsigned)((M / TOK + 3) / 4)), dim3(256), 0, stream, M, T, C,
-                           c(x), dy, c(R), c(bder), dpre);
-    else
-        hipLaunchKernelGGL((ddlerp_bwd_mid_kernel<D, 2>), dim3((unsigned)((M / TOK + 1) / 2)), dim3(256), 0, stream, M, T, C,
-                           c(x), dy, c(R), c(bder), dpre);
+    hipLaunchKernelGGL((ddlerp_bwd_mid_kernel<D, 2>), dim3((unsigned)((M / TOK + 1) / 2)), dim3(256), 0, stream, M, T, C, c(x), dy,
+                       c(R), c(bder), dpre);
     hipLaunchKernelGGL(ddlerp_bwd_main_kernel<D>, dim3(ncb, nsplit), dim3(256), 0, stream, M, T, C, tiles_per_split, c(x), dy,
                        c(alpha), c(Lw), c(R), c(beta), c(bmid), dpre, static_cast<__bf16*>(dx), partial);
     hipLaunchKernelGGL(ddlerp_param_reduce_kernel<D>, dim3((ParamPartial<D>::TOTAL / 4 + 255) / 256, ncb), dim3(256), 0,
