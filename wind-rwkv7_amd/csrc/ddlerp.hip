@@ -25,43 +25,6 @@ struct Dy4 {  // the four upstream gradients, each [M, C]
     const __bf16* p[4];
 };
 
-// x tile and its token-shifted difference for 16 tokens x 64 channels starting at channel c0.
-struct XTile {
-    TileF x, xx;
-};
-// the row before token m at the lane's channels: the token before it, at a sequence's start (has_prev false: to be read as
-// zeros) the row itself
-struct PrevRow {
-    const __bf16* row;
-    bool has_prev;
-};
-__device__ __forceinline__ PrevRow prev_row(const __bf16* __restrict__ x, long m, int T, int C, int c) {
-    const bool inside = (m % T) != 0;
-    const __bf16* row = x + m * C + c;
-    return {inside ? row - C : row, inside};
-}
-__device__ __forceinline__ XTile load_x_tile(const __bf16* __restrict__ x, long m0, int T, int C, int c0, const Lane& L) {
-    XTile r;
-    const long m = m0 + L.n;
-    const PrevRow before = prev_row(x, m, T, C, c0 + 8 * L.g);
-    // 16-byte accesses: blocks 2p and 2p+1 of the tile are the interleaved channels of chan16 (frag.hpp); every
-    // per-channel operand of these kernels is indexed through the same map
-    const __bf16* row = x + m * C + c0 + 8 * L.g;
-#pragma unroll
-    for (int pr = 0; pr < NBLK / 2; pr++) {
-        const bf16x8 cur = *reinterpret_cast<const bf16x8*>(row + 32 * pr);
-        bf16x8 prev = {};
-        if (before.has_prev) prev = *reinterpret_cast<const bf16x8*>(before.row + 32 * pr);
-#pragma unroll
-        for (int hlf = 0; hlf < 2; hlf++) {
-            const f32x4 c = to_f32(hlf ? __builtin_shufflevector(cur, cur, 4, 5, 6, 7) : __builtin_shufflevector(cur, cur, 0, 1, 2, 3));
-            const f32x4 q = to_f32(hlf ? __builtin_shufflevector(prev, prev, 4, 5, 6, 7) : __builtin_shufflevector(prev, prev, 0, 1, 2, 3));
-            r.x.f[2 * pr + hlf] = c;
-            r.xx.f[2 * pr + hlf] = q - c;
-        }
-    }
-    return r;
-}
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
@@ -455,42 +418,32 @@ __global__ __launch_bounds__(256) void ddlerp_bwd_mid_kernel(long M, int T, int 
 
 // ------------------------------------------------------------------------------------------------
 // Forward 2 gives a block one 64-channel block and a range of token tiles: the block's 16 KiB of weight
-// fragments (R) are staged in LDS once, in the order the matrix instructions take them (16 bytes per lane per
-// pair), and every wavefront walks its tiles.  Fetching the fragments per tile from memory in the middle of
-// dependent arithmetic, as a tile-per-wavefront kernel must, left the kernel waiting for loads most of the time.
+// fragments (R) are staged in LDS once, in the order the matrix instructions take them (16 bytes per lane), and
+// every wavefront walks its tiles, the next one's operands on their way.  A tile's rows of x, of bmid and of the four
+// streams move as whole lines (see above) through the wavefront's own part of LDS; as pieces of 16 rows, 20
+// instructions of 28 ns of a compute unit's time per tile and channel block, 4096, 8192, 16384, 32768 tokens x 768 channels
+// took 12.1, 20.3, 33.4, 72 us; now 9.0, 13.6, 25.7, 59, of which the bytes are 6, 13, 25, 50 at the rate of a copy.
 // ------------------------------------------------------------------------------------------------
+// A lane group g holds mid indices 8g .. 8g+7 of each 32: the order of a contraction is free if both operands agree.
 template <int D>
 struct LerpWeights {   // LDS image for one 64-channel block
-    static constexpr int ND = D / 16;
-    bf16x8 R[4][NBLK][ND / 2][WAVE];   // (F(R_k[c.., 16j..]), F(R_k[c.., 16j+16..]))  lane = channel, reg = d
+    bf16x8 R[4][NBLK][D / 32][WAVE];   // F(R_k[c.., 32j + 8g ..])  lane = channel
     float beta[4][64];
 };
 template <int D>
 __device__ __forceinline__ void stage_lerp_weights(LerpWeights<D>& w, const __bf16* __restrict__ R,
                                                    const __bf16* __restrict__ beta, int C, int c0) {
-    constexpr int ND = D / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const Lane L;
-    // wavefront k stages R_k
+    const int thread = threadIdx.x;
 #pragma unroll
-    for (int cb = 0; cb < NBLK; cb++) {
-        const long ch = c0 + chan16(cb, L.n);
+    for (int k = 0; k < 4; k++)
 #pragma unroll
-        for (int j = 0; j < ND / 2; j++) {
-            const __bf16* rrow = R + ((long)wave * C + ch) * D + 32 * j + 4 * L.g;
-            w.R[wave][cb][j][lane] = __builtin_shufflevector(*reinterpret_cast<const bf16x4*>(rrow),
-                                                             *reinterpret_cast<const bf16x4*>(rrow + 16), 0, 1, 2, 3, 4, 5, 6, 7);
+        for (int i = 0; i < D / 32; i++) {   // R_k from channel c0 on, as it lies in memory: 256 pieces a time
+            const int p = thread + 256 * i, ch = p / (D / 8), j = p % (D / 8) / 4, g = p % 4;
+            // channel block and lane of a channel: chan16 the other way round
+            const int cb = 2 * (ch >> 5) + (ch >> 2 & 1), n = 4 * (ch >> 3 & 3) + (ch & 3);
+            w.R[k][cb][j][n + 16 * g] = piece_at(R + ((long)k * C + c0) * D, 16 * p);
         }
-    }
-    w.beta[wave][lane] = (float)beta[(long)wave * C + c0 + lane];
-}
-// this lane's mid-index fragments of one token row (bmid or dpre), as pairs
-template <int NPAIR>
-__device__ __forceinline__ void load_mid_pairs(bf16x8 (&out)[NPAIR], const __bf16* __restrict__ row, const Lane& L) {
-#pragma unroll
-    for (int j = 0; j < NPAIR; j++)
-        out[j] = __builtin_shufflevector(*reinterpret_cast<const bf16x4*>(row + 32 * j + 4 * L.g),
-                                         *reinterpret_cast<const bf16x4*>(row + 32 * j + 16 + 4 * L.g), 0, 1, 2, 3, 4, 5, 6, 7);
+    w.beta[thread >> 6][thread & 63] = (float)beta[(long)(thread >> 6) * C + c0 + (thread & 63)];
 }
 
 // forward 2: y_k = x + xx * (bmid_k R_k^T + beta_k).  Block = (64 channels, range of token tiles).
@@ -499,33 +452,81 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int
                                                               const __bf16* __restrict__ x,
                                                               const __bf16* __restrict__ R, const __bf16* __restrict__ beta,
                                                               const __bf16* __restrict__ bmid, __bf16* __restrict__ y) {
-    constexpr int ND = D / 16;
+    constexpr int MP = 4 * D / 8;   // pieces of a row of bmid
+    struct Image {                  // of one wavefront's tile
+        bf16x8 x[(TOK + 1) * 8], mid[TOK * MP], out[TOK * 8];   // x: from the row before the tile on
+    };
     __shared__ LerpWeights<D> w;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ Image img_all[4];
+    const int lane = threadIdx.x & 63, l8 = lane >> 3, piece = lane & 7;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    Image& img = img_all[wave];
     const Lane L;
     const int c0 = blockIdx.x * 64;
     const long ntiles = M / TOK;
     const long tile_begin = (long)blockIdx.y * tiles_per_split;
     const long tile_end = tile_begin + tiles_per_split < ntiles ? tile_begin + tiles_per_split : ntiles;
+    const unsigned row_bytes = 2 * C, lane_bytes = l8 * row_bytes + 16 * piece;   // (16 rows: 32 C bytes, below 2^32)
+    struct Rows {
+        bf16x8 x[2], before, mid[MP / 4];
+    };
+    auto fetch = [&](long tile) {
+        Rows r;
+        const long m0 = tile * TOK;
+        const __bf16* xt = x + m0 * C + c0;
+#pragma unroll
+        for (int i = 0; i < 2; i++) r.x[i] = piece_at(xt, lane_bytes + 8 * i * row_bytes);
+        r.before = piece_at(m0 % T != 0 ? xt - C : xt, 16 * piece);
+#pragma unroll
+        for (int i = 0; i < MP / 4; i++) r.mid[i] = piece_at(bmid + m0 * (4 * D) + 512 * i, 16 * lane);
+        return r;
+    };
+    // a column of sixteen rows in sixteen different banks of 16 bytes
+    auto mid_slot = [](int row, int p) { return MP * row + (p ^ row); };
+    long tile = tile_begin + wave;
+    Rows next;
+    if (tile < tile_end) next = fetch(tile);
     stage_lerp_weights<D>(w, R, beta, C, c0);
     __syncthreads();
-    for (long tile = tile_begin + wave; tile < tile_end; tile += 4) {
+    for (; tile < tile_end; tile += 4) {
         const long m0 = tile * TOK;
-        const XTile xt = load_x_tile(x, m0, T, C, c0, L);
-        bf16x8 bm[4 * ND / 2];
-        load_mid_pairs(bm, bmid + (m0 + L.n) * (4 * D), L);
+        const bf16x8 zero = {};
+#pragma unroll
+        for (int i = 0; i < 2; i++) img.x[piece_slot(1 + l8 + 8 * i, piece)] = next.x[i];
+        if (l8 == 0) img.x[piece_slot(0, piece)] = m0 % T != 0 ? next.before : zero;
+#pragma unroll
+        for (int i = 0; i < MP / 4; i++) img.mid[mid_slot((lane + 64 * i) / MP, (lane + 64 * i) % MP)] = next.mid[i];
+        wave_lds_order();
+        next = fetch(tile + 4 < tile_end ? tile + 4 : tile);   // (past the end: this one again, not used)
+        f32x4 xv[NBLK], xx[NBLK];
+#pragma unroll
+        for (int cb = 0; cb < NBLK; cb++) {
+            xv[cb] = to_f32(half_of(img.x[piece_slot(L.n + 1, 4 * (cb >> 1) + L.g)], cb & 1));
+            xx[cb] = to_f32(half_of(img.x[piece_slot(L.n, 4 * (cb >> 1) + L.g)], cb & 1)) - xv[cb];
+        }
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            TileB out;
+            bf16x8 bm[D / 32];
+#pragma unroll
+            for (int j = 0; j < D / 32; j++) bm[j] = img.mid[mid_slot(L.n, (D / 8) * k + 4 * j + L.g)];
+            bf16x4 o[NBLK];
 #pragma unroll
             for (int cb = 0; cb < NBLK; cb++) {
                 f32x4 c = *reinterpret_cast<const f32x4*>(&w.beta[k][chan16(cb, 4 * L.g)]);
 #pragma unroll
-                for (int j = 0; j < ND / 2; j++) c = mma8(c, w.R[k][cb][j][lane], bm[k * (ND / 2) + j]);
-                out.f[cb] = to_bf16(xt.x.f[cb] + xt.xx.f[cb] * c);
+                for (int j = 0; j < D / 32; j++) c = mma8(c, w.R[k][cb][j][lane], bm[j]);
+                o[cb] = to_bf16(xv[cb] + xx[cb] * c);
             }
-            store_rows16(y + ((long)k * M + m0) * C + c0, C, L, out);
+            wave_lds_order();
+#pragma unroll
+            for (int pr = 0; pr < 2; pr++) img.out[piece_slot(L.n, 4 * pr + L.g)] = join(o[2 * pr], o[2 * pr + 1]);
+            wave_lds_order();
+            __bf16* dst = y + ((long)k * M + m0) * C + c0;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                *reinterpret_cast<bf16x8*>(reinterpret_cast<char*>(dst) + (lane_bytes + 8 * i * row_bytes)) = img.out[piece_slot(l8 + 8 * i, piece)];
         }
+        wave_lds_order();
     }
 }
 
@@ -863,12 +864,13 @@ int param_splits(long M, int ncb) {
     if (s < 1) s = 1;
     return (int)s;
 }
-// token-tile ranges of forward 2: a few blocks per compute unit of an MI355X (256) over the channel blocks, at
-// least four tiles (one per wavefront) each
+// token-tile ranges of forward 2: as many blocks over the channel blocks as the machine holds at once (at rank 32 LDS and
+// registers allow three per compute unit), at least four tiles (one per wavefront) each.  Two streams' rows in LDS, two blocks
+// per compute unit, in one round / in two: 14.4 / 15.9 us instead of 13.6 at 8192 tokens x 768 channels
 struct StreamSplit {
     int nsplit, tiles_per_split;
 };
-StreamSplit stream_splits(long M, int ncb, int slots) {   // slots: blocks the machine holds at once, times rounds
+StreamSplit stream_splits(long M, int ncb, int slots) {
     const long ntiles = M / TOK;
     long s = slots / ncb > 0 ? slots / ncb : 1;
     if (s > ntiles / 4) s = ntiles / 4;
@@ -907,7 +909,7 @@ void forward_rank(long M, int T, int C, const void* x, const void* alpha, const 
     else
         hipLaunchKernelGGL((ddlerp_fwd_mid_kernel<D, 2>), dim3((unsigned)((ntiles + 1) / 2)), dim3(256), 0, stream, M, T, C,
                            c(x), c(alpha), c(Lw), static_cast<__bf16*>(bmid), static_cast<__bf16*>(bder));
-    const StreamSplit sp = stream_splits(M, C / 64, 4 * compute_units());   // two blocks per compute unit, two rounds
+    const StreamSplit sp = stream_splits(M, C / 64, 3 * compute_units());
     hipLaunchKernelGGL(ddlerp_fwd_out2_kernel<D>, dim3(C / 64, sp.nsplit), dim3(256), 0, stream, M, T, C, sp.tiles_per_split,
                        c(x), c(R), c(beta), c(bmid), static_cast<__bf16*>(y));
 }
