@@ -57,6 +57,13 @@ def test_expand_loras_parity_other_head_sizes(B, T, C, D, N):
     print(f'expand_loras head size {N} worst', max(errs.items(), key=lambda kv: kv[1]))
 
 
+# rank 16, tiles of 16 tokens to pairs of wavefronts: one pair idle, rounds that differ between a block's pairs, blocks without a
+# tile (1025 tiles of one head over 512 blocks), counts of heads that are no multiple of the four shares of the sum over them
+@pytest.mark.parametrize('B,T,C,N', [(1, 48, 320, 64), (5, 16, 64, 64), (25, 656, 64, 64), (2, 80, 1088, 64), (3, 48, 192, 32)])
+def test_expand_loras_rank_16_tiles(B, T, C, N):
+    check(*run_both(B, T, C, 16, seed=700 + T + C, scale=0.5, head_size=N))
+
+
 def test_expand_loras_parity_cfg4_shape():
     """[8,1024,768] with rank 16: the time-mixer block's shape; inputs ~ N(0,1) as in the reference's script."""
     errs = check(*run_both(8, 1024, 768, 16, seed=4))

@@ -37,7 +37,7 @@ def makefile_flags():
 
 FLAGS, EXTRA = makefile_flags()
 FLAGS = FLAGS + ['-S', '--cuda-device-only']
-FILES = ['wkv7_fused.hip', 'wkv7_bwd.hip', 'wkv7_fwd.hip', 'wkv7_wide.hip', 'ddlerp.hip', 'expand_loras.hip', 'mixer_decode.hip',
+FILES = ['wkv7_fused.hip', 'wkv7_bwd.hip', 'wkv7_fwd.hip', 'wkv7_wide.hip', 'ddlerp.hip', 'expand_loras.hip', 'expand_loras16.hip', 'mixer_decode.hip',
          'linear_wgrad.hip', 'selftest.hip', 'wkv7_f32.hip']
 WINDOW = 16   # instructions; a matrix instruction has long finished after that many
 
