@@ -13,10 +13,13 @@ constexpr int REC = 4 * HEAD * D + 4 * HEAD;   // floats of a partial record: dW
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
-// forward for rank 16: block = (head, range of token tiles).  The head's weights and biases are staged in
-// LDS once and each wavefront walks its tiles with the next tile's inputs already in flight - the generic
-// kernel fetches forty weight fragments per tile from memory in the middle of dependent arithmetic
-// and spends most of its time waiting for them.
+// forward: block = (head, range of token tiles).  The head's weights and biases are staged in LDS once and each wavefront
+// walks its tiles with the next tile's inputs already in flight; tiles move as whole lines through the wavefront's part of LDS
+// (see ddlerp.hip: 16 rows per instruction cost 28 ns of a compute unit's time, whole lines 9 and, stored, 20).
+// 16 rows per instruction and two rounds of two blocks per compute unit took 20.9, 22.1, 47 us at 7056, 8192, 16384 tokens x 768
+// channels, 49.5 at 8192 x 1536; whole lines and three blocks per compute unit in one round 16.9, 17.9, 35.9, 36.4 (two rounds of
+// either two or three: 18.9 and 19.6 at 7056).  The bytes are 13, 15, 30, 30 at the rate of a copy, the instructions, a fifth of
+// them transcendental, 11 at 8192 x 768.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, int tiles_per_split,
                                                                  const __bf16* __restrict__ w_in,
@@ -24,65 +27,81 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
                                                                  __bf16* __restrict__ w_out, __bf16* __restrict__ k_out,
                                                                  __bf16* __restrict__ kk_out, __bf16* __restrict__ b_out) {
     __shared__ bf16x4 sW[4 * NBLK][WAVE];    // F(W_i[c0 + 16cb .., :])    lane = channel, reg = rank index
-    __shared__ float sBias[4][HEAD];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ __attribute__((aligned(16))) float sBias[4][HEAD];
+    __shared__ bf16x8 s_tile[4][2][TOK * 8];
+    const int lane = threadIdx.x & 63, l8 = lane >> 3, piece = lane & 7;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Lane L;
     const int h = blockIdx.x, split = blockIdx.y;
     const int c0 = h * HEAD;
     const long ntiles = M / TOK;
     const long tile_begin = (long)split * tiles_per_split;
     const long tile_end = tile_begin + tiles_per_split < ntiles ? tile_begin + tiles_per_split : ntiles;
-    // Channel order inside the head: nothing here depends on which 16 channels form a block (the norm sums all
-    // 64, the rest is elementwise), so blocks 2p and 2p+1 interleave in groups of four - register r of block cb
-    // in column group g is channel 32p + 8g + 4(cb & 1) + r - and a lane's pieces of the two blocks are 8
-    // contiguous channels: one 16-byte access instead of two of 8.
-    auto chan = [](int cb, int j) { return 32 * (cb >> 1) + 8 * (j >> 2) + 4 * (cb & 1) + (j & 3); };   // j = 4g + r
-#pragma unroll
-    for (int cb = 0; cb < NBLK; cb++)
-        sW[wave * NBLK + cb][lane] = *reinterpret_cast<const bf16x4*>(lw.W[wave] + (long)(c0 + chan(cb, L.n)) * 16 + 4 * L.g);
-    sBias[wave][lane] = (float)lw.bias[wave][c0 + lane];
-    __syncthreads();
-    auto bias4 = [&](int i, int cb) { return *reinterpret_cast<const f32x4*>(&sBias[i][chan(cb, 4 * L.g)]); };
-    auto load_tile = [&](const __bf16* p) {   // p: this lane's row, channel c0
-        TileB t;
-#pragma unroll
-        for (int pr = 0; pr < 2; pr++) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(p + 32 * pr + 8 * L.g);
-            t.f[2 * pr] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
-            t.f[2 * pr + 1] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
-        }
-        return t;
-    };
-    auto store_tile = [&](__bf16* p, const TileB& t) {
-#pragma unroll
-        for (int pr = 0; pr < 2; pr++)
-            *reinterpret_cast<bf16x8*>(p + 32 * pr + 8 * L.g) =
-                __builtin_shufflevector(t.f[2 * pr], t.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-    };
+    const unsigned row_bytes = 2 * C, lane_bytes = l8 * row_bytes + 16 * piece, act_bytes = 2 * (D * L.n + 4 * L.g);
+    auto(&buf)[2][TOK * 8] = s_tile[wave];
 
     struct TileIn {
-        TileB wi, ki;
+        bf16x8 wi[2], ki[2];
         bf16x4 act[4];
     };
     auto fetch = [&](long tile) {
         TileIn t;
         const long m0 = tile * TOK;
-        t.wi = load_tile(w_in + (m0 + L.n) * C + c0);
-        t.ki = load_tile(k_in + (m0 + L.n) * C + c0);
 #pragma unroll
-        for (int i = 0; i < 4; i++) t.act[i] = load_act<1>(in.p[i], m0, L).f[0];
+        for (int i = 0; i < 2; i++) {
+            t.wi[i] = piece_at(w_in + (m0 * C + c0), lane_bytes + 8 * i * row_bytes);
+            t.ki[i] = piece_at(k_in + (m0 * C + c0), lane_bytes + 8 * i * row_bytes);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) t.act[i] = *reinterpret_cast<const bf16x4*>(reinterpret_cast<const char*>(in.p[i] + m0 * D) + act_bytes);
         return t;
     };
     long tile = tile_begin + wave;
     TileIn nxt;
     if (tile < tile_end) nxt = fetch(tile);
+    // channel blocks follow the interleaved order of chan16 (frag.hpp): nothing here depends on which 16 channels form a block
+#pragma unroll
+    for (int cb = 0; cb < NBLK; cb++)
+        sW[wave * NBLK + cb][lane] = *reinterpret_cast<const bf16x4*>(lw.W[wave] + (long)(c0 + chan16(cb, L.n)) * D + 4 * L.g);
+    sBias[wave][lane] = (float)lw.bias[wave][c0 + lane];
+    __syncthreads();
+    auto bias4 = [&](int i, int cb) { return *reinterpret_cast<const f32x4*>(&sBias[i][chan16(cb, 4 * L.g)]); };
+    auto store = [&](__bf16* p0, const TileB& t0, __bf16* p1, const TileB& t1, long off) {   // two tiles
+#pragma unroll
+        for (int pr = 0; pr < 2; pr++) {
+            buf[0][piece_slot(L.n, 4 * pr + L.g)] = join(t0.f[2 * pr], t0.f[2 * pr + 1]);
+            buf[1][piece_slot(L.n, 4 * pr + L.g)] = join(t1.f[2 * pr], t1.f[2 * pr + 1]);
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            piece_at(p0 + off, lane_bytes + 8 * i * row_bytes) = buf[0][piece_slot(l8 + 8 * i, piece)];
+            piece_at(p1 + off, lane_bytes + 8 * i * row_bytes) = buf[1][piece_slot(l8 + 8 * i, piece)];
+        }
+        wave_lds_order();
+    };
     for (; tile < tile_end; tile += 4) {
-        const TileIn cur = nxt;
+        const long off = tile * TOK * C + c0;
+        bf16x4 act[4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            buf[0][piece_slot(l8 + 8 * i, piece)] = nxt.wi[i];
+            buf[1][piece_slot(l8 + 8 * i, piece)] = nxt.ki[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) act[i] = nxt.act[i];
+        wave_lds_order();
+        TileB wi, ki;
+#pragma unroll
+        for (int cb = 0; cb < NBLK; cb++) {
+            wi.f[cb] = half_of(buf[0][piece_slot(L.n, 4 * (cb >> 1) + L.g)], cb & 1);
+            ki.f[cb] = half_of(buf[1][piece_slot(L.n, 4 * (cb >> 1) + L.g)], cb & 1);
+        }
+        wave_lds_order();
         nxt = fetch(tile + 4 < tile_end ? tile + 4 : tile);   // past the end: the current tile again (never used)
-        const long off = (tile * TOK + L.n) * C + c0;
         bf16x4 tz;
         {
-            f32x4 t = to_f32(cur.act[0]);
+            f32x4 t = to_f32(act[0]);
 #pragma unroll
             for (int q = 0; q < 4; q++) t[q] = tanhf_(t[q]);
             tz = to_bf16(t);
@@ -92,12 +111,12 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
         float ss = 0.f;
 #pragma unroll
         for (int cb = 0; cb < NBLK; cb++) {
-            const f32x4 kin = to_f32(cur.ki.f[cb]);
+            const f32x4 kin = to_f32(ki.f[cb]);
             z.f[cb] = mma(kin, sW[0 * NBLK + cb][lane], tz);
-            const f32x4 pa = mma(bias4(1, cb), sW[1 * NBLK + cb][lane], cur.act[1]);
-            const f32x4 pma = mma(bias4(2, cb), sW[2 * NBLK + cb][lane], cur.act[2]);
-            const f32x4 pmk = mma(bias4(3, cb), sW[3 * NBLK + cb][lane], cur.act[3]);
-            const f32x4 u = bias4(0, cb) + to_f32(cur.wi.f[cb]);
+            const f32x4 pa = mma(bias4(1, cb), sW[1 * NBLK + cb][lane], act[1]);
+            const f32x4 pma = mma(bias4(2, cb), sW[2 * NBLK + cb][lane], act[2]);
+            const f32x4 pmk = mma(bias4(3, cb), sW[3 * NBLK + cb][lane], act[3]);
+            const f32x4 u = bias4(0, cb) + to_f32(wi.f[cb]);
             f32x4 w, k;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
@@ -111,8 +130,7 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
             wo.f[cb] = to_bf16(w);
             ko.f[cb] = to_bf16(k);
         }
-        store_tile(w_out + off, wo);
-        store_tile(k_out + off, ko);
+        store(w_out, wo, k_out, ko, off);
         const float inorm = rsqrtf(fmaxf(group_sum(ss), 1e-12f));
         TileB kko, bo;
 #pragma unroll
@@ -121,8 +139,7 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
             kko.f[cb] = to_bf16(kk);
             bo.f[cb] = to_bf16(-kk * a.f[cb]);
         }
-        store_tile(kk_out + off, kko);
-        store_tile(b_out + off, bo);
+        store(kk_out, kko, b_out, bo, off);
     }
 }
 
@@ -487,10 +504,10 @@ int lora16_splits(long M, int H) {
 
 void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, __bf16* const outs[4],
                             hipStream_t stream) {
-    // two blocks fit a compute unit: two full rounds of 512, at least four token tiles (one per wavefront) each
+    // three blocks fit a compute unit, all of them in one round; at least four token tiles (one per wavefront) each
     const int H = C / HEAD;
     const long ntiles = M / TOK;
-    long nsplit = 4 * compute_units() / H;
+    long nsplit = 3 * compute_units() / H;
     if (nsplit > ntiles / 4) nsplit = ntiles / 4;
     if (nsplit < 1) nsplit = 1;
     const int tiles_per_split = (int)((ntiles + nsplit - 1) / nsplit);
