@@ -59,9 +59,10 @@ def test_ddlerp_around_the_few_token_limit(B, T, C, D):
     check(*run_both(B, T, C, D, seed=500 + T + D))
 
 
-# an odd count of tiles beyond the few-token limit, and an odd count of channel blocks for the two images: one and three
+# an odd count of tiles beyond the few-token limit, an odd count of channel blocks for the two images (one and three), and an odd
+# count of token ranges for the two groups of a block in the second backward pass (441 tiles in 41 ranges of 11)
 @pytest.mark.parametrize('D', [32, 64])
-@pytest.mark.parametrize('B,T,C', [(1, 4112, 64), (257, 16, 192)])
+@pytest.mark.parametrize('B,T,C', [(1, 4112, 64), (257, 16, 192), (7, 1008, 768)])
 def test_ddlerp_odd_channel_blocks(B, T, C, D):
     check(*run_both(B, T, C, D, seed=600 + T + D))
 

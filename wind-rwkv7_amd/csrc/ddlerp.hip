@@ -538,8 +538,9 @@ struct ParamPartial {   // per (split, 64-channel block); element counts
 };
 __host__ __device__ constexpr int dmap(int jj, int j) { return 8 * (j >> 2) + 4 * jj + (j & 3); }
 
-template <int D>
-__global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(long M, int T, int C, int tiles_per_split,
+// G groups of four wavefronts per block, each with a range of its own; their sums meet in LDS before the record is written.
+template <int D, int G>
+__global__ __launch_bounds__(256 * G, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(long M, int T, int C, int tiles_per_split,
                                                                  const __bf16* __restrict__ x, Dy4 dy,
                                                                  const __bf16* __restrict__ alpha,
                                                                  const __bf16* __restrict__ Lw,
@@ -554,18 +555,31 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
     // Each wavefront's own weight fragments, [k][32-wide half]: 8 KiB in LDS at rank 32 ([wavefront][k][lane]); at
     // rank 64 the streamed images below leave no room for 16 KiB per wavefront and they stay in registers.
     constexpr bool W_LDS = HH == 1;
-    __shared__ bf16x8 s_R[W_LDS ? 4 : 1][W_LDS ? 4 : 1][W_LDS ? WAVE : 1], s_L[W_LDS ? 4 : 1][W_LDS ? 4 : 1][W_LDS ? WAVE : 1];
     bf16x8 r_R[W_LDS ? 1 : 4][HH], r_L[W_LDS ? 1 : 4][HH];
     // LDS images of a tile's streamed rows (elements; row pitches padded by 16 bytes against bank conflicts)
     constexpr int ROW_LD = 64 + 8, MID_LD = 4 * D + 8;
-    __shared__ __attribute__((aligned(16))) __bf16 s_x[2][17 * ROW_LD], s_row[2][4][16 * ROW_LD], s_mid[2][2][16 * MID_LD];
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    struct Images {
+        __bf16 x[2][17 * ROW_LD], row[2][4][16 * ROW_LD], mid[2][2][16 * MID_LD];
+    };
+    constexpr int NEX = 16 * HH + 5;   // the group's sums: dR, dL, dbeta, dalpha
+    __shared__ __attribute__((aligned(16))) union {
+        struct {
+            bf16x8 R[W_LDS ? 4 : 1][W_LDS ? 4 : 1][W_LDS ? WAVE : 1], L[W_LDS ? 4 : 1][W_LDS ? 4 : 1][W_LDS ? WAVE : 1];
+            Images img[G];
+        } s;
+        f32x4 ex[G > 1 ? 4 : 1][G > 1 ? NEX : 1][WAVE];   // at the end
+    } lds;
+    auto &s_R = lds.s.R, &s_L = lds.s.L;
+    const int lane = threadIdx.x & 63, group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6 & 3);
+    auto &s_x = lds.s.img[group].x;
+    auto &s_row = lds.s.img[group].row;
+    auto &s_mid = lds.s.img[group].mid;
     const Lane L;
     const int cw = blockIdx.x * 64 + 16 * w;   // this wavefront's channel j is cw + j
     const long ntiles = M / TOK;
-    const long lo = (long)blockIdx.y * tiles_per_split;
-    const long hi = lo + tiles_per_split < ntiles ? lo + tiles_per_split : ntiles;
+    const long lo = ((long)blockIdx.y * G + group) * tiles_per_split;
+    const long hi = lo + tiles_per_split < ntiles ? lo + tiles_per_split : ntiles;   // (a last group's range can be empty)
     const bf16x4 eye = identity_bf16(L);
     const int cl = cw + 4 * L.g;          // the four contiguous channels of this lane in token layout
 
@@ -583,8 +597,10 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
                 transpose(*reinterpret_cast<const bf16x4*>(Lw + (long)(k * D + 32 * hh + dmap(0, L.n)) * C + cl), eye),
                 transpose(*reinterpret_cast<const bf16x4*>(Lw + (long)(k * D + 32 * hh + dmap(1, L.n)) * C + cl), eye), 0, 1, 2, 3, 4, 5, 6, 7);
             if constexpr (W_LDS) {
-                s_R[w][k][lane] = fr;
-                s_L[w][k][lane] = fl;
+                if (G == 1 || k * G / 4 == group) {   // (read behind the first barrier)
+                    s_R[w][k][lane] = fr;
+                    s_L[w][k][lane] = fl;
+                }
             } else {
                 r_R[k][hh] = fr;
                 r_L[k][hh] = fl;
@@ -601,14 +617,12 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
 #pragma unroll
         for (int j = 0; j < 2 * HH; j++) accR[k][j] = accL[k][j] = zero4();
     }
-    if (lo >= hi) return;   // (cannot happen with the launcher's ranges)
-
     // The streamed operands of a tile - 17 rows of x (one above the tile), 16 rows of each dy, of bmid and of dpre,
     // 18 KiB - are fetched ONCE per block with full 128-byte lines (16 bytes per thread, five loads each), parked in
     // registers for a tile, and written to one of two LDS images from which the wavefronts take their pieces.
     // (Each wavefront fetching its own 32-byte pieces of the rows, and all four the same rows of bmid and dpre,
     // moved four times the bytes between L2 and the compute units and ran at the rate of that link.)
-    const int t = threadIdx.x;
+    const int t = threadIdx.x & 255;
     auto stage_tile = [&](long tile) { return tile < lo ? lo : tile; };   // (past the range: loaded and never used)
     // bmid / dpre: 16 rows of 4D elements, 8 per thread and pass, HH passes
     auto mid_row = [&](int ps) { return (8 * t + 2048 * ps) / (4 * D); };
@@ -712,12 +726,15 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
     // Iteration i works on image i&1 while the registers hold the tile after it, fetched during iteration i-1; they
     // are written to the other image (last read before the previous barrier) and refilled for the tile after that.
     long next = warm ? hi : hi - 1;   // the tile the registers are fetched for
-    fetch(next);
-    park(0);
-    fetch(--next);
+    const bool active = G == 1 || lo < hi;
+    if (active) {
+        fetch(next);
+        park(0);
+        fetch(--next);
+    }
     __syncthreads();
     int it = 0;
-    if (warm) {
+    if (active && warm) {
         park(1);
         fetch(--next);
         body(hi, tpos + TOK, 0, std::false_type{});
@@ -730,6 +747,35 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
         body(tile, tpos, it & 1, std::true_type{});
         __syncthreads();
         tpos = tpos >= TOK ? tpos - TOK : T - TOK;
+    }
+    if constexpr (G > 1) {
+        for (; it < tiles_per_split + 1; it++) __syncthreads();   // the same number of barriers for every group
+        static_assert(G == 2 && sizeof(lds.ex) <= sizeof(lds.s), "");
+        f32x4* const ex = &lds.ex[w][0][lane];
+        if (group == 1) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+#pragma unroll
+                for (int j = 0; j < 2 * HH; j++) {
+                    ex[(4 * HH * k + j) * WAVE] = accR[k][j];
+                    ex[(4 * HH * k + 2 * HH + j) * WAVE] = accL[k][j];
+                }
+                ex[(16 * HH + k) * WAVE] = vbeta[k];
+            }
+            ex[(16 * HH + 4) * WAVE] = valpha;
+        }
+        __syncthreads();
+        if (group == 1) return;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+#pragma unroll
+            for (int j = 0; j < 2 * HH; j++) {
+                accR[k][j] += ex[(4 * HH * k + j) * WAVE];
+                accL[k][j] += ex[(4 * HH * k + 2 * HH + j) * WAVE];
+            }
+            vbeta[k] += ex[(16 * HH + k) * WAVE];
+        }
+        valpha += ex[(16 * HH + 4) * WAVE];
     }
     // this block's partial record: dR [4][64][D], dL [4D][64], dbeta [4][64], dalpha [64]
     float* out = partial + ((long)blockIdx.y * gridDim.x + blockIdx.x) * P::TOTAL;
@@ -753,30 +799,34 @@ __global__ __launch_bounds__(256, D == 32 ? 2 : 1) void ddlerp_bwd_main_kernel(l
     if (L.n == 0) *reinterpret_cast<f32x4*>(out + P::DR + P::DL + P::DBETA + jw + 4 * L.g) = sa;
 }
 
-// sums the partial records over the token splits and scatters them to dR [4][C][D], dL [4D][C],
-// dbeta [4][C], dalpha [C] (all fp32)
+// Sums the partial records over the token splits and scatters them to dR [4][C][D], dL [4D][C], dbeta [4][C], dalpha [C] (all
+// fp32): a thread has four elements of the record and an eighth of the records; the order of the additions is fixed.  (All
+// records to a thread, four at a time: the same time at few records, 75 us instead of 8 for the 512 of 65536 tokens x 64.)
+constexpr int REDUCE_SHARES = 8, REDUCE_COLS = 256 / REDUCE_SHARES;
 template <int D>
 __global__ __launch_bounds__(256) void ddlerp_param_reduce_kernel(int C, int nsplit, const float* __restrict__ partial,
                                                                   float* __restrict__ dR, float* __restrict__ dL,
                                                                   float* __restrict__ dbeta,
                                                                   float* __restrict__ dalpha) {
     using P = ParamPartial<D>;
+    __shared__ f32x4 part[REDUCE_SHARES][REDUCE_COLS];
     const int ncb = C / 64;
     const int cblk = blockIdx.y;
     const int c0 = cblk * 64;
-    const int e = 4 * (blockIdx.x * 256 + threadIdx.x);   // one thread per four elements of the record
-    if (e >= P::TOTAL) return;
-    // four running sums, so that four loads are in flight at a time; the order of the additions is fixed
-    f32x4 s4[4] = {zero4(), zero4(), zero4(), zero4()};
-    const float* src = partial + (long)cblk * P::TOTAL + e;
-    const long pitch = (long)ncb * P::TOTAL;
-    int sp = 0;
-    for (; sp + 4 <= nsplit; sp += 4) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) s4[u] += *reinterpret_cast<const f32x4*>(src + (sp + u) * pitch);
+    const int col = threadIdx.x % REDUCE_COLS, share = threadIdx.x / REDUCE_COLS;
+    const int e = 4 * (blockIdx.x * REDUCE_COLS + col);
+    f32x4 s = zero4();
+    if (e < P::TOTAL) {
+        const float* src = partial + (long)cblk * P::TOTAL + e;
+        const long pitch = (long)ncb * P::TOTAL;
+#pragma unroll 4
+        for (int sp = share; sp < nsplit; sp += REDUCE_SHARES) s += *reinterpret_cast<const f32x4*>(src + sp * pitch);
     }
-    for (; sp < nsplit; sp++) s4[0] += *reinterpret_cast<const f32x4*>(src + sp * pitch);
-    const f32x4 s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    part[share][col] = s;
+    __syncthreads();
+    if (share != 0 || e >= P::TOTAL) return;
+#pragma unroll
+    for (int i = 1; i < REDUCE_SHARES; i++) s += part[i][col];
     float* dst;
     if (e < P::DR) {
         const int d = e % D, c = (e / D) % 64, k = e / (64 * D);
@@ -837,8 +887,8 @@ __global__ __launch_bounds__(256) void first_streams_kernel(int C, const X* __re
 // ------------------------------------------------------------------------------------------------
 namespace {
 constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
-// Token ranges of the second backward pass: two blocks per compute unit of an MI355X (256) over the channel
-// blocks, at least eight tiles each (every block spends one more tile on its carry and writes a 66 KiB record
+// Token ranges of the second backward pass: two groups per compute unit of an MI355X (256) over the channel
+// blocks, at least eight tiles each (every group spends one more tile on its carry, and a block writes a 66 KiB record
 // that the reduction reads back).
 int param_splits(long M, int ncb) {
     const long ntiles = M / TOK;
@@ -913,10 +963,21 @@ void backward_rank(long M, int T, int C, const void* x, const void* alpha, const
 
     hipLaunchKernelGGL((ddlerp_bwd_mid_kernel<D, 2>), dim3((unsigned)((M / TOK + 1) / 2)), dim3(256), 0, stream, M, T, C, c(x), dy,
                        c(R), c(bder), dpre);
-    hipLaunchKernelGGL(ddlerp_bwd_main_kernel<D>, dim3(ncb, nsplit), dim3(256), 0, stream, M, T, C, tiles_per_split, c(x), dy,
-                       c(alpha), c(Lw), c(R), c(beta), c(bmid), dpre, static_cast<__bf16*>(dx), partial);
-    hipLaunchKernelGGL(ddlerp_param_reduce_kernel<D>, dim3((ParamPartial<D>::TOTAL / 4 + 255) / 256, ncb), dim3(256), 0,
-                       stream, C, nsplit, partial,
+    // Two groups to a block where two would share a compute unit anyway (registers allow it at rank 32): half the records.  Second
+    // pass + sums, us, two / one: 8192 tokens x 768 channels 39.1 / 42.6, 4096 x 768 29.8 / 32.3; where a group would have a compute
+    // unit to itself, or the blocks are more than a round, two to a block are slower: 1024 x 768 26.2 / 20.5, 8192 x 1536 77 / 59
+    const bool two = D == 32 && (long)ncb * nsplit > compute_units() && (long)ncb * ((nsplit + 1) / 2) <= compute_units();
+    const int records = two ? (nsplit + 1) / 2 : nsplit;
+    if constexpr (D == 32) {
+        if (two)
+            hipLaunchKernelGGL((ddlerp_bwd_main_kernel<D, 2>), dim3(ncb, records), dim3(512), 0, stream, M, T, C, tiles_per_split, c(x), dy,
+                               c(alpha), c(Lw), c(R), c(beta), c(bmid), dpre, static_cast<__bf16*>(dx), partial);
+    }
+    if (!two)
+        hipLaunchKernelGGL((ddlerp_bwd_main_kernel<D, 1>), dim3(ncb, records), dim3(256), 0, stream, M, T, C, tiles_per_split, c(x), dy,
+                           c(alpha), c(Lw), c(R), c(beta), c(bmid), dpre, static_cast<__bf16*>(dx), partial);
+    hipLaunchKernelGGL(ddlerp_param_reduce_kernel<D>, dim3((ParamPartial<D>::TOTAL / 4 + REDUCE_COLS - 1) / REDUCE_COLS, ncb), dim3(256), 0,
+                       stream, C, records, partial,
                        static_cast<float*>(dR), static_cast<float*>(dL), static_cast<float*>(dbeta),
                        static_cast<float*>(dalpha));
 }
