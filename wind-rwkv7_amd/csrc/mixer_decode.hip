@@ -414,46 +414,105 @@ __device__ __forceinline__ void expand_tile(HeadTile& s, const HeadArgs& A, int 
     lds_barrier();
 }
 
-// token n of the tile on value rows chan16(ib, .) of the state; y goes to LDS
-__device__ __forceinline__ void update_state(HeadTile& s, f32x4 (&S)[NBLK], int n, int ib, const Lane& L) {
-    auto vec = [&](const __bf16 (&a)[TOK][HeadTile::LD], int jb) { return to_f32(*reinterpret_cast<const bf16x4*>(&a[n][chan16(jb, 4 * L.g)])); };
-    float sa = 0.f;
+// A wavefront's sixteen value rows of the state, 16 ib ..: register i of lane (n, g) is columns 4n .. 4n + 3 of row 4i + g, so that
+// a load or store is 1 KiB in one piece and a token's vectors are four channels per lane.  (As the fragments of the sequence
+// kernels, four lanes to a row and sixteen columns each, every access touched sixteen rows, 28 ns of a compute unit's time
+// instead of 9 to load and 20 to store, the vectors were four times the LDS reads, and the sums over a row went through the LDS
+// crossbar: the head kernel of a step at 768 channels and 1, 32, 256, 512 sequences 6.9, 9.4, 25.4, 38.8 -> 5.9, 7.7, 20.5, 35.8
+// us, where the states of 256 sequences are 100 MB to move, 20 us at the rate of a copy.)
+__device__ __forceinline__ void load_state(f32x4 (&S)[NBLK], const void* s, int state_f32, int bh, int ib, const Lane& L) {
+    const long off = ((long)bh * HEAD + 16 * ib + L.g) * HEAD + 4 * L.n;
 #pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) {
-        const f32x4 a = vec(s.kk, jb);
-#pragma unroll
-        for (int q = 0; q < 4; q++) sa += S[jb][q] * a[q];
+    for (int i = 0; i < NBLK; i++) {
+        if (s == nullptr) S[i] = zero4();
+        else if (state_f32) S[i] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(s) + off + 4 * i * HEAD);
+        else S[i] = to_f32(*reinterpret_cast<const bf16x4*>(static_cast<const __bf16*>(s) + off + 4 * i * HEAD));
     }
-    sa = group_sum(sa);   // over the four lanes that share the state's row
-    const float vrow = (float)s.v[n][chan16(ib, L.n)];
-    float acc = 0.f;
+}
+__device__ __forceinline__ void store_state(const f32x4 (&S)[NBLK], void* s, int state_f32, int bh, int ib, const Lane& L) {
+    if (s == nullptr) return;
+    const long off = ((long)bh * HEAD + 16 * ib + L.g) * HEAD + 4 * L.n;
 #pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) {
-        const f32x4 d = *reinterpret_cast<const f32x4*>(&s.decay[n][chan16(jb, 4 * L.g)]);
-        const f32x4 b = vec(s.b, jb), k = vec(s.k, jb), r = vec(s.r, jb);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            S[jb][q] = S[jb][q] * d[q] + sa * b[q] + vrow * k[q];
-            acc += S[jb][q] * r[q];
-        }
+    for (int i = 0; i < NBLK; i++) {
+        if (state_f32) *reinterpret_cast<f32x4*>(static_cast<float*>(s) + off + 4 * i * HEAD) = S[i];
+        else *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(s) + off + 4 * i * HEAD) = to_bf16(S[i]);
     }
-    acc = group_sum(acc);
-    if (L.g == 0) s.y[n][chan16(ib, L.n)] = acc;
+}
+// a lane's part of a token's vectors: its four columns, and of v its four rows
+struct TokenVectors {
+    bf16x4 kk, b, k, r;
+    f32x4 decay;
+    __bf16 v[NBLK];
+};
+__device__ __forceinline__ TokenVectors token_vectors(const HeadTile& s, int n, int ib, const Lane& L) {
+    TokenVectors t;
+    auto vec = [&](const __bf16 (&a)[TOK][HeadTile::LD]) { return *reinterpret_cast<const bf16x4*>(&a[n][4 * L.n]); };
+    t.kk = vec(s.kk), t.b = vec(s.b), t.k = vec(s.k), t.r = vec(s.r);
+    t.decay = *reinterpret_cast<const f32x4*>(&s.decay[n][4 * L.n]);
+#pragma unroll
+    for (int i = 0; i < NBLK; i++) t.v[i] = s.v[n][16 * ib + 4 * i + L.g];
+    return t;
+}
+// token n of the tile on a wavefront's rows of the state; y goes to LDS
+__device__ __forceinline__ void update_state(HeadTile& s, f32x4 (&S)[NBLK], const TokenVectors& t, int n, int ib, const Lane& L) {
+    const f32x4 a = to_f32(t.kk), b = to_f32(t.b), k = to_f32(t.k), r = to_f32(t.r), d = t.decay;
+    float sa[NBLK], y[NBLK];
+#pragma unroll
+    for (int i = 0; i < NBLK; i++) sa[i] = (S[i][0] * a[0] + S[i][1] * a[1]) + (S[i][2] * a[2] + S[i][3] * a[3]);
+#pragma unroll
+    for (int i = 0; i < NBLK; i++) sa[i] = row_sum(sa[i]);   // over the sixteen lanes that share the state's row
+#pragma unroll
+    for (int i = 0; i < NBLK; i++) {
+        const float vrow = (float)t.v[i];
+#pragma unroll
+        for (int q = 0; q < 4; q++) S[i][q] = S[i][q] * d[q] + sa[i] * b[q] + vrow * k[q];
+        y[i] = (S[i][0] * r[0] + S[i][1] * r[1]) + (S[i][2] * r[2] + S[i][3] * r[3]);
+    }
+#pragma unroll
+    for (int i = 0; i < NBLK; i++) y[i] = row_sum(y[i]);
+    const float out = L.n < 2 ? (L.n == 0 ? y[0] : y[1]) : (L.n == 2 ? y[2] : y[3]);   // lanes n < 4: row 4n + g
+    if (L.n < NBLK) s.y[n][16 * ib + 4 * L.n + L.g] = out;
+}
+// tokens 0 .. n - 1 of the tile one after the other, the next one's vectors on their way
+__device__ __forceinline__ void update_tokens(HeadTile& s, f32x4 (&S)[NBLK], int n, int ib, const Lane& L) {
+    TokenVectors t = token_vectors(s, 0, ib, L);
+    for (int i = 0; i < n; i++) {
+        const TokenVectors next = token_vectors(s, i + 1 < n ? i + 1 : i, ib, L);
+        update_state(s, S, t, i, ib, L);
+        t = next;
+    }
 }
 
-// GroupNorm, bonus and gate of token n, lane = channel; out: its row
-__device__ __forceinline__ void finish_token(const HeadTile& s, const float* ln_params, int C, int h, int n, __bf16* out_row, int lane) {
+// GroupNorm, bonus and gate of tokens first, first + step, .. below end, lane = channel; row(n): token n's row of the output.
+// AT_ONCE at a time: a token is three sums over the wavefront, two of them one after the other.
+template <int AT_ONCE, class Row>
+__device__ __forceinline__ void finish_tokens(const HeadTile& s, const float* ln_params, int C, int h, int first, int step, int end, int lane,
+                                              Row row) {
     auto head_sum = [](float x) {
         x = row_sum(x);
         return group_sum(x);
     };
-    const float y = s.y[n][lane];
-    const float mean = head_sum(y) * (1.f / HEAD);
-    const float istd = rsqrtf(head_sum((y - mean) * (y - mean)) * (1.f / HEAD) + LN_EPS);
     const float* lp = ln_params + h * HEAD + lane;
-    const float dot = head_sum((float)s.r[n][lane] * (float)s.k[n][lane] * lp[2 * (long)C]);
-    const float out = ((y - mean) * istd * lp[0] + lp[C] + dot * (float)s.v[n][lane]) * (float)s.g[n][lane];
-    out_row[h * HEAD + lane] = (__bf16)out;
+    const float scale = lp[0], shift = lp[C], bonus = lp[2 * (long)C];
+    for (int n0 = first; n0 < end; n0 += AT_ONCE * step) {
+        int n[AT_ONCE];
+        float y[AT_ONCE], mean[AT_ONCE], var[AT_ONCE], dot[AT_ONCE];
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; j++) {
+            n[j] = n0 + j * step < end ? n0 + j * step : n0;   // (past the last: the first again, not stored)
+            y[j] = s.y[n[j]][lane];
+            mean[j] = head_sum(y[j]) * (1.f / HEAD);
+            dot[j] = head_sum((float)s.r[n[j]][lane] * (float)s.k[n[j]][lane] * bonus);
+        }
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; j++) var[j] = head_sum((y[j] - mean[j]) * (y[j] - mean[j])) * (1.f / HEAD);
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; j++) {
+            const float istd = rsqrtf(var[j] + LN_EPS);
+            const float out = ((y[j] - mean[j]) * istd * scale + shift + dot[j] * (float)s.v[n[j]][lane]) * (float)s.g[n[j]][lane];
+            if (n0 + j * step < end) row(n[j])[h * HEAD + lane] = (__bf16)out;
+        }
+    }
 }
 
 // One token per sequence: block = (some rows of a 16-row tile, head).  Every wavefront asks for the first state it updates
@@ -470,23 +529,19 @@ __global__ __launch_bounds__(256 * GROUPS) void decode_head_kernel(const HeadArg
     const int ib = wave & 3, group = wave >> 2;
     f32x4 S[NBLK], Sn[NBLK];
     auto fetch = [&](f32x4 (&D)[NBLK], int r) {
-        const int bh = (row0 + (r < end ? r : end - 1)) * A.H + h;
-#pragma unroll
-        for (int jb = 0; jb < NBLK; jb++) D[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+        load_state(D, A.state_in, A.state_f32, (row0 + (r < end ? r : end - 1)) * A.H + h, ib, L);
     };
     fetch(S, r0 + group);
     expand_tile(s, A, h, row0, A.rows - 1, wave, L);
     for (int r = r0 + group; r < end; r += GROUPS) {
         fetch(Sn, r + GROUPS);   // (past the last row: that row again, unused)
-        update_state(s, S, r, ib, L);
+        update_state(s, S, token_vectors(s, r, ib, L), r, ib, L);
+        store_state(S, A.state, A.state_f32, (row0 + r) * A.H + h, ib, L);
 #pragma unroll
-        for (int jb = 0; jb < NBLK; jb++) {
-            store_state_frag(A.state, A.state_f32, (row0 + r) * A.H + h, ib, jb, L, S[jb]);
-            S[jb] = Sn[jb];
-        }
+        for (int i = 0; i < NBLK; i++) S[i] = Sn[i];
     }
     lds_barrier();
-    for (int r = r0 + wave; r < end; r += 4 * GROUPS) finish_token(s, A.ln_params, A.C, h, r, A.ya + (long)(row0 + r) * A.C, lane);
+    finish_tokens<1>(s, A.ln_params, A.C, h, r0 + wave, 4 * GROUPS, end, lane, [&](int r) { return A.ya + (long)(row0 + r) * A.C; });
 }
 
 // T tokens per sequence, one after the other on a state that stays in registers: block = (sequence, head).
@@ -496,24 +551,22 @@ __global__ __launch_bounds__(256) void prompt_head_kernel(const HeadArgs A) {
     const Lane L;
     const int h = blockIdx.x, seq = blockIdx.y, bh = seq * A.H + h;
     f32x4 S[NBLK];
-#pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+    load_state(S, A.state_in, A.state_f32, bh, ib, L);
     for (int t0 = 0; t0 < A.T; t0 += TOK) {
         const int first = seq * A.T + t0, n = A.T - t0 < TOK ? A.T - t0 : TOK;
         expand_tile(s, A, h, first, first + n - 1, ib, L);
-        for (int t = 0; t < n; t++) update_state(s, S, t, ib, L);
+        update_tokens(s, S, n, ib, L);
         lds_barrier();
-        for (int t = ib; t < n; t += 4) finish_token(s, A.ln_params, A.C, h, t, A.ya + (long)(first + t) * A.C, lane);
+        finish_tokens<4>(s, A.ln_params, A.C, h, ib, 4, n, lane, [&](int t) { return A.ya + (long)(first + t) * A.C; });
         lds_barrier();   // (the next tile overwrites what the epilogue reads)
     }
-#pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.state, A.state_f32, bh, ib, jb, L, S[jb]);
+    store_state(S, A.state, A.state_f32, bh, ib, L);
 }
 
 // The recurrence alone, token by token, with its operands in memory: the tokens of a prompt after its last whole chunk, whose
 // state the sequence kernels would multiply in bf16.  Block = (sequence, head).  Bound by latency: 11 tokens x 2 x 12 heads take
-// 10.4 us, of a token's two row sums one after the other, a barrier and the epilogue (operands of the next token asked for
-// one token ahead: 11.0).  The same tokens through the four kernels of a step instead: 26 us more for the prompt.
+// 8.5 us, of a token's two row sums one after the other, a barrier and the epilogue (one token at a time there and no vectors
+// asked for ahead: 9.3; with fragments of the state 10.8).  The same tokens through the four kernels of a step instead: 26 us more for the prompt.
 struct TokensArgs {
     const __bf16 *w, *k, *b, *r, *v, *kk, *g;   // at the sequences' first token
     __bf16* y;
@@ -529,8 +582,7 @@ __global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
     const Lane L;
     const int bh = blockIdx.x, seq = bh / A.H, h = bh - seq * A.H;
     f32x4 S[NBLK];
-#pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.state_in, A.state_f32, bh, ib, jb, L);
+    load_state(S, A.state_in, A.state_f32, bh, ib, L);
     // 16 bytes per thread and load: eight channels of one of the sixteen tokens, two tensors at a time (wavefronts 0, 1 and 2, 3)
     const int row = (threadIdx.x & 127) >> 3, c = 8 * (threadIdx.x & 7);
     const bool second = threadIdx.x >= 128;
@@ -549,14 +601,12 @@ __global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
         for (int q = 0; q < 4; q++) d[q] = __expf(-__expf(d[q]));
         *reinterpret_cast<f32x4*>(&s.decay[row][c + (second ? 4 : 0)]) = d;
         lds_barrier();
-        for (int i = 0; i < n; i++) update_state(s, S, i, ib, L);
+        update_tokens(s, S, n, ib, L);
         lds_barrier();
-        for (int i = ib; i < n; i += 4)
-            finish_token(s, A.ln_params, A.C, h, i, A.y + (long)seq * A.seq + (long)(t0 + i) * A.C, lane);
+        finish_tokens<4>(s, A.ln_params, A.C, h, ib, 4, n, lane, [&](int i) { return A.y + (long)seq * A.seq + (long)(t0 + i) * A.C; });
         lds_barrier();   // (the next sixteen overwrite what the epilogue reads)
     }
-#pragma unroll
-    for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.state, A.state_f32, bh, ib, jb, L, S[jb]);
+    store_state(S, A.state, A.state_f32, bh, ib, L);
 }
 
 constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
