@@ -169,7 +169,10 @@ __global__ __launch_bounds__(256) void decode_lerp_kernel(const MixIn in, int C,
 
 // ------------------------------------------------------------------------------------------------
 // 2./4. linear: out_s = in_s W_s^T for up to nine (input, weight) pairs.  Block = CB x 16 output columns of one pair
-// x RT 16-row tiles; its four wavefronts take every fourth 32-channel step of the contraction.  LERP: the input is the
+// x RT 16-row tiles; its four wavefronts take every fourth 64-channel step of the contraction.  The weights arrive as whole
+// lines and pass through LDS (16 rows per instruction, as fragments lie, cost a compute unit three times the lookups; us, six first-half pairs / output
+// projection, then -> now: 768 channels, one sequence 5.8 / 3.8 -> 5.7 / 3.4, 32 10.1 / 3.7 -> 9.0 / 3.6, 64 11.3 / 4.0 -> 10.5 / 3.9; 2048
+// channels, 16 sequences 20.7 / 6.4 -> 18.8 / 5.2).  LERP: the input is the
 // pair's token-shifted stream y_k = x + xx (mid_k R_k^T + beta_k), made 32 channels at a time where it is multiplied (one
 // row of R per lane, ordered so that the two 16-channel results are the lane's eight contiguous channels 8g .. 8g+7).
 // Every column block repeats that for its stream, so few columns per block where the launch is latency (a tile or two),
@@ -192,8 +195,19 @@ struct LinArgs {
 template <bool LERP, int CB, int RT>
 __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, const MixIn mix) {
     constexpr int NW = 4;
-    __shared__ f32x4 part[NW][RT][CB][WAVE];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int U = CB * RT == 1 ? 3 : CB * RT <= 4 ? 2 : 1;   // steps of a wavefront in flight
+    // R too passes through LDS where there are several column blocks: its fragments touch two lines per four lanes, not four, and
+    // a launch that is all latency pays the way (one sequence 6.1 us instead of 5.7; 64 sequences 10.5 instead of 10.9).
+    constexpr bool R_LINES = LERP && CB > 1;
+    constexpr int AREAS = CB * RT == 1 ? U : 1;                 // (latency: all of them written before the first is read)
+    struct Weights {   // of a wavefront's 64 channels: W as pieces of rows (piece_slot), R as rows of four pieces (r_slot)
+        bf16x8 w[CB][16 * 8], r[R_LINES ? 64 * 4 : 1];
+    };
+    __shared__ union {
+        Weights weights[NW][AREAS];
+        f32x4 part[NW][RT][CB][WAVE];
+    } lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l8 = lane >> 3, piece = lane & 7;
     const Lane L;
     // which pair this block belongs to (the descriptor fields through scalar selects, not an indexed copy of the
     // argument struct)
@@ -241,65 +255,107 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, con
             irow[t] = in + (long)trow[t] * C + 8 * L.g;
         }
     }
-    const __bf16* wrow[CB];   // lane = output column
+    const __bf16* wcol[CB];   // the column blocks' first rows of W
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++) wrow[cb] = W + (long)((col0 + 16 * cb < N ? col0 + 16 * cb : col0) + L.n) * C + 8 * L.g;
-    // row j of the step's two R fragments: channel 8(n/4) + 4j + n%4
-    const __bf16* rrow = LERP ? mix.R + ((long)ks * C + 8 * (L.n >> 2) + (L.n & 3)) * R_MIX + 8 * L.g : nullptr;
+    for (int cb = 0; cb < CB; cb++) wcol[cb] = W + (long)(col0 + 16 * cb < N ? col0 + 16 * cb : col0) * C;
+    const unsigned w_bytes = 2 * ((unsigned)l8 * C + 8 * piece), w_rows8 = 16 * (unsigned)C;
+    // row j of a 32-channel step's two R fragments: channel 8(n/4) + 4j + n%4
+    const __bf16* rrow = LERP ? mix.R + ((long)ks * C + (R_LINES ? 0 : 8 * (L.n >> 2) + (L.n & 3))) * R_MIX + (R_LINES ? 8 * lane : 8 * L.g) : nullptr;
+    // in LDS sixteen such rows' pieces lie in different banks of 16 bytes
+    auto r_slot = [](int channel, int p) { return 4 * channel + (p ^ (channel >> 3 & 3)); };
     const __bf16* brow = LERP ? mix.beta + (long)ks * C + 8 * L.g : nullptr;
     f32x4 acc[RT][CB];
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
         for (int cb = 0; cb < CB; cb++) acc[t][cb] = zero4();
-    const int nk = C / 32;
-    constexpr int U = CB * RT == 1 ? 6 : CB * RT <= 4 ? 3 : 2;
+    const int nk = C / 64;
     for (int s0 = wave; s0 < nk; s0 += NW * U) {   // U steps of this wavefront at a time, all loads before the products
-        bf16x8 wv[U][CB], iv[U][RT], pv[U][RT], r0[U], r1[U], be[U];
+        bf16x8 wv[U][CB][2], iv[U][RT][2], pv[U][RT][2], rv[U][4], be[U][2];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int s = s0 + NW * u < nk ? s0 + NW * u : s0;   // (past the end: the first step again, not used)
+            const int c = 64 * (s0 + NW * u < nk ? s0 + NW * u : s0);   // (past the end: the first step again, not used)
 #pragma unroll
-            for (int cb = 0; cb < CB; cb++) wv[u][cb] = *reinterpret_cast<const bf16x8*>(wrow[cb] + 32 * s);
+            for (int cb = 0; cb < CB; cb++)
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
-                iv[u][t] = *reinterpret_cast<const bf16x8*>(irow[t] + 32 * s);
-                if constexpr (LERP) pv[u][t] = *reinterpret_cast<const bf16x8*>(prow[t] + 32 * s);
-            }
+                for (int i = 0; i < 2; i++) wv[u][cb][i] = piece_at(wcol[cb] + c, w_bytes + i * w_rows8);
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    iv[u][t][i] = *reinterpret_cast<const bf16x8*>(irow[t] + c + 32 * i);
+                    if constexpr (LERP) pv[u][t][i] = *reinterpret_cast<const bf16x8*>(prow[t] + c + 32 * i);
+                }
             if constexpr (LERP) {
-                r0[u] = *reinterpret_cast<const bf16x8*>(rrow + (long)32 * s * R_MIX);
-                r1[u] = *reinterpret_cast<const bf16x8*>(rrow + (long)(32 * s + 4) * R_MIX);
-                be[u] = *reinterpret_cast<const bf16x8*>(brow + 32 * s);
+#pragma unroll
+                for (int i = 0; i < 4; i++) rv[u][i] = *reinterpret_cast<const bf16x8*>(rrow + (long)(c + (R_LINES ? 16 * i : 32 * (i >> 1) + 4 * (i & 1))) * R_MIX);
+#pragma unroll
+                for (int i = 0; i < 2; i++) be[u][i] = *reinterpret_cast<const bf16x8*>(brow + c + 32 * i);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+        auto park = [&](int u) {
+            Weights& mine = lds.weights[wave][u % AREAS];
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) mine.w[cb][piece_slot(l8 + 8 * i, piece)] = wv[u][cb][i];
+            if constexpr (R_LINES) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) mine.r[r_slot(16 * i + (lane >> 2), lane & 3)] = rv[u][i];
+            }
+        };
+        if constexpr (AREAS == U) {
+#pragma unroll
+            for (int u = 0; u < U; u++) park(u);
+            wave_lds_order();
+        }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (s0 + NW * u >= nk) break;
+            if constexpr (AREAS != U) {
+                park(u);
+                wave_lds_order();
+            }
+            const Weights& mine = lds.weights[wave][u % AREAS];
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
-                if constexpr (LERP) {
-                    const f32x4 c0 = mma8(to_f32(lo4(be[u])), r0[u], bm[t]);   // lane = token, channels 8g + r
-                    const f32x4 c1 = mma8(to_f32(hi4(be[u])), r1[u], bm[t]);   // channels 8g + 4 + r
-                    pv[u][t] = or_zero(pv[u][t], zero[t]);
-                    const f32x4 x0 = to_f32(lo4(iv[u][t])), x1 = to_f32(hi4(iv[u][t]));
-                    iv[u][t] = cat8(to_bf16(x0 + (to_f32(lo4(pv[u][t])) - x0) * c0), to_bf16(x1 + (to_f32(hi4(pv[u][t])) - x1) * c1));
+            for (int i = 0; i < 2; i++) {   // 32 channels
+                bf16x8 wf[CB], r0 = rv[u][2 * i], r1 = rv[u][2 * i + 1];
+                if constexpr (R_LINES) {
+                    const int channel = 32 * i + 8 * (L.n >> 2) + (L.n & 3);
+                    r0 = mine.r[r_slot(channel, L.g)], r1 = mine.r[r_slot(channel + 4, L.g)];
                 }
 #pragma unroll
-                for (int cb = 0; cb < CB; cb++) acc[t][cb] = mma8(acc[t][cb], wv[u][cb], iv[u][t]);
+                for (int cb = 0; cb < CB; cb++) wf[cb] = mine.w[cb][piece_slot(L.n, 4 * i + L.g)];
+#pragma unroll
+                for (int t = 0; t < RT; t++) {
+                    bf16x8 in8 = iv[u][t][i];
+                    if constexpr (LERP) {
+                        const f32x4 c0 = mma8(to_f32(lo4(be[u][i])), r0, bm[t]);   // lane = token, channels 8g + r
+                        const f32x4 c1 = mma8(to_f32(hi4(be[u][i])), r1, bm[t]);   // channels 8g + 4 + r
+                        const bf16x8 p8 = or_zero(pv[u][t][i], zero[t]);
+                        const f32x4 x0 = to_f32(lo4(in8)), x1 = to_f32(hi4(in8));
+                        in8 = cat8(to_bf16(x0 + (to_f32(lo4(p8)) - x0) * c0), to_bf16(x1 + (to_f32(hi4(p8)) - x1) * c1));
+                    }
+#pragma unroll
+                    for (int cb = 0; cb < CB; cb++) acc[t][cb] = mma8(acc[t][cb], wf[cb], in8);
+                }
             }
+            if constexpr (AREAS != U) wave_lds_order();
         }
+        wave_lds_order();
     }
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
-        for (int cb = 0; cb < CB; cb++) part[wave][t][cb][lane] = acc[t][cb];
+        for (int cb = 0; cb < CB; cb++) lds.part[wave][t][cb][lane] = acc[t][cb];
     __syncthreads();
     for (int o = wave; o < RT * CB; o += NW) {   // a wavefront finishes a 16 x 16 result
         const int t = o / CB, cb = o % CB;
-        f32x4 r = part[0][t][cb][lane];   // lane = token, reg = column 4g + r
+        f32x4 r = lds.part[0][t][cb][lane];   // lane = token, reg = column 4g + r
 #pragma unroll
-        for (int w = 1; w < NW; w++) r += part[w][t][cb][lane];
+        for (int w = 1; w < NW; w++) r += lds.part[w][t][cb][lane];
         if (act) {
             r = to_f32(to_bf16(r));
 #pragma unroll
@@ -640,7 +696,8 @@ int head_rows_per_block(int B, int H) {
 // the streams are written once (decode_lerp_kernel, a launch more) and multiplied by the grouped kernel of the sequence path,
 // whose tiles share both operands through LDS.  us, linear / lerp + grouped: 768 channels 128 rows 13.3/13.2, 192 17.0/13.3,
 // 256 18.1/13.8, 512 25.0/17.3; 1024 channels 128 rows 14.8/14.4; 1280 channels 96 rows 17.0/15.9; 2048 channels 32 rows
-// 19.6/20.8, 48 33.3/21.2, 128 38.9/22.2, 256 73.5/27, 512 133/57 (and the launch costs about one).
+// 19.6/20.8, 48 33.3/21.2, 128 38.9/22.2, 256 73.5/27, 512 133/57 (and the launch costs about one).  (Linear with its weights as
+// fragments; as whole lines it takes about a tenth less.)
 bool streams_in_memory(long rows, long C) { return rows * C * C >= (rows >= 160 ? 110000000 : 160000000) && rows > 32; }
 // The output projection alone makes nothing again, and the grouped kernel's tiles are few for it (2048 channels, 256 rows
 // 14.2/17.8 us, 512 rows 27.8/18.4; 1536 channels, 512 rows 19.8/15).
