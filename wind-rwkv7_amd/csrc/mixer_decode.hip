@@ -54,7 +54,8 @@ __device__ __forceinline__ bf16x8 cat8(bf16x4 a, bf16x4 b) { return __builtin_sh
 
 // ------------------------------------------------------------------------------------------------
 // 1. mid = tanh((x + xx alpha) L^T),  xx = x_prev - x.  Block = 16 of the 128 columns x one 16-row tile; its NW wavefronts
-// take every NW-th 32-channel step of the contraction.
+// take every NW-th 64-channel step of the contraction, weights and tokens as whole lines through LDS; us, fragments straight from
+// memory -> so: 768 channels, one sequence 4.9 -> 4.9, 32 5.9 -> 5.1, 256 6.4 -> 5.4; 2048 channels, 16 sequences 9.6 -> 6.6.
 // ------------------------------------------------------------------------------------------------
 constexpr int MID = 4 * R_MIX;
 
@@ -73,7 +74,7 @@ struct TokenRows {
 };
 __device__ __forceinline__ TokenRows token_rows(const MixIn& in, int row, int C) {
     const int m = row < in.rows ? row : in.rows - 1;
-    const int seq = m / in.T;
+    const int seq = in.T == 1 ? m : m / in.T;   // (a division is 40 instructions at the head of a launch that is all latency)
     TokenRows r;
     r.at = (long)m * C;
     const bool start = m == seq * in.T;
@@ -87,45 +88,90 @@ __device__ __forceinline__ bf16x8 or_zero(bf16x8 v, bool zero) { return zero ? b
 template <int NW, int U>   // wavefronts, and steps of a wavefront in flight at a time
 __global__ __launch_bounds__(64 * NW) void decode_mid_kernel(const MixIn in, int C, const __bf16* __restrict__ alpha,
                                                          const __bf16* __restrict__ Lw, __bf16* __restrict__ x_carry) {
-    __shared__ f32x4 part[NW][WAVE];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int AREAS = NW <= 4 ? U : 1;   // all of a round written before the first is read, where there is room
+    struct Image {   // of a wavefront's 64 channels, pieces of rows (piece_slot): the weights; the input, hi and lo
+        bf16x8 w[TOK * 8], a[2][TOK * 8];
+    };
+    __shared__ union {
+        Image img[NW][AREAS];
+        f32x4 part[NW][WAVE];
+    } lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l8 = lane >> 3, piece = lane & 7;
     const Lane L;
     const int ob = blockIdx.x, row = blockIdx.y * TOK + L.n;
-    const TokenRows tr = token_rows(in, row, C);
-    const __bf16 *xrow = in.x + tr.at + 8 * L.g, *prow = tr.prev_of + tr.prev + 8 * L.g;
-    const __bf16* lrow = Lw + (long)(16 * ob + L.n) * C + 8 * L.g;   // lane = mid index
+    const __bf16 *xrow[2], *prow[2];
+    bool zero[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const TokenRows tr = token_rows(in, blockIdx.y * TOK + l8 + 8 * i, C);
+        xrow[i] = in.x + tr.at + 8 * piece;
+        prow[i] = tr.prev_of + tr.prev + 8 * piece;
+        zero[i] = tr.zero;
+    }
+    const unsigned w_bytes = 2 * ((unsigned)l8 * C + 8 * piece), w_rows8 = 16 * (unsigned)C;
     f32x4 acc0 = zero4(), acc1 = zero4();
-    const int nk = C / 32;
+    const int nk = C / 64;
     for (int s0 = wave; s0 < nk; s0 += NW * U) {   // U steps of this wavefront at a time, all loads before the products
-        bf16x8 xc[U], xp[U], al[U], lw[U];
+        bf16x8 xc[U][2], xp[U][2], al[U], lw[U][2];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int c = 32 * (s0 + NW * u < nk ? s0 + NW * u : s0);   // (past the end: the first step again, not used)
-            xc[u] = *reinterpret_cast<const bf16x8*>(xrow + c);
-            xp[u] = *reinterpret_cast<const bf16x8*>(prow + c);
-            al[u] = *reinterpret_cast<const bf16x8*>(alpha + c + 8 * L.g);
-            lw[u] = *reinterpret_cast<const bf16x8*>(lrow + c);
+            const int c = 64 * (s0 + NW * u < nk ? s0 + NW * u : s0);   // (past the end: the first step again, not used)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                xc[u][i] = *reinterpret_cast<const bf16x8*>(xrow[i] + c);
+                xp[u][i] = *reinterpret_cast<const bf16x8*>(prow[i] + c);
+                lw[u][i] = piece_at(Lw + (long)16 * ob * C + c, w_bytes + i * w_rows8);
+            }
+            al[u] = *reinterpret_cast<const bf16x8*>(alpha + c + 8 * piece);
         }
         __builtin_amdgcn_sched_barrier(0);
+        auto park = [&](int u) {
+            Image& mine = lds.img[wave][u % AREAS];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                // the interpolated input as a bf16 pair (hi + lo), as the sequence kernel has it: it feeds tanh', which
+                // is steep, and must not be rounded to 8 bits before the C-term sum
+                bf16x4 h[2], l[2];
+                const bf16x8 p8 = or_zero(xp[u][i], zero[i]);
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    const f32x4 cv = to_f32(half_of(xc[u][i], hf));
+                    const f32x4 av = cv + (to_f32(half_of(p8, hf)) - cv) * to_f32(half_of(al[u], hf));
+                    h[hf] = to_bf16(av);
+                    l[hf] = to_bf16(av - to_f32(h[hf]));
+                }
+                const int slot = piece_slot(l8 + 8 * i, piece);
+                mine.w[slot] = lw[u][i];
+                mine.a[0][slot] = join(h[0], h[1]);
+                mine.a[1][slot] = join(l[0], l[1]);
+            }
+        };
+        if constexpr (AREAS == U) {
+#pragma unroll
+            for (int u = 0; u < U; u++) park(u);
+            wave_lds_order();
+        }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (s0 + NW * u >= nk) break;
-            // the interpolated input as a bf16 pair (hi + lo), as the sequence kernel has it: it feeds tanh', which
-            // is steep, and must not be rounded to 8 bits before the C-term sum
-            bf16x4 h[2], l[2];
-            xp[u] = or_zero(xp[u], tr.zero);
-#pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                const f32x4 cv = to_f32(hf ? hi4(xc[u]) : lo4(xc[u]));
-                const f32x4 av = cv + (to_f32(hf ? hi4(xp[u]) : lo4(xp[u])) - cv) * to_f32(hf ? hi4(al[u]) : lo4(al[u]));
-                h[hf] = to_bf16(av);
-                l[hf] = to_bf16(av - to_f32(h[hf]));
+            if constexpr (AREAS != U) {
+                park(u);
+                wave_lds_order();
             }
-            acc0 = mma8(acc0, lw[u], cat8(h[0], h[1]));   // lane = token
-            acc1 = mma8(acc1, lw[u], cat8(l[0], l[1]));
+            const Image& mine = lds.img[wave][u % AREAS];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int slot = piece_slot(L.n, 4 * i + L.g);
+                const bf16x8 wf = mine.w[slot];            // lane = mid index
+                acc0 = mma8(acc0, wf, mine.a[0][slot]);   // lane = token
+                acc1 = mma8(acc1, wf, mine.a[1][slot]);
+            }
+            if constexpr (AREAS != U) wave_lds_order();
         }
+        wave_lds_order();
     }
-    part[wave][lane] = acc0 + acc1;
+    __syncthreads();
+    lds.part[wave][lane] = acc0 + acc1;
     // the tokens to hand on, the last of each sequence: dealt over all blocks
     if (x_carry) {
         const int per_row = C / 8, nseq = in.rows / in.T;
@@ -138,9 +184,9 @@ __global__ __launch_bounds__(64 * NW) void decode_mid_kernel(const MixIn in, int
     }
     __syncthreads();
     if (wave != 0) return;
-    f32x4 t = part[0][lane];   // lane = token, reg = column 4g + r
+    f32x4 t = lds.part[0][lane];   // lane = token, reg = column 4g + r
 #pragma unroll
-    for (int w = 1; w < NW; w++) t += part[w][lane];
+    for (int w = 1; w < NW; w++) t += lds.part[w][lane];
 #pragma unroll
     for (int r = 0; r < 4; r++) t[r] = tanhf_(t[r]);
     *reinterpret_cast<bf16x4*>(in.mid + (long)row * MID + 16 * ob + 4 * L.g) = to_bf16(t);
@@ -738,12 +784,12 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
     auto c = [](const void* q) { return static_cast<const __bf16*>(q); };
     const MixIn mix{c(x), c(x_prev), c(mw.time_maa_w2), c(mw.time_maa), mid, rows, T};
 
-    // (one round of loads for four wavefronts up to 768 channels; beyond, sixteen: 2048 channels 9.3 -> 6.5 us)
+    // (one round of loads for four wavefronts up to 768 channels; beyond, sixteen: 2048 channels, one sequence, 9.3 -> 6.5 us)
     if (C <= 768)
-        hipLaunchKernelGGL((decode_mid_kernel<4, 6>), dim3(MID / 16, ntiles), dim3(256), 0, stream, mix, C, c(mw.time_maa_x),
+        hipLaunchKernelGGL((decode_mid_kernel<4, 3>), dim3(MID / 16, ntiles), dim3(256), 0, stream, mix, C, c(mw.time_maa_x),
                            c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
     else
-        hipLaunchKernelGGL((decode_mid_kernel<16, 4>), dim3(MID / 16, ntiles), dim3(1024), 0, stream, mix, C, c(mw.time_maa_x),
+        hipLaunchKernelGGL((decode_mid_kernel<16, 2>), dim3(MID / 16, ntiles), dim3(1024), 0, stream, mix, C, c(mw.time_maa_x),
                            c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
     {
         LinArgs a{};
