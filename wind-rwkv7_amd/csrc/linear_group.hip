@@ -10,8 +10,8 @@
 //
 // Both operands lie with the contraction index fastest, so a tile goes from memory to LDS without passing registers
 // (buffer_load ... lds) and from LDS into v_mfma_f32_32x32x16_bf16 as it lies: eight consecutive k of one row per lane and
-// 16-byte read.  The pieces of 16 bytes of a row are permuted by the row number on the way into LDS (by choosing which
-// piece a lane fetches), which makes those reads free of bank conflicts.  A block of four wavefronts (2 x 2) computes
+// 16-byte read.  The pieces of 16 bytes of a row are permuted by the number of its pair of rows on the way into LDS (by choosing
+// which piece a lane fetches), which keeps those reads out of each other's banks.  A block of four wavefronts (2 x 2) computes
 // 64 TMB tokens x 64 TNB columns; what bounds it is the LDS read rate against the matrix rate: 32 x 32 blocks TMB x TNB
 // per wavefront need TMB + TNB reads of 1 KB for TMB TNB instructions of 32 cycles.  Two blocks share a compute unit, so
 // one's matrix work covers the other's barriers and last loads.

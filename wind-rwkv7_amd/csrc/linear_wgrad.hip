@@ -249,7 +249,7 @@ __device__ __forceinline__ void wgrad_block(WgradLds<S>& lds, const WgradArgs& g
             // Rounds in which everything staged and fetched is a whole step.  The masks, selects and pointer choices of the other
             // rounds are half of their 143 instructions a step, and with one wavefront per SIMD nothing hides them: the
             // gradients of a 768-channel block's nine products, 8192 tokens, 77.6 -> 69.6 us (18 matrix instructions of 32 cycles
-            // a step of 1440; 4 row pitches of other bank offsets, 32 bytes or 64, 69.4).
+            // a step of 1440).  Row pitches with other bank offsets, 32 or 64 bytes, change nothing (69.4).
             const __bf16 *a_step = a_first + (long)(2 + DEPTH) * STEP * g.lda, *b_step = b_first + (long)(2 + DEPTH) * STEP * g.ldb;
             for (; base + 2 * DEPTH + 1 < nfull; base += DEPTH) {
 #pragma unroll
