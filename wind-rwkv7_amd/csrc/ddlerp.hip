@@ -10,7 +10,7 @@
 // The work is bandwidth-bound (x in, four streams out), but its inner products (C x 4D and 4D x C per
 // token) only stay off the critical path on the matrix cores, so every contraction is a 16x16x32 MFMA on
 // fragments (see frag.hpp): token tiles of 16 rows, channel blocks of 64.
-#include "frag.hpp"
+#include "row_lines.hpp"
 #include "device_info.hpp"
 #include "ddlerp_kernels.hpp"
 #include <type_traits>

@@ -15,7 +15,7 @@ constexpr int REC = 4 * HEAD * D + 4 * HEAD;   // floats of a partial record: dW
 // ------------------------------------------------------------------------------------------------
 // forward: block = (head, range of token tiles).  The head's weights and biases are staged in LDS once and each wavefront
 // walks its tiles with the next tile's inputs already in flight; tiles move as whole lines through the wavefront's part of LDS
-// (see ddlerp.hip: 16 rows per instruction cost 28 ns of a compute unit's time, whole lines 9 and, stored, 20).
+// (row_lines.hpp).
 // 16 rows per instruction and two rounds of two blocks per compute unit took 20.9, 22.1, 47 us at 7056, 8192, 16384 tokens x 768
 // channels, 49.5 at 8192 x 1536; whole lines and three blocks per compute unit in one round 16.9, 17.9, 35.9, 36.4 (two rounds of
 // either two or three: 18.9 and 19.6 at 7056).  The bytes are 13, 15, 30, 30 at the rate of a copy, the instructions, a fifth of

@@ -1,6 +1,6 @@
 // What the expand_loras kernels of both files share: operands, activations, fragments.
 #pragma once
-#include "frag.hpp"
+#include "row_lines.hpp"
 #include "expand_loras_kernels.hpp"
 
 namespace wkv {

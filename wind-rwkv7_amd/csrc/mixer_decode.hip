@@ -23,7 +23,7 @@
 
 #include "device_info.hpp"
 #include "linear_kernels.hpp"
-#include "frag.hpp"
+#include "row_lines.hpp"
 #include "ln_epilogue.hpp"
 #include "wkv7_common.hpp"
 
