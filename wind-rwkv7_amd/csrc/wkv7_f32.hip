@@ -566,16 +566,20 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
 // never divided by: the range of w stays the recurrence's), and likewise backwards, so
 //     dq_j = D(0..j) S^T dy_j + sum_{i<=j} D(i+1..j) ((sa_i.dy_j) b_i + (v_i.dy_j) k_i)       da_j: dsa_j, decays up to j - 1
 //     dk_i = D(i+1..15) E^T v_i + sum_{j>=i} D(i+1..j) (v_i.dy_j) q_j + sum_{j>i} D(i+1..j-1) (v_i.dsa_j) a_j       db_i: sa_i
-// each of them a Horner scheme in the decays: twelve multiply-adds per column and pair i <= j instead of thirteen per column,
-// token and ROW of the state.  With W_t the sum of all terms, times their own q, a, b or k, whose decays contain token t,
-//     dw_t = -exp(w_t) W_t,   W_t = M_t - a_t da_t,   M_{t+1} = W_t + b_t db_t + k_t dk_t - q_t dq_t.
+// each of them a Horner scheme in the decays: fifteen multiply-adds per column and pair i <= j instead of thirteen per column,
+// token and ROW of the state.  The gradient of a decay, R_t = sum over rows of dS_t * S_{t-1} and dw_t = -exp(w_t) decay_t R_t,
+// is two more such schemes: z = sum over rows of S * E, then down the tokens + q xq (R_t so far), * decay, + a xa with xq, xa =
+// S^T [dy dsa] for the terms of S, times D(0..t-1); and dk_i, db_i as their own schemes have them at token t, times k_i, b_i and
+// D(i+1..t-1).  (W_t = decay_t R_t is also what is left of W_{t-1} after four terms have come and gone, three multiply-adds less,
+// but the terms do not carry decay_t: from w = 3.3 on, the difference is rounding, 2e-4 of it there and all of it at 4.)
 // What needs the rows of the states - S^T [dy dsa], E^T [v sa], the sums of S * E for M_0 and the four 16 x 16 products of row
 // vectors - is one pass of matrix instructions over them.  All of it in fp64, whose multiply-add is as fast as fp32's here and
 // whose matrix instruction takes twice as long: a sum over rows averages the roundings of its terms, a sum of the terms'
 // sums does not, and in fp32 the errors would be 1.7e-7 where recomputing the states row by row left 0.9e-7.
-// Bound: memory, 90 KB per chunk and 64 columns: 8 x 1024 tokens x 12 heads of 64 142 us for 553 MB (without the matrix
-// instructions 123, without the pairs of tokens 132, without either 118), where recomputing the states took 221; 32 x 1024 x 12
-// 848 -> 529, 8 x 1024 x 6 heads of 128 473 -> 211, 8 x 1024 x 16 heads of 32 157 -> 92.
+// Bound: memory, 90 KB per chunk and 64 columns: 8 x 1024 tokens x 12 heads of 64 152 us for 553 MB (148 with dw as that
+// difference, and then 123/142 of it without the matrix instructions, 132 without the pairs of tokens, 118 without either),
+// where recomputing the states took 218; 32 x 1024 x 12 852 -> 560, 8 x 1024 x 6 heads of 128 477 -> 221, 8 x 1024 x 16 heads
+// of 32 157 -> 101.  Errors at 8 x 1024 x 12 against fp64: dq, dk 0.42e-7, dw 0.64e-7 (0.69 as a difference), da, db 0.98e-7.
 template <int CR, int COLS>   // head size, columns of a block
 __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w, const float* __restrict__ q,
                                                                const float* __restrict__ k, const float* __restrict__ v,
@@ -694,19 +698,13 @@ __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, con
         }
         __syncthreads();
     }
-    double dec[CH], qv[CH], av[CH], dqv[CH], dav[CH];
-    double P = 1., M = 0.;
+    double qv[CH], av[CH], dqv[CH], dav[CH], R[CH];
+    float dec[CH];   // (to fp64 where it is used: sixteen double decays would not fit the registers)
 #pragma unroll
     for (int t = 0; t < CH; t++) {
         const float ew = expf(cw[t]);
         es[t][lane] = ew, dec[t] = expf(-ew);
-        qv[t] = cq[t], av[t] = ca[t];
-        dqv[t] = xqv[t], dav[t] = xav[t];
-        M += av[t] * (P * dav[t]);
-        P *= dec[t];
-        M += qv[t] * (P * dqv[t]);
     }
-    M += P * z;
     // the pairs i <= j, i upwards and j downwards; the products of row vectors are read AHEAD pairs early
     constexpr int AHEAD = 1;
     d4 ahead[AHEAD];
@@ -720,28 +718,36 @@ __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, con
     for (int x = 0; x < AHEAD; x++) read_next(ahead[x]);
 #pragma unroll
     for (int i = 0; i < CH; i++) {
-        const double bi = cb[i], ki = ck[i];
+        asm volatile("" : "+v"(cb[i]), "+v"(ck[i]));   // (fp32 until now)
+        const double bi = cb[i], ki = ck[i], deci = dec[i];
         double dki = ys[0][i][lane], dbi = ys[1][i][lane];
 #pragma unroll
         for (int j = CH - 1; j >= i; j--) {
             const d4 m = ahead[slot];
             read_next(ahead[slot]);
             slot = (slot + 1) % AHEAD;
-            dqv[j] = dqv[j] * dec[i] + (m[G_SY] * bi + m[G_VY] * ki);
+            const double decj = dec[j];
+            if (i == 0) {   // the terms of the entering state: tokens downwards, as this first round of pairs goes
+                asm volatile("" : "+v"(cq[j]), "+v"(ca[j]), "+v"(xqv[j]), "+v"(xav[j]));   // (fp32 until now)
+                qv[j] = cq[j], av[j] = ca[j], dqv[j] = xqv[j], dav[j] = xav[j];
+                R[j] = z + qv[j] * dqv[j];
+                z = R[j] * decj + av[j] * dav[j];
+            }
+            dqv[j] = dqv[j] * deci + (m[G_SY] * bi + m[G_VY] * ki);
             dki += m[G_VY] * qv[j], dbi += m[G_SY] * qv[j];
             if (j > i) {
-                dav[j] = dav[j] * dec[i] + (m[G_SD] * bi + m[G_VD] * ki);
-                dki = dki * dec[j] + m[G_VD] * av[j], dbi = dbi * dec[j] + m[G_SD] * av[j];
+                R[j] = R[j] * deci + (ki * dki + bi * dbi);
+                dav[j] = dav[j] * deci + (m[G_SD] * bi + m[G_VD] * ki);
+                dki = dki * decj + m[G_VD] * av[j], dbi = dbi * decj + m[G_SD] * av[j];
             }
-            asm volatile("" : "+v"(dqv[j]), "+v"(dav[j]), "+v"(dki), "+v"(dbi) : : "memory");   // (else every pair's operands are in registers at once)
+            asm volatile("" : "+v"(dqv[j]), "+v"(dav[j]), "+v"(dki), "+v"(dbi), "+v"(R[j]), "+v"(dec[j]) : : "memory");   // (else every pair's operands are in registers at once)
         }
-        const double W = M - av[i] * dav[i];
-        M = W + (bi * dbi + ki * dki) - qv[i] * dqv[i];
         if (col_ok) {
             const long at = base + (long)i * ld;
             at_bytes<float>(dq + at, lane_col) = (float)dqv[i], at_bytes<float>(da + at, lane_col) = (float)dav[i];
             at_bytes<float>(dk + at, lane_col) = (float)dki, at_bytes<float>(db + at, lane_col) = (float)dbi;
-            at_bytes<float>(dw + at, lane_col) = -es[i][lane] * (dec[i] > 0. ? (float)W : 0.f);   // (W is a difference: not left to cancel)
+            const double ew = dec[i] > 0.f ? es[i][lane] : 0.f;   // (exp(w) may be infinite where the decay is zero)
+            at_bytes<float>(dw + at, lane_col) = (float)(-ew * deci * R[i]);
         }
     }
 }
