@@ -154,6 +154,22 @@ def test_f32_strong_decays(c_oracle, C, w):
         assert float(got.abs().max()) == 0.
 
 
+@pytest.mark.parametrize('C', [16, 32, 48, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize('blocks', [40, 600, 1100])
+def test_f32_gradients_of_few_and_many_chunks(c_oracle, blocks, C):
+    """The gradient kernels by blocks of one chunk and 32 columns: four wavefronts each, up to two blocks per compute unit (512);
+    one, up to one per SIMD (1024); 64 columns a wavefront (32 where a head has no more)."""
+    T, H = 32, 8
+    per = T // 16 * H * ((C + 31) // 32)
+    B = (blocks + per - 1) // per
+    d = inputs.wkv7_inputs(B, T, H, C, seed=500 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
+    g_ref = c_oracle.backward(*[d[n] for n in 'qwkvab'], d['s0'], d['dy'], d['dsT'])
+    ref = dict(zip(['dq', 'dw', 'dk', 'dv', 'da', 'db', 'ds0'], g_ref))
+    _, _, grads, _ = _run(d, B, T, H, C, True)
+    for n, g in zip(NAMES, grads):
+        assert seq_ref.rel_err(g.cpu(), ref['d' + n]) <= TOL, n
+
+
 @pytest.mark.parametrize('B,T,H,C', [(1, 48, 2, 64), (1, 32, 2, 128), (2, 48, 3, 16), (4, 512, 8, 64), (3, 512, 4, 128)])
 @pytest.mark.parametrize('w', [-1.0, 3.0, 3.5, 4.0])
 def test_f32_decay_gradient_where_every_decay_is_strong(c_oracle, B, T, H, C, w):
@@ -168,13 +184,21 @@ def test_f32_decay_gradient_where_every_decay_is_strong(c_oracle, B, T, H, C, w)
         assert seq_ref.rel_err(g.cpu(), ref['d' + n]) <= TOL, n
 
 
-@pytest.mark.parametrize('C', [64, 128])
-def test_f32_gradients_of_later_tokens_do_not_see_a_non_finite_dy(C):
+# blocks of 32 columns: 6 and 12, up to two per compute unit; 576, between two and four; 1088 and 1536, more (64 columns where a
+# head has them)
+@pytest.mark.parametrize('B,T,H,C', [(1, 48, 2, 64), (1, 48, 2, 128), (4, 48, 24, 64), (6, 48, 8, 128), (8, 48, 24, 64), (12, 48, 32, 48),
+                                     (10, 48, 40, 32)])
+def test_f32_gradients_of_later_tokens_do_not_see_a_non_finite_dy(B, T, H, C):
     """The gradients of a token depend on its own and later dy: an infinity in one token's dy leaves those of the tokens
-    after it, in the same chunk too, the same bits."""
-    B, T, H, at = 1, 48, 2, 21
+    after it, in the same chunk too, the same bits.  Likewise one in a k leaves dw, da and db of the tokens up to its own."""
+    at = 21
     d = inputs.wkv7_inputs(B, T, H, C, seed=440 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
     clean = _run(d, B, T, H, C, True)[2]
+    e = dict(d, k=d['k'].clone())
+    e['k'][0, at, 1, 7] = float('inf')
+    for n, g, h in zip(NAMES, _run(e, B, T, H, C, True)[2], clean):
+        if n in 'wab':
+            assert torch.equal(g[:, :at + 1], h[:, :at + 1]), n
     d['dy'] = d['dy'].clone()
     d['dy'][0, at, 1, 7] = float('inf')
     for n, g, h in zip(NAMES, _run(d, B, T, H, C, True)[2], clean):

@@ -572,13 +572,13 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
 // S^T [dy dsa] for the terms of S, times D(0..t-1); and dk_i, db_i as their own schemes have them at token t, times k_i, b_i and
 // D(i+1..t-1).  (W_t = decay_t R_t is also what is left of W_{t-1} after four terms have come and gone, three multiply-adds less,
 // but the terms do not carry decay_t: from w = 3.3 on, the difference is rounding, 2e-4 of it there and all of it at 4.)
-// What needs the rows of the states - S^T [dy dsa], E^T [v sa], the sums of S * E for M_0 and the four 16 x 16 products of row
+// What needs the rows of the states - S^T [dy dsa], E^T [v sa], the sums of S * E and the four 16 x 16 products of row
 // vectors - is one pass of matrix instructions over them.  All of it in fp64, whose multiply-add is as fast as fp32's here and
 // whose matrix instruction takes twice as long: a sum over rows averages the roundings of its terms, a sum of the terms'
 // sums does not, and in fp32 the errors would be 1.7e-7 where recomputing the states row by row left 0.9e-7.
 // Bound: memory, 90 KB per chunk and 64 columns: 8 x 1024 tokens x 12 heads of 64 152 us for 553 MB (148 with dw as that
-// difference, and then 123/142 of it without the matrix instructions, 132 without the pairs of tokens, 118 without either),
-// where recomputing the states took 218; 32 x 1024 x 12 852 -> 560, 8 x 1024 x 6 heads of 128 477 -> 221, 8 x 1024 x 16 heads
+// difference; of 142 on another machine, 123 without the matrix instructions, 132 without the pairs of tokens, 118 without
+// either), where recomputing the states took 218; 32 x 1024 x 12 852 -> 560, 8 x 1024 x 6 heads of 128 477 -> 221, 8 x 1024 x 16 heads
 // of 32 157 -> 101.  Errors at 8 x 1024 x 12 against fp64: dq, dk 0.42e-7, dw 0.64e-7 (0.69 as a difference), da, db 0.98e-7.
 template <int CR, int COLS>   // head size, columns of a block
 __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w, const float* __restrict__ q,
@@ -752,6 +752,191 @@ __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, con
     }
 }
 
+// The same gradients where the chunks are too few to fill the chip: four wavefronts to a chunk and 32 of its columns, which share
+// what one does one after the other above.  Bound: that chain, not memory (64 channels, 64 chunks: 11.5 us, of which the pairs 5.7
+// and the products 2.5; one wavefront 17.4; the recurrence's states recomputed row by row took 11.2, with twice the error in dq).
+//   A wavefront makes three of the twelve products (S or E times a token vector, and one of the four without a state);
+//   the 256 threads share the exponentials and the sums of S * E;
+//   the pairs are two wavefronts: dq and da, which need the products of row vectors only, and dk, db and dw;
+//   in both, the halves of a wavefront are two gradients of the same columns: lanes 0-31 dq | dk, lanes 32-63 da | db.
+// In fp64, and sums over rows in the same order as above.  (The pairs as loops over four i, a quarter of the instructions: 12.2 us;
+// the pairs' two wavefronts on other SIMDs for every second block: no gain where two blocks share a compute unit.)
+template <int CR>
+__global__ __launch_bounds__(256, 2) void wkv7_f32_grads_few_kernel(int T, int H, const float* __restrict__ w, const float* __restrict__ q,
+                                                                    const float* __restrict__ k, const float* __restrict__ v,
+                                                                    const float* __restrict__ a, const float* __restrict__ b,
+                                                                    const float* __restrict__ dy, const float* __restrict__ ckpt,
+                                                                    const float* __restrict__ work, float* __restrict__ dw,
+                                                                    float* __restrict__ dq, float* __restrict__ dk,
+                                                                    float* __restrict__ da, float* __restrict__ db) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    constexpr int CH = CH64, COLS = 32, STEPS = CR / 16, PAIRS = CH * (CH + 1) / 2;
+    __shared__ float prod[4][CH][COLS];                                       // S^T dy, S^T dsa, E^T v, E^T sa
+    __shared__ __attribute__((aligned(16))) double gx[PAIRS][4], gy[PAIRS][4];   // of tokens i <= j: sa.dy, v.dy | sa.dsa, v.dsa and v.dy, v.dsa | sa.dy, sa.dsa
+    __shared__ float es[CH][COLS], ds[CH][COLS];
+    __shared__ double zs[8][COLS];
+    auto pair = [](int i, int j) { return i * CH - i * (i - 1) / 2 + j - i; };
+    const int NC = T / CH, bh = blockIdx.x / NC, chunk = blockIdx.x - bh * NC, h = bh % H;
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int cl = lane % COLS, col0 = COLS * blockIdx.y;                     // (tid % COLS is the same column)
+    const bool upper = lane >= COLS, col_ok = CR % COLS == 0 || col0 + cl < CR;
+    const long base = seq_index((long)(bh / H) * T + (long)chunk * CH, H, h, 0, CR);
+    const unsigned ld = (unsigned)H * CR, lane_col = 4 * (col_ok ? col0 + cl : 0);   // (past the columns: column 0, nothing written)
+    const long nstate = saved_states(gridDim.x / NC, T, CR), st = (long)blockIdx.x * CR * CR;
+    const float *const sa = ckpt + nstate, *const dsa = work + nstate;
+
+    // what is read is asked for before anything waits (of the states and row vectors, four steps of 16 rows)
+    const float* const left = wv == 0 || wv == 3 ? sa : v;                    // the product of row vectors: sa.dy, v.dsa, v.dy, sa.dsa
+    const float* const right = wv == 0 || wv == 2 ? dy : dsa;
+    const float* const state = wv < 2 ? ckpt : work;                          // S with the right one, E with the left one
+    constexpr int EARLY = STEPS < 4 ? STEPS : 4;
+    f4 lrow[EARLY], rrow[EARLY];
+    f2 srow[EARLY][4];
+    const int c = col0 + 2 * n;
+    const unsigned row_at = 4 * ((unsigned)n * ld + 4 * g), state_at = 4 * (4 * g * CR + (CR % COLS == 0 || c < CR ? c : 0));
+    auto fetch = [&](int u) {
+        lrow[u % EARLY] = at_bytes<f4>(left + (base + 16 * u), row_at), rrow[u % EARLY] = at_bytes<f4>(right + (base + 16 * u), row_at);
+#pragma unroll
+        for (int s = 0; s < 4; s++) srow[u % EARLY][s] = at_bytes<f2>(state + (st + (16 * u + s) * CR), state_at);
+    };
+#pragma unroll
+    for (int u = 0; u < EARLY; u++) fetch(u);
+    float cw[CH / 8], zS[CR / 8], zE[CR / 8];                                 // eight tokens and eight rows by thread group
+    const unsigned group = tid / COLS;
+#pragma unroll
+    for (int m = 0; m < CH / 8; m++) cw[m] = at_bytes<float>(w + (base + (long)(8 * m) * ld), 4 * group * ld + lane_col);
+#pragma unroll
+    for (int m = 0; m < CR / 8; m++) {
+        zS[m] = at_bytes<float>(ckpt + (st + 8 * m * CR), 4 * group * CR + lane_col);
+        zE[m] = at_bytes<float>(work + (st + 8 * m * CR), 4 * group * CR + lane_col);
+    }
+    float x0[CH], x1[CH], x2[CH];                                             // wavefront 0: b, k; wavefront 1: q, a, and k | b
+    if (wv < 2) {
+        const float *const p0 = wv == 0 ? b : q, *const p1 = wv == 0 ? k : a, *const p2 = upper ? b : k;
+#pragma unroll
+        for (int t = 0; t < CH; t++) {
+            const long at = base + (long)t * ld;
+            x0[t] = at_bytes<float>(p0 + at, lane_col), x1[t] = at_bytes<float>(p1 + at, lane_col);
+            if (wv == 1) x2[t] = at_bytes<float>(p2 + at, lane_col);
+        }
+    }
+    {
+        double z = 0.;
+#pragma unroll
+        for (int m = 0; m < CR / 8; m++) z += (double)zS[m] * zE[m];
+        zs[group][cl] = z;
+#pragma unroll
+        for (int m = 0; m < CH / 8; m++) {
+            const float ew = expf(cw[m]);
+            es[8 * m + group][cl] = ew, ds[8 * m + group][cl] = expf(-ew);
+        }
+        auto mma = [](double x, double y, d4 acc) { return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc, 0, 0, 0); };
+        d4 gr = {}, x[2] = {};
+#pragma unroll
+        for (int u = 0; u < STEPS; u++) {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const double l = lrow[u % EARLY][s], r = rrow[u % EARLY][s], own = wv < 2 ? r : l;
+                gr = mma(l, r, gr);
+                x[0] = mma(own, srow[u % EARLY][s][0], x[0]), x[1] = mma(own, srow[u % EARLY][s][1], x[1]);
+            }
+            if (u + EARLY < STEPS) fetch(u + EARLY);
+        }
+        const int to_x = wv == 0 ? 0 : wv == 1 ? 3 : wv == 2 ? 1 : 2, to_y = wv == 0 ? 2 : wv == 1 ? 1 : wv == 2 ? 0 : 3;
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const int i = 4 * m + g;
+            *reinterpret_cast<f2*>(&prod[wv][i][2 * n]) = f2{(float)x[0][m], (float)x[1][m]};
+            if (i <= n) {
+                gx[pair(i, n)][to_x] = gr[m], gy[pair(i, n)][to_y] = gr[m];
+            }
+        }
+    }
+    __syncthreads();
+    if (wv >= 2) return;
+    // the products of the pairs are read AHEAD pairs early (eight of them spill)
+    constexpr int AHEAD = 4;
+    d2 ahead[AHEAD];
+    const double(*const gram)[4] = wv == 0 ? gx : gy;
+    int ni = 0, nj = CH - 1, slot = 0;   // (all known at compile time once the loops are unrolled)
+    auto read_next = [&](d2& m) {
+        if (ni < CH) m = *reinterpret_cast<const d2*>(&gram[pair(ni, nj)][2 * upper]);
+        if (nj > ni) nj--;
+        else ni++, nj = CH - 1;
+    };
+    auto next = [&] {
+        const d2 m = ahead[slot];
+        read_next(ahead[slot]);
+        slot = (slot + 1) % AHEAD;
+        return m;
+    };
+#pragma unroll
+    for (int x = 0; x < AHEAD; x++) read_next(ahead[x]);
+    double dec[CH];
+#pragma unroll
+    for (int t = 0; t < CH; t++) dec[t] = ds[t][cl];
+    if (wv == 0) {
+        float* const to = upper ? da : dq;
+        double x[CH];
+#pragma unroll
+        for (int t = 0; t < CH; t++) x[t] = prod[upper][t][cl];
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            const double bi = x0[i], ki = x1[i];
+#pragma unroll
+            for (int j = CH - 1; j >= i; j--) {
+                const d2 m = next();
+                const double more = x[j] * dec[i] + (m[0] * bi + m[1] * ki);
+                x[j] = i == j && upper ? x[j] : more;           // (da_j: tokens before j only)
+                asm volatile("" : "+v"(x[j]) : : "memory");   // (in this order, as above)
+            }
+            if (col_ok) at_bytes<float>(to + (base + (long)i * ld), lane_col) = (float)x[i];
+        }
+    } else {
+        float* const to = upper ? db : dk;
+        double R[CH], qv[CH], av[CH], z = 0.;
+#pragma unroll
+        for (int m = 0; m < 8; m++) z += zs[m][cl];
+#pragma unroll
+        for (int t = CH - 1; t >= 0; t--) {
+            qv[t] = x0[t], av[t] = x1[t];
+            R[t] = z + qv[t] * prod[0][t][cl];
+            z = R[t] * dec[t] + av[t] * prod[1][t][cl];
+            R[t] = upper ? 0. : R[t];
+        }
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            const double ci = x2[i];
+            double y = prod[2 + upper][i][cl];
+#pragma unroll
+            for (int j = CH - 1; j >= i; j--) {
+                const d2 m = next();
+                const double yq = m[0] * qv[j];
+                if (j > i) {   // (y waits for one multiply-add a pair)
+                    R[j] = R[j] * dec[i] + ci * (y + yq);
+                    y = y * dec[j] + (yq * dec[j] + m[1] * av[j]);
+                } else {
+                    y += yq;
+                }
+                asm volatile("" : "+v"(y), "+v"(R[j]) : : "memory");
+            }
+            if (col_ok) at_bytes<float>(to + (base + (long)i * ld), lane_col) = (float)y;
+        }
+#pragma unroll
+        for (int t = 0; t < CH; t++) {
+            // lanes 0-31: the other half of the sum
+            const unsigned long long bits = __builtin_bit_cast(unsigned long long, R[t]);
+            const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)bits, (unsigned)bits, false, false);
+            const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(bits >> 32), (unsigned)(bits >> 32), false, false);
+            const double Rt = R[t] + __builtin_bit_cast(double, (unsigned long long)hi[1] << 32 | lo[1]);
+            const float ew = es[t][cl];
+            if (col_ok && !upper) at_bytes<float>(dw + (base + (long)t * ld), lane_col) = (float)((dec[t] > 0. ? -ew : 0.f) * dec[t] * Rt);
+        }
+    }
+}
+
 // five tensors of n floats each to zero (what the two-blocks-per-head backward adds its parts onto)
 __global__ __launch_bounds__(256) void zero5_kernel(long n4, f4* __restrict__ p0, f4* __restrict__ p1, f4* __restrict__ p2,
                                                     f4* __restrict__ p3, f4* __restrict__ p4) {
@@ -824,24 +1009,28 @@ void launch_wkv7_f32_backward_split(int B, int T, int H, int C, const float* w, 
                                     float* work, float* dw, float* dq, float* dk, float* dv, float* da, float* db, float* ds0,
                                     hipStream_t stream) {
     launch_scan<true>(B, T, H, C, w, q, k, dy, a, b, dsT, dv, work, ds0, stream);
-    // 64 columns a wavefront; 32 where a head has no more, and while the wavefronts are few enough for the wait for the matrix
-    // instructions of half as many columns to count for more than half the lanes idling: up to one wavefront per SIMD (us in
-    // 64 / 32 columns, 64 channels: 64 chunks 20.3/16.5, 256 24.1/22.2, 512 28.7/29.1; 128 channels, 8 chunks 30.7/23.7)
-    const bool narrow = C <= 32 || (long)B * H * (T / CH64) * ((C + 31) / 32) <= 4 * compute_units();
-    auto go = [&](auto kernel, auto narrow_kernel) {
-        const int cols = narrow ? 32 : 64;
-        hipLaunchKernelGGL(narrow ? narrow_kernel : kernel, dim3(B * H * (T / CH64), (C + cols - 1) / cols), dim3(64), 0, stream, T, H, w, q, k,
-                           v, a, b, dy, ckpt, work, dw, dq, dk, da, db);
+    // Blocks of 32 columns, four wavefronts each, while all of them run at once (two to a compute unit, by registers); then a
+    // wavefront on 32 columns, up to one per SIMD, where the wait for the matrix instructions of half as many columns counts for
+    // more than half the lanes idling; then one on 64.  us in the three forms:
+    //   64 channels     64 chunks 11.5, 17.3, 21.6    256 16.8, 19.5, 23.0    320 28.5, 20.4, 24.1    512 31.8, 23.0, 25.7    640 44.2, 33.3, 26.9
+    //   128 channels    64 chunks 16.2, 24.3, 32.9    128 20.5, 25.7, 33.7    160 33.6, 26.6, 34.8    256 39.6, 29.4, 36.6    320 52.4, 45.0, 37.7
+    //   32 channels     256 chunks 11.0, 14.9         512 15.3, 16.2          640 25.5, 17.0
+    const long blocks = (long)B * H * (T / CH64) * ((C + 31) / 32);
+    const bool few = blocks <= 2 * compute_units(), narrow = C <= 32 || blocks <= 4 * compute_units();
+    auto go = [&](auto kernel, auto narrow_kernel, auto few_kernel) {
+        const int cols = few || narrow ? 32 : 64;
+        hipLaunchKernelGGL(few ? few_kernel : narrow ? narrow_kernel : kernel, dim3(B * H * (T / CH64), (C + cols - 1) / cols),
+                           dim3(few ? 256 : 64), 0, stream, T, H, w, q, k, v, a, b, dy, ckpt, work, dw, dq, dk, da, db);
     };
     switch (C) {
-        case 16: go(wkv7_f32_grads_kernel<16, 32>, wkv7_f32_grads_kernel<16, 32>); break;
-        case 32: go(wkv7_f32_grads_kernel<32, 32>, wkv7_f32_grads_kernel<32, 32>); break;
-        case 48: go(wkv7_f32_grads_kernel<48, 64>, wkv7_f32_grads_kernel<48, 32>); break;
-        case 64: go(wkv7_f32_grads_kernel<64, 64>, wkv7_f32_grads_kernel<64, 32>); break;
-        case 80: go(wkv7_f32_grads_kernel<80, 64>, wkv7_f32_grads_kernel<80, 32>); break;
-        case 96: go(wkv7_f32_grads_kernel<96, 64>, wkv7_f32_grads_kernel<96, 32>); break;
-        case 112: go(wkv7_f32_grads_kernel<112, 64>, wkv7_f32_grads_kernel<112, 32>); break;
-        default: go(wkv7_f32_grads_kernel<128, 64>, wkv7_f32_grads_kernel<128, 32>);
+        case 16: go(wkv7_f32_grads_kernel<16, 32>, wkv7_f32_grads_kernel<16, 32>, wkv7_f32_grads_few_kernel<16>); break;
+        case 32: go(wkv7_f32_grads_kernel<32, 32>, wkv7_f32_grads_kernel<32, 32>, wkv7_f32_grads_few_kernel<32>); break;
+        case 48: go(wkv7_f32_grads_kernel<48, 64>, wkv7_f32_grads_kernel<48, 32>, wkv7_f32_grads_few_kernel<48>); break;
+        case 64: go(wkv7_f32_grads_kernel<64, 64>, wkv7_f32_grads_kernel<64, 32>, wkv7_f32_grads_few_kernel<64>); break;
+        case 80: go(wkv7_f32_grads_kernel<80, 64>, wkv7_f32_grads_kernel<80, 32>, wkv7_f32_grads_few_kernel<80>); break;
+        case 96: go(wkv7_f32_grads_kernel<96, 64>, wkv7_f32_grads_kernel<96, 32>, wkv7_f32_grads_few_kernel<96>); break;
+        case 112: go(wkv7_f32_grads_kernel<112, 64>, wkv7_f32_grads_kernel<112, 32>, wkv7_f32_grads_few_kernel<112>); break;
+        default: go(wkv7_f32_grads_kernel<128, 64>, wkv7_f32_grads_kernel<128, 32>, wkv7_f32_grads_few_kernel<128>);
     }
 }
 
