@@ -320,7 +320,8 @@ int wind_rwkv7_ddlerp_backward(int B, int T, int C, int D,
  * overwritten and summed in a fixed order (the reference uses atomics, :181-189, and sums the per-head
  * partials of the rank-space gradients on the host, :207-210).
  * Requires head_size a multiple of 16 that divides C (the reference passes it on, :72-79), C % 64 == 0,
- * T % 16 == 0, D in {16, 32, 64}.  The backward workspace size does not depend on the head size. */
+ * T % 16 == 0, D in {16, 32, 64}.  The backward workspace size does not depend on the head size.  At rank 16 the backward
+ * also takes a workspace with the records of half as many blocks (one per compute unit) and is slower with it. */
 int wind_rwkv7_expand_loras_rank_supported(int D);
 size_t wind_rwkv7_expand_loras_bwd_workspace_bytes(int B, int T, int C, int D);
 int wind_rwkv7_expand_loras_forward(int B, int T, int C, int D, int head_size,

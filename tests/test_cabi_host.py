@@ -208,6 +208,22 @@ def test_mixer_decode_sizes_and_validation_on_host():
     assert call() == 1
 
 
+@pytest.mark.parametrize('B,T,C,D', [(8, 1024, 768, 16), (1, 16, 64, 16), (3, 48, 64, 16), (25, 656, 64, 16), (2, 64, 2048, 16), (2, 64, 256, 32)])
+def test_expand_loras_backward_takes_records_of_one_block_per_compute_unit_on_host(B, T, C, D):
+    """A workspace with the shares of d*_in, the statistics of the smallest head size and records of one block per compute unit
+    (256 without a device; four tiles of 16 tokens each at least) is enough at every rank, also where more is asked for."""
+    lib = _native.lib()
+    M, H = B * T, C // 64
+    a256 = lambda x: (x + 255) // 256 * 256
+    splits = max(1, min(256 // H, M // 16 // 4))
+    least = 4 * a256(M * H * D * 2) + splits * H * (4 * 64 * D + 4 * 64) * 4 + a256(M * (C // 16) * 8)
+    assert lib.wind_rwkv7_expand_loras_bwd_workspace_bytes(B, T, C, D) >= least
+    # (a missing list of strides is found after the workspace, and before anything is enqueued)
+    call = lambda ws, size: lib.wind_rwkv7_expand_loras_backward_to(B, T, C, D, 64, *[0x1000] * 24, None, *[0x1000] * 8, ws, size, None)
+    assert call(0x2000, least) == 1
+    assert call(0x2000, least - 1) == 6 and call(None, least) == 6 and call(0x2010, least) == 6
+
+
 def test_f32_entry_points_validate_on_host():
     lib = _native.lib()
     # the fp32 state every 16 tokens and one float per token and channel

@@ -70,6 +70,36 @@ def test_expand_loras_parity_cfg4_shape():
     print('expand_loras cfg4 errors', {k: f'{v:.2e}' for k, v in errs.items()})
 
 
+@pytest.mark.parametrize('B,T,C,N', [(8, 1024, 768, 64), (25, 656, 64, 64), (3, 48, 192, 32)])
+def test_expand_loras_rank_16_with_fewer_records(B, T, C, N):
+    """The backward with a workspace of one block per compute unit (what it has to take), one record more, and all that is asked for: what
+    is summed within a tile is the same bits, the sums over the tokens differ in the order of at most M / 16 fp32 tile sums,
+    2^-24 sqrt(1025) = 2e-6 of them for the longest here."""
+    from wind_rwkv import _native
+    lib, D, M, H = _native.lib(), 16, B * T, C // 64
+    d = inputs.expand_loras_inputs(B, T, C, D, 33, dtype=torch.bfloat16)
+    ins, dys = [d[n].to(DEV) for n in NAMES], [g.to(DEV) for g in d['dy']]
+    a256 = lambda x: (x + 255) // 256 * 256
+    record = H * (4 * 64 * D + 4 * 64) * 4
+    splits = max(1, min(torch.cuda.get_device_properties(0).multi_processor_count // H, M // 16 // 4))
+    least = 4 * a256(M * H * D * 2) + splits * record + a256(M * (C // 16) * 8)
+    asked = lib.wind_rwkv7_expand_loras_bwd_workspace_bytes(B, T, C, D)
+    assert asked >= least + record
+    results = []
+    for size in (asked, least, least + record):
+        out = [torch.full_like(x, float('nan')) for x in ins[:6]] + [torch.full_like(x, float('nan'), dtype=torch.float32) for x in ins[6:]]
+        guard = 4096   # (behind the bytes named: not to be written)
+        ws = torch.full((size + guard,), 7, dtype=torch.uint8, device=DEV)
+        p = lambda ts: [t.data_ptr() for t in ts]
+        _native.check(lib.wind_rwkv7_expand_loras_backward(B, T, C, D, N, *p(ins), *p(dys), *p(out), ws.data_ptr(), size,
+                                                           torch.cuda.current_stream().cuda_stream))
+        assert bool((ws[size:] == 7).all())
+        results.append(out)
+    for fewer in results[1:]:
+        for i, (x, y) in enumerate(zip(results[0], fewer)):
+            assert torch.equal(x, y) if i < 6 else seq_ref.rel_err(y.cpu(), x.cpu()) <= 1e-5, i
+
+
 def test_expand_loras_output_invariants():
     from wind_rwkv.rwkv7 import expand_loras
     d = inputs.expand_loras_inputs(2, 32, 128, 16, 5, dtype=torch.bfloat16)

@@ -703,7 +703,7 @@ int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_siz
     for (int i = 0; i < 4; i++)
         if (!acts[i] || !Ws[i] || !biases[i] || !dys[i] || !dacts[i] || !dWs[i] || !dbiases[i])
             return WIND_RWKV7_ERR_NULL_POINTER;
-    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_expand_loras_bwd_workspace_bytes(B, T, C, D));
+    rc = check_workspace(workspace, workspace_bytes, wkv::expand_loras_bwd_workspace_least_bytes((long)B * T, C, D));
     if (rc) return rc;
     if (!ld_din) return WIND_RWKV7_ERR_NULL_POINTER;
     long ld[4];
@@ -712,7 +712,7 @@ int wind_rwkv7_expand_loras_backward_to(int B, int T, int C, int D, int head_siz
         ld[i] = (long)ld_din[i];
     }
     wkv::launch_expand_loras_backward((long)B * T, C, D, head_size, w_in, k_in, acts, Ws, biases, dys, dw_in, dk_in, dacts, ld, dWs,
-                                      dbiases, workspace, static_cast<hipStream_t>(stream));
+                                      dbiases, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

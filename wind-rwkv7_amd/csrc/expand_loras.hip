@@ -535,8 +535,7 @@ constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
 // Blocks of the backward kernel per head.  The kernel holds one block per compute unit (one wavefront per SIMD),
 // so the grid must fit ONE round of the MI355X's 256 compute units: rounding 256 / H up gave 264 blocks at 12
 // heads, a second round of 8 blocks and twice the run time.  At least four token tiles (one per wavefront) each.
-int loras_splits(long M, int H, int D) {
-    if (D == 16) return lora16_splits(M, H);
+int loras_splits(long M, int H) {
     const long ntiles = M / TOK;
     long s = compute_units() / H;
     if (s > ntiles / 4) s = ntiles / 4;
@@ -549,12 +548,18 @@ bool expand_loras_rank_supported(int D) { return D == 16 || D == 32 || D == 64; 
 bool expand_loras_head_size_supported(int C, int HS) { return HS >= 16 && HS % 16 == 0 && C % HS == 0; }
 
 // (the statistics of the smallest head size are always included: the size does not depend on the head size)
+static size_t workspace_without_records(long M, int C, int D) {
+    return A256((size_t)M * (C / HEAD) * D * 2) * 4 + A256((size_t)M * (C / 16) * sizeof(HeadStat));
+}
+static size_t records_bytes(int nsplit, int C, int D) { return (size_t)nsplit * (C / HEAD) * (4 * HEAD * D + 4 * HEAD) * 4; }   // (whole 256)
 size_t expand_loras_bwd_workspace_bytes(long M, int C, int D) {
     const int H = C / HEAD;
-    const size_t din = A256((size_t)M * H * D * 2) * 4;
-    const size_t partial = A256((size_t)loras_splits(M, H, D) * H * (4 * HEAD * D + 4 * HEAD) * 4);
-    const size_t stats = A256((size_t)M * (C / 16) * sizeof(HeadStat));
-    return din + partial + stats;
+    return workspace_without_records(M, C, D) + records_bytes(D == 16 ? lora16_splits(M, H) : loras_splits(M, H), C, D);
+}
+// At rank 16 two blocks fit a compute unit and the workspace asked for has a record for each; a caller may bring one with the
+// records of one block per compute unit, what every rank needs, and gets as many blocks as it has records for.
+size_t expand_loras_bwd_workspace_least_bytes(long M, int C, int D) {
+    return workspace_without_records(M, C, D) + records_bytes(loras_splits(M, C / HEAD), C, D);
 }
 
 void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
@@ -619,7 +624,7 @@ void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in,
 void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                   const void* const Ws[4], const void* const biases[4], const void* const dys[4],
                                   void* dw_in, void* dk_in, void* const dacts[4], const long ld_dacts[4], void* const dWs[4],
-                                  void* const dbiases[4], void* workspace, hipStream_t stream) {
+                                  void* const dbiases[4], void* workspace, size_t workspace_bytes, hipStream_t stream) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     auto m = [](void* p) { return static_cast<__bf16*>(p); };
     auto f = [](void* p) { return static_cast<float*>(p); };
@@ -634,8 +639,9 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
         p += A256((size_t)M * H * D * 2);
     }
     float* partial = reinterpret_cast<float*>(p);
-    const int nsplit = loras_splits(M, H, D);
-    p += A256((size_t)nsplit * H * (4 * HEAD * D + 4 * HEAD) * 4);
+    const size_t held = (workspace_bytes - workspace_without_records(M, C, D)) / records_bytes(1, C, D);   // (records of all heads)
+    const int wanted = D == 16 ? lora16_splits(M, H) : loras_splits(M, H), nsplit = held < (size_t)wanted ? (int)held : wanted;
+    p += records_bytes(nsplit, C, D);
     HeadStat* stats = reinterpret_cast<HeadStat*>(p);
     const int tiles_per_split = (int)((M / TOK + nsplit - 1) / nsplit);
     const dim3 grid(H, nsplit), block(256);
@@ -650,7 +656,7 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
                        nullptr, nullptr, nullptr, nullptr, dy.p[2], dy.p[3], stats)
         if (D == 16) {
             WKV_LAUNCH_STAT(1);
-            launch_loras16_backward(M, C, c(w_in), c(k_in), in, lw, dy, m(dw_in), m(dk_in), part.p[0], partial, stats, HS, stream);
+            launch_loras16_backward(M, C, c(w_in), c(k_in), in, lw, dy, m(dw_in), m(dk_in), part.p[0], partial, nsplit, stats, HS, stream);
         } else if (D == 32) {
             WKV_LAUNCH_STAT(2);
             WKV_LAUNCH_BWD(2, true);
@@ -659,7 +665,7 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
             WKV_LAUNCH_BWD(4, true);
         }
 #undef WKV_LAUNCH_STAT
-    } else if (D == 16) launch_loras16_backward(M, C, c(w_in), c(k_in), in, lw, dy, m(dw_in), m(dk_in), part.p[0], partial, nullptr, HS, stream);
+    } else if (D == 16) launch_loras16_backward(M, C, c(w_in), c(k_in), in, lw, dy, m(dw_in), m(dk_in), part.p[0], partial, nsplit, nullptr, HS, stream);
     else if (D == 32) WKV_LAUNCH_BWD(2, false);
     else WKV_LAUNCH_BWD(4, false);
 #undef WKV_LAUNCH_BWD
@@ -668,7 +674,7 @@ void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in
                             {f(dWs[0]), f(dWs[1]), f(dWs[2]), f(dWs[3])},
                             {f(dbiases[0]), f(dbiases[1]), f(dbiases[2]), f(dbiases[3])}};
     if (D == 16) {
-        launch_loras16_reduce(M, C, part.p[0], partial, out, stream);
+        launch_loras16_reduce(M, C, nsplit, part.p[0], partial, out, stream);
         return;
     }
     const int rec = 4 * HEAD * D + 4 * HEAD, param_blocks = (rec + 255) / 256;

@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void expand_loras_reduce16_kernel(long M, int 
 // host side
 // ------------------------------------------------------------------------------------------------
 // Blocks of the backward kernel per head: two fit a compute unit, all of them in one round, at least one tile per pair of
-// wavefronts each.
+// wavefronts each (fewer where the workspace has fewer records).
 int lora16_splits(long M, int H) {
     const long ntiles = M / TOK;
     long s = 2 * compute_units() / H;
@@ -516,9 +516,9 @@ void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_i
 }
 
 void launch_loras16_backward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, const LoraDy& dy,
-                             __bf16* dw_in, __bf16* dk_in, __bf16* din, float* partial, const HeadStat* stats, int HS,
+                             __bf16* dw_in, __bf16* dk_in, __bf16* din, float* partial, int nsplit, const HeadStat* stats, int HS,
                              hipStream_t stream) {
-    const int H = C / HEAD, nsplit = lora16_splits(M, H);
+    const int H = C / HEAD;
     const int tiles_per_split = (int)((M / TOK + nsplit - 1) / nsplit);
     const dim3 grid(H, nsplit), block(256);
     if (stats)
@@ -529,10 +529,10 @@ void launch_loras16_backward(long M, int C, const __bf16* w_in, const __bf16* k_
                            dk_in, din, partial, stats, HS);
 }
 
-void launch_loras16_reduce(long M, int C, const __bf16* din, const float* partial, const LoraReduceOut& out, hipStream_t stream) {
+void launch_loras16_reduce(long M, int C, int nsplit, const __bf16* din, const float* partial, const LoraReduceOut& out, hipStream_t stream) {
     static_assert(REC % (4 * REDUCE_COLS) == 0, "whole blocks");
     const int H = C / HEAD, din_blocks = (int)(M / 8), param_blocks = REC / (4 * REDUCE_COLS);
-    hipLaunchKernelGGL(expand_loras_reduce16_kernel, dim3(din_blocks + param_blocks * H), dim3(256), 0, stream, M, H, lora16_splits(M, H),
+    hipLaunchKernelGGL(expand_loras_reduce16_kernel, dim3(din_blocks + param_blocks * H), dim3(256), 0, stream, M, H, nsplit,
                        din_blocks, param_blocks, din, partial, out);
 }
 

@@ -11,6 +11,7 @@ namespace wkv {
 bool expand_loras_rank_supported(int D);
 bool expand_loras_head_size_supported(int C, int HS);
 size_t expand_loras_bwd_workspace_bytes(long M, int C, int D);
+size_t expand_loras_bwd_workspace_least_bytes(long M, int C, int D);   // (what the backward still runs with)
 // outs: w_out, k_out, kk_out, b_out [M, C]
 void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                  const void* const Ws[4], const void* const biases[4], void* const outs[4],
@@ -19,6 +20,6 @@ void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in,
 void launch_expand_loras_backward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                   const void* const Ws[4], const void* const biases[4], const void* const dys[4],
                                   void* dw_in, void* dk_in, void* const dacts[4], const long ld_dacts[4], void* const dWs[4],
-                                  void* const dbiases[4], void* workspace, hipStream_t stream);
+                                  void* const dbiases[4], void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 }  // namespace wkv

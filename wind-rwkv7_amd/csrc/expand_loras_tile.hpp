@@ -91,8 +91,8 @@ void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_i
 // din: the heads' shares of the four d*_in, [M, H, 2, 16 / 4, 2, 4]: rank index 4g + r of i = 2 half + e at [half][g][e][r].
 // stats not null: the norm of each (token, head of HS channels) is read instead of summed over 64 channels
 void launch_loras16_backward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, const LoraDy& dy,
-                             __bf16* dw_in, __bf16* dk_in, __bf16* din, float* partial, const HeadStat* stats, int HS,
+                             __bf16* dw_in, __bf16* dk_in, __bf16* din, float* partial, int nsplit, const HeadStat* stats, int HS,
                              hipStream_t stream);
-void launch_loras16_reduce(long M, int C, const __bf16* din, const float* partial, const LoraReduceOut& out, hipStream_t stream);
+void launch_loras16_reduce(long M, int C, int nsplit, const __bf16* din, const float* partial, const LoraReduceOut& out, hipStream_t stream);
 
 }  // namespace wkv
