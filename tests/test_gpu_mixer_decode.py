@@ -38,9 +38,18 @@ def test_step_over_the_dispatch_of_its_kernels(B, H, state_dtype):
     assert seq_ref.rel_err(Sg.float().cpu(), Sw.float().cpu()) <= (2e-3 if state_dtype == torch.float32 else 8e-3)
 
 
-# rows no multiple of 16 or 64 and one past a multiple, heads past 256 and 2048 channels; the last also with the output grouped
-@pytest.mark.parametrize('B,H', [(161, 13), (33, 35), (257, 12), (400, 29)])
+# rows no multiple of 16 or 64 and one past a multiple, heads past 256 and 2048 channels; (750, 32) also with the output grouped,
+# (978, 10) by rows x channels^2 alone; (33, 35) one round of the linear kernel's widest blocks, (33, 43) more
+@pytest.mark.parametrize('B,H', [(161, 13), (33, 35), (257, 12), (400, 29), (33, 43), (750, 32), (978, 10)])
 def test_step_with_the_streams_in_memory(B, H):
+    test_step_over_the_dispatch_of_its_kernels(B, H, torch.float32)
+
+
+# the widths of the linear kernels' blocks: up to 256 blocks of 16, 32, 64 columns by a tile, else 64 by two tiles; at each line the
+# largest that fits and the smallest that does not, for the products with the interpolation (up to (64, 20)) and for the output
+@pytest.mark.parametrize('B,H', [(16, 20), (16, 21), (16, 1), (48, 12), (49, 12), (64, 19), (64, 20), (64, 16), (65, 16), (128, 16), (129, 16),
+                                 (256, 16), (257, 16)])
+def test_step_at_the_lines_of_its_linear_kernels(B, H):
     test_step_over_the_dispatch_of_its_kernels(B, H, torch.float32)
 
 

@@ -713,12 +713,6 @@ __global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
 
 constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
 int padded_rows(int B) { return (B + TOK - 1) / TOK * TOK; }
-// How much of the output a block of a linear kernel takes: the least that keeps the launch under so many blocks.  Below
-// them (about three blocks for two compute units) narrower blocks spread the loads wider; above, they repeat the
-// interpolation and re-read the inputs without any more of the chip to use.  us per step at 768 channels, 33 and 48
-// sequences: 16 columns 28.8 and 32.3, 32 columns 25.0 and 28.0; 64 x 2048 channels: 64 columns x 16 rows 69.6, x 32 rows 58.8.
-constexpr int LIN_BLOCKS = 400, LIN_SINGLE_BLOCKS = 320;
-
 }  // namespace
 
 // B: tokens in all (sequences times tokens per sequence).  (Four planes, eight with the streams in memory, and the hidden
@@ -729,42 +723,62 @@ size_t mixer_decode_workspace_bytes(int B, int C) {
     return 13 * A256(Bp * C * 2) + A256(Bp * R_GATE * 2) + A256(Bp * R_DECAY * 2) + 4 * A256(Bp * 16 * 2);
 }
 
+// (us below: a whole step, replayed from a graph)
+
 // A block repeats the expansion of its whole tile for the rows it updates, so it takes as many rows (up to 8) as leave about
-// one block per compute unit.  us per step at 768 channels: 16 sequences in blocks of 16 rows 34.8, of 1 row 22.7; 256
-// sequences in blocks of 4 rows 66, of 8 rows 54.
+// one block per compute unit.  In blocks of 1, 2, 4, 8 rows: 768 channels, 17 sequences 20.8, 20.9, 21.8, 23.3; 48 26.3, 25.1,
+// 23.7, 26.0; 128 41.1, 38.1, 33.7, 33.5; 256 60.2, 54.9, 47.9, 45.2; 192 channels, 176 23.3, 21.7, 21.1, 22.1.
 namespace {
 int head_rows_per_block(int B, int H) {
     int rpb = 1;
     while (rpb < 8 && (long)H * ((B + rpb - 1) / rpb) > compute_units()) rpb *= 2;
     return rpb;
 }
+
+// Blocks of a linear kernel for each tile (or two), of so many columns.
+int column_blocks(const LinArgs& a, int columns) {
+    int n = 0;
+    for (int i = 0; i < a.nseg; i++) n += (a.seg[i].N + columns - 1) / columns;
+    return n;
+}
+
 // The first-half products of many rows: every column block of the linear kernel makes its stream again, so from some rows on
 // the streams are written once (decode_lerp_kernel, a launch more) and multiplied by the grouped kernel of the sequence path,
-// whose tiles share both operands through LDS.  us, linear / lerp + grouped: 768 channels 128 rows 13.3/13.2, 192 17.0/13.3,
-// 256 18.1/13.8, 512 25.0/17.3; 1024 channels 128 rows 14.8/14.4; 1280 channels 96 rows 17.0/15.9; 2048 channels 32 rows
-// 19.6/20.8, 48 33.3/21.2, 128 38.9/22.2, 256 73.5/27, 512 133/57 (and the launch costs about one).  (Linear with its weights as
-// fragments; as whole lines it takes about a tenth less.)
-bool streams_in_memory(long rows, long C) { return rows * C * C >= (rows >= 160 ? 110000000 : 160000000) && rows > 32; }
-// The output projection alone makes nothing again, and the grouped kernel's tiles are few for it (2048 channels, 256 rows
-// 14.2/17.8 us, 512 rows 27.8/18.4; 1536 channels, 512 rows 19.8/15).
-bool output_grouped(long rows, long C) { return rows * C * C >= 1200000000; }
+// whose tiles share both operands through LDS: where the linear kernel's widest blocks take more than one round of the compute
+// units, and below 768 channels, where a round more costs less than the launch, from rows x channels^2 = 4e8 on.  Linear at its
+// best / streams: 768 channels, 160 rows (one round) 34.8/38.7, 176 42.0/42.5, 256 45.6/45.2, 512 66.5/66.8, 768 94.6/88.2;
+// 832 channels, 160 40.4/43.5, 192 44.0/44.5, 256 47.6/48.0, 384 64.4/63.1; 1024 channels, 128 (one round) 38.4/40.6, 160
+// 47.3/45.5, 256 54.8/51.9, 512 87.4/80.0; 1280 channels, 96 (one round) 40.9/42.4, 112 50.6/47.8; 2048 channels, 64 (one round)
+// 48.7/49.0, 96 66.0/57.0, 512 214/179; 704 channels, 224 40.8/43.0, 384 55.4/60.9, 768 84.9/85.3, 1024 100.8/98.1; 512
+// channels, 512 46.9/48.7, 1024 74.9/76.1, 1536 104.6/100.8.
+bool streams_in_memory(const LinArgs& a, long rows) {
+    const bool one_round = (long)column_blocks(a, 64) * ((a.ntiles + 1) / 2) <= compute_units();
+    return rows > 32 && ((a.C >= 768 && !one_round) || rows * a.C * a.C >= 400000000);
+}
+// The output projection alone makes nothing again, and the grouped kernel's tiles are few for it.  Linear / grouped: 1024
+// channels, 1024 rows 147.8/148.3, 1536 226.5/224.9; 1536 channels, 512 rows 114.3/116.5, 768 190.3/194.0, 1024 241.0/239.7;
+// 2048 channels, 512 rows 177.8/179.0, 640 218.9/223.8, 768 249.9/248.1, 1536 442.9/438.2.
+bool output_grouped(long rows, long C) { return rows * C * C >= 3000000000; }
 
+// How much of the output a block of a linear kernel takes: the least that leaves a compute unit no second block.  Narrower blocks
+// spread the loads wider; past one round they repeat the interpolation and re-read the inputs without any more of the chip to
+// use (16 columns of the products with it for one tile only: of two they lose to 32 already, 384 channels 18.4, 18.0).  In
+// columns x tiles of 16 x 1, 32 x 1, 64 x 1, 64 x 2: with the interpolation, 768 channels, 1 sequence 17.0, 18.2, 18.8, 19.3; 33
+// 22.5, 21.2, 23.0, 23.7; 64 27.1, 27.5, 26.3, 26.2; 128 38.7, 35.6, 35.7, 33.4; 384 channels, 48 21.4, 18.9, 19.4, 20.7; 1536
+// channels, 1 24.1, 21.9, 24.6, 26.5; 48 46.9, 38.8, 37.4, 40.8; the output, 768 channels, 48 23.8, 24.7, 25.4, 25.7; 256 45.0,
+// 45.3, 44.7, 45.5; 1024 channels, 96 38.0, 36.3, 37.1, 38.1; 2048 channels, 144 79.6, 75.1, 75.3, 73.1.
 template <bool LERP>
 void launch_linear(const LinArgs& a, const MixIn& mix, hipStream_t stream) {
-    auto blocks = [&](int columns) {
-        int n = 0;
-        for (int i = 0; i < a.nseg; i++) n += (a.seg[i].N + columns - 1) / columns;
-        return n;
-    };
+    auto one_round = [&](int columns) { return column_blocks(a, columns) * a.ntiles <= compute_units(); };
     const dim3 threads(256);
-    if (blocks(16) * a.ntiles <= LIN_BLOCKS)
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 1, 1>), dim3(blocks(16), a.ntiles), threads, 0, stream, a, mix);
-    else if (blocks(32) * a.ntiles <= LIN_BLOCKS)
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 2, 1>), dim3(blocks(32), a.ntiles), threads, 0, stream, a, mix);
-    else if (blocks(64) * a.ntiles <= LIN_SINGLE_BLOCKS)
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 1>), dim3(blocks(64), a.ntiles), threads, 0, stream, a, mix);
+    if ((!LERP || a.ntiles == 1) && one_round(16))
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 1, 1>), dim3(column_blocks(a, 16), a.ntiles), threads, 0, stream, a, mix);
+    else if (one_round(32))
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 2, 1>), dim3(column_blocks(a, 32), a.ntiles), threads, 0, stream, a, mix);
+    else if (one_round(64))
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 1>), dim3(column_blocks(a, 64), a.ntiles), threads, 0, stream, a, mix);
     else
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 2>), dim3(blocks(64), (a.ntiles + 1) / 2), threads, 0, stream, a, mix);
+        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 2>), dim3(column_blocks(a, 64), (a.ntiles + 1) / 2), threads, 0, stream, a, mix);
 }
 }  // namespace
 
@@ -784,7 +798,8 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
     auto c = [](const void* q) { return static_cast<const __bf16*>(q); };
     const MixIn mix{c(x), c(x_prev), c(mw.time_maa_w2), c(mw.time_maa), mid, rows, T};
 
-    // (one round of loads for four wavefronts up to 768 channels; beyond, sixteen: 2048 channels, one sequence, 9.3 -> 6.5 us)
+    // (one round of loads for four wavefronts up to 768 channels; beyond, sixteen.  us, a step in 4 / 16: 768 channels, 1 sequence
+    // 17.0/17.0, 48 23.6/24.2; 832 channels, 1 18.9/18.1; 2048 channels, 1 31.0/29.2, 256 92.8/91.4)
     if (C <= 768)
         hipLaunchKernelGGL((decode_mid_kernel<4, 3>), dim3(MID / 16, ntiles), dim3(256), 0, stream, mix, C, c(mw.time_maa_x),
                            c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
@@ -807,7 +822,7 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         a.C = C;
         a.rows = Bp;
         a.ntiles = ntiles;
-        if (streams_in_memory(rows, C)) {
+        if (streams_in_memory(a, rows)) {
             const long plane = (long)Bp * C;
             __bf16* const streams = take(4 * BC);
             hipLaunchKernelGGL(decode_lerp_kernel, dim3(C / 32, ntiles), dim3(256), 0, stream, mix, C, streams, plane);
