@@ -4,7 +4,7 @@
 // first-half products on four inputs, two second-half ones, the output projection, and as many input gradients: most are
 // too small to fill the chip on their own, each library call costs 10-15 us of host time, and the library knows neither
 // that two products add up to one input gradient nor that a concatenated output is cut into columns (some through tanh)
-// right after.  Here a launch takes up to eight problems on the same M tokens.  A problem is
+// right after.  Here a launch takes up to nine problems on the same M tokens (eight through the C interface).  A problem is
 //     D[m][n] = sum over up to two segments of  sum_k A[m][k] W[n][k]
 // with D's columns going to up to four tensors, each as it is, through tanh, or times 1 - aux^2 (the derivative).
 //
@@ -17,8 +17,9 @@
 // one's matrix work covers the other's barriers and last loads.
 //
 // Measured (us; in brackets the library's kernels for the same, replayed without host time): six first-half products of a
-// 768-channel block at 2006 / 8192 / 32768 tokens 21 (48) / 51 (70) / 169 (204); three input gradients with one second
-// segment at 8192 43 (66); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.6 (6.8) / 17.9 (16.9) / 92 (69).  Stages of
+// 768-channel block with their tanh and cut columns at 2006 / 8192 / 32768 tokens 21 (49) / 51 (69) / 170 (203); three input
+// gradients with one second segment at 8192 38 (55); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.1 (6.4) / 18 (16) /
+// 82-90 (70).  Stages of
 // 32 (half lines): 14 % slower at 65536 tokens; 256 x 192 tiles, one block per compute unit, a whole stage's operands in
 // registers: 13 % slower (768 contraction indices are twelve stages, too few to amortise its start and end alone);
 // walking the contraction from different places per tile: 5-15 % slower.
@@ -62,8 +63,8 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
     const int wm = wave >> 1, wn = wave & 1;
     const int lrow = tid / CPR;                      // this thread's row in a pass
     // (LDS answers sixteen lanes' 16-byte reads at a time, 256 bytes: two rows a line, so the pieces are permuted by pairs of
-    // rows.  By single rows, 47 % of the cycles that LDS was busy were conflicts, now 5 %; six products of a 768-channel block
-    // 42.4 -> 41.8 us, 65536 x 768 x 768 91 -> 90: LDS is busy 16 % of the time.)
+    // rows.  By single rows, 47 % of the cycles that LDS was busy were conflicts, now 5 %; six products of the sizes of a 768-channel
+    // block, each to one tensor as it is, 42.4 -> 41.8 us, 65536 x 768 x 768 91 -> 90: LDS is busy 16 % of the time.)
     auto swizzle = [](int row) { return (row >> 1) & 7; };
     static_assert(CPR == 8, "a row of a stage is one 128-byte line");
     const int piece = (tid % CPR) ^ swizzle(lrow);   // the piece of the row it fetches (RPP is a multiple of 8: the same in every pass)

@@ -26,8 +26,8 @@
 // A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
-//   1 x 256 tokens x 4 heads of 64   274 -> 99         8 x 1024 x 6 heads of 128   2420 -> 809
-//   8 x 1024 x 12 heads of 64        831 -> 427        32 x 1024 x 12 heads of 64  2395 -> 1373
+//   1 x 256 tokens x 4 heads of 64   274 -> 99-110     8 x 1024 x 6 heads of 128   2420 -> 811
+//   8 x 1024 x 12 heads of 64        831 -> 430        32 x 1024 x 12 heads of 64  2395 -> 1356
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
