@@ -1,0 +1,106 @@
+"""WKV7 by records in memory (few (batch, head) pairs) against the one-kernel form and against segments.
+
+The two ways run the same instructions on the same operands, so every output has to be the same bits.  A call takes records when
+its workspace holds them and the other way with the least that it accepts, so both are had through the C interface by the size of
+the workspace alone.
+"""
+import pytest
+import torch
+
+from oracle import inputs
+
+DEV = 'cuda'
+C = 64
+
+
+def _least(lib, B, T, H, interval):
+    """(forward, backward) bytes without records: the segments' maps, and what the backward keeps."""
+    NC, segments = T // 16, 1
+    while segments < 8 and B * H * segments * 2 <= 256 and NC % (segments * 2) == 0 and NC // (segments * 2) >= 32:
+        segments *= 2
+    maps = B * H * segments * 3 * C * C * 4 if segments >= 4 else 0
+    kept = B * H * (NC // 2 * 12288 if NC % 2 == 0 and interval == 32 else NC * 10240)
+    return max(maps, 256), kept + maps
+
+
+def test_workspace_sizes_at_the_lines_of_the_rule():
+    """Records from eight chunks (backward: from 96, or 48 and 2048 in all), for up to a quarter of the compute units' worth of (batch,
+    head) pairs and 6144 chunks, and not where a sequence runs as eight segments."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    for (B, T, H), (ahead, back) in {(1, 112, 4): (False, False), (1, 128, 4): (True, False), (1, 1520, 4): (True, False), (1, 1536, 4): (True, True),
+                                     (1, 752, 44): (True, False), (1, 768, 43): (True, True), (1, 768, 42): (True, False), (1, 1536, 64): (True, True),
+                                     (1, 1536, 65): (False, False), (1, 2048, 48): (True, True), (1, 2064, 48): (False, False),
+                                     (1, 4096, 12): (False, False), (1, 4080, 12): (True, True), (1, 4112, 12): (True, True),
+                                     (8, 1024, 12): (False, False)}.items():
+        chunks = B * H * (T // 16)
+        fwd, bwd = _least(lib, B, T, H, 32)
+        assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == (chunks * 13568 if ahead else fwd), (B, T, H)
+        kept = B * H * (T // 32 * 12288 if T % 32 == 0 else T // 16 * 10240)
+        assert lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == (kept + chunks * 10496 if back else bwd), (B, T, H)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('interval', [32, 16])
+@pytest.mark.parametrize('B,T,H,state', [(1, 128, 1, True), (3, 144, 3, False), (2, 160, 5, True), (1, 176, 8, True), (1, 1536, 1, False),
+                                         (2, 1552, 5, True), (1, 1568, 8, True), (3, 1584, 3, False), (1, 2048, 4, True), (1, 1024, 64, True),
+                                         (33, 1536, 1, False)])
+def test_records_give_the_bits_of_the_other_way(B, T, H, state, interval):
+    """Plain and attn_ln, forward without the kept states and, from 96 chunks, with them and backward; 8 to 11 and 96 to 99 chunks are
+    every remainder of the chain's registers, 2048 tokens run as four segments otherwise, 33 sequences reduce the parameter gradients in a launch of their own
+    (those sums alone are taken in another order)."""
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import set_checkpoint_interval
+    lib = _native.lib()
+    d = inputs.wkv7_inputs(B, T, H, C, seed=B + T + H, dtype=torch.bfloat16, s0_scale=0.3, dsT_scale=0.3)
+    x = [d[n].to(DEV).contiguous() for n in ('w', 'q', 'k', 'v', 'a', 'b')]
+    dy, s0, dsT = d['dy'].to(DEV).contiguous(), d['s0'].float().to(DEV).contiguous(), d['dsT'].float().to(DEV).contiguous()
+    gen = torch.Generator().manual_seed(T)
+    g = torch.randn(x[0].shape, generator=gen).bfloat16().to(DEV)
+    params = torch.randn(3, H * C, generator=gen).to(DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    ptr = lambda t: t.data_ptr()
+    ins, states = [ptr(t) for t in x], (ptr(s0), ptr(dsT)) if state else (None, None)
+    head = (B, T, H, C, _native.BF16, _native.F32)
+    mem = lambda n: torch.zeros(n, dtype=torch.uint8, device=DEV)
+    nan = lambda t: torch.full_like(t, float('nan'))
+    set_checkpoint_interval(interval)
+    try:
+        fwd, bwd = lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)
+        ln_bwd = lib.wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C)
+        least_fwd, least_bwd = _least(lib, B, T, H, interval)
+        assert fwd > least_fwd and (bwd > least_bwd) == (T >= 1024)
+        out = {}
+        for way, (f, b, lb) in {'records': (fwd, bwd, ln_bwd), 'least': (least_fwd, least_bwd, ln_bwd - (bwd - least_bwd))}.items():
+            ws, saved, ln_saved = mem(max(f, b, lb)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4])), mem(lib.wind_rwkv7_attn_ln_saved_bytes(*head[:4]))
+            y, y0, z, z0 = (nan(x[0]) for _ in range(4))
+            sT, s1, t0, t1 = (nan(s0) for _ in range(4))
+            grads, ln_grads = [nan(x[0]) for _ in range(6)], [nan(x[0]) for _ in range(7)]
+            ds0, ln_ds0, dparams = nan(s0), nan(s0), nan(params)
+            scratch, ln_scratch = torch.empty_like(saved), torch.empty_like(ln_saved)
+            _native.check(lib.wind_rwkv7_attn_prefill(*head, *ins, states[0], ptr(y0), ptr(scratch), ptr(s1), ptr(ws), f, stream))
+            _native.check(lib.wind_rwkv7_attn_forward(*head, *ins, states[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), f, stream))
+            _native.check(lib.wind_rwkv7_attn_backward(*head, *ins, ptr(dy), ptr(saved), states[1], *map(ptr, grads), ptr(ds0), ptr(ws), b, stream))
+            ln = (ptr(g), ptr(params))
+            _native.check(lib.wind_rwkv7_attn_ln_prefill(*head, *ins, *ln, states[0], ptr(z0), ptr(ln_scratch), ptr(t0), ptr(ws), f, stream))
+            _native.check(lib.wind_rwkv7_attn_ln_forward(*head, *ins, *ln, states[0], ptr(z), ptr(ln_saved), ptr(t1), ptr(ws), f, stream))
+            _native.check(lib.wind_rwkv7_attn_ln_backward(*head, *ins, *ln, ptr(dy), ptr(ln_saved), states[1], *map(ptr, ln_grads), ptr(dparams),
+                                                          ptr(ln_ds0), ptr(ws), lb, stream))
+            assert lib.wind_rwkv7_attn_forward(*head, *ins, states[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), least_fwd - 1, stream) == 6
+            assert lib.wind_rwkv7_attn_backward(*head, *ins, ptr(dy), ptr(saved), states[1], *map(ptr, grads), ptr(ds0), ptr(ws), least_bwd - 1, stream) == 6
+            torch.cuda.synchronize()
+            assert torch.equal(y, y0) and torch.equal(sT, s1) and torch.equal(z, z0) and torch.equal(t0, t1) and torch.equal(sT, t1)
+            out[way] = dict(y=y, sT=sT, z=z, ds0=ds0, ln_ds0=ln_ds0, dparams=dparams, **{f'd{i}': t for i, t in enumerate(grads)},
+                            **{f'ln_d{i}': t for i, t in enumerate(ln_grads)})
+        segmented = least_fwd > 256   # (the states entering the segments are composed there: fp32, but other sums)
+        for n, t in out['records'].items():
+            r = out['least'][n]
+            assert torch.isfinite(t.float()).all(), n
+            if segmented:
+                assert (t.float() - r.float()).norm() <= 2e-3 * r.float().norm(), n
+            elif n == 'dparams':
+                assert (t - r).norm() <= 1e-6 * r.norm()   # sums of B T terms in fp32, in another order
+            else:
+                assert torch.equal(t, r), n
+    finally:
+        set_checkpoint_interval(32)

@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -77,9 +78,12 @@ inline size_t rec_bwd_bytes(int B, int T, int H, bool ln = false) {
     if (pair_states(B, T, H)) return align_up((size_t)B * H * wkv::SavedPair::pairs(T / wkv::CHUNK) * wkv::SavedPair::BYTES);
     return align_up((size_t)chunks(B, T, H) * wkv::Saved::BYTES);
 }
-// the forward needs scratch only when the scan runs in segments; the argument is always checked
-inline size_t seg_bytes(int B, int T, int H) { return align_up(wkv::scan_segment_workspace_bytes(B, T, H)); }
-inline size_t fwd_ws_bytes(int B, int T, int H) { const size_t s = seg_bytes(B, T, H); return s ? s : 256; }
+// Scratch of the scan: the chunks' records, or the segments' maps and states.  The size queries ask for what the fastest way takes; a
+// call also accepts the least, with which there are no records.  (The forward's argument is always checked.)
+inline size_t scan_bytes(int B, int T, int H, bool fwd) { return align_up(wkv::scan_workspace_bytes(B, T, H, fwd)); }
+inline size_t scan_least_bytes(int B, int T, int H) { return align_up(wkv::scan_workspace_least_bytes(B, T, H)); }
+inline size_t fwd_ws_bytes(int B, int T, int H) { return std::max<size_t>(scan_bytes(B, T, H, true), 256); }
+inline size_t fwd_ws_least_bytes(int B, int T, int H) { return std::max<size_t>(scan_least_bytes(B, T, H), 256); }
 
 // ---- optional per-kernel timing (process-global, measurement only) ----
 struct Profile {
@@ -186,7 +190,7 @@ size_t wind_rwkv7_attn_fwd_workspace_bytes(int B, int T, int H, int C) {
 size_t wind_rwkv7_attn_bwd_workspace_bytes(int B, int T, int H, int C) {
     if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK) return 0;
     if (C != wkv::HEAD) return wkv::wide::record_bytes(B, T, H, C, false) + wkv::wide::kept_bytes(B, T, H, C);
-    return rec_bwd_bytes(B, T, H) + seg_bytes(B, T, H);
+    return rec_bwd_bytes(B, T, H) + scan_bytes(B, T, H, false);
 }
 
 // wide_centers (head sizes other than 64 only): y is attn_ln's kept output and is written centred, the centres there
@@ -200,7 +204,8 @@ static int attn_forward(int B, int T, int H, int C, int io_dtype, int state_dtyp
     rc = check_dtypes(io_dtype, state_dtype);
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !y || !s || !sT) return WIND_RWKV7_ERR_NULL_POINTER;   // (s0 may be null: a zero state)
-    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C));
+    rc = check_workspace(workspace, workspace_bytes,
+                         C != wkv::HEAD ? wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) : fwd_ws_least_bytes(B, T, H));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     Stamp st(0, stream);
@@ -211,7 +216,7 @@ static int attn_forward(int B, int T, int H, int C, int io_dtype, int state_dtyp
         return launch_status();
     }
     wkv::launch_fused_forward(B, T, H, state_dtype == WIND_RWKV7_F32, w, q, k, v, a, b, s0, sT, y, save ? s : nullptr,
-                              pair_states(B, T, H), stream, nullptr, nullptr, nullptr, nullptr, workspace);
+                              pair_states(B, T, H), stream, nullptr, nullptr, nullptr, nullptr, workspace, workspace_bytes);
     st.mark("wkv7_fused_kernel[fwd]");
     return launch_status();
 }
@@ -240,7 +245,7 @@ size_t wind_rwkv7_attn_prefill_static_bytes(int B, int T, int H, int C) {
     // problem before starting a graph capture has the lookup behind it; without a device it finds nothing and the
     // size is still returned.
     (void)static_scratch();
-    return rec_fwd_bytes(B, T, H) + fwd_ws_bytes(B, T, H);
+    return rec_fwd_bytes(B, T, H) + fwd_ws_least_bytes(B, T, H);
 }
 
 int wind_rwkv7_attn_prefill_static(int B, int T, int H, int C, int io_dtype, int state_dtype,
@@ -256,11 +261,11 @@ int wind_rwkv7_attn_prefill_static(int B, int T, int H, int C, int io_dtype, int
         return WIND_RWKV7_ERR_STATIC_LIMIT;
     char* base = static_cast<char*>(static_scratch());
     if (!base) return WIND_RWKV7_ERR_LAUNCH;
-    // the records first (every byte the kernels read of them is written by this call's prepare kernel first), the
-    // segment workspace behind them; nothing has to start at zero
+    // the scratch of the saved tensor's size first, the workspace behind it: all there is, so that the scan runs by records
+    // where they fit.  Nothing has to start at zero.
     const size_t rec = rec_fwd_bytes(B, T, H);
     return attn_forward(B, T, H, C, io_dtype, state_dtype, w, q, k, v, a, b, s0, y, base, sT, base + rec,
-                        fwd_ws_bytes(B, T, H), 0, stream);
+                        (size_t)WIND_RWKV7_STATIC_SCRATCH_BYTES - rec, 0, stream);
 }
 
 int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state_dtype,
@@ -275,7 +280,8 @@ int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !dy || !s) return WIND_RWKV7_ERR_NULL_POINTER;   // (dsT may be null: zero)
     if (!dw || !dq || !dk || !dv || !da || !db) return WIND_RWKV7_ERR_NULL_POINTER;            // (ds0 may be null: not wanted)
-    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C));
+    rc = check_workspace(workspace, workspace_bytes,
+                         C != wkv::HEAD ? wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) : rec_bwd_bytes(B, T, H) + scan_least_bytes(B, T, H));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     Stamp st(1, stream);
@@ -288,7 +294,7 @@ int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state
     }
     wkv::launch_fused_backward_scan(B, T, H, state_dtype == WIND_RWKV7_F32, w, q, a, b, dy, dsT, ds0, workspace,
                                     pair_states(B, T, H), stream, nullptr, nullptr,
-                                    static_cast<char*>(workspace) + rec_bwd_bytes(B, T, H));
+                                    static_cast<char*>(workspace) + rec_bwd_bytes(B, T, H), workspace_bytes - rec_bwd_bytes(B, T, H));
     st.mark("wkv7_fused_kernel[bwd]");
     wkv::launch_bwd_grads(B, T, H, w, q, k, v, a, b, dy, s, workspace, dw, dq, dk, dv, da, db,
                           pair_states(B, T, H) ? 3 : 1, stream);
@@ -320,7 +326,7 @@ size_t wind_rwkv7_attn_ln_bwd_workspace_bytes(int B, int T, int H, int C) {
     if (C != wkv::HEAD)
         return align256(wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)) +
                align256(wkv::lnheads::bwd_workspace_bytes((long)B * T, H, C)) + 4 * align256(wide_seq_bytes(B, T, H, C));
-    return rec_bwd_bytes(B, T, H, true) + seg_bytes(B, T, H) + seq_bytes(B, T, H) + ddot_bytes(B, T, H) + dpart_bytes(B, T, H);
+    return rec_bwd_bytes(B, T, H, true) + seq_bytes(B, T, H) + ddot_bytes(B, T, H) + dpart_bytes(B, T, H) + scan_bytes(B, T, H, false);
 }
 
 static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
@@ -334,7 +340,8 @@ static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_d
     rc = check_dtypes(io_dtype, state_dtype);
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !g || !params || !y || !s || !sT) return WIND_RWKV7_ERR_NULL_POINTER;
-    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_ln_fwd_workspace_bytes(B, T, H, C));
+    rc = check_workspace(workspace, workspace_bytes,
+                         C != wkv::HEAD ? wind_rwkv7_attn_ln_fwd_workspace_bytes(B, T, H, C) : fwd_ws_least_bytes(B, T, H));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (C != wkv::HEAD) {
@@ -355,7 +362,7 @@ static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_d
     // 86 us at B=8, H=12, T=1024.  With more heads than that the one-kernel form wins (no y_wkv round trip).
     if (2 * B * H <= wkv::compute_units()) {
         wkv::launch_fused_forward(B, T, H, state_dtype == WIND_RWKV7_F32, w, q, k, v, a, b, s0, sT, y_wkv, save ? s : nullptr,
-                                  pair_states(B, T, H), stream, nullptr, nullptr, nullptr, centers, workspace);
+                                  pair_states(B, T, H), stream, nullptr, nullptr, nullptr, centers, workspace, workspace_bytes);
         st.mark("wkv7_fused_kernel[fwd]");
     } else {
         wkv::launch_fused_forward(B, T, H, state_dtype == WIND_RWKV7_F32, w, q, k, v, a, b, s0, sT, y, save ? s : nullptr,
@@ -402,7 +409,9 @@ int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int st
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !g || !params || !dy || !s) return WIND_RWKV7_ERR_NULL_POINTER;
     if (!dw || !dq || !dk || !dv || !da || !db || !dg || !dparams) return WIND_RWKV7_ERR_NULL_POINTER;
-    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C));
+    rc = check_workspace(workspace, workspace_bytes,
+                         wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C) -
+                             (C != wkv::HEAD ? 0 : scan_bytes(B, T, H, false) - scan_least_bytes(B, T, H)));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (C != wkv::HEAD) {
@@ -425,10 +434,11 @@ int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int st
     }
     const char* y_wkv = static_cast<const char*>(s) + rec_fwd_bytes(B, T, H);
     char* rec = static_cast<char*>(workspace);
-    char* seg_ws = rec + rec_bwd_bytes(B, T, H, true);
-    char* dY = seg_ws + seg_bytes(B, T, H);
+    char* dY = rec + rec_bwd_bytes(B, T, H, true);
     float* ddot = reinterpret_cast<float*>(dY + seq_bytes(B, T, H));
     float* dpart = reinterpret_cast<float*>(reinterpret_cast<char*>(ddot) + ddot_bytes(B, T, H));
+    char* scan_ws = reinterpret_cast<char*>(dpart) + dpart_bytes(B, T, H);
+    const size_t scan_ws_bytes = workspace_bytes - (size_t)(scan_ws - rec);
     const float* centers = reinterpret_cast<const float*>(y_wkv + seq_bytes(B, T, H));
     const wkv::LnBackwardBuffers ln{k, v, g, y_wkv, params, centers, dg, dY, dv, ddot, dpart};
     Stamp st(1, stream);
@@ -436,11 +446,11 @@ int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int st
     st.mark("ln_epilogue_bwd_kernel");
     // the parameter-gradient partials are complete after the epilogue's backward: where the reverse scan leaves compute
     // units idle its launch reduces them too, else a launch of its own does at the end
-    const bool reduce_in_scan = wkv::fused_backward_scan_takes_dparams(B, T, H);
+    const bool reduce_in_scan = wkv::fused_backward_scan_takes_dparams(B, T, H, scan_ws_bytes);
     {
         wkv::launch_fused_backward_scan(B, T, H, state_dtype == WIND_RWKV7_F32, w, q, a, b, dY, dsT, ds0, rec,
                                         pair_states(B, T, H), stream, reduce_in_scan ? dpart : nullptr,
-                                        reduce_in_scan ? static_cast<float*>(dparams) : nullptr, seg_ws);
+                                        reduce_in_scan ? static_cast<float*>(dparams) : nullptr, scan_ws, scan_ws_bytes);
         st.mark("wkv7_fused_kernel[bwd]");
     }
     wkv::launch_bwd_grads(B, T, H, w, q, k, v, a, b, dY, s, rec, dw, dq, dk, dv, da, db,

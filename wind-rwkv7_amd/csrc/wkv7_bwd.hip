@@ -620,8 +620,8 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void dparams_reduce_kernel(int B, int H, int NC, const float* __restrict__ part,
                                                               float* __restrict__ dparams) {
-    __shared__ float red[16 * HEAD];
-    dparams_reduce_block(B, H, NC, part, dparams, blockIdx.x, blockIdx.y, red, 16);
+    __shared__ __attribute__((aligned(16))) float red[64 * HEAD];
+    dparams_reduce_block(B, H, NC, part, dparams, blockIdx.x, blockIdx.y, red, 64);
 }
 
 // ------------------------------------------------------------------------------------------------

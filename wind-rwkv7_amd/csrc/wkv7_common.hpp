@@ -156,23 +156,26 @@ __device__ __forceinline__ void store_pair(__bf16* __restrict__ p, int lane, bf1
 
 // attn_ln: dparams[p][h*64 + ch] = sum over batches and chunks of the per-chunk partials ([chunk][3][64] floats), in a
 // fixed order (the reference accumulates these with atomicAdd, attn_ln.cu:450-463, so its sums are order-dependent).
-// The work of one block for one (head, parameter): 64 channels x `groups` strided partial sums (one wavefront each),
-// combined through `red` ([groups][64] floats of LDS).
+// The work of one block for one (head, parameter): sixteen lanes take a record's 64 channels, `groups` of them (the block's
+// threads / 16) every groups-th of the B NC records, and the partial sums are combined through `red` ([groups][64] floats of
+// LDS).  What bounds it is the latency of its loads: 8 groups have 64 records on their way, where a wavefront per record (2 in
+// a small block, 4 bytes a lane) had 8 (attn_ln backward, 32 x 128 tokens x 2 heads, with the reduction in a block of two
+// wavefronts beside the scan: 67 -> 38 us).
 __device__ __forceinline__ void dparams_reduce_block(int B, int H, int NC, const float* __restrict__ part,
                                                      float* __restrict__ dparams, int h, int p, float* red, int groups) {
-    const int ch = threadIdx.x & 63, grp = threadIdx.x >> 6;
-    float acc = 0.f;
-    for (int bi = 0; bi < B; bi++) {
-        const long cid0 = ((long)bi * H + h) * NC;
-#pragma unroll 4
-        for (int c = grp; c < NC; c += groups) acc += part[((cid0 + c) * 3 + p) * HEAD + ch];
+    const int ch = 4 * (threadIdx.x & 15), grp = threadIdx.x >> 4;
+    f32x4 acc = zero4();
+#pragma unroll 8
+    for (int r = grp; r < B * NC; r += groups) {
+        const int bi = r / NC;
+        acc += *reinterpret_cast<const f32x4*>(part + ((((long)bi * H + h) * NC + (r - bi * NC)) * 3 + p) * HEAD + ch);
     }
-    red[grp * HEAD + ch] = acc;
+    *reinterpret_cast<f32x4*>(red + grp * HEAD + ch) = acc;
     __syncthreads();
-    if (grp == 0) {
+    if (threadIdx.x < HEAD) {
         float s = 0.f;
-        for (int g = 0; g < groups; g++) s += red[g * HEAD + ch];
-        dparams[(long)p * H * HEAD + (long)h * HEAD + ch] = s;
+        for (int g = 0; g < groups; g++) s += red[g * HEAD + threadIdx.x];
+        dparams[(long)p * H * HEAD + (long)h * HEAD + threadIdx.x] = s;
     }
 }
 

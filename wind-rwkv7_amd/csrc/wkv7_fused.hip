@@ -56,9 +56,12 @@ constexpr int fused_producers(int cuts) { return __builtin_popcount(cuts); }
 // (measured: one such wavefront, with a step between request and use, 122 us at B8 T1024 H12 against 86 us; the work
 // cut in two steps over four wavefronts 109 us - the statistics held across the barrier spill)
 constexpr int LN_WAVES = 3;
+// PREPARE: no ring and no chain; a block of one producer wavefront leaves one chunk's operands in memory, for
+// wkv7_records_scan_kernel.
 // VS: blocks per (batch, head), each owning 4 / VS of the four value blocks (16 value rows each) of the state
 // (MAP: two sets of chain wavefronts and nothing to store)
-constexpr int fused_threads(int cuts, bool ln, int vs = 1, bool map = false) {
+constexpr int fused_threads(int cuts, bool ln, int vs = 1, bool map = false, bool prepare = false) {
+    if (prepare) return 64;
     return ((map ? 2 : 1) * (4 / vs) + fused_producers(cuts) + (ln ? LN_WAVES : 0) + (map ? 0 : 1)) * 64;
 }
 constexpr int FUSE_SLOTS = 4;                   // ring slots; a producer stores in its last two segments only
@@ -106,10 +109,11 @@ struct FusedArgs {
     // ([B*H*NSEG][64][64] fp32 then).  NSEG = 1, LS = NC: the whole sequence in one block.
     int NSEG, LS;
     float* maps;                                // MAP: [B*H*NSEG][2][64][64], N in fragment order and M transposed
+    unsigned char* records;                     // PREPARE and wkv7_records_scan_kernel: [B*H][NC] ring slots in processing order
 };
 
 #define STEP_BARRIER() step_barrier()
-#define SEG(k) do { if constexpr ((CUTS >> (k)) & 1) STEP_BARRIER(); } while (0)
+#define SEG(k) do { if constexpr (!PREPARE && ((CUTS >> (k)) & 1)) STEP_BARRIER(); } while (0)
 // (the scheduling barriers keep each segment's arithmetic inside its step: the compiler would otherwise move it
 // freely across the barrier, which only orders LDS traffic, and unbalance the steps)
 __device__ __forceinline__ void step_barrier() {
@@ -134,8 +138,9 @@ __device__ __forceinline__ void lds_pair(unsigned char* p, int lane, bf16x4 u, b
     *reinterpret_cast<bf16x8*>(p + lane * 16) = __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool MAP = false>
-__global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_kernel(const FusedArgs A) {
+template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool MAP = false, bool PREPARE = false>
+__global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv7_fused_kernel(const FusedArgs A) {
+    static_assert(!PREPARE || (!SAVE && !LN && !MAP && VS == 1 && CUTS == 0xc00), "one wavefront, no steps to cut the work into");
     static_assert(!MAP || (!SAVE && !LN), "the map pass keeps and writes nothing but the maps");
     static_assert((CUTS >> 10 & 3) == 3, "the two storing segments are separate steps (ring slots are sized for that)");
     static_assert(!LN || FWD, "the epilogue belongs to the forward direction");
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
     constexpr int P = fused_producers(CUTS);
     constexpr int YRING = FUSE_SLOTS * SLOT;    // attn_ln: two slots of 4 KiB, the chain's fp32 output of one chunk each
     constexpr int ORING = YRING + (LN ? 2 * 4096 : 0), OSLOT = out_slot(NCH);
-    __shared__ __attribute__((aligned(16))) unsigned char ring[ORING + OUT_SLOTS * OSLOT];
+    __shared__ __attribute__((aligned(16))) unsigned char ring[PREPARE ? 16 : ORING + OUT_SLOTS * OSLOT];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Two blocks per head: blocks i and i + 8 are the two halves of one head, so that (blocks going to the eight XCDs
@@ -156,13 +161,15 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
         if ((int)blockIdx.x >= scan_blocks) {   // (the whole block, before any step barrier)
             const int e = (int)blockIdx.x - scan_blocks;
             dparams_reduce_block(A.B, A.H, A.NC, A.dparams_part, A.dparams, e % A.H, e / A.H, reinterpret_cast<float*>(ring),
-                                 (int)blockDim.x / 64);
+                                 (int)blockDim.x / 16);
             return;
         }
     }
-    const int unit = VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);   // (batch, head, segment)
+    // PREPARE: block ids in turn over the (batch, head)s rounded up to eight, so that a record is written on the XCD that reads it
+    const int heads8 = (A.BH + 7) & ~7;
+    const int unit = PREPARE ? (int)blockIdx.x % heads8 : VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);   // (batch, head, segment)
     const int vb0 = VS == 1 ? 0 : (int)((blockIdx.x >> 3) & 1) * NCH;    // first value block of this block
-    if (VS == 2 && unit >= A.BH * A.NSEG) return;   // (the whole block, before any barrier)
+    if ((VS == 2 || PREPARE) && unit >= A.BH * A.NSEG) return;   // (the whole block, before any barrier)
     // (the attn_ln form is never segmented: its launches are for many heads)
     const int bh = LN ? unit : unit / A.NSEG, seg = LN ? 0 : unit - bh * A.NSEG;
     const int NC = A.NC;            // chunks of the sequence: what the kept arrays are indexed with
@@ -259,11 +266,11 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
             return;
         }
     }
-    if (wave >= NCW && wave < NCW + P) {
+    if (PREPARE || (wave >= NCW && wave < NCW + P)) {
         // ------------------------------------------------------------------------------------------------
         // producer p: chunks p, p + P, ... in processing order; segment k of chunk st runs in step st + k
         // ------------------------------------------------------------------------------------------------
-        const int p = wave - NCW;
+        const int p = PREPARE ? (int)blockIdx.x / heads8 : wave - NCW;
         struct In {
             TileB w, q, k, v, a, b;   // backward: v holds dy, k unused
         };
@@ -282,9 +289,10 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
         };
         In nxt = fetch(p);
         int done = 0;
-        for (; done < p; done++) STEP_BARRIER();
+        if constexpr (!PREPARE)
+            for (; done < p; done++) STEP_BARRIER();
         for (int st = p; st < LS; st += P) {
-            unsigned char* slot = ring + (st % FUSE_SLOTS) * SLOT;
+            unsigned char* const slot = PREPARE ? A.records + ((long)unit * NC + st) * SLOT : ring + (st % FUSE_SLOTS) * SLOT;
             const In cur = nxt;
             const bf16x4 eye = identity_bf16(L);
             // ---- segments 0, 1: decay factors and the scaled operands, two blocks of 16 key channels each ----
@@ -375,7 +383,7 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
                 lds_pair(slot + SL_Y + 2048, lane, QKB0, QKB1);
             }
             *reinterpret_cast<float*>(slot + SL_FW + (16 * (L.n >> 2) + 4 * L.g + (L.n & 3)) * 4) = fw1;
-            nxt = fetch(st + P);
+            if constexpr (!PREPARE) nxt = fetch(st + P);
             SEG(10);
             // ---- segment 7: the shared operands of the chain ----
 #pragma unroll
@@ -388,12 +396,14 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
             lds_pair(slot + SL_J, lane, Mm[0], Mm[1]);
             lds_pair(slot + SL_J + 1024, lane, Mm[2], Mm[3]);
             SEG(11);
+            if constexpr (PREPARE) return;
             done += P;
         }
         for (; done < STEPS; done++) STEP_BARRIER();
         return;
     }
 
+    if constexpr (PREPARE) return;
     if (!MAP && wave == NCW + P + (LN ? LN_WAVES : 0)) {
         // ------------------------------------------------------------------------------------------------
         // store wavefront: after its barrier number P + 3 + st the results of chunk st are in their out slot
@@ -589,6 +599,196 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP)) void wkv7_fused_k
 }
 
 // ------------------------------------------------------------------------------------------------
+// The chain over records in memory: few (batch, head)s, where one block each (or two) would leave most of the chip idle and a
+// step of the one-kernel form, 0.556 us, is the time its producers take, ten wavefronts on one compute unit.  There the chunks are
+// prepared first, each by a wavefront of its own all over the chip (the PREPARE form above: the ring slot of a chunk, 13.25 KiB forward,
+// 10.25 KiB backward, goes to memory), and this kernel walks them with nothing but the chain: 0.21 us a chunk.
+// A block per value block (16 rows of the state), so four per (batch, head), of two wavefronts on two SIMDs:
+//   * the chain wavefront reads its operands straight into registers, RECORDS_AHEAD records ahead (7.25 KiB each, whole lines; 8 ahead
+//     is no faster), multiplies, and leaves the state and U^T of the chunk in LDS.  It waits for nobody but the barrier of a round.
+//   * the output wavefront takes them a round later: forward Y, and every store, of which none stands behind the chain's loads.
+// What bounds a round is the chain's own dependent instructions: two matrix instructions, a sum, four matrix instructions, the decay.
+// Measured, whole call (forward keeping a state per pair / backward with the gradient kernel, us; one kernel -> records), 64-channel
+// heads: 2 x 992 tokens x 12 heads 41.7 -> 26.8 / 58.8 -> 44.8, 1 x 256 x 4 17.4 -> 10.5 / 31.8 -> 25.7, 1 x 1024 x 64 44 -> 36 / 79 -> 71.
+// The same bits as the one-kernel form: the same instructions on the same operands.  Other forms, forward at 2 x 992 x 12: records through LDS rings
+// by loader wavefronts, two value blocks to a block 31.4 (what the wavefronts read from LDS is its time), four 39.8; one wavefront
+// doing the output and the stores as well 32.9.
+// ------------------------------------------------------------------------------------------------
+constexpr int RECORDS_AHEAD = 4;
+
+// x times entry 4 JB + R of the sixteen that a row of sixteen lanes holds
+template <int K>
+__device__ __forceinline__ float times_row_lane(float x, float held) {
+    return x * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, held), 0x150 + K, 0xf, 0xf, true));
+}
+template <int JB>
+__device__ __forceinline__ f32x4 times_decay(f32x4 x, float held) {
+    return (f32x4){times_row_lane<4 * JB>(x[0], held), times_row_lane<4 * JB + 1>(x[1], held), times_row_lane<4 * JB + 2>(x[2], held),
+                   times_row_lane<4 * JB + 3>(x[3], held)};
+}
+
+// the barrier of a wavefront whose own LDS accesses are done
+__device__ __forceinline__ void done_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <bool FWD, bool SAVE, bool CENTRED>
+__global__ __launch_bounds__(128) void wkv7_records_scan_kernel(const FusedArgs A) {
+    constexpr int RECORD = FWD ? SLOT_FWD : SLOT_BWD, AHEAD = RECORDS_AHEAD;
+    constexpr int OUT = 2048 + 512;   // the chain's results of a chunk: the state before it (bf16), U^T
+    __shared__ __attribute__((aligned(16))) unsigned char outs[2 * OUT];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if constexpr (!FWD) {
+        const int extra = A.dparams != nullptr ? 3 * A.H : 0, scan_blocks = (int)gridDim.x - extra;
+        if ((int)blockIdx.x >= scan_blocks) {   // (the whole block, before any barrier)
+            const int e = (int)blockIdx.x - scan_blocks;
+            dparams_reduce_block(A.B, A.H, A.NC, A.dparams_part, A.dparams, e % A.H, e / A.H, reinterpret_cast<float*>(outs), (int)blockDim.x / 16);
+            return;
+        }
+    }
+    // the four value blocks of a (batch, head) are 8 block ids apart: the same XCD, whose L2 brings a record in once
+    const int bh = 8 * (int)(blockIdx.x >> 5) + (int)(blockIdx.x & 7), ib = (int)(blockIdx.x >> 3) & 3;
+    if (bh >= A.BH) return;   // (the whole block, before any barrier)
+    const int NC = A.NC;      // barriers of either wavefront: the chain's results of round st are in LDS behind barrier st + 1
+    const Lane L;
+    auto chunk_of = [&](int st) -> int { return FWD ? st : NC - 1 - st; };
+    const int NP = SavedPair::pairs(NC);
+    auto keeps = [&](int c) {   // forward the state only where a pair of chunks begins, backward the dstate only where one ends and a run starts
+        if (!A.paired) return true;
+        return FWD ? !(c & 1) : SavedPair::keeps(c, NC) && SavedPair::ds_kept((long)bh * NP + (c >> 1), c >> 1, NP, A.ds_run);
+    };
+    // Everything in memory by descriptors on this (batch, head)'s part and 32-bit offsets
+    auto rsrc = [](const void* base, long bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (unsigned)bytes, 0x00020000); };
+    const auto rec = rsrc(A.records + (long)bh * NC * RECORD, (long)NC * RECORD);
+    auto record = [&](int st) { return min(st, NC - 1) * RECORD; };   // (behind the last one: that one again)
+    auto piece = [&](int st, int off) {
+        return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rec, lane * 16, record(st) + off, 0));
+    };
+    // fetch(i, st): record st into register set i; round(i, st)
+    auto walk = [&](auto&& fetch, auto&& round) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            fetch(i, i);
+            __builtin_amdgcn_sched_barrier(0);   // (in the loop's order: what is waited for there is counted)
+        }
+        int st = 0;
+        for (; st + AHEAD <= NC; st += AHEAD) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                round(i, st + i);
+                __builtin_amdgcn_sched_barrier(0);   // (a round's operands are waited for in that round)
+                fetch(i, st + i + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            if (st + i < NC) round(i, st + i);
+    };
+
+    if (wave == 1) {
+        // output wavefront: forward Y = QK V + QB U + wq S^T; the kept state and U^T; all stores
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        // A store that is not to be is one to an offset behind the end: no branch, so the number of accesses behind a load is
+        // known where the compiler waits for it.
+        constexpr unsigned NOWHERE = 0x40000000;
+        const long per_head = A.paired ? (long)NP * SavedPair::BYTES : (long)NC * Saved::BYTES;
+        const auto saved = rsrc(reinterpret_cast<unsigned char*>(A.saved) + (SAVE ? bh * per_head : 0), SAVE ? per_head : 0);
+        const int row = A.H * HEAD * 2;                                  // bytes
+        const long token0 = (long)(bh / A.H) * A.T * A.H + bh % A.H;     // of this (batch, head), in heads
+        const auto y_to = rsrc(A.y + (FWD ? token0 * HEAD : 0), FWD ? (long)A.T * row : 0);
+        const auto cen_to = rsrc(A.centers + (CENTRED ? token0 * 4 : 0), CENTRED ? (long)A.T * A.H * 16 : 0);
+        const unsigned y_lane = L.n * row + (32 * (ib / 2) + 8 * L.g + 4 * (ib % 2)) * 2;
+        const unsigned cen_lane = L.g == 0 ? (L.n * A.H * 4 + ib) * 4 : NOWHERE;
+        struct {
+            bf16x8 iv, yp[3];
+        } op[AHEAD];
+        walk(
+            [&](int i, int st) {
+                if constexpr (FWD) {
+                    op[i].iv = piece(st, SL_I + ib * 1024);
+#pragma unroll
+                    for (int k = 0; k < 3; k++) op[i].yp[k] = piece(st, SL_Y + k * 1024);
+                }
+            },
+            [&](int i, int st) {
+                done_barrier();
+                const int c = chunk_of(st);
+                const unsigned char* const o = outs + (st & 1) * OUT;
+                const bf16x8 s01 = reinterpret_cast<const bf16x8*>(o + lane * 32)[0], s23 = reinterpret_cast<const bf16x8*>(o + lane * 32)[1];
+                const bf16x4 u = *reinterpret_cast<const bf16x4*>(o + 2048 + lane * 8);
+                if constexpr (SAVE) {
+                    // bytes from this (batch, head)'s first: this value block's part of the kept state and of U^T
+                    const unsigned ck = (A.paired ? SavedPair::ds(c >> 1, ib) : Saved::ckpt(c, ib)) * 2;
+                    const unsigned ut = ((A.paired ? SavedPair::ut(c >> 1, c) : Saved::ut(c)) + ib * FRAG_ELEMS) * 2;
+                    const unsigned to = keeps(c) ? ck + lane * 32 : NOWHERE;
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, s01), saved, to, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, s23), saved, to + 16, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, u), saved, lane * 8, ut, 0);
+                }
+                if constexpr (FWD) {
+                    const bf16x8 VU = __builtin_shufflevector(op[i].iv, __builtin_shufflevector(u, u, 0, 1, 2, 3, 0, 1, 2, 3), 4, 5, 6, 7, 8, 9, 10, 11);
+                    f32x4 y = mma8(zero4(), s01, op[i].yp[0]);   // F(Y_ib): lane = token, reg = value channel
+                    y = mma8(y, s23, op[i].yp[1]);
+                    y = mma8(y, VU, op[i].yp[2]);
+                    if constexpr (CENTRED) {   // (see the fused kernel: attn_ln's kept output, centred per block)
+                        const float cen = row_sum16_bf16(y) * (1.f / 16);
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, cen), cen_to, cen_lane, c * CHUNK * A.H * 16, 0);
+                        y = y - cen;
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, to_bf16(y)), y_to, y_lane, c * CHUNK * row, 0);
+                }
+            });
+        return;
+    }
+    // chain wavefront: value rows 16 ib .. 16 ib + 15 of the state
+    __builtin_amdgcn_s_setprio(3);
+    f32x4 S[NBLK];
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) S[jb] = load_state_frag(A.s_in, A.s_in_f32, bh, ib, jb, L);
+    struct {
+        bf16x8 j[6], iv;
+        float fw;
+    } ops[AHEAD];
+    walk(
+        [&](int i, int st) {
+            auto& op = ops[i];
+#pragma unroll
+            for (int k = 0; k < 2; k++) op.j[k] = piece(st, SL_J + k * 1024);
+            op.iv = piece(st, SL_I + ib * 1024);
+#pragma unroll
+            for (int k = 2; k < 6; k++) op.j[k] = piece(st, SL_J + k * 1024);
+            op.fw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rec, (16 * (L.n >> 2) + 4 * L.g + (L.n & 3)) * 4, record(st) + SL_FW, 0));
+        },
+        [&](int i, int st) {
+            const auto& op = ops[i];
+            const bf16x4 b0 = to_bf16(S[0]), b1 = to_bf16(S[1]), b2 = to_bf16(S[2]), b3 = to_bf16(S[3]);
+            const bf16x8 s01 = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+            const bf16x8 s23 = __builtin_shufflevector(b2, b3, 0, 1, 2, 3, 4, 5, 6, 7);
+            const bf16x4 U0 = __builtin_shufflevector(op.iv, op.iv, 0, 1, 2, 3);
+            const f32x4 Ua = mma8(to_f32(U0), op.j[0], s01);   // + F(S_ib Wm^T), two independent halves
+            const f32x4 Uc = mma8(zero4(), op.j[1], s23);
+            unsigned char* const o = outs + (st & 1) * OUT;
+            reinterpret_cast<bf16x8*>(o + lane * 32)[0] = s01;
+            reinterpret_cast<bf16x8*>(o + lane * 32)[1] = s23;
+            auto decay = [&] { S[0] = times_decay<0>(S[0], op.fw), S[1] = times_decay<1>(S[1], op.fw), S[2] = times_decay<2>(S[2], op.fw), S[3] = times_decay<3>(S[3], op.fw); };
+            if constexpr (!FWD) decay();
+            const bf16x4 u = to_bf16(Ua + Uc);
+            const bf16x8 VU = __builtin_shufflevector(op.iv, __builtin_shufflevector(u, u, 0, 1, 2, 3, 0, 1, 2, 3), 4, 5, 6, 7, 8, 9, 10, 11);
+            *reinterpret_cast<bf16x4*>(o + 2048 + lane * 8) = u;
+#pragma unroll
+            for (int jb = 0; jb < NBLK; jb++) S[jb] = mma8(S[jb], op.j[2 + jb], VU);
+            if constexpr (FWD) decay();
+            done_barrier();
+        });
+#pragma unroll
+    for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.s_out, A.s_out_f32, bh, ib, jb, L, S[jb]);
+}
+
+// ------------------------------------------------------------------------------------------------
 // host launchers
 // ------------------------------------------------------------------------------------------------
 namespace {
@@ -605,7 +805,7 @@ FusedArgs fused_args(int B, int T, int H, int state_f32, int nseg) {
     return A;
 }
 
-// Long sequences on few heads (scan_segments > 1): the maps of all segments, then the states entering them.  After
+// Long sequences on few heads (ScanPlan::segments > 1): the maps of all segments, then the states entering them.  After
 // this A.s_in is the per-segment array and the kernel proper can be launched over B*H*nseg units.
 template <bool FWD>
 void segment_states(FusedArgs& A, int state_f32, void* seg_ws, hipStream_t stream) {
@@ -624,20 +824,42 @@ void segment_states(FusedArgs& A, int state_f32, void* seg_ws, hipStream_t strea
     launch_segment_carry(A.BH, A.NSEG, state_f32, A.s_in, maps, s_seg, stream);
     A.s_in = s_seg, A.s_in_f32 = 1;
 }
+
+// The chunks' records, then the chain over them.
+template <bool FWD>
+void by_records(FusedArgs A, bool save, void* ws, unsigned extra, hipStream_t stream) {
+    A.records = static_cast<unsigned char*>(ws);
+    FusedArgs P = A;
+    P.dparams = nullptr, P.dparams_part = nullptr;
+    constexpr int CUTS = 0xc00;
+    hipLaunchKernelGGL((wkv7_fused_kernel<FWD, false, false, CUTS, 1, false, true>), dim3((unsigned)((A.BH + 7) & ~7) * A.NC), dim3(64), 0, stream, P);
+    const dim3 grid(32 * ((A.BH + 7) / 8) + extra), block(128);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, A); };
+    if constexpr (!FWD) go(wkv7_records_scan_kernel<false, true, false>);
+    else if (A.centers) save ? go(wkv7_records_scan_kernel<true, true, true>) : go(wkv7_records_scan_kernel<true, false, true>);
+    else save ? go(wkv7_records_scan_kernel<true, true, false>) : go(wkv7_records_scan_kernel<true, false, false>);
+}
 }  // namespace
+
+size_t scan_record_bytes(bool fwd) { return fwd ? SLOT_FWD : SLOT_BWD; }
 
 void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v,
                           const void* a, const void* b, const void* s_in, void* s_out, void* y, void* saved,
                           int paired, hipStream_t stream, const void* g, const void* params, void* y_wkv, float* centers,
-                          void* seg_ws) {
+                          void* ws, size_t ws_bytes) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
-    const int nseg = params ? 1 : scan_segments(B, T, H);   // (the one-kernel attn_ln forward is for many heads)
+    const ScanPlan plan = params ? ScanPlan{false, 1} : scan_plan(B, T, H, ws_bytes, saved ? SCAN_FORWARD : SCAN_PREFILL);   // (the one-kernel attn_ln forward is for many heads)
+    const int nseg = plan.segments;
     FusedArgs A = fused_args(B, T, H, state_f32, nseg);
     A.w = c(w), A.q = c(q), A.k = c(k), A.v = c(v), A.a = c(a), A.b = c(b);
     A.saved = static_cast<__bf16*>(saved), A.s_in = s_in, A.s_out = s_out, A.y = static_cast<__bf16*>(y);
     A.g = c(g), A.params = static_cast<const float*>(params), A.y_wkv = static_cast<__bf16*>(y_wkv), A.centers = centers;
     A.paired = paired;
-    if (nseg > 1) segment_states<true>(A, state_f32, seg_ws, stream);
+    if (plan.records) {
+        by_records<true>(A, saved != nullptr, ws, 0, stream);
+        return;
+    }
+    if (nseg > 1) segment_states<true>(A, state_f32, ws, stream);
     const int units = B * H * nseg;
     auto go = [&](auto kernel, int threads, int vs = 1) {
         hipLaunchKernelGGL(kernel, dim3(fused_grid(units, vs)), dim3(threads), 0, stream, A);
@@ -662,25 +884,34 @@ void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, con
     }
 }
 
-bool fused_backward_scan_takes_dparams(int B, int T, int H) {
-    const int units = B * H * scan_segments(B, T, H);
+bool fused_backward_scan_takes_dparams(int B, int T, int H, size_t ws_bytes) {
+    const ScanPlan plan = scan_plan(B, T, H, ws_bytes, SCAN_BACKWARD);
+    // Beside a scan by records there is room everywhere, but its blocks have two wavefronts, and the more sequences a head has the
+    // longer theirs take: 32 x 128 tokens x 2 heads 38.0 -> 37.6 us, 64 x 512 tokens x 1 head 75 in the scan, 66 on their own.
+    if (plan.records) return B <= 32;
+    const int units = B * H * plan.segments;
     const int scan_blocks = (int)fused_grid(units, fused_split(units) ? 2 : 1);
     return scan_blocks + 3 * H <= compute_units();
 }
 
 void launch_fused_backward_scan(int B, int T, int H, int state_f32, const void* w, const void* q, const void* a,
                                 const void* b, const void* dy, const void* ds_in, void* ds_out, void* saved,
-                                int paired, hipStream_t stream, const float* dparams_part, float* dparams, void* seg_ws) {
+                                int paired, hipStream_t stream, const float* dparams_part, float* dparams, void* ws, size_t ws_bytes) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
-    const int nseg = scan_segments(B, T, H);
+    const ScanPlan plan = scan_plan(B, T, H, ws_bytes, SCAN_BACKWARD);
+    const int nseg = plan.segments;
     FusedArgs A = fused_args(B, T, H, state_f32, nseg);
     A.w = c(w), A.q = c(q), A.a = c(a), A.b = c(b), A.dy = c(dy);
     A.saved = static_cast<__bf16*>(saved), A.s_in = ds_in, A.s_out = ds_out;
     A.paired = paired, A.ds_run = paired ? dstate_run(B, T, H) : 1;
     A.dparams_part = dparams_part, A.dparams = dparams;
-    if (nseg > 1) segment_states<false>(A, state_f32, seg_ws, stream);
-    const int units = B * H * nseg;
     const unsigned extra = dparams ? 3 * H : 0;
+    if (plan.records) {
+        by_records<false>(A, true, ws, extra, stream);
+        return;
+    }
+    if (nseg > 1) segment_states<false>(A, state_f32, ws, stream);
+    const int units = B * H * nseg;
     if (fused_split(units))
         hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_TEN, 2>), dim3(fused_grid(units, 2) + extra), dim3(fused_threads(CUTS_TEN, false, 2)), 0, stream, A);
     else

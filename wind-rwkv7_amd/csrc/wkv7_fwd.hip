@@ -93,13 +93,36 @@ __global__ __launch_bounds__(256) void ln_epilogue_kernel(int T, int H, int nchu
 // it does not pay (measured forward+backward, 12 heads: 1024 tokens 133 us in two segments against 103 in one block).
 // Four segments fit up to a quarter of the compute units' worth of (batch, head) pairs (64: 8192 tokens 876 -> 768 us,
 // 60 pairs: 4096 tokens 459 -> 425 us, 2048 tokens 242 -> 246 us against the unsegmented kernel).
-int scan_segments(int B, int T, int H) {
+static int scan_segments(int B, int T, int H) {
     const int BH = B * H, NC = T / CHUNK;
     int g = 1;
     while (g < 8 && BH * g * 2 <= compute_units() && NC % (g * 2) == 0 && NC / (g * 2) >= 32) g *= 2;
     return g >= 4 ? g : 1;
 }
-size_t scan_segment_workspace_bytes(int B, int T, int H) {
+// By records where they are the fastest (forward, keeping a state per pair / whole backward, us; one launch or segments -> records):
+//   * four blocks per (batch, head) have a compute unit each: 64 pairs x 1024 tokens 44 -> 36 / 80 -> 71, 80 44.8 -> 49.2 / 91 -> 87,
+//     96 45.0 -> 53.4 / 95 -> 100;
+//   * from eight chunks on (without kept states: 1 pair x 128 tokens 11.6 -> 8.2; below, four chunks 8.4 -> 7.6, the gain is not worth
+//     the scratch).  A training pass has two launches more then, and a short one waits for its launches: eager forward + backward
+//     of attn on a host that takes 88-95 us for it, 4 x 512 tokens x 12 heads 88-91 -> 92-95, 4 x 768 99 -> 83, 1 x 1024 x 4 95 -> 95,
+//     4 x 1024 x 12 116 -> 95, of attn_ln 1 x 1024 x 4 115 -> 120.  So there from 96 chunks on, or 48 and 2048 in all;
+//   * up to 6144 chunks in all, 80 MiB of records, behind which writing and reading them is what counts (48 pairs x 2048 tokens 65 -> 56 /
+//     118 -> 108; 64 x 2048 71 -> 74 / 137 -> 136; 96 x 1024 above);
+//   * not where a sequence runs as eight segments (12 pairs x 4096 tokens 61 -> 69 / 94 -> 100; as four: 12 x 2048 57 -> 41 / 75 -> 57,
+//     32 x 3200 80 -> 73 / 143 -> 137).
+static bool scan_by_records(int B, int T, int H, ScanUse use) {
+    const long BH = (long)B * H, NC = T / CHUNK, least = use == SCAN_PREFILL ? 8 : BH * NC >= 2048 ? 48 : 96;
+    return NC >= least && 4 * BH <= compute_units() && BH * NC <= 6144 && scan_segments(B, T, H) < 8;
+}
+static size_t records_bytes(int B, int T, int H, bool fwd) { return (size_t)B * H * (T / CHUNK) * scan_record_bytes(fwd); }
+ScanPlan scan_plan(int B, int T, int H, size_t ws_bytes, ScanUse use) {
+    const bool records = scan_by_records(B, T, H, use) && ws_bytes >= records_bytes(B, T, H, use != SCAN_BACKWARD);
+    return {records, records ? 1 : scan_segments(B, T, H)};
+}
+size_t scan_workspace_bytes(int B, int T, int H, bool fwd) {
+    return scan_by_records(B, T, H, fwd ? SCAN_PREFILL : SCAN_BACKWARD) ? records_bytes(B, T, H, fwd) : scan_workspace_least_bytes(B, T, H);
+}
+size_t scan_workspace_least_bytes(int B, int T, int H) {
     const int g = scan_segments(B, T, H);
     return g == 1 ? 0 : (size_t)B * H * g * 3 * HEAD * HEAD * sizeof(float);   // N, M^T and the entering state per segment
 }

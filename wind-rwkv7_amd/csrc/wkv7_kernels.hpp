@@ -5,11 +5,19 @@
 
 namespace wkv {
 
-// Long sequences on few (batch, head) pairs run as segments (scan_segments > 1), which needs
-// scan_segment_workspace_bytes of scratch (seg_ws, 256-byte aligned; unused and may be null otherwise).
-int scan_segments(int B, int T, int H);
-size_t scan_segment_workspace_bytes(int B, int T, int H);
-// One launch for chunk preparation + state scan (wkv7_fused.hip).  `saved`: B*H*(T/16) records of Saved::BYTES, or with
+// How the state scan of either direction runs: by records in memory (wkv7_fused.hip), or in one kernel, long sequences on
+// few (batch, head) pairs as `segments` > 1 of them.  ws: 256-byte aligned scratch, scan_workspace_bytes of it for the way that is
+// fastest; with less, but scan_workspace_least_bytes (0: ws may be null), the way without records.
+struct ScanPlan {
+    bool records;
+    int segments;
+};
+enum ScanUse { SCAN_PREFILL, SCAN_FORWARD, SCAN_BACKWARD };   // forward without and with what a backward pass needs
+ScanPlan scan_plan(int B, int T, int H, size_t ws_bytes, ScanUse use);
+size_t scan_workspace_bytes(int B, int T, int H, bool fwd);
+size_t scan_workspace_least_bytes(int B, int T, int H);
+size_t scan_record_bytes(bool fwd);   // of one chunk
+// Chunk preparation + state scan (wkv7_fused.hip).  `saved`: B*H*(T/16) records of Saved::BYTES, or with
 // `paired` (an even number of chunks) one SavedPair per 32 tokens: the state entering the pair and U^T of both chunks
 // (forward: may be null, then nothing is kept for a backward pass).  params != nullptr: attn_ln - y receives
 // (group_norm(y_wkv) * ln_w + ln_b + (q.k.bonus) v) * g and, if saved, y_wkv the plain output for the backward pass,
@@ -19,16 +27,15 @@ size_t scan_segment_workspace_bytes(int B, int T, int H);
 void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, const void* q, const void* k, const void* v,
                           const void* a, const void* b, const void* s_in, void* s_out, void* y, void* saved,
                           int paired, hipStream_t stream, const void* g = nullptr, const void* params = nullptr,
-                          void* y_wkv = nullptr, float* centers = nullptr, void* seg_ws = nullptr);
-// Long sequences on few heads (scan_segments(B, T, H) > 1; not with params): the two launchers above and below run the
+                          void* y_wkv = nullptr, float* centers = nullptr, void* ws = nullptr, size_t ws_bytes = 0);
+// Long sequences on few heads (ScanPlan::segments > 1; not with params): the two launchers above and below run the
 // sequence as that many segments per (batch, head) - a first launch of the same kernel leaves each segment's affine
-// map, segment_carry composes them, then the kernel proper starts every segment from the state entering it.  seg_ws:
-// scan_segment_workspace_bytes(B, T, H) of scratch.
+// map, segment_carry composes them, then the kernel proper starts every segment from the state entering it.
 void launch_segment_carry(int BH, int nseg, int state_f32, const void* s_in, const float* maps, float* s_seg,
                           hipStream_t stream);
 // dparams != nullptr (attn_ln; only where fused_backward_scan_takes_dparams: the scan leaves that many compute units
 // idle): the launch also carries the blocks of launch_dparams_reduce, which then is not called.
-bool fused_backward_scan_takes_dparams(int B, int T, int H);
+bool fused_backward_scan_takes_dparams(int B, int T, int H, size_t ws_bytes);
 // How many consecutive pairs of chunks a wavefront of the gradient kernel takes as one run after the fused reverse scan
 // with a state per pair (SavedPair::ds_kept): 6, 3 or 1, whichever leaves the wavefronts the least uneven; negative
 // for runs that are cut per (batch, head) and handed out head-major (16 heads or more: their rows are long).
@@ -36,7 +43,7 @@ int dstate_run(int B, int T, int H);
 void launch_fused_backward_scan(int B, int T, int H, int state_f32, const void* w, const void* q, const void* a,
                                 const void* b, const void* dy, const void* ds_in, void* ds_out, void* saved,
                                 int paired, hipStream_t stream, const float* dparams_part = nullptr,
-                                float* dparams = nullptr, void* seg_ws = nullptr);
+                                float* dparams = nullptr, void* ws = nullptr, size_t ws_bytes = 0);
 // attn_ln: y = (group_norm(y_wkv) * ln_w + ln_b + (q.k.bonus) v) * g; centers: the centres y_wkv was kept with, or null
 void launch_ln_epilogue(int B, int T, int H, const void* y_wkv, const float* centers, const void* q, const void* k,
                         const void* v, const void* g, const void* params, void* y, hipStream_t stream);
