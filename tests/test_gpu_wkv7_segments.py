@@ -1,0 +1,59 @@
+"""WKV7 on few heads, the sequence cut into segments of uneven lengths, against the way that a call with the least scratch takes."""
+import pytest
+import torch
+
+from oracle import inputs
+
+DEV = 'cuda'
+C = 64
+
+
+def _scratch(B, T, H, segments):
+    return max(B * H * segments * 3 * C * C * 4, 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H,segments,least,states', [
+    (1, 3200, 40, 5, 4, torch.float32),     # 200 chunks, the shortest segments there are; with less scratch as four
+    (1, 3872, 48, 5, 0, torch.bfloat16),    # 242 chunks: no equal segments; with less scratch one block per head
+    (3, 4896, 12, 7, 0, torch.float32),     # 36 pairs, 306 chunks
+    (2, 3328, 16, 5, 4, None),              # 208 chunks, no states in
+    (1, 7744, 24, 10, 4, torch.float32),    # 484 chunks; more than eight segments
+])
+def test_segments_agree_with_the_other_way(B, T, H, segments, least, states):
+    """Every token goes through the same products; only the states at the cuts come from elsewhere, in fp32 (2e-3: a bf16 rounding
+    of what follows from them, as between one call and two that carry the state)."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    d = inputs.wkv7_inputs(B, T, H, C, seed=T + H, dtype=torch.bfloat16, s0_scale=0.3, dsT_scale=0.3)
+    x = [d[n].to(DEV).contiguous() for n in ('w', 'q', 'k', 'v', 'a', 'b')]
+    dy = d['dy'].to(DEV).contiguous()
+    dt = states or torch.float32
+    s0, dsT = (d[n].to(dt).to(DEV).contiguous() for n in ('s0', 'dsT'))
+    ptr = lambda t: t.data_ptr()
+    given = (ptr(s0), ptr(dsT)) if states else (None, None)
+    head = (B, T, H, C, _native.BF16, _native.F32 if dt == torch.float32 else _native.BF16)
+    stream = torch.cuda.current_stream().cuda_stream
+    mem = lambda n: torch.zeros(n, dtype=torch.uint8, device=DEV)
+    nan = lambda t: torch.full_like(t, float('nan'))
+    kept = B * H * (T // 32) * 12288
+    full = _scratch(B, T, H, segments)
+    assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == full and lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == kept + full
+    out = []
+    for f in (full, _scratch(B, T, H, least)):
+        b = kept + (f if f > 256 else 0)
+        ws, saved = mem(max(f, b)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4]))
+        y, y0, sT, s1, ds0 = nan(x[0]), nan(x[0]), nan(s0), nan(s0), nan(s0)
+        grads = [nan(x[0]) for _ in range(6)]
+        _native.check(lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), f, stream))
+        _native.check(lib.wind_rwkv7_attn_backward(*head, *map(ptr, x), ptr(dy), ptr(saved), given[1], *map(ptr, grads), ptr(ds0), ptr(ws), b, stream))
+        scratch = torch.empty_like(saved)
+        _native.check(lib.wind_rwkv7_attn_prefill(*head, *map(ptr, x), given[0], ptr(y0), ptr(scratch), ptr(s1), ptr(ws), f, stream))
+        if f > 256:
+            assert lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), _scratch(B, T, H, least) - 1, stream) == 6
+        torch.cuda.synchronize()
+        assert torch.equal(y, y0) and torch.equal(sT, s1)
+        out.append([y, sT, ds0] + grads)
+    for i, (t, r) in enumerate(zip(*out)):
+        assert torch.isfinite(t.float()).all(), i
+        assert (t.float() - r.float()).norm() <= (4e-3 if t.dtype == torch.bfloat16 and i in (1, 2) else 2e-3) * r.float().norm(), i

@@ -103,12 +103,14 @@ struct FusedArgs {
     float* dparams;
     int B;
     int ds_run;                                 // backward, paired: see SavedPair::ds_kept
-    // Long sequences on few heads: a (batch, head)'s NC chunks as NSEG segments of LS, a block each.  The MAP form of
-    // the kernel leaves every segment's affine map (S_out = S_in M + N) in `maps`, segment_carry_kernel composes them
-    // into the state entering each segment, and the kernel proper starts each segment from its entry of s_in
-    // ([B*H*NSEG][64][64] fp32 then).  NSEG = 1, LS = NC: the whole sequence in one block.
-    int NSEG, LS;
-    float* maps;                                // MAP: [B*H*NSEG][2][64][64], N in fragment order and M transposed
+    // Long sequences on few heads: a (batch, head)'s NC chunks as NSEG = PER + 1 segments, PER of them at a time, a block each.
+    // The state entering segment 0 is known, and nobody needs the map of the last one.  So a first pass (pass = 1) runs segment 0
+    // as the kernel proper does and leaves the affine map (S_out = S_in M + N) of segments 1 .. PER - 1 in `maps`,
+    // segment_carry_kernel composes them from the state that segment 0 left in entry 0 of s_seg into those entering the
+    // segments after it, and the second pass (pass = 2) starts segments 1 .. PER from their entries.
+    // pass = 0, NSEG = PER = 1, L0 = NC: the whole sequence in one block.
+    int pass, NSEG, PER, L0;                    // L0: chunks of segment 0 (the rest is divided evenly)
+    float* maps;                                // first pass: [B*H*PER][2][64][64], N in fragment order and M transposed
     unsigned char* records;                     // PREPARE and wkv7_records_scan_kernel: [B*H][NC] ring slots in processing order
 };
 
@@ -138,8 +140,12 @@ __device__ __forceinline__ void lds_pair(unsigned char* p, int lane, bf16x4 u, b
     *reinterpret_cast<bf16x8*>(p + lane * 16) = __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool MAP = false, bool PREPARE = false>
-__global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv7_fused_kernel(const FusedArgs A) {
+constexpr int fused_ring(bool fwd, bool ln) { return FUSE_SLOTS * (fwd ? SLOT_FWD : SLOT_BWD) + (ln ? 2 * 4096 : 0); }
+constexpr int fused_lds(bool fwd, bool ln, int vs) { return fused_ring(fwd, ln) + OUT_SLOTS * out_slot(4 / vs); }
+
+// GUESTS: the launch may have more wavefronts than this form uses
+template <bool FWD, bool SAVE, bool LN, int CUTS, int VS, bool MAP, bool PREPARE, bool GUESTS>
+__device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* const ring) {
     static_assert(!PREPARE || (!SAVE && !LN && !MAP && VS == 1 && CUTS == 0xc00), "one wavefront, no steps to cut the work into");
     static_assert(!MAP || (!SAVE && !LN), "the map pass keeps and writes nothing but the maps");
     static_assert((CUTS >> 10 & 3) == 3, "the two storing segments are separate steps (ring slots are sized for that)");
@@ -150,8 +156,7 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv
     constexpr int SLOT = FWD ? SLOT_FWD : SLOT_BWD;
     constexpr int P = fused_producers(CUTS);
     constexpr int YRING = FUSE_SLOTS * SLOT;    // attn_ln: two slots of 4 KiB, the chain's fp32 output of one chunk each
-    constexpr int ORING = YRING + (LN ? 2 * 4096 : 0), OSLOT = out_slot(NCH);
-    __shared__ __attribute__((aligned(16))) unsigned char ring[PREPARE ? 16 : ORING + OUT_SLOTS * OSLOT];
+    constexpr int ORING = fused_ring(FWD, LN), OSLOT = out_slot(NCH);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Two blocks per head: blocks i and i + 8 are the two halves of one head, so that (blocks going to the eight XCDs
@@ -169,15 +174,23 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv
     const int heads8 = (A.BH + 7) & ~7;
     const int unit = PREPARE ? (int)blockIdx.x % heads8 : VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);   // (batch, head, segment)
     const int vb0 = VS == 1 ? 0 : (int)((blockIdx.x >> 3) & 1) * NCH;    // first value block of this block
-    if ((VS == 2 || PREPARE) && unit >= A.BH * A.NSEG) return;   // (the whole block, before any barrier)
+    if ((VS == 2 || PREPARE) && unit >= A.BH * A.PER) return;   // (the whole block, before any barrier)
     // (the attn_ln form is never segmented: its launches are for many heads)
-    const int bh = LN ? unit : unit / A.NSEG, seg = LN ? 0 : unit - bh * A.NSEG;
+    const int bh = LN ? unit : unit / A.PER, seg = LN ? 0 : unit - bh * A.PER + (A.pass == 2 ? 1 : 0);
     const int NC = A.NC;            // chunks of the sequence: what the kept arrays are indexed with
-    const int LS = A.LS;            // chunks this block walks
+    auto segment_start = [&](int s) -> int { return s == 0 ? 0 : A.NSEG == 1 ? NC : A.L0 + (s - 1) * (NC - A.L0) / (A.NSEG - 1); };
+    const int first = LN ? 0 : segment_start(seg);
+    const int LS = LN ? NC : segment_start(seg + 1) - first;   // chunks this block walks
     const int STEPS = LS + P + 2;   // barriers every wavefront executes
     const Lane L;
     // processing order: forward walks the chunks up, backward down; segments are numbered in that order too
-    auto chunk_of = [&](int st) -> int { return FWD ? seg * LS + st : NC - 1 - (seg * LS + st); };
+    auto chunk_of = [&](int st) -> int { return FWD ? first + st : NC - 1 - (first + st); };
+    if constexpr (GUESTS) {
+        if (wave >= fused_threads(CUTS, LN, VS, MAP, PREPARE) / 64) {
+            for (int k = 0; k < STEPS; k++) STEP_BARRIER();
+            return;
+        }
+    }
 
     // Buffer loads: a tile is addressed as (descriptor of the tensor's rows of this (batch, head), wave-uniform chunk
     // offset, one 32-bit byte offset per lane that never changes), so no 64-bit address lives in vector registers;
@@ -500,7 +513,7 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv
 #pragma unroll
             for (int r = 0; r < 4; r++) S[jb][r] = (part == 1 && 16 * ib + L.n == 16 * jb + 4 * L.g + r) ? 1.f : 0.f;
         } else {
-            S[jb] = load_state_frag(A.s_in, A.s_in_f32, unit, ib, jb, L);   // (one entry per segment when there are several)
+            S[jb] = load_state_frag(A.s_in, A.s_in_f32, A.pass == 2 ? unit : bh, ib, jb, L);
         }
     }
 
@@ -592,10 +605,29 @@ __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, MAP, PREPARE)) void wkv
                 for (int r = 0; r < 4; r++) dst[(16 * jb + 4 * L.g + r) * HEAD + 16 * ib + L.n] = S[jb][r];
             }
         }
-    } else if (seg == A.NSEG - 1) {   // the segment walked last leaves the sequence's final state
+    } else if (A.pass == 1 || seg == A.NSEG - 1) {   // the first segment in a pass of its own; the one walked last: the sequence's final state
 #pragma unroll
-        for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.s_out, A.s_out_f32, bh, ib, jb, L, S[jb]);
+        for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.s_out, A.s_out_f32, A.pass == 1 ? unit : bh, ib, jb, L, S[jb]);
     }
+}
+
+template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool PREPARE = false>
+__global__ __launch_bounds__(fused_threads(CUTS, LN, VS, false, PREPARE)) void wkv7_fused_kernel(const FusedArgs A) {
+    __shared__ __attribute__((aligned(16))) unsigned char ring[PREPARE ? 16 : fused_lds(FWD, LN, VS)];
+    fused_block<FWD, SAVE, LN, CUTS, VS, false, PREPARE, false>(A, ring);
+}
+
+// The first pass over segments: the first one of each (batch, head) as above, the maps of the others.  Bound as those forms are: a
+// chunk of a map takes the producers 0.8 us, one of the kernel proper as long while the rest of the chip writes nothing.
+// Against the maps of PER equal segments and then a scan of those (forward with states kept + backward with the gradient kernel, us):
+// 1 x 16384 tokens x 32 heads 723 -> 687, 1 x 8192 x 64 720 -> 655, 4 x 8192 x 12 579 -> 540, 1 x 4096 x 12 154 -> 150.
+template <bool FWD, bool SAVE, int CUTS, int VS>
+__global__ __launch_bounds__(fused_threads(CUTS, false, VS, true)) void wkv7_first_pass_kernel(const FusedArgs A) {
+    static_assert(fused_threads(CUTS, false, VS, true) >= fused_threads(CUTS, false, VS), "the maps take more wavefronts");
+    __shared__ __attribute__((aligned(16))) unsigned char ring[fused_lds(FWD, false, VS)];
+    const int unit = VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);
+    if (unit % A.PER == 0) fused_block<FWD, SAVE, false, CUTS, VS, false, false, true>(A, ring);
+    else fused_block<FWD, false, false, CUTS, VS, true, false, false>(A, ring);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -796,33 +828,38 @@ namespace {
 inline unsigned fused_grid(int units, int vs) { return vs == 1 ? units : 16 * ((units + 7) / 8); }
 inline bool fused_split(int units) { return 2 * units <= compute_units(); }
 
-FusedArgs fused_args(int B, int T, int H, int state_f32, int nseg) {
+FusedArgs fused_args(int B, int T, int H, int state_f32, int per) {
     FusedArgs A{};
     A.T = T, A.H = H, A.NC = T / CHUNK, A.BH = B * H, A.B = B;
     A.s_in_f32 = A.s_out_f32 = state_f32;
-    A.NSEG = nseg, A.LS = A.NC / nseg;
+    A.PER = per, A.NSEG = per == 1 ? 1 : per + 1;
+    A.L0 = per == 1 ? A.NC : first_segment_chunks(A.NC, per);
     A.ds_run = 1;
     return A;
 }
 
-// Long sequences on few heads (ScanPlan::segments > 1): the maps of all segments, then the states entering them.  After
-// this A.s_in is the per-segment array and the kernel proper can be launched over B*H*nseg units.
+// Long sequences on few heads (ScanPlan::segments > 1): the first pass, then the states entering the segments of the second.  After
+// this A.s_in is the per-segment array and the kernel proper can be launched over the B*H*PER units of the second pass.
 template <bool FWD>
-void segment_states(FusedArgs& A, int state_f32, void* seg_ws, hipStream_t stream) {
-    const int units = A.BH * A.NSEG;
+void first_pass(FusedArgs& A, bool save, void* seg_ws, hipStream_t stream) {
+    const int units = A.BH * A.PER;
     float* maps = static_cast<float*>(seg_ws);
     float* s_seg = maps + (size_t)units * 2 * HEAD * HEAD;
     FusedArgs M = A;
-    M.maps = maps, M.saved = nullptr, M.y = nullptr, M.centers = nullptr, M.s_in = nullptr, M.s_out = nullptr;
+    M.pass = 1, M.maps = maps, M.s_out = s_seg, M.s_out_f32 = 1;
     M.dparams = nullptr, M.dparams_part = nullptr;
-    if (fused_split(units))
-        hipLaunchKernelGGL((wkv7_fused_kernel<FWD, false, false, CUTS_TEN, 2, true>), dim3(fused_grid(units, 2)),
-                           dim3(fused_threads(CUTS_TEN, false, 2, true)), 0, stream, M);
-    else
-        hipLaunchKernelGGL((wkv7_fused_kernel<FWD, false, false, CUTS_EIGHT_EVEN, 1, true>), dim3(fused_grid(units, 1)),
-                           dim3(fused_threads(CUTS_EIGHT_EVEN, false, 1, true)), 0, stream, M);
-    launch_segment_carry(A.BH, A.NSEG, state_f32, A.s_in, maps, s_seg, stream);
-    A.s_in = s_seg, A.s_in_f32 = 1;
+    auto go = [&](auto kernel, int vs, int threads) { hipLaunchKernelGGL(kernel, dim3(fused_grid(units, vs)), dim3(threads), 0, stream, M); };
+    if (fused_split(units)) {
+        constexpr int THREADS = fused_threads(CUTS_TEN, false, 2, true);
+        if (save) go(wkv7_first_pass_kernel<FWD, true, CUTS_TEN, 2>, 2, THREADS);
+        else if constexpr (FWD) go(wkv7_first_pass_kernel<FWD, false, CUTS_TEN, 2>, 2, THREADS);
+    } else {
+        constexpr int THREADS = fused_threads(CUTS_EIGHT_EVEN, false, 1, true);
+        if (save) go(wkv7_first_pass_kernel<FWD, true, CUTS_EIGHT_EVEN, 1>, 1, THREADS);
+        else if constexpr (FWD) go(wkv7_first_pass_kernel<FWD, false, CUTS_EIGHT_EVEN, 1>, 1, THREADS);
+    }
+    launch_segment_carry(A.BH, A.PER, maps, s_seg, stream);
+    A.pass = 2, A.s_in = s_seg, A.s_in_f32 = 1;
 }
 
 // The chunks' records, then the chain over them.
@@ -832,7 +869,7 @@ void by_records(FusedArgs A, bool save, void* ws, unsigned extra, hipStream_t st
     FusedArgs P = A;
     P.dparams = nullptr, P.dparams_part = nullptr;
     constexpr int CUTS = 0xc00;
-    hipLaunchKernelGGL((wkv7_fused_kernel<FWD, false, false, CUTS, 1, false, true>), dim3((unsigned)((A.BH + 7) & ~7) * A.NC), dim3(64), 0, stream, P);
+    hipLaunchKernelGGL((wkv7_fused_kernel<FWD, false, false, CUTS, 1, true>), dim3((unsigned)((A.BH + 7) & ~7) * A.NC), dim3(64), 0, stream, P);
     const dim3 grid(32 * ((A.BH + 7) / 8) + extra), block(128);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, A); };
     if constexpr (!FWD) go(wkv7_records_scan_kernel<false, true, false>);
@@ -859,7 +896,7 @@ void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, con
         by_records<true>(A, saved != nullptr, ws, 0, stream);
         return;
     }
-    if (nseg > 1) segment_states<true>(A, state_f32, ws, stream);
+    if (nseg > 1) first_pass<true>(A, saved != nullptr, ws, stream);
     const int units = B * H * nseg;
     auto go = [&](auto kernel, int threads, int vs = 1) {
         hipLaunchKernelGGL(kernel, dim3(fused_grid(units, vs)), dim3(threads), 0, stream, A);
@@ -910,7 +947,7 @@ void launch_fused_backward_scan(int B, int T, int H, int state_f32, const void* 
         by_records<false>(A, true, ws, extra, stream);
         return;
     }
-    if (nseg > 1) segment_states<false>(A, state_f32, ws, stream);
+    if (nseg > 1) first_pass<false>(A, true, ws, stream);
     const int units = B * H * nseg;
     if (fused_split(units))
         hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_TEN, 2>), dim3(fused_grid(units, 2) + extra), dim3(fused_threads(CUTS_TEN, false, 2)), 0, stream, A);

@@ -8,32 +8,33 @@
 #include "wkv7_common.hpp"
 #include "wkv7_kernels.hpp"
 
+#include <algorithm>
+
 namespace wkv {
 
 // ------------------------------------------------------------------------------------------------
-// Composes the segment maps in processing order: S_in(0) = s0, S_in(g+1) = S_in(g) M_g + N_g, all in fp32 (fp32
-// matrix instructions).  maps: as written by the MAP form of wkv7_fused_kernel; s_seg: [pair][segment][64][64]
-// floats, the state entering each segment.
+// Composes the segment maps in processing order: S(g) = S(g-1) M_g + N_g for g = 1 .. PER - 1, all in fp32 (fp32
+// matrix instructions).  maps: as written by wkv7_first_pass_kernel ([pair][g]; g = 0 is not there); s_seg: [pair][g][64][64]
+// floats, the state leaving segment g: entry 0 is there.
 // The value rows of a state go through the maps independently, so a block takes 16 of them (four blocks per (batch,
 // head)) and its four wavefronts a block of 16 key columns each: 16 matrix instructions per wavefront and segment,
-// then the row block's four fragments change hands through LDS.  All maps a wavefront needs (NSEG <= 8: seven times
+// then the row block's four fragments change hands through LDS.  All maps a wavefront needs (PER <= 12: eleven times
 // 20 registers) are requested before the first product.  (One block per (batch, head), a wavefront per 16 rows doing
 // all four column blocks: 64 dependent-by-fours matrix instructions per segment, 2.8 us each, 23 us at 8 segments.)
 // ------------------------------------------------------------------------------------------------
-constexpr int CARRY_MAX_SEG = 8;
-__global__ __launch_bounds__(256) void segment_carry_kernel(int NSEG, int s0_f32, const void* __restrict__ s0,
-                                                            const float* __restrict__ maps, float* __restrict__ s_seg) {
+constexpr int CARRY_MAX_SEG = 12;
+__global__ __launch_bounds__(256) void segment_carry_kernel(int PER, const float* __restrict__ maps, float* s_seg) {
     __shared__ f32x4 xch[2][NBLK][WAVE];
     const int jb = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int bh = blockIdx.x >> 2, ib = blockIdx.x & 3;
     const Lane L;
     f32x4 S[NBLK];
 #pragma unroll
-    for (int kb = 0; kb < NBLK; kb++) S[kb] = load_state_frag(s0, s0_f32, bh, ib, kb, L);
+    for (int kb = 0; kb < NBLK; kb++) S[kb] = load_state_frag(s_seg, 1, bh * PER, ib, kb, L);
     f32x4 n[CARRY_MAX_SEG - 1], mt[CARRY_MAX_SEG - 1][NBLK];
 #pragma unroll
     for (int g = 0; g < CARRY_MAX_SEG - 1; g++) {
-        const long e = (long)bh * NSEG + (g < NSEG - 1 ? g : NSEG - 2);   // (past the end: a valid map, not used)
+        const long e = (long)bh * PER + (g < PER - 1 ? g + 1 : PER - 1);   // (past the end: a valid map, not used)
         const float* N = maps + (e * 2 + 0) * HEAD * HEAD;
         const float* MT = maps + (e * 2 + 1) * HEAD * HEAD;
         n[g] = *reinterpret_cast<const f32x4*>(N + (16 * ib + L.n) * HEAD + 16 * jb + 4 * L.g);
@@ -41,15 +42,14 @@ __global__ __launch_bounds__(256) void segment_carry_kernel(int NSEG, int s0_f32
         for (int kb = 0; kb < NBLK; kb++)   // A operand of S[ib][kb] M[kb][jb]: F(M[kb][jb]^T) = the (jb, kb) block of MT
             mt[g][kb] = *reinterpret_cast<const f32x4*>(MT + (16 * jb + L.n) * HEAD + 16 * kb + 4 * L.g);
     }
-    store_state_frag(s_seg, 1, bh * NSEG, ib, jb, L, jb == 0 ? S[0] : jb == 1 ? S[1] : jb == 2 ? S[2] : S[3]);
 #pragma unroll
     for (int g = 0; g < CARRY_MAX_SEG - 1; g++) {
-        if (g < NSEG - 1) {   // (uniform; no load inside)
+        if (g < PER - 1) {   // (uniform; no load inside)
             f32x4 a0 = mma_f32(n[g], mt[g][0], S[0]), a1 = mma_f32(zero4(), mt[g][1], S[1]);
             a0 = mma_f32(a0, mt[g][2], S[2]);
             a1 = mma_f32(a1, mt[g][3], S[3]);
             const f32x4 T = a0 + a1;
-            store_state_frag(s_seg, 1, bh * NSEG + g + 1, ib, jb, L, T);
+            store_state_frag(s_seg, 1, bh * PER + g + 1, ib, jb, L, T);
             xch[g & 1][jb][lane] = T;
             __syncthreads();
 #pragma unroll
@@ -85,20 +85,33 @@ __global__ __launch_bounds__(256) void ln_epilogue_kernel(int T, int H, int nchu
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
-// Segments per (batch, head) for long sequences on few heads: a power of two, at most 8, that spreads the (batch, head)s
-// over an MI355X's 256 compute units, with at least 32 chunks per segment; 1 = the whole sequence in one block (or two).
-// A segmented pass is two launches of the one-kernel organisation (wkv7_fused.hip: every segment's affine map, then
-// the scan proper from the composed entering states) with the carry between them, so it costs twice a launch's fixed
+// Segments per (batch, head) and pass for long sequences on few heads (the whole sequence is one more): up to 8, as many as the
+// (batch, head)s leave compute units, each of 40 chunks or more; 1 = the whole sequence in one block (or two).
+// A segmented pass is two launches of the one-kernel organisation (wkv7_fused.hip: the first segment and the others' affine maps,
+// then the scan proper from the composed entering states) with the carry between them, so it costs twice a launch's fixed
 // 11-14 us, the carry's 3 us per segment, and 1.2 us per chunk and segment instead of 0.55: below four segments
 // it does not pay (measured forward+backward, 12 heads: 1024 tokens 133 us in two segments against 103 in one block).
 // Four segments fit up to a quarter of the compute units' worth of (batch, head) pairs (64: 8192 tokens 876 -> 768 us,
 // 60 pairs: 4096 tokens 459 -> 425 us, 2048 tokens 242 -> 246 us against the unsegmented kernel).
-static int scan_segments(int B, int T, int H) {
+// scan_segments_least: 4 or 8 of them, in whole chunks each, from 32; what a call with scratch for no more than that runs.
+// scan_segments_most: any number, of uneven lengths if need be, and of an even number of chunks in all.  Forward + backward, us, least -> most:
+// 40 heads x 16384 tokens 1070 (4) -> 920 (6), 48 pairs x 8192 540 (4) -> 507 (5), 40 x 3200 244 -> 224 (5).  Past eight where a segment has
+// one block and not two: 24 x 16384 618 (8) -> 572 (10), 20 x 8192 306 -> 276 (12), 17 x 16384 514 -> 429 (12).
+static int scan_segments_least(int B, int T, int H) {
     const int BH = B * H, NC = T / CHUNK;
     int g = 1;
     while (g < 8 && BH * g * 2 <= compute_units() && NC % (g * 2) == 0 && NC / (g * 2) >= 32) g *= 2;
     return g >= 4 ? g : 1;
 }
+static int scan_segments_most(int B, int T, int H) {
+    const int BH = B * H, NC = T / CHUNK, least = scan_segments_least(B, T, H);
+    const int g = NC % 2 ? 1 : std::min({2 * 8 * BH > compute_units() ? CARRY_MAX_SEG : 8, compute_units() / BH, NC / 40});
+    return g >= 4 && g > least ? g : least;
+}
+// Chunks of the segment that the first pass walks while it makes the maps of the others.  Its stores make its step longer than
+// theirs.  Forward + backward, us, at 0.7 / 0.8 / 0.9 / 1 of another segment's chunks: 1 x 16384 tokens x 32 heads 692 / 687 / 692 / 698,
+// 4 x 8192 x 12 545 / 540 / 542 / 542.
+int first_segment_chunks(int NC, int per) { return (int)(NC * 0.8 / (per + 0.8)); }
 // By records where they are the fastest (forward, keeping a state per pair / whole backward, us; one launch or segments -> records):
 //   * four blocks per (batch, head) have a compute unit each: 64 pairs x 1024 tokens 44 -> 36 / 80 -> 71, 80 44.8 -> 49.2 / 91 -> 87,
 //     96 45.0 -> 53.4 / 95 -> 100;
@@ -112,24 +125,23 @@ static int scan_segments(int B, int T, int H) {
 //     32 x 3200 80 -> 73 / 143 -> 137).
 static bool scan_by_records(int B, int T, int H, ScanUse use) {
     const long BH = (long)B * H, NC = T / CHUNK, least = use == SCAN_PREFILL ? 8 : BH * NC >= 2048 ? 48 : 96;
-    return NC >= least && 4 * BH <= compute_units() && BH * NC <= 6144 && scan_segments(B, T, H) < 8;
+    return NC >= least && 4 * BH <= compute_units() && BH * NC <= 6144 && scan_segments_least(B, T, H) < 8;
 }
 static size_t records_bytes(int B, int T, int H, bool fwd) { return (size_t)B * H * (T / CHUNK) * scan_record_bytes(fwd); }
+// N, M^T and the entering state per segment
+static size_t segments_bytes(int B, int H, int g) { return g == 1 ? 0 : (size_t)B * H * g * 3 * HEAD * HEAD * sizeof(float); }
 ScanPlan scan_plan(int B, int T, int H, size_t ws_bytes, ScanUse use) {
-    const bool records = scan_by_records(B, T, H, use) && ws_bytes >= records_bytes(B, T, H, use != SCAN_BACKWARD);
-    return {records, records ? 1 : scan_segments(B, T, H)};
+    if (scan_by_records(B, T, H, use) && ws_bytes >= records_bytes(B, T, H, use != SCAN_BACKWARD)) return {true, 1};
+    const int most = scan_segments_most(B, T, H);
+    return {false, ws_bytes >= segments_bytes(B, H, most) ? most : scan_segments_least(B, T, H)};
 }
 size_t scan_workspace_bytes(int B, int T, int H, bool fwd) {
-    return scan_by_records(B, T, H, fwd ? SCAN_PREFILL : SCAN_BACKWARD) ? records_bytes(B, T, H, fwd) : scan_workspace_least_bytes(B, T, H);
+    return scan_by_records(B, T, H, fwd ? SCAN_PREFILL : SCAN_BACKWARD) ? records_bytes(B, T, H, fwd) : segments_bytes(B, H, scan_segments_most(B, T, H));
 }
-size_t scan_workspace_least_bytes(int B, int T, int H) {
-    const int g = scan_segments(B, T, H);
-    return g == 1 ? 0 : (size_t)B * H * g * 3 * HEAD * HEAD * sizeof(float);   // N, M^T and the entering state per segment
-}
+size_t scan_workspace_least_bytes(int B, int T, int H) { return segments_bytes(B, H, scan_segments_least(B, T, H)); }
 
-void launch_segment_carry(int BH, int nseg, int state_f32, const void* s_in, const float* maps, float* s_seg,
-                          hipStream_t stream) {
-    hipLaunchKernelGGL(segment_carry_kernel, dim3(4 * BH), dim3(256), 0, stream, nseg, state_f32, s_in, maps, s_seg);
+void launch_segment_carry(int BH, int per, const float* maps, float* s_seg, hipStream_t stream) {
+    hipLaunchKernelGGL(segment_carry_kernel, dim3(4 * BH), dim3(256), 0, stream, per, maps, s_seg);
 }
 
 void launch_ln_epilogue(int B, int T, int H, const void* y_wkv, const float* centers, const void* q, const void* k,

@@ -29,10 +29,10 @@ void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, con
                           int paired, hipStream_t stream, const void* g = nullptr, const void* params = nullptr,
                           void* y_wkv = nullptr, float* centers = nullptr, void* ws = nullptr, size_t ws_bytes = 0);
 // Long sequences on few heads (ScanPlan::segments > 1; not with params): the two launchers above and below run the
-// sequence as that many segments per (batch, head) - a first launch of the same kernel leaves each segment's affine
-// map, segment_carry composes them, then the kernel proper starts every segment from the state entering it.
-void launch_segment_carry(int BH, int nseg, int state_f32, const void* s_in, const float* maps, float* s_seg,
-                          hipStream_t stream);
+// sequence as that many segments per (batch, head) and one more - a first pass walks the first and leaves the affine maps of
+// the next ones, segment_carry composes them, then the kernel proper starts every segment but the first from the state entering it.
+void launch_segment_carry(int BH, int per, const float* maps, float* s_seg, hipStream_t stream);
+int first_segment_chunks(int NC, int per);   // of the segment that the first pass walks
 // dparams != nullptr (attn_ln; only where fused_backward_scan_takes_dparams: the scan leaves that many compute units
 // idle): the launch also carries the blocks of launch_dparams_reduce, which then is not called.
 bool fused_backward_scan_takes_dparams(int B, int T, int H, size_t ws_bytes);
