@@ -33,6 +33,8 @@
 #include "wkv7_common.hpp"
 #include "wkv7_kernels.hpp"
 
+#include <type_traits>
+
 namespace wkv {
 
 // A producer's work on a chunk has twelve possible cut points (see the SEG() marks in the kernel); bit k of CUTS says
@@ -103,13 +105,13 @@ struct FusedArgs {
     float* dparams;
     int B;
     int ds_run;                                 // backward, paired: see SavedPair::ds_kept
-    // Long sequences on few heads: a (batch, head)'s NC chunks as NSEG = PER + 1 segments, PER of them at a time, a block each.
-    // The state entering segment 0 is known, and nobody needs the map of the last one.  So a first pass (pass = 1) runs segment 0
+    // Long sequences on few heads: a (batch, head)'s NC chunks as PER + 1 segments, PER of them at a time, a block each.
+    // The state entering segment 0 is known, and nobody needs the map of the last one.  So a first pass (PASS = 1) runs segment 0
     // as the kernel proper does and leaves the affine map (S_out = S_in M + N) of segments 1 .. PER - 1 in `maps`,
     // segment_carry_kernel composes them from the state that segment 0 left in entry 0 of s_seg into those entering the
-    // segments after it, and the second pass (pass = 2) starts segments 1 .. PER from their entries.
-    // pass = 0, NSEG = PER = 1, L0 = NC: the whole sequence in one block.
-    int pass, NSEG, PER, L0;                    // L0: chunks of segment 0 (the rest is divided evenly)
+    // segments after it, and the second pass (PASS = 2) starts segments 1 .. PER from their entries.
+    // PASS = 0, PER = 1: the whole sequence in one block.
+    int PER, L0;                                // L0: chunks of segment 0 (the rest is divided evenly)
     float* maps;                                // first pass: [B*H*PER][2][64][64], N in fragment order and M transposed
     unsigned char* records;                     // PREPARE and wkv7_records_scan_kernel: [B*H][NC] ring slots in processing order
 };
@@ -143,11 +145,11 @@ __device__ __forceinline__ void lds_pair(unsigned char* p, int lane, bf16x4 u, b
 constexpr int fused_ring(bool fwd, bool ln) { return FUSE_SLOTS * (fwd ? SLOT_FWD : SLOT_BWD) + (ln ? 2 * 4096 : 0); }
 constexpr int fused_lds(bool fwd, bool ln, int vs) { return fused_ring(fwd, ln) + OUT_SLOTS * out_slot(4 / vs); }
 
-// GUESTS: the launch may have more wavefronts than this form uses
-template <bool FWD, bool SAVE, bool LN, int CUTS, int VS, bool MAP, bool PREPARE, bool GUESTS>
+template <bool FWD, bool SAVE, bool LN, int CUTS, int VS, bool MAP, bool PREPARE, int PASS>
 __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* const ring) {
     static_assert(!PREPARE || (!SAVE && !LN && !MAP && VS == 1 && CUTS == 0xc00), "one wavefront, no steps to cut the work into");
-    static_assert(!MAP || (!SAVE && !LN), "the map pass keeps and writes nothing but the maps");
+    static_assert(!MAP || (!SAVE && !LN && PASS == 1), "the map form keeps and writes nothing but the maps");
+    static_assert(PASS == 0 || (!LN && !PREPARE), "the one-kernel attn_ln form is for many heads");
     static_assert((CUTS >> 10 & 3) == 3, "the two storing segments are separate steps (ring slots are sized for that)");
     static_assert(!LN || FWD, "the epilogue belongs to the forward direction");
     static_assert(VS == 1 || (VS == 2 && !LN), "the epilogue needs the whole head in one block");
@@ -175,17 +177,20 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
     const int unit = PREPARE ? (int)blockIdx.x % heads8 : VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);   // (batch, head, segment)
     const int vb0 = VS == 1 ? 0 : (int)((blockIdx.x >> 3) & 1) * NCH;    // first value block of this block
     if ((VS == 2 || PREPARE) && unit >= A.BH * A.PER) return;   // (the whole block, before any barrier)
-    // (the attn_ln form is never segmented: its launches are for many heads)
-    const int bh = LN ? unit : unit / A.PER, seg = LN ? 0 : unit - bh * A.PER + (A.pass == 2 ? 1 : 0);
     const int NC = A.NC;            // chunks of the sequence: what the kept arrays are indexed with
-    auto segment_start = [&](int s) -> int { return s == 0 ? 0 : A.NSEG == 1 ? NC : A.L0 + (s - 1) * (NC - A.L0) / (A.NSEG - 1); };
-    const int first = LN ? 0 : segment_start(seg);
-    const int LS = LN ? NC : segment_start(seg + 1) - first;   // chunks this block walks
+    int bh = unit, seg = 0, first = 0, LS = NC;   // this block walks LS chunks from `first` on
+    if constexpr (PASS != 0) {
+        auto segment_start = [&](int k) { return k == 0 ? 0 : A.L0 + (k - 1) * (NC - A.L0) / A.PER; };
+        bh = unit / A.PER;
+        seg = unit - bh * A.PER + (PASS == 2 ? 1 : 0);
+        first = segment_start(seg);
+        LS = segment_start(seg + 1) - first;
+    }
     const int STEPS = LS + P + 2;   // barriers every wavefront executes
     const Lane L;
     // processing order: forward walks the chunks up, backward down; segments are numbered in that order too
     auto chunk_of = [&](int st) -> int { return FWD ? first + st : NC - 1 - (first + st); };
-    if constexpr (GUESTS) {
+    if constexpr (PASS == 1 && !MAP) {   // (the launch has the map form's wavefronts)
         if (wave >= fused_threads(CUTS, LN, VS, MAP, PREPARE) / 64) {
             for (int k = 0; k < STEPS; k++) STEP_BARRIER();
             return;
@@ -513,7 +518,7 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
 #pragma unroll
             for (int r = 0; r < 4; r++) S[jb][r] = (part == 1 && 16 * ib + L.n == 16 * jb + 4 * L.g + r) ? 1.f : 0.f;
         } else {
-            S[jb] = load_state_frag(A.s_in, A.s_in_f32, A.pass == 2 ? unit : bh, ib, jb, L);
+            S[jb] = load_state_frag(A.s_in, A.s_in_f32, PASS == 2 ? unit : bh, ib, jb, L);
         }
     }
 
@@ -605,16 +610,16 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
                 for (int r = 0; r < 4; r++) dst[(16 * jb + 4 * L.g + r) * HEAD + 16 * ib + L.n] = S[jb][r];
             }
         }
-    } else if (A.pass == 1 || seg == A.NSEG - 1) {   // the first segment in a pass of its own; the one walked last: the sequence's final state
+    } else if (PASS != 2 || seg == A.PER) {   // the first segment in a pass of its own; the one walked last: the sequence's final state
 #pragma unroll
-        for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.s_out, A.s_out_f32, A.pass == 1 ? unit : bh, ib, jb, L, S[jb]);
+        for (int jb = 0; jb < NBLK; jb++) store_state_frag(A.s_out, A.s_out_f32, PASS == 1 ? unit : bh, ib, jb, L, S[jb]);
     }
 }
 
-template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool PREPARE = false>
+template <bool FWD, bool SAVE, bool LN, int CUTS, int VS = 1, bool PREPARE = false, int PASS = 0>
 __global__ __launch_bounds__(fused_threads(CUTS, LN, VS, false, PREPARE)) void wkv7_fused_kernel(const FusedArgs A) {
     __shared__ __attribute__((aligned(16))) unsigned char ring[PREPARE ? 16 : fused_lds(FWD, LN, VS)];
-    fused_block<FWD, SAVE, LN, CUTS, VS, false, PREPARE, false>(A, ring);
+    fused_block<FWD, SAVE, LN, CUTS, VS, false, PREPARE, PASS>(A, ring);
 }
 
 // The first pass over segments: the first one of each (batch, head) as above, the maps of the others.  Bound as those forms are: a
@@ -626,8 +631,8 @@ __global__ __launch_bounds__(fused_threads(CUTS, false, VS, true)) void wkv7_fir
     static_assert(fused_threads(CUTS, false, VS, true) >= fused_threads(CUTS, false, VS), "the maps take more wavefronts");
     __shared__ __attribute__((aligned(16))) unsigned char ring[fused_lds(FWD, false, VS)];
     const int unit = VS == 1 ? (int)blockIdx.x : 8 * (int)(blockIdx.x >> 4) + (int)(blockIdx.x & 7);
-    if (unit % A.PER == 0) fused_block<FWD, SAVE, false, CUTS, VS, false, false, true>(A, ring);
-    else fused_block<FWD, false, false, CUTS, VS, true, false, false>(A, ring);
+    if (unit % A.PER == 0) fused_block<FWD, SAVE, false, CUTS, VS, false, false, 1>(A, ring);
+    else fused_block<FWD, false, false, CUTS, VS, true, false, 1>(A, ring);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -832,8 +837,7 @@ FusedArgs fused_args(int B, int T, int H, int state_f32, int per) {
     FusedArgs A{};
     A.T = T, A.H = H, A.NC = T / CHUNK, A.BH = B * H, A.B = B;
     A.s_in_f32 = A.s_out_f32 = state_f32;
-    A.PER = per, A.NSEG = per == 1 ? 1 : per + 1;
-    A.L0 = per == 1 ? A.NC : first_segment_chunks(A.NC, per);
+    A.PER = per, A.L0 = first_segment_chunks(A.NC, per);
     A.ds_run = 1;
     return A;
 }
@@ -846,7 +850,7 @@ void first_pass(FusedArgs& A, bool save, void* seg_ws, hipStream_t stream) {
     float* maps = static_cast<float*>(seg_ws);
     float* s_seg = maps + (size_t)units * 2 * HEAD * HEAD;
     FusedArgs M = A;
-    M.pass = 1, M.maps = maps, M.s_out = s_seg, M.s_out_f32 = 1;
+    M.maps = maps, M.s_out = s_seg, M.s_out_f32 = 1;
     M.dparams = nullptr, M.dparams_part = nullptr;
     auto go = [&](auto kernel, int vs, int threads) { hipLaunchKernelGGL(kernel, dim3(fused_grid(units, vs)), dim3(threads), 0, stream, M); };
     if (fused_split(units)) {
@@ -859,7 +863,7 @@ void first_pass(FusedArgs& A, bool save, void* seg_ws, hipStream_t stream) {
         else if constexpr (FWD) go(wkv7_first_pass_kernel<FWD, false, CUTS_EIGHT_EVEN, 1>, 1, THREADS);
     }
     launch_segment_carry(A.BH, A.PER, maps, s_seg, stream);
-    A.pass = 2, A.s_in = s_seg, A.s_in_f32 = 1;
+    A.s_in = s_seg, A.s_in_f32 = 1;
 }
 
 // The chunks' records, then the chain over them.
@@ -909,15 +913,20 @@ void launch_fused_forward(int B, int T, int H, int state_f32, const void* w, con
         if (saved) go(wkv7_fused_kernel<true, true, true, CUTS>, fused_threads(CUTS, true));
         else go(wkv7_fused_kernel<true, false, true, CUTS>, fused_threads(CUTS, true));
     } else {
-        if (split) {
-            constexpr int CUTS2 = CUTS_TEN;
-            if (saved) go(wkv7_fused_kernel<true, true, false, CUTS2, 2>, fused_threads(CUTS2, false, 2), 2);
-            else go(wkv7_fused_kernel<true, false, false, CUTS2, 2>, fused_threads(CUTS2, false, 2), 2);
-        } else {
-            constexpr int CUTS1 = CUTS_EIGHT_EVEN;
-            if (saved) go(wkv7_fused_kernel<true, true, false, CUTS1>, fused_threads(CUTS1, false));
-            else go(wkv7_fused_kernel<true, false, false, CUTS1>, fused_threads(CUTS1, false));
-        }
+        auto pass = [&](auto which) {
+            constexpr int PASS = decltype(which)::value;
+            if (split) {
+                constexpr int CUTS2 = CUTS_TEN;
+                if (saved) go(wkv7_fused_kernel<true, true, false, CUTS2, 2, false, PASS>, fused_threads(CUTS2, false, 2), 2);
+                else go(wkv7_fused_kernel<true, false, false, CUTS2, 2, false, PASS>, fused_threads(CUTS2, false, 2), 2);
+            } else {
+                constexpr int CUTS1 = CUTS_EIGHT_EVEN;
+                if (saved) go(wkv7_fused_kernel<true, true, false, CUTS1, 1, false, PASS>, fused_threads(CUTS1, false));
+                else go(wkv7_fused_kernel<true, false, false, CUTS1, 1, false, PASS>, fused_threads(CUTS1, false));
+            }
+        };
+        if (nseg > 1) pass(std::integral_constant<int, 2>());
+        else pass(std::integral_constant<int, 0>());
     }
 }
 
@@ -949,10 +958,17 @@ void launch_fused_backward_scan(int B, int T, int H, int state_f32, const void* 
     }
     if (nseg > 1) first_pass<false>(A, true, ws, stream);
     const int units = B * H * nseg;
-    if (fused_split(units))
-        hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_TEN, 2>), dim3(fused_grid(units, 2) + extra), dim3(fused_threads(CUTS_TEN, false, 2)), 0, stream, A);
-    else
-        hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_EIGHT_EVEN>), dim3(fused_grid(units, 1) + extra), dim3(fused_threads(CUTS_EIGHT_EVEN, false)), 0, stream, A);
+    auto pass = [&](auto which) {
+        constexpr int PASS = decltype(which)::value;
+        if (fused_split(units))
+            hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_TEN, 2, false, PASS>), dim3(fused_grid(units, 2) + extra),
+                               dim3(fused_threads(CUTS_TEN, false, 2)), 0, stream, A);
+        else
+            hipLaunchKernelGGL((wkv7_fused_kernel<false, true, false, CUTS_EIGHT_EVEN, 1, false, PASS>), dim3(fused_grid(units, 1) + extra),
+                               dim3(fused_threads(CUTS_EIGHT_EVEN, false)), 0, stream, A);
+    };
+    if (nseg > 1) pass(std::integral_constant<int, 2>());
+    else pass(std::integral_constant<int, 0>());
 }
 
 }  // namespace wkv
