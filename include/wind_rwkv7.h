@@ -425,6 +425,14 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
                                   const void* const* x, const long long* ld_x,
                                   void* const* dW, int out_dtype,
                                   void* workspace, size_t workspace_bytes, void* stream);
+/* The same for the weights of one time mixer: up to nine, those above and the output projection. */
+#define WIND_RWKV7_BLOCK_WGRADS_MAX 9
+size_t wind_rwkv7_block_wgrads_workspace_bytes(int n, long long tokens, const int* O, const int* I);
+int wind_rwkv7_block_wgrads(int n, long long tokens, const int* O, const int* I,
+                            const void* const* dy, const long long* ld_dy,
+                            const void* const* x, const long long* ld_x,
+                            void* const* dW, int out_dtype,
+                            void* workspace, size_t workspace_bytes, void* stream);
 
 /* Working copies of up to WIND_RWKV7_PACK_MAX parameters in one launch: dst [rows, cols] in dst_dtype, and, where dstT is
  * given (dst_dtype bf16, rows % 16 == 0), the transposed copy dstT[c * ldT + r] (ldT >= rows, a multiple of 8).  cols is a

@@ -303,6 +303,20 @@ def test_linear_wgrad_group_sizes_and_validation_on_host():
     assert call(ws=None) == 6 and call(ws_bytes=need - 1) == 6 and call(ws=0x7010) == 6
 
 
+def test_block_wgrads_take_nine_on_host():
+    """The same as a group of up to nine: 9 problems of a block are 79 tiles, in three token ranges on 256 compute units."""
+    import ctypes
+    lib = _native.lib()
+    ints = lambda *v: (ctypes.c_int * len(v))(*v)
+    O, I = (768, 768, 768, 768, 128, 32, 96, 768, 768), (768, 768, 768, 768, 768, 768, 768, 128, 64)
+    sizes = lib.wind_rwkv7_block_wgrads_workspace_bytes
+    assert sizes(9, 8192, ints(*O), ints(*I)) == 3 * 4 * (4 * 16 * 192 * 192 + 3 * 256 * (128 + 32 + 96 + 128 + 64))
+    assert sizes(8, 8192, ints(*O), ints(*I)) == lib.wind_rwkv7_linear_wgrad_group_workspace_bytes(8, 8192, ints(*O), ints(*I)) > 0
+    assert sizes(10, 8192, ints(*O, 64), ints(*I, 64)) == 0 and sizes(0, 8192, ints(*O), ints(*I)) == 0
+    assert lib.wind_rwkv7_block_wgrads(10, 8192, None, None, None, None, None, None, None, 1, None, 0, None) == 2
+    assert lib.wind_rwkv7_block_wgrads(9, 8192, None, None, None, None, None, None, None, 1, None, 0, None) == 1
+
+
 def test_python_wrapper_raises_on_cpu_tensors():
     import torch
     from wind_rwkv.rwkv7 import attn

@@ -299,7 +299,7 @@ constexpr ShapeInfo kShapes[5] = {{3, 3, 2, 2}, {2, 1, 4, 1}, {2, 2, 4, 1}, {2, 
 // a longer token range, so there are fewer fp32 partial tiles to write and to sum (three 768 x 768 problems at
 // 8192 tokens: 48 tiles x 5 ranges instead of 3 x (16 x 16), 35 MB of partials instead of 113 MB), and problems
 // too small to fill the machine on their own share one launch.
-constexpr int WGRAD_MAX_JOBS = 8;
+constexpr int WGRAD_MAX_JOBS = 9;
 struct WgradGroup {
     WgradArgs job[WGRAD_MAX_JOBS];
     int first_tile[WGRAD_MAX_JOBS + 1];   // job j owns the grid's tiles first_tile[j] .. first_tile[j+1]-1

@@ -40,7 +40,7 @@ namespace py = pybind11;
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
     X(ddlerp_first_workspace_bytes) X(ddlerp_first) X(neutral_rows_keep) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
-    X(linear_wgrad_group_workspace_bytes) X(linear_wgrad_group) X(mixer_decode_workspace_bytes) X(mixer_decode) \
+    X(block_wgrads_workspace_bytes) X(block_wgrads) X(mixer_decode_workspace_bytes) X(mixer_decode) \
     X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
 struct Lib {
@@ -700,7 +700,10 @@ struct Products {
     }
 };
 
-// dW = dy^T x for several pairs on the same tokens: one grouped launch (a single pair goes through its own entry point)
+// dW = dy^T x for several pairs on the same tokens: one grouped launch (a single pair goes through its own entry point).  Whatever
+// runs on its own leaves fp32 partial tiles from every compute unit, 147 KB each, which are written and read again: a 768 x 768 product
+// of 8192 tokens is 22 us + 8 of sums for 12 us of products.  So all of a pass go together; the nine of a block there, us with their sums:
+// eight and the output projection 90, projections and LoRA factors 88, one launch 78.
 struct WeightGrads {
     std::vector<int> O, I;
     std::vector<const void*> dy, x;
@@ -717,9 +720,9 @@ struct WeightGrads {
             check(L.linear_wgrad(tokens, O[0], I[0], dy[0], ld_dy[0], x[0], ld_x[0], dW[0], WIND_RWKV7_F32, ptr(ws), ws.numel(), stream));
             return;
         }
-        const Tensor ws = scratch_bytes(L.linear_wgrad_group_workspace_bytes(n, tokens, O.data(), I.data()), like);
-        check(L.linear_wgrad_group(n, tokens, O.data(), I.data(), dy.data(), ld_dy.data(), x.data(), ld_x.data(), dW.data(), WIND_RWKV7_F32,
-                                   ptr(ws), ws.numel(), stream));
+        const Tensor ws = scratch_bytes(L.block_wgrads_workspace_bytes(n, tokens, O.data(), I.data()), like);
+        check(L.block_wgrads(n, tokens, O.data(), I.data(), dy.data(), ld_dy.data(), x.data(), ld_x.data(), dW.data(), WIND_RWKV7_F32,
+                             ptr(ws), ws.numel(), stream));
     }
 };
 
@@ -896,12 +899,12 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         const bool kept = G.at[i] < G.kept;
         return static_cast<float*>((kept ? flat : unwanted).data_ptr()) + G.at[i] - (kept ? 0 : G.kept);
     };
-    {
-        WeightGrads wg;
-        if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
+    WeightGrads wg;   // (run at the end: everything that they multiply is kept until then)
+    if (need(WO)) wg.add(ptr(dout), C, ptr(ya), C, g(WO));
+    if (!st.attn) {
         wg.run(M, dout, stream);
+        return;
     }
-    if (!st.attn) return;
     if (G.total > G.kept) unwanted = at::empty({G.total - G.kept}, flat.options());
     const WeightLayout W(C);
     const Activations A(s, true);
@@ -951,7 +954,6 @@ void block_backward(const Block& s, const Tensor& xb, const Tensor& weights, con
         }
         p.run(M, xb);
     }
-    WeightGrads wg;   // (all at the end: everything that they multiply is kept until then)
     if (need(WR)) wg.add(d(P), C, a(A.streams), C, g(WR));
     if (need(GATE_W1)) wg.add(d(o_g1), R_GATE, a(A.streams), C, g(GATE_W1));
     if (need(WK)) wg.add(d(8 * P), C, a(A.streams + 2 * P), C, g(WK));
