@@ -226,6 +226,15 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
     return r;
 }
 
+// Results that no kernel reads again soon leave past the caches (non-temporal): what a kernel and the ones behind it read then stays
+// in them.  The kept states, U^T and outputs of the WKV7 scans and the gradients, forward + backward of attn, us: 12 x 1024 tokens x 12 heads
+// 197 -> 178, 16 x 1024 x 12 211 -> 198, 24 x 1024 x 12 362 -> 337, 8 x 1024 x 32 276 -> 255, 8 x 2048 x 12 257 -> 248; 8 x 1024 x 12 138 -> 137 and
+// 64 x 1024 x 12 758 -> 756 (753 with the gradients through the caches, which is 1 to 5 % slower everywhere below).
+// Loads that way (half lines each) are slower: 8 x 2048 x 12 253 -> 269.
+constexpr int STREAMED = 2;   // of a buffer store
+template <class V>
+__device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontemporal_store(x, static_cast<V*>(to)); }
+
 // Load a [16 tokens x 64 channels] tile whose row n starts at p + n*ld (elements).
 __device__ __forceinline__ TileB load_rows(const __bf16* __restrict__ p, long ld, const Lane& L) {
     TileB t;

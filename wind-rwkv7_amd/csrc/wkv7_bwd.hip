@@ -236,7 +236,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         for (int pr = 0; pr < NBLK / 2; pr++)
             __builtin_amdgcn_raw_buffer_store_b128(
                 __builtin_bit_cast(i32x4, __builtin_shufflevector(x.f[2 * pr], x.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7)), r,
-                voff_n + 16 * L.g + 64 * pr, 0, 0);
+                voff_n + 16 * L.g + 64 * pr, 0, STREAMED);
     };
     auto frags4 = [&](const __bf16* p, int ln) {                      // load_frags: four fragments, [i][lane] x 8 B
         TileB x;

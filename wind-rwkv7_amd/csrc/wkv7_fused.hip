@@ -450,20 +450,20 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
                 }
                 if (keep) {
 #pragma unroll
-                    for (int i = 0; i < 2 * NCH; i++) *reinterpret_cast<bf16x8*>(saved + ck + i * 1024 + lane * 16) = piece(out_ck(NCH) + i * 1024);
+                    for (int i = 0; i < 2 * NCH; i++) store_streamed(saved + ck + i * 1024 + lane * 16, piece(out_ck(NCH) + i * 1024));
                 }
                 if constexpr (NCH == 4) {
 #pragma unroll
-                    for (int i = 0; i < 2; i++) *reinterpret_cast<bf16x8*>(saved + ut + i * 1024 + lane * 16) = piece(out_ut(NCH) + i * 1024);
+                    for (int i = 0; i < 2; i++) store_streamed(saved + ut + i * 1024 + lane * 16, piece(out_ut(NCH) + i * 1024));
                 } else {
-                    *reinterpret_cast<bf16x8*>(saved + ut + lane * 16) = piece(out_ut(NCH));
+                    store_streamed(saved + ut + lane * 16, piece(out_ut(NCH)));
                 }
             }
             if constexpr (FWD && !LN) {
                 // y by rows: a lane's 16 bytes are the fragments of value blocks 2p and 2p + 1 (8 contiguous channels)
 #pragma unroll
                 for (int pp = 0; pp < NCH / 2; pp++)
-                    *reinterpret_cast<bf16x8*>(A.y + y_lane + (long)c * CHUNK * row_ld + 32 * pp) = piece(out_y(NCH) + pp * 1024);
+                    store_streamed(A.y + y_lane + (long)c * CHUNK * row_ld + 32 * pp, piece(out_y(NCH) + pp * 1024));
                 if (A.centers != nullptr && lane < 16) {   // token `lane`: the centres of this block's value blocks
                     float* dst = A.centers + 4 * (((long)(bh / A.H) * A.T + c * CHUNK + lane) * A.H + bh % A.H) + vb0;
                     const float* src = reinterpret_cast<const float*>(o + out_cen(NCH)) + lane * NCH;
