@@ -230,10 +230,15 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
 // in them.  The kept states, U^T and outputs of the WKV7 scans and the gradients, forward + backward of attn, us: 12 x 1024 tokens x 12 heads
 // 197 -> 178, 16 x 1024 x 12 211 -> 198, 24 x 1024 x 12 362 -> 337, 8 x 1024 x 32 276 -> 255, 8 x 2048 x 12 257 -> 248; 8 x 1024 x 12 138 -> 137 and
 // 64 x 1024 x 12 758 -> 756 (753 with the gradients through the caches, which is 1 to 5 % slower everywhere below).
-// Loads that way (half lines each) are slower: 8 x 2048 x 12 253 -> 269.
+// The same at other head sizes and in fp32, whose kept states are larger: wkv7_wide.hip, wkv7_f32.hip.  Loads that way pay where a
+// kernel reads whole lines for the last time (load_streamed); of half lines they are slower: 8 x 2048 x 12 253 -> 269.
+// What the next kernel reads stays in the caches: the chunks' records of other head sizes written past them 220 -> 262 us at 8 x 1024 x 6 x 128,
+// the states of a decoding step 45 -> 46 (read past them as well: 53), attn_ln's kept output out of the one-kernel form 743 -> 751.
 constexpr int STREAMED = 2;   // of a buffer store
 template <class V>
 __device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontemporal_store(x, static_cast<V*>(to)); }
+template <class V>
+__device__ __forceinline__ V load_streamed(const void* from) { return __builtin_nontemporal_load(static_cast<const V*>(from)); }
 
 // Load a [16 tokens x 64 channels] tile whose row n starts at p + n*ld (elements).
 __device__ __forceinline__ TileB load_rows(const __bf16* __restrict__ p, long ld, const Lane& L) {
@@ -265,6 +270,12 @@ __device__ __forceinline__ void store_rows16(__bf16* __restrict__ p, long ld, co
 #pragma unroll
     for (int pr = 0; pr < NBLK / 2; pr++)
         *reinterpret_cast<bf16x8*>(row + 32 * pr) = __builtin_shufflevector(t.f[2 * pr], t.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+}
+__device__ __forceinline__ void store_rows16_streamed(__bf16* __restrict__ p, long ld, const Lane& L, const TileB& t) {
+    __bf16* row = p + (long)L.n * ld + 8 * L.g;
+#pragma unroll
+    for (int pr = 0; pr < NBLK / 2; pr++)
+        store_streamed(row + 32 * pr, __builtin_shufflevector(t.f[2 * pr], t.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7));
 }
 __device__ __forceinline__ void store_rows(__bf16* __restrict__ p, long ld, const Lane& L, const TileB& t) {
     __bf16* row = p + (long)L.n * ld + 4 * L.g;

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256) void ln_epilogue_bwd_kernel(int T, int H, int 
     const TileB y = load_rows16(ln.y_wkv + ca.row0, ca.ld, L);
     const LnParams p = load_ln_params(ln.params, ca.bh % H, H, L);
     const LnBackward r = ln_backward(uncentre(y, ln.centers, ca.row0 / HEAD + (long)L.n * H), q, k, v, g, dy, p);
-    store_rows16(ln.dg + ca.row0, ca.ld, L, r.dg);
+    store_rows16_streamed(ln.dg + ca.row0, ca.ld, L, r.dg);
     store_rows16(ln.dY + ca.row0, ca.ld, L, r.dy);
     store_rows16(ln.dv + ca.row0, ca.ld, L, r.dv_bonus);
     if (L.g == 0) ln.ddot[(long)cid * CHUNK + L.n] = r.ddot;

@@ -249,8 +249,8 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
             const int tok = e / ROWS, ch = e % ROWS;
             const unsigned at = (unsigned)tok * ld + (unsigned)(part * ROWS + ch);
             if (FULL || part * ROWS + ch < CR) {
-                (y + base)[at] = yout[buf][tok][ch];
-                if (sav != nullptr) (sav + base)[at] = saout[buf][tok][ch];
+                __builtin_nontemporal_store(yout[buf][tok][ch], (y + base) + at);
+                if (sav != nullptr) __builtin_nontemporal_store(saout[buf][tok][ch], (sav + base) + at);
             }
         }
     };
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
             float* const to = ckpt + ((long)bh * NC + chunk_start(n) / CH) * CR * CR;
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                if (row_ok(r)) *reinterpret_cast<f4*>(to + (state_off + r * CR)) = S[r];
+                if (row_ok(r)) __builtin_nontemporal_store(S[r], reinterpret_cast<f4*>(to + (state_off + r * CR)));
             }
         }
         // a token's operands are requested from LDS one token ahead
@@ -578,7 +578,8 @@ __global__ __launch_bounds__(64 * NW) void wkv7_f32_bwd_thin_kernel(int T, int H
 // sums does not, and in fp32 the errors would be 1.7e-7 where recomputing the states row by row left 0.9e-7.
 // Bound: memory, 90 KB per chunk and 64 columns: 8 x 1024 tokens x 12 heads of 64 152 us for 553 MB (148 with dw as that
 // difference; of 142 on another machine, 123 without the matrix instructions, 132 without the pairs of tokens, 118 without
-// either), where recomputing the states took 218; 32 x 1024 x 12 852 -> 560, 8 x 1024 x 6 heads of 128 477 -> 221, 8 x 1024 x 16 heads
+// either; 142 with the states read and the results written past the caches, a pass with its scans' stores so as well 435 -> 417), where
+// recomputing the states took 218; 32 x 1024 x 12 852 -> 560, 8 x 1024 x 6 heads of 128 477 -> 221, 8 x 1024 x 16 heads
 // of 32 157 -> 101.  Errors at 8 x 1024 x 12 against fp64: dq, dk 0.42e-7, dw 0.64e-7 (0.69 as a difference), da, db 0.98e-7.
 template <int CR, int COLS>   // head size, columns of a block
 __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, const float* __restrict__ w, const float* __restrict__ q,
@@ -630,7 +631,7 @@ __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, con
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const long at = st + (16 * u + s) * CR;
-            to.S[s] = at_bytes<f2>(ckpt + at, lane_at), to.E[s] = at_bytes<f2>(work + at, lane_at);
+            to.S[s] = __builtin_nontemporal_load(&at_bytes<f2>(ckpt + at, lane_at)), to.E[s] = __builtin_nontemporal_load(&at_bytes<f2>(work + at, lane_at));
         }
         return to;
     };
@@ -744,10 +745,10 @@ __global__ __launch_bounds__(64, 2) void wkv7_f32_grads_kernel(int T, int H, con
         }
         if (col_ok) {
             const long at = base + (long)i * ld;
-            at_bytes<float>(dq + at, lane_col) = (float)dqv[i], at_bytes<float>(da + at, lane_col) = (float)dav[i];
-            at_bytes<float>(dk + at, lane_col) = (float)dki, at_bytes<float>(db + at, lane_col) = (float)dbi;
+            __builtin_nontemporal_store((float)dqv[i], &at_bytes<float>(dq + at, lane_col)), __builtin_nontemporal_store((float)dav[i], &at_bytes<float>(da + at, lane_col));
+            __builtin_nontemporal_store((float)dki, &at_bytes<float>(dk + at, lane_col)), __builtin_nontemporal_store((float)dbi, &at_bytes<float>(db + at, lane_col));
             const double ew = dec[i] > 0.f ? es[i][lane] : 0.f;   // (exp(w) may be infinite where the decay is zero)
-            at_bytes<float>(dw + at, lane_col) = (float)(-ew * deci * R[i]);
+            __builtin_nontemporal_store((float)(-ew * deci * R[i]), &at_bytes<float>(dw + at, lane_col));
         }
     }
 }

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void ln_epilogue_kernel(int T, int H, int nchu
     const TileB g = load_rows16(g_ + ca.row0, ca.ld, L);
     const LnParams p = load_ln_params(params, ca.bh % H, H, L);
     const TileF yf = uncentre(yw, centers, ca.row0 / HEAD + (long)L.n * H);   // (row0 / 64 = token * H + head of the chunk's first token)
-    store_rows16(y_ + ca.row0, ca.ld, L, ln_forward(yf, q, k, v, g, p));
+    store_rows16_streamed(y_ + ca.row0, ca.ld, L, ln_forward(yf, q, k, v, g, p));
 }
 
 // ------------------------------------------------------------------------------------------------

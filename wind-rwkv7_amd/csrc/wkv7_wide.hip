@@ -96,7 +96,7 @@ __device__ __forceinline__ TB<NB> fragments(const RawTile<NB>& t) {
 __device__ __forceinline__ void store_pair_rows(__bf16* __restrict__ p, long ld, int i, const Lane& L, bf16x4 even, bf16x4 odd) {
     const u32x2 x = __builtin_bit_cast(u32x2, even), y = __builtin_bit_cast(u32x2, odd);
     const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false), s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-    *reinterpret_cast<u32x4*>(p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1)) = u32x4{s0[0], s1[0], s0[1], s1[1]};
+    store_streamed(p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1), u32x4{s0[0], s1[0], s0[1], s1[1]});
 }
 
 // F(X Y^T), contraction over the C channels
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
                 for (int m = 0; m < (PIECES + 64 * LW - 1) / (64 * LW); m++) {
                     const int e = ht + 64 * LW * m, jb = e / (W * 32), in = e % (W * 32);
                     __bf16* const to = kept + (jb < NB ? K::ck(cid, jb, ib0) : K::ut(cid, ib0)) + in * 8;
-                    if (e < PIECES && in / 32 < blocks) *reinterpret_cast<f32x4*>(to) = *reinterpret_cast<const f32x4*>(from + e * 16);
+                    if (e < PIECES && in / 32 < blocks) store_streamed(to, *reinterpret_cast<const f32x4*>(from + e * 16));
                 }
             }
             if constexpr (FWD) {
@@ -369,8 +369,8 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
                 for (int e = ht; e < 32 * W; e += 64 * LW) {
                     const int token = e / (2 * W), piece = e % (2 * W);
                     if (piece / 2 < blocks)
-                        *reinterpret_cast<f32x4*>(y_ + ca.row0 + (long)token * ca.ld + 16 * ib0 + 8 * piece) =
-                            *reinterpret_cast<const f32x4*>(from + KEPT_BYTES + e * 16);
+                        store_streamed(y_ + ca.row0 + (long)token * ca.ld + 16 * ib0 + 8 * piece,
+                                       *reinterpret_cast<const f32x4*>(from + KEPT_BYTES + e * 16));
                 }
                 if (centers != nullptr && ht < 16 * W) {
                     const int token = ht / W, blk = ht % W;
@@ -516,7 +516,9 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
 // in LDS, decay factors are made twice, and the next key block's states are loaded into the registers just used; that is 248
 // of 256 registers at C = 128 (all of it held: 484 and one wavefront).  With 16-byte accesses to the sequences' rows (the
 // outputs of an even key block wait in LDS for the odd one's): 110 -> 90 us at 8 x 1024 tokens x 6 heads of 128, where its 390
-// MB take 73 us at a copy's rate.
+// MB take 73 us at a copy's rate.  Kept states written and read past the caches and results written so (store_streamed), which leaves the
+// records and the sequences in them: grads 92 -> 78, the five kernels of a pass 269 -> 233, 8 x 1024 x 8 heads of 96 243 -> 190, 32 x 1024 x 6 of
+// 128 983 -> 939.
 // ------------------------------------------------------------------------------------------------
 template <int NB>
 __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks, const __bf16* __restrict__ w_,
@@ -559,8 +561,8 @@ __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks
     bf16x4 s0n[NB], dsn[NB];
 #pragma unroll
     for (int ib = 0; ib < NB; ib++) {
-        s0n[ib] = load_frag(kept_f + K::ck(cid, 0, ib), lane);
-        dsn[ib] = load_frag(kept_b + K::ck(cid, 0, ib), lane);
+        s0n[ib] = load_streamed<bf16x4>(kept_f + K::ck(cid, 0, ib) + 4 * lane);
+        dsn[ib] = load_streamed<bf16x4>(kept_b + K::ck(cid, 0, ib) + 4 * lane);
     }
     __builtin_amdgcn_sched_barrier(0);
     const TB<NB> w = fragments(w_raw), q = fragments(q_raw), k = fragments(k_raw), a = fragments(a_raw), b = fragments(b_raw), v = fragments(v_raw), dy = fragments(dy_raw);
@@ -629,8 +631,8 @@ __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks
             UdS = mma(UdS, dsT, mine[VS_U][ib][lane]);   // U dS
             VdS = mma(VdS, dsT, mine[VS_V][ib][lane]);   // V dS
             if (jb + 1 < NB) {   // into the same registers: the next key block's, a whole key block ahead of their use
-                s0n[ib] = load_frag(kept_f + K::ck(cid, jb + 1, ib), lane);
-                dsn[ib] = load_frag(kept_b + K::ck(cid, jb + 1, ib), lane);
+                s0n[ib] = load_streamed<bf16x4>(kept_f + K::ck(cid, jb + 1, ib) + 4 * lane);
+                dsn[ib] = load_streamed<bf16x4>(kept_b + K::ck(cid, jb + 1, ib) + 4 * lane);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
