@@ -229,7 +229,7 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
 // Results that no kernel reads again soon leave past the caches (non-temporal): what a kernel and the ones behind it read then stays
 // in them.  The kept states, U^T and outputs of the WKV7 scans and the gradients, forward + backward of attn, us: 12 x 1024 tokens x 12 heads
 // 197 -> 178, 16 x 1024 x 12 211 -> 198, 24 x 1024 x 12 362 -> 337, 8 x 1024 x 32 276 -> 255, 8 x 2048 x 12 257 -> 248; 8 x 1024 x 12 138 -> 137 and
-// 64 x 1024 x 12 758 -> 756 (753 with the gradients through the caches, which is 1 to 5 % slower everywhere below).
+// 64 x 1024 x 12 758 -> 753 (the gradients through the caches there: launch_bwd_grads).
 // The same at other head sizes and in fp32, whose kept states are larger: wkv7_wide.hip, wkv7_f32.hip.  Loads that way pay where a
 // kernel reads whole lines for the last time (load_streamed); of half lines they are slower: 8 x 2048 x 12 253 -> 269.
 // What the next kernel reads stays in the caches: the chunks' records of other head sizes written past them 220 -> 262 us at 8 x 1024 x 6 x 128,
