@@ -292,8 +292,8 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(int T, int H, int nchu
 // workers left in a double buffer one chunk ago to memory, 16 bytes per lane; one LDS-only barrier per chunk.
 // Forward + backward, us, against workers that fetch and store for themselves: 1 x 512 tokens x 4 heads of 128 106 -> 92,
 // 8 x 1024 x 6 heads of 128 319 -> 312, 16 x 1024 x 6 heads of 128 571 -> 554, 4 x 1024 x 5 heads of 112 161 -> 142.  Bound:
-// the kept states' 113 MB per direction at 8 x 1024 x 6 heads of 128 (without the stores the two scans together take 76 us
-// instead of 129, without the loads 98).
+// the kept states' 113 MB per direction at 8 x 1024 x 6 heads of 128 and the round of fetch, LDS and barrier (with two helpers and the
+// states through the caches 129 us for the two scans, without the stores 76, without the loads 98).
 // ------------------------------------------------------------------------------------------------
 template <int NB, bool FWD>
 struct ScanOps {
@@ -302,7 +302,11 @@ struct ScanOps {
     f32x4 fw[NB];
 };
 
-constexpr int scan_helpers(int W) { return W == 4 ? 4 : 2; }
+// Loading and storing wavefronts, half each.  A chunk's 26 KiB of operands at head size 128 are 26 loads and LDS writes, which take one
+// wavefront as long as the workers' round.  Forward + backward, us, with 2 (4 workers: 4) / 4 / 6 / 8 of them: two workers, 8 x 1024 tokens x 6
+// heads of 128 216 / 210 / 201 / 205, 8 x 1024 x 8 of 96 187 / 185 / 181 / 176; four, 16 x 1024 x 6 of 128 466 / 466 / 469 / 463, 32 x 1024 x 6 939 /
+// 937 / 938 / 933.  Beside one worker two: 1 x 2048 x 6 of 128 164 / 178, 4 x 1024 x 5 of 112 125 / 132.
+constexpr int scan_helpers(int W) { return W >= 2 ? 8 : 2; }
 
 template <int NB, bool FWD, bool KEEP, int W>
 __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
