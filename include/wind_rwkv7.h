@@ -330,6 +330,14 @@ int wind_rwkv7_expand_loras_forward(int B, int T, int C, int D, int head_size,
                                     const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
                                     const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
                                     void* w_out, void* k_out, void* kk_out, void* b_out, void* stream);
+/* The same for sequences padded to whole chunks: what wind_rwkv7_neutral_rows_keep(B, T, C, T - 16, w_out, k_out, b_out, kept) would
+ * do behind it is done with it (at rank 16 and head size 64 in the one launch).  T is a multiple of 16; kept NULL: nothing of it. */
+int wind_rwkv7_expand_loras_forward_padded(int B, int T, int C, int D, int head_size,
+                                           const void* w_in, const void* k_in,
+                                           const void* z_in, const void* a_in, const void* ma_in, const void* mk_in,
+                                           const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
+                                           const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
+                                           void* w_out, void* k_out, void* kk_out, void* b_out, void* kept, void* stream);
 int wind_rwkv7_expand_loras_backward(int B, int T, int C, int D, int head_size,
                                      const void* w_in, const void* k_in,
                                      const void* z_in, const void* a_in, const void* ma_in, const void* mk_in,

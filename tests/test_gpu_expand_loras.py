@@ -120,3 +120,25 @@ def test_expand_loras_rejects_unsupported():
     assert lib.wind_rwkv7_expand_loras_forward(1, 16, 128, 16, 96, *p, None) == 9   # heads that do not tile the channels
     assert lib.wind_rwkv7_expand_loras_forward(1, 16, 64, 8, 64, *p, None) == 8
     assert lib.wind_rwkv7_expand_loras_forward(1, 16, 96, 16, 64, *p, None) == 9
+
+
+@pytest.mark.parametrize('B,T,C,D,N', [(1, 16, 64, 16, 64), (3, 48, 128, 16, 64), (5, 80, 192, 16, 64), (2, 1008, 768, 16, 64),
+                                       (2, 48, 128, 32, 64), (2, 32, 192, 16, 48)])
+def test_padded_sequences_give_the_bits_of_two_calls(B, T, C, D, N):
+    """The last chunk of every sequence neutral in the outputs and as it is in `kept`, in the one launch at rank 16 and head size 64."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    gen = torch.Generator().manual_seed(T + C)
+    rn = lambda *shape: torch.randn(*shape, generator=gen).bfloat16().to(DEV)
+    ins = [rn(B, T, C), rn(B, T, C)] + [rn(B, T, D) for _ in range(4)] + [rn(C, D) for _ in range(4)] + [rn(C) for _ in range(4)]
+    stream = torch.cuda.current_stream().cuda_stream
+    ptrs = [t.data_ptr() for t in ins]
+    new = lambda: ([torch.full_like(ins[0], float('nan')) for _ in range(4)], torch.full((3, B, 16, C), float('nan'), dtype=torch.bfloat16, device=DEV))
+    (one, kept1), (two, kept2) = new(), new()
+    at = lambda ts: [t.data_ptr() for t in ts]
+    _native.check(lib.wind_rwkv7_expand_loras_forward_padded(B, T, C, D, N, *ptrs, *at(one), kept1.data_ptr(), stream))
+    _native.check(lib.wind_rwkv7_expand_loras_forward(B, T, C, D, N, *ptrs, *at(two), stream))
+    _native.check(lib.wind_rwkv7_neutral_rows_keep(B, T, C, T - 16, two[0].data_ptr(), two[1].data_ptr(), two[3].data_ptr(), kept2.data_ptr(), stream))
+    torch.cuda.synchronize()
+    for a, b in zip(one + [kept1], two + [kept2]):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

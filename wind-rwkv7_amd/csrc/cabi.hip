@@ -658,8 +658,19 @@ int wind_rwkv7_expand_loras_forward(int B, int T, int C, int D, int head_size,
                                     const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
                                     const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
                                     void* w_out, void* k_out, void* kk_out, void* b_out, void* stream) {
+    return wind_rwkv7_expand_loras_forward_padded(B, T, C, D, head_size, w_in, k_in, z_in, a_in, ma_in, mk_in, Wz, Wa, Wma, Wmk, w_bias, a_bias,
+                                                  ma_bias, mk_bias, w_out, k_out, kk_out, b_out, nullptr, stream);
+}
+
+int wind_rwkv7_expand_loras_forward_padded(int B, int T, int C, int D, int head_size,
+                                           const void* w_in, const void* k_in,
+                                           const void* z_in, const void* a_in, const void* ma_in, const void* mk_in,
+                                           const void* Wz, const void* Wa, const void* Wma, const void* Wmk,
+                                           const void* w_bias, const void* a_bias, const void* ma_bias, const void* mk_bias,
+                                           void* w_out, void* k_out, void* kk_out, void* b_out, void* kept, void* stream) {
     const int rc = check_loras(B, T, C, D, head_size);
     if (rc) return rc;
+    if (kept && T % wkv::CHUNK != 0) return WIND_RWKV7_ERR_BAD_SHAPE;
     const void* const acts[4] = {z_in, a_in, ma_in, mk_in};
     const void* const Ws[4] = {Wz, Wa, Wma, Wmk};
     const void* const biases[4] = {w_bias, a_bias, ma_bias, mk_bias};
@@ -667,7 +678,10 @@ int wind_rwkv7_expand_loras_forward(int B, int T, int C, int D, int head_size,
     if (!w_in || !k_in) return WIND_RWKV7_ERR_NULL_POINTER;
     for (int i = 0; i < 4; i++)
         if (!acts[i] || !Ws[i] || !biases[i] || !outs[i]) return WIND_RWKV7_ERR_NULL_POINTER;
-    wkv::launch_expand_loras_forward((long)B * T, C, D, head_size, w_in, k_in, acts, Ws, biases, outs, static_cast<hipStream_t>(stream));
+    const bool here = kept && D == 16 && head_size == wkv::HEAD && (long long)B * T / wkv::CHUNK <= 0x7fffffffLL;
+    wkv::launch_expand_loras_forward((long)B * T, C, D, head_size, w_in, k_in, acts, Ws, biases, outs, static_cast<hipStream_t>(stream),
+                                     here ? T : 0, here ? kept : nullptr);
+    if (kept && !here) return wind_rwkv7_neutral_rows_keep(B, T, C, T - wkv::CHUNK, w_out, k_out, b_out, kept, stream);
     return launch_status();
 }
 

@@ -564,7 +564,7 @@ size_t expand_loras_bwd_workspace_least_bytes(long M, int C, int D) {
 
 void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in, const void* k_in, const void* const acts[4],
                                  const void* const Ws[4], const void* const biases[4], void* const outs[4],
-                                 hipStream_t stream) {
+                                 hipStream_t stream, int padded_T, void* kept) {
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
     auto m = [](void* p) { return static_cast<__bf16*>(p); };
     const LoraIn in{{c(acts[0]), c(acts[1]), c(acts[2]), c(acts[3])}};
@@ -615,7 +615,7 @@ void launch_expand_loras_forward(long M, int C, int D, int HS, const void* w_in,
                        m(outs[1]), m(outs[2]), m(outs[3]))
     if (D == 16) {
         __bf16* const o[4] = {m(outs[0]), m(outs[1]), m(outs[2]), m(outs[3])};
-        launch_loras16_forward(M, C, c(w_in), c(k_in), in, lw, o, stream);
+        launch_loras16_forward(M, C, c(w_in), c(k_in), in, lw, o, stream, padded_T, kept);
     } else if (D == 32) WKV_LAUNCH_FWD(2);
     else WKV_LAUNCH_FWD(4);
 #undef WKV_LAUNCH_FWD

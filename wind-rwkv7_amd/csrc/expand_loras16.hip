@@ -21,11 +21,21 @@ constexpr int REC = 4 * HEAD * D + 4 * HEAD;   // floats of a partial record: dW
 // either two or three: 18.9 and 19.6 at 7056).  The bytes are 13, 15, 30, 30 at the rate of a copy, the instructions, a fifth of
 // them transcendental, 11 at 8192 x 768.
 // ------------------------------------------------------------------------------------------------
+// PADDED: a sequence's last chunk belongs to the tokens behind its whole chunks (`kept`, [3][sequences][16][C], takes its w, k and b) and
+// gets what leaves the recurrence's state as it is instead: decay 1, k = b = 0.  (As a launch of its own behind this one a prompt of
+// 2 x 1003 tokens took 113.9 us, so 111.8.)
+struct PaddedRows {
+    int chunks;   // of a sequence
+    long plane;
+    __bf16* kept;
+};
+template <bool PADDED>
 __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, int tiles_per_split,
                                                                  const __bf16* __restrict__ w_in,
                                                                  const __bf16* __restrict__ k_in, LoraIn in, LoraW lw,
                                                                  __bf16* __restrict__ w_out, __bf16* __restrict__ k_out,
-                                                                 __bf16* __restrict__ kk_out, __bf16* __restrict__ b_out) {
+                                                                 __bf16* __restrict__ kk_out, __bf16* __restrict__ b_out,
+                                                                 const PaddedRows padded) {
     __shared__ bf16x4 sW[4 * NBLK][WAVE];    // F(W_i[c0 + 16cb .., :])    lane = channel, reg = rank index
     __shared__ __attribute__((aligned(16))) float sBias[4][HEAD];
     __shared__ bf16x8 s_tile[4][2][TOK * 8];
@@ -66,7 +76,17 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
     sBias[wave][lane] = (float)lw.bias[wave][c0 + lane];
     __syncthreads();
     auto bias4 = [&](int i, int cb) { return *reinterpret_cast<const f32x4*>(&sBias[i][chan16(cb, 4 * L.g)]); };
-    auto store = [&](__bf16* p0, const TileB& t0, __bf16* p1, const TileB& t1, long off) {   // two tiles
+    bool last = false;   // PADDED: this tile is a sequence's last chunk
+    long kept_at = 0;
+    auto put = [&](__bf16* p, unsigned bytes, int plane, bf16x8 v) {   // plane: w, k, b, or negative
+        if (PADDED && last && plane >= 0) {
+            piece_at(padded.kept + (plane * padded.plane + kept_at), bytes) = v;
+            const __bf16 none = (__bf16)(plane == 0 ? -80.f : 0.f);
+            v = (bf16x8){none, none, none, none, none, none, none, none};
+        }
+        piece_at(p, bytes) = v;
+    };
+    auto store = [&](__bf16* p0, const TileB& t0, int plane0, __bf16* p1, const TileB& t1, int plane1, long off) {   // two tiles
 #pragma unroll
         for (int pr = 0; pr < 2; pr++) {
             buf[0][piece_slot(L.n, 4 * pr + L.g)] = join(t0.f[2 * pr], t0.f[2 * pr + 1]);
@@ -75,13 +95,18 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
         wave_lds_order();
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            piece_at(p0 + off, lane_bytes + 8 * i * row_bytes) = buf[0][piece_slot(l8 + 8 * i, piece)];
-            piece_at(p1 + off, lane_bytes + 8 * i * row_bytes) = buf[1][piece_slot(l8 + 8 * i, piece)];
+            put(p0 + off, lane_bytes + 8 * i * row_bytes, plane0, buf[0][piece_slot(l8 + 8 * i, piece)]);
+            put(p1 + off, lane_bytes + 8 * i * row_bytes, plane1, buf[1][piece_slot(l8 + 8 * i, piece)]);
         }
         wave_lds_order();
     };
     for (; tile < tile_end; tile += 4) {
         const long off = tile * TOK * C + c0;
+        if constexpr (PADDED) {
+            const int sequence = (int)tile / padded.chunks;
+            last = (int)tile - sequence * padded.chunks == padded.chunks - 1;
+            kept_at = (long)sequence * TOK * C + c0;
+        }
         bf16x4 act[4];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
@@ -130,7 +155,7 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
             wo.f[cb] = to_bf16(w);
             ko.f[cb] = to_bf16(k);
         }
-        store(w_out, wo, k_out, ko, off);
+        store(w_out, wo, 0, k_out, ko, 1, off);
         const float inorm = rsqrtf(fmaxf(group_sum(ss), 1e-12f));
         TileB kko, bo;
 #pragma unroll
@@ -139,7 +164,7 @@ __global__ __launch_bounds__(256) void expand_loras_fwd16_kernel(long M, int C, 
             kko.f[cb] = to_bf16(kk);
             bo.f[cb] = to_bf16(-kk * a.f[cb]);
         }
-        store(kk_out, kko, b_out, bo, off);
+        store(kk_out, kko, -1, b_out, bo, 2, off);
     }
 }
 
@@ -503,7 +528,7 @@ int lora16_splits(long M, int H) {
 }
 
 void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, __bf16* const outs[4],
-                            hipStream_t stream) {
+                            hipStream_t stream, int padded_T, void* kept) {
     // three blocks fit a compute unit, all of them in one round; at least four token tiles (one per wavefront) each
     const int H = C / HEAD;
     const long ntiles = M / TOK;
@@ -511,8 +536,12 @@ void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_i
     if (nsplit > ntiles / 4) nsplit = ntiles / 4;
     if (nsplit < 1) nsplit = 1;
     const int tiles_per_split = (int)((ntiles + nsplit - 1) / nsplit);
-    hipLaunchKernelGGL(expand_loras_fwd16_kernel, dim3(H, (unsigned)nsplit), dim3(256), 0, stream, M, C, tiles_per_split, w_in, k_in, in,
-                       lw, outs[0], outs[1], outs[2], outs[3]);
+    const PaddedRows padded{padded_T / TOK, kept ? M / padded_T * TOK * C : 0, static_cast<__bf16*>(kept)};
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(H, (unsigned)nsplit), dim3(256), 0, stream, M, C, tiles_per_split, w_in, k_in, in, lw, outs[0],
+                           outs[1], outs[2], outs[3], padded);
+    };
+    kept ? go(expand_loras_fwd16_kernel<true>) : go(expand_loras_fwd16_kernel<false>);
 }
 
 void launch_loras16_backward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, const LoraDy& dy,

@@ -87,7 +87,7 @@ __device__ __forceinline__ f32x4 load_bias(const __bf16* __restrict__ b, int c, 
 // the rank-16 kernels (expand_loras16.hip); forward: heads of 64 channels; splits: blocks of the backward kernel per head
 int lora16_splits(long M, int H);
 void launch_loras16_forward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, __bf16* const outs[4],
-                            hipStream_t stream);
+                            hipStream_t stream, int padded_T = 0, void* kept = nullptr);
 // din: the heads' shares of the four d*_in, [M, H, 2, 16 / 4, 2, 4]: rank index 4g + r of i = 2 half + e at [half][g][e][r].
 // stats not null: the norm of each (token, head of HS channels) is read instead of summed over 64 channels
 void launch_loras16_backward(long M, int C, const __bf16* w_in, const __bf16* k_in, const LoraIn& in, const LoraW& lw, const LoraDy& dy,

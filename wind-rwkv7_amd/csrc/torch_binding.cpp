@@ -38,8 +38,8 @@ namespace py = pybind11;
     X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward_split)                       \
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
-    X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_backward) X(cast_to_bf16)             \
-    X(ddlerp_first_workspace_bytes) X(ddlerp_first) X(neutral_rows_keep) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
+    X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_forward_padded) X(expand_loras_backward) X(cast_to_bf16)             \
+    X(ddlerp_first_workspace_bytes) X(ddlerp_first) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(block_wgrads_workspace_bytes) X(block_wgrads) X(mixer_decode_workspace_bytes) X(mixer_decode) \
     X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
 
@@ -799,14 +799,12 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
         second.add(a(A.tw1), w(DECAY_W2), R_DECAY, C), second.to(a(A.w2), C);
         second.run(M, xb);
     }
-    check(L.expand_loras_forward(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2), w(MA_W2),
-                                 w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b), stream));
     const int whole = (int)(valid / 16 * 16), rest = (int)(valid - whole);
     Tensor kept;
-    if (rest && whole) {
-        kept = at::empty({3, B, T - whole, C}, xb.options());
-        check(L.neutral_rows_keep(B, T, C, whole, a(A.w), a(A.k2), a(A.b), ptr(kept), stream));
-    }
+    if (rest && whole) kept = at::empty({3, B, T - whole, C}, xb.options());   // (T is valid rounded up: the last chunk)
+    check(L.expand_loras_forward_padded(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2),
+                                        w(MA_W2), w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b),
+                                        kept.defined() ? ptr(kept) : nullptr, stream));
     if (whole) {
         const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
         check((save ? L.attn_ln_forward : L.attn_ln_prefill)(

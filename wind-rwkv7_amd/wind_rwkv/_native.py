@@ -72,6 +72,7 @@ SIGNATURES = {
     'wind_rwkv7_expand_loras_rank_supported': (_i, [_i]),
     'wind_rwkv7_expand_loras_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_expand_loras_forward': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp]),
+    'wind_rwkv7_expand_loras_forward_padded': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 5 + [_vp]),
     'wind_rwkv7_expand_loras_backward': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp] * 14 + [_vp, _sz, _vp]),
     'wind_rwkv7_expand_loras_backward_to': (_i, [_i] * 5 + [_vp] * 14 + [_vp] * 4 + [_vp] * 7 + [_vp] * 8 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_f32_saved_bytes': (_sz, [_i] * 4),
