@@ -229,7 +229,7 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
 // Results that no kernel reads again soon leave past the caches (non-temporal): what a kernel and the ones behind it read then stays
 // in them.  The kept states, U^T and outputs of the WKV7 scans and the gradients, forward + backward of attn, us: 12 x 1024 tokens x 12 heads
 // 197 -> 178, 16 x 1024 x 12 211 -> 198, 24 x 1024 x 12 362 -> 337, 8 x 1024 x 32 276 -> 255, 8 x 2048 x 12 257 -> 248; 8 x 1024 x 12 138 -> 137 and
-// 64 x 1024 x 12 758 -> 753 (the gradients through the caches there: launch_bwd_grads).
+// 64 x 1024 x 12 758 -> 730-741, of these the gradients as whole lines: half a line at a time is slower past the caches there (757) than through them.
 // The same at other head sizes and in fp32, whose kept states are larger: wkv7_wide.hip, wkv7_f32.hip.  Loads that way pay where a
 // kernel reads whole lines for the last time (load_streamed); of half lines they are slower: 8 x 2048 x 12 253 -> 269.
 // What the next kernel reads stays in the caches: the chunks' records of other head sizes written past them 220 -> 262 us at 8 x 1024 x 6 x 128,
@@ -271,11 +271,28 @@ __device__ __forceinline__ void store_rows16(__bf16* __restrict__ p, long ld, co
     for (int pr = 0; pr < NBLK / 2; pr++)
         *reinterpret_cast<bf16x8*>(row + 32 * pr) = __builtin_shufflevector(t.f[2 * pr], t.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7);
 }
-__device__ __forceinline__ void store_rows16_streamed(__bf16* __restrict__ p, long ld, const Lane& L, const TileB& t) {
-    __bf16* row = p + (long)L.n * ld + 8 * L.g;
+// A tile in the order of load_rows16 as whole lines: a lane holds pieces g and 4 + g of row n, so lanes n and n + 8 change one each (row_ror 8;
+// the banks of lanes 8 .. 15, then of 0 .. 7), and eight lanes of rows 0 .. 7, then of 8 .. 15, have the 128 bytes of a row together.
+struct WholeLines {
+    i32x4 top, bottom;
+    __device__ __forceinline__ explicit WholeLines(const TileB& t) {
+        const i32x4 lo = __builtin_bit_cast(i32x4, __builtin_shufflevector(t.f[0], t.f[1], 0, 1, 2, 3, 4, 5, 6, 7));
+        const i32x4 hi = __builtin_bit_cast(i32x4, __builtin_shufflevector(t.f[2], t.f[3], 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-    for (int pr = 0; pr < NBLK / 2; pr++)
-        store_streamed(row + 32 * pr, __builtin_shufflevector(t.f[2 * pr], t.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+        for (int i = 0; i < 4; i++) {
+            top[i] = __builtin_amdgcn_update_dpp(lo[i], hi[i], 0x128, 0xf, 0xc, false);
+            bottom[i] = __builtin_amdgcn_update_dpp(hi[i], lo[i], 0x128, 0xf, 0x3, false);
+        }
+    }
+    // of `top`; `bottom`'s row is eight behind
+    static __device__ __forceinline__ int row(const Lane& L) { return L.n & 7; }
+    static __device__ __forceinline__ int piece(const Lane& L) { return L.g + 4 * (L.n >> 3); }
+};
+__device__ __forceinline__ void store_rows16_streamed(__bf16* __restrict__ p, long ld, const Lane& L, const TileB& t) {
+    const WholeLines x(t);
+    __bf16* const to = p + WholeLines::row(L) * ld + 8 * WholeLines::piece(L);
+    store_streamed(to, x.top);
+    store_streamed(to + 8 * ld, x.bottom);
 }
 __device__ __forceinline__ void store_rows(__bf16* __restrict__ p, long ld, const Lane& L, const TileB& t) {
     __bf16* row = p + (long)L.n * ld + 4 * L.g;

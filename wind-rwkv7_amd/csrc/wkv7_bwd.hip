@@ -19,8 +19,6 @@
 #include "wkv7_common.hpp"
 #include "wkv7_kernels.hpp"
 
-#include <type_traits>
-
 namespace wkv {
 
 // ------------------------------------------------------------------------------------------------
@@ -145,7 +143,7 @@ __device__ __forceinline__ bf16x4 state_t(const unsigned char* p, int ib, int jb
 }
 }   // namespace pairlds
 
-template <bool LN, int MODE, bool PAST>   // PAST: results past the caches
+template <bool LN, int MODE>
 __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunks,
                                                         const __bf16* __restrict__ w_, const __bf16* __restrict__ q_,
                                                         const __bf16* __restrict__ k_, const __bf16* __restrict__ v_,
@@ -232,13 +230,23 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         }
         return x;
     };
-    auto put16 = [&](__bf16* t, long row0, const TileB& x) {          // store_rows16
+    // Whole lines (see WholeLines): as half lines past the caches 73.7 MB of gradients at 8 x 1024 tokens x 12 heads reached memory as 80.4,
+    // and forward + backward of attn took, us: 16 x 1024 x 12 199 (now 192), 32 x 1024 x 12 411 (397), 64 x 1024 x 12 757 (through the caches
+    // 752, now 730-741), 1 x 16384 x 32 680 (670), 8 x 2048 x 12 247 (241).
+    const unsigned put_off = (unsigned)(WholeLines::row(L) * H * HEAD) * 2 + 16 * WholeLines::piece(L);
+    auto put16 = [&](__bf16* t, long row0, const TileB& x) {
         const Rsrc r = rs(t + row0);
+        if constexpr (LN) {   // (no registers to spare: as whole lines 184 -> 184.5 us, 307 -> 309)
 #pragma unroll
-        for (int pr = 0; pr < NBLK / 2; pr++)
-            __builtin_amdgcn_raw_buffer_store_b128(
-                __builtin_bit_cast(i32x4, __builtin_shufflevector(x.f[2 * pr], x.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7)), r,
-                voff_n + 16 * L.g + 64 * pr, 0, PAST ? STREAMED : 0);
+            for (int pr = 0; pr < NBLK / 2; pr++)
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    __builtin_bit_cast(i32x4, __builtin_shufflevector(x.f[2 * pr], x.f[2 * pr + 1], 0, 1, 2, 3, 4, 5, 6, 7)), r,
+                    voff_n + 16 * L.g + 64 * pr, 0, STREAMED);
+            return;
+        }
+        const WholeLines x2(x);
+        __builtin_amdgcn_raw_buffer_store_b128(x2.top, r, put_off, 0, STREAMED);
+        __builtin_amdgcn_raw_buffer_store_b128(x2.bottom, r, put_off, 8 * H * HEAD * 2, STREAMED);
     };
     auto frags4 = [&](const __bf16* p, int ln) {                      // load_frags: four fragments, [i][lane] x 8 B
         TileB x;
@@ -658,20 +666,13 @@ void launch_bwd_grads(int B, int T, int H, const void* w, const void* q, const v
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k), c(v), c(a), c(b),
                            c(dy), c(rec_fwd), c(rec_bwd), m(dw), m(dq), m(dk), m(dv), m(da), m(db), ln_params, ln_ddot, ds_run);
     };
-    auto form = [&](auto past_caches) {
-        constexpr bool PAST = decltype(past_caches)::value;
-        if (fused == 3) {
-            if (ln_params) go(bwd_grads_kernel<true, 3, PAST>);
-            else go(bwd_grads_kernel<false, 3, PAST>);
-        } else {
-            if (ln_params) go(bwd_grads_kernel<true, 1, PAST>);
-            else go(bwd_grads_kernel<false, 1, PAST>);
-        }
-    };
-    // The gradients past the caches (forward + backward, us, without -> with): 8192 chunks 143 -> 141, 12288 209 -> 198, 32768 (1 x 16384 x 32)
-    // 689 -> 684; but 49152 753 -> 756 (why not there is not known: the line is where the measurements change sides).
-    if (nchunks <= 40960) form(std::true_type());
-    else form(std::false_type());
+    if (fused == 3) {
+        if (ln_params) go(bwd_grads_kernel<true, 3>);
+        else go(bwd_grads_kernel<false, 3>);
+    } else {
+        if (ln_params) go(bwd_grads_kernel<true, 1>);
+        else go(bwd_grads_kernel<false, 1>);
+    }
 }
 
 int dstate_run(int B, int T, int H) {

@@ -428,7 +428,7 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
         // ------------------------------------------------------------------------------------------------
         unsigned char* const saved = reinterpret_cast<unsigned char*>(A.saved);
         const long row_ld = (long)A.H * HEAD;
-        const long y_lane = ((long)(bh / A.H) * A.T + L.n) * row_ld + (long)(bh % A.H) * HEAD + 32 * (vb0 / 2) + 8 * L.g;   // elements
+        const long y_head = (long)(bh / A.H) * A.T * row_ld + (long)(bh % A.H) * HEAD;   // elements
         for (int k = 1; k <= STEPS; k++) {
             STEP_BARRIER();
             const int st = k - (P + 3);
@@ -461,9 +461,16 @@ __device__ __forceinline__ void fused_block(const FusedArgs& A, unsigned char* c
             }
             if constexpr (FWD && !LN) {
                 // y by rows: a lane's 16 bytes are the fragments of value blocks 2p and 2p + 1 (8 contiguous channels)
+                if constexpr (NCH == 4) {   // whole lines: eight lanes a row
 #pragma unroll
-                for (int pp = 0; pp < NCH / 2; pp++)
-                    store_streamed(A.y + y_lane + (long)c * CHUNK * row_ld + 32 * pp, piece(out_y(NCH) + pp * 1024));
+                    for (int i = 0; i < 2; i++) {
+                        const int row = 8 * i + (lane >> 3), pc = lane & 7;
+                        store_streamed(A.y + y_head + (long)(c * CHUNK + row) * row_ld + 8 * pc,
+                                       *reinterpret_cast<const bf16x8*>(o + out_y(NCH) + (pc >> 2) * 1024 + (16 * (pc & 3) + row) * 16));
+                    }
+                } else {
+                    store_streamed(A.y + y_head + (long)(c * CHUNK + L.n) * row_ld + 32 * (vb0 / 2) + 8 * L.g, piece(out_y(NCH)));
+                }
                 if (A.centers != nullptr && lane < 16) {   // token `lane`: the centres of this block's value blocks
                     float* dst = A.centers + 4 * (((long)(bh / A.H) * A.T + c * CHUNK + lane) * A.H + bh % A.H) + vb0;
                     const float* src = reinterpret_cast<const float*>(o + out_cen(NCH)) + lane * NCH;
