@@ -116,10 +116,11 @@ int wind_rwkv7_attn_prefill(int B, int T, int H, int C, int io_dtype, int state_
                             void* workspace, size_t workspace_bytes, void* stream);
 
 /* wind_rwkv7_attn_prefill for callers that cannot allocate or pass device scratch: code under HIP-graph capture,
- * tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The scratch and
- * workspace of wind_rwkv7_attn_prefill live in a device array that is part of the library's code object
- * (WIND_RWKV7_STATIC_SCRATCH_BYTES per GPU, held from the library's load on that GPU until the process ends), so the
- * call allocates nothing and takes inputs and outputs only.  y and sT are bit-identical to wind_rwkv7_attn_prefill.
+ * tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The
+ * workspace of wind_rwkv7_attn_prefill lives in a device array that is part of the library's code object
+ * (WIND_RWKV7_STATIC_ARRAY_BYTES per GPU, held from the library's load on that GPU until the process ends), so the
+ * call allocates nothing and takes inputs and outputs only.  y and sT are bit-identical to wind_rwkv7_attn_prefill with a
+ * workspace of the size that its query asks for.
  * Limit: wind_rwkv7_attn_prefill_static_bytes(B,T,H,C) <= WIND_RWKV7_STATIC_SCRATCH_BYTES (about 3200 chunks of
  * 16 tokens x heads, e.g. B*H*T <= 52 000 at C = 64), else WIND_RWKV7_ERR_STATIC_LIMIT and nothing is enqueued.
  * All calls on one GPU share that GPU's array: two calls whose kernels may overlap in time (different streams, or
@@ -127,6 +128,7 @@ int wind_rwkv7_attn_prefill(int B, int T, int H, int C, int io_dtype, int state_
  * The array's device address is looked up once per GPU, by the first wind_rwkv7_attn_prefill_static_bytes or
  * wind_rwkv7_attn_prefill_static call with that GPU current: make that first call outside a graph capture. */
 #define WIND_RWKV7_STATIC_SCRATCH_BYTES (32u << 20)
+#define WIND_RWKV7_STATIC_ARRAY_BYTES (44u << 20)   /* what the largest problem within that limit takes, 3276 chunks by records */
 size_t wind_rwkv7_attn_prefill_static_bytes(int B, int T, int H, int C);
 int wind_rwkv7_attn_prefill_static(int B, int T, int H, int C, int io_dtype, int state_dtype,
                                    const void* w, const void* q, const void* k, const void* v,

@@ -24,7 +24,7 @@
 // address until the process ends.  In host code the array's NAME is only a handle for hipGetSymbolAddress - the
 // device address is looked up once per device (with that device current) and only that pointer is ever handed to a
 // kernel, a copy or a memset.
-static __device__ __align__(256) unsigned char scratch[WIND_RWKV7_STATIC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[WIND_RWKV7_STATIC_ARRAY_BYTES];
 
 namespace {
 
@@ -261,11 +261,12 @@ int wind_rwkv7_attn_prefill_static(int B, int T, int H, int C, int io_dtype, int
         return WIND_RWKV7_ERR_STATIC_LIMIT;
     char* base = static_cast<char*>(static_scratch());
     if (!base) return WIND_RWKV7_ERR_LAUNCH;
-    // the scratch of the saved tensor's size first, the workspace behind it: all there is, so that the scan runs by records
-    // where they fit.  Nothing has to start at zero.
-    const size_t rec = rec_fwd_bytes(B, T, H);
-    return attn_forward(B, T, H, C, io_dtype, state_dtype, w, q, k, v, a, b, s0, y, base, sT, base + rec,
-                        (size_t)WIND_RWKV7_STATIC_SCRATCH_BYTES - rec, 0, stream);
+    // The whole array is the workspace (a pass that keeps nothing stores nothing in `s`), and no more of it than
+    // wind_rwkv7_attn_prefill's query asks for: the scan plans by that size, and another plan gives other roundings.
+    // Nothing has to start at zero.
+    const size_t ws = fwd_ws_bytes(B, T, H);
+    if (ws > (size_t)WIND_RWKV7_STATIC_ARRAY_BYTES) return WIND_RWKV7_ERR_STATIC_LIMIT;   // (no problem within the limit above)
+    return attn_forward(B, T, H, C, io_dtype, state_dtype, w, q, k, v, a, b, s0, y, base, sT, base, ws, 0, stream);
 }
 
 int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state_dtype,
