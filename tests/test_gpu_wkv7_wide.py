@@ -127,3 +127,16 @@ def test_strongly_coupled_tokens(c_oracle, C, corr, gate):
     d['b'] = (gate * kk).bfloat16()
     d['w'] = (-4.0 - 2.0 * torch.rand(B, T, H, C, generator=gen)).bfloat16()
     print(check(run_device(d, torch.float32), run_oracle(c_oracle, d, torch.float32)), flush=True)
+
+
+@pytest.mark.parametrize('B,T,H,C', [(4, 1024, 48, 16), (8, 1024, 48, 16), (6, 1024, 9, 80), (4, 1024, 8, 96), (8, 1024, 8, 96), (5, 1024, 6, 128),
+                                     (8, 1024, 6, 128)])
+def test_sequences_do_not_depend_on_their_number(B, T, H, C):
+    """Both sides of the lines from which kept states (104, 204 and 208 MiB) and at 96 and 128 channels gradients go past the caches
+    (162, 325, 233 and 373).  A batch gives the bits of its sequences one by one, which are below every line."""
+    d = inputs.wkv7_inputs(B, T, H, C, seed=B + C, dtype=torch.bfloat16, s0_scale=0.3, dsT_scale=0.3)
+    whole = run_device(d, torch.float32)
+    for i in (0, B - 1):
+        one = run_device({n: t[i:i + 1].contiguous() for n, t in d.items()}, torch.float32)
+        for n, t in one.items():
+            assert torch.isfinite(t).all() and torch.equal(t, whole[n][i:i + 1]), (i, n)

@@ -93,10 +93,14 @@ __device__ __forceinline__ TB<NB> fragments(const RawTile<NB>& t) {
 }
 
 // fragments 2i and 2i + 1 to memory, 16 bytes per lane: the same swap is its own inverse
+template <bool PAST>
 __device__ __forceinline__ void store_pair_rows(__bf16* __restrict__ p, long ld, int i, const Lane& L, bf16x4 even, bf16x4 odd) {
     const u32x2 x = __builtin_bit_cast(u32x2, even), y = __builtin_bit_cast(u32x2, odd);
     const auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false), s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-    store_streamed(p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1), u32x4{s0[0], s1[0], s0[1], s1[1]});
+    const u32x4 both = {s0[0], s1[0], s0[1], s1[1]};
+    __bf16* const to = p + (long)L.n * ld + 32 * i + 16 * (L.g & 1) + 8 * (L.g >> 1);
+    if constexpr (PAST) store_streamed(to, both);
+    else *reinterpret_cast<u32x4*>(to) = both;
 }
 
 // F(X Y^T), contraction over the C channels
@@ -308,7 +312,7 @@ struct ScanOps {
 // 937 / 938 / 933.  Beside one worker two: 1 x 2048 x 6 of 128 164 / 178, 4 x 1024 x 5 of 112 125 / 132.
 constexpr int scan_helpers(int W) { return W >= 2 ? 8 : 2; }
 
-template <int NB, bool FWD, bool KEEP, int W>
+template <int NB, bool FWD, bool KEEP, int W, bool PAST>
 __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
                                                                           const void* __restrict__ s_in, void* __restrict__ s_out,
                                                                           __bf16* __restrict__ y_, __bf16* __restrict__ kept,
@@ -364,7 +368,11 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
                 for (int m = 0; m < (PIECES + 64 * LW - 1) / (64 * LW); m++) {
                     const int e = ht + 64 * LW * m, jb = e / (W * 32), in = e % (W * 32);
                     __bf16* const to = kept + (jb < NB ? K::ck(cid, jb, ib0) : K::ut(cid, ib0)) + in * 8;
-                    if (e < PIECES && in / 32 < blocks) store_streamed(to, *reinterpret_cast<const f32x4*>(from + e * 16));
+                    if (e < PIECES && in / 32 < blocks) {
+                        const f32x4 x = *reinterpret_cast<const f32x4*>(from + e * 16);
+                        if constexpr (PAST) store_streamed(to, x);
+                        else *reinterpret_cast<f32x4*>(to) = x;
+                    }
                 }
             }
             if constexpr (FWD) {
@@ -522,9 +530,9 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
 // outputs of an even key block wait in LDS for the odd one's): 110 -> 90 us at 8 x 1024 tokens x 6 heads of 128, where its 390
 // MB take 73 us at a copy's rate.  Kept states written and read past the caches and results written so (store_streamed), which leaves the
 // records and the sequences in them: grads 92 -> 78, the five kernels of a pass 269 -> 233, 8 x 1024 x 8 heads of 96 243 -> 190, 32 x 1024 x 6 of
-// 128 983 -> 939.
+// 128 983 -> 939.  What goes that way when: PastCaches.
 // ------------------------------------------------------------------------------------------------
-template <int NB>
+template <int NB, bool KEPT_PAST, bool OUT_PAST>
 __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks, const __bf16* __restrict__ w_,
                                                     const __bf16* __restrict__ q_, const __bf16* __restrict__ k_,
                                                     const __bf16* __restrict__ v_, const __bf16* __restrict__ a_,
@@ -562,11 +570,15 @@ __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks
         DT.f[ib] = load_frag(kept_b + K::ut(cid, ib), lane);   // F(D_ib^T)
     }
     // the state fragments of key block jb + 1 are requested while block jb is worked on
+    auto kept_frag = [&](const __bf16* p) {
+        if constexpr (KEPT_PAST) return load_streamed<bf16x4>(p + 4 * lane);
+        else return load_frag(p, lane);
+    };
     bf16x4 s0n[NB], dsn[NB];
 #pragma unroll
     for (int ib = 0; ib < NB; ib++) {
-        s0n[ib] = load_streamed<bf16x4>(kept_f + K::ck(cid, 0, ib) + 4 * lane);
-        dsn[ib] = load_streamed<bf16x4>(kept_b + K::ck(cid, 0, ib) + 4 * lane);
+        s0n[ib] = kept_frag(kept_f + K::ck(cid, 0, ib));
+        dsn[ib] = kept_frag(kept_b + K::ck(cid, 0, ib));
     }
     __builtin_amdgcn_sched_barrier(0);
     const TB<NB> w = fragments(w_raw), q = fragments(q_raw), k = fragments(k_raw), a = fragments(a_raw), b = fragments(b_raw), v = fragments(v_raw), dy = fragments(dy_raw);
@@ -635,8 +647,8 @@ __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks
             UdS = mma(UdS, dsT, mine[VS_U][ib][lane]);   // U dS
             VdS = mma(VdS, dsT, mine[VS_V][ib][lane]);   // V dS
             if (jb + 1 < NB) {   // into the same registers: the next key block's, a whole key block ahead of their use
-                s0n[ib] = load_streamed<bf16x4>(kept_f + K::ck(cid, jb + 1, ib) + 4 * lane);
-                dsn[ib] = load_streamed<bf16x4>(kept_b + K::ck(cid, jb + 1, ib) + 4 * lane);
+                s0n[ib] = kept_frag(kept_f + K::ck(cid, jb + 1, ib));
+                dsn[ib] = kept_frag(kept_b + K::ck(cid, jb + 1, ib));
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -664,13 +676,13 @@ __global__ __launch_bounds__(256, 2) void grads_kernel(int T, int H, int nchunks
         __bf16* const dst[5] = {dq_, da_, dk_, db_, dw_};
 #pragma unroll
         for (int x = 0; x < 5; x++) {
-            if (jb & 1) store_pair_rows(dst[x] + ca.row0, ca.ld, jb / 2, L, waiting[threadIdx.x >> 6][x][lane], grads[x]);
+            if (jb & 1) store_pair_rows<OUT_PAST>(dst[x] + ca.row0, ca.ld, jb / 2, L, waiting[threadIdx.x >> 6][x][lane], grads[x]);
             else if (jb + 1 < NB) waiting[threadIdx.x >> 6][x][lane] = grads[x];
             else store_frag_rows(dst[x] + ca.row0, ca.ld, jb, L, grads[x]);
         }
     }
 #pragma unroll
-    for (int i = 0; i < NB / 2; i++) store_pair_rows(dv_ + ca.row0, ca.ld, i, L, to_bf16(dv[2 * i]), to_bf16(dv[2 * i + 1]));
+    for (int i = 0; i < NB / 2; i++) store_pair_rows<OUT_PAST>(dv_ + ca.row0, ca.ld, i, L, to_bf16(dv[2 * i]), to_bf16(dv[2 * i + 1]));
     if constexpr (NB & 1) store_frag_rows(dv_ + ca.row0, ca.ld, NB - 1, L, to_bf16(dv[NB - 1]));
 }
 
@@ -790,19 +802,48 @@ inline int scan_rows(int BH, int NB) {
     return 4;
 }
 
+// Which of a training pass's tensors go past the caches, by what the pass touches (thirteen sequences, the kept states of both
+// directions) against a last-level cache of 256 MiB.  Forward + backward, us, through the caches / past them, on one set of inputs and on three in turn:
+//   * kept states from 160 MiB on: 4 x 1024 tokens x 48 heads of 16 (104 MiB) 95 / 100, 107 / 108, 8 x 1024 x 48 (204) 203 / 180, 210 / 193; 5 x 1024 x 24 of
+//     32 (143) 107 / 108, 114 / 120, 8 x 1024 x 24 189 / 179, 186 / 168; 5 x 1024 x 16 of 48 (158) 114 / 118, 126 / 134; 11 x 256 x 9 of 80 (97) 79 / 81, 76 / 78,
+//     6 x 1024 x 9 (208) 167 / 150, 169 / 169.  Of 96 and 128 channels at any size: 2 x 256 x 8 of 96 57 / 56, 54 / 52, 4 x 1024 x 8 118 / 119, 125 / 119,
+//     2 x 256 x 6 of 128 72 / 70, 66 / 64;
+//   * the gradients of 96 and 128 channels from 256 MiB on: 5 x 1024 x 6 of 128 (233 MiB) 156 / 160, 163 / 166, 8 x 1024 x 6 243 / 215, 231 / 230, 16 x 1024 x 6
+//     493 / 473, 494 / 473; 8 x 1024 x 8 of 96 217 / 186, 214 / 209.  Never where a row of a head is no multiple of the 64 bytes that a store takes
+//     of it (48, 80, 112 channels: 32 x 1024 x 16 of 48 736 / 821, 34 x 1024 x 9 of 80 857 / 942, 36 x 1024 x 6 of 112 939 / 1000), nor of 32
+//     channels (8 x 1024 x 24 168 / 174, 32 x 1024 x 24 652 / 660).
+struct PastCaches {
+    bool kept, out;
+    static constexpr bool whole_halves(int NB) { return NB == 6 || NB == 8; }
+    PastCaches(int B, int T, int H, int NB) {
+        const size_t tokens = (size_t)B * T * H, bytes = 13 * tokens * 32 * NB + 2 * tokens / CHUNK * (NB + 1) * NB * FRAG_ELEMS * sizeof(__bf16);
+        kept = whole_halves(NB) || bytes > (size_t)160 << 20;
+        out = whole_halves(NB) && bytes > (size_t)256 << 20;
+    }
+};
+
 template <int NB, bool FWD, bool KEEP>
 void scan(int B, int T, int H, int state_f32, const __bf16* rec, const void* s_in, void* s_out, __bf16* y, __bf16* kept, float* centers,
           hipStream_t stream) {
-    auto launch = [&](auto width) {
+    auto launch = [&](auto width, auto past) {
         constexpr int W = decltype(width)::value;
-        hipLaunchKernelGGL((scan_kernel<NB, FWD, KEEP, W>), dim3(B * H, (NB + W - 1) / W), dim3(64 * (W + scan_helpers(W))), 0, stream, T, H,
-                           state_f32, rec, s_in, s_out, y, kept, centers);
+        hipLaunchKernelGGL((scan_kernel<NB, FWD, KEEP, W, decltype(past)::value>), dim3(B * H, (NB + W - 1) / W), dim3(64 * (W + scan_helpers(W))), 0,
+                           stream, T, H, state_f32, rec, s_in, s_out, y, kept, centers);
     };
-    switch (scan_rows(B * H, NB)) {
-        case 1: launch(std::integral_constant<int, 1>()); break;
-        case 2: launch(std::integral_constant<int, 2>()); break;
-        default: launch(std::integral_constant<int, 4>());
+    auto go = [&](auto past) {
+        switch (scan_rows(B * H, NB)) {
+            case 1: launch(std::integral_constant<int, 1>(), past); break;
+            case 2: launch(std::integral_constant<int, 2>(), past); break;
+            default: launch(std::integral_constant<int, 4>(), past);
+        }
+    };
+    if constexpr (KEEP && !PastCaches::whole_halves(NB)) {
+        if (!PastCaches(B, T, H, NB).kept) {
+            go(std::false_type());
+            return;
+        }
     }
+    go(std::true_type());
 }
 
 template <int NB>
@@ -822,8 +863,13 @@ void backward(int B, int T, int H, int state_f32, const void* w, const void* q, 
     hipLaunchKernelGGL(bwd_prepare_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q),
                        c(a), c(b), c(dy), m(rec));
     scan<NB, false, true>(B, T, H, state_f32, c(rec), ds_in, ds_out, nullptr, m(kept_b), nullptr, stream);
-    hipLaunchKernelGGL(grads_kernel<NB>, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k),
-                       c(v), c(a), c(b), c(dy), c(kept_f), c(kept_b), m(dw), m(dq), m(dk), m(dv), m(da), m(db));
+    auto grads = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k), c(v), c(a), c(b), c(dy),
+                           c(kept_f), c(kept_b), m(dw), m(dq), m(dk), m(dv), m(da), m(db));
+    };
+    const PastCaches past(B, T, H, NB);
+    if constexpr (PastCaches::whole_halves(NB)) past.out ? grads(grads_kernel<NB, true, true>) : grads(grads_kernel<NB, true, false>);
+    else past.kept ? grads(grads_kernel<NB, true, false>) : grads(grads_kernel<NB, false, false>);
 }
 
 // calls f.template operator()<NB>() for the head size's NB
