@@ -435,7 +435,8 @@ int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const i
                                   const void* const* x, const long long* ld_x,
                                   void* const* dW, int out_dtype,
                                   void* workspace, size_t workspace_bytes, void* stream);
-/* The same for the weights of one time mixer: up to nine, those above and the output projection. */
+/* The same for the weights of one time mixer: up to nine, the output projection's first and those above.  The first may run in
+ * launches of its own, where that is faster. */
 #define WIND_RWKV7_BLOCK_WGRADS_MAX 9
 size_t wind_rwkv7_block_wgrads_workspace_bytes(int n, long long tokens, const int* O, const int* I);
 int wind_rwkv7_block_wgrads(int n, long long tokens, const int* O, const int* I,

@@ -304,7 +304,8 @@ def test_linear_wgrad_group_sizes_and_validation_on_host():
 
 
 def test_block_wgrads_take_nine_on_host():
-    """The same as a group of up to nine: 9 problems of a block are 79 tiles, in three token ranges on 256 compute units."""
+    """As a group of up to nine: 9 problems of a block are 79 tiles, in three token ranges on 256 compute units.  The first apart where
+    all of them together fall badly on the compute units, in memory that both launches use one after the other."""
     import ctypes
     lib = _native.lib()
     ints = lambda *v: (ctypes.c_int * len(v))(*v)
@@ -312,6 +313,12 @@ def test_block_wgrads_take_nine_on_host():
     sizes = lib.wind_rwkv7_block_wgrads_workspace_bytes
     assert sizes(9, 8192, ints(*O), ints(*I)) == 3 * 4 * (4 * 16 * 192 * 192 + 3 * 256 * (128 + 32 + 96 + 128 + 64))
     assert sizes(8, 8192, ints(*O), ints(*I)) == lib.wind_rwkv7_linear_wgrad_group_workspace_bytes(8, 8192, ints(*O), ints(*I)) > 0
+    for C, tokens, apart in ((768, 8192, False), (1024, 2048, False), (1024, 4096, True), (1024, 8192, True), (1152, 8192, False), (1344, 8192, False),
+                             (1408, 1024, False), (1408, 2048, True), (1536, 8192, True), (2048, 1024, False), (2048, 2048, True)):
+        o, i = (C, C, C, C, 128, 32, 96, C, C), (C, C, C, C, C, C, C, 128, 64)
+        one, eight = (lib.wind_rwkv7_linear_wgrad_workspace_bytes(tokens, C, C),
+                      lib.wind_rwkv7_linear_wgrad_group_workspace_bytes(8, tokens, ints(*o[1:]), ints(*i[1:])))
+        assert (sizes(9, tokens, ints(*o), ints(*i)) == max(one, eight)) == apart, (C, tokens)
     assert sizes(10, 8192, ints(*O, 64), ints(*I, 64)) == 0 and sizes(0, 8192, ints(*O), ints(*I)) == 0
     assert lib.wind_rwkv7_block_wgrads(10, 8192, None, None, None, None, None, None, None, 1, None, 0, None) == 2
     assert lib.wind_rwkv7_block_wgrads(9, 8192, None, None, None, None, None, None, None, 1, None, 0, None) == 1

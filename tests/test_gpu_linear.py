@@ -327,6 +327,37 @@ def test_linear_wgrad_group_matches_fp64_products(tokens, shapes):
         assert torch.equal(w.cpu(), want)
 
 
+@pytest.mark.parametrize('tokens,shapes,apart', [
+    (2048, [(1408, 1408)] * 2 + [(128, 1408), (1408, 1408), (32, 1408), (1408, 1408), (96, 1408), (1408, 128), (1408, 64)], True),
+    (1999, [(1408, 1408)] * 2 + [(128, 1408), (1408, 1408), (32, 1408), (1408, 1408), (96, 1408), (1408, 128), (1408, 64)], True),
+    (1000, [(1408, 1408)] * 2 + [(128, 1408), (1408, 1408), (32, 1408), (1408, 1408), (96, 1408), (1408, 128), (1408, 64)], False),
+    (20000, [(768, 2112), (2112, 768)], True),             # the second on its own as well
+    (20000, [(768, 2112)], False),
+])
+def test_block_wgrads_match_fp64_products(tokens, shapes, apart):
+    """The weight gradients of a block on both sides of the line from which the first runs apart, in one workspace that starts as NaN
+    (1e-5: fp32 sums over the tokens, as above)."""
+    import ctypes
+    from wind_rwkv import _native
+    lib = _native.lib()
+    n = len(shapes)
+    g = torch.Generator(DEV).manual_seed(tokens + n)
+    dys = [torch.randn(tokens, O, generator=g, device=DEV).bfloat16() for O, _ in shapes]
+    xs = [torch.randn(tokens, I, generator=g, device=DEV).bfloat16() for _, I in shapes]
+    dW = [torch.full(s, float('nan'), device=DEV) for s in shapes]
+    O, I = (ctypes.c_int * n)(*[s[0] for s in shapes]), (ctypes.c_int * n)(*[s[1] for s in shapes])
+    ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+    lds = lambda ts: (ctypes.c_longlong * n)(*[t.stride(0) for t in ts])
+    need = lib.wind_rwkv7_block_wgrads_workspace_bytes(n, tokens, O, I)
+    if 1 < n <= 8:
+        assert (need != lib.wind_rwkv7_linear_wgrad_group_workspace_bytes(n, tokens, O, I)) == apart
+    ws = torch.full((need // 4,), float('nan'), device=DEV)
+    _native.check(lib.wind_rwkv7_block_wgrads(n, tokens, O, I, ptrs(dys), lds(dys), ptrs(xs), lds(xs), ptrs(dW), _native.F32, ws.data_ptr(), need,
+                                              torch.cuda.current_stream().cuda_stream))
+    for dy, x, w in zip(dys, xs, dW):
+        assert _rel(w.cpu(), (dy.double().T @ x.double()).cpu()) <= 1e-5
+
+
 def test_linear_wgrad_group_falls_back_for_different_token_counts():
     from wind_rwkv.rwkv7.linear import linear_wgrad_group
     g = torch.Generator().manual_seed(3)

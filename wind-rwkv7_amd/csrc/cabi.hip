@@ -883,17 +883,17 @@ int wind_rwkv7_linear_wgrad(long long tokens, int O, int I, const void* dy, long
     return launch_status();
 }
 
-static size_t wgrads_workspace_bytes(int most, int n, long long tokens, const int* O, const int* I) {
-    if (n < 1 || n > most || !O || !I) return 0;
+static size_t wgrads_workspace_bytes(bool block, int n, long long tokens, const int* O, const int* I) {
+    if (n < 1 || n > (block ? WIND_RWKV7_BLOCK_WGRADS_MAX : WIND_RWKV7_WGRAD_GROUP_MAX) || !O || !I) return 0;
     for (int j = 0; j < n; j++)
         if (check_linear(tokens, O[j], I[j])) return 0;
-    return align_up(wkv::linear_wgrad_group_workspace_bytes(n, (long)tokens, O, I));
+    return align_up((block ? wkv::block_wgrads_workspace_bytes : wkv::linear_wgrad_group_workspace_bytes)(n, (long)tokens, O, I));
 }
 
-static int wgrads(int most, int n, long long tokens, const int* O, const int* I, const void* const* dy, const long long* ld_dy,
+static int wgrads(bool block, int n, long long tokens, const int* O, const int* I, const void* const* dy, const long long* ld_dy,
                   const void* const* x, const long long* ld_x, void* const* dW, int out_dtype, void* workspace, size_t workspace_bytes,
                   void* stream) {
-    if (n < 1 || n > most) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (n < 1 || n > (block ? WIND_RWKV7_BLOCK_WGRADS_MAX : WIND_RWKV7_WGRAD_GROUP_MAX)) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (!O || !I || !dy || !ld_dy || !x || !ld_x || !dW) return WIND_RWKV7_ERR_NULL_POINTER;
     if (out_dtype != WIND_RWKV7_BF16 && out_dtype != WIND_RWKV7_F32) return WIND_RWKV7_ERR_DTYPE;
     long ldy[WIND_RWKV7_BLOCK_WGRADS_MAX], ldx[WIND_RWKV7_BLOCK_WGRADS_MAX];
@@ -907,32 +907,32 @@ static int wgrads(int most, int n, long long tokens, const int* O, const int* I,
         ldy[j] = (long)ld_dy[j];
         ldx[j] = (long)ld_x[j];
     }
-    const int rc = check_workspace(workspace, workspace_bytes, wgrads_workspace_bytes(most, n, tokens, O, I));
+    const int rc = check_workspace(workspace, workspace_bytes, wgrads_workspace_bytes(block, n, tokens, O, I));
     if (rc) return rc;
-    if (!wkv::launch_linear_wgrad_group(n, (long)tokens, O, I, dy, ldy, x, ldx, dW, out_dtype == WIND_RWKV7_F32, workspace,
-                                        static_cast<hipStream_t>(stream)))
+    if (!(block ? wkv::launch_block_wgrads : wkv::launch_linear_wgrad_group)(n, (long)tokens, O, I, dy, ldy, x, ldx, dW, out_dtype == WIND_RWKV7_F32,
+                                                                            workspace, static_cast<hipStream_t>(stream)))
         return WIND_RWKV7_ERR_CHANNELS;
     return launch_status();
 }
 
 size_t wind_rwkv7_linear_wgrad_group_workspace_bytes(int n, long long tokens, const int* O, const int* I) {
-    return wgrads_workspace_bytes(WIND_RWKV7_WGRAD_GROUP_MAX, n, tokens, O, I);
+    return wgrads_workspace_bytes(false, n, tokens, O, I);
 }
 
 int wind_rwkv7_linear_wgrad_group(int n, long long tokens, const int* O, const int* I, const void* const* dy,
                                   const long long* ld_dy, const void* const* x, const long long* ld_x, void* const* dW,
                                   int out_dtype, void* workspace, size_t workspace_bytes, void* stream) {
-    return wgrads(WIND_RWKV7_WGRAD_GROUP_MAX, n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_dtype, workspace, workspace_bytes, stream);
+    return wgrads(false, n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_dtype, workspace, workspace_bytes, stream);
 }
 
 size_t wind_rwkv7_block_wgrads_workspace_bytes(int n, long long tokens, const int* O, const int* I) {
-    return wgrads_workspace_bytes(WIND_RWKV7_BLOCK_WGRADS_MAX, n, tokens, O, I);
+    return wgrads_workspace_bytes(true, n, tokens, O, I);
 }
 
 int wind_rwkv7_block_wgrads(int n, long long tokens, const int* O, const int* I, const void* const* dy, const long long* ld_dy,
                             const void* const* x, const long long* ld_x, void* const* dW, int out_dtype, void* workspace,
                             size_t workspace_bytes, void* stream) {
-    return wgrads(WIND_RWKV7_BLOCK_WGRADS_MAX, n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_dtype, workspace, workspace_bytes, stream);
+    return wgrads(true, n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_dtype, workspace, workspace_bytes, stream);
 }
 
 int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream) {

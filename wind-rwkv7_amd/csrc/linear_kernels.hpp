@@ -25,6 +25,10 @@ size_t linear_wgrad_group_workspace_bytes(int n, long tokens, const int* O, cons
 bool launch_linear_wgrad_group(int n, long tokens, const int* O, const int* I, const void* const* dy, const long* ld_dy,
                                const void* const* x, const long* ld_x, void* const* dW, bool out_f32, void* workspace,
                                hipStream_t stream);
+// The same, or the first problem in launches of its own ahead of the others, whichever is the faster.
+size_t block_wgrads_workspace_bytes(int n, long tokens, const int* O, const int* I);
+bool launch_block_wgrads(int n, long tokens, const int* O, const int* I, const void* const* dy, const long* ld_dy,
+                         const void* const* x, const long* ld_x, void* const* dW, bool out_f32, void* workspace, hipStream_t stream);
 
 // Column blocks of token-major bf16 matrices (csrc/cols.hip): piece = `width` columns (a multiple of 8) of M rows
 // from (src, src_ld, src_col0) to (dst, dst_ld, dst_col0); offsets and strides multiples of 8 elements.

@@ -567,4 +567,53 @@ bool launch_linear_wgrad_group(int n, long tokens, const int* O, const int* I, c
     return true;
 }
 
+// ---- those of a block: all in one launch, or the first (the output projection, as large as any) on its own ahead of the others ----
+namespace {
+// us of the products of one launch: rounds of blocks over the compute units, 0.5 us a step of 32 tokens, a tenth more where the token
+// ranges are no whole share of the XCDs, each of which then reads nearly all ranges
+double products_us(long tiles, long ksplit, long tokens) {
+    const long cus = compute_units(), rounds = (tiles * ksplit + cus - 1) / cus;
+    return 0.5 * (8 % ksplit && ksplit % 8 ? 1.1 : 1.0) * ((tokens + STEP - 1) / STEP) * rounds / ksplit;
+}
+// One launch saves two others, their start and their partial tiles, 10 to 20 us; it loses where the grid of all falls badly on the
+// compute units.  The nine of a block with their sums, us, eight and the output projection -> all: 768 channels 2048 tokens 50 -> 38, 8192 78
+// -> 75, 32768 227 -> 231, 65536 384 -> 446; 1024 channels (128 tiles x 2 ranges + 36 x 7 -> 164 x 1) 2048 70 -> 58, 4096 88.5 -> 88.4, 8192 132 ->
+// 154; 1152 8192 172 -> 148; 1408 (222 + 64 x 4 -> 286, a second round) 1024 75 -> 75, 2048 91 -> 100, 8192 206 -> 276; 2048 (a third
+// round) 1024 126 -> 126, 2048 164 -> 172, 8192 427 -> 490.  The line is drawn at 15 us, between these; it misses 832 and 896
+// channels from 32768 tokens on (3 to 6 % better apart) and 640 at 16384 (119 -> 129).
+// Error of the sums against fp64 at 768 channels, eight / the first -> all: 2048 tokens 1.3e-7 / 0.8e-7 -> 1.5e-7, 8192 2.7e-7 / 1.4e-7 ->
+// 3.2e-7 (longer ranges; the bf16 operands' rounding is 2e-3).
+bool first_alone(int n, long tokens, const int* O, const int* I) {
+    GroupPlan all, rest;
+    if (n < 2 || !group_plan(n, tokens, O, I, all)) return false;
+    const WgradPlan first = linear_wgrad_plan(tokens, O[0], I[0]);
+    double apart = products_us(first.ntiles, first.ksplit, tokens);
+    if (n == 2) {
+        const WgradPlan second = linear_wgrad_plan(tokens, O[1], I[1]);
+        apart += products_us(second.ntiles, second.ksplit, tokens);
+    } else {
+        if (!group_plan(n - 1, tokens, O + 1, I + 1, rest)) return false;
+        apart += products_us(rest.first_tile[n - 1], rest.ksplit, tokens);
+    }
+    return products_us(all.first_tile[n], all.ksplit, tokens) > apart + 15.0;
+}
+}  // namespace
+
+size_t block_wgrads_workspace_bytes(int n, long tokens, const int* O, const int* I) {
+    if (!first_alone(n, tokens, O, I)) return linear_wgrad_group_workspace_bytes(n, tokens, O, I);
+    // (one after the other on a stream: the same memory)
+    const size_t first = linear_wgrad_plan(tokens, O[0], I[0]).partial_bytes;
+    const size_t rest = n == 2 ? linear_wgrad_plan(tokens, O[1], I[1]).partial_bytes : linear_wgrad_group_workspace_bytes(n - 1, tokens, O + 1, I + 1);
+    return first > rest ? first : rest;
+}
+
+bool launch_block_wgrads(int n, long tokens, const int* O, const int* I, const void* const* dy, const long* ld_dy, const void* const* x,
+                         const long* ld_x, void* const* dW, bool out_f32, void* workspace, hipStream_t stream) {
+    if (!first_alone(n, tokens, O, I)) return launch_linear_wgrad_group(n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_f32, workspace, stream);
+    launch_linear_wgrad(tokens, O[0], I[0], dy[0], ld_dy[0], x[0], ld_x[0], dW[0], out_f32, workspace, stream);
+    if (n > 2) return launch_linear_wgrad_group(n - 1, tokens, O + 1, I + 1, dy + 1, ld_dy + 1, x + 1, ld_x + 1, dW + 1, out_f32, workspace, stream);
+    launch_linear_wgrad(tokens, O[1], I[1], dy[1], ld_dy[1], x[1], ld_x[1], dW[1], out_f32, workspace, stream);
+    return true;
+}
+
 }  // namespace wkv

@@ -700,10 +700,10 @@ struct Products {
     }
 };
 
-// dW = dy^T x for several pairs on the same tokens: one grouped launch (a single pair goes through its own entry point).  Whatever
-// runs on its own leaves fp32 partial tiles from every compute unit, 147 KB each, which are written and read again: a 768 x 768 product
-// of 8192 tokens is 22 us + 8 of sums for 12 us of products.  So all of a pass go together; the nine of a block there, us with their sums:
-// eight and the output projection 90, projections and LoRA factors 88, one launch 78.
+// dW = dy^T x for several pairs on the same tokens, the output projection's first (a single pair goes through its own entry point).
+// Whatever runs on its own leaves fp32 partial tiles from every compute unit, 147 KB each, which are written and read again: a 768 x 768 product
+// of 8192 tokens is 22 us + 8 of sums for 12 us of products.  So all of a pass go together, unless the grid that makes falls badly on
+// the compute units: that is decided behind the entry point (first_alone in linear_wgrad.hip).
 struct WeightGrads {
     std::vector<int> O, I;
     std::vector<const void*> dy, x;
