@@ -92,6 +92,10 @@ size_t wind_rwkv7_attn_saved_bytes(int B, int T, int H, int C);
 size_t wind_rwkv7_attn_fwd_workspace_bytes(int B, int T, int H, int C);
 size_t wind_rwkv7_attn_bwd_workspace_bytes(int B, int T, int H, int C);
 
+/* Of these for the forward, what wind_rwkv7_attn_forward and wind_rwkv7_attn_ln_forward make use of: a call that keeps something for a
+ * backward pass writes its chunks' operands to memory (13.25 KiB each) from more chunks on than one that keeps nothing. */
+size_t wind_rwkv7_attn_train_workspace_bytes(int B, int T, int H, int C);
+
 /* y, sT = WKV7(w, q, k, v, a, b, s0), and `s` for backward.
  * Replaces cuda_forward (attn.cu:108-128) / the operator wind::forward (attn.cpp:10-13,25).
  *   S_t = S_{t-1} diag(exp(-exp(w_t))) + (S_{t-1} a_t) b_t^T + v_t k_t^T ;  y_t = S_t q_t

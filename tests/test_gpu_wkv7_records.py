@@ -24,8 +24,8 @@ def _least(lib, B, T, H, interval):
 
 
 def test_workspace_sizes_at_the_lines_of_the_rule():
-    """Records from eight chunks (backward: from 96, or 48 and 2048 in all), for up to a quarter of the compute units' worth of (batch,
-    head) pairs and 6144 chunks, and not where a sequence runs as eight segments."""
+    """Records from eight chunks (backward, and a forward that keeps something for it: from 96, or 48 and 2048 in all), for up to a quarter
+    of the compute units' worth of (batch, head) pairs and 6144 chunks, and not where a sequence runs as eight segments."""
     from wind_rwkv import _native
     lib = _native.lib()
     for (B, T, H), (ahead, back) in {(1, 112, 4): (False, False), (1, 128, 4): (True, False), (1, 1520, 4): (True, False), (1, 1536, 4): (True, True),
@@ -38,6 +38,31 @@ def test_workspace_sizes_at_the_lines_of_the_rule():
         assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == (chunks * 13568 if ahead else fwd), (B, T, H)
         kept = B * H * (T // 32 * 12288 if T % 32 == 0 else T // 16 * 10240)
         assert lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == (kept + chunks * 10496 if back else bwd), (B, T, H)
+        assert lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == (chunks * 13568 if back else fwd), (B, T, H)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('ln', [False, True])
+@pytest.mark.parametrize('B,T,H', [(1, 1536, 64), (1, 496, 64), (1, 256, 4), (1, 8192, 8)])
+def test_a_node_keeps_what_its_backward_reads(B, T, H, ln):
+    """Between forward and backward a node holds the saved tensor beside its outputs and not the scan's scratch: records (6144 chunks,
+    80 MiB), records that only a forward without gradients would write (64 pairs x 31 chunks), none, segments' maps."""
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import attn, attn_ln
+    lib = _native.lib()
+    d = inputs.wkv7_inputs(B, T, H, C, seed=H, dtype=torch.bfloat16)
+    x = [d[n].reshape(B, T, H * C).to(DEV).requires_grad_() for n in ('q', 'w', 'k', 'v', 'a', 'b')]
+    g = x[0].detach().clone()
+    params = torch.ones(3, H * C, device=DEV)
+    go = lambda: attn_ln(*x, g, params, C) if ln else attn(*x, C)
+    go()   # (kernels loaded, pools filled)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    y = go()
+    held = torch.cuda.memory_allocated() - before
+    saved = (lib.wind_rwkv7_attn_ln_saved_bytes if ln else lib.wind_rwkv7_attn_saved_bytes)(B, T, H, C)
+    wanted = y.numel() * 2 + saved + B * H * C * C * 2   # (sT: a node output, gone where nobody asked for it)
+    assert held <= wanted + 3 * 1024, (held, wanted)     # the pool's granularity, 512 bytes, and the 256 of a call without scratch
 
 
 @pytest.mark.gpu

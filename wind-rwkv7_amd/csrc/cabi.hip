@@ -80,9 +80,9 @@ inline size_t rec_bwd_bytes(int B, int T, int H, bool ln = false) {
 }
 // Scratch of the scan: the chunks' records, or the segments' maps and states.  The size queries ask for what the fastest way takes; a
 // call also accepts the least, with which there are no records.  (The forward's argument is always checked.)
-inline size_t scan_bytes(int B, int T, int H, bool fwd) { return align_up(wkv::scan_workspace_bytes(B, T, H, fwd)); }
+inline size_t scan_bytes(int B, int T, int H, wkv::ScanUse use) { return align_up(wkv::scan_workspace_bytes(B, T, H, use)); }
 inline size_t scan_least_bytes(int B, int T, int H) { return align_up(wkv::scan_workspace_least_bytes(B, T, H)); }
-inline size_t fwd_ws_bytes(int B, int T, int H) { return std::max<size_t>(scan_bytes(B, T, H, true), 256); }
+inline size_t fwd_ws_bytes(int B, int T, int H, wkv::ScanUse use) { return std::max<size_t>(scan_bytes(B, T, H, use), 256); }
 inline size_t fwd_ws_least_bytes(int B, int T, int H) { return std::max<size_t>(scan_least_bytes(B, T, H), 256); }
 
 // ---- optional per-kernel timing (process-global, measurement only) ----
@@ -184,13 +184,18 @@ size_t wind_rwkv7_attn_saved_bytes(int B, int T, int H, int C) {
 size_t wind_rwkv7_attn_fwd_workspace_bytes(int B, int T, int H, int C) {
     if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK) return 0;
     if (C != wkv::HEAD) return wkv::wide::record_bytes(B, T, H, C, true);
-    return fwd_ws_bytes(B, T, H);
+    return fwd_ws_bytes(B, T, H, wkv::SCAN_PREFILL);
+}
+
+size_t wind_rwkv7_attn_train_workspace_bytes(int B, int T, int H, int C) {
+    if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK || C != wkv::HEAD) return wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C);
+    return fwd_ws_bytes(B, T, H, wkv::SCAN_FORWARD);
 }
 
 size_t wind_rwkv7_attn_bwd_workspace_bytes(int B, int T, int H, int C) {
     if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK) return 0;
     if (C != wkv::HEAD) return wkv::wide::record_bytes(B, T, H, C, false) + wkv::wide::kept_bytes(B, T, H, C);
-    return rec_bwd_bytes(B, T, H) + scan_bytes(B, T, H, false);
+    return rec_bwd_bytes(B, T, H) + scan_bytes(B, T, H, wkv::SCAN_BACKWARD);
 }
 
 // wide_centers (head sizes other than 64 only): y is attn_ln's kept output and is written centred, the centres there
@@ -264,7 +269,7 @@ int wind_rwkv7_attn_prefill_static(int B, int T, int H, int C, int io_dtype, int
     // The whole array is the workspace (a pass that keeps nothing stores nothing in `s`), and no more of it than
     // wind_rwkv7_attn_prefill's query asks for: the scan plans by that size, and another plan gives other roundings.
     // Nothing has to start at zero.
-    const size_t ws = fwd_ws_bytes(B, T, H);
+    const size_t ws = fwd_ws_bytes(B, T, H, wkv::SCAN_PREFILL);
     if (ws > (size_t)WIND_RWKV7_STATIC_ARRAY_BYTES) return WIND_RWKV7_ERR_STATIC_LIMIT;   // (no problem within the limit above)
     return attn_forward(B, T, H, C, io_dtype, state_dtype, w, q, k, v, a, b, s0, y, base, sT, base, ws, 0, stream);
 }
@@ -327,7 +332,7 @@ size_t wind_rwkv7_attn_ln_bwd_workspace_bytes(int B, int T, int H, int C) {
     if (C != wkv::HEAD)
         return align256(wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)) +
                align256(wkv::lnheads::bwd_workspace_bytes((long)B * T, H, C)) + 4 * align256(wide_seq_bytes(B, T, H, C));
-    return rec_bwd_bytes(B, T, H, true) + seq_bytes(B, T, H) + ddot_bytes(B, T, H) + dpart_bytes(B, T, H) + scan_bytes(B, T, H, false);
+    return rec_bwd_bytes(B, T, H, true) + seq_bytes(B, T, H) + ddot_bytes(B, T, H) + dpart_bytes(B, T, H) + scan_bytes(B, T, H, wkv::SCAN_BACKWARD);
 }
 
 static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
@@ -412,7 +417,7 @@ int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int st
     if (!dw || !dq || !dk || !dv || !da || !db || !dg || !dparams) return WIND_RWKV7_ERR_NULL_POINTER;
     rc = check_workspace(workspace, workspace_bytes,
                          wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C) -
-                             (C != wkv::HEAD ? 0 : scan_bytes(B, T, H, false) - scan_least_bytes(B, T, H)));
+                             (C != wkv::HEAD ? 0 : scan_bytes(B, T, H, wkv::SCAN_BACKWARD) - scan_least_bytes(B, T, H)));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (C != wkv::HEAD) {

@@ -31,9 +31,9 @@ namespace py = pybind11;
 
 #define WIND_SYMBOLS(X)                                                                                              \
     X(strerror) X(checkpoint_interval) X(head_size_supported) X(attn_head_size_supported)                            \
-    X(attn_saved_bytes) X(attn_fwd_workspace_bytes) X(attn_bwd_workspace_bytes)                                      \
+    X(attn_saved_bytes) X(attn_fwd_workspace_bytes) X(attn_train_workspace_bytes) X(attn_bwd_workspace_bytes)        \
     X(attn_forward) X(attn_prefill) X(attn_backward)                                                                 \
-    X(attn_ln_saved_bytes) X(attn_ln_fwd_workspace_bytes) X(attn_ln_bwd_workspace_bytes)                             \
+    X(attn_ln_saved_bytes) X(attn_ln_bwd_workspace_bytes)                                                            \
     X(attn_ln_forward) X(attn_ln_prefill) X(attn_ln_backward)                                                        \
     X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward_split)                       \
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
@@ -143,20 +143,32 @@ void same_interval(const Kept& k) {
                 "): set it between whole forward + backward passes only");
 }
 
+// The forward's saved tensor and its scratch: one allocation where the scratch is nothing to speak of, or nothing is kept behind the
+// call; otherwise two, so that a node keeps what its backward pass reads and no more.
+struct ForwardMemory {
+    Tensor kept, own;
+    void* workspace;
+    size_t bytes;
+    ForwardMemory(const Shape& s, size_t saved_bytes, bool saves, const Tensor& like)
+        : bytes(std::max<size_t>((saves ? L.attn_train_workspace_bytes : L.attn_fwd_workspace_bytes)(s.B, s.T, s.H, s.C), 256)) {
+        const size_t first = (saved_bytes + 255) / 256 * 256;
+        const bool apart = saves && bytes > 256;
+        kept = scratch_bytes(first + (apart ? 0 : bytes), like);
+        if (apart) own = scratch_bytes(bytes, like);
+        workspace = apart ? ptr(own) : static_cast<char*>(ptr(kept)) + first;
+    }
+};
+
 struct Wkv7 : torch::autograd::Function<Wkv7> {
     static variable_list run(const Shape& s, const Tensor& w, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& a,
                              const Tensor& b, const Tensor& s0, Tensor* saved) {
         Tensor y = at::empty_like(v);
         Tensor sT = at::empty({s.B, s.H, s.C, s.C}, s0.defined() ? s0.options() : v.options());
-        // one allocation for the saved tensor and the forward's scratch behind it (both are multiples of 256 bytes)
-        const size_t ws = std::max<size_t>(L.attn_fwd_workspace_bytes(s.B, s.T, s.H, s.C), 256);
-        const size_t keep_bytes = saved ? (L.attn_saved_bytes(s.B, s.T, s.H, s.C) + 255) / 256 * 256 : 0;
-        Tensor mem = scratch_bytes(keep_bytes + ws, v);
-        char* base = static_cast<char*>(mem.data_ptr());
+        const ForwardMemory mem(s, saved ? L.attn_saved_bytes(s.B, s.T, s.H, s.C) : 0, saved, v);
         check((saved ? L.attn_forward : L.attn_prefill)(
             s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, state_code(s0), ptr(w), ptr(q), ptr(k), ptr(v), ptr(a), ptr(b), ptr(s0), ptr(y),
-            base, ptr(sT), base + keep_bytes, ws, stream_of(v)));
-        if (saved) *saved = mem;
+            ptr(mem.kept), ptr(sT), mem.workspace, mem.bytes, stream_of(v)));
+        if (saved) *saved = mem.kept;
         return {y, sT};
     }
     // (a node takes no undefined tensor: without an initial state `state` is any tensor)
@@ -267,14 +279,11 @@ struct Wkv7Ln : torch::autograd::Function<Wkv7Ln> {
                              const Tensor& b, const Tensor& g, const Tensor& params, const Tensor& s0, Tensor* saved) {
         Tensor y = at::empty_like(v);
         Tensor sT = at::empty({s.B, s.H, s.C, s.C}, s0.defined() ? s0.options() : v.options());
-        const size_t ws = std::max<size_t>(L.attn_ln_fwd_workspace_bytes(s.B, s.T, s.H, s.C), 256);
-        const size_t keep_bytes = (L.attn_ln_saved_bytes(s.B, s.T, s.H, s.C) + 255) / 256 * 256;
-        Tensor mem = scratch_bytes(keep_bytes + ws, v);
-        char* base = static_cast<char*>(mem.data_ptr());
+        const ForwardMemory mem(s, L.attn_ln_saved_bytes(s.B, s.T, s.H, s.C), saved, v);
         check((saved ? L.attn_ln_forward : L.attn_ln_prefill)(
             s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, state_code(s0), ptr(w), ptr(q), ptr(k), ptr(v), ptr(a), ptr(b), ptr(g), ptr(params),
-            ptr(s0), ptr(y), base, ptr(sT), base + keep_bytes, ws, stream_of(v)));
-        if (saved) *saved = mem;
+            ptr(s0), ptr(y), ptr(mem.kept), ptr(sT), mem.workspace, mem.bytes, stream_of(v)));
+        if (saved) *saved = mem.kept;
         return {y, sT};
     }
     static variable_list forward(AutogradContext* ctx, Shape s, bool has_s0, const Tensor& w, const Tensor& q, const Tensor& k,
@@ -806,7 +815,7 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
                                         w(MA_W2), w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b),
                                         kept.defined() ? ptr(kept) : nullptr, stream));
     if (whole) {
-        const Tensor ws = scratch_bytes(L.attn_ln_fwd_workspace_bytes(B, T, H, N), xb);
+        const Tensor ws = scratch_bytes((save ? L.attn_train_workspace_bytes : L.attn_fwd_workspace_bytes)(B, T, H, N), xb);
         check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
             B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln),
             ptr(s0), ptr(f.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));

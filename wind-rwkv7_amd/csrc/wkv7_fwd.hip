@@ -135,8 +135,8 @@ ScanPlan scan_plan(int B, int T, int H, size_t ws_bytes, ScanUse use) {
     const int most = scan_segments_most(B, T, H);
     return {false, ws_bytes >= segments_bytes(B, H, most) ? most : scan_segments_least(B, T, H)};
 }
-size_t scan_workspace_bytes(int B, int T, int H, bool fwd) {
-    return scan_by_records(B, T, H, fwd ? SCAN_PREFILL : SCAN_BACKWARD) ? records_bytes(B, T, H, fwd) : segments_bytes(B, H, scan_segments_most(B, T, H));
+size_t scan_workspace_bytes(int B, int T, int H, ScanUse use) {
+    return scan_by_records(B, T, H, use) ? records_bytes(B, T, H, use != SCAN_BACKWARD) : segments_bytes(B, H, scan_segments_most(B, T, H));
 }
 size_t scan_workspace_least_bytes(int B, int T, int H) { return segments_bytes(B, H, scan_segments_least(B, T, H)); }
 

@@ -14,7 +14,7 @@ struct ScanPlan {
 };
 enum ScanUse { SCAN_PREFILL, SCAN_FORWARD, SCAN_BACKWARD };   // forward without and with what a backward pass needs
 ScanPlan scan_plan(int B, int T, int H, size_t ws_bytes, ScanUse use);
-size_t scan_workspace_bytes(int B, int T, int H, bool fwd);
+size_t scan_workspace_bytes(int B, int T, int H, ScanUse use);
 size_t scan_workspace_least_bytes(int B, int T, int H);
 size_t scan_record_bytes(bool fwd);   // of one chunk
 // Chunk preparation + state scan (wkv7_fused.hip).  `saved`: B*H*(T/16) records of Saved::BYTES, or with

@@ -52,9 +52,14 @@ def _sized(workspace, nbytes):
     return workspace if workspace.numel() else torch.empty(max(nbytes, 1), dtype=torch.uint8, device=workspace.device)
 
 
+def _forward_workspace_bytes(B, T, H, C, save):
+    lib = _native.lib()
+    return (lib.wind_rwkv7_attn_train_workspace_bytes if save else lib.wind_rwkv7_attn_fwd_workspace_bytes)(B, T, H, C)
+
+
 def _attn_forward_impl(w, q, k, v, a, b, s0, y, s, sT, workspace, entry='wind_rwkv7_attn_forward'):
     B, T, H, C = w.shape
-    workspace = _sized(workspace, _native.lib().wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C))
+    workspace = _sized(workspace, _forward_workspace_bytes(B, T, H, C, entry == 'wind_rwkv7_attn_forward'))
     with torch.cuda.device(w.device):
         _native.check(getattr(_native.lib(), entry)(
             B, T, H, C, _native.BF16, _state_code(s0),
@@ -175,7 +180,7 @@ def _sizes(B, T, H, C):
         if T % lib.wind_rwkv7_chunk_len():
             _native.check(4)
         _native.check(2)
-    return saved, lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)
+    return saved, lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)
 
 
 @torch.compiler.assume_constant_result
@@ -224,7 +229,7 @@ def fw_attn(w, q, k, v, a, b, s0, save=True):
     y = torch.empty_like(v)
     sT = torch.empty(B, H, C, C, dtype=s0.dtype, device=w.device)   # (s0 may be the empty stand-in for a zero state)
     s = torch.empty(B, H, T // 16, _saved_unit(C), dtype=torch.bfloat16, device=w.device)
-    ws = _workspace(lambda: _sizes(B, T, H, C)[1], w.device)
+    ws = _workspace(lambda: _forward_workspace_bytes(B, T, H, C, save), w.device)
     if save:
         _launch('attn_forward', _attn_forward_impl, w, q, k, v, a, b, s0, y, s, sT, ws)
     else:
@@ -238,7 +243,7 @@ def bw_attn(w, q, k, v, a, b, s, dy, dsT, want_ds0=True):
     B, T, H, C = w.shape
     dw, dq, dk, dv, da, db = [torch.empty_like(x) for x in (w, q, k, v, a, b)]
     ds0 = torch.empty(B, H, C, C, dtype=dsT.dtype, device=w.device) if want_ds0 else no_state(dsT.dtype, w.device)
-    ws = _workspace(lambda: _sizes(B, T, H, C)[2], w.device)
+    ws = _workspace(lambda: _sizes(B, T, H, C)[1], w.device)
     _launch('attn_backward', _attn_backward_impl, w, q, k, v, a, b, dy, s, dsT, dw, dq, dk, dv, da, db, ds0, ws)
     return dw, dq, dk, dv, da, db, ds0
 

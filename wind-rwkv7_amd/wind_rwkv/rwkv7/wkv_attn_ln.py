@@ -8,8 +8,8 @@ Mirrors the reference's rwkv7_attn_ln.py: ``attn_ln(r,w,k,v,a,b,g,params,HEAD_SI
 import torch
 
 from .. import _native
-from .wkv_attn import (_OPS, _any_length, _interval_now, _same_interval, _check_sequences, _check_step, _differentiating, _launch, _no_cpu, _ptr,
-                       _sized, _state_code, _stream, _workspace, no_state)
+from .wkv_attn import (_OPS, _any_length, _interval_now, _same_interval, _check_sequences, _check_step, _differentiating, _forward_workspace_bytes,
+                       _launch, _no_cpu, _ptr, _sized, _state_code, _stream, _workspace, no_state)
 
 _OPS.define('attn_ln_forward(Tensor w, Tensor q, Tensor k, Tensor v, Tensor a, Tensor b, Tensor g, Tensor params, '
             'Tensor s0, Tensor(a!) y, Tensor(b!) s, Tensor(c!) sT, Tensor(d!) workspace) -> ()')
@@ -23,7 +23,7 @@ _OPS.define('attn_ln_backward(Tensor w, Tensor q, Tensor k, Tensor v, Tensor a, 
 
 def _fwd_impl(w, q, k, v, a, b, g, params, s0, y, s, sT, workspace, entry='wind_rwkv7_attn_ln_forward'):
     B, T, H, C = w.shape
-    workspace = _sized(workspace, _native.lib().wind_rwkv7_attn_ln_fwd_workspace_bytes(B, T, H, C))
+    workspace = _sized(workspace, _forward_workspace_bytes(B, T, H, C, entry == 'wind_rwkv7_attn_ln_forward'))
     with torch.cuda.device(w.device):
         _native.check(getattr(_native.lib(), entry)(
             B, T, H, C, _native.BF16, _state_code(s0),
@@ -65,8 +65,7 @@ def _sizes(B, T, H, C):
         if T % lib.wind_rwkv7_chunk_len():
             _native.check(4)
         _native.check(2)
-    return (saved, lib.wind_rwkv7_attn_ln_fwd_workspace_bytes(B, T, H, C),
-            lib.wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C))
+    return saved, lib.wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C)
 
 
 @torch.compiler.assume_constant_result
@@ -84,7 +83,7 @@ def fw_attn_ln(w, q, k, v, a, b, g, params, s0, save=True):
     y = torch.empty_like(v)
     sT = torch.empty(B, H, C, C, dtype=s0.dtype, device=w.device)   # (s0 may be the empty stand-in for a zero state)
     s = torch.empty(B, H, T // 16, _saved_unit(C), dtype=torch.bfloat16, device=w.device)
-    ws = _workspace(lambda: _sizes(B, T, H, C)[1], w.device)
+    ws = _workspace(lambda: _forward_workspace_bytes(B, T, H, C, save), w.device)
     _launch(*(('attn_ln_forward', _fwd_impl) if save else ('attn_ln_prefill', _prefill_impl)),
             w, q, k, v, a, b, g, params, s0, y, s, sT, ws)
     return y, sT, s
@@ -97,7 +96,7 @@ def bw_attn_ln(w, q, k, v, a, b, g, params, s, dy, dsT, want_ds0=True):
     dw, dq, dk, dv, da, db, dg = [torch.empty_like(x) for x in (w, q, k, v, a, b, g)]
     ds0 = torch.empty(B, H, C, C, dtype=dsT.dtype, device=w.device) if want_ds0 else no_state(dsT.dtype, w.device)
     dparams = torch.empty_like(params)
-    ws = _workspace(lambda: _sizes(B, T, H, C)[2], w.device)
+    ws = _workspace(lambda: _sizes(B, T, H, C)[1], w.device)
     _launch('attn_ln_backward', _bwd_impl, w, q, k, v, a, b, g, params, dy, s, dsT,
             dw, dq, dk, dv, da, db, dg, dparams, ds0, ws)
     return dw, dq, dk, dv, da, db, dg, dparams, ds0
