@@ -55,14 +55,13 @@ def test_a_node_keeps_what_its_backward_reads(B, T, H, ln):
     g = x[0].detach().clone()
     params = torch.ones(3, H * C, device=DEV)
     go = lambda: attn_ln(*x, g, params, C) if ln else attn(*x, C)
-    go()   # (kernels loaded, pools filled)
-    torch.cuda.synchronize()
-    before = torch.cuda.memory_allocated()
+    requested = lambda: torch.cuda.memory_stats()['requested_bytes.all.current']   # (not the pool's blocks, which may be larger)
+    before = requested()
     y = go()
-    held = torch.cuda.memory_allocated() - before
+    held = requested() - before
     saved = (lib.wind_rwkv7_attn_ln_saved_bytes if ln else lib.wind_rwkv7_attn_saved_bytes)(B, T, H, C)
-    wanted = y.numel() * 2 + saved + B * H * C * C * 2   # (sT: a node output, gone where nobody asked for it)
-    assert held <= wanted + 3 * 1024, (held, wanted)     # the pool's granularity, 512 bytes, and the 256 of a call without scratch
+    wanted = y.numel() * 2 + saved
+    assert wanted <= held <= wanted + 256, (held, wanted)   # the 256 of a call without scratch; (sT goes where nobody asked for it)
 
 
 @pytest.mark.gpu
