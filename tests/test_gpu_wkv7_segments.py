@@ -1,8 +1,10 @@
-"""WKV7 on few heads, the sequence cut into segments of uneven lengths, against the way that a call with the least scratch takes."""
+"""WKV7 on few heads, the sequence cut into segments of uneven lengths, against the way that a call with the least scratch takes, and
+against the fp64 oracle with states that outlive a segment: with the decays of the other tests, 0.75 a token, nothing of one is left behind it,
+and what the segments' matrices do to it would not be seen."""
 import pytest
 import torch
 
-from oracle import inputs
+from oracle import inputs, seq_ref
 
 DEV = 'cuda'
 C = 64
@@ -57,3 +59,30 @@ def test_segments_agree_with_the_other_way(B, T, H, segments, least, states):
     for i, (t, r) in enumerate(zip(*out)):
         assert torch.isfinite(t.float()).all(), i
         assert (t.float() - r.float()).norm() <= (4e-3 if t.dtype == torch.bfloat16 and i in (1, 2) else 2e-3) * r.float().norm(), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H,segments', [
+    (1, 4096, 3, 8),      # eight equal ones and the first
+    (1, 5760, 17, 9),     # more than eight
+    (1, 7744, 17, 12),    # as many as there are
+    (1, 3232, 32, 5),     # 202 chunks, uneven
+])
+def test_segments_with_long_memory_against_the_oracle(c_oracle, B, T, H, segments):
+    """Decays of 0.9985 a token and a tenth of the removal: half of what enters a segment leaves it (without it y, sT and the gradients
+    are off by half of themselves).  1e-2: the gate of every bf16 pass."""
+    from wind_rwkv import _native
+    from wind_rwkv.rwkv7.wkv_attn import WindRWKV7
+    assert _native.lib().wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == _scratch(B, T, H, segments)
+    d = inputs.wkv7_inputs(B, T, H, C, seed=T + H, dtype=torch.bfloat16, s0_scale=1.0, dsT_scale=1.0)
+    d['w'], d['b'] = (d['w'].float() - 6).bfloat16(), (d['b'].float() * 0.1).bfloat16()
+    xs = [d[n].to(DEV).requires_grad_() for n in ('w', 'q', 'k', 'v', 'a', 'b')]
+    s0 = d['s0'].to(DEV).requires_grad_()
+    y, sT, _ = WindRWKV7.apply(*xs, s0)
+    torch.autograd.backward([y, sT], [d['dy'].to(DEV), d['dsT'].to(DEV)])
+    args = [d[n] for n in 'qwkvab']
+    ref = list(c_oracle.forward(*args, d['s0'])) + list(c_oracle.backward(*args, d['s0'], d['dy'], d['dsT']))
+    got = [y, sT] + [xs[i].grad for i in (1, 0, 2, 3, 4, 5)] + [s0.grad]
+    errs = {n: seq_ref.rel_err(t.detach().float().cpu(), r) for n, t, r in zip(('y', 'sT', 'dq', 'dw', 'dk', 'dv', 'da', 'db', 'ds0'), got, ref)}
+    print({n: f'{e:.1e}' for n, e in errs.items()})
+    assert all(e <= 1e-2 for e in errs.values()), errs

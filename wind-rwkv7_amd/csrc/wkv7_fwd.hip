@@ -18,11 +18,13 @@ namespace wkv {
 // floats, the state leaving segment g: entry 0 is there.
 // The value rows of a state go through the maps independently, so a block takes 16 of them (four blocks per (batch,
 // head)) and its four wavefronts a block of 16 key columns each: 16 matrix instructions per wavefront and segment,
-// then the row block's four fragments change hands through LDS.  All maps a wavefront needs (PER <= 12: eleven times
-// 20 registers) are requested before the first product.  (One block per (batch, head), a wavefront per 16 rows doing
+// then the row block's four fragments change hands through LDS.  All maps a wavefront needs (PER <= MOST: MOST - 1 times
+// 20 registers) are requested before the first product, and what is requested is read whether there or not: eight segments through the
+// form for twelve took 10.9 us instead of 7.9.  (One block per (batch, head), a wavefront per 16 rows doing
 // all four column blocks: 64 dependent-by-fours matrix instructions per segment, 2.8 us each, 23 us at 8 segments.)
 // ------------------------------------------------------------------------------------------------
 constexpr int CARRY_MAX_SEG = 12;
+template <int MOST>
 __global__ __launch_bounds__(256) void segment_carry_kernel(int PER, const float* __restrict__ maps, float* s_seg) {
     __shared__ f32x4 xch[2][NBLK][WAVE];
     const int jb = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -31,9 +33,9 @@ __global__ __launch_bounds__(256) void segment_carry_kernel(int PER, const float
     f32x4 S[NBLK];
 #pragma unroll
     for (int kb = 0; kb < NBLK; kb++) S[kb] = load_state_frag(s_seg, 1, bh * PER, ib, kb, L);
-    f32x4 n[CARRY_MAX_SEG - 1], mt[CARRY_MAX_SEG - 1][NBLK];
+    f32x4 n[MOST - 1], mt[MOST - 1][NBLK];
 #pragma unroll
-    for (int g = 0; g < CARRY_MAX_SEG - 1; g++) {
+    for (int g = 0; g < MOST - 1; g++) {
         const long e = (long)bh * PER + (g < PER - 1 ? g + 1 : PER - 1);   // (past the end: a valid map, not used)
         const float* N = maps + (e * 2 + 0) * HEAD * HEAD;
         const float* MT = maps + (e * 2 + 1) * HEAD * HEAD;
@@ -43,7 +45,7 @@ __global__ __launch_bounds__(256) void segment_carry_kernel(int PER, const float
             mt[g][kb] = *reinterpret_cast<const f32x4*>(MT + (16 * jb + L.n) * HEAD + 16 * kb + 4 * L.g);
     }
 #pragma unroll
-    for (int g = 0; g < CARRY_MAX_SEG - 1; g++) {
+    for (int g = 0; g < MOST - 1; g++) {
         if (g < PER - 1) {   // (uniform; no load inside)
             f32x4 a0 = mma_f32(n[g], mt[g][0], S[0]), a1 = mma_f32(zero4(), mt[g][1], S[1]);
             a0 = mma_f32(a0, mt[g][2], S[2]);
@@ -141,7 +143,8 @@ size_t scan_workspace_bytes(int B, int T, int H, ScanUse use) {
 size_t scan_workspace_least_bytes(int B, int T, int H) { return segments_bytes(B, H, scan_segments_least(B, T, H)); }
 
 void launch_segment_carry(int BH, int per, const float* maps, float* s_seg, hipStream_t stream) {
-    hipLaunchKernelGGL(segment_carry_kernel, dim3(4 * BH), dim3(256), 0, stream, per, maps, s_seg);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(4 * BH), dim3(256), 0, stream, per, maps, s_seg); };
+    per <= 8 ? go(segment_carry_kernel<8>) : go(segment_carry_kernel<CARRY_MAX_SEG>);
 }
 
 void launch_ln_epilogue(int B, int T, int H, const void* y_wkv, const float* centers, const void* q, const void* k,
