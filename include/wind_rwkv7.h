@@ -72,9 +72,8 @@ int wind_rwkv7_chunk_len(void);
  * gradient kernel): 32 (default) or 16.  At 32 the chunks work in pairs - two-level chunking: 16-token products, a
  * 64x64 checkpoint only every second chunk, and the gradient kernel carries the state across the pair itself, which
  * moves 512 bytes less per token and head in each direction.  At 16 there is a checkpoint per chunk, as in the
- * reference (attn.cu:92-94).  32 applies to sequences with an even number of chunks (long sequences on few heads,
- * which run as segments of at least 32 chunks, always have one); an odd number keeps a state per chunk whatever the setting.  It
- * concerns head size 64; the kernels of the other head sizes keep a state per chunk.  The setting is process-wide and is read by the size queries, the
+ * reference (attn.cu:92-94).  32 applies to sequences with an even number of chunks; an odd number keeps a state per chunk whatever
+ * the setting.  It concerns head size 64; the kernels of the other head sizes keep a state per chunk.  The setting is process-wide and is read by the size queries, the
  * forward and the backward entry points alike: a forward call, the queries that size its buffers and its backward call
  * must all run under the same value.  Results agree within the rounding of a bf16 state (both are held to the same
  * tolerance against the fp64 recurrence).  The reference has no such switch.

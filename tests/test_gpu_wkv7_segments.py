@@ -15,17 +15,22 @@ def _scratch(B, T, H, segments):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('B,T,H,segments,least,states', [
-    (1, 3200, 40, 5, 4, torch.float32),     # 200 chunks, the shortest segments there are; with less scratch as four
-    (1, 3872, 48, 5, 0, torch.bfloat16),    # 242 chunks: no equal segments; with less scratch one block per head
-    (3, 4896, 12, 7, 0, torch.float32),     # 36 pairs, 306 chunks
-    (2, 3328, 16, 5, 4, None),              # 208 chunks, no states in
-    (1, 7744, 24, 10, 4, torch.float32),    # 484 chunks; more than eight segments
+@pytest.mark.parametrize('B,T,H,segments,least,states,interval', [
+    (1, 3200, 40, 5, 4, torch.float32, 32),     # 200 chunks, the shortest segments there are; with less scratch as four
+    (1, 3872, 48, 5, 0, torch.bfloat16, 32),    # 242 chunks: no equal segments; with less scratch one block per head
+    (3, 4896, 12, 7, 0, torch.float32, 32),     # 36 pairs, 306 chunks
+    (3, 4896, 12, 7, 0, torch.float32, 16),     # a state per chunk
+    (2, 3328, 16, 5, 4, None, 32),              # 208 chunks, no states in
+    (1, 7744, 24, 10, 4, torch.float32, 32),    # 484 chunks; more than eight segments
+    (1, 8176, 24, 10, 0, torch.bfloat16, 32),   # 511 chunks: a state per chunk
+    (1, 3216, 40, 5, 0, None, 32),              # 201
+    (2, 6160, 8, 8, 0, torch.float32, 32),      # 385, two blocks per segment
 ])
-def test_segments_agree_with_the_other_way(B, T, H, segments, least, states):
+def test_segments_agree_with_the_other_way(B, T, H, segments, least, states, interval):
     """Every token goes through the same products; only the states at the cuts come from elsewhere, in fp32 (2e-3: a bf16 rounding
     of what follows from them, as between one call and two that carry the state)."""
     from wind_rwkv import _native
+    from wind_rwkv.rwkv7 import set_checkpoint_interval
     lib = _native.lib()
     d = inputs.wkv7_inputs(B, T, H, C, seed=T + H, dtype=torch.bfloat16, s0_scale=0.3, dsT_scale=0.3)
     x = [d[n].to(DEV).contiguous() for n in ('w', 'q', 'k', 'v', 'a', 'b')]
@@ -38,24 +43,28 @@ def test_segments_agree_with_the_other_way(B, T, H, segments, least, states):
     stream = torch.cuda.current_stream().cuda_stream
     mem = lambda n: torch.zeros(n, dtype=torch.uint8, device=DEV)
     nan = lambda t: torch.full_like(t, float('nan'))
-    kept = B * H * (T // 32) * 12288
-    full = _scratch(B, T, H, segments)
-    assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == full and lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == kept + full
-    out = []
-    for f in (full, _scratch(B, T, H, least)):
-        b = kept + (f if f > 256 else 0)
-        ws, saved = mem(max(f, b)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4]))
-        y, y0, sT, s1, ds0 = nan(x[0]), nan(x[0]), nan(s0), nan(s0), nan(s0)
-        grads = [nan(x[0]) for _ in range(6)]
-        _native.check(lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), f, stream))
-        _native.check(lib.wind_rwkv7_attn_backward(*head, *map(ptr, x), ptr(dy), ptr(saved), given[1], *map(ptr, grads), ptr(ds0), ptr(ws), b, stream))
-        scratch = torch.empty_like(saved)
-        _native.check(lib.wind_rwkv7_attn_prefill(*head, *map(ptr, x), given[0], ptr(y0), ptr(scratch), ptr(s1), ptr(ws), f, stream))
-        if f > 256:
-            assert lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), _scratch(B, T, H, least) - 1, stream) == 6
-        torch.cuda.synchronize()
-        assert torch.equal(y, y0) and torch.equal(sT, s1)
-        out.append([y, sT, ds0] + grads)
+    kept = B * H * ((T // 32) * 12288 if T % 32 == 0 and interval == 32 else (T // 16) * 10240)
+    set_checkpoint_interval(interval)
+    try:
+        full = _scratch(B, T, H, segments)
+        assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == full and lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == kept + full
+        out = []
+        for f in (full, _scratch(B, T, H, least)):
+            b = kept + (f if f > 256 else 0)
+            ws, saved = mem(max(f, b)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4]))
+            y, y0, sT, s1, ds0 = nan(x[0]), nan(x[0]), nan(s0), nan(s0), nan(s0)
+            grads = [nan(x[0]) for _ in range(6)]
+            _native.check(lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), f, stream))
+            _native.check(lib.wind_rwkv7_attn_backward(*head, *map(ptr, x), ptr(dy), ptr(saved), given[1], *map(ptr, grads), ptr(ds0), ptr(ws), b, stream))
+            scratch = torch.empty_like(saved)
+            _native.check(lib.wind_rwkv7_attn_prefill(*head, *map(ptr, x), given[0], ptr(y0), ptr(scratch), ptr(s1), ptr(ws), f, stream))
+            if f > 256:
+                assert lib.wind_rwkv7_attn_forward(*head, *map(ptr, x), given[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), _scratch(B, T, H, least) - 1, stream) == 6
+            torch.cuda.synchronize()
+            assert torch.equal(y, y0) and torch.equal(sT, s1)
+            out.append([y, sT, ds0] + grads)
+    finally:
+        set_checkpoint_interval(32)
     for i, (t, r) in enumerate(zip(*out)):
         assert torch.isfinite(t.float()).all(), i
         assert (t.float() - r.float()).norm() <= (4e-3 if t.dtype == torch.bfloat16 and i in (1, 2) else 2e-3) * r.float().norm(), i
@@ -67,6 +76,8 @@ def test_segments_agree_with_the_other_way(B, T, H, segments, least, states):
     (1, 5760, 17, 9),     # more than eight
     (1, 7744, 17, 12),    # as many as there are
     (1, 3232, 32, 5),     # 202 chunks, uneven
+    (1, 3088, 33, 4),     # 193, a state per chunk
+    (1, 6160, 17, 9),     # 385
 ])
 def test_segments_with_long_memory_against_the_oracle(c_oracle, B, T, H, segments):
     """Decays of 0.9985 a token and a tenth of the removal: half of what enters a segment leaves it (without it y, sT and the gradients

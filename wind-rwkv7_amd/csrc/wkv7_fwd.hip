@@ -87,18 +87,21 @@ __global__ __launch_bounds__(256) void ln_epilogue_kernel(int T, int H, int nchu
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
-// Segments per (batch, head) and pass for long sequences on few heads (the whole sequence is one more): up to 8, as many as the
-// (batch, head)s leave compute units, each of 40 chunks or more; 1 = the whole sequence in one block (or two).
+// Segments per (batch, head) and pass for long sequences on few heads (the whole sequence is one more): four up to 8 or 12, as many as the
+// (batch, head)s leave compute units and no more than a fortieth of the chunks; 1 = the whole sequence in one block (or two).  It is cut in
+// one more than that, the first one 0.8 of the others: 200 chunks at 5 are 27 and 34 or 35, 480 at 12 30 and 37 or 38.
 // A segmented pass is two launches of the one-kernel organisation (wkv7_fused.hip: the first segment and the others' affine maps,
 // then the scan proper from the composed entering states) with the carry between them, so it costs twice a launch's fixed
 // 11-14 us, the carry's 3 us per segment, and 1.2 us per chunk and segment instead of 0.55: below four segments
 // it does not pay (measured forward+backward, 12 heads: 1024 tokens 133 us in two segments against 103 in one block).
 // Four segments fit up to a quarter of the compute units' worth of (batch, head) pairs (64: 8192 tokens 876 -> 768 us,
 // 60 pairs: 4096 tokens 459 -> 425 us, 2048 tokens 242 -> 246 us against the unsegmented kernel).
-// scan_segments_least: 4 or 8 of them, in whole chunks each, from 32; what a call with scratch for no more than that runs.
-// scan_segments_most: any number, of uneven lengths if need be, and of an even number of chunks in all.  Forward + backward, us, least -> most:
-// 40 heads x 16384 tokens 1070 (4) -> 920 (6), 48 pairs x 8192 540 (4) -> 507 (5), 40 x 3200 244 -> 224 (5).  Past eight where a segment has
-// one block and not two: 24 x 16384 618 (8) -> 572 (10), 20 x 8192 306 -> 276 (12), 17 x 16384 514 -> 429 (12).
+// scan_segments_least: 4 or 8 of them where that divides the chunks and leaves each 32; what a call with scratch for no more than that
+// runs.  (Segments need not divide the chunks; the condition says how much scratch a call has to bring, which is not to grow.)
+// scan_segments_most: any number.  Forward + backward, us, least -> most: 40 heads x 16384 tokens 1070 (4) -> 920 (6), 48 pairs x 8192 540 (4) ->
+// 507 (5), 40 x 3200 244 -> 224 (5).  Past eight where a segment has one block and not two: 24 x 16384 618 (8) -> 572 (10), 20 x 8192
+// 306 -> 276 (12), 17 x 16384 514 -> 429 (12).  Odd numbers of chunks, which keep a state per chunk: 32 x 16368 1423 (1) -> 810 (8), 24 x 8176 678 -> 341
+// (10), 12 x 12272 840 -> 336 (8), 30 x 4112 336 -> 242 (6), 64 x 4080 467 -> 406 (4), 64 x 2608 299 -> 276 (4).
 static int scan_segments_least(int B, int T, int H) {
     const int BH = B * H, NC = T / CHUNK;
     int g = 1;
@@ -107,7 +110,7 @@ static int scan_segments_least(int B, int T, int H) {
 }
 static int scan_segments_most(int B, int T, int H) {
     const int BH = B * H, NC = T / CHUNK, least = scan_segments_least(B, T, H);
-    const int g = NC % 2 ? 1 : std::min({2 * 8 * BH > compute_units() ? CARRY_MAX_SEG : 8, compute_units() / BH, NC / 40});
+    const int g = std::min({2 * 8 * BH > compute_units() ? CARRY_MAX_SEG : 8, compute_units() / BH, NC / 40});
     return g >= 4 && g > least ? g : least;
 }
 // Chunks of the segment that the first pass walks while it makes the maps of the others.  Its stores make its step longer than
