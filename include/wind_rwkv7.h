@@ -87,13 +87,19 @@ int wind_rwkv7_set_checkpoint_interval(int tokens);
  * ([B,H,T/16,C,C] bf16 there).  Its layout is private to the library. */
 size_t wind_rwkv7_attn_saved_bytes(int B, int T, int H, int C);
 
-/* Bytes of scratch the forward / backward call needs (contents undefined afterwards). */
+/* Bytes of scratch for the forward / backward call (contents undefined afterwards).  The call plans by the size that it is given: these
+ * are what its fastest way takes, with anything more it does the same, and with anything less, down to the least below, it runs another way
+ * (head size 64, few heads: no records of the chunks in memory, fewer segments), whose results differ by roundings. */
 size_t wind_rwkv7_attn_fwd_workspace_bytes(int B, int T, int H, int C);
 size_t wind_rwkv7_attn_bwd_workspace_bytes(int B, int T, int H, int C);
 
 /* Of these for the forward, what wind_rwkv7_attn_forward and wind_rwkv7_attn_ln_forward make use of: a call that keeps something for a
  * backward pass writes its chunks' operands to memory (13.25 KiB each) from more chunks on than one that keeps nothing. */
 size_t wind_rwkv7_attn_train_workspace_bytes(int B, int T, int H, int C);
+
+/* The least that a call accepts (WIND_RWKV7_ERR_WORKSPACE below it); wind_rwkv7_attn_ln_forward and _prefill accept the forward's. */
+size_t wind_rwkv7_attn_fwd_workspace_least_bytes(int B, int T, int H, int C);
+size_t wind_rwkv7_attn_bwd_workspace_least_bytes(int B, int T, int H, int C);
 
 /* y, sT = WKV7(w, q, k, v, a, b, s0), and `s` for backward.
  * Replaces cuda_forward (attn.cu:108-128) / the operator wind::forward (attn.cpp:10-13,25).
@@ -168,6 +174,7 @@ int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state
 size_t wind_rwkv7_attn_ln_saved_bytes(int B, int T, int H, int C);
 size_t wind_rwkv7_attn_ln_fwd_workspace_bytes(int B, int T, int H, int C);
 size_t wind_rwkv7_attn_ln_bwd_workspace_bytes(int B, int T, int H, int C);
+size_t wind_rwkv7_attn_ln_bwd_workspace_least_bytes(int B, int T, int H, int C);
 
 int wind_rwkv7_attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
                                const void* w, const void* q, const void* k, const void* v,

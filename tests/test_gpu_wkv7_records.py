@@ -13,16 +13,6 @@ DEV = 'cuda'
 C = 64
 
 
-def _least(lib, B, T, H, interval):
-    """(forward, backward) bytes without records: the segments' maps, and what the backward keeps."""
-    NC, segments = T // 16, 1
-    while segments < 8 and B * H * segments * 2 <= 256 and NC % (segments * 2) == 0 and NC // (segments * 2) >= 32:
-        segments *= 2
-    maps = B * H * segments * 3 * C * C * 4 if segments >= 4 else 0
-    kept = B * H * (NC // 2 * 12288 if NC % 2 == 0 and interval == 32 else NC * 10240)
-    return max(maps, 256), kept + maps
-
-
 def test_workspace_sizes_at_the_lines_of_the_rule():
     """Records from eight chunks (backward, and a forward that keeps something for it: from 96, or 48 and 2048 in all), for up to a quarter
     of the compute units' worth of (batch, head) pairs and 6144 chunks, and not where a sequence runs as eight segments."""
@@ -34,9 +24,11 @@ def test_workspace_sizes_at_the_lines_of_the_rule():
                                      (1, 4096, 12): (False, False), (1, 4080, 12): (True, True), (1, 4112, 12): (True, True),
                                      (8, 1024, 12): (False, False)}.items():
         chunks = B * H * (T // 16)
-        fwd, bwd = _least(lib, B, T, H, 32)
+        fwd, bwd = lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_least_bytes(B, T, H, C)
         assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == (chunks * 13568 if ahead else fwd), (B, T, H)
         kept = B * H * (T // 32 * 12288 if T % 32 == 0 else T // 16 * 10240)
+        maps = {(1, 1536, 64): 0, (1, 2048, 48): 4, (1, 4096, 12): 8}.get((B, T, H), 0) * B * H * 3 * C * C * 4
+        assert (fwd, bwd) == (max(maps, 256), kept + maps), (B, T, H)
         assert lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == (kept + chunks * 10496 if back else bwd), (B, T, H)
         assert lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == (chunks * 13568 if back else fwd), (B, T, H)
 
@@ -92,10 +84,12 @@ def test_records_give_the_bits_of_the_other_way(B, T, H, state, interval):
     try:
         fwd, bwd = lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C)
         ln_bwd = lib.wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C)
-        least_fwd, least_bwd = _least(lib, B, T, H, interval)
+        least_fwd, least_bwd = lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_least_bytes(B, T, H, C)
+        least_ln_bwd = lib.wind_rwkv7_attn_ln_bwd_workspace_least_bytes(B, T, H, C)
+        assert ln_bwd - least_ln_bwd == bwd - least_bwd
         assert fwd > least_fwd and (bwd > least_bwd) == (T >= 1024)
         out = {}
-        for way, (f, b, lb) in {'records': (fwd, bwd, ln_bwd), 'least': (least_fwd, least_bwd, ln_bwd - (bwd - least_bwd))}.items():
+        for way, (f, b, lb) in {'records': (fwd, bwd, ln_bwd), 'least': (least_fwd, least_bwd, least_ln_bwd)}.items():
             ws, saved, ln_saved = mem(max(f, b, lb)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4])), mem(lib.wind_rwkv7_attn_ln_saved_bytes(*head[:4]))
             y, y0, z, z0 = (nan(x[0]) for _ in range(4))
             sT, s1, t0, t1 = (nan(s0) for _ in range(4))
@@ -112,6 +106,9 @@ def test_records_give_the_bits_of_the_other_way(B, T, H, state, interval):
                                                           ptr(ln_ds0), ptr(ws), lb, stream))
             assert lib.wind_rwkv7_attn_forward(*head, *ins, states[0], ptr(y), ptr(saved), ptr(sT), ptr(ws), least_fwd - 1, stream) == 6
             assert lib.wind_rwkv7_attn_backward(*head, *ins, ptr(dy), ptr(saved), states[1], *map(ptr, grads), ptr(ds0), ptr(ws), least_bwd - 1, stream) == 6
+            assert lib.wind_rwkv7_attn_ln_forward(*head, *ins, *ln, states[0], ptr(z), ptr(ln_saved), ptr(t1), ptr(ws), least_fwd - 1, stream) == 6
+            assert lib.wind_rwkv7_attn_ln_backward(*head, *ins, *ln, ptr(dy), ptr(ln_saved), states[1], *map(ptr, ln_grads), ptr(dparams),
+                                                   ptr(ln_ds0), ptr(ws), least_ln_bwd - 1, stream) == 6
             torch.cuda.synchronize()
             assert torch.equal(y, y0) and torch.equal(sT, s1) and torch.equal(z, z0) and torch.equal(t0, t1) and torch.equal(sT, t1)
             out[way] = dict(y=y, sT=sT, z=z, ds0=ds0, ln_ds0=ln_ds0, dparams=dparams, **{f'd{i}': t for i, t in enumerate(grads)},

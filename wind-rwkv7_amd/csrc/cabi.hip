@@ -58,9 +58,10 @@ int check_workspace(const void* ws, size_t have, size_t need) {
 }
 
 inline long long chunks(int B, int T, int H) { return (long long)B * H * (T / wkv::CHUNK); }
-// One organisation for head size 64: blocks that prepare and scan in one launch (operands through LDS), one or two per
-// (batch, head), or for long sequences on few heads one or two per segment of a (batch, head)'s sequence.  What one
-// direction leaves in memory per chunk: a state + U^T.
+// Head size 64: blocks that prepare and scan in one launch (operands through LDS), one or two per (batch, head), or for long
+// sequences on few heads one or two per segment of a (batch, head)'s sequence; on few heads that are no longer than that a launch
+// that prepares the chunks and one that scans them (scan_plan in wkv7_fwd.hip).  What one direction leaves in memory per chunk: a
+// state + U^T.
 // With an even number of chunks the kernels keep a state only per pair of chunks, in both directions: the
 // forward the state entering the pair (the gradient kernel advances it across the pair's first chunk itself), the
 // backward the dstate arriving at its end.
@@ -79,7 +80,7 @@ inline size_t rec_bwd_bytes(int B, int T, int H, bool ln = false) {
     return align_up((size_t)chunks(B, T, H) * wkv::Saved::BYTES);
 }
 // Scratch of the scan: the chunks' records, or the segments' maps and states.  The size queries ask for what the fastest way takes; a
-// call also accepts the least, with which there are no records.  (The forward's argument is always checked.)
+// call also accepts the least, with which there are no records and fewer segments.  (The forward's argument is always checked.)
 inline size_t scan_bytes(int B, int T, int H, wkv::ScanUse use) { return align_up(wkv::scan_workspace_bytes(B, T, H, use)); }
 inline size_t scan_least_bytes(int B, int T, int H) { return align_up(wkv::scan_workspace_least_bytes(B, T, H)); }
 inline size_t fwd_ws_bytes(int B, int T, int H, wkv::ScanUse use) { return std::max<size_t>(scan_bytes(B, T, H, use), 256); }
@@ -198,6 +199,16 @@ size_t wind_rwkv7_attn_bwd_workspace_bytes(int B, int T, int H, int C) {
     return rec_bwd_bytes(B, T, H) + scan_bytes(B, T, H, wkv::SCAN_BACKWARD);
 }
 
+size_t wind_rwkv7_attn_fwd_workspace_least_bytes(int B, int T, int H, int C) {
+    if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK || C != wkv::HEAD) return wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C);
+    return fwd_ws_least_bytes(B, T, H);
+}
+
+size_t wind_rwkv7_attn_bwd_workspace_least_bytes(int B, int T, int H, int C) {
+    if (check_shape(B, T, H, C, true) != WIND_RWKV7_OK || C != wkv::HEAD) return wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C);
+    return rec_bwd_bytes(B, T, H) + scan_least_bytes(B, T, H);
+}
+
 // wide_centers (head sizes other than 64 only): y is attn_ln's kept output and is written centred, the centres there
 static int attn_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
                         const void* w, const void* q, const void* k, const void* v,
@@ -209,8 +220,7 @@ static int attn_forward(int B, int T, int H, int C, int io_dtype, int state_dtyp
     rc = check_dtypes(io_dtype, state_dtype);
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !y || !s || !sT) return WIND_RWKV7_ERR_NULL_POINTER;   // (s0 may be null: a zero state)
-    rc = check_workspace(workspace, workspace_bytes,
-                         C != wkv::HEAD ? wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) : fwd_ws_least_bytes(B, T, H));
+    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     Stamp st(0, stream);
@@ -286,8 +296,7 @@ int wind_rwkv7_attn_backward(int B, int T, int H, int C, int io_dtype, int state
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !dy || !s) return WIND_RWKV7_ERR_NULL_POINTER;   // (dsT may be null: zero)
     if (!dw || !dq || !dk || !dv || !da || !db) return WIND_RWKV7_ERR_NULL_POINTER;            // (ds0 may be null: not wanted)
-    rc = check_workspace(workspace, workspace_bytes,
-                         C != wkv::HEAD ? wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) : rec_bwd_bytes(B, T, H) + scan_least_bytes(B, T, H));
+    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_bwd_workspace_least_bytes(B, T, H, C));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     Stamp st(1, stream);
@@ -335,6 +344,11 @@ size_t wind_rwkv7_attn_ln_bwd_workspace_bytes(int B, int T, int H, int C) {
     return rec_bwd_bytes(B, T, H, true) + seq_bytes(B, T, H) + ddot_bytes(B, T, H) + dpart_bytes(B, T, H) + scan_bytes(B, T, H, wkv::SCAN_BACKWARD);
 }
 
+size_t wind_rwkv7_attn_ln_bwd_workspace_least_bytes(int B, int T, int H, int C) {
+    const size_t all = wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C);
+    return !all || C != wkv::HEAD ? all : all - scan_bytes(B, T, H, wkv::SCAN_BACKWARD) + scan_least_bytes(B, T, H);
+}
+
 static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
                            const void* w, const void* q, const void* k, const void* v,
                            const void* a, const void* b, const void* g, const void* params,
@@ -346,8 +360,7 @@ static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_d
     rc = check_dtypes(io_dtype, state_dtype);
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !g || !params || !y || !s || !sT) return WIND_RWKV7_ERR_NULL_POINTER;
-    rc = check_workspace(workspace, workspace_bytes,
-                         C != wkv::HEAD ? wind_rwkv7_attn_ln_fwd_workspace_bytes(B, T, H, C) : fwd_ws_least_bytes(B, T, H));
+    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (C != wkv::HEAD) {
@@ -415,9 +428,7 @@ int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int st
     if (rc) return rc;
     if (!w || !q || !k || !v || !a || !b || !g || !params || !dy || !s) return WIND_RWKV7_ERR_NULL_POINTER;
     if (!dw || !dq || !dk || !dv || !da || !db || !dg || !dparams) return WIND_RWKV7_ERR_NULL_POINTER;
-    rc = check_workspace(workspace, workspace_bytes,
-                         wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C) -
-                             (C != wkv::HEAD ? 0 : scan_bytes(B, T, H, wkv::SCAN_BACKWARD) - scan_least_bytes(B, T, H)));
+    rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_ln_bwd_workspace_least_bytes(B, T, H, C));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (C != wkv::HEAD) {

@@ -40,6 +40,9 @@ SIGNATURES = {
     'wind_rwkv7_attn_saved_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_fwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_train_workspace_bytes': (_sz, [_i] * 4),
+    'wind_rwkv7_attn_fwd_workspace_least_bytes': (_sz, [_i] * 4),
+    'wind_rwkv7_attn_bwd_workspace_least_bytes': (_sz, [_i] * 4),
+    'wind_rwkv7_attn_ln_bwd_workspace_least_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_forward': (_i, [_i] * 6 + [_vp] * 7 + [_vp] * 3 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_prefill': (_i, [_i] * 6 + [_vp] * 7 + [_vp] * 3 + [_vp, _sz, _vp]),
