@@ -125,10 +125,13 @@ def test_large_mean_both_forward_forms(c_oracle):
         assert e_few < 0.1 and e_many < 0.1 and abs(e_few - e_many) < 0.3 * max(e_few, e_many), (name, e_few, e_many)
 
 
-def test_large_mean_long_sequence_on_few_heads(c_oracle):
-    """The same property on the path of long sequences on few heads (2 heads, 2048 tokens: the sequence in segments, a
-    block per segment): the kept output is written centred there too."""
-    d = _offset_inputs(1, 2048, 2, 20.0, seed=273)
+@pytest.mark.parametrize('T,scratch', [(2048, 2 * 128 * 13568), (4096, 2 * 8 * 3 * 64 * 64 * 4)])
+def test_large_mean_long_sequence_on_few_heads(c_oracle, T, scratch):
+    """The same property where few heads run by records of their chunks (2 heads, 2048 tokens) and as eight segments of a sequence
+    (4096): the kept output is written centred there too."""
+    from wind_rwkv import _native
+    assert _native.lib().wind_rwkv7_attn_train_workspace_bytes(1, T, 2, 64) == scratch
+    d = _offset_inputs(1, T, 2, 20.0, seed=273)
     got, ref = device(d, torch.float32), oracle(c_oracle, d, torch.float32)
     for name in ('y', 'dq', 'dk', 'dv', 'dg'):
         err = seq_ref.rel_err(got[name], ref[name])

@@ -53,13 +53,13 @@ def check(got, ref, tol=TOL_BF16):
     (2, 64, 3, torch.float32, 0.1, 0.1),
     (2, 64, 3, torch.bfloat16, 0.1, 0.1),       # the reference's state dtype
     (3, 272, 5, torch.float32, 0.1, 0.0),       # chunk count not a multiple of the scan's prefetch depth
-    (1, 2048, 2, torch.float32, 0.1, 0.1),
-    (1, 2080, 2, torch.float32, 0.1, 0.1),      # 130 chunks: only two segments would fit, so one block per half head
-    (1, 2112, 2, torch.float32, 0.1, 0.1),      # 132 chunks: four segments of 33, pairs of chunks straddle them
-    (1, 6160, 3, torch.bfloat16, 0.1, 0.1),     # 385 chunks: no even split, two blocks per head over the whole sequence
+    (1, 2048, 2, torch.float32, 0.1, 0.1),      # this one and the next three by records of their chunks
+    (1, 2080, 2, torch.float32, 0.1, 0.1),
+    (1, 2112, 2, torch.float32, 0.1, 0.1),
+    (1, 6160, 3, torch.bfloat16, 0.1, 0.1),     # 385 chunks, a state per chunk
     (25, 32, 12, torch.float32, 0.1, 0.1),      # 300 (batch, head) pairs: more blocks than compute units
     (19, 48, 12, torch.float32, 0.0, 0.1),      # 228 pairs
-    (5, 2048, 12, torch.float32, 0.1, 0.1),     # 60 pairs: four segments of 32 chunks, one block per segment
+    (5, 2048, 12, torch.float32, 0.1, 0.1),     # 60 pairs, 7680 chunks: four segments, one block per segment
     (1, 4096, 3, torch.bfloat16, 0.1, 0.1),     # eight segments, two blocks per segment
 ])
 def test_parity_small(c_oracle, B, T, H, state_dtype, s0s, dsTs):
@@ -173,8 +173,8 @@ def test_interval_change_between_forward_and_backward_is_an_error():
 
 
 def test_parity_long_sequences_on_a_quarter_of_the_machine(c_oracle):
-    """64 (batch, head) pairs x 2048 tokens: more pairs than the segmented scans take (a fifth of the compute units), so
-    the one-kernel organisation walks 128 chunks per head; y, sT, the six gradients and ds0 against the oracle."""
+    """64 (batch, head) pairs x 2048 tokens: as many pairs as the segmented scans take (a quarter of the compute units), four
+    segments each; y, sT, the six gradients and ds0 against the oracle."""
     d = inputs.wkv7_inputs(2, 2048, 32, 64, seed=61, dtype=torch.bfloat16, s0_scale=0.1, dsT_scale=0.1)
     errs = check(run_device(d, torch.float32), run_oracle(c_oracle, d, torch.float32))
     print('B2 T2048 H32:', {k: f'{v:.2e}' for k, v in errs.items()})

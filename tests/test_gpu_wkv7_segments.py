@@ -49,6 +49,7 @@ def test_segments_agree_with_the_other_way(B, T, H, segments, least, states, int
         full = _scratch(B, T, H, segments)
         assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == full and lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == kept + full
         out = []
+        assert lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C) == _scratch(B, T, H, least)
         for f in (full, _scratch(B, T, H, least)):
             b = kept + (f if f > 256 else 0)
             ws, saved = mem(max(f, b)), mem(lib.wind_rwkv7_attn_saved_bytes(*head[:4]))
@@ -97,3 +98,57 @@ def test_segments_with_long_memory_against_the_oracle(c_oracle, B, T, H, segment
     errs = {n: seq_ref.rel_err(t.detach().float().cpu(), r) for n, t, r in zip(('y', 'sT', 'dq', 'dw', 'dk', 'dv', 'da', 'db', 'ds0'), got, ref)}
     print({n: f'{e:.1e}' for n, e in errs.items()})
     assert all(e <= 1e-2 for e in errs.values()), errs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H,segments', [
+    (1, 3872, 48, 5),     # 242 chunks
+    (1, 8176, 24, 10),    # 511: a state per chunk
+    (1, 4096, 3, 8),      # two blocks per segment
+])
+def test_attn_ln_in_segments_agrees_with_the_other_way(B, T, H, segments):
+    """attn_ln's kept output centred in segments, its parameter gradients beside or behind the segmented scan, and the workspace's order, against
+    the call with the least scratch (eight equal segments have no other way: there the plain operator and the epilogue's kernels)."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    d = inputs.attn_ln_inputs(B, T, H, C, seed=T + H, dtype=torch.bfloat16)
+    x = [d[n].to(DEV).contiguous() for n in ('w', 'q', 'k', 'v', 'a', 'b', 'g')]
+    gen = torch.Generator().manual_seed(T)
+    s0, dsT = ((torch.randn(B, H, C, C, generator=gen)).to(DEV) for _ in range(2))
+    dy, params = d['dy'].to(DEV).contiguous(), d['params'].to(DEV)
+    ptr = lambda t: t.data_ptr()
+    nan = lambda t: torch.full_like(t, float('nan'))
+    mem = lambda n: torch.zeros(n, dtype=torch.uint8, device=DEV)
+    head = (B, T, H, C, _native.BF16, _native.F32)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == _scratch(B, T, H, segments)
+    fwd = lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C), lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C)
+    bwd = lib.wind_rwkv7_attn_ln_bwd_workspace_bytes(B, T, H, C), lib.wind_rwkv7_attn_ln_bwd_workspace_least_bytes(B, T, H, C)
+    out = []
+    for f, b in zip(fwd, bwd):
+        guard = 4096
+        ws, saved = mem(max(f, b) + guard), mem(lib.wind_rwkv7_attn_ln_saved_bytes(B, T, H, C))
+        y, sT, ds0, dparams, grads = nan(dy), nan(s0), nan(s0), nan(params), [nan(dy) for _ in range(7)]
+        ws[f:] = 77
+        _native.check(lib.wind_rwkv7_attn_ln_forward(*head, *map(ptr, x), ptr(params), ptr(s0), ptr(y), ptr(saved), ptr(sT), ptr(ws), f, stream))
+        assert (ws[f:] == 77).all()
+        ws[b:] = 77
+        _native.check(lib.wind_rwkv7_attn_ln_backward(*head, *map(ptr, x), ptr(params), ptr(dy), ptr(saved), ptr(dsT), *map(ptr, grads), ptr(dparams),
+                                                      ptr(ds0), ptr(ws), b, stream))
+        assert (ws[b:] == 77).all()
+        out.append(dict(y=y, sT=sT, ds0=ds0, dparams=dparams, **dict(zip(('dw', 'dq', 'dk', 'dv', 'da', 'db', 'dg'), grads))))
+    if fwd[0] == fwd[1]:   # one way only: the plain operator, the epilogue on its output and back
+        out[1] = {}
+        from wind_rwkv.rwkv7.wkv_attn import WindRWKV7
+        seqs = [t.clone().requires_grad_() for t in x[:6]]
+        h0 = s0.clone().requires_grad_()
+        y, sT, _ = WindRWKV7.apply(*seqs, h0)
+        leaf = {n: t.detach().double().requires_grad_() for n, t in dict(y=y, q=x[1], k=x[2], v=x[3], g=x[6], p=params).items()}
+        z = seq_ref.attn_ln_epilogue(leaf['y'], leaf['q'], leaf['k'], leaf['v'], leaf['g'], leaf['p'])
+        z.backward(dy.double())
+        torch.autograd.backward([y, sT], [leaf['y'].grad.bfloat16(), dsT])
+        out[1] = dict(y=z.detach(), sT=sT, ds0=h0.grad, dparams=leaf['p'].grad, dg=leaf['g'].grad, dw=seqs[0].grad, da=seqs[4].grad, db=seqs[5].grad,
+                      **{'d' + n: seqs[i].grad.double() + leaf[n].grad for n, i in (('q', 1), ('k', 2), ('v', 3))})
+    for n, t in out[0].items():
+        e = seq_ref.rel_err(t.detach().double().cpu(), out[1][n].detach().double().cpu())
+        assert e <= (1e-2 if fwd[0] == fwd[1] else 2e-3), (n, e)
