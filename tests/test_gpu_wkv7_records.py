@@ -15,22 +15,27 @@ C = 64
 
 def test_workspace_sizes_at_the_lines_of_the_rule():
     """Records from eight chunks (backward, and a forward that keeps something for it: from 96, or 48 and 2048 in all), for up to a quarter
-    of the compute units' worth of (batch, head) pairs and 6144 chunks, and not where a sequence runs as eight segments."""
+    of the compute units' worth of (batch, head) pairs and 6144 chunks (forward 5120 where a sequence runs as four segments otherwise, 3584 as
+    five), and not where a sequence runs as six or more."""
     from wind_rwkv import _native
     lib = _native.lib()
-    for (B, T, H), (ahead, back) in {(1, 112, 4): (False, False), (1, 128, 4): (True, False), (1, 1520, 4): (True, False), (1, 1536, 4): (True, True),
-                                     (1, 752, 44): (True, False), (1, 768, 43): (True, True), (1, 768, 42): (True, False), (1, 1536, 64): (True, True),
-                                     (1, 1536, 65): (False, False), (1, 2048, 48): (True, True), (1, 2064, 48): (False, False),
-                                     (1, 4096, 12): (False, False), (1, 4080, 12): (True, True), (1, 4112, 12): (True, True),
-                                     (8, 1024, 12): (False, False)}.items():
+    # prefill, training forward, backward by records; equal segments of the least scratch, and the segments otherwise
+    for (B, T, H), (ahead, train, back, least, most) in {
+            (1, 112, 4): (False, False, False, 0, 0), (1, 128, 4): (True, False, False, 0, 0), (1, 1520, 4): (True, False, False, 0, 0),
+            (1, 1536, 4): (True, True, True, 0, 0), (1, 752, 44): (True, False, False, 0, 0), (1, 768, 43): (True, True, True, 0, 0),
+            (1, 768, 42): (True, False, False, 0, 0), (1, 1536, 64): (True, True, True, 0, 0), (1, 1536, 65): (False, False, False, 0, 0),
+            (1, 2048, 40): (True, True, True, 4, 4), (1, 2048, 48): (False, False, True, 4, 4), (1, 2064, 48): (False, False, False, 0, 0),
+            (1, 3200, 17): (True, True, True, 4, 5), (1, 3200, 18): (False, False, True, 4, 5), (1, 3216, 12): (True, True, True, 0, 5),
+            (1, 3840, 12): (False, False, False, 4, 6), (1, 4096, 12): (False, False, False, 8, 8), (1, 4080, 12): (False, False, False, 0, 6),
+            (8, 1024, 12): (False, False, False, 0, 0)}.items():
         chunks = B * H * (T // 16)
-        fwd, bwd = lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C), lib.wind_rwkv7_attn_bwd_workspace_least_bytes(B, T, H, C)
-        assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == (chunks * 13568 if ahead else fwd), (B, T, H)
         kept = B * H * (T // 32 * 12288 if T % 32 == 0 else T // 16 * 10240)
-        maps = {(1, 1536, 64): 0, (1, 2048, 48): 4, (1, 4096, 12): 8}.get((B, T, H), 0) * B * H * 3 * C * C * 4
-        assert (fwd, bwd) == (max(maps, 256), kept + maps), (B, T, H)
-        assert lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == (kept + chunks * 10496 if back else bwd), (B, T, H)
-        assert lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == (chunks * 13568 if back else fwd), (B, T, H)
+        maps = lambda segments: segments * B * H * 3 * C * C * 4
+        assert lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, C) == (chunks * 13568 if ahead else max(maps(most), 256)), (B, T, H)
+        assert lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) == (chunks * 13568 if train else max(maps(most), 256)), (B, T, H)
+        assert lib.wind_rwkv7_attn_bwd_workspace_bytes(B, T, H, C) == kept + (chunks * 10496 if back else maps(most)), (B, T, H)
+        assert lib.wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C) == max(maps(least), 256), (B, T, H)
+        assert lib.wind_rwkv7_attn_bwd_workspace_least_bytes(B, T, H, C) == kept + maps(least), (B, T, H)
 
 
 @pytest.mark.gpu

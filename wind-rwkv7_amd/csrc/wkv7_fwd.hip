@@ -124,13 +124,17 @@ int first_segment_chunks(int NC, int per) { return (int)(NC * 0.8 / (per + 0.8))
 //     the scratch).  A training pass has two launches more then, and a short one waits for its launches: eager forward + backward
 //     of attn on a host that takes 88-95 us for it, 4 x 512 tokens x 12 heads 88-91 -> 92-95, 4 x 768 99 -> 83, 1 x 1024 x 4 95 -> 95,
 //     4 x 1024 x 12 116 -> 95, of attn_ln 1 x 1024 x 4 115 -> 120.  So there from 96 chunks on, or 48 and 2048 in all;
-//   * up to 6144 chunks in all, 80 MiB of records, behind which writing and reading them is what counts (48 pairs x 2048 tokens 65 -> 56 /
-//     118 -> 108; 64 x 2048 71 -> 74 / 137 -> 136; 96 x 1024 above);
-//   * not where a sequence runs as eight segments (12 pairs x 4096 tokens 61 -> 69 / 94 -> 100; as four: 12 x 2048 57 -> 41 / 75 -> 57,
-//     32 x 3200 80 -> 73 / 143 -> 137).
+//   * up to 6144 chunks in all, 80 MiB of records, behind which writing and reading them is what counts (96 x 1024 above);
+//   * less far where the sequence runs as segments otherwise, and not at all where those are six or more.  Forward keeping a state
+//     per pair / whole backward, us, segments -> records, four: 24 heads x 3072 tokens 65 -> 64 / 113 -> 108, 40 x 2048 (5120 chunks) 59 -> 56 / 106 ->
+//     104, 32 x 2560 60 -> 59 / 109 -> 108, 32 x 2576 60 -> 66, 48 x 2048 59 -> 64 / 114 -> 105, 32 x 3072 65 -> 77 / 119 -> 115; five: 16 x 3200 (3200 chunks)
+//     61 -> 60 / 95 -> 88, 20 x 3200 61 -> 64 / 98 -> 92, 24 x 3200 61 -> 66 / 110 -> 112; six: 12 x 3840 62 -> 69 / 95 -> 94, 24 x 3840 71 -> 84 / 118 -> 126;
+//     eight: 8 x 4096 55 -> 68 / 73 -> 84, 4 x 8192 85 -> 127 / 102 -> 132.
 static bool scan_by_records(int B, int T, int H, ScanUse use) {
     const long BH = (long)B * H, NC = T / CHUNK, least = use == SCAN_PREFILL ? 8 : BH * NC >= 2048 ? 48 : 96;
-    return NC >= least && 4 * BH <= compute_units() && BH * NC <= 6144 && scan_segments_least(B, T, H) < 8;
+    const int segments = scan_segments_most(B, T, H);
+    const long most = segments > 5 ? 0 : segments == 1 || use == SCAN_BACKWARD ? 6144 : segments == 4 ? 5120 : 3584;
+    return NC >= least && 4 * BH <= compute_units() && BH * NC <= most;
 }
 static size_t records_bytes(int B, int T, int H, bool fwd) { return (size_t)B * H * (T / CHUNK) * scan_record_bytes(fwd); }
 // N, M^T and the entering state per segment
