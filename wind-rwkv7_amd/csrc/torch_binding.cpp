@@ -144,7 +144,10 @@ void same_interval(const Kept& k) {
 }
 
 // The forward's saved tensor and its scratch: one allocation where the scratch is nothing to speak of, or nothing is kept behind the
-// call; otherwise two, so that a node keeps what its backward pass reads and no more.
+// call; otherwise two, so that a node keeps what its backward pass reads and no more (1 x 1536 tokens x 64 heads 63 MB instead of 142).  Eager
+// passes take the same time either way; in a captured one the gradients get the memory that the scratch leaves, and are slower to
+// write there: 1 x 2048 x 40 152 -> 160 us, 1 x 3072 x 24 171 -> 171, 2 x 1024 x 12 101 -> 101.  So not at other head sizes, whose states are five times
+// the records (8 x 1024 x 6 of 128 226 -> 240).
 struct ForwardMemory {
     Tensor kept, own;
     void* workspace;
@@ -152,7 +155,7 @@ struct ForwardMemory {
     ForwardMemory(const Shape& s, size_t saved_bytes, bool saves, const Tensor& like)
         : bytes(std::max<size_t>((saves ? L.attn_train_workspace_bytes : L.attn_fwd_workspace_bytes)(s.B, s.T, s.H, s.C), 256)) {
         const size_t first = (saved_bytes + 255) / 256 * 256;
-        const bool apart = saves && bytes > 256;
+        const bool apart = saves && bytes > 256 && L.head_size_supported(s.C);
         kept = scratch_bytes(first + (apart ? 0 : bytes), like);
         if (apart) own = scratch_bytes(bytes, like);
         workspace = apart ? ptr(own) : static_cast<char*>(ptr(kept)) + first;
