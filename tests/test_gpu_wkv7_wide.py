@@ -140,3 +140,16 @@ def test_sequences_do_not_depend_on_their_number(B, T, H, C):
         one = run_device({n: t[i:i + 1].contiguous() for n, t in d.items()}, torch.float32)
         for n, t in one.items():
             assert torch.isfinite(t).all() and torch.equal(t, whole[n][i:i + 1]), (i, n)
+
+
+@pytest.mark.parametrize('B,T,H,C', [(20, 48, 15, 16), (2, 48, 3, 16), (20, 48, 15, 32), (9, 80, 16, 32), (3, 48, 3, 32), (20, 48, 8, 48), (4, 48, 24, 48),
+                                     (10, 48, 10, 80), (5, 48, 12, 80)])
+def test_forward_that_keeps_nothing_gives_the_bits_of_the_one_that_does(c_oracle, B, T, H, C):
+    """The scan's forms by working wavefronts (16 channels one, 32 up to two, others up to four: pairs below and past the compute units) and
+    whether states are kept, which decides on the wavefronts beside them."""
+    from wind_rwkv.rwkv7.wkv_attn import fw_attn
+    d = inputs.wkv7_inputs(B, T, H, C, seed=B + C, dtype=torch.bfloat16, s0_scale=0.3, dsT_scale=0.3)
+    got = run_device(d, torch.float32)
+    check(got, run_oracle(c_oracle, d, torch.float32))
+    y, sT, _ = fw_attn(*[d[n].to(DEV) for n in ('w', 'q', 'k', 'v', 'a', 'b')], d['s0'].to(DEV), save=False)
+    assert torch.equal(y.float().cpu(), got['y']) and torch.equal(sT.cpu(), got['sT'])

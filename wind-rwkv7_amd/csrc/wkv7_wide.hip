@@ -306,20 +306,14 @@ struct ScanOps {
     f32x4 fw[NB];
 };
 
-// Loading and storing wavefronts, half each.  A chunk's 26 KiB of operands at head size 128 are 26 loads and LDS writes, which take one
-// wavefront as long as the workers' round.  Forward + backward, us, with 2 (4 workers: 4) / 4 / 6 / 8 of them: two workers, 8 x 1024 tokens x 6
-// heads of 128 216 / 210 / 201 / 205, 8 x 1024 x 8 of 96 187 / 185 / 181 / 176; four, 16 x 1024 x 6 of 128 466 / 466 / 469 / 463, 32 x 1024 x 6 939 /
-// 937 / 938 / 933.  Beside one worker two: 1 x 2048 x 6 of 128 164 / 178, 4 x 1024 x 5 of 112 125 / 132.
-constexpr int scan_helpers(int W) { return W >= 2 ? 8 : 2; }
-
-template <int NB, bool FWD, bool KEEP, int W, bool PAST>
-__global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
+template <int NB, bool FWD, bool KEEP, int W, int HELPERS, bool PAST>
+__global__ __launch_bounds__(64 * (W + HELPERS)) void scan_kernel(int T, int H, int state_f32, const __bf16* __restrict__ rec,
                                                                           const void* __restrict__ s_in, void* __restrict__ s_out,
                                                                           __bf16* __restrict__ y_, __bf16* __restrict__ kept,
                                                                           float* __restrict__ centers) {
     using R = Rec<NB, FWD>;
     using K = Kept<NB>;
-    constexpr int C = 16 * NB, NP = (NB + 1) / 2, LW = scan_helpers(W) / 2;   // LW wavefronts load, as many store; key blocks are contracted two at a time (one 16x16x32 instruction)
+    constexpr int C = 16 * NB, NP = (NB + 1) / 2, LW = HELPERS / 2;   // LW wavefronts load, as many store; key blocks are contracted two at a time (one 16x16x32 instruction)
     constexpr int NU = (R::SHARED_BYTES + 1023) / 1024;   // units of 1 KiB (16 bytes per lane) of the shared run; then one per working wavefront
     constexpr int UPW = (NU + W + LW - 1) / LW;           // units per loading wavefront
     constexpr int SLOT = (NU + W) * 1024, SLOTS = 3, DG = 3;    // ring; chunks a fetch runs ahead of its hand-over
@@ -380,9 +374,14 @@ __global__ __launch_bounds__(64 * (W + scan_helpers(W))) void scan_kernel(int T,
 #pragma unroll
                 for (int e = ht; e < 32 * W; e += 64 * LW) {
                     const int token = e / (2 * W), piece = e % (2 * W);
-                    if (piece / 2 < blocks)
-                        store_streamed(y_ + ca.row0 + (long)token * ca.ld + 16 * ib0 + 8 * piece,
-                                       *reinterpret_cast<const f32x4*>(from + KEPT_BYTES + e * 16));
+                    if (piece / 2 < blocks) {
+                        const f32x4 x = *reinterpret_cast<const f32x4*>(from + KEPT_BYTES + e * 16);
+                        __bf16* const to = y_ + ca.row0 + (long)token * ca.ld + 16 * ib0 + 8 * piece;
+                        // (past the caches, but not rows of 64 bytes or less in a pass that writes nothing else: 64 x 512 tokens x 48 heads of 16
+                        // 308 -> 297 us, 32 x 512 x 16 of 32 72.5 -> 70.5; of 96 bytes 16 x 1024 x 12 84 past them, 87 through them)
+                        if constexpr (KEEP || NB > 2) store_streamed(to, x);
+                        else *reinterpret_cast<f32x4*>(to) = x;
+                    }
                 }
                 if (centers != nullptr && ht < 16 * W) {
                     const int token = ht / W, blk = ht % W;
@@ -794,10 +793,10 @@ constexpr size_t kept_bytes() { return (size_t)Kept<NB>::ELEMS * sizeof(__bf16);
 inline const __bf16* c(const void* p) { return static_cast<const __bf16*>(p); }
 inline __bf16* m(void* p) { return static_cast<__bf16*>(p); }
 
-// Value blocks per block of the scan: the fewest of 1, 2, 4 that still leave every block a compute unit of its own.
+// Value blocks per block of the scan: the fewest of 1, 2, 4 that still leave every block a compute unit of its own, and no more than there are.
 inline int scan_rows(int BH, int NB) {
     for (int rows = 1; rows < 4; rows *= 2) {
-        if ((long)BH * ((NB + rows - 1) / rows) <= compute_units()) return rows;
+        if (rows >= NB || (long)BH * ((NB + rows - 1) / rows) <= compute_units()) return rows;
     }
     return 4;
 }
@@ -825,17 +824,32 @@ struct PastCaches {
 template <int NB, bool FWD, bool KEEP>
 void scan(int B, int T, int H, int state_f32, const __bf16* rec, const void* s_in, void* s_out, __bf16* y, __bf16* kept, float* centers,
           hipStream_t stream) {
-    auto launch = [&](auto width, auto past) {
-        constexpr int W = decltype(width)::value;
-        hipLaunchKernelGGL((scan_kernel<NB, FWD, KEEP, W, decltype(past)::value>), dim3(B * H, (NB + W - 1) / W), dim3(64 * (W + scan_helpers(W))), 0,
+    auto launch = [&](auto width, auto helpers, auto past) {
+        constexpr int W = decltype(width)::value, HELPERS = decltype(helpers)::value;
+        hipLaunchKernelGGL((scan_kernel<NB, FWD, KEEP, W, HELPERS, decltype(past)::value>), dim3(B * H, (NB + W - 1) / W), dim3(64 * (W + HELPERS)), 0,
                            stream, T, H, state_f32, rec, s_in, s_out, y, kept, centers);
     };
+    // Loading and storing wavefronts, half each.  A chunk's 26 KiB of operands at head size 128 are 26 loads and LDS writes, which take one
+    // wavefront as long as the workers' round.  Forward + backward, us, with 2 (4 workers: 4) / 4 / 6 / 8 of them: two workers, 8 x 1024 tokens x 6
+    // heads of 128 216 / 210 / 201 / 205, 8 x 1024 x 8 of 96 187 / 185 / 181 / 176; four, 16 x 1024 x 6 of 128 466 / 466 / 469 / 463, 32 x 1024 x 6 939 /
+    // 937 / 938 / 933.  Beside one worker two: 1 x 2048 x 6 of 128 164 / 178, 4 x 1024 x 5 of 112 125 / 132.
+    // Four where there is less to move: beside four workers that keep no states (forward alone, eight / four: 32 x 64 x 12 of 48 20.3 / 18.2, 32 x 64 x
+    // 8 of 80 20.7 / 18.4, 32 x 512 x 12 of 80 136 / 133), at 16 channels, and at 32 where the blocks share compute units (four workers and eight
+    // helpers / now, forward + backward: 64 x 32 x 48 of 16 67.7 / 54.7, 16 x 256 x 48 105 / 101, 64 x 128 x 16 of 32 131 / 127; forward alone 64 x 32 x 48
+    // 28.6 / 22.6, 16 x 256 x 48 35.9 / 33.4; where they do not 16 x 512 x 12 of 32 85 / 89).
+    using std::integral_constant;
     auto go = [&](auto past) {
-        switch (scan_rows(B * H, NB)) {
-            case 1: launch(std::integral_constant<int, 1>(), past); break;
-            case 2: launch(std::integral_constant<int, 2>(), past); break;
-            default: launch(std::integral_constant<int, 4>(), past);
+        const int rows = scan_rows(B * H, NB);
+        if constexpr (NB > 2) {
+            if (rows == 4) return launch(integral_constant<int, 4>(), integral_constant<int, KEEP ? 8 : 4>(), past);
         }
+        if constexpr (NB == 2) {
+            if (rows == 2 && B * H > compute_units()) return launch(integral_constant<int, 2>(), integral_constant<int, 4>(), past);
+        }
+        if constexpr (NB > 1) {
+            if (rows == 2) return launch(integral_constant<int, 2>(), integral_constant<int, 8>(), past);
+        }
+        launch(integral_constant<int, 1>(), integral_constant<int, NB == 1 ? 4 : 2>(), past);
     };
     if constexpr (KEEP && !PastCaches::whole_halves(NB)) {
         if (!PastCaches(B, T, H, NB).kept) {
