@@ -234,6 +234,12 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
 // kernel reads whole lines for the last time (load_streamed); of half lines they are slower: 8 x 2048 x 12 253 -> 269.
 // What the next kernel reads stays in the caches: the chunks' records of other head sizes written past them 220 -> 262 us at 8 x 1024 x 6 x 128,
 // the states of a decoding step 45 -> 46 (read past them as well: 53), attn_ln's kept output out of the one-kernel form 743 -> 751.
+// Of what the next kernel of attn_ln or of the block reads, it made no difference or was better past them, each on its own (replayed passes on
+// three sets of tensors, us, past / through): the WKV7 output of two blocks per head, half a line each, with its centres 8 x 1024 x 12 195.5 /
+// 195, 4 x 1024 x 12 131.5 / 133.5, 16 x 512 x 8 143 / 141.5, 1 x 8192 x 32 523 / 523.5, in plain attn 8 x 1024 x 12 140.4 / 139.6, 4 x 2048 x 24 270 / 270,
+// 1 x 8192 x 32 371 / 375; the epilogue's output 195.5 / 196.5, 131.5 / 132.5, 523 / 525.5; its dg 195.5 / 197, 131.5 / 134; attn_ln's gradients, half lines,
+// 195.5 / 199, 131.5 / 135, 113.8 / 118.4 (8 x 512 x 12).  The block 8 x 1024 x 12: 604 past, 601 / 604 / 602 / 607 through.
+// On a pass so small that nothing leaves the caches the stores cost 0.6 us in all: 1 x 256 x 4 48.8 past, 48.0 through.
 constexpr int STREAMED = 2;   // of a buffer store
 template <class V>
 __device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontemporal_store(x, static_cast<V*>(to)); }

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         }
         return x;
     };
-    // Whole lines (see WholeLines): as half lines past the caches 73.7 MB of gradients at 8 x 1024 tokens x 12 heads reached memory as 80.4,
+    // Whole lines (see WholeLines): as half lines past the caches 75.5 MB of gradients at 8 x 1024 tokens x 12 heads reached memory as 82.4,
     // and forward + backward of attn took, us: 16 x 1024 x 12 199 (now 192), 32 x 1024 x 12 411 (397), 64 x 1024 x 12 757 (through the caches
     // 752, now 730-741), 1 x 16384 x 32 680 (670), 8 x 2048 x 12 247 (241).
     const unsigned put_off = (unsigned)(WholeLines::row(L) * H * HEAD) * 2 + 16 * WholeLines::piece(L);
