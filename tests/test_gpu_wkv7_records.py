@@ -40,10 +40,10 @@ def test_workspace_sizes_at_the_lines_of_the_rule():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('ln', [False, True])
-@pytest.mark.parametrize('B,T,H', [(1, 1536, 64), (1, 496, 64), (1, 256, 4), (1, 8192, 8)])
-def test_a_node_keeps_what_its_backward_reads(B, T, H, ln):
-    """Between forward and backward a node holds the saved tensor beside its outputs and not the scan's scratch: records (6144 chunks,
-    80 MiB), records that only a forward without gradients would write (64 pairs x 31 chunks), none, segments' maps."""
+@pytest.mark.parametrize('B,T,H,scratch', [(1, 1536, 64, False), (1, 496, 64, False), (1, 256, 4, False), (1, 1536, 4, True)])
+def test_a_node_keeps_what_its_backward_reads(B, T, H, scratch, ln):
+    """Between forward and backward a node holds the saved tensor beside its outputs, and of the scan's scratch no more than 32 MiB: records
+    (6144 chunks, 80 MiB), records that only a forward without gradients would write (64 pairs x 31 chunks), none, few of them."""
     from wind_rwkv import _native
     from wind_rwkv.rwkv7 import attn, attn_ln
     lib = _native.lib()
@@ -58,6 +58,9 @@ def test_a_node_keeps_what_its_backward_reads(B, T, H, ln):
     held = requested() - before
     saved = (lib.wind_rwkv7_attn_ln_saved_bytes if ln else lib.wind_rwkv7_attn_saved_bytes)(B, T, H, C)
     wanted = y.numel() * 2 + saved
+    if scratch:
+        wanted += lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C)
+        assert B * H * T // 16 * 13568 == lib.wind_rwkv7_attn_train_workspace_bytes(B, T, H, C) <= 32 << 20
     assert wanted <= held <= wanted + 256, (held, wanted)   # the 256 of a call without scratch; (sT goes where nobody asked for it)
 
 

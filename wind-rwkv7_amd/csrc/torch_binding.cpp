@@ -143,21 +143,24 @@ void same_interval(const Kept& k) {
                 "): set it between whole forward + backward passes only");
 }
 
-// The forward's saved tensor and its scratch: one allocation where the scratch is nothing to speak of, or nothing is kept behind the
-// call; otherwise two, so that a node keeps what its backward pass reads and no more (1 x 1536 tokens x 64 heads 63 MB instead of 142).  Eager
-// passes take the same time either way; in a captured one the gradients get the memory that the scratch leaves, and are slower to
-// write there: 1 x 2048 x 40 152 -> 160 us, 1 x 3072 x 24 171 -> 171, 2 x 1024 x 12 101 -> 101.  So not at other head sizes, whose states are five times
-// the records (8 x 1024 x 6 of 128 226 -> 240).
+// The forward's saved tensor and its scratch: two allocations where the scratch is large, so that a node keeps what its backward pass
+// reads and no more (1 x 1536 tokens x 64 heads 63 MB instead of 142), and the second as large as the backward's workspace where they are of a
+// size, so that the pool hands it on.  Forward + backward in a captured pass, us, one allocation / two / two of a size: 1 x 2048 x 40 152 / 160 /
+// 149 (the gradients get the scratch's memory where the sizes differ), 1 x 1536 x 64 173 / 176 / 150, 1 x 2560 x 20 146 / - / 135, attn_ln 4 x 1024 x 12
+// 132 / 132 / 123; eager the same.
+// One allocation below 32 MiB, what the L2s of the eight XCDs hold together: there memory that another XCD has just used costs more
+// than it saves (1 x 1536 x 8 heads 76.5 / - / 82.7, 1 x 1536 x 16 83.5 / - / 86.5).  And at other head sizes, whose states are five times the
+// records: 8 x 1024 x 6 of 128 226 / 240 / 226, 2 x 512 x 6 77 / 77 / 84.
 struct ForwardMemory {
     Tensor kept, own;
     void* workspace;
     size_t bytes;
-    ForwardMemory(const Shape& s, size_t saved_bytes, bool saves, const Tensor& like)
+    ForwardMemory(const Shape& s, size_t saved_bytes, size_t backward_bytes, bool saves, const Tensor& like)
         : bytes(std::max<size_t>((saves ? L.attn_train_workspace_bytes : L.attn_fwd_workspace_bytes)(s.B, s.T, s.H, s.C), 256)) {
         const size_t first = (saved_bytes + 255) / 256 * 256;
-        const bool apart = saves && bytes > 256 && L.head_size_supported(s.C);
+        const bool apart = saves && bytes > 32 << 20 && L.head_size_supported(s.C);
         kept = scratch_bytes(first + (apart ? 0 : bytes), like);
-        if (apart) own = scratch_bytes(bytes, like);
+        if (apart) own = scratch_bytes(backward_bytes <= 2 * bytes ? std::max(bytes, backward_bytes) : bytes, like);
         workspace = apart ? ptr(own) : static_cast<char*>(ptr(kept)) + first;
     }
 };
@@ -167,7 +170,7 @@ struct Wkv7 : torch::autograd::Function<Wkv7> {
                              const Tensor& b, const Tensor& s0, Tensor* saved) {
         Tensor y = at::empty_like(v);
         Tensor sT = at::empty({s.B, s.H, s.C, s.C}, s0.defined() ? s0.options() : v.options());
-        const ForwardMemory mem(s, saved ? L.attn_saved_bytes(s.B, s.T, s.H, s.C) : 0, saved, v);
+        const ForwardMemory mem(s, saved ? L.attn_saved_bytes(s.B, s.T, s.H, s.C) : 0, L.attn_bwd_workspace_bytes(s.B, s.T, s.H, s.C), saved, v);
         check((saved ? L.attn_forward : L.attn_prefill)(
             s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, state_code(s0), ptr(w), ptr(q), ptr(k), ptr(v), ptr(a), ptr(b), ptr(s0), ptr(y),
             ptr(mem.kept), ptr(sT), mem.workspace, mem.bytes, stream_of(v)));
@@ -192,12 +195,11 @@ struct Wkv7 : torch::autograd::Function<Wkv7> {
         c10::DeviceGuard guard(t[0].device());
         const Tensor dy = contiguous_or_zeros(grads[0], t[3]);
         const Tensor dsT = grads[1].defined() ? grads[1].contiguous() : Tensor();
+        const Tensor mem = scratch_bytes(L.attn_bwd_workspace_bytes(s.B, s.T, s.H, s.C), dy);   // (ahead of the gradients: see ForwardMemory)
         variable_list d(6);
         for (auto& g : d) g = at::empty_like(t[3]);
         Tensor ds0;
         if (kp.has_s0 && ctx->needs_input_grad(6)) ds0 = at::empty({s.B, s.H, s.C, s.C}, t[3].options().dtype(kp.state_type));
-        const size_t ws = L.attn_bwd_workspace_bytes(s.B, s.T, s.H, s.C);
-        const Tensor mem = scratch_bytes(ws, dy);
         check(L.attn_backward(s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, kp.state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16,
                               ptr(t[0]), ptr(t[1]), ptr(t[2]), ptr(t[3]), ptr(t[4]), ptr(t[5]), ptr(dy), ptr(t[6]), ptr(dsT), ptr(d[0]),
                               ptr(d[1]), ptr(d[2]), ptr(d[3]), ptr(d[4]), ptr(d[5]), ptr(ds0), ptr(mem), mem.numel(), stream_of(dy)));
@@ -282,7 +284,7 @@ struct Wkv7Ln : torch::autograd::Function<Wkv7Ln> {
                              const Tensor& b, const Tensor& g, const Tensor& params, const Tensor& s0, Tensor* saved) {
         Tensor y = at::empty_like(v);
         Tensor sT = at::empty({s.B, s.H, s.C, s.C}, s0.defined() ? s0.options() : v.options());
-        const ForwardMemory mem(s, L.attn_ln_saved_bytes(s.B, s.T, s.H, s.C), saved, v);
+        const ForwardMemory mem(s, L.attn_ln_saved_bytes(s.B, s.T, s.H, s.C), L.attn_ln_bwd_workspace_bytes(s.B, s.T, s.H, s.C), saved, v);
         check((saved ? L.attn_ln_forward : L.attn_ln_prefill)(
             s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, state_code(s0), ptr(w), ptr(q), ptr(k), ptr(v), ptr(a), ptr(b), ptr(g), ptr(params),
             ptr(s0), ptr(y), ptr(mem.kept), ptr(sT), mem.workspace, mem.bytes, stream_of(v)));
@@ -307,11 +309,11 @@ struct Wkv7Ln : torch::autograd::Function<Wkv7Ln> {
         c10::DeviceGuard guard(t[0].device());
         const Tensor dy = contiguous_or_zeros(grads[0], t[3]);
         const Tensor dsT = grads[1].defined() ? grads[1].contiguous() : Tensor();
+        const Tensor mem = scratch_bytes(L.attn_ln_bwd_workspace_bytes(s.B, s.T, s.H, s.C), dy);
         variable_list d(7);
         for (auto& x : d) x = at::empty_like(t[3]);
         Tensor dparams = at::empty_like(t[7]), ds0;
         if (kp.has_s0 && ctx->needs_input_grad(8)) ds0 = at::empty({s.B, s.H, s.C, s.C}, t[3].options().dtype(kp.state_type));
-        const Tensor mem = scratch_bytes(L.attn_ln_bwd_workspace_bytes(s.B, s.T, s.H, s.C), dy);
         check(L.attn_ln_backward(s.B, s.T, s.H, s.C, WIND_RWKV7_BF16, kp.state_type == at::kFloat ? WIND_RWKV7_F32 : WIND_RWKV7_BF16,
                                  ptr(t[0]), ptr(t[1]), ptr(t[2]), ptr(t[3]), ptr(t[4]), ptr(t[5]), ptr(t[6]), ptr(t[7]), ptr(dy), ptr(t[8]),
                                  ptr(dsT), ptr(d[0]), ptr(d[1]), ptr(d[2]), ptr(d[3]), ptr(d[4]), ptr(d[5]), ptr(d[6]), ptr(dparams), ptr(ds0),
