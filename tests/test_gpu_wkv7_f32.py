@@ -128,6 +128,40 @@ def test_f32_backward_entry_points_agree(B, T, H, C):
         assert seq_ref.rel_err(h.cpu(), g.cpu()) <= 1e-5, n
 
 
+@pytest.mark.parametrize('B,T,H,C', [(1, 48, 5, 64), (12, 80, 8, 64), (17, 48, 8, 64), (33, 32, 8, 64), (12, 48, 8, 48),
+                                     (2, 48, 3, 128), (5, 80, 8, 128), (9, 48, 8, 128), (5, 48, 8, 112)])
+def test_f32_scan_forms_and_unaligned_sequences(c_oracle, B, T, H, C):
+    """4, 2 and 1 blocks a head of up to 64 channels (2 again past a head per compute unit), 8, 4 and 2 above, against the oracle; and
+    sequences that start one float into an allocation, which the moves read four channels at a time: the same bits."""
+    from wind_rwkv import _native
+    lib = _native.lib()
+    d = inputs.wkv7_inputs(B, T, H, C, seed=600 + B + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
+    args = [d[n] for n in 'qwkvab']
+    stream = torch.cuda.current_stream().cuda_stream
+    state = (B, H, C, C)
+    s0, dsT = d['s0'].float().to(DEV).contiguous(), d['dsT'].float().to(DEV).contiguous()
+    out = {}
+    for shift in (0, 1):
+        def seq(t=None):
+            x = torch.full((B * T * H * C + 4,), float('nan'), device=DEV)[shift:shift + B * T * H * C].view(B, T, H, C)
+            return x if t is None else x.copy_(t)
+        xs, dy = [seq(d[n].float()) for n in NAMES], seq(d['dy'].float())
+        y, grads = seq(), [seq() for _ in range(6)]
+        sT, ds0 = torch.empty(state, device=DEV), torch.empty(state, device=DEV)
+        s = torch.empty(lib.wind_rwkv7_attn_f32_saved_bytes(B, T, H, C) // 4, device=DEV)
+        need = lib.wind_rwkv7_attn_f32_bwd_workspace_bytes(B, T, H, C)
+        ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+        p = lambda *ts: [t.data_ptr() for t in ts]
+        _native.check(lib.wind_rwkv7_attn_f32_forward(B, T, H, C, *p(*xs, s0, y, s, sT), stream))
+        _native.check(lib.wind_rwkv7_attn_f32_backward_split(B, T, H, C, *p(*xs, dy, s, dsT, *grads, ds0), ws.data_ptr(), need, stream))
+        out[shift] = dict(zip(['y', 'sT', 'ds0'] + ['d' + n for n in NAMES], [y, sT, ds0] + grads))
+    ref = dict(zip(['y', 'sT'], c_oracle.forward(*args, d['s0'])))
+    ref.update(zip(['dq', 'dw', 'dk', 'dv', 'da', 'db', 'ds0'], c_oracle.backward(*args, d['s0'], d['dy'], d['dsT'])))
+    for n, t in out[0].items():
+        assert seq_ref.rel_err(t.cpu(), ref[n]) <= TOL, n
+        assert torch.equal(t, out[1][n]), n
+
+
 @pytest.mark.parametrize('C', [16, 64, 80])
 @pytest.mark.parametrize('w', [2.0, 4.5, 30.0])
 def test_f32_strong_decays(c_oracle, C, w):

@@ -79,6 +79,37 @@ def mixed_pairs(asm):
     return found
 
 
+def early_lane_reads(asm):
+    """v_fmac_f32_dpp instructions (written as such in the sources, so that the compiler does not place the two wait states a
+    lane-crossing operand needs behind a vector instruction that writes it) with a writer of that operand less than two before them."""
+    ins = [t.strip() for t in asm.split('\n')]
+    ins = [t for t in ins if t and not t.startswith((';', '.'))]
+    found = []
+    for i, t in enumerate(ins):
+        m = re.match(r'v_fmac_f32_dpp v\d+, v(\d+),', t)
+        if not m:
+            continue
+        waits = 0
+        for p in reversed(ins[max(i - 2, 0):i]):
+            d = re.match(r'v_\w+\s+(v\d+|v\[\d+:\d+\])(?:,\s*(v\d+))?', p)
+            written = _regs(d.group(1)) if d else set()
+            if d and 'swap' in p.split()[0] and d.group(2):
+                written |= _regs(d.group(2))
+            if waits < 2 and (int(m.group(1)) in written or p.endswith(':')):   # (a label: what ran before is not seen here)
+                found.append((p, t))
+            waits += 1 + (int(p.split()[1]) if p.startswith('s_nop') else 0)
+    return found
+
+
+def test_scanner_sees_an_early_lane_read():
+    asm = '''
+        v_mul_f32_e32 v7, v1, v2
+        v_add_f32_e32 v9, v1, v2
+        v_fmac_f32_dpp v3, v7, v4 row_ror:8 row_mask:0xf bank_mask:0xf
+    '''
+    assert len(early_lane_reads(asm)) == 1 and not early_lane_reads(asm.replace('v_add', 's_nop 0\nv_add'))
+
+
 def test_flags_are_the_makefiles():
     assert '--offload-arch=gfx950' in FLAGS and '-O3' in FLAGS
     assert EXTRA['wkv7_fused.hip'] == ['-mllvm', '-amdgpu-mfma-vgpr-form'] and 'expand_loras.hip' not in EXTRA
@@ -119,6 +150,9 @@ def test_no_matrix_instructions_of_different_shapes_chained_through_the_accumula
             results = list(pool.map(compile_one, FILES))
     bad = {name: pairs[:3] for name, asm in results if (pairs := mixed_pairs(asm))}
     assert not bad, bad
+    early = {name: pairs[:3] for name, asm in results if (pairs := early_lane_reads(asm))}
+    assert not early, early
+    assert any('v_fmac_f32_dpp' in asm for _, asm in results)   # (what the scan is for)
     # The WKV7 kernels must not spill to scratch memory.  In the lock-step kernels a spilling wavefront holds up all
     # the others at every barrier; in the gradient kernel every reload of a spilled register makes the compiler wait
     # for ALL outstanding memory operations (scratch accesses count as loads of unknown order), which ends the overlap

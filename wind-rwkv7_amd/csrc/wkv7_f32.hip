@@ -6,20 +6,26 @@
 // the bf16 kernels are within 1e-2.  It is the token-by-token recurrence itself,
 //     sa = S a_t;   S <- S diag(exp(-exp(w_t))) + sa b_t^T + v_t k_t^T;   y_t = S q_t,
 // with the state in registers, spread thin so that a token costs few instructions per wavefront and little LDS
-// traffic: a thread holds R rows x 4 columns.  A block works at a width C of 64 or 128 channels (a smaller head is
-// padded: channels and rows past the head size read as zero and are never written); the C / 4 lanes that share a
-// state row are one DPP row (C = 64) or two neighbouring ones (C = 128), so a row sum (S a, S q, dS k, dS b) is four
-// DPP adds (and one lane swap); a wavefront holds 4 or 2 such row groups, and a column sum over them (S^T dy, dS^T v,
-// ...) is three (one) of gfx950's lane swaps (col_sum4, store_col_sums), then LDS across the wavefronts.  The vectors
-// of a token are read as one 16-byte LDS access each, one token ahead of their use.
+// traffic: a thread holds R rows x 4 or 8 columns, LPR lanes share a row.  A block works at a width C of 64 or 128 channels (a smaller
+// head is padded: channels and rows past the head size read as zero and are never written).  With 16 lanes to a row (a DPP row) a row
+// sum (S a, S q, dS k, dS b) is four DPP adds, with 32 one lane swap more, with 8 three; a column sum over the row groups of a wavefront
+// (S^T dy, dS^T v, ...) is three (one) of gfx950's lane swaps (col_sum4, store_col_sums), then LDS across the wavefronts.  The vectors
+// of a token are read one token ahead of their use.
 // The value rows of a state never mix, so a head is cut over blocks by rows (scan_split).  In the scan, four or eight
 // wavefronts of a block carry the recurrence and touch LDS only; four more fetch the next chunk, turn it into operands in
 // the other half of a double buffer and carry the results of the chunk before to memory, with one barrier per chunk.
 // (Staging by the recurrence's own wavefronts, between barriers, was a fifth of its time: 227 -> 183 us at 8 x 1024 tokens
-// x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  Bound: vector issue, 89 % of the cycles with eight wavefronts of
-// the recurrence on a compute unit, so what can wait is done for many tokens at once: the row sums of S (decay q) for four
-// (quad_sums), what the row vectors add to y once per chunk by the lane that keeps a token (518 -> 463 instructions per
-// chunk; forward / backward scan 183 / 187 -> 166 / 181 us, 6 heads of 128 384 / 375 -> 325 / 336).
+// x 12 heads of 64, 793 -> 388 us at 4096 tokens x 4 heads.)  Bound: vector issue (a wavefront alone on a SIMD gets an instruction in about
+// every seven cycles, two of them one in four) and, with eight columns a lane, LDS reads, so:
+//   * what can wait is done for many tokens at once: the row sums of S (decay q) for four (quad_sums), what the row vectors add to y
+//     once per chunk by the lane that keeps a token;
+//   * the moves take four channels a thread (303 -> 167 vector instructions a chunk);
+//   * 8 lanes and 8 columns instead of 16 and 4 where the head is cut in two or not at all (of 128 channels 16 and 8 instead of 32 and 4):
+//     half as many row sums, 822 instructions a chunk for eight rows instead of 998.  Twice the LDS reads would undo it (8 x 1024 x 12 heads of
+//     64 416 -> 438 us, forward + backward), so a lane reads four of its eight columns, the lane eight away in the DPP row, which has
+//     the same columns of another row, the other four, and they are operands of each other's instructions (fma_other_row).
+// Forward + backward with these three and bkq as floats, us: 8 x 1024 x 12 heads of 64 419 -> 396, 24 x 1024 x 12 1154 -> 1097, 1 x 1024 x 16
+// 235 -> 226, 8 x 1024 x 6 of 128 788 -> 681, 8 x 512 x 8 of 96 422 -> 363, 32 x 128 x 16 of 32 185 -> 168.
 // The forward keeps the state every CHUNK tokens and S a of every token.  The backward is the same scan in the other
 // direction (it keeps the state gradient arriving at every chunk's end and dsa of every token, and leaves dv and ds0)
 // and then a kernel in which every chunk is on its own and makes the other five gradients.
@@ -47,6 +53,7 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float seq4 __attribute__((ext_vector_type(4), aligned(4)));   // four of a sequence's channels, whose address is a float's
 
 // gfx950's lane-swap instructions, one swap and one add for two values at once: v_permlane32_swap exchanges lanes
 // 32-63 of its first register with lanes 0-31 of its second, so with X and Y two values to be summed over the lane
@@ -124,9 +131,25 @@ __device__ __forceinline__ V& at_bytes(float* p, unsigned o) {
     return *reinterpret_cast<V*>(reinterpret_cast<char*>(p) + o);
 }
 
+// the value of the lane eight away in a DPP row (row_ror 8), as an operand of the instruction that uses it
+__device__ __forceinline__ float other_row(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, true));
+}
+
+// acc + other_row(x) y (the compiler does not make a multiply-add of such an operand)
+__device__ __forceinline__ float fma_other_row(float x, float y, float acc) {
+    asm("v_fmac_f32_dpp %0, %1, %2 row_ror:8 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(x), "v"(y));
+    return acc;
+}
+
 // sum over the LPR lanes that share a state row (16: a DPP row; 32: two neighbouring DPP rows), result in all of them
 template <int LPR>
 __device__ __forceinline__ float row_sum(float x) {
+    if constexpr (LPR == 8) {
+        x += dpp<0xB1>(x);     // quad_perm [1,0,3,2]
+        x += dpp<0x4E>(x);     // quad_perm [2,3,0,1]
+        return x + dpp<0x141>(x);   // row_half_mirror
+    }
     x = row_sum16(x);
     if constexpr (LPR == 32) x = swap_add16(x, x);   // both operands the same: every lane gets this row plus its neighbour
     return x;
@@ -145,22 +168,35 @@ __device__ __forceinline__ void store_col_sums(float* to, f4 p, int col0, int ib
 }
 
 // Several values at once summed over lanes, each lane ending up with ONE of the sums: a halving of the values is a select of
-// what a lane keeps, one of what it gives away and an add.  pair_sums: over the 64 lanes, lane l gets the sum of x z (l even)
-// or y z (l odd); a multiply-add takes the kept product, which is not rounded by itself.  quad_sums: over the LPR lanes of a
-// state row, lane l gets that of x[l % 4], in eleven instructions (and a swap) for four sums that would be sixteen one by
-// one, four swaps and four selects.
-__device__ __forceinline__ float pair_sums(float x, float y, float z, int lane) {
+// what a lane keeps, one of what it gives away and an add.  pair_sums: over 16 lanes (a DPP row) or 32 (two), lane l gets the sum
+// of x (l even) or y (l odd).  quad_sums: over the LPR lanes of a state row, lane l gets that of x[sums_token(l) % 4], in eleven instructions
+// (and a swap; ten for eight lanes) for four sums that would be sixteen one by one, four swaps and four selects.
+template <int LANES>
+__device__ __forceinline__ float pair_sums(float x, float y, int lane) {
     const bool odd = lane & 1;
-    float s = fmaf(odd ? y : x, z, dpp<0xB1>((odd ? x : y) * z));   // quad_perm [1,0,3,2]
-    s += dpp<0x4E>(s);                                              // quad_perm [2,3,0,1]
-    s += dpp<0x124>(s);                                             // row_ror 4
-    s += dpp<0x128>(s);                                             // row_ror 8
-    s = swap_add16(s, s);
-    return swap_add32(s, s);
+    float s = (odd ? y : x) + dpp<0xB1>(odd ? x : y);   // quad_perm [1,0,3,2]
+    s += dpp<0x4E>(s);                                  // quad_perm [2,3,0,1]
+    s += dpp<0x124>(s);                                 // row_ror 4
+    s += dpp<0x128>(s);                                 // row_ror 8
+    if constexpr (LANES == 32) s = swap_add16(s, s);
+    return s;
+}
+// which of the first min(LPR, 16) tokens a lane's sums are of
+template <int LPR>
+__device__ __forceinline__ int sums_token(int lane_of_row) {
+    if constexpr (LPR == 8) return 2 * (lane_of_row & 2) + (lane_of_row >> 1 & 2) + (lane_of_row & 1);
+    return lane_of_row % 16;
 }
 template <int LPR>
 __device__ __forceinline__ float quad_sums(const float (&x)[4], int lane) {
-    const bool odd = lane & 1, upper = lane & 2;
+    const bool odd = lane & 1;
+    if constexpr (LPR == 8) {
+        const bool upper = lane & 4;   // (the mirror of eight lanes exchanges their halves)
+        const float even = (upper ? x[2] : x[0]) + dpp<0x141>(upper ? x[0] : x[2]), odds = (upper ? x[3] : x[1]) + dpp<0x141>(upper ? x[1] : x[3]);
+        const float s = (odd ? odds : even) + dpp<0xB1>(odd ? even : odds);
+        return s + dpp<0x4E>(s);
+    }
+    const bool upper = lane & 2;
     const float lo = (odd ? x[1] : x[0]) + dpp<0xB1>(odd ? x[0] : x[1]), hi = (odd ? x[3] : x[2]) + dpp<0xB1>(odd ? x[2] : x[3]);
     float s = (upper ? hi : lo) + dpp<0x4E>(upper ? lo : hi);
     s += dpp<0x124>(s);
@@ -178,7 +214,7 @@ __host__ __device__ inline long saved_states(long BH, int T, int C) { return BH 
 // is the forward's step with (a, decay q, b, k, v) in the places of (b, k, a, decay q, dy): two row sums on the state
 // before its update, a rank-one term with the first of them and one with the row vector.  v, s0, y, ckpt, sT are then
 // dy, dsT, dv, the workspace of the gradient kernel below (E arriving at every chunk's end, dsa of every token) and ds0.
-template <int C, int R, int NW, int NP, bool FULL, bool ADJ>
+template <int C, int LPR, int R, int NW, int NP, bool FULL, bool ADJ>
 __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, int H, int CR, const float* __restrict__ w,
                                                              const float* __restrict__ q, const float* __restrict__ k,
                                                              const float* __restrict__ v, const float* __restrict__ a,
@@ -186,16 +222,22 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
                                                              float* __restrict__ y, float* __restrict__ ckpt,
                                                              float* __restrict__ sT) {
     typedef float f2 __attribute__((ext_vector_type(2)));
-    constexpr int CH = CH64, LPR = C / 4, GPW = 64 / LPR, ROWS = NW * GPW * R, NSPLIT = C / ROWS, NH = C / 64;
-    constexpr int PT = 64 * NP, PER = CH * C / PT, TPJ = PT / C;
-    static_assert(C % ROWS == 0 && (CH * C) % PT == 0 && PT % C == 0 && (CH * ROWS) % PT == 0, "whole tokens and rows per thread");
+    constexpr int CH = CH64, Q = C / (4 * LPR), GPW = 64 / LPR, ROWS = NW * GPW * R, NSPLIT = C / ROWS;
+    constexpr int PT = 64 * NP, QPT = C / 4, TPJ = PT / QPT, PER = CH / TPJ;   // moving: QPT threads, four channels each, per token
+    constexpr int LDO = ROWS + 4, QPR = ROWS / 4;                              // results: a token's rows, QPR pieces of four
+    constexpr bool SHARE = LPR == 8;                                           // of two pieces a lane reads one
+    constexpr int KT = LPR < CH ? LPR : CH, KEPT = CH / KT;                    // of KT tokens a lane keeps one's results, KEPT times
+    static_assert(C % ROWS == 0 && PT % QPT == 0 && CH % TPJ == 0 && (CH * QPR) % 64 == 0, "whole tokens and rows per thread");
     __shared__ __attribute__((aligned(16))) float in[2][FWD_VECS][CH][C];   // the slot of q holds decay * q
-    __shared__ f2 bkq[2][CH][NH];                                           // (b . q, k . q) of every token, per 64 channels
-    __shared__ __attribute__((aligned(16))) float yout[2][CH][ROWS + 1], saout[2][CH][ROWS + 1];
+    // (b . q, k . q) of every token (as floats: the half of a pair that nobody uses is a register the compiler
+    // reuses at once, behind a wait for everything in flight, a sixth of the backward scan)
+    __shared__ __attribute__((aligned(8))) float bkq[2][CH][2];
+    __shared__ __attribute__((aligned(16))) float yout[2][CH][LDO], saout[2][CH][LDO];
     const int bh = blockIdx.x / NSPLIT, part = blockIdx.x % NSPLIT, h = bh % H;
     const long bt0 = (long)(bh / H) * T;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, jb = lane % LPR, rl = (wv * GPW + lane / LPR) * R;
-    const int row0 = part * ROWS + rl, col0 = 4 * jb;
+    const int row0 = part * ROWS + rl;
+    auto col = [&](int x) { return 4 * jb + 4 * LPR * (SHARE ? x ^ (lane >> 3 & 1) : x); };   // piece x < Q of a lane's columns: four from here on
     const float* const src[FWD_VECS] = {w, q, k, v, a, b};
     float* const sav = ckpt == nullptr ? nullptr : ckpt + saved_states(gridDim.x / NSPLIT, T, CR);
     // Addresses are a base per chunk that is the same in every lane (scalar registers) plus a small 32-bit offset per
@@ -206,20 +248,21 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
     const int NC = T / CH;
     auto chunk_start = [&](int n) { return CH * (ADJ ? NC - 1 - n : n); };   // first token of the n-th chunk in the order of the walk
     auto chunk_base = [&](int n) { return seq_index(bt0 + chunk_start(n), H, h, 0, CR); };
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
 
-    // ---- moving data: thread ptid of PT ----
-    const int ptid = threadIdx.x - 64 * NW, pch = ptid % C;
+    // ---- moving data: thread ptid of PT, four channels of every TPJ-th token ----
+    const int ptid = threadIdx.x - 64 * NW, pch = 4 * (ptid % QPT), ptok = ptid / QPT;
     const bool stage_ok = FULL || pch < CR;
-    const unsigned tok_off = 4 * ((unsigned)(ptid / C) * ld + (stage_ok ? pch : 0));   // (token, channel) this thread stages, in bytes
-    float pre[FWD_VECS][PER];
+    const unsigned tok_off = 4 * ((unsigned)ptok * ld + (stage_ok ? pch : 0));   // in bytes
+    f4 pre[FWD_VECS][PER];
     auto fetch = [&](int n) {
         const long base = chunk_base(n < NC ? n : NC - 1);   // (past the last chunk: the same one again, not used)
 #pragma unroll
         for (int vec = 0; vec < FWD_VECS; vec++) {
 #pragma unroll
             for (int j = 0; j < PER; j++) {
-                const float x = at_bytes<float>(src[vec] + (base + (long)(TPJ * j) * ld), tok_off);
-                pre[vec][j] = stage_ok ? x : 0.f;
+                const f4 x = at_bytes<seq4>(src[vec] + (base + (long)(TPJ * j) * ld), tok_off);
+                pre[vec][j] = stage_ok ? x : zero;
             }
         }
     };
@@ -229,28 +272,33 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
     auto stage = [&](int buf) {
 #pragma unroll
         for (int j = 0; j < PER; j++) {
-            const int tok = TPJ * j + ptid / C;
-            const float d = expf(-expf(pre[V_DEC][j]));
-            in[buf][V_DEC][tok][pch] = d;
-            in[buf][V_Q][tok][pch] = d * pre[V_Q][j];
-            in[buf][V_K][tok][pch] = pre[V_K][j];
-            in[buf][V_V][tok][pch] = pre[V_V][j];
-            in[buf][V_A][tok][pch] = pre[V_A][j];
-            in[buf][V_B][tok][pch] = pre[V_B][j];
-            const float bkq_lane = pair_sums(pre[V_B][j], pre[V_K][j], pre[V_Q][j], lane);   // lane 0: b . q, lane 1: k . q
-            if (lane < 2) reinterpret_cast<float*>(&bkq[buf][tok][pch >> 6])[lane] = bkq_lane;
+            const int tok = TPJ * j + ptok;
+            auto put = [&](int vec, f4 x) { *reinterpret_cast<f4*>(&in[buf][vec][tok][pch]) = x; };
+            f4 d;
+#pragma unroll
+            for (int i = 0; i < 4; i++) d[i] = expf(-expf(pre[V_DEC][j][i]));
+            put(V_DEC, d);
+            put(V_Q, d * pre[V_Q][j]);
+            put(V_K, pre[V_K][j]);
+            put(V_V, pre[V_V][j]);
+            put(V_A, pre[V_A][j]);
+            put(V_B, pre[V_B][j]);
+            const float bkq_lane = pair_sums<QPT>(dot4(pre[V_B][j], pre[V_Q][j]), dot4(pre[V_K][j], pre[V_Q][j]), lane);   // even lanes: b . q, odd ones: k . q
+            if (pch < 8) bkq[buf][tok][lane & 1] = bkq_lane;
         }
     };
     auto copy_out = [&](int n, int buf) {
         const long base = chunk_base(n);
+        constexpr int PIECES = CH * QPR;   // of either result
 #pragma unroll
-        for (int m = 0; m < CH * ROWS / PT; m++) {
-            const int e = ptid + PT * m;
-            const int tok = e / ROWS, ch = e % ROWS;
+        for (int m = 0; m < (2 * PIECES + PT - 1) / PT; m++) {
+            const int e = ptid + PT * m, which = e / PIECES, i = e % PIECES;   // (which: the same for a wavefront)
+            const int tok = i / QPR, ch = 4 * (i % QPR);
             const unsigned at = (unsigned)tok * ld + (unsigned)(part * ROWS + ch);
             if (FULL || part * ROWS + ch < CR) {
-                __builtin_nontemporal_store(yout[buf][tok][ch], (y + base) + at);
-                if (sav != nullptr) __builtin_nontemporal_store(saout[buf][tok][ch], (sav + base) + at);
+                if (which == 0) __builtin_nontemporal_store(*reinterpret_cast<const f4*>(&yout[buf][tok][ch]), reinterpret_cast<seq4*>((y + base) + at));
+                else if (which == 1 && sav != nullptr)
+                    __builtin_nontemporal_store(*reinterpret_cast<const f4*>(&saout[buf][tok][ch]), reinterpret_cast<seq4*>((sav + base) + at));
             }
         }
     };
@@ -270,45 +318,61 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
     }
 
     // ---- the recurrence ----
-    const bool col_ok = FULL || col0 < CR;
-    const unsigned state_off = (unsigned)(row0 * CR + (col_ok ? col0 : 0));  // this thread's first row in a CR x CR state
-    auto row_ok = [&](int r) { return FULL || (col_ok && row0 + r < CR); };
-    const f4 zero = {0.f, 0.f, 0.f, 0.f};
-    f4 S[R];
+    auto col_ok = [&](int x) { return FULL || col(x) < CR; };
+    auto state_off = [&](int r, int x) { return (unsigned)((row0 + r) * CR + col(x)); };  // in a CR x CR state
+    auto state_ok = [&](int r, int x) { return FULL || (col_ok(x) && row0 + r < CR); };
+    f4 S[R][Q];
 #pragma unroll
     for (int r = 0; r < R; r++)
-        S[r] = row_ok(r) ? *reinterpret_cast<const f4*>(s0 + (long)bh * CR * CR + (state_off + r * CR)) : zero;
+#pragma unroll
+        for (int x = 0; x < Q; x++)
+            S[r][x] = state_ok(r, x) ? *reinterpret_cast<const f4*>(s0 + (long)bh * CR * CR + state_off(r, x)) : zero;
+    const int kept_token = sums_token<LPR>(jb);   // of each KT
+    [[maybe_unused]] const bool in_quad[4] = {(lane & 3) == 0, (lane & 3) == 1, (lane & 3) == 2, (lane & 3) == 3};
+    // x in lanes 4 k .. 4 k + 3 of every DPP row, `to` elsewhere
+    auto into_quad = [](float to, float x, int k) {
+        auto move = [&](auto mask) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, to), __builtin_bit_cast(int, x), 0xE4, 0xf, decltype(mask)::value, false));
+        };   // (quad_perm [0,1,2,3])
+        using std::integral_constant;
+        return k == 0 ? move(integral_constant<int, 1>()) : k == 1 ? move(integral_constant<int, 2>()) : k == 2 ? move(integral_constant<int, 4>())
+                                                                                                             : move(integral_constant<int, 8>());
+    };
     auto walk = [&](int n, int buf) {
         if (ckpt != nullptr) {
             float* const to = ckpt + ((long)bh * NC + chunk_start(n) / CH) * CR * CR;
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (row_ok(r)) __builtin_nontemporal_store(S[r], reinterpret_cast<f4*>(to + (state_off + r * CR)));
-            }
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int x = 0; x < Q; x++) {
+                    if (state_ok(r, x)) __builtin_nontemporal_store(S[r][x], reinterpret_cast<f4*>(to + state_off(r, x)));
+                }
         }
         // a token's operands are requested from LDS one token ahead
         struct Ops {
-            f4 dec, x1, x2, u1, u2;   // operands of the two row sums, column vectors of the two rank-one terms
+            f4 dec[Q], x1[Q], x2[Q], u1[Q], u2[Q];   // operands of the two row sums, column vectors of the two rank-one terms
             RowVals<R> vr;
             float bq;
         };
         auto read_ops = [&](int t) {
             Ops o;
-            o.dec = *reinterpret_cast<const f4*>(&in[buf][V_DEC][t][col0]);
-            o.x1 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_B : V_A][t][col0]);
-            o.u1 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_A : V_B][t][col0]);
-            o.u2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_Q : V_K][t][col0]);
-            o.x2 = *reinterpret_cast<const f4*>(&in[buf][ADJ ? V_K : V_Q][t][col0]);
+            auto read = [&](f4 (&to)[Q], int vec) {
+#pragma unroll
+                for (int x = 0; x < (SHARE ? 1 : Q); x++) to[x] = *reinterpret_cast<const f4*>(&in[buf][vec][t][col(x)]);
+            };
+            read(o.dec, V_DEC);
+            read(o.x1, ADJ ? V_B : V_A);
+            read(o.u1, ADJ ? V_A : V_B);
+            read(o.u2, ADJ ? V_Q : V_K);
+            read(o.x2, ADJ ? V_K : V_Q);
             o.vr = lds_rows<R>(&in[buf][V_V][t][row0]);
-            if constexpr (ADJ) {
-                o.bq = bkq[buf][t][0][0];
-                if constexpr (NH == 2) o.bq += bkq[buf][t][1][0];
-            }
+            if constexpr (ADJ) o.bq = bkq[buf][t][0];
             return o;
         };
         Ops ahead = read_ops(ADJ ? CH - 1 : 0);
-        RowVals<R> ykeep = {}, sakeep = {};
+        RowVals<R> ykeep[KEPT] = {}, sakeep[KEPT] = {};
         float ypart[R][4];   // four tokens' terms of S (decay * q)
+        [[maybe_unused]] float sa4[R];
 #pragma unroll
         for (int i = 0; i < CH; i++) {
             const int t = ADJ ? CH - 1 - i : i;
@@ -318,33 +382,68 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
             RowVals<R> sar;
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                sar.x[r] = row_sum<LPR>(dot4(S[r], o.x1));
+                // element c of piece x of a token's vector, times s; the same plus acc
+                auto times = [&](const f4 (&v)[Q], int x, int c, float s) { return s * (SHARE && x ? other_row(v[0][c]) : v[x][c]); };
+                auto fma_at = [&](const f4 (&v)[Q], int x, int c, float s, float acc) {
+                    return SHARE && x ? fma_other_row(v[0][c], s, acc) : fmaf(v[x][c], s, acc);
+                };
+                float p1[Q], p2[Q];
+#pragma unroll
+                for (int x = 0; x < Q; x++) {
+                    p1[x] = times(o.x1, x, 0, S[r][x][0]), p2[x] = times(o.x2, x, 0, S[r][x][0]);
+#pragma unroll
+                    for (int c = 1; c < 4; c++) p1[x] = fma_at(o.x1, x, c, S[r][x][c], p1[x]), p2[x] = fma_at(o.x2, x, c, S[r][x][c], p2[x]);
+                }
+#pragma unroll
+                for (int x = 1; x < Q; x++) p1[0] += p1[x], p2[0] += p2[x];
+                sar.x[r] = row_sum<LPR>(p1[0]);
                 if constexpr (ADJ) sar.x[r] += o.vr.x[r] * o.bq;
-                ypart[r][t % 4] = dot4(S[r], o.x2);
-                S[r] = S[r] * o.dec + sar.x[r] * o.u1 + o.vr.x[r] * o.u2;
+                ypart[r][t % 4] = p2[0];
+#pragma unroll
+                for (int x = 0; x < Q; x++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        // (in this order: the small term is the one rounded by itself.  y against fp64 9.14e-8; with the decayed state
+                        // rounded first 9.39e-8, with sa b added last 9.57e-8)
+                        S[r][x][c] = fma_at(o.u2, x, c, o.vr.x[r], fma_at(o.dec, x, c, S[r][x][c], times(o.u1, x, c, sar.x[r])));
             }
-            // lane t of a row's lanes keeps token t's results (a store per token by one lane would be a branch per token,
-            // which nothing is scheduled across); 32 lanes per row: both of its DPP rows hold and store the same
+            // a lane of a row keeps one token's results of each KT (a store per token by one lane would be a branch per token,
+            // which nothing is scheduled across); 32 lanes per row: both of its DPP rows hold and store the same.  The lanes of a
+            // quad keep four tokens in a row, so the selects are between four and a move into one quad.
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                sakeep.x[r] = jb % CH == t ? sar.x[r] : sakeep.x[r];
-                if (i % 4 == 3) {
-                    const float y4 = quad_sums<LPR>(ypart[r], lane);
-                    ykeep.x[r] = jb % CH / 4 == t / 4 ? y4 : ykeep.x[r];
+                if constexpr (LPR == 8) {
+                    float& sa = sakeep[t / KT].x[r];
+                    sa = kept_token == t % KT ? sar.x[r] : sa;
+                    if (i % 4 == 3) {
+                        const float y4 = quad_sums<LPR>(ypart[r], lane);   // (by every lane, not by those alone that keep it)
+                        float& yk = ykeep[t / KT].x[r];
+                        yk = kept_token / 4 == t % KT / 4 ? y4 : yk;
+                    }
+                    asm volatile("" : "+v"(sa));   // (here and now: put off, it keeps every token's operands alive)
+                } else {
+                    sa4[r] = i % 4 == 0 || in_quad[t % 4] ? sar.x[r] : sa4[r];
+                    asm volatile("" : "+v"(sa4[r]));   // (here and now: put off, it keeps every token's operands alive)
+                    if (i % 4 == 3) {
+                        sakeep[0].x[r] = into_quad(sakeep[0].x[r], sa4[r], t / 4);
+                        ykeep[0].x[r] = into_quad(ykeep[0].x[r], quad_sums<LPR>(ypart[r], lane), t / 4);
+                    }
                 }
-                asm volatile("" : "+v"(sakeep.x[r]));   // (here and now: put off, it keeps every token's operands alive)
             }
         }
-        // what the row vectors add to y, once for the token that a lane keeps
-        f2 sc = bkq[buf][jb % CH][0];
-        if constexpr (NH == 2) sc += bkq[buf][jb % CH][1];
-        const RowVals<R> vr = lds_rows<R>(&in[buf][V_V][jb % CH][row0]);
+        // what the row vectors add to y, once for the tokens that a lane keeps
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            float yr = ykeep.x[r] + vr.x[r] * sc[1];
-            if constexpr (!ADJ) yr += sakeep.x[r] * sc[0];
-            yout[buf][jb % CH][rl + r] = yr;
-            saout[buf][jb % CH][rl + r] = sakeep.x[r];
+        for (int m = 0; m < KEPT; m++) {
+            const int t = KT * m + kept_token;
+            const f2 sc = *reinterpret_cast<const f2*>(bkq[buf][t]);
+            const RowVals<R> vr = lds_rows<R>(&in[buf][V_V][t][row0]);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float yr = ykeep[m].x[r] + vr.x[r] * sc[1];
+                if constexpr (!ADJ) yr += sakeep[m].x[r] * sc[0];
+                yout[buf][t][rl + r] = yr;
+                saout[buf][t][rl + r] = sakeep[m].x[r];
+            }
         }
     };
     lds_barrier();
@@ -353,9 +452,11 @@ __global__ __launch_bounds__(64 * (NW + NP)) void wkv7_f32_scan_kernel(int T, in
         lds_barrier();
     }
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        if (row_ok(r)) *reinterpret_cast<f4*>(sT + (long)bh * CR * CR + (state_off + r * CR)) = S[r];
-    }
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int x = 0; x < Q; x++) {
+            if (state_ok(r, x)) *reinterpret_cast<f4*>(sT + (long)bh * CR * CR + state_off(r, x)) = S[r][x];
+        }
 }
 
 template <int C, int R, int NW, int WIN, bool FULL>
@@ -982,16 +1083,15 @@ static void launch_scan(int B, int T, int H, int C, const float* w, const float*
     // wavefront x rows per thread
     auto width64 = [&](auto full) {
         constexpr bool F = decltype(full)::value;
-        if (split == 4) launch(wkv7_f32_scan_kernel<64, 1, 4, 4, F, ADJ>, 512);
-        else if (split == 2 && B * H > compute_units()) launch(wkv7_f32_scan_kernel<64, 2, 4, 4, F, ADJ>, 512);
-        else if (split == 2) launch(wkv7_f32_scan_kernel<64, 1, 8, 4, F, ADJ>, 768);
-        else launch(wkv7_f32_scan_kernel<64, 2, 8, 4, F, ADJ>, 768);
+        if (split == 4) launch(wkv7_f32_scan_kernel<64, 16, 1, 4, 4, F, ADJ>, 512);
+        else if (split == 2) launch(wkv7_f32_scan_kernel<64, 8, 1, 4, 4, F, ADJ>, 512);
+        else launch(wkv7_f32_scan_kernel<64, 8, 1, 8, 4, F, ADJ>, 768);
     };
     auto width128 = [&](auto full) {
         constexpr bool F = decltype(full)::value;
-        if (split == 8) launch(wkv7_f32_scan_kernel<128, 2, 4, 4, F, ADJ>, 512);
-        else if (split == 4) launch(wkv7_f32_scan_kernel<128, 2, 8, 4, F, ADJ>, 768);
-        else launch(wkv7_f32_scan_kernel<128, 4, 8, 4, F, ADJ>, 768);
+        if (split == 8) launch(wkv7_f32_scan_kernel<128, 32, 2, 4, 4, F, ADJ>, 512);
+        else if (split == 4) launch(wkv7_f32_scan_kernel<128, 16, 1, 8, 4, F, ADJ>, 768);
+        else launch(wkv7_f32_scan_kernel<128, 16, 2, 8, 4, F, ADJ>, 768);
     };
     if (C == 64) width64(std::true_type());
     else if (C < 64) width64(std::false_type());
