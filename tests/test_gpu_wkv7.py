@@ -122,6 +122,30 @@ def test_parity_runs_of_pairs_that_do_not_divide_evenly(c_oracle, B, T, H):
     print('runs of pairs, errors', {k: f'{v:.2e}' for k, v in errs.items()})
 
 
+@pytest.mark.parametrize('B,T,H,ln', [(2, 1024, 16, False), (3, 768, 15, False), (33, 32, 16, False), (9, 480, 4, False), (2, 1024, 16, True),
+                                      (3, 768, 15, True), (9, 480, 4, True)])
+def test_a_chunk_per_wavefront_gives_the_bits_of_a_pair_per_wavefront(B, T, H, ln):
+    """Gradients of a batch with more chunks than four per compute unit (2048, 2160, 1056, 1080), a pair of chunks per wavefront, and
+    of its sequences one by one (1024, 720, 32, 120), a chunk per wavefront.  (attn_ln up to 128 heads, where its forward has one form.)"""
+    from wind_rwkv.rwkv7 import attn, attn_ln
+    d = inputs.wkv7_inputs(B, T, H, 64, seed=B + T, dtype=torch.bfloat16, s0_scale=0.3)
+    x = [d[n].reshape(B, T, H * 64).to(DEV) for n in ('q', 'w', 'k', 'v', 'a', 'b')]
+    s0, dy = d['s0'].float().to(DEV), d['dy'].reshape(B, T, H * 64).to(DEV)
+    gen = torch.Generator().manual_seed(T)
+    g, params = torch.randn(x[0].shape, generator=gen).bfloat16().to(DEV), torch.randn(3, H * 64, generator=gen).to(DEV)
+
+    def grads(rows):
+        leaves = [t[rows].detach().clone().requires_grad_() for t in x + [g]]
+        y = attn_ln(*leaves, params, 64, s0=s0[rows]) if ln else attn(*leaves[:6], 64, s0=s0[rows])
+        return torch.autograd.grad(y, leaves if ln else leaves[:6], dy[rows])
+
+    whole = grads(slice(None))
+    assert all(torch.isfinite(t.float()).all() for t in whole)
+    for b in range(0, B, max(1, B - 1)):   # the first and the last sequence
+        for n, t in zip('qwkvabg', grads(slice(b, b + 1))):
+            assert torch.equal(t[0], whole['qwkvabg'.index(n)][b]), n
+
+
 @pytest.fixture
 def checkpoint_interval(request):
     """Runs the test under the given number of tokens between kept states and restores the default (32)."""

@@ -93,6 +93,12 @@ __global__ __launch_bounds__(256) void ln_epilogue_bwd_kernel(int T, int H, int 
 // What a pair needs from memory besides the tiles that go straight into arithmetic arrives by global -> LDS loads
 // (no registers, so nothing is live across the chunk before): both states and, for either chunk, w, k, b, v and U^T,
 // 36 KiB per wavefront; only q, a, dY and dab_u^T of the next chunk wait in registers.  Needs an even number of chunks.
+// MODE 4: the same arrays, but a wavefront takes ONE chunk and ends, where there are no more chunks than wavefronts that run at once
+// (four per compute unit): bound by latency there, and half of it was the pair's other chunk.  The wavefront of the later chunk
+// advances the forward state as above; that of the earlier one hands the dstate on to itself first, from the later chunk's w, q,
+// a, dY and dab_u^T.  The same instructions on the same operands: the same bits.  Forward + backward, us, MODE 3 -> 4:
+// attn 1 x 256 tokens x 4 heads 48.8 -> 42.6, 8 x 64 x 12 34.8 -> 26.5, 1 x 1024 x 16 (1024 chunks) 96.8 -> 90.9, attn_ln
+// 1 x 256 x 4 61.8 -> 53.6, 1 x 1024 x 16 112 -> 105.  With more chunks every wavefront has a pair to do either way.
 namespace pairlds {   // byte offsets inside a wavefront's 36 KiB
 constexpr int STASH = 0;              // the state entering the pair: [ib][half][lane] x 16 B (fragments jb = 2 half, 2 half + 1)
 constexpr int CARRY = 8192;           // the dstate arriving at the end of the current chunk, same layout
@@ -159,8 +165,9 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
     // loads the next chunk's nine input tiles while it works on the current one.  With ~380 live registers only one
     // wavefront fits a SIMD, so without this the kernel alternates between waiting for memory and computing (measured:
     // 64 us of pure memory time + 34 us of arithmetic = 98 us); the prefetch lets the two overlap.
-    static_assert(MODE == 1 || MODE == 3, "a state per chunk, or per pair of chunks");
-    constexpr bool LDSP = MODE == 3;                  // states per pair in both directions, prefetched into LDS
+    static_assert(MODE == 1 || MODE == 3 || MODE == 4, "a state per chunk, or per pair of chunks");
+    constexpr bool LDSP = MODE != 1;                  // states per pair in both directions, prefetched into LDS
+    constexpr bool ONE = MODE == 4;                   // a wavefront takes one chunk of a pair, and no other
     constexpr int AFTER_PREFETCH = 10;
     constexpr bool PAIRED = LDSP;                     // an item is a pair of chunks
     using RF = Saved;
@@ -181,7 +188,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
     const int RUN = MODE == 3 ? (ds_run < 0 ? -ds_run : ds_run) : 1;
     const bool HM = MODE == 3 && ds_run < 0;
     const int BH = nchunks / NC, RH = (NP + RUN - 1) / RUN;
-    const int nruns = HM ? BH * RH : (nitems + RUN - 1) / RUN;
+    const int nruns = ONE ? nchunks : HM ? BH * RH : (nitems + RUN - 1) / RUN;
     if (id0 >= nruns) return;
     // the pair a run starts with (its last one)
     auto run_first_item = [&](int i) {
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
     // to itself it builds all twelve first, and with the scalar registers that takes it runs out of them)
     // Order: what the state advance at the head of the pair needs first (the entering state and the tiles of the earlier
     // chunk, 18 loads), then the dstate and the later chunk's tiles (18 loads).
-    auto dma_pair = [&](int walk, bool carried) {   // carried: the dstate is already in place (handed on by the pair before)
+    auto dma_pair = [&](int walk, bool carried, bool earlier = false) {   // carried: the dstate is already in place (handed on by the pair before)
         const int item = pair_of(walk);
         const int bh = item / NP, p = item - bh * NP;
         const long c0 = (long)bh * NC + 2 * p;
@@ -321,7 +328,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
                 dma16(r, lane * 32, (i >> 1) * 2048 + (i & 1) * 16, dst + i * 1024);
             __builtin_amdgcn_sched_barrier(0);
         };
-        auto tiles = [&](int e) {                     // w, k, b, v and U^T of chunk 2p + e
+        auto tiles = [&](int e, bool w_alone = false) {   // w, k, b, v and U^T of chunk 2p + e
             const ChunkAddr ca((int)c0 + e, T, H);
             unsigned char* set = mine + pairlds::TILES + e * pairlds::SET;
             const __bf16* const src[4] = {w_, k_, b_, v_};
@@ -331,23 +338,86 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
 #pragma unroll
                 for (int pr = 0; pr < NBLK / 2; pr++) dma16(r, voff_rows, 64 * pr, set + t * 2048 + pr * 1024);
                 __builtin_amdgcn_sched_barrier(0);
+                if (w_alone) return;
             }
             const Rsrc ru = rs(rec_fwd + SavedPair::ut(item, 2 * p + e));
 #pragma unroll
             for (int i = 0; i < 2; i++) dma16(ru, lane * 16, i * 1024, set + 8192 + i * 1024);
             __builtin_amdgcn_sched_barrier(0);
         };
+        if (earlier) {                                // MODE 4: what the dstate is handed on with comes first
+            state(1);
+            tiles(1, true);
+            state(0);
+            tiles(0);
+            return;
+        }
         state(0);
         tiles(0);
         if (!carried) state(1);
         tiles(1);
     };
     constexpr int DMA_SECOND_HALF = 18;   // loads of a pair that the state advance does not wait for
-    int item = run_first_item(id0), cid = first_chunk(item);
+    int item, cid;
     bool first = true;   // MODE 3: the later chunk of a pair, which is handled first
-    In nxt = fetch(cid, item, true);
-    if constexpr (LDSP) dma_pair(item, false);
+    if constexpr (ONE) {
+        const int bh = id0 / NC, c = id0 - bh * NC;
+        cid = id0;
+        item = bh * NP + c / 2;
+        first = c & 1;
+    } else {
+        item = run_first_item(id0);
+        cid = first_chunk(item);
+    }
+    In nxt;
+    // the dstate for the chunk before in time, dS diag(fw) + dY^T wq + dab_u^T wa, in place
+    auto hand_dstate_on = [&](const TileB& wq, const TileB& wa, const TileF& fw, const TileB& dYT, const TileB& DT) {
+#pragma unroll
+        for (int jb = 0; jb < NBLK; jb++) {
+            const bf16x4 waT = transpose(wa.f[jb], eye), wqT = transpose(wq.f[jb], eye);
+#pragma unroll
+            for (int ib = 0; ib < NBLK; ib++) {
+                bf16x4* slot = reinterpret_cast<bf16x4*>(mine + pairlds::CARRY + (2 * ib + (jb >> 1)) * 1024 + lane * 16 + (jb & 1) * 8);
+                *slot = to_bf16(mma2(to_f32(*slot) * fw.f[jb], wqT, waT, dYT.f[ib], DT.f[ib]));
+            }
+        }
+    };
     bool started = false;   // MODE 3: whether the wavefront's first pair is in (its loads have nothing to hide behind)
+    // attn_ln, MODE 4: what the end of the chunk adds, requested first (MODE 3 has no registers to hold it and reads it there)
+    [[maybe_unused]] bf16x4 dv_part[NBLK];
+    [[maybe_unused]] f32x4 bonus_of[NBLK];
+    [[maybe_unused]] float ddot_of = 0.f;
+    auto bonus_at = [&](int bh, int jb) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs(ln_params + 2L * H * HEAD + (long)(bh % H) * HEAD), 4 * chan16(jb, 4 * L.g), 0, 0));
+    };
+    auto ddot_at = [&](int c) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs(ln_ddot + (long)c * CHUNK), 4 * L.n, 0, 0)); };
+    auto dv_at = [&](long row0, int ib) { return ld8(rs(dv_ + row0), voff_n + 2 * chan16(ib, 4 * L.g)); };
+    if constexpr (LN && ONE) {
+        const ChunkAddr ca(cid, T, H);
+#pragma unroll
+        for (int i = 0; i < NBLK; i++) dv_part[i] = dv_at(ca.row0, i), bonus_of[i] = bonus_at(ca.bh, i);
+        ddot_of = ddot_at(cid);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (ONE && !first) {
+        const In later = fetch(cid + 1, item, true);
+        __builtin_amdgcn_sched_barrier(0);
+        dma_pair(item, false, true);
+        nxt = fetch(cid, item, true);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int SECOND_HALF = 8 + 10 + 10;   // the entering state, the tiles of this chunk, its registers
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SECOND_HALF) : "memory");
+        const Decay d = chunk_decay(pairlds::tile(mine + pairlds::TILES + pairlds::SET, 0, lane));
+        TileB dYT;
+#pragma unroll
+        for (int ib = 0; ib < NBLK; ib++) dYT.f[ib] = transpose(later.dy.f[ib], eye);
+        hand_dstate_on(to_bf16(mul(later.q, d.P)), to_bf16(mul(later.a, d.Px)), d.fw, dYT, later.DT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        started = true;
+    } else {
+        nxt = fetch(cid, item, true);
+        if constexpr (LDSP) dma_pair(item, false);
+    }
     for (;;) {
     const ChunkAddr ca(cid, T, H);
     const In cur = nxt;
@@ -495,16 +565,18 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
     // next chunk's tiles and states: they have the rest of this chunk's arithmetic to arrive
     int nitem = item, ncid = cid - 1;
     bool nfirst = false;
-    if (!PAIRED || !first) {   // (the earlier chunk of a pair follows its later one directly)
+    if (ONE) {
+        nitem = nitems;
+    } else if (!PAIRED || !first) {   // (the earlier chunk of a pair follows its later one directly)
         nitem = next_item(item);
         nfirst = true;
         ncid = nitem < nitems ? first_chunk(nitem) : cid;
     }
-    const bool more = nitem < nitems;
+    const bool more = !ONE && nitem < nitems;
     // whether this chunk hands its dstate on: a pair's later chunk to its earlier one, and a pair's earlier chunk to the
     // pair before it in the run (same (batch, head))
-    const bool hand_on = PAIRED && (first || (MODE == 3 && more && nitem == item - 1 && item % NP != 0));
-    nxt = fetch(ncid, more ? nitem : item, more);
+    const bool hand_on = PAIRED && !ONE && (first || (MODE == 3 && more && nitem == item - 1 && item % NP != 0));
+    if constexpr (!ONE) nxt = fetch(ncid, more ? nitem : item, more);
 
     // dv = QK^T dY + kf dS^T + AK^T dab_u          (rows = tokens)
     TileB out;
@@ -518,7 +590,7 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         else for (int jb = 0; jb < NBLK; jb++) dsi.f[jb] = dS[ib][jb];
         acc = mma2(acc, dsi.f[0], dsi.f[1], kf.f[0], kf.f[1]);
         acc = mma2(acc, dsi.f[2], dsi.f[3], kf.f[2], kf.f[3]);
-        if constexpr (LN) acc += to_f32(ld8(rs(dv_ + ca.row0), voff_n + 2 * chan16(ib, 4 * L.g)));
+        if constexpr (LN) acc += to_f32(ONE ? dv_part[ib] : dv_at(ca.row0, ib));
         out.f[ib] = to_bf16(acc);
     }
     put16(dv_, ca.row0, out);
@@ -531,23 +603,14 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         }
     }
     if constexpr (PAIRED) {
-        // the dstate for the pair's earlier chunk, dS diag(fw) + dY^T wq + dab_u^T wa, here rather than in the loop below
+        // the dstate for the pair's earlier chunk, here rather than in the loop below
         // (which makes the same transposes again) so that dS is dead before that loop starts
-        if (hand_on) {   // (else the next pair's dstate is on its way into this buffer)
-#pragma unroll
-        for (int jb = 0; jb < NBLK; jb++) {
-            const bf16x4 waT = transpose(wa.f[jb], eye), wqT = transpose(wq.f[jb], eye);
-#pragma unroll
-            for (int ib = 0; ib < NBLK; ib++) {
-                bf16x4* slot = reinterpret_cast<bf16x4*>(mine + pairlds::CARRY + (2 * ib + (jb >> 1)) * 1024 + lane * 16 + (jb & 1) * 8);
-                *slot = to_bf16(mma2(to_f32(*slot) * d.fw.f[jb], wqT, waT, dYT.f[ib], DT.f[ib]));   // (in place)
-            }
-        }
-        }
+        if (hand_on)   // (else the next pair's dstate is on its way into this buffer)
+            hand_dstate_on(wq, wa, d.fw, dYT, DT);
     }
 
     float ddot = 0.f;
-    if constexpr (LN) ddot = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs(ln_ddot + (long)cid * CHUNK), 4 * L.n, 0, 0));
+    if constexpr (LN) ddot = ONE ? ddot_of : ddot_at(cid);
 
     // key-channel gradients, one block of 16 key channels at a time
     TileB o_dq, o_da, o_dk, o_db, o_dw;
@@ -558,12 +621,13 @@ __global__ __launch_bounds__(256) void bwd_grads_kernel(int T, int H, int nchunk
         // ([2][H*64] of the parameters); requested first, used last
         bf16x4 k_re = {}, q_re = {};
         f32x4 bonus = zero4();
-        if constexpr (LN) {
+        if constexpr (LN && ONE) {
+            k_re = k.f[jb], q_re = q.f[jb], bonus = bonus_of[jb];
+        } else if constexpr (LN) {
             const unsigned piece = voff_n + 2 * chan16(jb, 4 * L.g);
             k_re = ld8(rs(k_ + ca.row0), piece);
             q_re = ld8(rs(q_ + ca.row0), piece);
-            bonus = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                rs(ln_params + 2L * H * HEAD + (long)(ca.bh % H) * HEAD), 4 * chan16(jb, 4 * L.g), 0, 0));
+            bonus = bonus_at(ca.bh, jb);
         }
         const bf16x4 bwiT = transpose(bwi.f[jb], eye), kwiT = transpose(kwi.f[jb], eye);
         const bf16x4 waT = transpose(wa.f[jb], eye), wqT = transpose(wq.f[jb], eye);
@@ -660,13 +724,17 @@ void launch_bwd_grads(int B, int T, int H, const void* w, const void* q, const v
     const int num_cu = compute_units();
     const int NP = SavedPair::pairs(T / CHUNK), run = ds_run < 0 ? -ds_run : ds_run;
     // what a wavefront takes at a time: a run of pairs (cut per (batch, head) or from the flattened pairs), or a chunk
-    const int items = fused != 3 ? nchunks : ds_run < 0 ? B * H * ((NP + run - 1) / run) : (B * H * NP + run - 1) / run;
+    const bool one = fused == 3 && nchunks <= 4 * num_cu;   // (MODE 4; up to 512 pairs, so runs of one: every dstate is there)
+    const int items = fused != 3 || one ? nchunks : ds_run < 0 ? B * H * ((NP + run - 1) / run) : (B * H * NP + run - 1) / run;
     const int blocks = (items + 3) / 4 < num_cu ? (items + 3) / 4 : num_cu;
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, T, H, nchunks, c(w), c(q), c(k), c(v), c(a), c(b),
                            c(dy), c(rec_fwd), c(rec_bwd), m(dw), m(dq), m(dk), m(dv), m(da), m(db), ln_params, ln_ddot, ds_run);
     };
-    if (fused == 3) {
+    if (one) {
+        if (ln_params) go(bwd_grads_kernel<true, 4>);
+        else go(bwd_grads_kernel<false, 4>);
+    } else if (fused == 3) {
         if (ln_params) go(bwd_grads_kernel<true, 3>);
         else go(bwd_grads_kernel<false, 3>);
     } else {
