@@ -69,6 +69,40 @@ def test_group_with_two_segments_and_cut_columns(M):
     assert bool((target[:, :16] == 7).all() and (target[:, 80:96] == 7).all() and (target[:, 112:] == 7).all())
 
 
+def _steps(x):
+    """The distance of neighbouring bf16 values at x (float64)."""
+    return torch.exp2(torch.floor(torch.log2(x.abs().clamp_min(2.0 ** -126))) - 7)
+
+
+# the two sides of the series' line among them, in every column of a tile; 64 tokens and 128 of it
+@pytest.mark.parametrize('tokens', [510, 20400])
+def test_tanh_of_every_normal_bf16_value(tokens):
+    """W = 1, so the sums are the inputs: tanh is within 2e-6 of itself before it is rounded, half a step and 5e-4 of one."""
+    values = torch.arange(0, 65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    values = values[values.isfinite() & (values.abs() >= 2.0 ** -126)]
+    A = values.repeat(-(-tokens * 128 // values.numel()))[:tokens * 128].view(tokens, 128).contiguous().to(DEV)
+    eye = torch.eye(128, device=DEV, dtype=torch.bfloat16)
+    out, plain = torch.empty_like(A), torch.empty(tokens, 64, device=DEV, dtype=torch.bfloat16)
+    _run([_problem([(A, eye)], [(out[:, :64], 1, None), (out[:, 64:], 1, None)]), _problem([(A[:, :64], eye[:64, :64])], [(plain, 0, None)])], tokens)
+    assert torch.equal(plain, A[:, :64])
+    want = torch.tanh(A.double())
+    assert bool(((out.double() - want).abs() <= 0.501 * _steps(want)).all())
+
+
+# columns to one, two and four tensors: the derivative's operands are read four columns a lane
+@pytest.mark.parametrize('M', [1, 33, 129, 2500])
+@pytest.mark.parametrize('widths', [(16,), (16, 32), (64, 48, 16, 80)])
+def test_derivative_in_every_column(M, widths):
+    gen = torch.Generator().manual_seed(M + sum(widths))
+    N = sum(widths)
+    A = torch.randn(M, N, generator=gen).bfloat16().to(DEV)
+    aux = [torch.rand(M, w, generator=gen).bfloat16().to(DEV) for w in widths]
+    outs = [torch.full((M, w), float('nan'), device=DEV, dtype=torch.bfloat16) for w in widths]
+    _run([_problem([(A, torch.eye(N, device=DEV, dtype=torch.bfloat16))], [(o, 2, y) for o, y in zip(outs, aux)])], M)
+    want = A.double() * (1 - torch.cat(aux, 1).double() ** 2)
+    assert bool(((torch.cat(outs, 1).double() - want).abs() <= 0.501 * _steps(want) + 2.0 ** -22 * A.double().abs()).all())
+
+
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize('off', [0, 1])
 def test_packed_weights(dtype, off):

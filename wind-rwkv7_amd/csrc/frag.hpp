@@ -243,6 +243,15 @@ __device__ __forceinline__ TileF to_f32(const TileB& x) {
 constexpr int STREAMED = 2;   // of a buffer store
 template <class V>
 __device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontemporal_store(x, static_cast<V*>(to)); }
+// 16 bytes to memory at device scope: written through the XCD's L2, so that the end of the kernel, which writes back whatever that still holds
+// for the other XCDs' L2s, finds nothing left to do, and kept in the last-level cache for whoever reads them next.
+// (s_nop: two wait states before the registers of a store of more than eight bytes may be written, which the compiler sees to for its own stores.)
+template <class V>
+__device__ __forceinline__ void store_through(void* to, V x) {
+    static_assert(sizeof(V) == 16, "one access");
+    typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(to), "v"(__builtin_bit_cast(u32x4_t, x)) : "memory");
+}
 template <class V>
 __device__ __forceinline__ V load_streamed(const void* from) { return __builtin_nontemporal_load(static_cast<const V*>(from)); }
 

@@ -17,9 +17,11 @@
 // one's matrix work covers the other's barriers and last loads.
 //
 // Measured (us; in brackets the library's kernels for the same, replayed without host time): six first-half products of a
-// 768-channel block with their tanh and cut columns at 2006 / 8192 / 32768 tokens 21 (49) / 51 (69) / 170 (203); three input
-// gradients with one second segment at 8192 38 (55); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.1 (6.4) / 18 (16) /
-// 82-90 (70).  Stages of
+// 768-channel block with their tanh and cut columns at 2006 / 8192 / 32768 tokens 19.5 (49) / 50 (69) / 170 (203); three input
+// gradients with one second segment at 8192 38 (55); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.1 (6.4) / 16.5 (16) /
+// 82-90 (70).  Of the 54 us of six on inputs out of memory the matrix instructions alone take 28 (their rate on these numbers, not on
+// zeros, is 1.3 PFLOP/s), with the LDS reads 32, with the loads 39; the output is the rest.  Blocks that stay and fetch the next tile's
+// first stage while they write this one's output: 54.  Stages of
 // 32 (half lines): 14 % slower at 65536 tokens; 256 x 192 tiles, one block per compute unit, a whole stage's operands in
 // registers: 13 % slower (768 contraction indices are twelve stages, too few to amortise its start and end alone);
 // walking the contraction from different places per tile: 5-15 % slower.
@@ -30,6 +32,15 @@
 
 namespace wkv {
 namespace {
+
+// tanh by the hardware's exponential: (1 - t) / (1 + t) with t = exp(-2 |x|), and where the difference loses digits the series to x^5 (its next
+// term, 17/315 x^7, is 5e-8 of the value at 0.1): 1e-6 of the value at most, and the result is rounded to bf16.  The library's takes three
+// times the instructions, sixty-four times a lane.
+__device__ __forceinline__ float tanh_of(float x) {
+    const float a = fabsf(x), t = __builtin_amdgcn_exp2f(a * -2.8853900817779268f);   // 2 log2(e)
+    const float x2 = a * a, small = a * fmaf(x2, fmaf(x2, 2.f / 15, -1.f / 3), 1.f);
+    return copysignf(a < 0.1f ? small : (1.f - t) * __builtin_amdgcn_rcpf(1.f + t), x);
+}
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 using Rsrc = __amdgpu_buffer_rsrc_t;
@@ -166,10 +177,62 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
                     acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[ks & 1][nb], a[ks & 1][mb], acc[mb][nb], 0, 0, 0);
         }
     }
-    // Register r of lane l of block (mb, nb): token 32 mb + l % 32, column 32 nb + 8 (r / 4) + 4 (l / 32) + r % 4.  Two lanes
-    // swap their halves so that a lane has eight consecutive columns of a token; the wavefront's tile then goes through LDS
-    // and leaves in rows (as it lies in registers every store would touch 32 rows for 32 bytes each: 8192 x 768 x 64, which
-    // is all output, 13 us instead of 9).
+    // Register r of lane l of block (mb, nb): token 32 mb + l % 32, column 32 nb + 8 (r / 4) + 4 (l / 32) + r % 4.  Eight columns lie in one
+    // output tensor, so what is done to the registers 4 q .. 4 q + 3 is the same for the whole wavefront: tanh and its derivative
+    // are applied here, to the sums as bf16, as they leave, with all of the derivative's operands requested at once.  (Row by row on the way
+    // out, each lane finding its tensor and waiting for its operand: the two gradients through tanh of a 768-channel block at 32768 tokens 40.6 us, now
+    // 35.6; six first halves at 512 tokens 13.9, now 13.5.)
+    const int m_first = m0 + 32 * TMB * wm, n_first = n0 + 32 * TNB * wn;
+    const bool plain = p.npieces == 1 && p.op[0] == LINEAR_PLAIN;
+    auto tensor_of = [&](int col) {
+        int t = 0;
+#pragma unroll
+        for (int k = 1; k < LinearProblem::PIECES; k++) t += k < p.npieces && col >= p.start[k] ? 1 : 0;
+        return t;
+    };
+    auto of = [&](int t, auto f) {
+        auto r = f(0);
+#pragma unroll
+        for (int k = 1; k < LinearProblem::PIECES; k++) r = t == k ? f(k) : r;
+        return r;
+    };
+    if (!plain) {
+        bf16x4 y[TMB][TNB][4];
+#pragma unroll
+        for (int nb = 0; nb < TNB; nb++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int col = n_first + 32 * nb + 8 * q, t = tensor_of(col);
+                const bool wanted = of(t, [&](int k) { return p.op[k]; }) == LINEAR_TANH_GRAD && col < p.N;
+                const int width = of(t, [&](int k) { return p.width[k]; });
+                const __bf16* const aux = of(t, [&](int k) { return p.aux[k]; }) + (col - of(t, [&](int k) { return p.start[k]; }) + 4 * half);
+#pragma unroll
+                for (int mb = 0; mb < TMB; mb++) {
+                    y[mb][nb][q] = bf16x4{};
+                    if (wanted) y[mb][nb][q] = *reinterpret_cast<const bf16x4*>(aux + (long)min(m_first + 32 * mb + r32, M - 1) * width);
+                }
+            }
+#pragma unroll
+        for (int nb = 0; nb < TNB; nb++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int t = tensor_of(n_first + 32 * nb + 8 * q), op = of(t, [&](int k) { return p.op[k]; });
+                if (op != LINEAR_PLAIN) {
+#pragma unroll
+                    for (int mb = 0; mb < TMB; mb++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float f = (float)(__bf16)acc[mb][nb][4 * q + e], g = (float)y[mb][nb][q][e];
+                            acc[mb][nb][4 * q + e] = op == LINEAR_TANH ? tanh_of(f) : f * (1.f - g * g);
+                        }
+                }
+            }
+    }
+    // Two lanes swap their halves so that a lane has eight consecutive columns of a token; the wavefront's tile then goes through
+    // LDS and leaves in rows (as it lies in registers every store would touch 32 rows for 32 bytes each: 8192 x 768 x 64, which
+    // is all output, 13 us instead of 9), through the L2: what the end of the kernel writes back of the output is a time in which
+    // nothing else runs (one 768 x 768 product at 8192 tokens 17.9 -> 16.5 us, two second halves 10.3 -> 9.0, six first halves at 2006 tokens 21.4 -> 19.5;
+    // past all caches faster still where the output is more than they hold, but the block, which reads it next, 615 -> 619).
     constexpr int CH = 4 * TNB, PITCH = 32 * TNB * 2 + 16;   // 16-byte pieces per row of the wavefront; its LDS row, bank-shifted
     static_assert(4 * 32 * TMB * PITCH <= STAGES * (64 * TMB + 64 * TNB) * BK * 2, "the output tile fits where the stages were");
     arrived(0);
@@ -195,42 +258,24 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
         m = m0 + 32 * TMB * wm + row, col = n0 + 32 * TNB * wn + 8 * ch;
         return reinterpret_cast<const bf16x8*>(mine + row * PITCH + ch * 16);
     };
-    if (p.npieces == 1 && p.op[0] == LINEAR_PLAIN) {
+    if (plain) {
 #pragma unroll
         for (int i = 0; i < 2 * TMB * TNB; i++) {
             int m, col;
             const bf16x8* v = rows_of(i, m, col);
-            if (m < M && col < p.N) *reinterpret_cast<bf16x8*>(p.out[0] + (long)m * p.ld_out[0] + col) = *v;
+            if (m < M && col < p.N) store_through(p.out[0] + (long)m * p.ld_out[0] + col, *v);
         }
         return;
     }
-#pragma unroll 1
+#pragma unroll
     for (int i = 0; i < 2 * TMB * TNB; i++) {
         int m, col;
-        const bf16x8* src = rows_of(i, m, col);
-        if (m >= M || col >= p.N) continue;
-        int t = 0;   // the output tensor these columns belong to (eight columns lie in one)
-#pragma unroll
-        for (int k = 1; k < LinearProblem::PIECES; k++) t += k < p.npieces && col >= p.start[k] ? 1 : 0;
-        auto of = [&](auto f) {
-            auto r = f(0);
-#pragma unroll
-            for (int k = 1; k < LinearProblem::PIECES; k++) r = t == k ? f(k) : r;
-            return r;
-        };
-        const int c = col - of([&](int k) { return p.start[k]; }), op = of([&](int k) { return p.op[k]; });
-        bf16x8 v = *src;
-        if (op != LINEAR_PLAIN) {
-            bf16x8 y = {};
-            if (op == LINEAR_TANH_GRAD)
-                y = *reinterpret_cast<const bf16x8*>(of([&](int k) { return p.aux[k]; }) + (long)m * of([&](int k) { return p.width[k]; }) + c);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float f = (float)v[e], g = (float)y[e];
-                v[e] = (__bf16)(op == LINEAR_TANH ? tanhf(f) : f * (1.f - g * g));
-            }
+        const bf16x8* v = rows_of(i, m, col);
+        if (m < M && col < p.N) {
+            const int t = tensor_of(col);
+            __bf16* const out = of(t, [&](int k) { return p.out[k]; }) + (long)m * of(t, [&](int k) { return p.ld_out[k]; });
+            store_through(out + (col - of(t, [&](int k) { return p.start[k]; })), *v);
         }
-        *reinterpret_cast<bf16x8*>(of([&](int k) { return p.out[k]; }) + (long)m * of([&](int k) { return p.ld_out[k]; }) + c) = v;
     }
 }
 
