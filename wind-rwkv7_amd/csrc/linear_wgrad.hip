@@ -274,8 +274,8 @@ __device__ __forceinline__ void wgrad_block(WgradLds<S>& lds, const WgradArgs& g
         for (int nb = 0; nb < TNB; nb++)
 #pragma unroll
             for (int qd = 0; qd < 4; qd++)
-                *reinterpret_cast<f32x4*>(out + ((mb * TNB + nb) * 4 + qd) * 256) =
-                    f32x4{acc[mb][nb][4 * qd], acc[mb][nb][4 * qd + 1], acc[mb][nb][4 * qd + 2], acc[mb][nb][4 * qd + 3]};
+                store_through(out + ((mb * TNB + nb) * 4 + qd) * 256,   // (nine products of a block at 8192 tokens 64.1 -> 62.6 us)
+                              f32x4{acc[mb][nb][4 * qd], acc[mb][nb][4 * qd + 1], acc[mb][nb][4 * qd + 2], acc[mb][nb][4 * qd + 3]});
 }
 
 template <class S>

@@ -18,7 +18,9 @@ __device__ __forceinline__ bf16x8& piece_at(__bf16* base, unsigned bytes) {
 }
 // 16 bytes there through the L2 (see store_through in frag.hpp), as a store that the compiler counts: behind one that it does not see it would wait
 // for what was requested before it to be written as well
-__device__ __forceinline__ void store_through_at(__bf16* base, unsigned bytes, bf16x8 v) {
+template <class V>
+__device__ __forceinline__ void store_through_at(void* base, unsigned bytes, V v) {
+    static_assert(sizeof(V) == 16, "one access");
     typedef unsigned words __attribute__((ext_vector_type(4)));
     constexpr int DEVICE_SCOPE = 16;
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(words, v), __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000), bytes, 0, DEVICE_SCOPE);
