@@ -531,12 +531,15 @@ __device__ __forceinline__ void load_state(f32x4 (&S)[NBLK], const void* s, int 
         else S[i] = to_f32(*reinterpret_cast<const bf16x4*>(static_cast<const __bf16*>(s) + off + 4 * i * HEAD));
     }
 }
+template <bool THROUGH = false>   // a float32 state through the L2 (store_through_at)
 __device__ __forceinline__ void store_state(const f32x4 (&S)[NBLK], void* s, int state_f32, int bh, int ib, const Lane& L) {
     if (s == nullptr) return;
-    const long off = ((long)bh * HEAD + 16 * ib + L.g) * HEAD + 4 * L.n;
+    const int in_head = (16 * ib + L.g) * HEAD + 4 * L.n;
+    const long head = (long)bh * HEAD * HEAD, off = head + in_head;
 #pragma unroll
     for (int i = 0; i < NBLK; i++) {
-        if (state_f32) *reinterpret_cast<f32x4*>(static_cast<float*>(s) + off + 4 * i * HEAD) = S[i];
+        if (THROUGH && state_f32) store_through_at(static_cast<float*>(s) + head, 4 * (in_head + 4 * i * HEAD), S[i]);
+        else if (state_f32) *reinterpret_cast<f32x4*>(static_cast<float*>(s) + off + 4 * i * HEAD) = S[i];
         else *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(s) + off + 4 * i * HEAD) = to_bf16(S[i]);
     }
 }
@@ -619,7 +622,7 @@ __device__ __forceinline__ void finish_tokens(const HeadTile& s, const float* ln
 
 // One token per sequence: block = (some rows of a 16-row tile, head).  Every wavefront asks for the first state it updates
 // before the expansion starts, and for the next before it updates one.
-template <int GROUPS>   // row groups: a wavefront updates every GROUPS-th of the block's rows
+template <int GROUPS, bool THROUGH>   // row groups: a wavefront updates every GROUPS-th of the block's rows
 __global__ __launch_bounds__(256 * GROUPS) void decode_head_kernel(const HeadArgs A, int rows_per_block) {
     __shared__ HeadTile s;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -638,7 +641,7 @@ __global__ __launch_bounds__(256 * GROUPS) void decode_head_kernel(const HeadArg
     for (int r = r0 + group; r < end; r += GROUPS) {
         fetch(Sn, r + GROUPS);   // (past the last row: that row again, unused)
         update_state(s, S, token_vectors(s, r, ib, L), r, ib, L);
-        store_state(S, A.state, A.state_f32, (row0 + r) * A.H + h, ib, L);
+        store_state<THROUGH>(S, A.state, A.state_f32, (row0 + r) * A.H + h, ib, L);
 #pragma unroll
         for (int i = 0; i < NBLK; i++) S[i] = Sn[i];
     }
@@ -734,6 +737,11 @@ int head_rows_per_block(int B, int H) {
     while (rpb < 8 && (long)H * ((B + rpb - 1) / rpb) > compute_units()) rpb *= 2;
     return rpb;
 }
+
+// The new states are written through the L2s while these, 32 MiB in all, hold most of them at the kernel's end and would be
+// written back then; more than that leaves in the course of the kernel by itself.  12 heads, left to the end / through, 8 sequences (a row to a block) 19.6 /
+// 19.6, 32 23.0 / 22.6, 64 26.9 / 25.9, 96 31.5 / 30.8, 128 (24 MiB) 32.6 / 32.1, 170 38.3 / 39.0, 256 43.7 / 44.1.
+bool states_through(int B, int H) { return (long)B * H * HEAD * HEAD * (long)sizeof(float) <= 24 << 20; }
 
 // Blocks of a linear kernel for each tile (or two), of so many columns.
 int column_blocks(const LinArgs& a, int columns) {
@@ -850,9 +858,11 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         if (T > 1)
             hipLaunchKernelGGL(prompt_head_kernel, dim3(H, B), dim3(256), 0, stream, a);
         else if (rpb == 1)
-            hipLaunchKernelGGL(decode_head_kernel<1>, grid, dim3(256), 0, stream, a, rpb);
+            hipLaunchKernelGGL((decode_head_kernel<1, false>), grid, dim3(256), 0, stream, a, rpb);
+        else if (states_through(B, H))
+            hipLaunchKernelGGL((decode_head_kernel<2, true>), grid, dim3(512), 0, stream, a, rpb);
         else
-            hipLaunchKernelGGL(decode_head_kernel<2>, grid, dim3(512), 0, stream, a, rpb);
+            hipLaunchKernelGGL((decode_head_kernel<2, false>), grid, dim3(512), 0, stream, a, rpb);
     }
     {
         LinArgs a{};
