@@ -193,6 +193,16 @@ int wind_rwkv7_attn_ln_prefill(int B, int T, int H, int C, int io_dtype, int sta
                                void* y, void* scratch, void* sT,
                                void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same for sequences of T - 16 + n tokens, 0 < n < 16 (head size 64, bf16): their last chunk in w, k, b leaves a state as it is
+ * (wind_rwkv7_neutral_rows), and kept [3,B,16,H*64] bf16 holds what its w, k and b were.  The n tokens are then taken by
+ * wind_rwkv7_attn_ln_tokens; y behind them is undefined. */
+int wind_rwkv7_attn_ln_prefill_ragged(int B, int T, int H, int C, int n, int state_dtype,
+                                      const void* w, const void* q, const void* k, const void* v,
+                                      const void* a, const void* b, const void* g, const void* params,
+                                      const void* kept, const void* s0,
+                                      void* y, void* scratch, void* sT,
+                                      void* workspace, size_t workspace_bytes, void* stream);
+
 int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int state_dtype,
                                 const void* w, const void* q, const void* k, const void* v,
                                 const void* a, const void* b, const void* g, const void* params,
@@ -466,6 +476,9 @@ typedef struct {
     long long ldT;
 } wind_rwkv7_pack;
 int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream);
+/* ... and in the same launch what wind_rwkv7_pad_rows does. */
+int wind_rwkv7_pack_weights_pad_rows(int n, const wind_rwkv7_pack* tensors, int B, int T, int T_out, int C, const void* x, void* out, void* last,
+                                     void* stream);
 
 /* Products of token-major bf16 matrices with weights, up to WIND_RWKV7_LINEAR_GROUP_MAX of them on the same M tokens in one
  * launch; replaces the matmuls of TimeMixer.forward (time_mixer.py:120-131, :167) and of their input gradients.  A problem is

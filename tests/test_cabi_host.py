@@ -399,6 +399,16 @@ def test_pad_rows_validates_on_host():
     assert lib.wind_rwkv7_pad_rows(2, 32, 19, 64, 0x1000, 0x2000, 0x3000, None) == 2   # token T-1 is not among the output's
 
 
+def test_ragged_prefill_validates_on_host():
+    lib = _native.lib()
+    ok = [2, 32, 3, 64, 5, _native.F32] + [0x1000] * 9 + [None, 0x2000, 0x3000, 0x4000, 0x5000, 1 << 40, None]
+    for idx, val, code in [(0, 0, 2), (1, 31, 4), (2, 0, 2), (3, 128, 3), (4, 0, 2), (4, 16, 2), (5, 7, 5), (6, None, 1), (14, None, 1), (16, None, 1),
+                           (17, None, 1), (18, None, 1)]:
+        bad = list(ok)
+        bad[idx] = val
+        assert lib.wind_rwkv7_attn_ln_prefill_ragged(*bad) == code, (idx, val)
+
+
 def test_attn_ln_tokens_validates_on_host():
     lib = _native.lib()
     ok = [2, 32, 3, 64, 16, 5, _native.F32] + [0x1000] * 8 + [16, 0, None, 0x2000, 0x3000, None]

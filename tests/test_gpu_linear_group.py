@@ -22,6 +22,27 @@ def _problem(segments, pieces):
     return p
 
 
+def _pad_and_pack(x, T_out):
+    from wind_rwkv import _native
+    B, T, C = x.shape
+    a = torch.randn(80, 192, device=DEV)
+    dst, out, last = torch.zeros(80, 192, device=DEV, dtype=torch.bfloat16), torch.full((B, T_out, C), 7., device=DEV, dtype=torch.bfloat16), torch.empty_like(x[:, 0])
+    arr = (_native.Pack * 1)()
+    p = arr[0]
+    p.src, p.dst, p.rows, p.cols, p.src_dtype, p.dst_dtype, p.dstT, p.ldT = a.data_ptr(), dst.data_ptr(), 80, 192, _native.F32, _native.BF16, None, 0
+    _native.check(_native.lib().wind_rwkv7_pack_weights_pad_rows(1, arr, B, T, T_out, C, x.data_ptr(), out.data_ptr(), last.data_ptr(),
+                                                                 torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return torch.equal(dst, a.bfloat16()), out, last
+
+
+@pytest.mark.parametrize('B,T,T_out,C', [(1, 1, 16, 8), (3, 33, 48, 72), (2, 1003, 1008, 768)])
+def test_rows_padded_beside_packed_weights(B, T, T_out, C):
+    x = torch.randn(B, T, C, device=DEV).bfloat16()
+    packed, out, last = _pad_and_pack(x, T_out)
+    assert packed and torch.equal(out[:, :T], x) and not out[:, T:].any() and torch.equal(last, x[:, -1])
+
+
 def _run(problems, M):
     from wind_rwkv import _native
     arr = (_native.Linear * len(problems))(*problems)

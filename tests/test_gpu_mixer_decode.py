@@ -135,3 +135,27 @@ def test_pad_rows(B, T, T_out, C):
     n = min(T, T_out)
     assert torch.equal(out[:, :n], x[:, :n]) and not out[:, n:].any()
     assert T_out < T or torch.equal(last, x[:, -1])
+
+
+# one sequence and more, two chunks and more; from 16 heads on the epilogue goes through the chunks head by head; 140 (batch, head)s: the one-kernel form
+@pytest.mark.parametrize('B,T,H,n', [(1, 32, 1, 1), (2, 48, 3, 15), (3, 112, 17, 7), (1, 1024, 12, 9), (140, 32, 1, 3)])
+@pytest.mark.parametrize('f32', [True, False])
+def test_ragged_prefill_is_prefill_and_tokens(B, T, H, n, f32):
+    from wind_rwkv import _native
+    lib, stream, gen = _native.lib(), torch.cuda.current_stream().cuda_stream, torch.Generator().manual_seed(T + H)
+    rn = lambda *s: torch.randn(*s, generator=gen).to(DEV)
+    seqs = [(rn(B, T, H * 64) * 0.3).bfloat16() for _ in range(7)]   # w q k v a b g
+    params, s0 = rn(3, H * 64), rn(B, H, 64, 64).to(torch.float32 if f32 else torch.bfloat16)
+    kept = torch.empty(3, B, 16, H * 64, device=DEV, dtype=torch.bfloat16)
+    _native.check(lib.wind_rwkv7_neutral_rows_keep(B, T, H * 64, T - 16, seqs[0].data_ptr(), seqs[2].data_ptr(), seqs[5].data_ptr(), kept.data_ptr(), stream))
+    ptrs, state = [t.data_ptr() for t in (*seqs, params)], _native.F32 if f32 else _native.BF16
+    ws = torch.empty(max(16, lib.wind_rwkv7_attn_fwd_workspace_bytes(B, T, H, 64)), device=DEV, dtype=torch.uint8)
+    scratch = torch.empty(lib.wind_rwkv7_attn_ln_saved_bytes(B, T, H, 64), device=DEV, dtype=torch.uint8)
+    (y1, S1), (y2, S2) = ((torch.full_like(seqs[0], float('nan')), torch.empty_like(s0)) for _ in range(2))
+    end = lambda S: (scratch.data_ptr(), S.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+    _native.check(lib.wind_rwkv7_attn_ln_prefill(B, T, H, 64, _native.BF16, state, *ptrs, s0.data_ptr(), y1.data_ptr(), *end(S1)))
+    _native.check(lib.wind_rwkv7_attn_ln_tokens(B, T, H, 64, T - 16, n, state, kept[0].data_ptr(), ptrs[1], kept[1].data_ptr(), ptrs[3], ptrs[4],
+                                                kept[2].data_ptr(), ptrs[6], ptrs[7], 16, 0, S1.data_ptr(), y1.data_ptr(), S1.data_ptr(), stream))
+    _native.check(lib.wind_rwkv7_attn_ln_prefill_ragged(B, T, H, 64, n, state, *ptrs, kept.data_ptr(), s0.data_ptr(), y2.data_ptr(), *end(S2)))
+    valid = T - 16 + n
+    assert torch.equal(S1, S2) and torch.equal(y1[:, :valid], y2[:, :valid])

@@ -349,12 +349,18 @@ size_t wind_rwkv7_attn_ln_bwd_workspace_least_bytes(int B, int T, int H, int C) 
     return !all || C != wkv::HEAD ? all : all - scan_bytes(B, T, H, wkv::SCAN_BACKWARD) + scan_least_bytes(B, T, H);
 }
 
+// The tokens of a prompt's last chunk, which the sequence kernels were given as neutral ones: n of them, with their own w, k, b
+struct TailTokens {
+    int n;
+    const void *w, *k, *b;   // [B,16,H*64]
+};
+
 static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_dtype,
                            const void* w, const void* q, const void* k, const void* v,
                            const void* a, const void* b, const void* g, const void* params,
                            const void* s0,
                            void* y, void* s, void* sT,
-                           void* workspace, size_t workspace_bytes, int save, void* stream_) {
+                           void* workspace, size_t workspace_bytes, int save, void* stream_, const TailTokens* tail = nullptr) {
     int rc = check_shape(B, T, H, C, true);
     if (rc) return rc;
     rc = check_dtypes(io_dtype, state_dtype);
@@ -363,6 +369,10 @@ static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_d
     rc = check_workspace(workspace, workspace_bytes, wind_rwkv7_attn_fwd_workspace_least_bytes(B, T, H, C));
     if (rc) return rc;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
+    auto tokens = [&](const wkv::KeptOutput* epilogue) {
+        wkv::launch_tokens(B, T, H, T - wkv::CHUNK, tail->n, wkv::CHUNK, 0, state_dtype == WIND_RWKV7_F32, tail->w, q, tail->k, v, a, tail->b, g,
+                           params, sT, sT, y, stream, epilogue);
+    };
     if (C != wkv::HEAD) {
         char* y_wide = static_cast<char*>(s) + wind_rwkv7_attn_saved_bytes(B, T, H, C);
         float* centers = reinterpret_cast<float*>(y_wide + wide_seq_bytes(B, T, H, C));
@@ -388,6 +398,13 @@ static int attn_ln_forward(int B, int T, int H, int C, int io_dtype, int state_d
                                   pair_states(B, T, H), stream,
                                   g, params, y_wkv, centers);
         st.mark("wkv7_fused_kernel[fwd]");
+        if (tail) tokens(nullptr);
+        return launch_status();
+    }
+    if (tail) {
+        const wkv::KeptOutput kept{y_wkv, centers, k};
+        tokens(&kept);
+        st.mark("epilogue_tokens_kernel");
         return launch_status();
     }
     wkv::launch_ln_epilogue(B, T, H, y_wkv, centers, q, k, v, g, params, y, stream);
@@ -413,6 +430,24 @@ int wind_rwkv7_attn_ln_prefill(int B, int T, int H, int C, int io_dtype, int sta
                                void* workspace, size_t workspace_bytes, void* stream) {
     return attn_ln_forward(B, T, H, C, io_dtype, state_dtype, w, q, k, v, a, b, g, params, s0, y, scratch, sT, workspace,
                            workspace_bytes, 0, stream);
+}
+
+int wind_rwkv7_attn_ln_prefill_ragged(int B, int T, int H, int C, int n, int state_dtype,
+                                      const void* w, const void* q, const void* k, const void* v,
+                                      const void* a, const void* b, const void* g, const void* params,
+                                      const void* kept, const void* s0,
+                                      void* y, void* scratch, void* sT,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+    if (n < 1 || n >= wkv::CHUNK) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (C != wkv::HEAD) return WIND_RWKV7_ERR_HEAD_SIZE;
+    const int rc = check_shape(B, T, H, C, true);
+    if (rc) return rc;
+    if (!kept) return WIND_RWKV7_ERR_NULL_POINTER;
+    const size_t part = (size_t)B * wkv::CHUNK * H * C * 2;   // bytes
+    auto at = [&](int i) { return static_cast<const char*>(kept) + i * part; };
+    const TailTokens tail{n, at(0), at(1), at(2)};
+    return attn_ln_forward(B, T, H, C, WIND_RWKV7_BF16, state_dtype, w, q, k, v, a, b, g, params, s0, y, scratch, sT, workspace,
+                           workspace_bytes, 0, stream, &tail);
 }
 
 int wind_rwkv7_attn_ln_backward(int B, int T, int H, int C, int io_dtype, int state_dtype,
@@ -951,7 +986,7 @@ int wind_rwkv7_block_wgrads(int n, long long tokens, const int* O, const int* I,
     return wgrads(true, n, tokens, O, I, dy, ld_dy, x, ld_x, dW, out_dtype, workspace, workspace_bytes, stream);
 }
 
-int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream) {
+static int pack_weights(int n, const wind_rwkv7_pack* tensors, const wkv::PadRows& pad, void* stream) {
     if (n < 1 || n > WIND_RWKV7_PACK_MAX) return WIND_RWKV7_ERR_BAD_SHAPE;
     if (!tensors) return WIND_RWKV7_ERR_NULL_POINTER;
     wkv::PackTensor P[WIND_RWKV7_PACK_MAX];
@@ -969,8 +1004,25 @@ int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream)
         P[t] = wkv::PackTensor{u.src, u.dst, u.dstT, u.rows, u.cols, (long)u.ldT, u.src_dtype == WIND_RWKV7_F32, u.dst_dtype == WIND_RWKV7_F32,
                                src % 16 == 0};
     }
-    wkv::launch_pack_weights(n, P, static_cast<hipStream_t>(stream));
+    wkv::launch_pack_weights(n, P, pad, static_cast<hipStream_t>(stream));
     return launch_status();
+}
+
+int wind_rwkv7_pack_weights(int n, const wind_rwkv7_pack* tensors, void* stream) { return pack_weights(n, tensors, wkv::PadRows{}, stream); }
+
+static int check_pad(int B, int T, int T_out, int C, const void* x, const void* out, const void* last) {
+    if (B <= 0 || T <= 0 || T_out <= 0 || C <= 0 || C % 8 != 0 || (long long)B * T * C > (1LL << 38) || (long long)B * T_out * C > (1LL << 38))
+        return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (last && T_out < T) return WIND_RWKV7_ERR_BAD_SHAPE;
+    if (!x || !out) return WIND_RWKV7_ERR_NULL_POINTER;
+    return WIND_RWKV7_OK;
+}
+
+int wind_rwkv7_pack_weights_pad_rows(int n, const wind_rwkv7_pack* tensors, int B, int T, int T_out, int C, const void* x, void* out, void* last,
+                                     void* stream) {
+    const int rc = check_pad(B, T, T_out, C, x, out, last);
+    if (rc) return rc;
+    return pack_weights(n, tensors, wkv::PadRows{B, T, T_out, C, x, out, last}, stream);
 }
 
 int wind_rwkv7_linear_group(int n, long long M, const wind_rwkv7_linear* problems, void* stream) {
@@ -1032,11 +1084,9 @@ int wind_rwkv7_neutral_rows_keep(int B, int T, int C, int first, void* w, void* 
 }
 
 int wind_rwkv7_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, void* stream) {
-    if (B <= 0 || T <= 0 || T_out <= 0 || C <= 0 || C % 8 != 0 || (long long)B * T * C > (1LL << 38) || (long long)B * T_out * C > (1LL << 38))
-        return WIND_RWKV7_ERR_BAD_SHAPE;
-    if (last && T_out < T) return WIND_RWKV7_ERR_BAD_SHAPE;
-    if (!x || !out) return WIND_RWKV7_ERR_NULL_POINTER;
-    wkv::launch_pad_rows(B, T, T_out, C, x, out, last, static_cast<hipStream_t>(stream));
+    const int rc = check_pad(B, T, T_out, C, x, out, last);
+    if (rc) return rc;
+    wkv::launch_pad_rows(wkv::PadRows{B, T, T_out, C, x, out, last}, static_cast<hipStream_t>(stream));
     return launch_status();
 }
 

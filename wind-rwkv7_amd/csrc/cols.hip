@@ -11,7 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "frag.hpp"
+#include "pad_rows.hpp"
 
 namespace wkv {
 namespace {
@@ -78,26 +78,14 @@ __global__ __launch_bounds__(256) void neutral_rows_kernel(int T, int C, int fir
     *reinterpret_cast<bf16x8*>(b + at) = zero;
 }
 
-// Bound by the launch (stored through the L2 3.5 -> 3.2): 2 x 1003 tokens x 768 channels take 3.4-4.1 us; a fill, a copy and a copy of the last token, 11.
-__global__ __launch_bounds__(256) void pad_rows_kernel(int T, int T_out, int C, long vectors, const __bf16* __restrict__ x,
-                                                       __bf16* __restrict__ out, __bf16* __restrict__ last) {
-    const long v = (long)blockIdx.x * 256 + threadIdx.x;
-    if (v >= vectors) return;
-    const int per_row = C / 8, col = (int)(v % per_row) * 8;
-    const long row = v / per_row, b = row / T_out;
-    const int t = (int)(row - b * T_out);
-    bf16x8 r = {};
-    if (t < T) r = *reinterpret_cast<const bf16x8*>(x + (b * T + t) * C + col);
-    store_through(out + row * C + col, r);
-    if (last != nullptr && t == T - 1) *reinterpret_cast<bf16x8*>(last + b * C + col) = r;
-}
+// Bound by the launch (stored through the L2 3.5 -> 3.2 us): 2 x 1003 tokens x 768 channels take 3.4-4.1 us; a fill, a copy and a copy of the last token, 11.
+__global__ __launch_bounds__(256) void pad_rows_kernel(const PadArgs p) { pad_rows_block(p, blockIdx.x); }
 
 }  // namespace
 
-void launch_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, hipStream_t stream) {
-    const long vectors = (long)B * T_out * (C / 8);
-    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)((vectors + 255) / 256)), dim3(256), 0, stream, T, T_out, C, vectors,
-                       static_cast<const __bf16*>(x), static_cast<__bf16*>(out), static_cast<__bf16*>(last));
+void launch_pad_rows(const PadRows& p, hipStream_t stream) {
+    const PadArgs a(p);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3(a.blocks), dim3(256), 0, stream, a);
 }
 
 void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, hipStream_t stream) {

@@ -50,7 +50,12 @@ void launch_cast_to_bf16(int n, const void* const* src, const int* src_f32, cons
                          const long long* dst_offset, void* dst, hipStream_t stream);
 
 // x [B,T,C] to out [B,T_out,C]: the first T tokens, zeros behind them; last (may be null) [B,C]: token T - 1, if out has it
-void launch_pad_rows(int B, int T, int T_out, int C, const void* x, void* out, void* last, hipStream_t stream);
+struct PadRows {
+    int B, T, T_out, C;   // B = 0: nothing to pad
+    const void* x;
+    void *out, *last;
+};
+void launch_pad_rows(const PadRows& p, hipStream_t stream);
 // rows first .. T-1 of w, k, b [B, T, C] (bf16): decay 1, k = b = 0; kept (may be null) [3, B, T-first, C]: what they were
 void launch_neutral_rows(int B, int T, int C, int first, void* w, void* k, void* b, void* kept, hipStream_t stream);
 
@@ -63,7 +68,7 @@ struct PackTensor {
     int src_f32, dst_f32, src_aligned;   // src_aligned: to 16 bytes
 };
 constexpr int PACK_MAX_TENSORS = 32;
-void launch_pack_weights(int n, const PackTensor* tensors, hipStream_t stream);
+void launch_pack_weights(int n, const PackTensor* tensors, const PadRows& pad, hipStream_t stream);   // pad: in the same launch
 
 // D[m][n] = sum_k A0[m][k] W0[n][k] (+ sum_k A1[m][k] W1[n][k]); see linear_group.hip.  K[1] = 0: one segment.  The columns
 // start[t] .. start[t] + width[t] - 1 go to out[t] (row stride ld_out[t]); aux[t]: [M, width[t]].

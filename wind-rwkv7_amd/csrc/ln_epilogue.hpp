@@ -10,6 +10,7 @@
 // the reference needs a shared-memory reduction across warps with four block barriers for each.
 #pragma once
 #include "frag.hpp"
+#include "wkv7_common.hpp"
 
 namespace wkv {
 
@@ -107,6 +108,28 @@ __device__ __forceinline__ TileB ln_forward(const TileF& y, const TileB& q, cons
         out.f[ib] = to_bf16(x2 * to_f32(g.f[ib]));
     }
     return out;
+}
+
+// What the epilogue as a stage of its own reads and writes: [B,T,H*64] tensors, y_wkv as it is kept
+struct LnForwardArgs {
+    int T, H;
+    const __bf16* y_wkv;
+    const float* centers;
+    const __bf16 *q, *k, *v, *g;
+    const float* params;
+    __bf16* y;
+};
+// a wavefront's chunk
+__device__ __forceinline__ void ln_forward_chunk(const LnForwardArgs& A, int cid, const Lane& L) {
+    const ChunkAddr ca(cid, A.T, A.H);
+    const TileB yw = load_rows16(A.y_wkv + ca.row0, ca.ld, L);
+    const TileB q = load_rows16(A.q + ca.row0, ca.ld, L);
+    const TileB k = load_rows16(A.k + ca.row0, ca.ld, L);
+    const TileB v = load_rows16(A.v + ca.row0, ca.ld, L);
+    const TileB g = load_rows16(A.g + ca.row0, ca.ld, L);
+    const LnParams p = load_ln_params(A.params, ca.bh % A.H, A.H, L);
+    const TileF yf = uncentre(yw, A.centers, ca.row0 / HEAD + (long)L.n * A.H);   // (row0 / 64 = token * H + head of the chunk's first token)
+    store_rows16_streamed(A.y + ca.row0, ca.ld, L, ln_forward(yf, q, k, v, g, p));
 }
 
 // backward of the epilogue for one chunk.  y is the saved WKV7 output.

@@ -681,11 +681,10 @@ struct TokensArgs {
     const void* state_in;                       // null: zeros
     void* state;                                // may be state_in itself
 };
-__global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
-    __shared__ HeadTile s;
+__device__ __forceinline__ void tokens_block(HeadTile& s, const TokensArgs& A, const int bh) {
     const int lane = threadIdx.x & 63, ib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Lane L;
-    const int bh = blockIdx.x, seq = bh / A.H, h = bh - seq * A.H;
+    const int seq = bh / A.H, h = bh - seq * A.H;
     f32x4 S[NBLK];
     load_state(S, A.state_in, A.state_f32, bh, ib, L);
     // 16 bytes per thread and load: eight channels of one of the sixteen tokens, two tensors at a time (wavefronts 0, 1 and 2, 3)
@@ -712,6 +711,21 @@ __global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
         lds_barrier();   // (the next sixteen overwrite what the epilogue reads)
     }
     store_state(S, A.state, A.state_f32, bh, ib, L);
+}
+__global__ __launch_bounds__(256) void tokens_kernel(const TokensArgs A) {
+    __shared__ HeadTile s;
+    tokens_block(s, A, blockIdx.x);
+}
+// The same as the first blocks of the launch that applies the epilogue to the chunks before those tokens (all but a sequence's last
+// chunk: the tokens are in that one).  Neither stage fills the chip or waits for the other: 2 x 1003 tokens x 12 heads 6.6 + 8.6 us in two launches,
+// so 10.0 (the blocks' LDS leaves seven of them to a compute unit, which the epilogue does not need).
+__global__ __launch_bounds__(256) void epilogue_tokens_kernel(const TokensArgs A, int tokens_blocks, const LnForwardArgs E, int chunks) {
+    __shared__ HeadTile s;
+    if ((int)blockIdx.x < tokens_blocks) return tokens_block(s, A, blockIdx.x);   // (the whole block)
+    const int wid = (blockIdx.x - tokens_blocks) * 4 + (threadIdx.x >> 6);
+    if (wid >= chunks) return;
+    const int NC = E.T / CHUNK, i = E.H >= 16 ? head_major_chunk(wid, chunks, E.T - CHUNK) : wid, bh = i / (NC - 1);
+    ln_forward_chunk(E, i + bh, Lane());   // (chunk c of NC - 1 of each (batch, head), as one of NC)
 }
 
 constexpr size_t A256(size_t x) { return (x + 255) / 256 * 256; }
@@ -885,13 +899,20 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
 
 void launch_tokens(int B, int T, int H, int first, int n, int wkb_T, int wkb_first, int state_f32, const void* w, const void* q, const void* k,
                    const void* v, const void* a, const void* b, const void* g, const void* params, const void* state_in, void* state,
-                   void* y, hipStream_t stream) {
+                   void* y, hipStream_t stream, const KeptOutput* epilogue) {
     const int C = H * HEAD;
     auto at = [&](const void* p, int token) { return static_cast<const __bf16*>(p) + (long)token * C; };
     const TokensArgs A{at(w, wkb_first), at(k, wkb_first), at(b, wkb_first), at(q, first), at(v, first), at(a, first), at(g, first),
                        static_cast<__bf16*>(y) + (long)first * C, (long)wkb_T * C, (long)T * C, n, H, C, state_f32,
                        static_cast<const float*>(params), state_in, state};
-    hipLaunchKernelGGL(tokens_kernel, dim3((unsigned)(B * H)), dim3(256), 0, stream, A);
+    if (epilogue == nullptr || T <= CHUNK) {
+        hipLaunchKernelGGL(tokens_kernel, dim3((unsigned)(B * H)), dim3(256), 0, stream, A);
+        return;
+    }
+    auto whole = [&](const void* p) { return static_cast<const __bf16*>(p); };
+    const LnForwardArgs E{T, H, whole(epilogue->y_wkv), epilogue->centers, whole(q), whole(epilogue->k), whole(v), whole(g), A.ln_params, static_cast<__bf16*>(y)};
+    const int chunks = B * H * (T / CHUNK - 1);
+    hipLaunchKernelGGL(epilogue_tokens_kernel, dim3((unsigned)(B * H + (chunks + 3) / 4)), dim3(256), 0, stream, A, B * H, E, chunks);
 }
 
 }  // namespace wkv

@@ -23,9 +23,15 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
                          const void* state_in, void* state, void* y, void* x_carry, void* workspace, hipStream_t stream);
 
 // WKV7 with the GroupNorm + bonus + gate epilogue, token by token on a state in fp32 registers: n tokens from `first` on of
-// q, v, a, g and y [B,T,H*64]; of w, k, b [B,wkb_T,H*64] the n from wkb_first on.  State as above.
+// q, v, a, g and y [B,T,H*64]; of w, k, b [B,wkb_T,H*64] the n from wkb_first on.  State as above.  epilogue not null (the tokens are in
+// the last chunk of T, a multiple of 16): in the same launch also the attn_ln epilogue of the chunks before, from their kept output.
+struct KeptOutput {
+    const void* y_wkv;      // [B,T,H*64], centred with `centers` (see Centred in ln_epilogue.hpp)
+    const float* centers;
+    const void* k;          // [B,T,H*64]
+};
 void launch_tokens(int B, int T, int H, int first, int n, int wkb_T, int wkb_first, int state_f32, const void* w, const void* q, const void* k,
                    const void* v, const void* a, const void* b, const void* g, const void* params, const void* state_in, void* state,
-                   void* y, hipStream_t stream);
+                   void* y, hipStream_t stream, const KeptOutput* epilogue = nullptr);
 
 }  // namespace wkv

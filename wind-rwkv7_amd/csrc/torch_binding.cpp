@@ -34,14 +34,14 @@ namespace py = pybind11;
     X(attn_saved_bytes) X(attn_fwd_workspace_bytes) X(attn_train_workspace_bytes) X(attn_bwd_workspace_bytes)        \
     X(attn_forward) X(attn_prefill) X(attn_backward)                                                                 \
     X(attn_ln_saved_bytes) X(attn_ln_bwd_workspace_bytes)                                                            \
-    X(attn_ln_forward) X(attn_ln_prefill) X(attn_ln_backward)                                                        \
+    X(attn_ln_forward) X(attn_ln_prefill) X(attn_ln_prefill_ragged) X(attn_ln_backward)                                                        \
     X(attn_f32_saved_bytes) X(attn_f32_forward) X(attn_f32_prefill) X(attn_f32_backward_split)                       \
     X(attn_f32_bwd_workspace_bytes)                                                                                  \
     X(ddlerp_bwd_workspace_bytes) X(ddlerp_forward) X(ddlerp_backward)                                               \
     X(expand_loras_bwd_workspace_bytes) X(expand_loras_forward) X(expand_loras_forward_padded) X(expand_loras_backward) X(cast_to_bf16)             \
     X(ddlerp_first_workspace_bytes) X(ddlerp_first) X(attn_ln_tokens) X(pad_rows) X(linear_wgrad_workspace_bytes) X(linear_wgrad)           \
     X(block_wgrads_workspace_bytes) X(block_wgrads) X(mixer_decode_workspace_bytes) X(mixer_decode) \
-    X(mixer_prompt) X(linear_group) X(pack_weights) X(expand_loras_backward_to)
+    X(mixer_prompt) X(linear_group) X(pack_weights) X(pack_weights_pad_rows) X(expand_loras_backward_to)
 
 struct Lib {
 #define X(name) decltype(&wind_rwkv7_##name) name = nullptr;
@@ -621,7 +621,12 @@ struct WeightLayout {
 using B16 = c10::BFloat16;
 B16* at_elem(const Tensor& t, int64_t o) { return static_cast<B16*>(t.data_ptr()) + o; }
 
-void pack_weights(const WeightLayout& L_, const variable_list& p, const Tensor& buf, bool transposed) {
+// A prompt's rows on their way to whole chunks, in the launch that packs the weights: x [B,T,C] to out, [B,C] of it to last (may be undefined)
+struct Padding {
+    Tensor x, out, last;
+};
+
+void pack_weights(const WeightLayout& L_, const variable_list& p, const Tensor& buf, bool transposed, const Padding& pad = {}) {
     wind_rwkv7_pack t[PARAMS];
     for (int i = 0; i < PARAMS; i++) {
         const auto shape = param_shape(i, L_.C);
@@ -643,7 +648,11 @@ void pack_weights(const WeightLayout& L_, const variable_list& p, const Tensor& 
         turn(DECAY_W1, L_.Tw1, W_DECAY_AAA_MA), turn(AAA_W1, L_.Tw1 + R_DECAY, W_DECAY_AAA_MA);
         turn(MA_W1, L_.Tw1 + R_DECAY + R_LORA, W_DECAY_AAA_MA);
     }
-    check(L.pack_weights(PARAMS, t, stream_of(buf)));
+    if (pad.x.defined())
+        check(L.pack_weights_pad_rows(PARAMS, t, pad.x.size(0), pad.x.size(1), pad.out.size(1), pad.x.size(2), ptr(pad.x), ptr(pad.out), ptr(pad.last),
+                                      stream_of(buf)));
+    else
+        check(L.pack_weights(PARAMS, t, stream_of(buf)));
 }
 
 struct Block {   // the sizes of a call
@@ -783,16 +792,16 @@ struct First {
 
 // x [B,T,C] bf16 contiguous, T a multiple of 16.  `save`: keep what the backward needs.  `first` / s0: a carried state
 // (undefined: zero).  `valid` < T (head size 64, not with `save`): the tokens from there on are padding, y has none of
-// them.  The sequence kernels then take the whole chunks and leave the tokens after them to attn_ln_tokens, which keeps the
+// them.  The sequence kernels then take the whole chunks and leave the tokens after them to attn_ln_prefill_ragged's second half, which keeps the
 // state in fp32 from token to token (a chunk's products would round those tokens' share of it to bf16 operands).
 void block_forward(const Block& s, const Tensor& xb, const variable_list& p, bool save, int64_t valid, const First& first,
-                   const Tensor& s0, const BlockBuffers& f) {
+                   const Tensor& s0, const BlockBuffers& f, const Padding& pad = {}) {
     const int B = s.B, T = s.T, C = s.C, H = s.H, N = s.N();
     const int64_t M = s.rows(), P = s.plane();
     void* stream = stream_of(xb);
     const WeightLayout W(C);
     const Activations A(s, save);
-    pack_weights(W, p, f.weights, save);
+    pack_weights(W, p, f.weights, save, pad);
     auto a = [&](int64_t o) -> void* { return at_elem(f.acts, o); };
     auto w = [&](int i) -> void* { return at_elem(f.weights, W.at_.at[i]); };
     check(L.ddlerp_forward(B, T, C, R_MIX, ptr(xb), w(MAA_X), w(MAA_W1), w(MAA_W2), w(MAA), a(A.mid), a(A.der), a(A.streams), stream));
@@ -819,17 +828,18 @@ void block_forward(const Block& s, const Tensor& xb, const variable_list& p, boo
     check(L.expand_loras_forward_padded(B, T, C, R_LORA, N, a(A.w2), a(A.k), a(A.kk1), a(A.a1), a(A.ma1), a(A.mk1), w(KKK_W2), w(AAA_W2),
                                         w(MA_W2), w(MK_W2), w(DECAY), w(AAAAA), w(MISC_A), w(MISC_K), a(A.w), a(A.k2), a(A.kk), a(A.b),
                                         kept.defined() ? ptr(kept) : nullptr, stream));
-    if (whole) {
+    if (whole && rest) {
+        const Tensor ws = scratch_bytes(L.attn_fwd_workspace_bytes(B, T, H, N), xb);
+        check(L.attn_ln_prefill_ragged(B, T, H, N, rest, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g),
+                                       at_elem(f.weights, W.ln), ptr(kept), ptr(s0), ptr(f.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
+    } else if (whole) {
         const Tensor ws = scratch_bytes((save ? L.attn_train_workspace_bytes : L.attn_fwd_workspace_bytes)(B, T, H, N), xb);
         check((save ? L.attn_ln_forward : L.attn_ln_prefill)(
             B, T, H, N, WIND_RWKV7_BF16, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g), at_elem(f.weights, W.ln),
             ptr(s0), ptr(f.ya), ptr(f.saved), ptr(f.sT), ptr(ws), ws.numel(), stream));
-    }
-    if (rest) {
-        const int64_t part = kept.defined() ? kept.stride(0) : 0;
-        check(L.attn_ln_tokens(B, T, H, N, whole, rest, state_code(f.sT), whole ? at_elem(kept, 0) : a(A.w), a(A.r),
-                               whole ? at_elem(kept, part) : a(A.k2), a(A.v), a(A.kk), whole ? at_elem(kept, 2 * part) : a(A.b), a(A.g),
-                               at_elem(f.weights, W.ln), whole ? T - whole : T, 0, whole ? ptr(f.sT) : ptr(s0), ptr(f.ya), ptr(f.sT), stream));
+    } else {   // (fewer tokens than a chunk)
+        check(L.attn_ln_tokens(B, T, H, N, 0, rest, state_code(f.sT), a(A.w), a(A.r), a(A.k2), a(A.v), a(A.kk), a(A.b), a(A.g),
+                               at_elem(f.weights, W.ln), T, 0, ptr(s0), ptr(f.ya), ptr(f.sT), stream));
     }
     Products out;
     if (!rest) {
@@ -1147,14 +1157,13 @@ py::object mixer(const Tensor& x, const py::dict& own, const py::dict& norm, int
     const at::ScalarType state_type = s0.defined() ? s0.scalar_type() : stateful ? at::kFloat : at::kBFloat16;
     if (T % 16 && s.N() == 64 && T <= SHORT_PROMPT && s.B * T <= SHORT_PROMPT_ROWS) return short_prompt(s.B, T, s.C, H, x, p, x_prev, s0, state_type, return_state);
     Tensor xb = dense_bf16(x), carry;
+    Padding pad;
     if (s.T != T) {
-        const Tensor whole = at::empty({s.B, s.T, s.C}, xb.options());
-        if (return_state && x.scalar_type() == at::kBFloat16) carry = at::empty({s.B, s.C}, xb.options());   // (the carried token keeps x's own type)
-        check(L.pad_rows((int)s.B, (int)T, (int)s.T, (int)s.C, ptr(xb), ptr(whole), ptr(carry), stream_of(xb)));
-        xb = whole;
+        pad.x = xb, pad.out = xb = at::empty({s.B, s.T, s.C}, xb.options());
+        if (return_state && x.scalar_type() == at::kBFloat16) pad.last = carry = at::empty({s.B, s.C}, xb.options());   // (the carried token keeps x's own type)
     }
     const BlockBuffers f(s, xb, false, T, state_type);
-    block_forward(s, xb, p, false, T, x_prev.defined() ? First(x.select(1, 0), x_prev) : First(), s0, f);
+    block_forward(s, xb, p, false, T, x_prev.defined() ? First(x.select(1, 0), x_prev) : First(), s0, f, pad);
     if (!return_state) return py::cast(f.y);
     return py::make_tuple(f.y, py::make_tuple(carry.defined() ? carry : x.select(1, T - 1).clone(), f.sT));
 }

@@ -65,23 +65,10 @@ __global__ __launch_bounds__(256) void segment_carry_kernel(int PER, const float
 // attn_ln epilogue: one wavefront per chunk applies GroupNorm + bonus + gate to the WKV7 output the scan
 // left in y_wkv (kept, bf16, for the backward pass; centred per block when `centers` is given, see ln_epilogue.hpp).
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void ln_epilogue_kernel(int T, int H, int nchunks, const __bf16* __restrict__ y_wkv,
-                                                          const float* __restrict__ centers, const __bf16* __restrict__ q_, const __bf16* __restrict__ k_,
-                                                          const __bf16* __restrict__ v_, const __bf16* __restrict__ g_,
-                                                          const float* __restrict__ params, __bf16* __restrict__ y_) {
+__global__ __launch_bounds__(256) void ln_epilogue_kernel(const LnForwardArgs A, int nchunks) {
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wid >= nchunks) return;
-    const int cid = H >= 16 ? head_major_chunk(wid, nchunks, T) : wid;   // (long rows: see head_major_chunk)
-    const Lane L;
-    const ChunkAddr ca(cid, T, H);
-    const TileB yw = load_rows16(y_wkv + ca.row0, ca.ld, L);
-    const TileB q = load_rows16(q_ + ca.row0, ca.ld, L);
-    const TileB k = load_rows16(k_ + ca.row0, ca.ld, L);
-    const TileB v = load_rows16(v_ + ca.row0, ca.ld, L);
-    const TileB g = load_rows16(g_ + ca.row0, ca.ld, L);
-    const LnParams p = load_ln_params(params, ca.bh % H, H, L);
-    const TileF yf = uncentre(yw, centers, ca.row0 / HEAD + (long)L.n * H);   // (row0 / 64 = token * H + head of the chunk's first token)
-    store_rows16_streamed(y_ + ca.row0, ca.ld, L, ln_forward(yf, q, k, v, g, p));
+    ln_forward_chunk(A, A.H >= 16 ? head_major_chunk(wid, nchunks, A.T) : wid, Lane());   // (long rows: see head_major_chunk)
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -158,8 +145,8 @@ void launch_ln_epilogue(int B, int T, int H, const void* y_wkv, const float* cen
                         const void* v, const void* g, const void* params, void* y, hipStream_t stream) {
     const int nchunks = B * H * (T / CHUNK);
     auto c = [](const void* p) { return static_cast<const __bf16*>(p); };
-    hipLaunchKernelGGL(ln_epilogue_kernel, dim3((nchunks + 3) / 4), dim3(256), 0, stream, T, H, nchunks, c(y_wkv), centers, c(q),
-                       c(k), c(v), c(g), static_cast<const float*>(params), static_cast<__bf16*>(y));
+    const LnForwardArgs A{T, H, c(y_wkv), centers, c(q), c(k), c(v), c(g), static_cast<const float*>(params), static_cast<__bf16*>(y)};
+    hipLaunchKernelGGL(ln_epilogue_kernel, dim3((nchunks + 3) / 4), dim3(256), 0, stream, A, nchunks);
 }
 
 }  // namespace wkv

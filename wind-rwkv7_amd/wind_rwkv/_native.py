@@ -54,6 +54,7 @@ SIGNATURES = {
     'wind_rwkv7_attn_ln_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_ln_forward': (_i, [_i] * 6 + [_vp] * 9 + [_vp] * 3 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_ln_prefill': (_i, [_i] * 6 + [_vp] * 9 + [_vp] * 3 + [_vp, _sz, _vp]),
+    'wind_rwkv7_attn_ln_prefill_ragged': (_i, [_i] * 6 + [_vp] * 10 + [_vp] * 3 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_ln_backward': (_i, [_i] * 6 + [_vp] * 8 + [_vp] * 3 + [_vp] * 9 + [_vp, _sz, _vp]),
     'wind_rwkv7_attn_decode': (_i, [_i] * 5 + [_vp] * 6 + [_vp, _vp, _vp]),
     'wind_rwkv7_attn_ln_decode': (_i, [_i] * 5 + [_vp] * 8 + [_vp, _vp, _vp]),
@@ -86,6 +87,7 @@ SIGNATURES = {
     'wind_rwkv7_attn_f32_bwd_workspace_bytes': (_sz, [_i] * 4),
     'wind_rwkv7_attn_f32_backward_split': (_i, [_i] * 4 + [_vp] * 6 + [_vp] * 3 + [_vp] * 7 + [_vp, _sz] + [_vp]),
     'wind_rwkv7_pack_weights': (_i, [_i, _vp, _vp]),
+    'wind_rwkv7_pack_weights_pad_rows': (_i, [_i, _vp] + [_i] * 4 + [_vp] * 4),
     'wind_rwkv7_linear_group': (_i, [_i, _ll, _vp, _vp]),
     'wind_rwkv7_linear_wgrad_workspace_bytes': (_sz, [_ll, _i, _i]),
     'wind_rwkv7_linear_wgrad': (_i, [_ll, _i, _i, _vp, _ll, _vp, _ll, _vp, _i, _vp, _sz, _vp]),
