@@ -18,7 +18,7 @@
 //
 // Measured (us; in brackets the library's kernels for the same, replayed without host time): six first-half products of a
 // 768-channel block with their tanh and cut columns at 2006 / 8192 / 32768 tokens 19.5 (49) / 50 (69) / 170 (203); three input
-// gradients with one second segment at 8192 38 (55); a single 768 x 768 product at 512 / 8192 / 65536 tokens 8.1 (6.4) / 16.5 (16) /
+// gradients with one second segment at 8192 38 (55); a single 768 x 768 product at 512 / 8192 / 65536 tokens 7.3 (6.4) / 15.5 (16) /
 // 82-90 (70).  Of the 54 us of six on inputs out of memory the matrix instructions alone take 28 (their rate on these numbers, not on
 // zeros, is 1.3 PFLOP/s), with the LDS reads 32, with the loads 39; the output is the rest.  Blocks that stay and fetch the next tile's
 // first stage while they write this one's output: 54.  Stages of
@@ -29,6 +29,8 @@
 #include "device_info.hpp"
 
 #include "frag.hpp"
+
+#include <cstddef>
 
 namespace wkv {
 namespace {
@@ -43,6 +45,8 @@ __device__ __forceinline__ float tanh_of(float x) {
 }
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 using Rsrc = __amdgpu_buffer_rsrc_t;
 
 constexpr int BK = 64;           // contraction indices per stage: whole 128-byte lines of a row
@@ -55,10 +59,9 @@ struct Tile {
 };
 
 struct GroupArgs {
+    // what a block finds its tile by: of problem j its tiles (0 past the last problem), and 4 times those in a row of blocks + TNB
+    i32x16 tiles, columns;   // tiles[15]: M
     LinearProblem p[MAX_PROBLEMS];
-    int first_tile[MAX_PROBLEMS + 1];   // problem j owns tiles first_tile[j] .. first_tile[j+1]-1
-    int shape[MAX_PROBLEMS];            // TNB
-    int M, n;
 };
 
 // STAGES in LDS: two where blocks share a compute unit; four in launches that have less than a block per compute unit, where
@@ -66,6 +69,21 @@ struct GroupArgs {
 template <int TMB, int TNB, int STAGES>
 __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProblem& p, const int M, const int m0, const int n0) {
     using S = Tile<TMB, TNB>;
+    // (what the first loads need, at once: see linear_group_kernel)
+    struct Operands {
+        const __bf16 *A[2], *W[2];
+        long lda[2], ldw[2];
+    };
+    struct Lengths {
+        int K[2], N, npieces;
+    };
+    static_assert(offsetof(LinearProblem, lda) == offsetof(Operands, lda) && offsetof(LinearProblem, K) == sizeof(Operands) &&
+                  offsetof(LinearProblem, npieces) == sizeof(Operands) + offsetof(Lengths, npieces), "the head of a LinearProblem");
+    i32x16 operand_words = *reinterpret_cast<const i32x16*>(&p);
+    i32x4 length_words = *reinterpret_cast<const i32x4*>(p.K);
+    asm volatile("" : "+s"(operand_words), "+s"(length_words));
+    const Operands o = __builtin_bit_cast(Operands, operand_words);
+    const Lengths len = __builtin_bit_cast(Lengths, length_words);
     constexpr int CPR = BK / 8;                      // 16-byte pieces per row
     constexpr int RPP = 256 / CPR;                   // rows per pass of the block
     constexpr int QA = S::BM / RPP, QB = S::BN / RPP, LOADS = QA + QB;
@@ -89,18 +107,18 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
             for (int r = 0; r < 16; r++) acc[mb][nb][r] = 0.f;
 
     // stages of both segments in a row
-    const int nk0 = (p.K[0] + BK - 1) / BK, nk = nk0 + (p.K[1] + BK - 1) / BK;
+    const int nk0 = (len.K[0] + BK - 1) / BK, nk = nk0 + (len.K[1] + BK - 1) / BK;
     Rsrc ra, rb;
     unsigned aoff[QA], boff[QB];
     int kseg = 0;
     auto enter_segment = [&](int g) {   // descriptors at the tile's first rows; rows past the ends repeat the last
-        ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.A[g] + (long)m0 * p.lda[g]), 0, 0x7fffffff, 0x00020000);
-        rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.W[g] + (long)n0 * p.ldw[g]), 0, 0x7fffffff, 0x00020000);
+        ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(o.A[g] + (long)m0 * o.lda[g]), 0, 0x7fffffff, 0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(o.W[g] + (long)n0 * o.ldw[g]), 0, 0x7fffffff, 0x00020000);
 #pragma unroll
-        for (int q = 0; q < QA; q++) aoff[q] = (unsigned)min(lrow + RPP * q, M - 1 - m0) * (unsigned)p.lda[g] * 2;
+        for (int q = 0; q < QA; q++) aoff[q] = (unsigned)min(lrow + RPP * q, M - 1 - m0) * (unsigned)o.lda[g] * 2;
 #pragma unroll
-        for (int q = 0; q < QB; q++) boff[q] = (unsigned)min(lrow + RPP * q, p.N - 1 - n0) * (unsigned)p.ldw[g] * 2;
-        kseg = p.K[g];
+        for (int q = 0; q < QB; q++) boff[q] = (unsigned)min(lrow + RPP * q, len.N - 1 - n0) * (unsigned)o.ldw[g] * 2;
+        kseg = len.K[g];
     };
     auto k_of = [&](int kt) { return BK * (kt >= nk0 ? kt - nk0 : kt); };
     auto issue = [&](int kt) {
@@ -148,7 +166,7 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
         for (int mb = 0; mb < TMB; mb++) a[set][mb] = *reinterpret_cast<const bf16x8*>(st + a_base + mb * 32 * BK * 2 + rd[ks]);
 #pragma unroll
         for (int nb = 0; nb < TNB; nb++) b[set][nb] = *reinterpret_cast<const bf16x8*>(st + b_base + nb * 32 * BK * 2 + rd[ks]);
-        if (ks > 0 && 16 * ks >= p.K[kt >= nk0 ? 1 : 0] - k_of(kt)) {   // past a segment's end: zeros
+        if (ks > 0 && 16 * ks >= len.K[kt >= nk0 ? 1 : 0] - k_of(kt)) {   // past a segment's end: zeros
 #pragma unroll
             for (int mb = 0; mb < TMB; mb++) a[set][mb] = bf16x8{};
 #pragma unroll
@@ -158,6 +176,11 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
 #pragma unroll
     for (int st = 0; st < STAGES; st++)
         if (st < nk) issue(st);
+    // (where a single tensor takes the output, while the operands are on their way)
+    __bf16* out0 = p.out[0];
+    long ld_out0 = p.ld_out[0];
+    int op0 = p.op[0];
+    asm volatile("" : "+s"(out0), "+s"(ld_out0), "+s"(op0));
     arrived(min(nk - 1, STAGES - 1));
     read(0, 0, 0);
     for (int kt = 0; kt < nk; kt++) {
@@ -183,11 +206,11 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
     // out, each lane finding its tensor and waiting for its operand: the two gradients through tanh of a 768-channel block at 32768 tokens 40.6 us, now
     // 35.6; six first halves at 512 tokens 13.9, now 13.5.)
     const int m_first = m0 + 32 * TMB * wm, n_first = n0 + 32 * TNB * wn;
-    const bool plain = p.npieces == 1 && p.op[0] == LINEAR_PLAIN;
+    const bool plain = len.npieces == 1 && op0 == LINEAR_PLAIN;
     auto tensor_of = [&](int col) {
         int t = 0;
 #pragma unroll
-        for (int k = 1; k < LinearProblem::PIECES; k++) t += k < p.npieces && col >= p.start[k] ? 1 : 0;
+        for (int k = 1; k < LinearProblem::PIECES; k++) t += k < len.npieces && col >= p.start[k] ? 1 : 0;
         return t;
     };
     auto of = [&](int t, auto f) {
@@ -203,7 +226,7 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int col = n_first + 32 * nb + 8 * q, t = tensor_of(col);
-                const bool wanted = of(t, [&](int k) { return p.op[k]; }) == LINEAR_TANH_GRAD && col < p.N;
+                const bool wanted = of(t, [&](int k) { return p.op[k]; }) == LINEAR_TANH_GRAD && col < len.N;
                 const int width = of(t, [&](int k) { return p.width[k]; });
                 const __bf16* const aux = of(t, [&](int k) { return p.aux[k]; }) + (col - of(t, [&](int k) { return p.start[k]; }) + 4 * half);
 #pragma unroll
@@ -263,7 +286,7 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
         for (int i = 0; i < 2 * TMB * TNB; i++) {
             int m, col;
             const bf16x8* v = rows_of(i, m, col);
-            if (m < M && col < p.N) store_through(p.out[0] + (long)m * p.ld_out[0] + col, *v);
+            if (m < M && col < len.N) store_through(out0 + (long)m * ld_out0 + col, *v);
         }
         return;
     }
@@ -271,7 +294,7 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
     for (int i = 0; i < 2 * TMB * TNB; i++) {
         int m, col;
         const bf16x8* v = rows_of(i, m, col);
-        if (m < M && col < p.N) {
+        if (m < M && col < len.N) {
             const int t = tensor_of(col);
             __bf16* const out = of(t, [&](int k) { return p.out[k]; }) + (long)m * of(t, [&](int k) { return p.ld_out[k]; });
             store_through(out + (col - of(t, [&](int k) { return p.start[k]; })), *v);
@@ -285,31 +308,29 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void linear_group_kernel(
     // Blocks go to the eight XCDs in turn (block b to XCD b % 8), and each XCD has an L2 of its own.  An XCD takes a run of
     // consecutive tiles, i.e. some row blocks of a problem with all their column blocks: it reads each of its rows of the
     // input once and keeps the weight.
-    const int nt = G.first_tile[G.n];
-    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
-    int t = -1;
-    {   // problem by problem: tiles of XCD x are [T x / 8, T (x+1) / 8) of each problem's T
-        int rest = i;
-#pragma unroll 1
-        for (int j = 0; j < G.n && t < 0; j++) {
-            const int T = G.first_tile[j + 1] - G.first_tile[j];
-            const int lo = T * x / 8, hi = T * (x + 1) / 8;
-            if (rest < hi - lo) t = G.first_tile[j] + lo + rest;
-            else rest -= hi - lo;
-        }
-    }
-    if (t < 0 || t >= nt) return;   // (whole block)
-    int j = 0;
+    // All of it in scalar registers before it is looked at, and so with a tile's operands and its output: left to the compiler these are
+    // scalar loads where each is used, seven one after the other before the first load of an operand (77 x 8 x 8 3.9 -> 3.1 us, one
+    // 768 x 768 product at 512 tokens 8.3 -> 7.3, at 2006 10.7 -> 9.5, two second halves at 2006 5.6 -> 4.9, four input gradients at 512 12.0 -> 10.7).
+    i32x16 tiles = G.tiles, columns = G.columns;
+    asm volatile("" : "+s"(tiles), "+s"(columns));
+    const unsigned x = blockIdx.x % 8;
+    unsigned rest = blockIdx.x / 8, tile = 0;
+    int j = -1, of_row = 5;
 #pragma unroll
-    for (int k = 1; k < MAX_PROBLEMS; k++) j += (k < G.n && t >= G.first_tile[k]) ? 1 : 0;
+    for (int k = 0; k < MAX_PROBLEMS; k++) {   // problem by problem: tiles of XCD x are [T x / 8, T (x+1) / 8) of each problem's T
+        const unsigned T = tiles[k], lo = T * x / 8, here = T * (x + 1) / 8 - lo;
+        const bool found = j < 0 && rest < here;
+        j = found ? k : j, tile = found ? lo + rest : tile, of_row = found ? columns[k] : of_row;
+        rest -= here;   // (not looked at any more once it is found)
+    }
+    if (j < 0) return;   // (whole block)
     const LinearProblem& p = G.p[j];
-    const int bn = 64 * G.shape[j], ncol = (p.N + bn - 1) / bn;
-    const int tile = t - G.first_tile[j];
-    const int m0 = tile / ncol * (64 * TMB), n0 = tile % ncol * bn;
-    switch (G.shape[j]) {
-        case 1: gemm_tile<TMB, 1, STAGES>(lds, p, G.M, m0, n0); break;
-        case 2: gemm_tile<TMB, 2, STAGES>(lds, p, G.M, m0, n0); break;
-        default: gemm_tile<TMB, 3, STAGES>(lds, p, G.M, m0, n0); break;
+    const unsigned ncol = of_row >> 2, shape = of_row & 3;
+    const int M = tiles[15], m0 = tile / ncol * (64 * TMB), n0 = tile % ncol * (64 * shape);
+    switch (shape) {
+        case 1: gemm_tile<TMB, 1, STAGES>(lds, p, M, m0, n0); break;
+        case 2: gemm_tile<TMB, 2, STAGES>(lds, p, M, m0, n0); break;
+        default: gemm_tile<TMB, 3, STAGES>(lds, p, M, m0, n0); break;
     }
 }
 
@@ -317,18 +338,19 @@ __global__ __launch_bounds__(256, STAGES == 2 ? 2 : 1) void linear_group_kernel(
 
 void launch_linear_group(int n, long M, const LinearProblem* problems, hipStream_t stream) {
     GroupArgs G{};
-    G.n = n;
-    G.M = (int)M;
+    static_assert(MAX_PROBLEMS < 15, "one place is left for M");
+    G.tiles[15] = (int)M;
     // Columns per block (64 times this): as many of a problem's as the shape allows, since wide tiles read least per product.
+    int all = 0;
     auto plan = [&](int rows, int widest) {
-        G.first_tile[0] = 0;
+        all = 0;
         for (int j = 0; j < n; j++) {
             const int N = problems[j].N, blocks = (N + 63) / 64;
-            G.shape[j] = blocks < widest ? blocks : widest == 3 && N % 192 != 0 && N <= 256 ? 2 : widest;
-            const int bn = 64 * G.shape[j];
-            G.first_tile[j + 1] = G.first_tile[j] + (int)((M + rows - 1) / rows) * ((N + bn - 1) / bn);
+            const int shape = blocks < widest ? blocks : widest == 3 && N % 192 != 0 && N <= 256 ? 2 : widest, ncol = (blocks + shape - 1) / shape;
+            G.columns[j] = 4 * ncol + shape;
+            all += G.tiles[j] = (int)((M + rows - 1) / rows) * ncol;
         }
-        return G.first_tile[n];
+        return all;
     };
     for (int j = 0; j < n; j++) G.p[j] = problems[j];
     // 128 tokens x 192 columns where that gives every compute unit a block; else 64 tokens, and narrower until most have one
@@ -340,14 +362,14 @@ void launch_linear_group(int n, long M, const LinearProblem* problems, hipStream
     for (int x = 0; x < 8; x++) {
         int c = 0;
         for (int j = 0; j < n; j++) {
-            const int T = G.first_tile[j + 1] - G.first_tile[j];
+            const int T = G.tiles[j];
             c += T * (x + 1) / 8 - T * x / 8;
         }
         most = c > most ? c : most;
     }
     const dim3 grid(8 * most), block(256);
     if (!small) hipLaunchKernelGGL((linear_group_kernel<2, 2>), grid, block, 0, stream, G);
-    else if (G.first_tile[n] > compute_units()) hipLaunchKernelGGL((linear_group_kernel<1, 2>), grid, block, 0, stream, G);
+    else if (all > compute_units()) hipLaunchKernelGGL((linear_group_kernel<1, 2>), grid, block, 0, stream, G);
     else hipLaunchKernelGGL((linear_group_kernel<1, 4>), grid, block, 0, stream, G);
 }
 
