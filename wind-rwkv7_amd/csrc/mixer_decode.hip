@@ -233,13 +233,25 @@ struct LinSeg {
     int stream;          // LERP: which interpolation
 };
 constexpr int MAX_SEGS = 9;
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 struct LinArgs {
+    i32x16 plan;                 // of the launch: blocks of each pair (0 past the last one); PLAN_C and so on
     LinSeg seg[MAX_SEGS];
     int nseg, C, rows, ntiles;   // rows: output rows that exist (stores beyond are dropped)
 };
 
+enum { PLAN_C = 13, PLAN_ROWS, PLAN_TILES };
+static_assert(MAX_SEGS <= PLAN_C && sizeof(LinSeg) == 40 && sizeof(MixIn) == 48, "what the kernel below takes into scalar registers");
+
+template <class T>
+__device__ __forceinline__ T* global_pointer(int lo, int hi) {   // (an address that the compiler has lost sight of, to global memory all the same)
+    return (T*)(__attribute__((address_space(1))) T*)((unsigned long)(unsigned)lo | (unsigned long)(unsigned)hi << 32);
+}
+
 template <bool LERP, int CB, int RT>
-__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, const MixIn mix) {
+__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, const MixIn mix_arg) {
     constexpr int NW = 4;
     constexpr int U = CB * RT == 1 ? 3 : CB * RT <= 4 ? 2 : 1;   // steps of a wavefront in flight
     // R too passes through LDS where there are several column blocks: its fragments touch two lines per four lanes, not four, and
@@ -255,41 +267,39 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, con
     } lds;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l8 = lane >> 3, piece = lane & 7;
     const Lane L;
-    // which pair this block belongs to (the descriptor fields through scalar selects, not an indexed copy of the
-    // argument struct)
-    int blk = blockIdx.x;
-    const __bf16* __restrict__ in = nullptr;
-    const __bf16* __restrict__ W = nullptr;
-    __bf16* __restrict__ out = nullptr;
-    int N = 0, act = 0, ks = 0;
-    bool found = false;
+    // Which pair this block belongs to.  The plan and the token shift's operands come in one cluster of scalar loads, then the pair's
+    // own in another: left to the compiler each is loaded where it is looked at, a chain of twelve before the first load of a weight
+    // (a replayed step of 12 heads, 1, 16, 64, 128 sequences 16.9, 19.1, 25.4, 32.0 -> 16.6, 18.7, 24.6, 31.2 us).
+    i32x16 plan = A.plan;
+    i32x8 m8 = *reinterpret_cast<const i32x8*>(&mix_arg);
+    i32x4 m4 = *reinterpret_cast<const i32x4*>(&mix_arg.mid);
+    if constexpr (LERP) asm volatile("" : "+s"(plan), "+s"(m8), "+s"(m4));
+    else asm volatile("" : "+s"(plan));
+    const MixIn mix = {global_pointer<const __bf16>(m8[0], m8[1]), global_pointer<const __bf16>(m8[2], m8[3]), global_pointer<const __bf16>(m8[4], m8[5]),
+                       global_pointer<const __bf16>(m8[6], m8[7]), global_pointer<__bf16>(m4[0], m4[1]), m4[2], m4[3]};
+    int blk = blockIdx.x, pair = -1, col_block = 0;
 #pragma unroll
     for (int i = 0; i < MAX_SEGS; i++) {
-        if (!found && i < A.nseg) {
-            const int nb = (A.seg[i].N + 16 * CB - 1) / (16 * CB);
-            if (blk < nb) {
-                found = true;
-                in = A.seg[i].in;
-                W = A.seg[i].W;
-                out = A.seg[i].out;
-                N = A.seg[i].N;
-                act = A.seg[i].tanh_out;
-                ks = A.seg[i].stream;
-            } else {
-                blk -= nb;
-            }
-        }
+        const bool found = pair < 0 && blk < plan[i];
+        pair = found ? i : pair, col_block = found ? blk : col_block;
+        blk -= plan[i];
     }
-    if (!found) return;   // (whole block; the grid is exactly the sum of the pairs' blocks)
-    const int C = A.C;
-    const int col0 = 16 * CB * blk;
+    if (pair < 0) return;   // (whole block; the grid is exactly the sum of the pairs' blocks)
+    i32x8 s8 = *reinterpret_cast<const i32x8*>(&A.seg[pair]);
+    i32x4 s4 = {A.seg[pair].tanh_out, A.seg[pair].stream, 0, 0};
+    asm volatile("" : "+s"(s8), "+s"(s4));
+    const __bf16* __restrict__ in = global_pointer<const __bf16>(s8[0], s8[1]);
+    const __bf16* __restrict__ W = global_pointer<const __bf16>(s8[2], s8[3]);
+    __bf16* __restrict__ out = global_pointer<__bf16>(s8[4], s8[5]);
+    const int N = s8[6], act = s8[7], ks = s4[1], C = plan[PLAN_C], rows = plan[PLAN_ROWS], ntiles = plan[PLAN_TILES];
+    const int col0 = 16 * CB * col_block;
     int trow[RT];       // this lane's row of each tile (a tile past the last repeats it and is not stored)
     const __bf16 *irow[RT], *prow[RT];
     bf16x8 bm[RT];
     bool zero[RT];
 #pragma unroll
     for (int t = 0; t < RT; t++) {
-        const int tile = blockIdx.y * RT + t < (unsigned)A.ntiles ? blockIdx.y * RT + t : A.ntiles - 1;
+        const int tile = blockIdx.y * RT + t < (unsigned)ntiles ? blockIdx.y * RT + t : ntiles - 1;
         trow[t] = tile * TOK + L.n;
         if constexpr (LERP) {
             const TokenRows tr = token_rows(mix, trow[t], C);
@@ -408,7 +418,7 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, con
             for (int q = 0; q < 4; q++) r[q] = tanhf_(r[q]);
         }
         const int row = (blockIdx.y * RT + t) * TOK + L.n;
-        if (row < A.rows && col0 + 16 * cb < N) *reinterpret_cast<bf16x4*>(out + (long)row * N + col0 + 16 * cb + 4 * L.g) = to_bf16(r);
+        if (row < rows && col0 + 16 * cb < N) *reinterpret_cast<bf16x4*>(out + (long)row * N + col0 + 16 * cb + 4 * L.g) = to_bf16(r);
     }
 }
 
@@ -790,17 +800,17 @@ bool output_grouped(long rows, long C) { return rows * C * C >= 3000000000; }
 // channels, 1 24.1, 21.9, 24.6, 26.5; 48 46.9, 38.8, 37.4, 40.8; the output, 768 channels, 48 23.8, 24.7, 25.4, 25.7; 256 45.0,
 // 45.3, 44.7, 45.5; 1024 channels, 96 38.0, 36.3, 37.1, 38.1; 2048 channels, 144 79.6, 75.1, 75.3, 73.1.
 template <bool LERP>
-void launch_linear(const LinArgs& a, const MixIn& mix, hipStream_t stream) {
+void launch_linear(LinArgs a, const MixIn& mix, hipStream_t stream) {
     auto one_round = [&](int columns) { return column_blocks(a, columns) * a.ntiles <= compute_units(); };
-    const dim3 threads(256);
-    if ((!LERP || a.ntiles == 1) && one_round(16))
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 1, 1>), dim3(column_blocks(a, 16), a.ntiles), threads, 0, stream, a, mix);
-    else if (one_round(32))
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 2, 1>), dim3(column_blocks(a, 32), a.ntiles), threads, 0, stream, a, mix);
-    else if (one_round(64))
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 1>), dim3(column_blocks(a, 64), a.ntiles), threads, 0, stream, a, mix);
-    else
-        hipLaunchKernelGGL((decode_linear_kernel<LERP, 4, 2>), dim3(column_blocks(a, 64), (a.ntiles + 1) / 2), threads, 0, stream, a, mix);
+    auto go = [&](auto kernel, int columns, int tiles) {
+        a.plan[PLAN_C] = a.C, a.plan[PLAN_ROWS] = a.rows, a.plan[PLAN_TILES] = a.ntiles;
+        for (int i = 0; i < a.nseg; i++) a.plan[i] = (a.seg[i].N + columns - 1) / columns;
+        hipLaunchKernelGGL(kernel, dim3(column_blocks(a, columns), (a.ntiles + tiles - 1) / tiles), dim3(256), 0, stream, a, mix);
+    };
+    if ((!LERP || a.ntiles == 1) && one_round(16)) go(decode_linear_kernel<LERP, 1, 1>, 16, 1);
+    else if (one_round(32)) go(decode_linear_kernel<LERP, 2, 1>, 32, 1);
+    else if (one_round(64)) go(decode_linear_kernel<LERP, 4, 1>, 64, 1);
+    else go(decode_linear_kernel<LERP, 4, 2>, 64, 2);
 }
 }  // namespace
 
