@@ -45,6 +45,22 @@ struct Dy4 {  // the four upstream gradients, each [M, C]
 struct Shifted {
     bf16x8 cur, prev;
 };
+// Whether each of a block's TPB tiles begins a sequence (sequences are whole tiles): one division, of 32-bit numbers that the whole block
+// shares.  (A remainder of 64-bit numbers per row was 180 instructions for each ahead of a block's first load, and two of them a tile in forward 2;
+// so 2016 tokens x 768 channels, forward 1 and 2, 7.9, 7.1 -> 7.7, 6.3 us, 8192, backward 1 and 2 too, 12.8, 12.9, 17.1, 35.8 -> 12.6, 12.5, 16.8, 35.2.)
+template <int TPB>
+struct TileStarts {
+    bool start[TPB];
+    __device__ __forceinline__ explicit TileStarts(int T) {
+        const unsigned per_sequence = (unsigned)T / TOK;
+        unsigned pos = blockIdx.x * TPB % per_sequence;
+#pragma unroll
+        for (int p = 0; p < TPB; p++) {
+            start[p] = pos == 0;
+            pos = pos + 1 == per_sequence ? 0 : pos + 1;
+        }
+    }
+};
 template <int TPB>
 struct TokenRows {   // this thread's tokens of a block's tiles: token t8 + 32 i, channels 8 piece of every channel block
     static constexpr int N = TPB / 2;
@@ -52,11 +68,12 @@ struct TokenRows {   // this thread's tokens of a block's tiles: token t8 + 32 i
     bool has_prev[N];
     long m[N];
     __device__ __forceinline__ TokenRows(const __bf16* __restrict__ x, long M, int T, int C, int t8, int piece) {
+        const TileStarts<TPB> tiles(T);
 #pragma unroll
         for (int i = 0; i < N; i++) {
             const long want = (long)blockIdx.x * (TPB * TOK) + t8 + 32 * i;
             m[i] = want < M ? want : M - 1;   // (rows of a spare tile: the last one again, never stored)
-            has_prev[i] = m[i] % T != 0;
+            has_prev[i] = t8 % TOK != 0 || !(t8 < TOK ? tiles.start[2 * i] : tiles.start[2 * i + 1]);
             row[i] = x + m[i] * C + 8 * piece;
         }
     }
@@ -119,10 +136,11 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_mid_few_kernel(long M, int T, 
     const int ncb = C / 64, db0 = NB * blockIdx.y;
     const __bf16* row[NR];
     bool has_prev[NR];
+    const TileStarts<TPB> tiles(T);
 #pragma unroll
     for (int i = 0; i < NR; i++) {
         const long want = (long)blockIdx.x * (TPB * TOK) + l8 + 8 * i, m = want < M ? want : M - 1;   // (a spare tile stores nothing)
-        has_prev[i] = m % T != 0;
+        has_prev[i] = (l8 + 8 * i) % TOK != 0 || !tiles.start[i / 2];
         row[i] = x + m * C + 8 * piece;
     }
     f32x4 acc[TPB][NB];
@@ -454,14 +472,17 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int
     const unsigned row_bytes = 2 * C, lane_bytes = l8 * row_bytes + 16 * piece;   // (16 rows: 32 C bytes, below 2^32)
     struct Rows {
         bf16x8 x[2], before, mid[MP / 4];
+        bool inside;   // the tile does not begin a sequence
     };
+    const unsigned per_sequence = (unsigned)T / TOK;   // (tiles are few enough for 32 bits)
     auto fetch = [&](long tile) {
         Rows r;
         const long m0 = tile * TOK;
         const __bf16* xt = x + m0 * C + c0;
 #pragma unroll
         for (int i = 0; i < 2; i++) r.x[i] = piece_at(xt, lane_bytes + 8 * i * row_bytes);
-        r.before = piece_at(m0 % T != 0 ? xt - C : xt, 16 * piece);
+        r.inside = (unsigned)tile % per_sequence != 0;
+        r.before = piece_at(r.inside ? xt - C : xt, 16 * piece);
 #pragma unroll
         for (int i = 0; i < MP / 4; i++) r.mid[i] = piece_at(bmid + m0 * (4 * D) + 512 * i, 16 * lane);
         return r;
@@ -478,7 +499,7 @@ __global__ __launch_bounds__(256) void ddlerp_fwd_out2_kernel(long M, int T, int
         const bf16x8 zero = {};
 #pragma unroll
         for (int i = 0; i < 2; i++) img.x[piece_slot(1 + l8 + 8 * i, piece)] = next.x[i];
-        if (l8 == 0) img.x[piece_slot(0, piece)] = m0 % T != 0 ? next.before : zero;
+        if (l8 == 0) img.x[piece_slot(0, piece)] = next.inside ? next.before : zero;
 #pragma unroll
         for (int i = 0; i < MP / 4; i++) img.mid[mid_slot((lane + 64 * i) / MP, (lane + 64 * i) % MP)] = next.mid[i];
         wave_lds_order();
@@ -722,7 +743,7 @@ __global__ __launch_bounds__(256 * G, D == 32 ? 2 : 1) void ddlerp_bwd_main_kern
             valpha += da * xxv;
         }
     };
-    int tpos = (int)(((hi - 1) * TOK) % T);
+    int tpos = (int)((unsigned)(hi - 1) % ((unsigned)T / TOK)) * TOK;
     const bool warm = hi < ntiles && tpos + TOK != T;   // the token after the range continues the sequence
     // Iteration i works on image i&1 while the registers hold the tile after it, fetched during iteration i-1; they
     // are written to the other image (last read before the previous barrier) and refilled for the tile after that.
