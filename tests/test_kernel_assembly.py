@@ -136,8 +136,11 @@ def test_scanner_sees_a_mixed_pair():
     assert len(mixed_pairs(partly)) == 1   # one register still holds the first instruction's result
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason='hipcc not found')
-def test_no_matrix_instructions_of_different_shapes_chained_through_the_accumulator():
+@pytest.fixture(scope='module')
+def assembly():
+    """[(file name, its assembly)]."""
+    if not os.path.exists(HIPCC):
+        pytest.skip('hipcc not found')
     with tempfile.TemporaryDirectory() as tmp:
         def compile_one(name):
             out = os.path.join(tmp, name + '.s')
@@ -147,7 +150,22 @@ def test_no_matrix_instructions_of_different_shapes_chained_through_the_accumula
             with open(out) as f:
                 return name, f.read()
         with ThreadPoolExecutor(max_workers=4) as pool:
-            results = list(pool.map(compile_one, FILES))
+            return list(pool.map(compile_one, FILES))
+
+
+def test_a_steps_linear_kernels_take_no_more_arguments_than_they_read(assembly):
+    """The host writes a kernel's arguments for every launch, which bounds a step of few sequences: nine pairs of 32 bytes, the plan and
+    the token shift's operands; one pair, the plan and a pointer for the output projection."""
+    sizes = {}
+    for size, name in re.findall(r'\.kernarg_segment_size:\s+(\d+)\n(?:.*\n)*?\s+\.name:\s+(\S+)', dict(assembly)['mixer_decode.hip']):
+        m = re.search(r'decode_linear_kernelILb([01])E', name)
+        if m:
+            sizes.setdefault(m.group(1), set()).add(int(size))
+    assert sizes == {'1': {64 + 9 * 32 + 48}, '0': {64 + 32 + 8}}
+
+
+def test_no_matrix_instructions_of_different_shapes_chained_through_the_accumulator(assembly):
+    results = assembly
     bad = {name: pairs[:3] for name, asm in results if (pairs := mixed_pairs(asm))}
     assert not bad, bad
     early = {name: pairs[:3] for name, asm in results if (pairs := early_lane_reads(asm))}

@@ -224,8 +224,7 @@ __global__ __launch_bounds__(256) void decode_lerp_kernel(const MixIn in, int C,
 // Every column block repeats that for its stream, so few columns per block where the launch is latency (a tile or two),
 // four and two tiles at a time where the work counts.
 // ------------------------------------------------------------------------------------------------
-struct LinSeg {
-    const __bf16* in;    // [Bp, C] (not LERP)
+struct alignas(32) LinSeg {
     const __bf16* W;     // [N, C]
     __bf16* out;         // [rows, N]
     int N;               // multiple of 16
@@ -233,17 +232,23 @@ struct LinSeg {
     int stream;          // LERP: which interpolation
 };
 constexpr int MAX_SEGS = 9;
-typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x16 __attribute__((ext_vector_type(16), aligned(32)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int mix_words8 __attribute__((ext_vector_type(8), aligned(8)));   // (as a MixIn lies)
+typedef int mix_words4 __attribute__((ext_vector_type(4), aligned(8)));
+// As many pairs as a launch has, and beside them only the input that it reads: the host writes a kernel's arguments anew for every
+// launch, and with 496 bytes for either kernel that bounded a step of few sequences (12 heads, one sequence: 15.4 us for the host to
+// issue the four launches, an eager step 19.0; with 400 and 104 bytes 13.2 and 17.1).
+template <int SEGS>
 struct LinArgs {
-    i32x16 plan;                 // of the launch: blocks of each pair (0 past the last one); PLAN_C and so on
-    LinSeg seg[MAX_SEGS];
-    int nseg, C, rows, ntiles;   // rows: output rows that exist (stores beyond are dropped)
+    i32x16 plan;   // of the launch: blocks of each pair (0 past the last one); PLAN_C and so on
+    LinSeg seg[SEGS];
 };
+template <bool LERP>
+using LinInput = std::conditional_t<LERP, MixIn, const __bf16*>;   // what is interpolated; else [Bp, C]
 
-enum { PLAN_C = 13, PLAN_ROWS, PLAN_TILES };
-static_assert(MAX_SEGS <= PLAN_C && sizeof(LinSeg) == 40 && sizeof(MixIn) == 48, "what the kernel below takes into scalar registers");
+enum { PLAN_C = 13, PLAN_ROWS, PLAN_TILES };   // rows: output rows that exist (stores beyond are dropped)
+static_assert(MAX_SEGS <= PLAN_C && sizeof(LinSeg) == 32 && sizeof(MixIn) == 48, "what the kernel below takes into scalar registers");
 
 template <class T>
 __device__ __forceinline__ T* global_pointer(int lo, int hi) {   // (an address that the compiler has lost sight of, to global memory all the same)
@@ -251,8 +256,8 @@ __device__ __forceinline__ T* global_pointer(int lo, int hi) {   // (an address 
 }
 
 template <bool LERP, int CB, int RT>
-__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, const MixIn mix_arg) {
-    constexpr int NW = 4;
+__global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs<LERP ? MAX_SEGS : 1> A, const LinInput<LERP> input) {
+    constexpr int NW = 4, SEGS = LERP ? MAX_SEGS : 1;
     constexpr int U = CB * RT == 1 ? 3 : CB * RT <= 4 ? 2 : 1;   // steps of a wavefront in flight
     // R too passes through LDS where there are several column blocks: its fragments touch two lines per four lanes, not four, and
     // a launch that is all latency pays the way (one sequence 6.1 us instead of 5.7; 64 sequences 10.5 instead of 10.9).
@@ -271,27 +276,32 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(const LinArgs A, con
     // own in another: left to the compiler each is loaded where it is looked at, a chain of twelve before the first load of a weight
     // (a replayed step of 12 heads, 1, 16, 64, 128 sequences 16.9, 19.1, 25.4, 32.0 -> 16.6, 18.7, 24.6, 31.2 us).
     i32x16 plan = A.plan;
-    i32x8 m8 = *reinterpret_cast<const i32x8*>(&mix_arg);
-    i32x4 m4 = *reinterpret_cast<const i32x4*>(&mix_arg.mid);
-    if constexpr (LERP) asm volatile("" : "+s"(plan), "+s"(m8), "+s"(m4));
-    else asm volatile("" : "+s"(plan));
-    const MixIn mix = {global_pointer<const __bf16>(m8[0], m8[1]), global_pointer<const __bf16>(m8[2], m8[3]), global_pointer<const __bf16>(m8[4], m8[5]),
-                       global_pointer<const __bf16>(m8[6], m8[7]), global_pointer<__bf16>(m4[0], m4[1]), m4[2], m4[3]};
+    MixIn mix{};
+    const __bf16* in = nullptr;
+    if constexpr (LERP) {
+        mix_words8 m8 = *reinterpret_cast<const mix_words8*>(&input);
+        mix_words4 m4 = *reinterpret_cast<const mix_words4*>(&input.mid);
+        asm volatile("" : "+s"(plan), "+s"(m8), "+s"(m4));
+        mix = {global_pointer<const __bf16>(m8[0], m8[1]), global_pointer<const __bf16>(m8[2], m8[3]), global_pointer<const __bf16>(m8[4], m8[5]),
+               global_pointer<const __bf16>(m8[6], m8[7]), global_pointer<__bf16>(m4[0], m4[1]), m4[2], m4[3]};
+    } else {
+        unsigned long at = (unsigned long)input;
+        asm volatile("" : "+s"(plan), "+s"(at));
+        in = global_pointer<const __bf16>(at, at >> 32);
+    }
     int blk = blockIdx.x, pair = -1, col_block = 0;
 #pragma unroll
-    for (int i = 0; i < MAX_SEGS; i++) {
+    for (int i = 0; i < SEGS; i++) {
         const bool found = pair < 0 && blk < plan[i];
         pair = found ? i : pair, col_block = found ? blk : col_block;
         blk -= plan[i];
     }
     if (pair < 0) return;   // (whole block; the grid is exactly the sum of the pairs' blocks)
     i32x8 s8 = *reinterpret_cast<const i32x8*>(&A.seg[pair]);
-    i32x4 s4 = {A.seg[pair].tanh_out, A.seg[pair].stream, 0, 0};
-    asm volatile("" : "+s"(s8), "+s"(s4));
-    const __bf16* __restrict__ in = global_pointer<const __bf16>(s8[0], s8[1]);
-    const __bf16* __restrict__ W = global_pointer<const __bf16>(s8[2], s8[3]);
-    __bf16* __restrict__ out = global_pointer<__bf16>(s8[4], s8[5]);
-    const int N = s8[6], act = s8[7], ks = s4[1], C = plan[PLAN_C], rows = plan[PLAN_ROWS], ntiles = plan[PLAN_TILES];
+    asm volatile("" : "+s"(s8));
+    const __bf16* __restrict__ W = global_pointer<const __bf16>(s8[0], s8[1]);
+    __bf16* __restrict__ out = global_pointer<__bf16>(s8[2], s8[3]);
+    const int N = s8[4], act = s8[5], ks = s8[6], C = plan[PLAN_C], rows = plan[PLAN_ROWS], ntiles = plan[PLAN_TILES];
     const int col0 = 16 * CB * col_block;
     int trow[RT];       // this lane's row of each tile (a tile past the last repeats it and is not stored)
     const __bf16 *irow[RT], *prow[RT];
@@ -768,9 +778,10 @@ int head_rows_per_block(int B, int H) {
 bool states_through(int B, int H) { return (long)B * H * HEAD * HEAD * (long)sizeof(float) <= 24 << 20; }
 
 // Blocks of a linear kernel for each tile (or two), of so many columns.
-int column_blocks(const LinArgs& a, int columns) {
+template <int SEGS>
+int column_blocks(const LinArgs<SEGS>& a, int columns) {
     int n = 0;
-    for (int i = 0; i < a.nseg; i++) n += (a.seg[i].N + columns - 1) / columns;
+    for (int i = 0; i < SEGS; i++) n += (a.seg[i].N + columns - 1) / columns;
     return n;
 }
 
@@ -783,9 +794,10 @@ int column_blocks(const LinArgs& a, int columns) {
 // 47.3/45.5, 256 54.8/51.9, 512 87.4/80.0; 1280 channels, 96 (one round) 40.9/42.4, 112 50.6/47.8; 2048 channels, 64 (one round)
 // 48.7/49.0, 96 66.0/57.0, 512 214/179; 704 channels, 224 40.8/43.0, 384 55.4/60.9, 768 84.9/85.3, 1024 100.8/98.1; 512
 // channels, 512 46.9/48.7, 1024 74.9/76.1, 1536 104.6/100.8.
-bool streams_in_memory(const LinArgs& a, long rows) {
-    const bool one_round = (long)column_blocks(a, 64) * ((a.ntiles + 1) / 2) <= compute_units();
-    return rows > 32 && ((a.C >= 768 && !one_round) || rows * a.C * a.C >= 400000000);
+bool streams_in_memory(const LinArgs<MAX_SEGS>& a, long rows) {
+    const long C = a.plan[PLAN_C];
+    const bool one_round = (long)column_blocks(a, 64) * ((a.plan[PLAN_TILES] + 1) / 2) <= compute_units();
+    return rows > 32 && ((C >= 768 && !one_round) || rows * C * C >= 400000000);
 }
 // The output projection alone makes nothing again, and the grouped kernel's tiles are few for it.  Linear / grouped: 1024
 // channels, 1024 rows 147.8/148.3, 1536 226.5/224.9; 1536 channels, 512 rows 114.3/116.5, 768 190.3/194.0, 1024 241.0/239.7;
@@ -800,14 +812,15 @@ bool output_grouped(long rows, long C) { return rows * C * C >= 3000000000; }
 // channels, 1 24.1, 21.9, 24.6, 26.5; 48 46.9, 38.8, 37.4, 40.8; the output, 768 channels, 48 23.8, 24.7, 25.4, 25.7; 256 45.0,
 // 45.3, 44.7, 45.5; 1024 channels, 96 38.0, 36.3, 37.1, 38.1; 2048 channels, 144 79.6, 75.1, 75.3, 73.1.
 template <bool LERP>
-void launch_linear(LinArgs a, const MixIn& mix, hipStream_t stream) {
-    auto one_round = [&](int columns) { return column_blocks(a, columns) * a.ntiles <= compute_units(); };
+void launch_linear(LinArgs<LERP ? MAX_SEGS : 1>& a, const LinInput<LERP>& input, hipStream_t stream) {   // (the blocks of each pair: filled in here)
+    const int ntiles = a.plan[PLAN_TILES];
+    auto one_round = [&](int columns) { return column_blocks(a, columns) * ntiles <= compute_units(); };
     auto go = [&](auto kernel, int columns, int tiles) {
-        a.plan[PLAN_C] = a.C, a.plan[PLAN_ROWS] = a.rows, a.plan[PLAN_TILES] = a.ntiles;
-        for (int i = 0; i < a.nseg; i++) a.plan[i] = (a.seg[i].N + columns - 1) / columns;
-        hipLaunchKernelGGL(kernel, dim3(column_blocks(a, columns), (a.ntiles + tiles - 1) / tiles), dim3(256), 0, stream, a, mix);
+        int blocks = 0;
+        for (int i = 0; i < (LERP ? MAX_SEGS : 1); i++) blocks += a.plan[i] = (a.seg[i].N + columns - 1) / columns;
+        hipLaunchKernelGGL(kernel, dim3(blocks, (ntiles + tiles - 1) / tiles), dim3(256), 0, stream, a, input);
     };
-    if ((!LERP || a.ntiles == 1) && one_round(16)) go(decode_linear_kernel<LERP, 1, 1>, 16, 1);
+    if ((!LERP || ntiles == 1) && one_round(16)) go(decode_linear_kernel<LERP, 1, 1>, 16, 1);
     else if (one_round(32)) go(decode_linear_kernel<LERP, 2, 1>, 32, 1);
     else if (one_round(64)) go(decode_linear_kernel<LERP, 4, 1>, 64, 1);
     else go(decode_linear_kernel<LERP, 4, 2>, 64, 2);
@@ -839,27 +852,24 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
         hipLaunchKernelGGL((decode_mid_kernel<16, 2>), dim3(MID / 16, ntiles), dim3(1024), 0, stream, mix, C, c(mw.time_maa_x),
                            c(mw.time_maa_w1), static_cast<__bf16*>(x_carry));
     {
-        LinArgs a{};
+        LinArgs<MAX_SEGS> a{};
         enum { XRG, XWA, XK, XV };
-        a.seg[0] = {nullptr, c(mw.Wr), r, C, 0, XRG};
-        a.seg[1] = {nullptr, c(mw.Wk), k, C, 0, XK};
-        a.seg[2] = {nullptr, c(mw.Wv), v, C, 0, XV};
-        a.seg[3] = {nullptr, c(mw.gate_w1), tg1, R_GATE, 1, XRG};
-        a.seg[4] = {nullptr, c(mw.time_decay_w1), tw1, R_DECAY, 1, XWA};
-        a.seg[5] = {nullptr, c(mw.time_kkk_w1), kk1, R_KKK, 0, XK};
-        a.seg[6] = {nullptr, c(mw.mk_w1), mk1, R_MK, 0, XK};
-        a.seg[7] = {nullptr, c(mw.time_aaa_w1), a1, R_AAA, 0, XWA};
-        a.seg[8] = {nullptr, c(mw.ma_w1), ma1, R_MA, 0, XWA};
-        a.nseg = 9;
-        a.C = C;
-        a.rows = Bp;
-        a.ntiles = ntiles;
+        a.seg[0] = {c(mw.Wr), r, C, 0, XRG};
+        a.seg[1] = {c(mw.Wk), k, C, 0, XK};
+        a.seg[2] = {c(mw.Wv), v, C, 0, XV};
+        a.seg[3] = {c(mw.gate_w1), tg1, R_GATE, 1, XRG};
+        a.seg[4] = {c(mw.time_decay_w1), tw1, R_DECAY, 1, XWA};
+        a.seg[5] = {c(mw.time_kkk_w1), kk1, R_KKK, 0, XK};
+        a.seg[6] = {c(mw.mk_w1), mk1, R_MK, 0, XK};
+        a.seg[7] = {c(mw.time_aaa_w1), a1, R_AAA, 0, XWA};
+        a.seg[8] = {c(mw.ma_w1), ma1, R_MA, 0, XWA};
+        a.plan[PLAN_C] = C, a.plan[PLAN_ROWS] = Bp, a.plan[PLAN_TILES] = ntiles;
         if (streams_in_memory(a, rows)) {
             const long plane = (long)Bp * C;
             __bf16* const streams = take(4 * BC);
             hipLaunchKernelGGL(decode_lerp_kernel, dim3(C / 32, ntiles), dim3(256), 0, stream, mix, C, streams, plane);
             LinearProblem p[MAX_SEGS]{};
-            for (int i = 0; i < a.nseg; i++) {
+            for (int i = 0; i < MAX_SEGS; i++) {
                 const LinSeg& s = a.seg[i];
                 p[i].A[0] = streams + s.stream * plane, p[i].W[0] = s.W;
                 p[i].lda[0] = p[i].ldw[0] = p[i].K[0] = C;
@@ -867,7 +877,7 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
                 p[i].out[0] = s.out, p[i].ld_out[0] = p[i].width[0] = s.N;
                 p[i].op[0] = s.tanh_out ? LINEAR_TANH : LINEAR_PLAIN;
             }
-            launch_linear_group(a.nseg, rows, p, stream);
+            launch_linear_group(MAX_SEGS, rows, p, stream);
         } else {
             launch_linear<true>(a, mix, stream);
         }
@@ -889,12 +899,9 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
             hipLaunchKernelGGL((decode_head_kernel<2, false>), grid, dim3(512), 0, stream, a, rpb);
     }
     {
-        LinArgs a{};
-        a.seg[0] = {ya, c(mw.Wo), static_cast<__bf16*>(y), C, 0, 0};
-        a.nseg = 1;
-        a.C = C;
-        a.rows = rows;
-        a.ntiles = ntiles;
+        LinArgs<1> a{};
+        a.seg[0] = {c(mw.Wo), static_cast<__bf16*>(y), C, 0, 0};
+        a.plan[PLAN_C] = C, a.plan[PLAN_ROWS] = rows, a.plan[PLAN_TILES] = ntiles;
         if (output_grouped(rows, C)) {
             LinearProblem p{};
             p.A[0] = ya, p.W[0] = c(mw.Wo);
@@ -902,7 +909,7 @@ void launch_mixer_decode(int B, int T, int C, int H, int state_f32, const MixerW
             p.npieces = 1, p.out[0] = static_cast<__bf16*>(y), p.ld_out[0] = p.width[0] = C;
             launch_linear_group(1, rows, &p, stream);
         } else {
-            launch_linear<false>(a, mix, stream);
+            launch_linear<false>(a, ya, stream);
         }
     }
 }
