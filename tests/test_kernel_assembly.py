@@ -38,7 +38,7 @@ def makefile_flags():
 FLAGS, EXTRA = makefile_flags()
 FLAGS = FLAGS + ['-S', '--cuda-device-only']
 FILES = ['wkv7_fused.hip', 'wkv7_bwd.hip', 'wkv7_fwd.hip', 'wkv7_wide.hip', 'ddlerp.hip', 'expand_loras.hip', 'expand_loras16.hip', 'mixer_decode.hip',
-         'linear_wgrad.hip', 'selftest.hip', 'wkv7_f32.hip']
+         'linear_wgrad.hip', 'selftest.hip', 'wkv7_f32.hip', 'linear_group.hip', 'cast_bf16.hip', 'cols.hip']
 WINDOW = 16   # instructions; a matrix instruction has long finished after that many
 
 MFMA = re.compile(r'(v_mfma_\w+)\s+([av]\[\d+:\d+\]),\s*(?:[av]\[\d+:\d+\]|v\d+),\s*(?:[av]\[\d+:\d+\]|v\d+),\s*([av]\[\d+:\d+\]|0)')
@@ -77,6 +77,101 @@ def mixed_pairs(asm):
                 if not pending:
                     break
     return found
+
+
+class Flow:
+    """Instructions and labels of an assembly listing in their order, and which may have run right before each."""
+
+    def __init__(self, asm):
+        self.ins, self.written_as_such = [], set()   # (the second: indices of what the sources write as assembly)
+        inside = False
+        for line in asm.split('\n'):
+            if '#ASMSTART' in line or '#ASMEND' in line:
+                inside = '#ASMSTART' in line
+                continue
+            t = line.split(';')[0].strip()
+            if not t or (t.startswith('.') and not t.endswith(':')):   # (directives; labels stay)
+                continue
+            if inside:
+                self.written_as_such.add(len(self.ins))
+            self.ins.append(t)
+        self.jumps = {}
+        for i, t in enumerate(self.ins):
+            m = re.match(r's_c?branch\S*\s+(\S+)', t)
+            if m:
+                self.jumps.setdefault(m.group(1) + ':', []).append(i)
+
+    def before(self, i):
+        """Indices of the instructions (no labels) that may have run right before instruction i."""
+        found, seen, todo = set(), set(), [i]
+        while todo:
+            j = todo.pop()
+            from_jumps = self.jumps.get(self.ins[j], []) if j != i else []
+            above = [j - 1] if j > 0 and not re.match(r's_branch\b|s_endpgm|s_setpc', self.ins[j - 1]) else []
+            for k in from_jumps + above:
+                if k in seen:
+                    continue
+                seen.add(k)
+                (todo.append if self.ins[k].endswith(':') else found.add)(k)
+        return found
+
+    def writers(self, i, regs, reach=None):
+        """The vector instructions that may have written the vector registers `regs` last before instruction i, with the wait states
+        between (those of another path from the same one: the fewest); `reach`: only those with fewer."""
+        found, best, todo = {}, {}, [(i, 0, frozenset(regs))]
+        while todo:
+            j, waits, left = todo.pop()
+            for k in self.before(j):
+                t = self.ins[k]
+                hit = left & written(t)
+                if hit:
+                    found[k] = min(waits, found.get(k, waits))
+                rest = left - hit
+                then = waits + 1 + (int(t.split()[1], 0) if t.startswith('s_nop') else 0)
+                rest = frozenset(r for r in rest if best.get((k, r), then + 1) > then)
+                best.update({(k, r): then for r in rest})
+                if rest and (reach is None or then < reach):
+                    todo.append((k, then, rest))
+        return found
+
+
+def written(t):
+    """Vector registers that an instruction writes."""
+    m = re.match(r'(v_\w+|ds_\w+|(?:global|buffer|flat|scratch)_load\w*)\s+(v\d+|v\[\d+:\d+\])(?:,\s*(v\d+))?', t)
+    if not m or (m.group(1).startswith('ds_') and not re.match(r'ds_(read|bpermute|permute|swizzle)', t)) or re.search(r'\slds\b', t):
+        return set()
+    return _regs(m.group(2)) | (_regs(m.group(3)) if 'swap' in m.group(1) and m.group(3) else set())
+
+
+def stores_of_matrix_results(asm):
+    """Stores that the sources write as assembly, of registers that a matrix instruction wrote last (or at an address in such): the compiler
+    keeps the distance which these need only for the stores that it makes itself."""
+    f, found = Flow(asm), []
+    for i in sorted(f.written_as_such):
+        if re.match(r'(global|buffer|flat)_store', f.ins[i]):
+            regs = set().union(*map(_regs, re.findall(r'\bv\d+\b|\bv\[\d+:\d+\]', f.ins[i])))
+            found += [(f.ins[k], f.ins[i]) for k in f.writers(i, regs) if 'mfma' in f.ins[k]]
+    return found
+
+
+def test_scanner_sees_a_store_of_matrix_results():
+    asm = '''
+        v_mfma_f32_32x32x16_bf16 v[16:31], v[0:3], v[4:7], v[16:31]
+        s_cbranch_scc1 .LBB0_2
+        v_mov_b32_e32 v20, 0
+    .LBB0_2:                                ; %some block
+        v_lshl_add_u64 v[8:9], s[0:1], 0, v[10:11]
+        ;;#ASMSTART
+        global_store_dwordx4 v[8:9], v[20:23], off sc1
+        s_nop 1
+        ;;#ASMEND
+        global_store_dwordx4 v[8:9], v[24:27], off
+        s_endpgm
+    '''
+    assert len(stores_of_matrix_results(asm)) == 1
+    assert not stores_of_matrix_results(asm.replace('v[20:23], off', 'v[32:35], off'))
+    assert not stores_of_matrix_results(asm.replace('v_lshl_add', 'ds_read_b128 v[20:23], v4\nv_lshl_add'))
+    assert stores_of_matrix_results(asm.replace('v_mov_b32_e32 v20, 0', 's_branch .LBB0_3'))   # (through the jump alone)
 
 
 def early_lane_reads(asm):
@@ -168,6 +263,9 @@ def test_no_matrix_instructions_of_different_shapes_chained_through_the_accumula
     results = assembly
     bad = {name: pairs[:3] for name, asm in results if (pairs := mixed_pairs(asm))}
     assert not bad, bad
+    stored = {name: pairs[:3] for name, asm in results if (pairs := stores_of_matrix_results(asm))}
+    assert not stored, stored
+    assert sum(len(Flow(asm).written_as_such) for name, asm in results if name == 'linear_group.hip')   # (what the scan is for)
     early = {name: pairs[:3] for name, asm in results if (pairs := early_lane_reads(asm))}
     assert not early, early
     assert any('v_fmac_f32_dpp' in asm for _, asm in results)   # (what the scan is for)

@@ -246,6 +246,8 @@ __device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontem
 // 16 bytes to memory at device scope: written through the XCD's L2, so that the end of the kernel, which writes back whatever that still holds
 // for the other XCDs' L2s, finds nothing left to do, and kept in the last-level cache for whoever reads them next.
 // (s_nop: two wait states before the registers of a store of more than eight bytes may be written, which the compiler sees to for its own stores.)
+// x is not the result of a matrix instruction as it stands: the distance a store needs behind that, too, the compiler keeps only for its own stores
+// (store_through_at in row_lines.hpp).
 template <class V>
 __device__ __forceinline__ void store_through(void* to, V x) {
     static_assert(sizeof(V) == 16, "one access");
