@@ -177,22 +177,11 @@ def test_scanner_sees_a_store_of_matrix_results():
 def early_lane_reads(asm):
     """v_fmac_f32_dpp instructions (written as such in the sources, so that the compiler does not place the two wait states a
     lane-crossing operand needs behind a vector instruction that writes it) with a writer of that operand less than two before them."""
-    ins = [t.strip() for t in asm.split('\n')]
-    ins = [t for t in ins if t and not t.startswith((';', '.'))]
-    found = []
-    for i, t in enumerate(ins):
+    f, found = Flow(asm), []
+    for i, t in enumerate(f.ins):
         m = re.match(r'v_fmac_f32_dpp v\d+, v(\d+),', t)
-        if not m:
-            continue
-        waits = 0
-        for p in reversed(ins[max(i - 2, 0):i]):
-            d = re.match(r'v_\w+\s+(v\d+|v\[\d+:\d+\])(?:,\s*(v\d+))?', p)
-            written = _regs(d.group(1)) if d else set()
-            if d and 'swap' in p.split()[0] and d.group(2):
-                written |= _regs(d.group(2))
-            if waits < 2 and (int(m.group(1)) in written or p.endswith(':')):   # (a label: what ran before is not seen here)
-                found.append((p, t))
-            waits += 1 + (int(p.split()[1]) if p.startswith('s_nop') else 0)
+        if m:
+            found += [(f.ins[k], t) for k, waits in f.writers(i, {int(m.group(1))}, reach=2).items() if waits < 2 and f.ins[k].startswith('v_')]
     return found
 
 
@@ -203,6 +192,20 @@ def test_scanner_sees_an_early_lane_read():
         v_fmac_f32_dpp v3, v7, v4 row_ror:8 row_mask:0xf bank_mask:0xf
     '''
     assert len(early_lane_reads(asm)) == 1 and not early_lane_reads(asm.replace('v_add', 's_nop 0\nv_add'))
+    # the writer at the end of a loop, the reader right behind its label: the branch is one wait state, the label none
+    loop = '''
+        v_mov_b32_e32 v7, 0
+        s_nop 1
+    .LBB0_2:                                ; =>This Inner Loop Header: Depth=1
+        v_fmac_f32_dpp v3, v7, v4 row_ror:8 row_mask:0xf bank_mask:0xf
+        v_mul_f32_e32 v7, v1, v2
+        s_cbranch_scc1 .LBB0_2
+        s_endpgm
+    '''
+    assert [w for w, _ in early_lane_reads(loop)] == ['v_mul_f32_e32 v7, v1, v2']
+    assert not early_lane_reads(loop.replace('s_cbranch', 's_add_u32 s0, s0, 1\ns_cbranch'))
+    # and one that the code falls through to
+    assert len(early_lane_reads(asm.replace('v_add_f32_e32 v9, v1, v2', '.LBB0_4:   ; %x'))) == 1
 
 
 def test_flags_are_the_makefiles():
