@@ -724,7 +724,8 @@ void launch_bwd_grads(int B, int T, int H, const void* w, const void* q, const v
     const int num_cu = compute_units();
     const int NP = SavedPair::pairs(T / CHUNK), run = ds_run < 0 ? -ds_run : ds_run;
     // what a wavefront takes at a time: a run of pairs (cut per (batch, head) or from the flattened pairs), or a chunk
-    const bool one = fused == 3 && nchunks <= 4 * num_cu;   // (MODE 4; up to 512 pairs, so runs of one: every dstate is there)
+    // (MODE 4: with runs of one, where the reverse scan keeps the dstate of every pair; dstate_run makes no others of so few pairs)
+    const bool one = fused == 3 && run == 1 && nchunks <= 4 * num_cu;
     const int items = fused != 3 || one ? nchunks : ds_run < 0 ? B * H * ((NP + run - 1) / run) : (B * H * NP + run - 1) / run;
     const int blocks = (items + 3) / 4 < num_cu ? (items + 3) / 4 : num_cu;
     auto go = [&](auto kernel) {
