@@ -46,7 +46,9 @@ __device__ __forceinline__ float tanh_of(float x) {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int problem_words16 __attribute__((ext_vector_type(16), aligned(8)));   // (as a LinearProblem lies)
+typedef int problem_words4 __attribute__((ext_vector_type(4), aligned(8)));
+static_assert(alignof(problem_words16) <= alignof(LinearProblem) && alignof(problem_words4) <= alignof(LinearProblem), "what is read as such");
 using Rsrc = __amdgpu_buffer_rsrc_t;
 
 constexpr int BK = 64;           // contraction indices per stage: whole 128-byte lines of a row
@@ -79,8 +81,8 @@ __device__ __forceinline__ void gemm_tile(unsigned char* lds, const LinearProble
     };
     static_assert(offsetof(LinearProblem, lda) == offsetof(Operands, lda) && offsetof(LinearProblem, K) == sizeof(Operands) &&
                   offsetof(LinearProblem, npieces) == sizeof(Operands) + offsetof(Lengths, npieces), "the head of a LinearProblem");
-    i32x16 operand_words = *reinterpret_cast<const i32x16*>(&p);
-    i32x4 length_words = *reinterpret_cast<const i32x4*>(p.K);
+    problem_words16 operand_words = *reinterpret_cast<const problem_words16*>(&p);
+    problem_words4 length_words = *reinterpret_cast<const problem_words4*>(p.K);
     asm volatile("" : "+s"(operand_words), "+s"(length_words));
     const Operands o = __builtin_bit_cast(Operands, operand_words);
     const Lengths len = __builtin_bit_cast(Lengths, length_words);

@@ -249,6 +249,7 @@ using LinInput = std::conditional_t<LERP, MixIn, const __bf16*>;   // what is in
 
 enum { PLAN_C = 13, PLAN_ROWS, PLAN_TILES };   // rows: output rows that exist (stores beyond are dropped)
 static_assert(MAX_SEGS <= PLAN_C && sizeof(LinSeg) == 32 && sizeof(MixIn) == 48, "what the kernel below takes into scalar registers");
+static_assert(alignof(i32x8) <= alignof(LinSeg) && alignof(mix_words8) <= alignof(MixIn) && alignof(mix_words4) <= alignof(MixIn), "what is read as such");
 
 template <class T>
 __device__ __forceinline__ T* global_pointer(int lo, int hi) {   // (an address that the compiler has lost sight of, to global memory all the same)
