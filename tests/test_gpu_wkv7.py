@@ -361,6 +361,22 @@ def test_absent_states_equal_zero_states(B, T, H):
         assert torch.equal(r, g)
 
 
+# (rows of 16 tokens and 2^26 channels on reach past 2 GiB of a tile's first byte)
+@pytest.mark.parametrize('at', [0, (1 << 31) - 1024, (1 << 31) - 512, 1 << 31, (1 << 32) - 2048])
+def test_stores_through_the_l2_reach_four_gib(at):
+    import ctypes
+    import os
+    from wind_rwkv import _native
+    st = ctypes.CDLL(os.path.join(os.path.dirname(_native.LIB_PATH), 'libwind_rwkv7_selftest.so'))
+    st.wind_rwkv7_selftest_store_through.argtypes = [ctypes.c_void_p, ctypes.c_longlong, ctypes.c_longlong, ctypes.c_void_p]
+    out = torch.empty(1 << 30, dtype=torch.int32, device=DEV)
+    here = out[at // 4:at // 4 + 256].fill_(-1)
+    assert st.wind_rwkv7_selftest_store_through(out.data_ptr(), at, 1 << 32, None) == 0
+    torch.cuda.synchronize()
+    want = torch.arange(64, dtype=torch.int32)[:, None] + torch.arange(4, dtype=torch.int32)
+    assert bool((here.view(64, 4).cpu() == want).all())
+
+
 def test_global_to_lds_load_lane_mapping():
     """The hardware fact the gradient kernel's state prefetch is built on: a global -> LDS load of 16 bytes per lane
     (global_load_lds_dwordx4) takes one memory address per lane but writes lane l's piece at the wave-uniform LDS

@@ -17,13 +17,14 @@ __device__ __forceinline__ bf16x8& piece_at(__bf16* base, unsigned bytes) {
     return *reinterpret_cast<bf16x8*>(reinterpret_cast<char*>(base) + bytes);
 }
 // 16 bytes there through the L2 (see store_through in frag.hpp), as a store that the compiler counts: behind one that it does not see it would wait
-// for what was requested before it to be written as well
+// for what was requested before it to be written as well.  base: the same for a wavefront; bytes: up to 2^32 - 32, as
+// far as piece_at reaches (a descriptor holds at most 2^32 - 1 bytes).
 template <class V>
 __device__ __forceinline__ void store_through_at(void* base, unsigned bytes, V v) {
     static_assert(sizeof(V) == 16, "one access");
     typedef unsigned words __attribute__((ext_vector_type(4)));
-    constexpr int DEVICE_SCOPE = 16;
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(words, v), __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000), bytes, 0, DEVICE_SCOPE);
+    constexpr int DEVICE_SCOPE = 16, FOUR_GIB = -1;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(words, v), __builtin_amdgcn_make_buffer_rsrc(base, 0, FOUR_GIB, 0x00020000), bytes, 0, DEVICE_SCOPE);
 }
 // LDS instructions of one wavefront run in their order: what its lanes have written, the others of them may read
 __device__ __forceinline__ void wave_lds_order() {

@@ -1,7 +1,7 @@
 // Device self-test of the fragment primitives (built into its own small library, used by the GPU
 // tests only).  Each entry runs one wavefront and writes plain row-major 16x16 results so the host can
 // compare with ordinary matrix arithmetic.
-#include "frag.hpp"
+#include "row_lines.hpp"
 
 namespace wkv {
 
@@ -222,7 +222,21 @@ __global__ __launch_bounds__(256) void lds_dma_kernel(const int* __restrict__ sr
     for (int i = t; i < 2 * 256 * 4; i += 256) out[i] = buf[i];
 }
 
+// store_through_at: lane l stores {l, l + 1, l + 2, l + 3} 16 l bytes behind `at` of `to`.
+__global__ __launch_bounds__(64) void store_through_kernel(unsigned char* to, unsigned at) {
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const int l = threadIdx.x;
+    store_through_at(to, at + 16 * l, i32x4{l, l + 1, l + 2, l + 3});
+}
+
 }  // namespace wkv
+
+// to: `at` + 1024 bytes or more, of at most 2^32
+extern "C" int wind_rwkv7_selftest_store_through(unsigned char* to, long long at, long long size, void* stream) {
+    if (at < 0 || at % 16 || at + 1024 > size || size > (1LL << 32)) return 1;
+    hipLaunchKernelGGL(wkv::store_through_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), to, (unsigned)at);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+}
 
 extern "C" int wind_rwkv7_selftest_mfma32_layout(float* out, void* stream) {
     hipLaunchKernelGGL(wkv::mfma32_layout_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), out);
