@@ -97,17 +97,18 @@ def _steps(x):
 
 # the two sides of the series' line among them, in every column of a tile; 64 tokens and 128 of it
 @pytest.mark.parametrize('tokens', [510, 20400])
-def test_tanh_of_every_normal_bf16_value(tokens):
-    """W = 1, so the sums are the inputs: tanh is within 2e-6 of itself before it is rounded, half a step and 5e-4 of one."""
+def test_tanh_of_every_finite_bf16_value(tokens):
+    """W = 1, so the sums are the inputs: tanh is the bf16 value nearest to its own in 64 bits.  (That is never closer to the middle between
+    two of them than 8e-6 of itself, so the step through 32 bits that torch's conversion takes does not matter.)"""
     values = torch.arange(0, 65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
-    values = values[values.isfinite() & (values.abs() >= 2.0 ** -126)]
+    values = values[values.isfinite()]
     A = values.repeat(-(-tokens * 128 // values.numel()))[:tokens * 128].view(tokens, 128).contiguous().to(DEV)
+    assert tokens * 128 >= values.numel()
     eye = torch.eye(128, device=DEV, dtype=torch.bfloat16)
     out, plain = torch.empty_like(A), torch.empty(tokens, 64, device=DEV, dtype=torch.bfloat16)
     _run([_problem([(A, eye)], [(out[:, :64], 1, None), (out[:, 64:], 1, None)]), _problem([(A[:, :64], eye[:64, :64])], [(plain, 0, None)])], tokens)
     assert torch.equal(plain, A[:, :64])
-    want = torch.tanh(A.double())
-    assert bool(((out.double() - want).abs() <= 0.501 * _steps(want)).all())
+    assert torch.equal(out, torch.tanh(A.double()).bfloat16())
 
 
 # columns to one, two and four tensors: the derivative's operands are read four columns a lane
