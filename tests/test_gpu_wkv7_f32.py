@@ -72,8 +72,8 @@ def test_f32_many_heads(c_oracle, C):
     _many_heads(c_oracle, 34, 4, C)
 
 
-# blocks per head: 64 channels 2 (70 heads), 2 (260); 128 channels 2 (70), 8 (16); 96 channels 4 (50)
-@pytest.mark.parametrize('B,H,C', [(14, 5, 64), (65, 4, 64), (14, 5, 128), (4, 4, 128), (10, 5, 96), (65, 4, 32)])
+# blocks per head: 64 channels 2 (70 heads), 2 (260); 128 channels 2 (70), 8 (16), 4 (192), 2 (264); 96 channels 4 (50); 80 channels 2 (320)
+@pytest.mark.parametrize('B,H,C', [(14, 5, 64), (65, 4, 64), (14, 5, 128), (4, 4, 128), (10, 5, 96), (65, 4, 32), (48, 4, 128), (66, 4, 128), (40, 8, 80)])
 def test_f32_blocks_per_head(c_oracle, B, H, C):
     """The scan cuts a head over more or fewer blocks by the number of (batch, head) pairs."""
     _many_heads(c_oracle, B, H, C)

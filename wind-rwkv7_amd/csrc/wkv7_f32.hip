@@ -32,8 +32,8 @@
 // A caller without a workspace gets the backward in one kernel: two blocks of four wavefronts per head, the walk back in
 // windows of recomputed states, and the gradients that sum over value rows added by the two blocks onto zeroed tensors
 // with atomics (two addends: the order does not show).  Forward + backward, microseconds, one kernel -> two:
-//   1 x 256 tokens x 4 heads of 64   274 -> 99-110     8 x 1024 x 6 heads of 128   2420 -> 811
-//   8 x 1024 x 12 heads of 64        831 -> 430        32 x 1024 x 12 heads of 64  2395 -> 1356
+//   1 x 256 tokens x 4 heads of 64   172 -> 67         8 x 1024 x 6 heads of 128   2225 -> 700
+//   8 x 1024 x 12 heads of 64        745 -> 388        32 x 1024 x 12 heads of 64  2215 -> 1298
 #include "wkv7_f32_kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -1051,17 +1051,18 @@ __global__ __launch_bounds__(256) void zero5_kernel(long n4, f4* __restrict__ p0
 }
 
 
-// Blocks per head in the scan.  Up to 64 channels: as many of 4, 2, 1 as still leave every block a compute unit of its own
-// (us per 1024 tokens: 98, 160, 250; 96 heads in 4 blocks each 184, in 2 165; 256 heads in 2 blocks each 340, in 1 290),
-// and 2 again past one head per compute unit, where several blocks share one and smaller ones fill it more evenly (384
-// heads x 512 tokens in 1 block each 264 us, in 2 245 us).  Above 64 channels a block has a compute unit to itself (LDS),
-// so the blocks run in rounds: the fewest rounds x time of a round (ns per token: 215, 350, 600 in 8, 4, 2 blocks; 192
-// heads x 256 tokens: 350, 275, 311 us).
+// Blocks per head in the scan, by the times of the forward one (us).  Up to 64 channels: as many of 4, 2, 1 as still leave every block a compute
+// unit of its own (1024 tokens: 97, 130, 203; 96 heads in 4 blocks each 145, in 2 131; 192 heads in 2 blocks each 234, in 1 206),
+// and 2 again past one head per compute unit, where several blocks share one and smaller ones fill it more evenly (512 tokens in 1 block
+// each, in 2: 288 heads 189, 162; 384 196, 182; 576 289, 273.  Where the heads fill whole rounds of the compute units, or nearly, 1 takes less: 448
+// heads 202, 220; 512 214, 232; 1024 411, 459; with the backward pass 4-7 %).  Above 64 channels a block has a compute unit to itself
+// (LDS), so the blocks run in rounds: the fewest rounds x time of a round (ns per token, 128 channels: 165, 220, 358 in 8, 4, 2
+// blocks; 512 tokens in 4, 2 blocks: 136 heads 341, 371; 192 376, 380; 264 581, 565; 320 628, 574; 448 870, 758).
 int scan_split(int BH, int C) {
     const long cus = compute_units(), n = BH;
     if (C <= 64) return 4 * n <= cus ? 4 : 2 * n <= cus || n > cus ? 2 : 1;
     auto cost = [&](int split, int ns) { return (split * n + cus - 1) / cus * ns; };
-    const long c8 = cost(8, 215), c4 = cost(4, 350), c2 = cost(2, 600);
+    const long c8 = cost(8, 165), c4 = cost(4, 220), c2 = cost(2, 358);
     return c8 <= c4 && c8 <= c2 ? 8 : c4 <= c2 ? 4 : 2;
 }
 
