@@ -244,7 +244,13 @@ constexpr int STREAMED = 2;   // of a buffer store
 template <class V>
 __device__ __forceinline__ void store_streamed(void* to, V x) { __builtin_nontemporal_store(x, static_cast<V*>(to)); }
 // 16 bytes to memory at device scope: written through the XCD's L2, so that the end of the kernel, which writes back whatever that still holds
-// for the other XCDs' L2s, finds nothing left to do, and kept in the last-level cache for whoever reads them next.
+// for the other XCDs' L2s, finds nothing left to do, and kept in the last-level cache for whoever reads them next.  That counts while the output is not many times
+// what the L2s hold (4 MiB each); behind that it is the same either way, so there is no line.  Through / left to the end, us, on three sets of tensors, 768 channels,
+// at 2048, 8192, 16384, 32768, 65536 tokens: one product 9.3 / 9.6, 15.8 / 16.8, 25.8 / 27.1, 55.1 / 54.7, 103.1 / 102.4 (one side's runs differ by
+// 2-4 %); three with the first halves 19.2 / 19.7, 48.0 / 48.8, 80.3 / 81.4, 153 / 152, 303 / 301; ddlerp 15.3 / 17.5, 27.7 / 29.3, 44.3 / 44.9,
+// 89.6 / 89.5, 170 / 172; LoRA expansion 9.7 / 12.0, 19.8 / 21.4, 40.8 / 40.0, 67.6 / 68.9, 145.0 / 145.5.  A block's forward + backward at the last three
+// 963.5 / 962.7, 1802 / 1802, 3311 / 3298.  Chunk records, with the scan that reads them, 1920, 3072, 4224, 5376, 6144 chunks 20.0 / 21.8, 30.6 / 31.0,
+// 40.6 / 40.8, 57.1 / 58.0, 58.1 / 58.4.
 // (s_nop: two wait states before the registers of a store of more than eight bytes may be written, which the compiler sees to for its own stores.)
 // x is not the result of a matrix instruction as it stands: the distance a store needs behind that, too, the compiler keeps only for its own stores
 // (store_through_at in row_lines.hpp).
