@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256) void neutral_rows_kernel(int T, int C, int fir
     *reinterpret_cast<bf16x8*>(b + at) = zero;
 }
 
-// Bound by the launch (stored through the L2 3.5 -> 3.2 us): 2 x 1003 tokens x 768 channels take 3.4-4.1 us; a fill, a copy and a copy of the last token, 11.
+// Bound by the launch: 2 x 1003 tokens x 768 channels take 3.2 us (3.5 not stored through the L2); a fill, a copy and a copy of the last token, 11.
 __global__ __launch_bounds__(256) void pad_rows_kernel(const PadArgs p) { pad_rows_block(p, blockIdx.x); }
 
 }  // namespace

@@ -237,8 +237,8 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef int mix_words8 __attribute__((ext_vector_type(8), aligned(8)));   // (as a MixIn lies)
 typedef int mix_words4 __attribute__((ext_vector_type(4), aligned(8)));
 // As many pairs as a launch has, and beside them only the input that it reads: the host writes a kernel's arguments anew for every
-// launch, and with 496 bytes for either kernel that bounded a step of few sequences (12 heads, one sequence: 15.4 us for the host to
-// issue the four launches, an eager step 19.0; with 400 and 104 bytes 13.2 and 17.1).
+// launch, and that bounds a step of few sequences (12 heads, one sequence, called eagerly, a process at the lower or the higher of the two
+// speeds at which the host runs: with 496 bytes for either kernel 19.5 or 17.4 us, with 400 and 104 19.3 or 17.1; replayed 16.7, 16.5).
 template <int SEGS>
 struct LinArgs {
     i32x16 plan;   // of the launch: blocks of each pair (0 past the last one); PLAN_C and so on

@@ -96,9 +96,10 @@ __global__ __launch_bounds__(256) void ln_epilogue_bwd_kernel(int T, int H, int 
 // MODE 4: the same arrays, but a wavefront takes ONE chunk and ends, where there are no more chunks than wavefronts that run at once
 // (four per compute unit): bound by latency there, and half of it was the pair's other chunk.  The wavefront of the later chunk
 // advances the forward state as above; that of the earlier one hands the dstate on to itself first, from the later chunk's w, q,
-// a, dY and dab_u^T.  The same instructions on the same operands: the same bits.  Forward + backward, us, MODE 3 -> 4:
-// attn 1 x 256 tokens x 4 heads 48.8 -> 42.6, 8 x 64 x 12 34.8 -> 26.5, 1 x 1024 x 16 (1024 chunks) 96.8 -> 90.9, attn_ln
-// 1 x 256 x 4 61.8 -> 53.6, 1 x 1024 x 16 112 -> 105.  With more chunks every wavefront has a pair to do either way.
+// a, dY and dab_u^T.  The same instructions on the same operands: the same bits.  Forward + backward replayed from a graph, us, MODE 3 -> 4:
+// attn 1 x 256 tokens x 4 heads 47.9 -> 41.8, 8 x 64 x 12 34.1 -> 26.0, 1 x 1024 x 16 (1024 chunks) 96.2 -> 90.6, attn_ln
+// 1 x 256 x 4 60.8 -> 52.7, 1 x 1024 x 16 112 -> 105.  (A pass called eagerly waits for the host as long as that takes more: 1 x 256 x 4
+// 84-88 either way.)  With more chunks every wavefront has a pair to do either way.
 namespace pairlds {   // byte offsets inside a wavefront's 36 KiB
 constexpr int STASH = 0;              // the state entering the pair: [ib][half][lane] x 16 B (fragments jb = 2 half, 2 half + 1)
 constexpr int CARRY = 8192;           // the dstate arriving at the end of the current chunk, same layout
