@@ -79,6 +79,17 @@ def test_f32_blocks_per_head(c_oracle, B, H, C):
     _many_heads(c_oracle, B, H, C)
 
 
+# (4 and 2 blocks a head have the same lanes and columns to a row of the state; the other gradients come from kernels chosen by the chunks)
+@pytest.mark.parametrize('C', [80, 128])
+def test_f32_two_blocks_a_head_give_the_bits_of_four(C):
+    B, T, H, few = 66, 32, 4, 16   # 264 heads: 2 blocks each; 64: 4
+    d = inputs.wkv7_inputs(B, T, H, C, seed=270 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
+    y, sT, grads, ds0 = _run(d, B, T, H, C, True)
+    y4, sT4, grads4, ds04 = _run({n: t[:few] for n, t in d.items()}, few, T, H, C, True)
+    for whole, part in ((y, y4), (sT, sT4), (ds0, ds04), (grads[NAMES.index('v')], grads4[NAMES.index('v')])):   # (what the scans make)
+        assert torch.equal(whole[:few], part)
+
+
 def _many_heads(c_oracle, B, H, C):
     T = 32
     d = inputs.wkv7_inputs(B, T, H, C, seed=260 + C, dtype=torch.float32, s0_scale=0.3, dsT_scale=1.0)
